@@ -88,6 +88,12 @@ PLAN_API = {
                                              c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp]),
     "bpt_plan_link_device": (ctypes.c_int, [c_vp, c_vp, c_i32, c_vp, c_vp, c_i32, c_i64, c_i32, c_vp, c_vp, c_i64, c_vp]),
 }
+# the same library, include/bptbuild.h: a batch's CSRs and plans in few launches
+BUILD_API = {
+    "bpt_build_csrs_device": (ctypes.c_int, [c_vp, c_vp, c_i64, c_i64, c_i32, ctypes.POINTER(c_vp * 5), ctypes.POINTER(c_vp * 5), c_vp,
+                                             c_vp, c_i64, c_vp]),
+    "bpt_build_wait": (ctypes.c_int, [c_vp]),
+}
 
 _graph = None
 _attn = None
@@ -126,7 +132,7 @@ def attn_lib():
 def plan_lib():
     global _plan
     if _plan is None:
-        _plan = _load(PLAN_SO, PLAN_API, "libbptplan (plans built on the GPU)")
+        _plan = _load(PLAN_SO, {**PLAN_API, **BUILD_API}, "libbptplan (plans built on the GPU)")
     return _plan
 
 

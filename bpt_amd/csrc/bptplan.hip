@@ -1,4 +1,4 @@
-// libbptplan — launch plans and row groups built on the GPU (gfx950), C ABI of include/bptplan.h.
+// libbptplan — launch plans and row groups built on the GPU (gfx950), C ABI of include/bptplan.h and include/bptbuild.h.
 //
 // The host builder (bptgraph.cpp) needs the index arrays on the host and tens of milliseconds per new graph.  Here the
 // same plan comes out of sorts and prefix sums over the device arrays: every step is a data-parallel kernel or a
@@ -16,6 +16,7 @@
 #include <cstdint>
 
 #include "../../include/bptattn.h"
+#include "../../include/bptbuild.h"
 #include "../../include/bptplan.h"
 
 namespace {
@@ -85,6 +86,200 @@ __global__ void k_iota_i32(int32_t *p, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
     if (i < n) p[i] = (int32_t)i;
 }
+
+// ---- stable radix sort --------------------------------------------------------------------------------------------------
+// A graph's sorts are small (10^4 .. 10^6 records, keys below the number of nodes), and there the library sort runs some twenty
+// merge launches of 5 us each whatever the key width.  Here a sort is two or three least-significant-digit passes of at most 9
+// bits (up to 18 key bits: two), each three launches: digit counts per tile of 2048 records, prefix over the tiles, stable
+// scatter; both CSR sides share the launches (blockIdx.y).  What bounds a pass at these sizes is the launches' latency
+// (4-10 us each), then the scatter's uncoalesced stores (576 k edges x 2 sides: 24 us with the 16-byte slots of the last pass).
+// Both CSR sides of an edge list, call to call with the read-back: 33 765 nodes / 576 k edges 398 -> 159 us, 65 535 / 3.3 M
+// 626 -> 420 us, 1 023 / 17 k 187 -> 113 us (host-bound).
+constexpr int RS_KPT = 8;                         // records per thread
+constexpr int RS_TILE = TPB * RS_KPT;
+constexpr int RS_MAX_BITS = 9;
+constexpr int RS_BINS = 1 << RS_MAX_BITS;
+constexpr int RS_PREFIX_TPB = 1024;
+
+struct RsPasses {
+    int n, bits;                                  // passes, digit bits of each
+};
+
+inline RsPasses rs_passes(uint64_t max_key) {
+    const unsigned b = bits_for(max_key);
+    RsPasses p;
+    p.n = (int)((b + RS_MAX_BITS - 1) / RS_MAX_BITS);
+    p.bits = (int)((b + p.n - 1) / p.n);
+    return p;
+}
+
+inline int64_t rs_tiles(int64_t n) { return (n + RS_TILE - 1) / RS_TILE; }
+
+// orders a wavefront's LDS accesses across its lanes: what one lane wrote is what another reads next
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// exclusive prefix sum of one value per thread over a block of NW wavefronts; sh holds NW + 1 ints
+template <int NW> __device__ __forceinline__ int32_t block_excl_sum(int32_t v, int32_t *sh, int32_t &total) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int32_t x = v;
+    for (int d = 1; d < 64; d <<= 1) {
+        const int32_t y = __shfl_up(x, d);
+        if (lane >= d) x += y;
+    }
+    __syncthreads();                              // (sh may still be in use by the caller's previous step)
+    if (lane == 63) sh[wave] = x;
+    __syncthreads();
+    int32_t before = 0, all = 0;
+    for (int w = 0; w < NW; ++w) {
+        const int32_t c = sh[w];
+        before += w < wave ? c : 0;
+        all += c;
+    }
+    total = all;
+    return before + x - v;
+}
+
+// counts[side][tile][bin]: how many records of the tile have the digit
+template <class Recs>
+__global__ __launch_bounds__(TPB) void k_rs_count(Recs recs, int64_t n, int shift, int bits, int32_t *counts) {
+    __shared__ int32_t h[RS_BINS];
+    const int bins = 1 << bits, side = blockIdx.y;
+    for (int b = threadIdx.x; b < bins; b += TPB) h[b] = 0;
+    __syncthreads();
+    const int64_t i0 = (int64_t)blockIdx.x * RS_TILE;
+    bool bad = false;
+    for (int r = 0; r < RS_KPT; ++r) {
+        const int64_t i = i0 + r * TPB + threadIdx.x;
+        const bool on = i < n;
+        const int d = on ? (int)((recs.key(side, i, bad) >> shift) & (uint32_t)(bins - 1)) : -1;
+        const int first = __builtin_amdgcn_readfirstlane(d);
+        const uint64_t same = __ballot(d == first);
+        if (same == ~uint64_t(0) && first >= 0) {             // (a high digit is often one value over a whole wavefront)
+            if ((threadIdx.x & 63) == 0) atomicAdd(&h[first], 64);
+        } else if (on) {
+            atomicAdd(&h[d], 1);
+        }
+    }
+    recs.report(side, __syncthreads_or(bad ? 1 : 0) != 0);
+    int32_t *out = counts + ((int64_t)side * gridDim.x + blockIdx.x) * bins;
+    for (int b = threadIdx.x; b < bins; b += TPB) out[b] = h[b];
+}
+
+// in place: counts[side][tile][bin] -> the records with that digit in the tiles before; totals[side][bin]: in all tiles.
+// A block owns 64 bins (one per lane), its 16 wavefronts share the tiles.
+__global__ __launch_bounds__(RS_PREFIX_TPB) void k_rs_prefix(int32_t *counts, int32_t *totals, int64_t n_tiles, int bins) {
+    __shared__ int32_t part[RS_PREFIX_TPB / 64][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = RS_PREFIX_TPB / 64;
+    const int bin = blockIdx.x * 64 + lane, side = blockIdx.y;
+    const int64_t per = (n_tiles + n_waves - 1) / n_waves, t0 = wave * per, t1 = t0 + per < n_tiles ? t0 + per : n_tiles;
+    int32_t *c = counts + (int64_t)side * n_tiles * bins + bin;
+    const bool on = bin < bins;
+    int32_t sum = 0;
+    if (on)
+        for (int64_t t = t0; t < t1; ++t) sum += c[t * bins];
+    part[wave][lane] = sum;
+    __syncthreads();
+    int32_t run = 0, all = 0;
+    for (int w = 0; w < n_waves; ++w) {
+        run += w < wave ? part[w][lane] : 0;
+        all += part[w][lane];
+    }
+    if (!on) return;
+    if (wave == 0) totals[side * bins + bin] = all;
+    for (int64_t t = t0; t < t1; t += 8) {            // (eight loads in flight: the stores in between would serialise them)
+        int32_t v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = t + j < t1 ? c[(t + j) * bins] : 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (t + j < t1) c[(t + j) * bins] = run;
+            run += v[j];
+        }
+    }
+}
+
+// Stable scatter of a tile: a wavefront ranks 64 records at a time among its lanes with the same digit (one ballot per digit bit)
+// on top of its running counts in LDS.
+template <class Recs, class Out>
+__global__ __launch_bounds__(TPB) void k_rs_scatter(Recs recs, Out out, int64_t n, int shift, int bits, const int32_t *counts,
+                                                    const int32_t *totals) {
+    constexpr int NW = TPB / 64;
+    __shared__ int32_t wh[NW][RS_BINS];
+    __shared__ int32_t sh[NW + 1];
+    const int bins = 1 << bits, side = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int b = threadIdx.x; b < bins; b += TPB)
+        for (int w = 0; w < NW; ++w) wh[w][b] = 0;
+    __syncthreads();
+    const int64_t i0 = (int64_t)blockIdx.x * RS_TILE + wave * (64 * RS_KPT) + lane;
+    const uint64_t below = (uint64_t(1) << lane) - 1;
+    uint32_t key[RS_KPT];
+    int32_t rank[RS_KPT];
+    bool bad = false;
+#pragma unroll
+    for (int r = 0; r < RS_KPT; ++r) key[r] = i0 + r * 64 < n ? recs.key(side, i0 + r * 64, bad) : 0u;
+#pragma unroll
+    for (int r = 0; r < RS_KPT; ++r) {
+        const bool on = i0 + r * 64 < n;
+        const int d = (int)((key[r] >> shift) & (uint32_t)(bins - 1));
+        uint64_t peers = __ballot(on);
+        for (int b = 0; b < bits; ++b) {
+            const bool bit = (d >> b) & 1;
+            const uint64_t m = __ballot(bit);
+            peers &= bit ? m : ~m;
+        }
+        const int32_t before = wh[wave][d];
+        rank[r] = before + __popcll(peers & below);
+        wave_lds_order();
+        if (on && (peers & below) == 0) wh[wave][d] = before + __popcll(peers);
+        wave_lds_order();
+    }
+    // where the tile's records of every digit start: two bins a thread
+    int32_t tot[2] = {0, 0}, pre[2] = {0, 0}, all;
+    const int b0 = 2 * threadIdx.x;
+    for (int t = 0; t < 2; ++t)
+        if (b0 + t < bins) {
+            tot[t] = totals[side * bins + b0 + t];
+            pre[t] = counts[((int64_t)side * gridDim.x + blockIdx.x) * bins + b0 + t];
+        }
+    int32_t start = block_excl_sum<NW>(tot[0] + tot[1], sh, all);
+    for (int t = 0; t < 2; ++t) {
+        if (b0 + t < bins) {
+            int32_t at = start + pre[t];
+            for (int w = 0; w < NW; ++w) {
+                const int32_t c = wh[w][b0 + t];
+                wh[w][b0 + t] = at;
+                at += c;
+            }
+        }
+        start += tot[t];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RS_KPT; ++r) {
+        const int64_t i = i0 + r * 64;
+        if (i < n) out.put(side, (int64_t)wh[wave][(key[r] >> shift) & (uint32_t)(bins - 1)] + rank[r], key[r], recs.val(side, i));
+    }
+}
+
+// records in plain arrays (the passes after the first)
+struct RsArrays {
+    const uint32_t *k[2];
+    const int32_t *v[2];
+    __device__ uint32_t key(int side, int64_t i, bool &) const { return k[side][i]; }
+    __device__ int32_t val(int side, int64_t i) const { return v[side][i]; }
+    __device__ void report(int, bool) const {}
+};
+struct RsToArrays {
+    uint32_t *k[2];
+    int32_t *v[2];
+    __device__ void put(int side, int64_t at, uint32_t key, int32_t val) const {
+        k[side][at] = key;
+        v[side][at] = val;
+    }
+};
 
 // ---- base plan ---------------------------------------------------------------------------------------------------------
 struct BaseWs {
@@ -682,91 +877,139 @@ bool graph_args_ok(int kind, int64_t length, int64_t a, int64_t b) {
 }
 
 // ---- CSR of an edge list ------------------------------------------------------------------------------------------------
-__global__ void k_csr_keys(const int64_t *rows, const int64_t *cols, int64_t n_edges, int64_t n_nodes, int32_t *info,
-                           uint32_t *key, int32_t *val) {
-    const int64_t e = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (e == 0) info[1] = 0;
-    if (e >= n_edges) return;
-    const int64_t r = rows[e], c = cols[e];
-    const bool ok = r >= 0 && r < n_nodes && c >= 0 && c < n_nodes;
-    if (!ok) atomicMax(&info[0], 1);
-    key[e] = ok ? (uint32_t)r : PAD32;
-    val[e] = (int32_t)e;
-}
+// Both sides of a graph (or one of them) in the same launches, blockIdx.y = side.  Edges sorted by row with their ids as
+// they come, so ascending edge id inside a row; the last pass writes the 64-bit eid and indices itself.
+struct CsrSide {
+    const int64_t *rows, *cols;
+    int64_t *indptr, *indices, *eid, *unit_row, *unit_ptr;
+    int32_t *info;
+    uint32_t *key_s;                  // rows of the slots, sorted
+    int32_t *lo_of, *unit_total;      // first slot of every row; units of every block of CSR_ROWS rows
+    int32_t *bad;                     // per tile of edges: an id out of range
+};
+struct CsrSides {
+    CsrSide side[2];
+};
 
-__global__ void k_csr_slots(const int64_t *cols, const int32_t *val_s, int64_t n_edges, const int32_t *info, int64_t *indices,
-                            int64_t *eid) {
-    const int64_t p = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (p >= n_edges || info[0]) return;
-    const int32_t e = val_s[p];
-    eid[p] = e;
-    indices[p] = cols[e];
-}
+struct CsrEdges {                     // records of the first pass: the edges themselves; an edge with a bad id sorts behind all rows
+    CsrSides g;
+    int64_t n_nodes;
+    __device__ uint32_t key(int side, int64_t e, bool &bad) const {
+        const int64_t r = g.side[side].rows[e], c = g.side[side].cols[e];
+        const bool ok = r >= 0 && r < n_nodes && c >= 0 && c < n_nodes;
+        bad = bad || !ok;
+        return ok ? (uint32_t)r : (uint32_t)n_nodes;
+    }
+    __device__ int32_t val(int, int64_t e) const { return (int32_t)e; }
+    __device__ void report(int side, bool bad) const {
+        if (threadIdx.x == 0) g.side[side].bad[blockIdx.x] = bad ? 1 : 0;
+    }
+};
+struct CsrSlots {                     // what the last pass writes
+    CsrSides g;
+    __device__ void put(int side, int64_t at, uint32_t key, int32_t e) const {
+        const CsrSide &c = g.side[side];
+        c.key_s[at] = key;
+        c.eid[at] = e;
+        c.indices[at] = c.cols[e];
+    }
+};
 
-// indptr[r] = first slot whose row is >= r; number of chunked units of every row
-__global__ void k_csr_indptr(const uint32_t *key_s, int64_t n_edges, int64_t n_nodes, int32_t chunk, const int32_t *info,
-                             int64_t *indptr, int32_t *lo_of, int32_t *n_units_of) {
-    const int64_t r = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (r > n_nodes || info[0]) return;
+constexpr int CSR_ROWS = TPB - 1;     // rows of a block of the two kernels below (one thread more: the end of the last row)
+
+// indptr[r] = first slot whose row is >= r; how many chunked units the block's rows give
+__global__ __launch_bounds__(TPB) void k_csr_rows(CsrSides g, int64_t n_edges, int64_t n_nodes, int32_t chunk) {
+    __shared__ int32_t lo_sh[TPB];
+    __shared__ int32_t sh[TPB / 64 + 1];
+    const CsrSide &c = g.side[blockIdx.y];
+    const int64_t r = (int64_t)blockIdx.x * CSR_ROWS + threadIdx.x;
     int64_t lo = 0, hi = n_edges;
-    while (lo < hi) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (key_s[mid] < (uint32_t)r) lo = mid + 1; else hi = mid;
+    if (r <= n_nodes) {
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) >> 1;
+            if (c.key_s[mid] < (uint32_t)r) lo = mid + 1; else hi = mid;
+        }
+        c.indptr[r] = lo;
+        c.lo_of[r] = (int32_t)lo;
     }
-    indptr[r] = lo;
-    lo_of[r] = (int32_t)lo;
+    lo_sh[threadIdx.x] = (int32_t)lo;
+    __syncthreads();
+    int32_t units = 0, total;
+    if (threadIdx.x < CSR_ROWS && r < n_nodes) units = (lo_sh[threadIdx.x + 1] - (int32_t)lo + chunk - 1) / chunk;
+    block_excl_sum<TPB / 64>(units, sh, total);
+    if (threadIdx.x == 0) c.unit_total[blockIdx.x] = total;
 }
 
-__global__ void k_csr_unit_counts(const int32_t *lo_of, int64_t n_nodes, int32_t chunk, const int32_t *info, int32_t *n_units_of) {
-    const int64_t r = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (r > n_nodes || info[0]) return;
-    n_units_of[r] = (r < n_nodes) ? (lo_of[r + 1] - lo_of[r] + chunk - 1) / chunk : 0;
-}
-
-// the units of builder.pyx:305-321: each row's slot range in chunks of at most `chunk` slots; empty rows give no unit
-__global__ void k_csr_units(const int32_t *lo_of, const int32_t *unit_base, int64_t n_nodes, int64_t n_edges, int32_t chunk,
-                            int32_t *info, int64_t *unit_row, int64_t *unit_ptr) {
-    const int64_t r = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (r > n_nodes || info[0]) return;
-    if (r == n_nodes) {
-        info[1] = unit_base[n_nodes];
-        unit_ptr[unit_base[n_nodes]] = n_edges;
-        return;
+// the units of builder.pyx:305-321: each row's slot range in chunks of at most `chunk` slots; empty rows give no unit.  A row
+// of more than CSR_FEW units is written by the whole block.
+constexpr int CSR_FEW = 8;
+__global__ __launch_bounds__(TPB) void k_csr_units(CsrSides g, int64_t n_edges, int64_t n_nodes, int32_t chunk, int64_t n_tiles) {
+    __shared__ int32_t sh[TPB / 64 + 1];
+    __shared__ int32_t many[TPB][3];
+    __shared__ int32_t n_many;
+    const CsrSide &c = g.side[blockIdx.y];
+    if (threadIdx.x == 0) n_many = 0;
+    int32_t part = 0, before, total;
+    for (int64_t b = threadIdx.x; b < (int64_t)blockIdx.x; b += TPB) part += c.unit_total[b];
+    block_excl_sum<TPB / 64>(part, sh, before);
+    const int64_t r = (int64_t)blockIdx.x * CSR_ROWS + threadIdx.x;
+    const bool mine = threadIdx.x < CSR_ROWS && r < n_nodes;
+    const int32_t lo = mine ? c.lo_of[r] : 0, hi = mine ? c.lo_of[r + 1] : 0, units = (hi - lo + chunk - 1) / chunk;
+    const int32_t at = before + block_excl_sum<TPB / 64>(units, sh, total);
+    if (units <= CSR_FEW) {
+        for (int32_t u = 0; u < units; ++u) {
+            c.unit_row[at + u] = r;
+            c.unit_ptr[at + u] = lo + (int64_t)u * chunk;
+        }
+    } else {
+        const int i = atomicAdd(&n_many, 1);
+        many[i][0] = (int32_t)threadIdx.x;
+        many[i][1] = at;
+        many[i][2] = lo;
     }
-    const int32_t b = lo_of[r], e = lo_of[r + 1];
-    int64_t u = unit_base[r];
-    for (int32_t p = b; p < e; p += chunk, ++u) {
-        unit_row[u] = r;
-        unit_ptr[u] = p;
+    __syncthreads();
+    for (int i = 0; i < n_many; ++i) {
+        const int64_t row = (int64_t)blockIdx.x * CSR_ROWS + many[i][0];
+        const int32_t first = many[i][1], slot = many[i][2], n = (c.lo_of[row + 1] - slot + chunk - 1) / chunk;
+        for (int32_t u = threadIdx.x; u < n; u += TPB) {
+            c.unit_row[first + u] = row;
+            c.unit_ptr[first + u] = slot + (int64_t)u * chunk;
+        }
+    }
+    if (blockIdx.x == gridDim.x - 1) {
+        bool bad = false;
+        for (int64_t t = threadIdx.x; t < n_tiles; t += TPB) bad = bad || c.bad[t] != 0;
+        const int any = __syncthreads_or(bad ? 1 : 0);
+        if (threadIdx.x == 0) {
+            c.info[0] = any ? 1 : 0;
+            c.info[1] = before + total;
+            c.unit_ptr[before + total] = n_edges;
+        }
     }
 }
 
 struct CsrWs {
-    uint32_t *key, *key_s;
-    int32_t *val, *val_s, *lo_of, *n_units_of, *unit_base;
-    void *tmp;
+    uint32_t *key[2];
+    int32_t *val[2];
+    int32_t *counts, *totals;
 };
 
-CsrWs csr_layout(Bump &b, int64_t n_edges, int64_t n_nodes, size_t tmp_bytes) {
+CsrWs csr_layout(Bump &b, int64_t n_edges, int64_t n_nodes, int n_sides, CsrSides &g) {
     CsrWs w;
-    w.key = b.take<uint32_t>(n_edges);
-    w.key_s = b.take<uint32_t>(n_edges);
-    w.val = b.take<int32_t>(n_edges);
-    w.val_s = b.take<int32_t>(n_edges);
-    w.lo_of = b.take<int32_t>(n_nodes + 1);
-    w.n_units_of = b.take<int32_t>(n_nodes + 1);
-    w.unit_base = b.take<int32_t>(n_nodes + 1);
-    w.tmp = b.take<char>((int64_t)tmp_bytes);
+    const int64_t row_blocks = (n_nodes + CSR_ROWS) / CSR_ROWS;
+    for (int i = 0; i < n_sides; ++i) {
+        g.side[i].key_s = b.take<uint32_t>(n_edges);
+        g.side[i].lo_of = b.take<int32_t>(n_nodes + 2);
+        g.side[i].unit_total = b.take<int32_t>(row_blocks);
+        g.side[i].bad = b.take<int32_t>(rs_tiles(n_edges));
+    }
+    w.key[0] = b.take<uint32_t>(n_sides * n_edges);
+    w.key[1] = b.take<uint32_t>(n_sides * n_edges);
+    w.val[0] = b.take<int32_t>(n_sides * n_edges);
+    w.val[1] = b.take<int32_t>(n_sides * n_edges);
+    w.counts = b.take<int32_t>(n_sides * rs_tiles(n_edges) * RS_BINS);
+    w.totals = b.take<int32_t>(n_sides * RS_BINS);
     return w;
-}
-
-hipError_t csr_temp_bytes(int64_t n_edges, int64_t n_nodes, size_t *out) {
-    size_t a = 0, b = 0;
-    hipError_t e;
-    if ((e = sort_pairs<uint32_t>(nullptr, a, nullptr, nullptr, nullptr, nullptr, n_edges + 1, 32, nullptr)) != hipSuccess) return e;
-    if ((e = scan_i32(nullptr, b, nullptr, nullptr, n_nodes + 1, nullptr)) != hipSuccess) return e;
-    *out = (a > b ? a : b) + 256;
-    return hipSuccess;
 }
 
 int sizes_ok(int64_t n_units, int64_t n_edges, int64_t n_rows, int64_t n_index_nodes, int32_t seg_len) {
@@ -790,9 +1033,75 @@ int sizes_ok(int64_t n_units, int64_t n_edges, int64_t n_rows, int64_t n_index_n
         }                                                                              \
     } while (0)
 
+// one stable sort pass over both sides: counts, prefix, scatter
+template <class Recs, class Out>
+int rs_pass(const Recs &recs, const Out &out, int64_t n, int n_sides, int shift, int bits, int32_t *counts, int32_t *totals, hipStream_t s) {
+    const dim3 tiles((unsigned)rs_tiles(n), (unsigned)n_sides);
+    const int bins = 1 << bits;
+    hipLaunchKernelGGL(k_rs_count<Recs>, tiles, dim3(TPB), 0, s, recs, n, shift, bits, counts);
+    HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(k_rs_prefix, dim3((unsigned)((bins + 63) / 64), (unsigned)n_sides), dim3(RS_PREFIX_TPB), 0, s, counts, totals,
+                       (int64_t)tiles.x, bins);
+    HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL((k_rs_scatter<Recs, Out>), tiles, dim3(TPB), 0, s, recs, out, n, shift, bits, counts, totals);
+    HIP_TRY(hipGetLastError());
+    return BPT_OK;
+}
+
+int csr_build(CsrSides g, int n_sides, int64_t n_edges, int64_t n_nodes, int32_t chunk, void *workspace, int64_t workspace_bytes,
+              hipStream_t s) {
+    if (n_edges < 0 || n_nodes < 0 || n_edges >= INT32_MAX || n_nodes >= INT32_MAX) return BPT_ERR_SIZE;
+    if (chunk < 1) return BPT_ERR_SHAPE;
+    if (!workspace) return BPT_ERR_NULL;
+    for (int i = 0; i < n_sides; ++i) {
+        const CsrSide &c = g.side[i];
+        if (!c.indptr || !c.unit_ptr || !c.info) return BPT_ERR_NULL;
+        if (n_edges > 0 && (!c.rows || !c.cols || !c.indices || !c.eid || !c.unit_row)) return BPT_ERR_NULL;
+    }
+    Bump bump{(char *)workspace, 0};
+    CsrWs w = csr_layout(bump, n_edges, n_nodes, n_sides, g);
+    if (workspace_bytes < (int64_t)bump.off) return BPT_ERR_WORKSPACE;
+    if (n_edges > 0) {
+        const RsPasses ps = rs_passes((uint64_t)n_nodes);       // (n_nodes: the key of an edge with a bad id)
+        const CsrEdges edges{g, n_nodes};
+        const CsrSlots slots{g};
+        RsToArrays to[2];
+        RsArrays from[2];
+        for (int t = 0; t < 2; ++t)
+            for (int i = 0; i < 2; ++i) {
+                const int64_t at = (i < n_sides ? i : 0) * n_edges;
+                to[t].k[i] = w.key[t] + at;
+                to[t].v[i] = w.val[t] + at;
+                from[t].k[i] = to[t].k[i];
+                from[t].v[i] = to[t].v[i];
+            }
+        for (int p = 0; p < ps.n; ++p) {
+            const int shift = p * ps.bits;
+            const bool first = p == 0, last = p == ps.n - 1;
+            int st;
+            if (first && last) st = rs_pass(edges, slots, n_edges, n_sides, shift, ps.bits, w.counts, w.totals, s);
+            else if (first) st = rs_pass(edges, to[0], n_edges, n_sides, shift, ps.bits, w.counts, w.totals, s);
+            else if (last) st = rs_pass(from[(p - 1) & 1], slots, n_edges, n_sides, shift, ps.bits, w.counts, w.totals, s);
+            else st = rs_pass(from[(p - 1) & 1], to[p & 1], n_edges, n_sides, shift, ps.bits, w.counts, w.totals, s);
+            if (st != BPT_OK) return st;
+        }
+    }
+    const dim3 rows((unsigned)((n_nodes + CSR_ROWS) / CSR_ROWS), (unsigned)n_sides);
+    hipLaunchKernelGGL(k_csr_rows, rows, dim3(TPB), 0, s, g, n_edges, n_nodes, chunk);
+    HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(k_csr_units, rows, dim3(TPB), 0, s, g, n_edges, n_nodes, chunk, n_edges > 0 ? rs_tiles(n_edges) : (int64_t)0);
+    HIP_TRY(hipGetLastError());
+    return BPT_OK;
+}
+
 }  // namespace
 
 extern "C" {
+
+int bpt_build_wait(void *stream) {
+    HIP_TRY(hipStreamSynchronize((hipStream_t)stream));
+    return BPT_OK;
+}
 
 int bpt_graph_count_device(int kind, int64_t length, int triu, int64_t a, int64_t b, int32_t *offsets, void *workspace,
                            int64_t workspace_bytes, void *stream) {
@@ -828,10 +1137,9 @@ int bpt_csr_device_bounds(int64_t n_edges, int64_t n_nodes, int32_t chunk_size, 
     if (!bounds) return BPT_ERR_NULL;
     if (n_edges < 0 || n_nodes < 0 || n_edges >= INT32_MAX || n_nodes >= INT32_MAX) return BPT_ERR_SIZE;
     if (chunk_size < 1) return BPT_ERR_SHAPE;
-    size_t tmp = 0;
-    HIP_TRY(csr_temp_bytes(n_edges, n_nodes, &tmp));
     Bump dry{nullptr, 0};
-    csr_layout(dry, n_edges, n_nodes, tmp);
+    CsrSides g;
+    csr_layout(dry, n_edges, n_nodes, 2, g);
     const int64_t by_rows = n_nodes + n_edges / chunk_size;
     bounds[0] = by_rows < n_edges ? by_rows : n_edges;
     bounds[1] = (int64_t)dry.off + 256;
@@ -841,31 +1149,22 @@ int bpt_csr_device_bounds(int64_t n_edges, int64_t n_nodes, int32_t chunk_size, 
 int bpt_csr_build_device(const int64_t *rows, const int64_t *cols, int64_t n_edges, int64_t n_nodes, int32_t chunk_size,
                          int64_t *indptr, int64_t *indices, int64_t *eid, int64_t *unit_row, int64_t *unit_ptr, int32_t *info,
                          void *workspace, int64_t workspace_bytes, void *stream) {
-    int64_t bounds[2];
-    const int st = bpt_csr_device_bounds(n_edges, n_nodes, chunk_size, bounds);
-    if (st != BPT_OK) return st;
-    if (!indptr || !unit_ptr || !info || !workspace) return BPT_ERR_NULL;
-    if (n_edges > 0 && (!rows || !cols || !indices || !eid || !unit_row)) return BPT_ERR_NULL;
-    if (workspace_bytes < bounds[1]) return BPT_ERR_WORKSPACE;
-    hipStream_t s = (hipStream_t)stream;
-    size_t tmp = 0;
-    HIP_TRY(csr_temp_bytes(n_edges, n_nodes, &tmp));
-    Bump bump{(char *)workspace, 0};
-    CsrWs w = csr_layout(bump, n_edges, n_nodes, tmp);
-    LAUNCH(k_fill_i32, 16, info, 16, 0);
-    size_t tb;
-    if (n_edges > 0) {
-        LAUNCH(k_csr_keys, n_edges, rows, cols, n_edges, n_nodes, info, w.key, w.val);
-        tb = tmp;
-        HIP_TRY(sort_pairs<uint32_t>(w.tmp, tb, w.key, w.key_s, w.val, w.val_s, n_edges, 32, s));
-        LAUNCH(k_csr_slots, n_edges, cols, w.val_s, n_edges, info, indices, eid);
+    CsrSides g{};
+    g.side[0] = CsrSide{rows, cols, indptr, indices, eid, unit_row, unit_ptr, info, nullptr, nullptr, nullptr, nullptr};
+    return csr_build(g, 1, n_edges, n_nodes, chunk_size, workspace, workspace_bytes, (hipStream_t)stream);
+}
+
+int bpt_build_csrs_device(const int64_t *src, const int64_t *dst, int64_t n_edges, int64_t n_nodes, int32_t chunk_size,
+                          int64_t *const out_side[5], int64_t *const in_side[5], int32_t *info, void *workspace,
+                          int64_t workspace_bytes, void *stream) {
+    if (!out_side || !in_side || !info) return BPT_ERR_NULL;
+    CsrSides g{};
+    for (int i = 0; i < 2; ++i) {
+        int64_t *const *o = i == 0 ? out_side : in_side;
+        g.side[i] = CsrSide{i == 0 ? src : dst, i == 0 ? dst : src, o[0], o[1], o[2], o[3], o[4], info + 2 * i,
+                            nullptr, nullptr, nullptr, nullptr};
     }
-    LAUNCH(k_csr_indptr, n_nodes + 1, w.key_s, n_edges, n_nodes, chunk_size, info, indptr, w.lo_of, w.n_units_of);
-    LAUNCH(k_csr_unit_counts, n_nodes + 1, w.lo_of, n_nodes, chunk_size, info, w.n_units_of);
-    tb = tmp;
-    HIP_TRY(scan_i32(w.tmp, tb, w.n_units_of, w.unit_base, n_nodes + 1, s));
-    LAUNCH(k_csr_units, n_nodes + 1, w.lo_of, w.unit_base, n_nodes, n_edges, chunk_size, info, unit_row, unit_ptr);
-    return BPT_OK;
+    return csr_build(g, 2, n_edges, n_nodes, chunk_size, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 int bpt_plan_device_bounds(int64_t n_units, int64_t n_edges, int64_t n_rows, int32_t seg_len, int32_t R, int64_t bounds[4]) {

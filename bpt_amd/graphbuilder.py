@@ -280,8 +280,8 @@ def nli_inter_graph_edges(premise_graphs, hypo_graphs):
 
 def get_csrs_device(src, dst, n_nodes, chunk_size=32):
     """get_csrs for an edge list that already lives on the GPU (int64 CUDA tensors): the same 6-tuple, built there by
-    libbptplan (bpt_csr_build_device: a stable radix sort by row, binary searches, a prefix sum) and bit for bit what
-    get_csrs returns for the same edges.  One synchronisation (the number of units of each side comes back)."""
+    libbptplan (bpt_build_csrs_device: a stable radix sort by row of both sides at once, binary searches, a prefix sum) and
+    bit for bit what get_csrs returns for the same edges.  One synchronisation (the number of units of each side comes back)."""
     import torch
     from ._lib import plan_lib
     if not (src.is_cuda and dst.is_cuda and src.dtype == torch.int64 and dst.dtype == torch.int64):
@@ -294,30 +294,26 @@ def get_csrs_device(src, dst, n_nodes, chunk_size=32):
     st = lib.bpt_csr_device_bounds(E, n, int(chunk_size), ctypes.byref(b))
     if st != 0:
         raise RuntimeError(f"bpt_csr_device_bounds: status {st}")
-    i64 = lambda k: torch.empty(max(k, 1), dtype=torch.int64, device=dev)
-    sides = []
+    max_units = int(b[0])
     with torch.cuda.device(dev):
         stream = torch.cuda.current_stream().cuda_stream
-        for rows, cols in ((src, dst), (dst, src)):
-            indptr, indices, eid = i64(n + 1), i64(E), i64(E)
-            unit_row, unit_ptr = i64(int(b[0])), i64(int(b[0]) + 1)
-            info = torch.empty(16, dtype=torch.int32, device=dev)
-            ws = torch.empty(int(b[1]), dtype=torch.uint8, device=dev)
-            st = lib.bpt_csr_build_device(rows.data_ptr() if E else None, cols.data_ptr() if E else None, E, n,
-                                          int(chunk_size), indptr.data_ptr(), indices.data_ptr(), eid.data_ptr(),
-                                          unit_row.data_ptr(), unit_ptr.data_ptr(), info.data_ptr(), ws.data_ptr(),
-                                          ws.numel(), stream)
-            if st != 0:
-                raise RuntimeError(f"bpt_csr_build_device: status {st}")
-            sides.append((indptr, indices[:E], eid[:E], unit_row, unit_ptr, info))
-    out = []
-    for indptr, indices, eid, unit_row, unit_ptr, info in sides:
-        err, n_units = info[:2].tolist()
-        if err:
-            raise ValueError("bptplan: row id, column id or edge id out of range")
-        out.append(((indptr, indices, eid), unit_row[:n_units].clone(), unit_ptr[:n_units + 1].clone()))
-    (out_csr, ROW, INDPTR_R), (in_csr, COL, INDPTR_C) = out
-    return out_csr, in_csr, ROW, INDPTR_R, COL, INDPTR_C
+        sides = [tuple(torch.empty(max(k, 1), dtype=torch.int64, device=dev) for k in (n + 1, E, E, max_units, max_units + 1))
+                 for _ in range(2)]
+        ptrs = [(ctypes.c_void_p * 5)(*(t.data_ptr() for t in side)) for side in sides]
+        ws = torch.empty(int(b[1]), dtype=torch.uint8, device=dev)
+        info = torch.empty(4, dtype=torch.int32, pin_memory=True)         # (written by the last kernel: no copy to wait for)
+        st = lib.bpt_build_csrs_device(src.data_ptr() if E else None, dst.data_ptr() if E else None, E, n, int(chunk_size),
+                                           ctypes.byref(ptrs[0]), ctypes.byref(ptrs[1]), info.data_ptr(), ws.data_ptr(), ws.numel(), stream)
+        if st != 0:
+            raise RuntimeError(f"bpt_build_csrs_device: status {st}")
+        st = lib.bpt_build_wait(stream)
+        if st != 0:
+            raise RuntimeError(f"bpt_build_wait: status {st}")
+    err_out, n_out, err_in, n_in = info.tolist()
+    if err_out or err_in:
+        raise ValueError("bptplan: row id, column id or edge id out of range")
+    (p_out, x_out, e_out, row, row_ptr), (p_in, x_in, e_in, col, col_ptr) = sides
+    return ((p_out, x_out[:E], e_out[:E]), (p_in, x_in[:E], e_in[:E]), row[:n_out], row_ptr[:n_out + 1], col[:n_in], col_ptr[:n_in + 1])
 
 
 def merge_graphs(graphs):

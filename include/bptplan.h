@@ -4,7 +4,7 @@
  * builds on the host for every batch and copies to the device (graph/base.py:84-86).  The kernels of bptattn.h
  * read a `bpt_plan` instead.  include/bptgraph.h derives that plan on the host (one device-to-host copy of the
  * index arrays per new graph plus tens of milliseconds of host work); the functions here derive an equivalent plan
- * from the same device arrays without leaving the GPU: sorts and prefix sums (rocPRIM) plus small kernels, all on
+ * from the same device arrays without leaving the GPU: sorts and prefix sums plus small kernels, all on
  * the caller's stream (a hipStream_t passed as void*, NULL = the default stream).  Nothing is allocated: outputs and the workspace are the caller's, sized by the bounds below.
  * The only host <-> device traffic is the caller's own read of the 16-int `info` blocks afterwards (they hold the
  * actual sizes and the validation result).  No counterpart in the reference.
