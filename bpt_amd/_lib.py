@@ -93,6 +93,13 @@ BUILD_API = {
     "bpt_build_csrs_device": (ctypes.c_int, [c_vp, c_vp, c_i64, c_i64, c_i32, ctypes.POINTER(c_vp * 5), ctypes.POINTER(c_vp * 5), c_vp,
                                              c_vp, c_i64, c_vp]),
     "bpt_build_wait": (ctypes.c_int, [c_vp]),
+    "bpt_build_plan_device": (ctypes.c_int, [c_vp, c_vp, c_i64, c_vp, c_vp, c_i64, c_i64, c_i64, c_i32,
+                                             c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp]),
+    "bpt_build_groups_bounds": (ctypes.c_int, [c_i64, c_i64, c_i64, c_i32, c_i32, ctypes.POINTER(c_i64 * 1)]),
+    "bpt_build_groups_count": (ctypes.c_int, [c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_i64, c_i64, c_i32, c_i32, c_i32, c_vp, c_vp, c_i64, c_vp]),
+    "bpt_build_groups_write": (ctypes.c_int, [c_vp, c_vp, c_i64, c_i64, c_i64, c_i32, c_i32, ctypes.POINTER(c_i32 * 16), c_i32,
+                                              c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp]),
+    "bpt_build_pair_numbers": (ctypes.c_int, [c_vp, c_vp, c_i64, c_i64, c_vp, c_vp, c_vp]),
 }
 
 _graph = None

@@ -14,6 +14,7 @@
 #include <rocprim/rocprim.hpp>
 
 #include <cstdint>
+#include <type_traits>
 
 #include "../../include/bptattn.h"
 #include "../../include/bptbuild.h"
@@ -90,13 +91,14 @@ __global__ void k_iota_i32(int32_t *p, int64_t n) {
 // ---- stable radix sort --------------------------------------------------------------------------------------------------
 // A graph's sorts are small (10^4 .. 10^6 records, keys below the number of nodes), and there the library sort runs some twenty
 // merge launches of 5 us each whatever the key width.  Here a sort is two or three least-significant-digit passes of at most 9
-// bits (up to 18 key bits: two), each three launches: digit counts per tile of 2048 records, prefix over the tiles, stable
+// bits (up to 18 key bits: two), each three launches: digit counts per tile of records, prefix over the tiles, stable
 // scatter; both CSR sides share the launches (blockIdx.y).  What bounds a pass at these sizes is the launches' latency
 // (4-10 us each), then the scatter's uncoalesced stores (576 k edges x 2 sides: 24 us with the 16-byte slots of the last pass).
 // Both CSR sides of an edge list, call to call with the read-back: 33 765 nodes / 576 k edges 398 -> 159 us, 65 535 / 3.3 M
 // 626 -> 420 us, 1 023 / 17 k 187 -> 113 us (host-bound).
-constexpr int RS_KPT = 8;                         // records per thread
-constexpr int RS_TILE = TPB * RS_KPT;
+// Records per thread of a tile: eight, or three for at most RS_FEW records, which then still give a tile to many CUs; the scatter
+// then sums up the tiles' counts itself (at most 86 of them) instead of waiting for a third launch.
+constexpr int RS_FEW = 1 << 16, RS_KPT_FEW = 3;
 constexpr int RS_MAX_BITS = 9;
 constexpr int RS_BINS = 1 << RS_MAX_BITS;
 constexpr int RS_PREFIX_TPB = 1024;
@@ -109,11 +111,12 @@ inline RsPasses rs_passes(uint64_t max_key) {
     const unsigned b = bits_for(max_key);
     RsPasses p;
     p.n = (int)((b + RS_MAX_BITS - 1) / RS_MAX_BITS);
-    p.bits = (int)((b + p.n - 1) / p.n);
+    p.bits = (int)((b + p.n - 1) / p.n);          // (one bit at least: the bins are taken in pairs)
     return p;
 }
 
-inline int64_t rs_tiles(int64_t n) { return (n + RS_TILE - 1) / RS_TILE; }
+inline int rs_per_thread(int64_t n) { return n <= RS_FEW ? RS_KPT_FEW : 8; }
+inline int64_t rs_tiles(int64_t n) { return (n + TPB * rs_per_thread(n) - 1) / (TPB * rs_per_thread(n)); }
 
 // orders a wavefront's LDS accesses across its lanes: what one lane wrote is what another reads next
 __device__ __forceinline__ void wave_lds_order() {
@@ -143,13 +146,13 @@ template <int NW> __device__ __forceinline__ int32_t block_excl_sum(int32_t v, i
 }
 
 // counts[side][tile][bin]: how many records of the tile have the digit
-template <class Recs>
+template <int RS_KPT, class Recs>
 __global__ __launch_bounds__(TPB) void k_rs_count(Recs recs, int64_t n, int shift, int bits, int32_t *counts) {
     __shared__ int32_t h[RS_BINS];
     const int bins = 1 << bits, side = blockIdx.y;
     for (int b = threadIdx.x; b < bins; b += TPB) h[b] = 0;
     __syncthreads();
-    const int64_t i0 = (int64_t)blockIdx.x * RS_TILE;
+    const int64_t i0 = (int64_t)blockIdx.x * (TPB * RS_KPT);
     bool bad = false;
     for (int r = 0; r < RS_KPT; ++r) {
         const int64_t i = i0 + r * TPB + threadIdx.x;
@@ -169,26 +172,27 @@ __global__ __launch_bounds__(TPB) void k_rs_count(Recs recs, int64_t n, int shif
 }
 
 // in place: counts[side][tile][bin] -> the records with that digit in the tiles before; totals[side][bin]: in all tiles.
-// A block owns 64 bins (one per lane), its 16 wavefronts share the tiles.
+// A block owns 16 bins, 64 threads share the tiles of each.
+constexpr int RS_PREFIX_BINS = 16, RS_PREFIX_PARTS = RS_PREFIX_TPB / RS_PREFIX_BINS;
 __global__ __launch_bounds__(RS_PREFIX_TPB) void k_rs_prefix(int32_t *counts, int32_t *totals, int64_t n_tiles, int bins) {
-    __shared__ int32_t part[RS_PREFIX_TPB / 64][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = RS_PREFIX_TPB / 64;
-    const int bin = blockIdx.x * 64 + lane, side = blockIdx.y;
-    const int64_t per = (n_tiles + n_waves - 1) / n_waves, t0 = wave * per, t1 = t0 + per < n_tiles ? t0 + per : n_tiles;
+    __shared__ int32_t part[RS_PREFIX_PARTS][RS_PREFIX_BINS];
+    const int lane = threadIdx.x % RS_PREFIX_BINS, mine = threadIdx.x / RS_PREFIX_BINS;
+    const int bin = blockIdx.x * RS_PREFIX_BINS + lane, side = blockIdx.y;
+    const int64_t per = (n_tiles + RS_PREFIX_PARTS - 1) / RS_PREFIX_PARTS, t0 = mine * per, t1 = t0 + per < n_tiles ? t0 + per : n_tiles;
     int32_t *c = counts + (int64_t)side * n_tiles * bins + bin;
     const bool on = bin < bins;
     int32_t sum = 0;
     if (on)
         for (int64_t t = t0; t < t1; ++t) sum += c[t * bins];
-    part[wave][lane] = sum;
+    part[mine][lane] = sum;
     __syncthreads();
     int32_t run = 0, all = 0;
-    for (int w = 0; w < n_waves; ++w) {
-        run += w < wave ? part[w][lane] : 0;
+    for (int w = 0; w < RS_PREFIX_PARTS; ++w) {
+        run += w < mine ? part[w][lane] : 0;
         all += part[w][lane];
     }
     if (!on) return;
-    if (wave == 0) totals[side * bins + bin] = all;
+    if (mine == 0) totals[side * bins + bin] = all;
     for (int64_t t = t0; t < t1; t += 8) {            // (eight loads in flight: the stores in between would serialise them)
         int32_t v[8];
 #pragma unroll
@@ -203,7 +207,8 @@ __global__ __launch_bounds__(RS_PREFIX_TPB) void k_rs_prefix(int32_t *counts, in
 
 // Stable scatter of a tile: a wavefront ranks 64 records at a time among its lanes with the same digit (one ballot per digit bit)
 // on top of its running counts in LDS.
-template <class Recs, class Out>
+// SUM: the tile sums up the counts itself (few tiles), else k_rs_prefix has.
+template <int RS_KPT, bool SUM, class Recs, class Out>
 __global__ __launch_bounds__(TPB) void k_rs_scatter(Recs recs, Out out, int64_t n, int shift, int bits, const int32_t *counts,
                                                     const int32_t *totals) {
     constexpr int NW = TPB / 64;
@@ -213,7 +218,7 @@ __global__ __launch_bounds__(TPB) void k_rs_scatter(Recs recs, Out out, int64_t 
     for (int b = threadIdx.x; b < bins; b += TPB)
         for (int w = 0; w < NW; ++w) wh[w][b] = 0;
     __syncthreads();
-    const int64_t i0 = (int64_t)blockIdx.x * RS_TILE + wave * (64 * RS_KPT) + lane;
+    const int64_t i0 = (int64_t)blockIdx.x * (TPB * RS_KPT) + wave * (64 * RS_KPT) + lane;
     const uint64_t below = (uint64_t(1) << lane) - 1;
     uint32_t key[RS_KPT];
     int32_t rank[RS_KPT];
@@ -239,11 +244,25 @@ __global__ __launch_bounds__(TPB) void k_rs_scatter(Recs recs, Out out, int64_t 
     // where the tile's records of every digit start: two bins a thread
     int32_t tot[2] = {0, 0}, pre[2] = {0, 0}, all;
     const int b0 = 2 * threadIdx.x;
-    for (int t = 0; t < 2; ++t)
-        if (b0 + t < bins) {
-            tot[t] = totals[side * bins + b0 + t];
-            pre[t] = counts[((int64_t)side * gridDim.x + blockIdx.x) * bins + b0 + t];
+    if (SUM) {
+        if (b0 < bins) {
+            const int2 *c = reinterpret_cast<const int2 *>(counts + (int64_t)side * gridDim.x * bins + b0);
+#pragma unroll 8
+            for (unsigned t = 0; t < gridDim.x; ++t) {
+                const int2 v = c[(int64_t)t * (bins / 2)];
+                tot[0] += v.x;
+                tot[1] += v.y;
+                pre[0] += t < blockIdx.x ? v.x : 0;
+                pre[1] += t < blockIdx.x ? v.y : 0;
+            }
         }
+    } else {
+        for (int t = 0; t < 2; ++t)
+            if (b0 + t < bins) {
+                tot[t] = totals[side * bins + b0 + t];
+                pre[t] = counts[((int64_t)side * gridDim.x + blockIdx.x) * bins + b0 + t];
+            }
+    }
     int32_t start = block_excl_sum<NW>(tot[0] + tot[1], sh, all);
     for (int t = 0; t < 2; ++t) {
         if (b0 + t < bins) {
@@ -282,33 +301,40 @@ struct RsToArrays {
 };
 
 // ---- base plan ---------------------------------------------------------------------------------------------------------
+// Five launches and the sort: clear; narrow the indices, check the units, find the rows; emit the items; their smallest and
+// largest neighbour; sort by the smallest.
+constexpr int ITEM_ROWS = TPB - 1;    // rows of a block of the first two kernels (one thread more: the end of the last row)
+
 struct BaseWs {
-    int32_t *c_items, *c_heavy, *c_slots, *b_items, *b_heavy, *b_slots, *seen, *items_tmp, *iota, *perm;
-    uint32_t *key, *key_s;
-    void *tmp;
+    int32_t *seen;
+    int4 *totals;                     // per block of ITEM_ROWS rows: items, heavy rows, slots, largest degree
+    int4 *items_tmp;                  // in row order
+    int2 *bounds_tmp;
+    uint32_t *key[2];
+    int32_t *val[2];
+    int32_t *counts, *bin_totals;
 };
 
-BaseWs base_layout(Bump &b, int64_t n_rows, int64_t n_edges, int64_t max_items, size_t tmp_bytes) {
+inline int64_t item_row_blocks(int64_t n_rows) { return (n_rows + ITEM_ROWS) / ITEM_ROWS; }
+
+BaseWs base_layout(Bump &b, int64_t n_rows, int64_t n_edges, int64_t max_items) {
     BaseWs w;
-    w.c_items = b.take<int32_t>(n_rows + 1);
-    w.c_heavy = b.take<int32_t>(n_rows + 1);
-    w.c_slots = b.take<int32_t>(n_rows + 1);
-    w.b_items = b.take<int32_t>(n_rows + 1);
-    w.b_heavy = b.take<int32_t>(n_rows + 1);
-    w.b_slots = b.take<int32_t>(n_rows + 1);
     w.seen = b.take<int32_t>(n_edges);
-    w.items_tmp = b.take<int32_t>(4 * max_items);
-    w.iota = b.take<int32_t>(max_items);
-    w.perm = b.take<int32_t>(max_items);
-    w.key = b.take<uint32_t>(max_items);
-    w.key_s = b.take<uint32_t>(max_items);
-    w.tmp = b.take<char>((int64_t)tmp_bytes);
+    w.totals = b.take<int4>(item_row_blocks(n_rows));
+    w.items_tmp = b.take<int4>(max_items);
+    w.bounds_tmp = b.take<int2>(max_items);
+    for (int i = 0; i < 2; ++i) {
+        w.key[i] = b.take<uint32_t>(max_items);
+        w.val[i] = b.take<int32_t>(max_items);
+    }
+    w.counts = b.take<int32_t>(rs_tiles(max_items) * RS_BINS);
+    w.bin_totals = b.take<int32_t>(RS_BINS);
     return w;
 }
 
-__global__ void k_base_init(int32_t *info, const int64_t *ipu, int64_t n_units, int64_t n_edges) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    for (int i = 0; i < 16; ++i) info[i] = 0;
+__global__ void k_plan_clear(int32_t *info, const int64_t *ipu, int64_t n_units, int64_t n_edges) {
+    if (threadIdx.x != 0) return;
+    for (int t = 0; t < 16; ++t) info[t] = 0;
     int err = 0;
     bool covers = (n_edges == 0);
     if (n_units > 0) {
@@ -321,90 +347,190 @@ __global__ void k_base_init(int32_t *info, const int64_t *ipu, int64_t n_units, 
     info[BPT_PI_FLAGS] = covers ? 1 : 0;
 }
 
-__global__ void k_check_units(const int64_t *row, const int64_t *ipu, int64_t n_units, int64_t n_rows, int32_t *info) {
-    const int64_t u = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (u >= n_units) return;
-    int err = 0;
-    if (row[u] < 0 || row[u] >= n_rows) err = 1;
-    if (u > 0 && row[u] < row[u - 1]) err = err > 2 ? err : 2;
-    if (ipu[u + 1] < ipu[u]) err = err > 2 ? err : 2;
-    if (err) atomicMax(&info[BPT_PI_ERR], err);
-}
-
-// rowptr[r] = start of the first unit whose row is >= r (rows without a unit are empty)
-__global__ void k_rowptr(const int64_t *row, const int64_t *ipu, int64_t n_units, int64_t n_rows, const int32_t *info,
-                         int32_t *rowptr) {
-    const int64_t r = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (r > n_rows || info[BPT_PI_ERR]) return;
-    int64_t lo = 0, hi = n_units;
-    while (lo < hi) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (row[mid] < r) lo = mid + 1; else hi = mid;
-    }
-    rowptr[r] = n_units > 0 ? (int32_t)ipu[lo] : 0;
-}
-
-__global__ void k_row_counts(const int32_t *rowptr, int64_t n_rows, int32_t seg_len, int32_t *info, int32_t *c_items,
-                             int32_t *c_heavy, int32_t *c_slots) {
-    const int64_t r = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (r > n_rows || info[BPT_PI_ERR]) return;
-    int32_t ni = 0, nh = 0, ns = 0;
-    if (r < n_rows) {
-        const int32_t deg = rowptr[r + 1] - rowptr[r];
-        ni = 1;
-        if (deg > seg_len) {
-            nh = 1;
-            ni = ns = (deg + seg_len - 1) / seg_len;
+// Three kinds of blocks: edge slots (indices to 32 bits, eid a permutation?), units (sorted?), rows (rowptr[r] = start of the
+// first unit whose row is >= r, and what the block's rows give).  Malformed arrays set info[BPT_PI_ERR]; what the row blocks
+// then wrote is not used.
+__global__ __launch_bounds__(TPB) void k_plan_narrow(const int64_t *row, const int64_t *ipu, int64_t n_units, const int64_t *eid,
+                                                     const int64_t *indices, int64_t n_edges, int64_t n_rows, int64_t n_index_nodes,
+                                                     int32_t seg_len, unsigned edge_blocks, unsigned unit_blocks, int32_t *info,
+                                                     int32_t *idx32, int32_t *eid32, int32_t *seen, int32_t *rowptr, int4 *totals) {
+    if (blockIdx.x < edge_blocks) {
+        const int64_t p = (int64_t)blockIdx.x * TPB + threadIdx.x;
+        if (p >= n_edges) return;
+        const int64_t e = eid[p], c = indices ? indices[p] : 0;
+        if (e < 0 || e >= n_edges || c < 0 || (indices && c >= n_index_nodes)) {
+            atomicMax(&info[BPT_PI_ERR], 1);
+            eid32[p] = 0;
+            idx32[p] = 0;
+            return;
         }
-        atomicMax(&info[BPT_PI_MAX_DEGREE], deg);
+        eid32[p] = (int32_t)e;
+        idx32[p] = (int32_t)c;
+        seen[e] = (int32_t)p;                          // (checked by k_plan_items' edge blocks: every slot finds itself there)
+        return;
     }
-    c_items[r] = ni;
-    c_heavy[r] = nh;
-    c_slots[r] = ns;
+    if (blockIdx.x < edge_blocks + unit_blocks) {
+        const int64_t u = (int64_t)(blockIdx.x - edge_blocks) * TPB + threadIdx.x;
+        if (u >= n_units) return;
+        int err = 0;
+        if (row[u] < 0 || row[u] >= n_rows) err = 1;
+        if (u > 0 && row[u] < row[u - 1]) err = err > 2 ? err : 2;
+        if (ipu[u + 1] < ipu[u]) err = err > 2 ? err : 2;
+        if (err) atomicMax(&info[BPT_PI_ERR], err);
+        return;
+    }
+    __shared__ int32_t start[TPB];
+    __shared__ int32_t sh[TPB / 64 + 1];
+    const unsigned blk = blockIdx.x - edge_blocks - unit_blocks;
+    const int64_t r = (int64_t)blk * ITEM_ROWS + threadIdx.x;
+    int32_t at = 0;
+    if (r <= n_rows && n_units > 0) {
+        int64_t lo = 0, hi = n_units;
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) >> 1;
+            if (row[mid] < r) lo = mid + 1; else hi = mid;
+        }
+        at = (int32_t)ipu[lo];
+    }
+    if (r <= n_rows) rowptr[r] = at;
+    start[threadIdx.x] = at;
+    __syncthreads();
+    int32_t deg = 0, n_seg = 0;
+    const bool mine = threadIdx.x < ITEM_ROWS && r < n_rows;
+    if (mine) {
+        deg = max(start[threadIdx.x + 1] - at, 0);
+        n_seg = deg > seg_len ? (deg - 1) / seg_len + 1 : 0;
+    }
+    int32_t items, heavy, slots;
+    block_excl_sum<TPB / 64>(mine ? max(n_seg, 1) : 0, sh, items);
+    block_excl_sum<TPB / 64>(n_seg > 0 ? 1 : 0, sh, heavy);
+    block_excl_sum<TPB / 64>(n_seg, sh, slots);
+    for (int d = 32; d > 0; d >>= 1) deg = max(deg, __shfl_xor(deg, d));
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = deg;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < TPB / 64; ++w) deg = max(deg, sh[w]);
+        totals[blk] = make_int4(items, heavy, slots, deg);
+    }
 }
 
-__global__ void k_emit_items(const int32_t *rowptr, int64_t n_rows, int32_t seg_len, const int32_t *b_items,
-                             const int32_t *b_heavy, const int32_t *b_slots, int32_t *info, int32_t *items, int32_t *heavy) {
-    const int64_t r = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (r > n_rows || info[BPT_PI_ERR]) return;
-    if (r == n_rows) {
-        info[BPT_PI_N_ITEMS] = b_items[n_rows];
-        info[BPT_PI_N_HEAVY] = b_heavy[n_rows];
-        info[BPT_PI_N_SLOTS] = b_slots[n_rows];
+// items of every row in row order, the heavy rows, the counts; a row of more than ITEM_FEW segments is written by the whole
+// block.  The blocks behind those of the rows finish the check that eid is a permutation: two slots of one edge left one
+// number in `seen`, and the other slot does not find itself (plain stores and loads: the two kernels 20 us for 576 k edges,
+// with a counter per edge and its clearing 27).
+constexpr int ITEM_FEW = 8;
+__global__ __launch_bounds__(TPB) void k_plan_items(const int32_t *rowptr, int64_t n_rows, int32_t seg_len, const int4 *totals,
+                                                    const int32_t *eid32, const int32_t *seen, int64_t n_edges, unsigned row_blocks,
+                                                    int32_t *info, int4 *items, int32_t *heavy) {
+    __shared__ int32_t sh[TPB / 64 + 1];
+    __shared__ int32_t many[TPB][3];                   // row, first item, first slot
+    __shared__ int32_t n_many;
+    if (info[BPT_PI_ERR]) return;
+    if (blockIdx.x >= row_blocks) {
+        const int64_t p = (int64_t)(blockIdx.x - row_blocks) * TPB + threadIdx.x;
+        if (p < n_edges && seen[eid32[p]] != (int32_t)p) atomicAnd(&info[BPT_PI_FLAGS], ~1);
         return;
     }
-    const int32_t begin = rowptr[r], end = rowptr[r + 1], deg = end - begin;
-    int4 *out = reinterpret_cast<int4 *>(items) + b_items[r];
-    if (deg <= seg_len) {
-        *out = make_int4((int32_t)r, begin, end, -1);
-        return;
+    if (threadIdx.x == 0) n_many = 0;
+    const bool last = blockIdx.x == row_blocks - 1;
+    int4 part = make_int4(0, 0, 0, 0);
+    for (unsigned b = threadIdx.x; b < blockIdx.x; b += TPB) {
+        const int4 t = totals[b];
+        part.x += t.x; part.y += t.y; part.z += t.z;
+        part.w = max(part.w, t.w);
     }
-    const int32_t n_seg = (deg + seg_len - 1) / seg_len, s0 = b_slots[r];
-    int32_t *hv = heavy + 3 * (int64_t)b_heavy[r];
-    hv[0] = (int32_t)r;
-    hv[1] = s0;
-    hv[2] = n_seg;
-    for (int32_t s = 0; s < n_seg; ++s) {
-        const int32_t b = begin + s * seg_len;
-        out[s] = make_int4((int32_t)r, b, min(end, b + seg_len), s0 + s);
+    int4 before;
+    block_excl_sum<TPB / 64>(part.x, sh, before.x);
+    block_excl_sum<TPB / 64>(part.y, sh, before.y);
+    block_excl_sum<TPB / 64>(part.z, sh, before.z);
+    if (last) atomicMax(&info[BPT_PI_MAX_DEGREE], threadIdx.x == 0 ? max(part.w, totals[blockIdx.x].w) : part.w);
+    const int64_t r = (int64_t)blockIdx.x * ITEM_ROWS + threadIdx.x;
+    const bool mine = threadIdx.x < ITEM_ROWS && r < n_rows;
+    const int32_t begin = mine ? rowptr[r] : 0, end = mine ? rowptr[r + 1] : 0, deg = end - begin;
+    const int32_t n_seg = deg > seg_len ? (deg - 1) / seg_len + 1 : 0;
+    int32_t n_items, n_heavy, n_slots;
+    const int32_t item = before.x + block_excl_sum<TPB / 64>(mine ? max(n_seg, 1) : 0, sh, n_items);
+    const int32_t hv = before.y + block_excl_sum<TPB / 64>(n_seg > 0 ? 1 : 0, sh, n_heavy);
+    const int32_t slot = before.z + block_excl_sum<TPB / 64>(n_seg, sh, n_slots);
+    if (mine && n_seg == 0) items[item] = make_int4((int32_t)r, begin, end, -1);
+    if (n_seg > 0) {
+        heavy[3 * (int64_t)hv] = (int32_t)r;
+        heavy[3 * (int64_t)hv + 1] = slot;
+        heavy[3 * (int64_t)hv + 2] = n_seg;
+        if (n_seg <= ITEM_FEW) {
+            for (int32_t t = 0; t < n_seg; ++t)
+                items[item + t] = make_int4((int32_t)r, begin + t * seg_len, min(end, begin + (t + 1) * seg_len), slot + t);
+        } else {
+            const int i = atomicAdd(&n_many, 1);
+            many[i][0] = (int32_t)r;
+            many[i][1] = item;
+            many[i][2] = slot;
+        }
+    }
+    __syncthreads();
+    for (int i = 0; i < n_many; ++i) {
+        const int32_t row = many[i][0], b = rowptr[row], e = rowptr[row + 1], n = (e - b - 1) / seg_len + 1;
+        for (int32_t t = threadIdx.x; t < n; t += TPB)
+            items[many[i][1] + t] = make_int4(row, b + t * seg_len, min(e, b + (t + 1) * seg_len), many[i][2] + t);
+    }
+    if (last && threadIdx.x == 0) {
+        info[BPT_PI_N_ITEMS] = before.x + n_items;
+        info[BPT_PI_N_HEAVY] = before.y + n_heavy;
+        info[BPT_PI_N_SLOTS] = before.z + n_slots;
     }
 }
 
-__global__ void k_narrow(const int64_t *eid, const int64_t *indices, int64_t n_edges, int64_t n_index_nodes, int32_t *info,
-                         int32_t *idx32, int32_t *eid32, int32_t *seen) {
-    const int64_t p = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (p >= n_edges) return;
-    const int64_t e = eid[p], c = indices ? indices[p] : 0;
-    if (e < 0 || e >= n_edges || c < 0 || (indices && c >= n_index_nodes)) {
-        atomicMax(&info[BPT_PI_ERR], 1);
-        eid32[p] = 0;
-        idx32[p] = 0;
-        return;
+// smallest and largest neighbour id of every item, sixteen lanes an item; an empty item: its own row id clipped to
+// n_index_nodes, twice
+__global__ __launch_bounds__(TPB) void k_item_bounds(const int4 *items, const int32_t *idx32, const int32_t *info, int64_t max_items,
+                                                     int64_t n_index_nodes, int64_t n_edges, int2 *bounds) {
+    const int64_t i = (int64_t)blockIdx.x * (TPB / 16) + (threadIdx.x >> 4);
+    if (i >= max_items || info[BPT_PI_ERR] || i >= info[BPT_PI_N_ITEMS]) return;
+    const int4 it = items[i];
+    int32_t lo, hi;
+    if (it.z > it.y && it.y >= 0 && it.z <= n_edges) {          // (an item list from elsewhere is not trusted with addresses)
+        lo = INT32_MAX;
+        hi = 0;
+        for (int32_t p = it.y + (threadIdx.x & 15); p < it.z; p += 16) {
+            lo = min(lo, idx32[p]);
+            hi = max(hi, idx32[p]);
+        }
+        for (int d = 8; d > 0; d >>= 1) {
+            lo = min(lo, __shfl_xor(lo, d, 16));
+            hi = max(hi, __shfl_xor(hi, d, 16));
+        }
+    } else {
+        lo = hi = (it.x >= 0 && it.x < n_index_nodes) ? it.x : (int32_t)n_index_nodes;
     }
-    eid32[p] = (int32_t)e;
-    idx32[p] = (int32_t)c;
-    if (atomicAdd(&seen[e], 1) != 0) atomicAnd(&info[BPT_PI_FLAGS], ~1);
+    if ((threadIdx.x & 15) == 0) bounds[i] = make_int2(lo, hi);
 }
+
+// the items as sort records, by their smallest or largest neighbour; places past the last item sort behind all of them
+struct ItemRecs {
+    const int2 *bounds;
+    const int32_t *info;
+    int largest;
+    uint32_t pad;
+    __device__ uint32_t key(int, int64_t i, bool &) const {
+        if (info[BPT_PI_ERR] || i >= info[BPT_PI_N_ITEMS]) return pad;
+        return (uint32_t)(largest ? bounds[i].y : bounds[i].x);
+    }
+    __device__ int32_t val(int, int64_t i) const { return (int32_t)i; }
+    __device__ void report(int, bool) const {}
+};
+struct ItemsSorted {
+    const int4 *items_tmp;
+    const int2 *bounds_tmp;
+    const int32_t *info;
+    int4 *items;
+    int2 *bounds;
+    __device__ void put(int, int64_t at, uint32_t, int32_t i) const {
+        if (info[BPT_PI_ERR] || i >= info[BPT_PI_N_ITEMS]) return;
+        items[at] = items_tmp[i];
+        if (bounds) bounds[at] = bounds_tmp[i];
+    }
+};
 
 // Sort key of every item: smallest (LARGEST = false) or largest neighbour id; an empty item takes its own row id,
 // clipped to n_index_nodes.  Positions past n_items get the padding key, which sorts behind every real one.
@@ -424,13 +550,6 @@ __global__ void k_item_keys(const int32_t *items, const int32_t *idx32, const in
         for (int32_t p = it.y + 1; p < it.z; ++p) k = LARGEST ? max(k, idx32[p]) : min(k, idx32[p]);
     }
     key[i] = (uint32_t)k;
-}
-
-__global__ void k_gather_items(const int32_t *items_tmp, const int32_t *perm, const int32_t *info, int64_t max_items,
-                               int32_t *items) {
-    const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
-    if (i >= max_items || info[BPT_PI_ERR] || i >= info[BPT_PI_N_ITEMS]) return;
-    reinterpret_cast<int4 *>(items)[i] = reinterpret_cast<const int4 *>(items_tmp)[perm[i]];
 }
 
 // ---- row groups --------------------------------------------------------------------------------------------------------
@@ -739,6 +858,475 @@ __global__ void k_edge_ids(const uint64_t *skey, const int32_t *slot_of, const i
     pair_eid[first[u] + __popc((uint32_t)ent_mask[old] & ((1u << m) - 1u))] = e;
 }
 
+// ---- row groups, short form -------------------------------------------------------------------------------------------
+// The same groups as above for groups whose edges fit a workgroup's LDS (at most GRP_MAX_EDGES) and at most GRP_MAX_GROUPS of
+// them, which are the plans of graphs up to some 10^5 nodes.  A group's records never meet another group's, so the device-wide
+// sorts of all edges (fifty launches a side) become one workgroup per group that sorts its 200-1000 records in LDS and forms
+// the entries, their order and the pair numbers there; one workgroup then numbers the groups; after the caller has read the
+// two counts and allocated exactly, every group writes its part of the arrays.  33 765 nodes / 576 k edges, base plan and tiles of
+// one side, call to call: 868 -> 227 us (65 535 / 3.3 M: 1690 -> 384, 1 023 / 17 k: 504 -> 165, mostly launches and the waits).
+constexpr int GRP_MAX_EDGES = 4096;
+constexpr int GRP_MAX_GROUPS = 16384;
+constexpr int GRP_ORDER_TPB = 1024;
+constexpr int GRP_ORDER_LDS = 8192;   // up to so many groups are sorted in LDS, more in global memory
+
+struct GroupRec {                     // what a group is known by before the groups are numbered
+    int32_t n_entries, n_pairs, key;            // key: smallest neighbour
+};
+
+struct ShortWs {
+    uint32_t *key[2];
+    int32_t *val[2];
+    int32_t *counts, *bin_totals, *jorder;
+    GroupRec *rec;
+    int32_t *loc_group, *loc_work, *loc_prefix;       // groups in locality order
+    int32_t *order, *entry0, *pair0, *chunks;         // final order: group as formed, first entry, first pair
+    int4 *entries;                                    // parked: neighbour, mask, first pair inside the group
+    int32_t *pairs;                                   // parked: edge ids in pair order
+};
+
+ShortWs short_layout(Bump &b, int64_t max_items, int64_t max_groups, int64_t n_edges) {
+    ShortWs w;
+    for (int i = 0; i < 2; ++i) {
+        w.key[i] = b.take<uint32_t>(max_items);
+        w.val[i] = b.take<int32_t>(max_items);
+    }
+    w.counts = b.take<int32_t>(rs_tiles(max_items) * RS_BINS);
+    w.bin_totals = b.take<int32_t>(RS_BINS);
+    w.jorder = b.take<int32_t>(max_items);
+    w.rec = b.take<GroupRec>(max_groups);
+    w.loc_group = b.take<int32_t>(max_groups);
+    w.loc_work = b.take<int32_t>(max_groups);
+    w.loc_prefix = b.take<int32_t>(max_groups);
+    w.order = b.take<int32_t>(max_groups);
+    w.entry0 = b.take<int32_t>(max_groups + 1);
+    w.pair0 = b.take<int32_t>(max_groups + 1);
+    w.chunks = b.take<int32_t>(9);
+    w.entries = b.take<int4>(n_edges);
+    w.pairs = b.take<int32_t>(n_edges);
+    return w;
+}
+
+struct ItemOrder {                    // last pass of the sort by largest neighbour
+    int32_t *jorder;
+    __device__ void put(int, int64_t at, uint32_t, int32_t i) const { jorder[at] = i; }
+};
+
+// The members of a group as formed, and where its results are parked: in the edge slots of its items, which no other group has,
+// one member's slots after the other's.
+struct GroupSlots {
+    int32_t begin[16], pre[17];
+    // by 16 threads; returns the smallest neighbour of the group
+    __device__ int32_t load(const int4 *items, const int2 *bounds, const int32_t *jorder, int32_t g, int32_t R, int32_t n_items, int64_t n_edges,
+                            int32_t seg_len, int2 *member) {
+        const int t = threadIdx.x;
+        int32_t len = 0, at = 0, lo = INT32_MAX;
+        const int64_t j = (int64_t)g * R + t;
+        int2 who = make_int2(-1, -1);
+        if (t < R && j < n_items) {
+            const int32_t item = jorder[j];
+            const int4 it = items[item];
+            who = make_int2(it.x, it.w);
+            if (it.y >= 0 && it.z > it.y && it.z <= n_edges) {
+                at = it.y;
+                len = min(it.z - it.y, seg_len);
+            }
+            if (bounds) lo = bounds[item].x;
+        }
+        int32_t incl = len;
+        for (int d = 1; d < 16; d <<= 1) {
+            const int32_t y = __shfl_up(incl, d, 16);
+            if (t >= d) incl += y;
+        }
+        for (int d = 8; d > 0; d >>= 1) lo = min(lo, __shfl_xor(lo, d, 16));
+        begin[t] = at;
+        pre[t] = incl - len;
+        if (t == 15) pre[16] = incl;
+        if (member && t < R) *member = who;
+        return lo;
+    }
+    __device__ int member_of(int x) const {
+        int m = 0;
+        for (int d = 8; d > 0; d >>= 1)
+            if (m + d < 16 && pre[m + d] <= x) m += d;
+        return m;
+    }
+    __device__ int32_t slot(int x) const {
+        const int m = member_of(x);
+        return begin[m] + (x - pre[m]);
+    }
+};
+
+// value of lane (lane ^ M): DPP where a pattern of 16 lanes does it, through the LDS crossbar else
+template <int M> __device__ __forceinline__ uint32_t lane_xor(uint32_t x) {
+    auto dpp = [](uint32_t v, auto ctrl) { return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, decltype(ctrl)::value, 0xf, 0xf, true); };
+    if constexpr (M == 1) return dpp(x, std::integral_constant<int, 0xB1>());                      // quad_perm 1 0 3 2
+    else if constexpr (M == 2) return dpp(x, std::integral_constant<int, 0x4E>());                 // quad_perm 2 3 0 1
+    else if constexpr (M == 4) return dpp(dpp(x, std::integral_constant<int, 0x141>()), std::integral_constant<int, 0x1B>());   // ^7, ^3
+    else if constexpr (M == 8) return dpp(x, std::integral_constant<int, 0x128>());                // row_ror 8
+    else return (uint32_t)__shfl_xor((int)x, M);
+}
+template <int M> __device__ __forceinline__ uint64_t lane_xor(uint64_t x) {
+    return (uint64_t)lane_xor<M>((uint32_t)x) | ((uint64_t)lane_xor<M>((uint32_t)(x >> 32)) << 32);
+}
+
+// the stages of stride M and below of a bitonic merge over 128 keys held by a wavefront, lane l the keys l and 64 + l
+template <int M, typename K> __device__ __forceinline__ void merge_lanes(K &a, K &b, bool up_a, bool up_b, int lane) {
+    if constexpr (M > 0) {
+        const bool lower = (lane & M) == 0;
+        const K ya = lane_xor<M>(a), yb = lane_xor<M>(b);
+        a = ((a < ya) == (lower == up_a)) ? a : ya;
+        b = ((b < yb) == (lower == up_b)) ? b : yb;
+        merge_lanes<(M >> 1), K>(a, b, up_a, up_b, lane);
+    }
+}
+
+template <int M, typename K> __device__ __forceinline__ void sort_lanes(K &a, K &b, int lane) {        // runs of 2 M
+    if constexpr (M > 1) sort_lanes<(M >> 1), K>(a, b, lane);
+    const bool up_a = M == 32 ? true : (lane & (2 * M)) == 0, up_b = M == 32 ? false : up_a;
+    merge_lanes<M, K>(a, b, up_a, up_b, lane);
+}
+
+// Ascending bitonic sort of n keys (a power of two from 128) in LDS by NT threads: 128 keys at a time in a wavefront's registers,
+// only the strides above that through LDS.  (All stages through LDS: k_group_form 66 us for 2200 tiles, so 45, and 24 since
+// nothing of a group waits for a global counter.)
+template <int NT, typename K> __device__ __forceinline__ void lds_sort(K *key, int n) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int c = wave * 128; c < n; c += NT * 2) {
+        K a = key[c + lane], b = key[c + 64 + lane];
+        sort_lanes<32, K>(a, b, lane);
+        const bool up = (c & 128) == 0;
+        if ((a > b) == up) { const K t = a; a = b; b = t; }
+        merge_lanes<32, K>(a, b, up, up, lane);
+        key[c + lane] = a;
+        key[c + 64 + lane] = b;
+    }
+    __syncthreads();
+    for (int k = 256; k <= n; k <<= 1) {
+        for (int j = k >> 1; j >= 128; j >>= 1) {
+            for (int t = threadIdx.x; t < (n >> 1); t += NT) {
+                const int i = ((t & ~(j - 1)) << 1) | (t & (j - 1)), l = i + j;
+                const K a = key[i], b = key[l];
+                if ((a > b) == ((i & k) == 0)) {
+                    key[i] = b;
+                    key[l] = a;
+                }
+            }
+            __syncthreads();
+        }
+        for (int c = wave * 128; c < n; c += NT * 2) {
+            K a = key[c + lane], b = key[c + 64 + lane];
+            const bool up = (c & k) == 0;
+            if ((a > b) == up) { const K t = a; a = b; b = t; }
+            merge_lanes<32, K>(a, b, up, up, lane);
+            key[c + lane] = a;
+            key[c + 64 + lane] = b;
+        }
+        __syncthreads();
+    }
+}
+
+inline __device__ int pow2_at_least(int n) {
+    int p = 128;
+    while (p < n) p <<= 1;
+    return p;
+}
+
+// One group: its records (neighbour, member, place in the member's item) sorted, an entry per neighbour and repeat, the entries
+// in the order asked for, the pairs numbered.  K: 32-bit keys where neighbour, member and place fit.
+template <int CAP, typename K>
+__global__ __launch_bounds__(TPB) void k_group_form(const int4 *items, const int2 *bounds, const int32_t *jorder, const int32_t *idx32,
+                                                    const int32_t *eid32, const int32_t *pinfo, int64_t n_edges, int32_t seg_len, int32_t R,
+                                                    int place_bits, int mode, GroupRec *rec, int4 *entries, int32_t *pairs) {
+    // (16 KB for 1024 edges with 32-bit keys: ten workgroups a CU)
+    __shared__ K key[CAP];
+    __shared__ uint32_t ekey[CAP], emask2[CAP / 2];                 // emask2: two entries' masks a word
+    __shared__ uint16_t erec[CAP], rec_ent[CAP], efirst[CAP];       // erec: a record of the entry
+    uint16_t *const rec_rep = reinterpret_cast<uint16_t *>(ekey), *const rec_cnt = rec_rep + CAP;      // (ekey is not in use yet then)
+    auto mask_of = [&](int u) { return (emask2[u >> 1] >> (16 * (u & 1))) & 0xFFFFu; };
+    __shared__ GroupSlots at;
+    __shared__ int32_t sh[TPB / 64 + 1];
+    const int32_t g = blockIdx.x, tid = threadIdx.x;
+    if (g >= n_groups_of(pinfo, R)) return;
+    int32_t smallest = 0;
+    if (tid < 16) smallest = at.load(items, bounds, jorder, g, R, pinfo[BPT_PI_N_ITEMS], n_edges, seg_len, nullptr);
+    __syncthreads();
+    const int n = at.pre[16], P = pow2_at_least(n);
+    for (int t = tid; t < P; t += TPB) {
+        K k = (K)~(K)0;
+        if (t < n) {
+            const int m = at.member_of(t), place = t - at.pre[m];
+            k = ((K)(uint32_t)idx32[at.begin[m] + place] << (place_bits + 4)) | (K)((m << place_bits) | place);
+        }
+        key[t] = k;
+        if (2 * t < n + 1) emask2[t] = 0;
+    }
+    __syncthreads();
+    lds_sort<TPB, K>(key, P);
+    auto same_edge = [&](int a, int b) { return (key[a] >> place_bits) == (key[b] >> place_bits); };
+    auto same_row = [&](int a, int b) { return (key[a] >> (place_bits + 4)) == (key[b] >> (place_bits + 4)); };
+    int rep_here = 0;
+    for (int i = tid; i < n; i += TPB)
+        if (i > 0 && same_edge(i, i - 1)) rep_here = 1;
+    const bool repeats = __syncthreads_or(rep_here) != 0;        // a member holds an edge more than once (multigraphs)
+    if (repeats) {
+        for (int i = tid; i < n; i += TPB) {
+            int t = 0;
+            for (int b = i - 1; b >= 0 && same_edge(b, i); --b) ++t;
+            rec_rep[i] = (uint16_t)t;
+        }
+        __syncthreads();
+    }
+    // entries: one per record that is the first of its neighbour with its repeat number
+    int n_ent = 0;
+    for (int i0 = 0; i0 < n; i0 += TPB) {
+        const int i = i0 + tid;
+        int fresh = 0;
+        if (i < n) {
+            fresh = 1;
+            if (!repeats) {
+                if (i > 0 && same_row(i, i - 1)) fresh = 0;
+            } else {
+                for (int b = i - 1; b >= 0 && same_row(b, i); --b)
+                    if (rec_rep[b] >= rec_rep[i]) { fresh = 0; break; }
+            }
+        }
+        int32_t in_round;
+        const int cnt = n_ent + block_excl_sum<TPB / 64>(fresh, sh, in_round);
+        if (i < n) {
+            rec_cnt[i] = (uint16_t)cnt;
+            if (!repeats) rec_ent[i] = (uint16_t)(cnt + fresh - 1);
+        }
+        n_ent += in_round;
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += TPB) {
+        int u;
+        if (repeats) {
+            int h = i;
+            while (h > 0 && same_row(h - 1, i)) --h;
+            u = rec_cnt[h] + rec_rep[i];
+            rec_ent[i] = (uint16_t)u;
+        } else {
+            u = rec_ent[i];
+        }
+        erec[u] = (uint16_t)i;
+        atomicOr(&emask2[u >> 1], 1u << (16 * (u & 1) + (int)((key[i] >> place_bits) & 15)));
+    }
+    __syncthreads();
+    // their order inside the group: as they are (ascending neighbour), by member mask, by (neighbour mod 16, neighbour)
+    const int PE = pow2_at_least(n_ent);
+    auto idx_of = [&](int u) { return (int32_t)(key[erec[u]] >> (place_bits + 4)); };
+    for (int u = tid; u < PE; u += TPB)
+        ekey[u] = u >= n_ent ? PAD32 : mode == 1 ? ((0xFFFFu ^ mask_of(u)) << 16) | (uint32_t)u : mode == 2 ? ((uint32_t)(idx_of(u) & 15) << 16) | (uint32_t)u
+                                                                                                            : (uint32_t)u;
+    __syncthreads();
+    if (mode != 0) lds_sort<TPB, uint32_t>(ekey, PE);
+    int n_pairs = 0;
+    for (int p0 = 0; p0 < n_ent; p0 += TPB) {
+        const int p = p0 + tid;
+        const int u = p < n_ent ? (int)(ekey[p] & 0xFFFFu) : 0;
+        int32_t in_round;
+        const uint32_t mask = p < n_ent ? mask_of(u) : 0u;
+        const int first = n_pairs + block_excl_sum<TPB / 64>(__popc(mask), sh, in_round);
+        if (p < n_ent) {
+            efirst[u] = (uint16_t)first;
+            entries[at.slot(p)] = make_int4(idx_of(u), (int32_t)mask, first, 0);
+        }
+        n_pairs += in_round;
+    }
+    __syncthreads();
+    for (int i = tid; i < n; i += TPB) {
+        const int u = rec_ent[i], m = (int)((key[i] >> place_bits) & 15), place = (int)(key[i] & (K)((1 << place_bits) - 1));
+        pairs[at.slot(efirst[u] + __popc(mask_of(u) & ((1u << m) - 1u)))] = eid32[at.begin[m] + place];
+    }
+    if (tid == 0) rec[g] = GroupRec{n_ent, n, smallest};
+}
+
+// One stable pass over n <= GRP_MAX_GROUPS words by one workgroup, from -> to (LDS or global memory); a wavefront owns a
+// contiguous part.  (A bitonic sort of the words in LDS took 73 us for 2200 groups, four passes and the rest 28.)
+template <int NW> __device__ void block_radix_pass(const uint32_t *from, uint32_t *to, int n, int shift, int bits, int32_t (*wh)[RS_BINS], int32_t *sh) {
+    const int bins = 1 << bits, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int per = ((n + NW * 64 - 1) / (NW * 64)) * 64, w0 = wave * per, w1 = min(w0 + per, n);
+    for (int b = threadIdx.x; b < NW * RS_BINS; b += NW * 64) wh[b / RS_BINS][b % RS_BINS] = 0;
+    __syncthreads();
+    for (int i = w0 + lane; i < w1; i += 64) atomicAdd(&wh[wave][(from[i] >> shift) & (uint32_t)(bins - 1)], 1);
+    __syncthreads();
+    int32_t sum = 0, all;
+    const int bin = threadIdx.x;
+    if (bin < bins)
+        for (int w = 0; w < NW; ++w) sum += wh[w][bin];
+    int32_t at = block_excl_sum<NW>(sum, sh, all);
+    if (bin < bins)
+        for (int w = 0; w < NW; ++w) {
+            const int32_t c = wh[w][bin];
+            wh[w][bin] = at;
+            at += c;
+        }
+    __syncthreads();
+    const uint64_t below = (uint64_t(1) << lane) - 1;
+    for (int i0 = w0; i0 < w1; i0 += 64) {
+        const bool on = i0 + lane < w1;
+        const uint32_t key = on ? from[i0 + lane] : 0u;
+        const int d = (int)((key >> shift) & (uint32_t)(bins - 1));
+        uint64_t peers = __ballot(on);
+        for (int b = 0; b < bits; ++b) {
+            const bool bit = (d >> b) & 1;
+            const uint64_t m = __ballot(bit);
+            peers &= bit ? m : ~m;
+        }
+        const int32_t start = wh[wave][d];
+        wave_lds_order();
+        if (on && (peers & below) == 0) wh[wave][d] = start + __popcll(peers);
+        wave_lds_order();
+        if (on) to[start + __popcll(peers & below)] = key;
+    }
+    __syncthreads();
+}
+
+// One workgroup numbers the groups: by locality, cut into 8 ranges of equal work, by decreasing work inside a range (or not),
+// and gives every group its place in the arrays.  out_info: the plan's info block and the groups'.
+__global__ __launch_bounds__(GRP_ORDER_TPB) void k_group_order(const GroupRec *rec, const int32_t *pinfo, int32_t R, int by_work, int g_bits,
+                                                               int key_bits, int work_bits, uint32_t *word0, uint32_t *word1, int32_t *loc_group,
+                                                               int32_t *loc_work, int32_t *loc_prefix, int32_t *order, int32_t *entry0,
+                                                               int32_t *pair0, int32_t *chunks, int32_t *out_info) {
+    constexpr int NW = GRP_ORDER_TPB / 64;
+    __shared__ int32_t wh[NW][RS_BINS];
+    __shared__ uint32_t lds0[GRP_ORDER_LDS], lds1[GRP_ORDER_LDS];
+    __shared__ int32_t sh[NW + 1], cut[9];
+    const int tid = threadIdx.x, ng = n_groups_of(pinfo, R);
+    const uint32_t g_mask = (1u << g_bits) - 1u;
+    uint32_t *from = ng <= GRP_ORDER_LDS ? lds0 : word0, *to = ng <= GRP_ORDER_LDS ? lds1 : word1;
+    auto sort = [&](int bits) {                           // the words by their `bits` bits above the group's number
+        const int passes = (bits + RS_MAX_BITS - 1) / RS_MAX_BITS, step = (bits + passes - 1) / passes;
+        for (int p = 0; p < passes; ++p) {
+            block_radix_pass<NW>(from, to, ng, g_bits + p * step, min(step, bits - p * step), wh, sh);
+            uint32_t *t = from; from = to; to = t;
+        }
+    };
+    for (int g = tid; g < ng; g += GRP_ORDER_TPB) from[g] = ((uint32_t)rec[g].key << g_bits) | (uint32_t)g;
+    __syncthreads();
+    sort(key_bits);
+    int64_t total = 0;
+    for (int l0 = 0; l0 < ng; l0 += GRP_ORDER_TPB) {
+        const int l = l0 + tid;
+        int32_t work = 0, in_round;
+        if (l < ng) {
+            const int32_t g = (int32_t)(from[l] & g_mask);
+            work = R == 16 ? 4 * ((rec[g].n_entries + R - 1) / R + 1) : FIXED_WORK + rec[g].n_pairs;
+            loc_group[l] = g;
+            loc_work[l] = work;
+        }
+        const int32_t before = block_excl_sum<NW>(work, sh, in_round);
+        if (l < ng) loc_prefix[l] = (int32_t)total + before;
+        total += in_round;
+    }
+    __syncthreads();
+    // cut[x] = number of groups whose midpoint lies before x/8 of the total: the midpoints ascend, so the group that crosses says so
+    if (tid <= 8) cut[tid] = tid == 0 ? 0 : ng;
+    __syncthreads();
+    for (int l = tid; l < ng; l += GRP_ORDER_TPB) {
+        const int64_t mid = (int64_t)loc_prefix[l] + loc_work[l] / 2, prev = l > 0 ? (int64_t)loc_prefix[l - 1] + loc_work[l - 1] / 2 : -1;
+        for (int x = 1; x <= 7; ++x)
+            if (mid >= total * x / 8 && prev < total * x / 8) cut[x] = l;
+    }
+    __syncthreads();
+    if (tid <= 8) chunks[tid] = cut[tid];
+    if (by_work) {
+        const uint32_t w_max = (1u << work_bits) - 1u;
+        for (int l = tid; l < ng; l += GRP_ORDER_TPB) {
+            uint32_t c = 0;
+            for (int x = 1; x <= 7; ++x) c += cut[x] <= l ? 1u : 0u;
+            from[l] = (((c << work_bits) | (w_max - (uint32_t)loc_work[l])) << g_bits) | (uint32_t)l;
+        }
+        __syncthreads();
+        sort(3 + work_bits);
+    }
+    int32_t n_entries = 0, n_pairs = 0;
+    for (int f0 = 0; f0 < ng; f0 += GRP_ORDER_TPB) {
+        const int f = f0 + tid;
+        int32_t ne = 0, np = 0, round_e, round_p;
+        if (f < ng) {
+            const int32_t g = loc_group[by_work ? (int)(from[f] & g_mask) : f];
+            order[f] = g;
+            ne = rec[g].n_entries;
+            np = rec[g].n_pairs;
+        }
+        const int32_t e0 = n_entries + block_excl_sum<NW>(ne, sh, round_e), p0 = n_pairs + block_excl_sum<NW>(np, sh, round_p);
+        if (f < ng) {
+            entry0[f] = e0;
+            pair0[f] = p0;
+        }
+        n_entries += round_e;
+        n_pairs += round_p;
+    }
+    if (tid < 16) out_info[tid] = pinfo[tid];
+    if (tid == 0) {
+        entry0[ng] = n_entries;
+        int32_t mx = 0;
+        for (int x = 0; x < 8; ++x) mx = max(mx, cut[x + 1] - cut[x]);
+        for (int i = 0; i < 16; ++i) out_info[16 + i] = i == BPT_GI_N_GROUPS ? ng : i == BPT_GI_N_ENTRIES ? n_entries : i == BPT_GI_MAX_CHUNK ? mx : 0;
+    }
+}
+
+// a group's part of the arrays; the block behind the last group writes what stands behind the last entry
+__global__ __launch_bounds__(TPB) void k_group_write(const int4 *items, const int32_t *jorder, const int32_t *pinfo, const GroupRec *rec,
+                                                     const int32_t *order, const int32_t *entry0, const int32_t *pair0, const int32_t *chunks,
+                                                     const int4 *parked, const int32_t *parked_pairs, int64_t n_edges, int32_t R, int32_t n_groups,
+                                                     int32_t n_entries, int32_t max_chunk, int32_t pad_entries, int32_t seg_len, int32_t *members,
+                                                     int32_t *grp_ptr,
+                                                     int4 *entries, int32_t *pair_eid, int32_t *grp_eids, int32_t *out_chunks, int32_t *ginfo) {
+    const int32_t f = blockIdx.x, tid = threadIdx.x;
+    if (f >= n_groups) {
+        if (tid == 0) {
+            grp_ptr[n_groups] = n_entries;
+            entries[n_entries] = make_int4(0, 0, 0, 0);
+        }
+        if (tid < 9) out_chunks[tid] = chunks[tid];
+        if (tid < 16) ginfo[tid] = tid == BPT_GI_N_GROUPS ? n_groups : tid == BPT_GI_N_ENTRIES ? n_entries : tid == BPT_GI_MAX_CHUNK ? max_chunk : 0;
+        for (int i = tid; i < pad_entries * R; i += TPB) grp_eids[(int64_t)n_entries * R + i] = (int32_t)n_edges;
+        return;
+    }
+    __shared__ GroupSlots at;
+    const int32_t g = order[f], e0 = entry0[f], p0 = pair0[f];
+    const GroupRec r = rec[g];
+    if (tid < 16) {
+        int2 member;
+        at.load(items, nullptr, jorder, g, R, pinfo[BPT_PI_N_ITEMS], n_edges, seg_len, &member);
+        if (tid < R) reinterpret_cast<int2 *>(members)[(int64_t)f * R + tid] = member;
+    }
+    if (tid == 0) grp_ptr[f] = e0;
+    __syncthreads();
+    if (e0 + r.n_entries > n_entries || r.n_pairs > at.pre[16] || r.n_entries > r.n_pairs) return;    // (counts that are not this workspace's)
+    for (int u = tid; u < r.n_entries; u += TPB) {
+        int4 e = parked[at.slot(u)];
+        e.z += p0;
+        entries[e0 + u] = e;
+    }
+    for (int x = tid; x < r.n_pairs; x += TPB) pair_eid[p0 + x] = parked_pairs[at.slot(x)];
+    for (int i = tid; i < r.n_entries * R; i += TPB) {
+        const int u = i / R, m = i - u * R;
+        const int4 e = parked[at.slot(u)];
+        const uint32_t mask = (uint32_t)e.y;
+        grp_eids[(int64_t)e0 * R + i] = (mask >> m) & 1u ? parked_pairs[at.slot(e.z + __popc(mask & ((1u << m) - 1u)))] : (int32_t)n_edges;
+    }
+}
+
+// ---- pair numbers of the other side ---------------------------------------------------------------------------------------
+__global__ void k_number_pairs(const int32_t *pair_eid, int64_t n_edges, int32_t *number) {
+    const int64_t x = (int64_t)blockIdx.x * TPB + threadIdx.x;
+    if (x >= n_edges) return;
+    const int32_t e = pair_eid[x];
+    if (e >= 0 && e < n_edges) number[e] = (int32_t)x;
+}
+
+__global__ void k_find_numbers(const int32_t *eids, int64_t n_slots, int64_t n_edges, const int32_t *number, int32_t *pairs) {
+    const int64_t i = (int64_t)blockIdx.x * TPB + threadIdx.x;
+    if (i >= n_slots) return;
+    const int32_t e = eids[i];
+    pairs[i] = e >= 0 && e < n_edges ? number[e] : 0;
+}
+
 // ---- link -----------------------------------------------------------------------------------------------------------------
 __global__ void k_positions(const int32_t *eids_src, const int32_t *ginfo_src, int32_t R_src, int64_t n_edges, int32_t *pos) {
     const int64_t j = (int64_t)blockIdx.x * TPB + threadIdx.x;
@@ -1038,13 +1626,67 @@ template <class Recs, class Out>
 int rs_pass(const Recs &recs, const Out &out, int64_t n, int n_sides, int shift, int bits, int32_t *counts, int32_t *totals, hipStream_t s) {
     const dim3 tiles((unsigned)rs_tiles(n), (unsigned)n_sides);
     const int bins = 1 << bits;
-    hipLaunchKernelGGL(k_rs_count<Recs>, tiles, dim3(TPB), 0, s, recs, n, shift, bits, counts);
+    const bool few = rs_per_thread(n) != 8;
+    if (few) hipLaunchKernelGGL((k_rs_count<RS_KPT_FEW, Recs>), tiles, dim3(TPB), 0, s, recs, n, shift, bits, counts);
+    else hipLaunchKernelGGL((k_rs_count<8, Recs>), tiles, dim3(TPB), 0, s, recs, n, shift, bits, counts);
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL(k_rs_prefix, dim3((unsigned)((bins + 63) / 64), (unsigned)n_sides), dim3(RS_PREFIX_TPB), 0, s, counts, totals,
-                       (int64_t)tiles.x, bins);
+    if (few) {
+        hipLaunchKernelGGL((k_rs_scatter<RS_KPT_FEW, true, Recs, Out>), tiles, dim3(TPB), 0, s, recs, out, n, shift, bits, counts, totals);
+    } else {
+        hipLaunchKernelGGL(k_rs_prefix, dim3((unsigned)((bins + RS_PREFIX_BINS - 1) / RS_PREFIX_BINS), (unsigned)n_sides), dim3(RS_PREFIX_TPB), 0,
+                           s, counts, totals, (int64_t)tiles.x, bins);
+        HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL((k_rs_scatter<8, false, Recs, Out>), tiles, dim3(TPB), 0, s, recs, out, n, shift, bits, counts, totals);
+    }
     HIP_TRY(hipGetLastError());
-    hipLaunchKernelGGL((k_rs_scatter<Recs, Out>), tiles, dim3(TPB), 0, s, recs, out, n, shift, bits, counts, totals);
-    HIP_TRY(hipGetLastError());
+    return BPT_OK;
+}
+
+// all passes of a sort of one side: recs to begin with, out at the end
+template <class Recs, class Out>
+int rs_sort(const Recs &recs, const Out &out, int64_t n, uint64_t max_key, uint32_t *const key[2], int32_t *const val[2], int32_t *counts,
+            int32_t *totals, hipStream_t s) {
+    const RsPasses ps = rs_passes(max_key);
+    RsToArrays to[2];
+    RsArrays from[2];
+    for (int t = 0; t < 2; ++t)
+        for (int i = 0; i < 2; ++i) {
+            to[t].k[i] = key[t];
+            to[t].v[i] = val[t];
+            from[t].k[i] = key[t];
+            from[t].v[i] = val[t];
+        }
+    for (int p = 0; p < ps.n; ++p) {
+        const bool first = p == 0, last = p == ps.n - 1;
+        const int shift = p * ps.bits;
+        int st;
+        if (first && last) st = rs_pass(recs, out, n, 1, shift, ps.bits, counts, totals, s);
+        else if (first) st = rs_pass(recs, to[0], n, 1, shift, ps.bits, counts, totals, s);
+        else if (last) st = rs_pass(from[(p - 1) & 1], out, n, 1, shift, ps.bits, counts, totals, s);
+        else st = rs_pass(from[(p - 1) & 1], to[p & 1], n, 1, shift, ps.bits, counts, totals, s);
+        if (st != BPT_OK) return st;
+    }
+    return BPT_OK;
+}
+
+struct ShortForm {
+    int64_t max_groups;
+    int place_bits, g_bits, work_bits;
+};
+
+// BPT_ERR_UNSUPPORTED where the groups are not built in the short form: a group may hold more edges than fit a workgroup's LDS,
+// or there may be more groups, or wider numbers, than one workgroup sorts as 32-bit words
+int short_form(int64_t max_items, int64_t n_edges, int64_t n_index_nodes, int32_t seg_len, int32_t R, ShortForm &f) {
+    if (max_items < 0 || n_edges < 0 || n_index_nodes < 0 || max_items >= INT32_MAX || n_edges >= INT32_MAX || n_index_nodes >= INT32_MAX - 1)
+        return BPT_ERR_SIZE;
+    if (R < 1 || R > 16 || seg_len < 1) return BPT_ERR_SHAPE;
+    if ((n_edges + 8) * R >= INT32_MAX) return BPT_ERR_SIZE;
+    f.max_groups = (max_items + R - 1) / R;
+    if ((int64_t)R * seg_len > GRP_MAX_EDGES || f.max_groups > GRP_MAX_GROUPS) return BPT_ERR_UNSUPPORTED;
+    f.place_bits = (int)bits_for((uint64_t)seg_len - 1);
+    f.g_bits = (int)bits_for((uint64_t)(f.max_groups > 0 ? f.max_groups - 1 : 0));
+    f.work_bits = (int)bits_for((uint64_t)(R == 16 ? 4 * (seg_len + 1) : FIXED_WORK + R * seg_len));
+    if ((int)bits_for((uint64_t)n_index_nodes) + f.g_bits > 32 || 3 + f.work_bits + f.g_bits > 32) return BPT_ERR_UNSUPPORTED;
     return BPT_OK;
 }
 
@@ -1179,7 +1821,7 @@ int bpt_plan_device_bounds(int64_t n_units, int64_t n_edges, int64_t n_rows, int
     size_t tmp = 0;
     HIP_TRY(temp_bytes(max_items, max_groups, n_edges, n_rows, &tmp));
     Bump a{nullptr, 0}, b{nullptr, 0}, c{nullptr, 0};
-    base_layout(a, n_rows, n_edges, max_items, tmp);
+    base_layout(a, n_rows, n_edges, max_items);
     group_layout(b, max_items, max_groups, n_edges, tmp);
     c.take<int32_t>(n_edges);
     size_t ws = a.off > b.off ? a.off : b.off;
@@ -1195,49 +1837,126 @@ int bpt_plan_build_device(const int64_t *row, const int64_t *indptr_units, int64
                           const int64_t *indices, int64_t n_edges, int64_t n_rows, int64_t n_index_nodes, int32_t seg_len,
                           int32_t *rowptr, int32_t *idx32, int32_t *eid32, int32_t *items, int32_t *heavy, int32_t *info,
                           void *workspace, int64_t workspace_bytes, void *stream) {
-    int64_t bounds[4];
+    return bpt_build_plan_device(row, indptr_units, n_units, eid, indices, n_edges, n_rows, n_index_nodes, seg_len, rowptr, idx32, eid32,
+                                 items, heavy, nullptr, info, workspace, workspace_bytes, stream);
+}
+
+int bpt_build_plan_device(const int64_t *row, const int64_t *indptr_units, int64_t n_units, const int64_t *eid,
+                          const int64_t *indices, int64_t n_edges, int64_t n_rows, int64_t n_index_nodes, int32_t seg_len,
+                          int32_t *rowptr, int32_t *idx32, int32_t *eid32, int32_t *items, int32_t *heavy, int32_t *item_bounds,
+                          int32_t *info, void *workspace, int64_t workspace_bytes, void *stream) {
     const int st = sizes_ok(n_units, n_edges, n_rows, n_index_nodes, seg_len);
     if (st != BPT_OK) return st;
     if (!rowptr || !items || !info || !workspace) return BPT_ERR_NULL;
     if (n_units > 0 && (!row || !indptr_units)) return BPT_ERR_NULL;
     if (n_edges > 0 && (!eid || !idx32 || !eid32)) return BPT_ERR_NULL;
-    const int bs = bpt_plan_device_bounds(n_units, n_edges, n_rows, seg_len, 0, bounds);
-    if (bs != BPT_OK) return bs;
-    if (bounds[1] > 0 && !heavy) return BPT_ERR_NULL;
-    if (workspace_bytes < bounds[3]) return BPT_ERR_WORKSPACE;
-    hipStream_t s = (hipStream_t)stream;
-    const int64_t max_items = bounds[0];
-    size_t tmp = 0;
-    HIP_TRY(temp_bytes(max_items, 0, n_edges, n_rows, &tmp));
+    const int64_t max_items = n_rows + n_edges / seg_len;
+    if (max_items >= INT32_MAX) return BPT_ERR_SIZE;
+    if (n_edges / ((int64_t)seg_len + 1) > 0 && !heavy) return BPT_ERR_NULL;
     Bump bump{(char *)workspace, 0};
-    BaseWs w = base_layout(bump, n_rows, n_edges, max_items, tmp);
+    BaseWs w = base_layout(bump, n_rows, n_edges, max_items);
+    if (workspace_bytes < (int64_t)bump.off) return BPT_ERR_WORKSPACE;
+    hipStream_t s = (hipStream_t)stream;
 
-    hipLaunchKernelGGL(k_base_init, dim3(1), dim3(1), 0, s, info, indptr_units, n_units, n_edges);
+    LAUNCH(k_plan_clear, 1, info, indptr_units, n_units, n_edges);
+    const unsigned edge_blocks = blocks_for(n_edges), unit_blocks = blocks_for(n_units), row_blocks = (unsigned)item_row_blocks(n_rows);
+    hipLaunchKernelGGL(k_plan_narrow, dim3(edge_blocks + unit_blocks + row_blocks), dim3(TPB), 0, s, row, indptr_units, n_units, eid, indices,
+                       n_edges, n_rows, n_index_nodes, seg_len, edge_blocks, unit_blocks, info, idx32, eid32, w.seen, rowptr, w.totals);
     HIP_TRY(hipGetLastError());
-    LAUNCH(k_check_units, n_units, row, indptr_units, n_units, n_rows, info);
-    LAUNCH(k_fill_i32, n_edges, w.seen, n_edges, 0);
-    LAUNCH(k_narrow, n_edges, eid, indices, n_edges, n_index_nodes, info, idx32, eid32, w.seen);
-    LAUNCH(k_rowptr, n_rows + 1, row, indptr_units, n_units, n_rows, info, rowptr);
-    LAUNCH(k_row_counts, n_rows + 1, rowptr, n_rows, seg_len, info, w.c_items, w.c_heavy, w.c_slots);
-    size_t tb = tmp;
-    HIP_TRY(scan_i32(w.tmp, tb, w.c_items, w.b_items, n_rows + 1, s));
-    tb = tmp;
-    HIP_TRY(scan_i32(w.tmp, tb, w.c_heavy, w.b_heavy, n_rows + 1, s));
-    tb = tmp;
-    HIP_TRY(scan_i32(w.tmp, tb, w.c_slots, w.b_slots, n_rows + 1, s));
-    LAUNCH(k_emit_items, n_rows + 1, rowptr, n_rows, seg_len, w.b_items, w.b_heavy, w.b_slots, info, w.items_tmp, heavy);
+    // without indices the items stay in row order, as on the host
+    int4 *const in_rows = indices ? w.items_tmp : reinterpret_cast<int4 *>(items);
+    int2 *const bounds = reinterpret_cast<int2 *>(item_bounds);
+    hipLaunchKernelGGL(k_plan_items, dim3(row_blocks + edge_blocks), dim3(TPB), 0, s, rowptr, n_rows, seg_len, w.totals, eid32, w.seen, n_edges,
+                       row_blocks, info, in_rows, heavy);
+    HIP_TRY(hipGetLastError());
+    if (max_items == 0 || (!indices && !bounds)) return BPT_OK;
+    LAUNCH(k_item_bounds, max_items * 16, in_rows, idx32, info, max_items, n_index_nodes, n_edges, indices ? w.bounds_tmp : bounds);
+    if (!indices) return BPT_OK;
+    const uint32_t pad = (uint32_t)n_index_nodes + 1;
+    const ItemRecs recs{w.bounds_tmp, info, 0, pad};
+    const ItemsSorted sorted{w.items_tmp, w.bounds_tmp, info, reinterpret_cast<int4 *>(items), bounds};
+    return rs_sort(recs, sorted, max_items, pad, w.key, w.val, w.counts, w.bin_totals, s);
+}
+
+int bpt_build_groups_bounds(int64_t max_items, int64_t n_edges, int64_t n_index_nodes, int32_t seg_len, int32_t R, int64_t bounds[1]) {
+    if (!bounds) return BPT_ERR_NULL;
+    ShortForm f;
+    const int st = short_form(max_items, n_edges, n_index_nodes, seg_len, R, f);
+    if (st != BPT_OK) return st;
+    Bump dry{nullptr, 0};
+    short_layout(dry, max_items, f.max_groups, n_edges);
+    bounds[0] = (int64_t)dry.off + 256;
+    return BPT_OK;
+}
+
+int bpt_build_groups_count(const int32_t *items, const int32_t *item_bounds, const int32_t *idx32, const int32_t *eid32,
+                           const int32_t *plan_info, int64_t max_items, int64_t n_edges, int64_t n_index_nodes, int32_t seg_len, int32_t R,
+                           int32_t by_mask, int32_t *out_info, void *workspace, int64_t workspace_bytes, void *stream) {
+    ShortForm f;
+    const int st = short_form(max_items, n_edges, n_index_nodes, seg_len, R, f);
+    if (st != BPT_OK) return st;
+    if (by_mask < 0 || (by_mask & 3) > 2 || by_mask > 6) return BPT_ERR_SHAPE;
+    if (!plan_info || !out_info || !workspace || (max_items > 0 && (!items || !item_bounds))) return BPT_ERR_NULL;
+    if (n_edges > 0 && (!idx32 || !eid32)) return BPT_ERR_NULL;
+    Bump bump{(char *)workspace, 0};
+    ShortWs w = short_layout(bump, max_items, f.max_groups, n_edges);
+    if (workspace_bytes < (int64_t)bump.off) return BPT_ERR_WORKSPACE;
+    hipStream_t s = (hipStream_t)stream;
+    const int4 *const it = reinterpret_cast<const int4 *>(items);
+    const int2 *const bd = reinterpret_cast<const int2 *>(item_bounds);
+    const int by_work = (by_mask & 4) ? 0 : 1, mode = by_mask & 3;
     if (max_items > 0) {
-        // locality order: by smallest neighbour id (without indices the items stay in row order, as on the host)
-        LAUNCH(k_iota_i32, max_items, w.iota, max_items);
-        const int32_t *perm = w.iota;
-        if (indices) {
-            LAUNCH(k_item_keys<false>, max_items, w.items_tmp, idx32, info, max_items, n_index_nodes, n_edges, w.key);
-            tb = tmp;
-            HIP_TRY(sort_pairs<uint32_t>(w.tmp, tb, w.key, w.key_s, w.iota, w.perm, max_items, 32, s));
-            perm = w.perm;
-        }
-        LAUNCH(k_gather_items, max_items, w.items_tmp, perm, info, max_items, items);
+        // the items in the order of their largest neighbour; R consecutive ones are a group
+        const uint32_t pad = (uint32_t)n_index_nodes + 1;
+        const int ss = rs_sort(ItemRecs{bd, plan_info, 1, pad}, ItemOrder{w.jorder}, max_items, pad, w.key, w.val, w.counts,
+                               w.bin_totals, s);
+        if (ss != BPT_OK) return ss;
+        const bool narrow = bits_for((uint64_t)n_index_nodes) + 4 + f.place_bits <= 31;
+        auto form = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)f.max_groups), dim3(TPB), 0, s, it, bd, w.jorder, idx32, eid32, plan_info, n_edges, seg_len, R,
+                               f.place_bits, mode, w.rec, w.entries, w.pairs);
+            return hipGetLastError();
+        };
+        const int cap = R * seg_len;
+        if (narrow) HIP_TRY(cap <= 1024 ? form(k_group_form<1024, uint32_t>) : cap <= 2048 ? form(k_group_form<2048, uint32_t>) : form(k_group_form<4096, uint32_t>));
+        else HIP_TRY(cap <= 1024 ? form(k_group_form<1024, uint64_t>) : cap <= 2048 ? form(k_group_form<2048, uint64_t>) : form(k_group_form<4096, uint64_t>));
     }
+    // (the words of the groups are sorted in the items' key arrays, which are free again)
+    hipLaunchKernelGGL(k_group_order, dim3(1), dim3(GRP_ORDER_TPB), 0, s, w.rec, plan_info, R, by_work, f.g_bits,
+                       (int)bits_for((uint64_t)n_index_nodes), f.work_bits, w.key[0], w.key[1], w.loc_group, w.loc_work, w.loc_prefix, w.order, w.entry0, w.pair0, w.chunks, out_info);
+    HIP_TRY(hipGetLastError());
+    return BPT_OK;
+}
+
+int bpt_build_groups_write(const int32_t *items, const int32_t *plan_info, int64_t max_items, int64_t n_edges, int64_t n_index_nodes,
+                           int32_t seg_len, int32_t R, const int32_t *group_counts, int32_t pad_entries, int32_t *members,
+                           int32_t *grp_ptr, int32_t *entries, int32_t *pair_eid, int32_t *grp_eids, int32_t *chunks, int32_t *group_info,
+                           void *workspace, int64_t workspace_bytes, void *stream) {
+    ShortForm f;
+    const int st = short_form(max_items, n_edges, n_index_nodes, seg_len, R, f);
+    if (st != BPT_OK) return st;
+    if (!plan_info || !group_counts || !grp_ptr || !entries || !grp_eids || !chunks || !group_info || !workspace) return BPT_ERR_NULL;
+    const int32_t ng = group_counts[BPT_GI_N_GROUPS], ne = group_counts[BPT_GI_N_ENTRIES];
+    if (ng < 0 || ng > f.max_groups || ne < 0 || ne > n_edges || pad_entries < 0) return BPT_ERR_SIZE;
+    if ((ng > 0 && (!items || !members)) || (n_edges > 0 && !pair_eid)) return BPT_ERR_NULL;
+    Bump bump{(char *)workspace, 0};
+    ShortWs w = short_layout(bump, max_items, f.max_groups, n_edges);
+    if (workspace_bytes < (int64_t)bump.off) return BPT_ERR_WORKSPACE;
+    hipStream_t s = (hipStream_t)stream;
+    hipLaunchKernelGGL(k_group_write, dim3((unsigned)ng + 1), dim3(TPB), 0, s, reinterpret_cast<const int4 *>(items), w.jorder, plan_info, w.rec,
+                       w.order, w.entry0, w.pair0, w.chunks, w.entries, w.pairs, n_edges, R, ng, ne, group_counts[BPT_GI_MAX_CHUNK], pad_entries,
+                       seg_len, members, grp_ptr, reinterpret_cast<int4 *>(entries), pair_eid, grp_eids, chunks, group_info);
+    HIP_TRY(hipGetLastError());
+    return BPT_OK;
+}
+
+int bpt_build_pair_numbers(const int32_t *pair_eid_theirs, const int32_t *grp_eids_mine, int64_t n_slots, int64_t n_edges, int32_t *number,
+                           int32_t *pairs, void *stream) {
+    if (n_edges < 0 || n_slots < 0 || n_edges >= INT32_MAX || n_slots >= INT32_MAX) return BPT_ERR_SIZE;
+    if ((n_edges > 0 && (!pair_eid_theirs || !number)) || (n_slots > 0 && (!grp_eids_mine || !pairs))) return BPT_ERR_NULL;
+    hipStream_t s = (hipStream_t)stream;
+    LAUNCH(k_number_pairs, n_edges, pair_eid_theirs, n_edges, number);
+    LAUNCH(k_find_numbers, n_slots, grp_eids_mine, n_slots, n_edges, number, pairs);
     return BPT_OK;
 }
 

@@ -528,7 +528,7 @@ def attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale=None, drop
             seg = _tile_seg_len(plan)
     tiles = seg is not None
     if tiles:
-        plan = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True)
+        plan = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, None))
         ref = ctypes.byref(plan.bias_rows(TILE_ROWS)["struct"] if bias_by_pair else plan.ensure_groups(TILE_ROWS)["struct"])
     elif not _attention_groups(plan, dropout_p, bias, q, k, cfg):
         ref = plan.ref
@@ -576,13 +576,14 @@ def attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, in
     dt = _dtype(q)
     def tile_plans(seg):
         """The two tile plans and the structs the kernels take, or None where a side does not cover every edge."""
-        pi = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True)
-        po = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg_len=seg, prefer_device=True)
+        order_src = _plan.tile_order_src(k.size(0), eid_r.size(0))
+        pi = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, None))
+        po = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, order_src))
         if not (pi.covers_all_edges and po.covers_all_edges):
             return None
         # the destination side writes (p, ds) by its own pair numbers; the source side finds them through its pair mapping
         return (pi, po, ctypes.byref(pi.bias_rows(TILE_ROWS)["struct"] if bias_by_pair else pi.ensure_groups(TILE_ROWS)["struct"]),
-                ctypes.byref(po.linked_to(pi, TILE_ROWS, order=_plan.tile_order_src(po.n_rows, po.n_edges), partner_order=None, pair_numbers=True)))
+                ctypes.byref(po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True)))
 
     # as in attention_forward: the tile plans straight away where the tile kernels are certain
     seg = _tile_seg_without_plan(col, eid_c.size(0), q, k, h, d, dropout_p, bias, cfg) if _tiles_backward(None, q.dtype, bias) else None

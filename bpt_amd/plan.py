@@ -14,7 +14,7 @@ import threading
 import numpy as np
 import torch
 
-from ._lib import PlanInfo, PlanStruct, check_graph, graph_lib, plan_lib
+from ._lib import BPT_ERR_UNSUPPORTED, PlanInfo, PlanStruct, check_graph, graph_lib, plan_lib
 
 DEFAULT_SEG_LEN = None  # edges per work item: None = chosen per plan by auto_seg_len
 FORCE_SEG_LEN = None    # testing hook: when set, replaces the automatic choice for plans built from now on
@@ -212,9 +212,16 @@ class Plan:
     """Device-resident plan of one CSR side; `.struct` is the `bpt_plan` passed to the C ABI."""
 
     def device_bytes(self):
-        """Device memory held by this plan, its row groups and pair mappings."""
-        return (_tensor_bytes(self._dev) + _tensor_bytes(list(self._groups.values())) + _tensor_bytes(list(self._links.values()))
-                + _tensor_bytes(list(self._bias_rows.values())))
+        """Device memory held by this plan, its row groups and pair mappings (added up again when one of those was added: the cache
+        asks every plan it holds whenever a graph is new, which cost 1.1 ms a step with 64 plans of a new graph each)."""
+        parts = (len(self._groups), len(self._links), len(self._bias_rows))
+        if self._bytes is None or self._bytes[0] != parts:
+            with self._lock:
+                held = [list(x.values()) for x in (self._groups, self._links, self._bias_rows)]
+            self._bytes = (parts, _tensor_bytes(self._dev) + sum(_tensor_bytes(x) for x in held))
+        return self._bytes[1]
+
+    _bytes = None
 
     def __init__(self, row, indptr, eid, indices, n_rows, n_index_nodes, device, seg_len=DEFAULT_SEG_LEN):
         arrays, info = build_plan_host(row, indptr, eid, indices, n_rows, n_index_nodes, seg_len)
@@ -363,6 +370,12 @@ def _build_on_device(eid, n_rows):
     return DEVICE_BUILD
 
 
+def _stream_of(device):
+    """The device's current stream as an integer handle (torch.cuda.current_stream() builds a Stream object, some 5 us a call)."""
+    get = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    return get(device.index) if get is not None else torch.cuda.current_stream(device).cuda_stream
+
+
 _PLAN_ERRORS = {1: "row id, column id or edge id out of range", 2: "row / indptr not sorted", 3: "sizes out of the int32 range"}
 
 
@@ -392,10 +405,14 @@ class DevicePlan:
     """Plan of one CSR side built on the GPU from the reference's int64 device tensors (include/bptplan.h): no copy
     of the index arrays to the host, only the 16-int size blocks come back.  Same interface as Plan."""
 
-    device_bytes = Plan.device_bytes
+    device_bytes, _bytes = Plan.device_bytes, None
 
-    def __init__(self, row, indptr, eid, indices, n_rows, n_index_nodes, device, seg_len=DEFAULT_SEG_LEN):
+    def __init__(self, row, indptr, eid, indices, n_rows, n_index_nodes, device, seg_len=DEFAULT_SEG_LEN, groups=None):
+        """groups = (R, order_mode): row groups the caller is going to ask for anyway (ensure_groups); they are formed behind the
+        base plan and both are read back in one synchronisation."""
         self.device = torch.device(device)
+        if self.device.index is None:
+            self.device = torch.device("cuda", torch.cuda.current_device())
         self.n_rows, self.n_edges, self.n_index_nodes = int(n_rows), int(eid.numel()), int(n_index_nodes)
         self.has_indices = indices is not None
         if indptr.numel() != row.numel() + 1:
@@ -410,36 +427,34 @@ class DevicePlan:
         U, E = int(row.numel()), self.n_edges
         b = (ctypes.c_int64 * 4)()
         _check_plan(lib.bpt_plan_device_bounds(U, E, self.n_rows, self.seg_len, 0, ctypes.byref(b)), "bpt_plan_device_bounds")
+        # (items: upper bound, at most n_edges / seg_len more than there are)
         self._max_items, max_heavy = int(b[0]), int(b[1])
         i32 = lambda *shape: torch.empty(shape, dtype=torch.int32, device=self.device)
-        rowptr, idx, eid32 = i32(self.n_rows + 1), i32(max(E, 1)), i32(max(E, 1))
-        items, heavy, info = i32(max(self._max_items, 1), 4), i32(max(max_heavy, 1), 3), i32(16)
+        d = self._dev = {"rowptr": i32(self.n_rows + 1), "idx": i32(max(E, 1)), "eid": i32(max(E, 1)),
+                         "items": i32(max(self._max_items, 1), 4), "bounds": i32(max(self._max_items, 1), 2), "heavy": i32(max(max_heavy, 1), 3)}
+        self._info = i32(16)
         ws = torch.empty(int(b[3]), dtype=torch.uint8, device=self.device)
         with torch.cuda.device(self.device):
-            st = lib.bpt_plan_build_device(row.data_ptr() if U else None, indptr.data_ptr() if U else None, U,
+            st = lib.bpt_build_plan_device(row.data_ptr() if U else None, indptr.data_ptr() if U else None, U,
                                            eid.data_ptr() if E else None,
                                            indices.data_ptr() if (indices is not None and E) else None, E, self.n_rows,
-                                           self.n_index_nodes, self.seg_len, rowptr.data_ptr(), idx.data_ptr(),
-                                           eid32.data_ptr(), items.data_ptr(), heavy.data_ptr(), info.data_ptr(),
-                                           ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
-        _check_plan(st, "bpt_plan_build_device")
-        h = info.cpu().tolist()                       # the one synchronisation of the build
+                                           self.n_index_nodes, self.seg_len, d["rowptr"].data_ptr(), d["idx"].data_ptr(),
+                                           d["eid"].data_ptr(), d["items"].data_ptr(), d["heavy"].data_ptr(), d["bounds"].data_ptr(),
+                                           self._info.data_ptr(), ws.data_ptr(), ws.numel(), _stream_of(self.device))
+            _check_plan(st, "bpt_build_plan_device")
+            formed = None if groups is None else self._form_groups(groups[0], self._by_mask(groups[0], groups[1]))
+        h = self._info.cpu().tolist() if formed is None else formed["info"]      # the one synchronisation of the build
         if h[0] != 0:
             raise ValueError("bptplan: " + _PLAN_ERRORS.get(h[0], f"error {h[0]}"))
         self.n_items, self.n_heavy, self.n_slots, self.max_degree = h[1], h[2], h[3], h[4]
         self.covers_all_edges = bool(h[5] & 1)
-        self._info = info
-        # the work lists were allocated for their upper bounds: keep what the build produced
-        items, heavy = items[:max(self.n_items, 1)].clone(), heavy[:max(self.n_heavy, 1)].clone()
-        self._max_items = max(self.n_items, 1)
-        self._dev = {"rowptr": rowptr, "idx": idx, "eid": eid32, "items": items, "heavy": heavy}
-        d = self._dev
-        torch.cuda.current_stream(self.device).synchronize()      # the plan is complete before any stream can use it
         self.struct = PlanStruct(
             d["rowptr"].data_ptr(), d["idx"].data_ptr() if E else None, d["eid"].data_ptr() if E else None,
             d["items"].data_ptr() if self.n_items else None, d["heavy"].data_ptr() if self.n_heavy else None,
             self.n_rows, E, self.n_items, self.n_heavy, self.n_slots)
         self.struct.n_index_nodes = self.n_index_nodes
+        if formed is not None:
+            self._write_groups(formed)
 
     def _auto_seg_len(self, row, indptr):
         """auto_seg_len on the device: the 90 % quantile of the non-empty rows' degrees."""
@@ -462,53 +477,110 @@ class DevicePlan:
         """The group order where a caller names none: tile groups by tile_order_dst, the others GROUP_ORDER."""
         return tile_order_dst(self.n_index_nodes) if R == TILE_GROUP_R else GROUP_ORDER
 
-    def ensure_groups(self, R=GROUP_R, order_mode=None):
-        """Row groups of R rows built on the GPU (bpt_plan_group_device).  Of order_mode only the entry order counts:
-        by member mask (+4), or for the aligned order of the host builder (+8), which is sequential by construction, its
-        parallel stand-in (entries by neighbour id mod 16, then id); else ascending neighbour."""
+    def _by_mask(self, R, order_mode):
+        """Of order_mode only the entry order counts: by member mask (+4), or for the aligned order of the host builder (+8), which
+        is sequential by construction, its parallel stand-in (entries by neighbour id mod 16, then id); else ascending neighbour;
+        + 4 where the groups of a range keep their locality order."""
         order_mode = self.default_order(R) if order_mode is None else order_mode
-        by_mask = (2 if order_mode & 8 else (1 if order_mode & 4 else 0)) + (0 if order_mode & 2 else 4)
+        return (2 if order_mode & 8 else (1 if order_mode & 4 else 0)) + (0 if order_mode & 2 else 4)
+
+    def _form_groups(self, R, by_mask):
+        """bpt_build_groups_count: the groups formed in a workspace and their sizes read back (one synchronisation), or None where
+        only bpt_plan_group_device builds them."""
+        lib, E, d = plan_lib(), self.n_edges, self._dev
+        b = (ctypes.c_int64 * 1)()
+        st = lib.bpt_build_groups_bounds(self._max_items, E, self.n_index_nodes, self.seg_len, R, ctypes.byref(b))
+        if st == BPT_ERR_UNSUPPORTED:
+            return None
+        _check_plan(st, "bpt_build_groups_bounds")
+        ws = torch.empty(int(b[0]), dtype=torch.uint8, device=self.device)
+        counts = torch.empty(32, dtype=torch.int32, pin_memory=True)
+        stream = _stream_of(self.device)
+        st = lib.bpt_build_groups_count(d["items"].data_ptr(), d["bounds"].data_ptr(), d["idx"].data_ptr(), d["eid"].data_ptr(),
+                                        self._info.data_ptr(), self._max_items, E, self.n_index_nodes, self.seg_len, R, int(by_mask),
+                                        counts.data_ptr(), ws.data_ptr(), ws.numel(), stream)
+        _check_plan(st, "bpt_build_groups_count")
+        _check_plan(lib.bpt_build_wait(stream), "bpt_build_wait")
+        info = counts.tolist()
+        return {"R": R, "by_mask": by_mask, "ws": ws, "info": info[:16], "counts": info[16:]}
+
+    def _write_groups(self, formed):
+        """bpt_build_groups_write: the arrays of the groups that _form_groups left in its workspace."""
+        lib, E, d, R = plan_lib(), self.n_edges, self._dev, formed["R"]
+        ng, ne, max_chunk = formed["counts"][:3]
+        i32 = lambda *shape: torch.empty(shape, dtype=torch.int32, device=self.device)
+        dev = {"members": i32(ng, R, 2), "grp_ptr": i32(ng + 1), "entries": i32(ne + 1, 4), "pair_eid": i32(E),
+               "eids": i32((ne + GROUP_PAD_ENTRIES) * R), "chunks": i32(9), "ginfo": i32(16)}
+        counts = (ctypes.c_int32 * 16)(*formed["counts"])
+        with torch.cuda.device(self.device):
+            stream = _stream_of(self.device)
+            st = lib.bpt_build_groups_write(d["items"].data_ptr(), self._info.data_ptr(), self._max_items, E, self.n_index_nodes, self.seg_len, R,
+                                            ctypes.byref(counts), GROUP_PAD_ENTRIES, dev["members"].data_ptr() if ng else None,
+                                            dev["grp_ptr"].data_ptr(), dev["entries"].data_ptr(), dev["pair_eid"].data_ptr() if E else None,
+                                            dev["eids"].data_ptr(), dev["chunks"].data_ptr(), dev["ginfo"].data_ptr(),
+                                            formed["ws"].data_ptr(), formed["ws"].numel(), stream)
+            _check_plan(st, "bpt_build_groups_write")
+            return self._keep_groups(dev, R, formed["by_mask"], ng, ne, max_chunk)
+
+    def _keep_groups(self, dev, R, by_mask, ng, ne, max_chunk):
+        st = PlanStruct.from_buffer_copy(self.struct)
+        st.grp_members = dev["members"].data_ptr() if ng else None
+        st.grp_ptr = dev["grp_ptr"].data_ptr()
+        st.grp_entries = dev["entries"].data_ptr()
+        st.grp_pairs = None
+        st.grp_chunks = dev["chunks"].data_ptr()
+        st.grp_max_chunk = max_chunk
+        st.n_groups = ng
+        st.grp_R = R
+        st.n_grp_entries = ne
+        st.grp_eids = dev["eids"].data_ptr()
+        hit = _Groups(dev=dev, struct=st, R=R, n_edges=self.n_edges)
+        self._wait()
+        self._groups[(R, by_mask)] = hit
+        return hit
+
+    def _wait(self):
+        """What was built is complete before another stream may read it."""
+        with torch.cuda.device(self.device):
+            _check_plan(plan_lib().bpt_build_wait(_stream_of(self.device)), "bpt_build_wait")
+
+    def ensure_groups(self, R=GROUP_R, order_mode=None):
+        """Row groups of R rows built on the GPU: bpt_build_groups_count / _write, or bpt_plan_group_device for groups of more than
+        4096 edges and plans of more than 16384 groups."""
+        by_mask = self._by_mask(R, order_mode)
         with self._lock:
             hit = self._groups.get((R, by_mask))
             if hit is None:
-                lib = plan_lib()
-                E = self.n_edges
-                b = (ctypes.c_int64 * 4)()
-                _check_plan(lib.bpt_plan_device_bounds(0, E, self.n_rows, self.seg_len, R, ctypes.byref(b)),
-                            "bpt_plan_device_bounds")
-                max_groups = (self._max_items + R - 1) // R
-                i32 = lambda *shape: torch.empty(shape, dtype=torch.int32, device=self.device)
-                members, grp_ptr, entries = i32(max(max_groups, 1), R, 2), i32(max_groups + 1), i32(E + 1, 4)
-                pair_eid, eids, chunks, ginfo = i32(max(E, 1)), i32((E + GROUP_PAD_ENTRIES) * R), i32(9), i32(16)
-                ws = torch.empty(int(b[3]), dtype=torch.uint8, device=self.device)
-                d = self._dev
                 with torch.cuda.device(self.device):
-                    st = lib.bpt_plan_group_device(d["items"].data_ptr(), d["idx"].data_ptr(), d["eid"].data_ptr(),
-                                                   self._info.data_ptr(), self._max_items, E, self.n_index_nodes,
-                                                   self.seg_len, R, int(by_mask), members.data_ptr(), grp_ptr.data_ptr(),
-                                                   entries.data_ptr(), pair_eid.data_ptr(), eids.data_ptr(),
-                                                   chunks.data_ptr(), ginfo.data_ptr(), ws.data_ptr(), ws.numel(),
-                                                   torch.cuda.current_stream().cuda_stream)
-                _check_plan(st, "bpt_plan_group_device")
-                ng, ne, max_chunk = ginfo.cpu().tolist()[:3]
-                dev = {"members": members[:ng].clone(), "grp_ptr": grp_ptr[:ng + 1].clone(),
-                       "entries": entries[:ne + 1].clone(), "pair_eid": pair_eid[:E].clone(),
-                       "eids": eids[:(ne + GROUP_PAD_ENTRIES) * R].clone(), "chunks": chunks, "ginfo": ginfo}
-                st = PlanStruct.from_buffer_copy(self.struct)
-                st.grp_members = dev["members"].data_ptr() if ng else None
-                st.grp_ptr = dev["grp_ptr"].data_ptr()
-                st.grp_entries = dev["entries"].data_ptr()
-                st.grp_pairs = None
-                st.grp_chunks = dev["chunks"].data_ptr()
-                st.grp_max_chunk = max_chunk
-                st.n_groups = ng
-                st.grp_R = R
-                st.n_grp_entries = ne
-                st.grp_eids = dev["eids"].data_ptr()
-                hit = _Groups(dev=dev, struct=st, R=R, n_edges=E)
-                torch.cuda.current_stream(self.device).synchronize()      # the clones above ran on the building stream
-                self._groups[(R, by_mask)] = hit
+                    formed = self._form_groups(R, by_mask)
+                hit = self._write_groups(formed) if formed is not None else self._groups_by_sort(R, by_mask)
         return hit
+
+    def _groups_by_sort(self, R, by_mask):
+        lib = plan_lib()
+        E = self.n_edges
+        b = (ctypes.c_int64 * 4)()
+        _check_plan(lib.bpt_plan_device_bounds(0, E, self.n_rows, self.seg_len, R, ctypes.byref(b)), "bpt_plan_device_bounds")
+        max_groups = (self._max_items + R - 1) // R
+        i32 = lambda *shape: torch.empty(shape, dtype=torch.int32, device=self.device)
+        members, grp_ptr, entries = i32(max(max_groups, 1), R, 2), i32(max_groups + 1), i32(E + 1, 4)
+        pair_eid, eids, chunks, ginfo = i32(max(E, 1)), i32((E + GROUP_PAD_ENTRIES) * R), i32(9), i32(16)
+        ws = torch.empty(int(b[3]), dtype=torch.uint8, device=self.device)
+        d = self._dev
+        with torch.cuda.device(self.device):
+            st = lib.bpt_plan_group_device(d["items"].data_ptr(), d["idx"].data_ptr(), d["eid"].data_ptr(),
+                                           self._info.data_ptr(), self._max_items, E, self.n_index_nodes,
+                                           self.seg_len, R, int(by_mask), members.data_ptr(), grp_ptr.data_ptr(),
+                                           entries.data_ptr(), pair_eid.data_ptr(), eids.data_ptr(),
+                                           chunks.data_ptr(), ginfo.data_ptr(), ws.data_ptr(), ws.numel(),
+                                           _stream_of(self.device))
+        _check_plan(st, "bpt_plan_group_device")
+        ng, ne, max_chunk = ginfo.cpu().tolist()[:3]
+        # (the arrays were allocated for their upper bounds: keep what the build produced)
+        dev = {"members": members[:ng].clone(), "grp_ptr": grp_ptr[:ng + 1].clone(),
+               "entries": entries[:ne + 1].clone(), "pair_eid": pair_eid[:E].clone(),
+               "eids": eids[:(ne + GROUP_PAD_ENTRIES) * R].clone(), "chunks": chunks, "ginfo": ginfo}
+        return self._keep_groups(dev, R, by_mask, ng, ne, max_chunk)
 
     def bias_rows(self, R=TILE_GROUP_R):
         """As Plan.bias_rows, from the groups built on the GPU."""
@@ -517,14 +589,14 @@ class DevicePlan:
         if hit is None:
             g = self.ensure_groups(R)
             hit = _bias_rows_of(g["struct"], g["dev"]["pair_eid"], g["dev"]["eids"], self.n_edges)
-            torch.cuda.current_stream(self.device).synchronize()      # complete before another stream may read it
+            self._wait()
             with self._lock:
                 self._bias_rows[R] = hit
         return hit
 
     def linked_to(self, plan_src, R=GROUP_R, order=None, partner_order=GROUP_ORDER_SRC, pair_numbers=False):
-        """As Plan.linked_to, with the pair mapping computed on the GPU (bpt_plan_link_device; the pair numbers by an
-        inverse permutation and a gather)."""
+        """As Plan.linked_to, with the pair mapping computed on the GPU (bpt_plan_link_device; the pair numbers by
+        bpt_build_pair_numbers: an inverse permutation and a gather)."""
         mine, theirs = self.ensure_groups(R, order), plan_src.ensure_groups(R, partner_order)
         key = (id(plan_src), R, order, partner_order) + ((True,) if pair_numbers else ())
         with self._lock:
@@ -544,10 +616,14 @@ class DevicePlan:
                     self._links[key] = hit
                     return hit[0]
                 if pair_numbers:
-                    number = torch.zeros(E + 1, dtype=torch.int32, device=self.device)
-                    number[theirs["dev"]["pair_eid"][:E].long()] = torch.arange(E, dtype=torch.int32, device=self.device)
-                    pairs = number[mine["dev"]["eids"].long()]          # absent members carry the edge id E: number 0
-                    torch.cuda.current_stream(self.device).synchronize()
+                    n_slots = mine["dev"]["eids"].numel()
+                    number, pairs = (torch.empty(max(k, 1), dtype=torch.int32, device=self.device) for k in (E, n_slots))
+                    with torch.cuda.device(self.device):
+                        _check_plan(plan_lib().bpt_build_pair_numbers(theirs["dev"]["pair_eid"].data_ptr() if E else None,
+                                                                      mine["dev"]["eids"].data_ptr(), n_slots, E, number.data_ptr(),
+                                                                      pairs.data_ptr(), _stream_of(self.device)),
+                                    "bpt_build_pair_numbers")
+                    self._wait()
                     st = PlanStruct.from_buffer_copy(mine["struct"])
                     st.grp_pairs = pairs.data_ptr()
                     hit = (st, pairs, plan_src)
@@ -560,10 +636,10 @@ class DevicePlan:
                     st = plan_lib().bpt_plan_link_device(mine["dev"]["eids"].data_ptr(), mine["dev"]["ginfo"].data_ptr(), R,
                                                          theirs["dev"]["eids"].data_ptr(), theirs["dev"]["ginfo"].data_ptr(), R,
                                                          E, GROUP_PAD_ENTRIES, pairs.data_ptr(), ws.data_ptr(), ws.numel(),
-                                                         torch.cuda.current_stream().cuda_stream)
+                                                         _stream_of(self.device))
                 _check_plan(st, "bpt_plan_link_device")
                 pairs = pairs[:n_pairs].clone()
-                torch.cuda.current_stream(self.device).synchronize()      # complete before another stream may read it
+                self._wait()
                 st = PlanStruct.from_buffer_copy(mine["struct"])
                 st.grp_pairs = pairs.data_ptr()
                 hit = (st, pairs, plan_src)
@@ -613,10 +689,11 @@ class PlanCache:
         return tuple((t.data_ptr(), t.numel(), t._version, t.device) if t is not None else None
                      for t in tensors) + (n_rows, n_index, seg_len, on_device)
 
-    def get(self, row, indptr, eid, indices, n_rows=None, n_index_nodes=None, seg_len=DEFAULT_SEG_LEN, prefer_device=False):
+    def get(self, row, indptr, eid, indices, n_rows=None, n_index_nodes=None, seg_len=DEFAULT_SEG_LEN, prefer_device=False, groups=None):
         """n_rows None: as many rows as `row` mentions (ops that only produce edge outputs).  prefer_device: build on the GPU
         whatever the graph's size, unless set_device_build() fixed the place (the tile kernels ask for this: the GPU
-        builder's groups of 16 run them as fast or faster on every graph measured)."""
+        builder's groups of 16 run them as fast or faster on every graph measured).  groups = (R, order_mode): row groups the caller
+        asks the plan for next; a plan built on the GPU for this call forms them along with it."""
         tensors = (row, indptr, eid, indices)
         on_device = _build_on_device(eid, n_rows) or bool(prefer_device and DEVICE_BUILD is None and eid.is_cuda and n_rows is not None)
         key = self._key(tensors, n_rows, n_index_nodes, seg_len, on_device)
@@ -632,7 +709,7 @@ class PlanCache:
         if on_device:
             nr = n_rows if n_rows is not None else (int(row[-1]) + 1 if row.numel() else 0)
             ni = n_index_nodes if n_index_nodes is not None else nr
-            plan = DevicePlan(row, indptr, eid, indices, nr, ni, eid.device, seg_len)
+            plan = DevicePlan(row, indptr, eid, indices, nr, ni, eid.device, seg_len, groups=groups)
         else:
             row_h = _host_i64(row)
             nr = n_rows if n_rows is not None else (int(row_h[-1]) + 1 if len(row_h) else 0)

@@ -19,6 +19,35 @@ int bpt_build_csrs_device(const int64_t *src, const int64_t *dst, int64_t n_edge
                           int64_t *const out_side[5], int64_t *const in_side[5], int32_t *info, void *workspace,
                           int64_t workspace_bytes, void *stream);
 
+/* bpt_plan_build_device (bptplan.h), and the smallest and the largest neighbour id of every item beside it (item_bounds: as many
+ * rows of 2 int32 as items, or NULL). */
+int bpt_build_plan_device(const int64_t *row, const int64_t *indptr_units, int64_t n_units, const int64_t *eid,
+                          const int64_t *indices, int64_t n_edges, int64_t n_rows, int64_t n_index_nodes, int32_t seg_len,
+                          int32_t *rowptr, int32_t *idx32, int32_t *eid32, int32_t *items, int32_t *heavy, int32_t *item_bounds,
+                          int32_t *info, void *workspace, int64_t workspace_bytes, void *stream);
+
+/* The row groups of bpt_plan_group_device (bptplan.h), bit for bit, in two calls between which the caller reads how large they
+ * are and allocates exactly: bpt_build_groups_count forms and numbers the groups in the workspace and writes out_info (int32[32],
+ * in memory the device can write: the plan's info block, then the groups' info block); bpt_build_groups_write, given the groups'
+ * info block on the host (group_counts), writes the arrays from the same workspace:
+ *   members (n_groups, R, 2)   grp_ptr (n_groups + 1)   entries (n_entries + 1, 4)   pair_eid (n_edges)
+ *   grp_eids ((n_entries + pad_entries) * R)            chunks (9)                   group_info: int32[16]
+ * bpt_build_groups_bounds: workspace bytes, or BPT_ERR_UNSUPPORTED where only bpt_plan_group_device builds the groups (more than
+ * 4096 edges a group, or more than 16384 groups). */
+int bpt_build_groups_bounds(int64_t max_items, int64_t n_edges, int64_t n_index_nodes, int32_t seg_len, int32_t R, int64_t bounds[1]);
+int bpt_build_groups_count(const int32_t *items, const int32_t *item_bounds, const int32_t *idx32, const int32_t *eid32,
+                           const int32_t *plan_info, int64_t max_items, int64_t n_edges, int64_t n_index_nodes, int32_t seg_len,
+                           int32_t R, int32_t by_mask, int32_t *out_info, void *workspace, int64_t workspace_bytes, void *stream);
+int bpt_build_groups_write(const int32_t *items, const int32_t *plan_info, int64_t max_items, int64_t n_edges,
+                           int64_t n_index_nodes, int32_t seg_len, int32_t R, const int32_t *group_counts, int32_t pad_entries,
+                           int32_t *members, int32_t *grp_ptr, int32_t *entries, int32_t *pair_eid, int32_t *grp_eids,
+                           int32_t *chunks, int32_t *group_info, void *workspace, int64_t workspace_bytes, void *stream);
+
+/* For every (entry, member) of one side's groups (grp_eids_mine, n_slots) the number of the same edge's pair on the other side
+ * (pair_eid_theirs, n_edges), 0 where there is none.  number: n_edges int32 of scratch. */
+int bpt_build_pair_numbers(const int32_t *pair_eid_theirs, const int32_t *grp_eids_mine, int64_t n_slots, int64_t n_edges,
+                           int32_t *number, int32_t *pairs, void *stream);
+
 /* Waits until everything enqueued on the stream has run (for a caller that reads an info block in pinned host memory). */
 int bpt_build_wait(void *stream);
 

@@ -5,6 +5,9 @@ import numpy as np
 import pytest
 import torch
 
+import parallel_plan_model as model
+from test_gpu_device_plan import check_base, check_groups
+
 pytestmark = pytest.mark.gpu
 
 DEV = "cuda:0"
@@ -31,3 +34,37 @@ def test_csrs_at_the_edges_of_tiles_and_digits(n, E, skew):
             assert a.dtype == torch.int64 and np.array_equal(a.cpu().numpy(), b)
     for a, b in zip(got[2:], want[2:]):
         assert a.dtype == torch.int64 and np.array_equal(a.cpu().numpy(), b)
+
+
+@pytest.mark.parametrize("order", [2, 6, 4], ids=["neighbour", "mask", "mask-local"])
+@pytest.mark.parametrize("n,n_index,E,seg,R", [
+    (70, 40, 3000, 64, 16),             # a group of the largest size: 1024 edges, many of them repeated
+    (70, 300, 5000, 128, 16),           # ... 2048
+    (50, 5000, 9000, 256, 16),          # ... 4096
+    (50, 5000, 9000, 257, 16),          # one more: groups by device-wide sorts
+    (33, 9, 2000, 512, 8),
+    (200, 3000000, 4000, 64, 16),       # neighbours that take 64-bit keys
+    (1, 1, 1, 1, 1),
+    (40000, 700, 20000, 8, 4),          # more groups than are sorted in LDS
+    (70000, 700, 20000, 8, 4),          # more groups than one workgroup numbers
+])
+def test_groups_at_the_edges_of_their_forms(n, n_index, E, seg, R, order):
+    from bpt_amd import graphbuilder as gb
+    from bpt_amd.plan import DevicePlan
+    rng = np.random.default_rng(n + seg)
+    rows, cols = rng.integers(0, n, E), rng.integers(0, n_index, E)
+    rows[: E // 4] = n // 2                                       # a row of many items
+    rows, cols = rows.astype(np.int64), cols.astype(np.int64)
+    eid = np.argsort(rows, kind="stable").astype(np.int64)
+    indptr = np.zeros(n + 1, dtype=np.int64)
+    np.cumsum(np.bincount(rows, minlength=n), out=indptr[1:])
+    row, units = gb.partition_csr(indptr, 32)
+    arrs = (row, units, eid, cols[eid])
+    want, info = model.base_plan(*arrs, n, n_index, seg)
+    by_mask = {2: 0, 6: 1, 4: 5}[order]
+    groups = model.group_plan(want, n_index, R, by_mask)
+    tens = tuple(torch.from_numpy(a).to(DEV) for a in arrs)
+    for asked_first in (True, False):                             # formed along with the base plan, or behind it
+        plan = DevicePlan(*tens, n, n_index, DEV, seg, groups=(R, order) if asked_first else None)
+        check_base(plan, want, info)
+        check_groups(plan.ensure_groups(R, order), groups, E)
