@@ -329,35 +329,39 @@ def merge_graphs(graphs):
     return cat(src), cat(dst), cat(et), cat(pos), v_shift
 
 
-_DEVICE_EDGES = {}           # (graph class, constructor arguments, device) -> (src, dst, etype, pos) device tensors
+_DEVICE_EDGES = {}           # (graph class, constructor arguments, device) -> (src, dst, etype, pos) device tensors and their part record
 _DEVICE_EDGES_MAX = 4096
 
 
 def merge_graphs_device(graphs, device):
     """merge_graphs with the result on the GPU: the edge lists of the single graphs are kept on the device per
     (class, length, ...) the way the reference caches them on the host (graph/base.py:12-26), and a batch is their
-    concatenation plus the node shifts (graph/lm.py:83-98), formed there; only the shifts and counts of the batch
-    (one number per graph) cross the bus.  Returns int64 device tensors (src, dst, etype, pos) and n_nodes."""
+    concatenation with the node ids shifted (graph/lm.py:83-98), written there by one launch per 64 graphs
+    (bpt_build_merge_device).  Returns int64 device tensors (src, dst, etype, pos) and n_nodes."""
     import torch
+    from ._lib import plan_lib
     device = torch.device(device)
-    parts, shifts, v_shift = [], [], 0
+    if device.type == "cuda" and device.index is None:
+        device = torch.device("cuda", torch.cuda.current_device())
+    parts, lists, n_edges, n_nodes = [], [], 0, 0
     for g in graphs:
-        key = (type(g).__name__,) + tuple(g.__reduce__()[1]) + (str(device),)
+        key = (type(g), g._length, g._triu, g._a, g._b, device)
         hit = _DEVICE_EDGES.get(key)
         if hit is None:
             if len(_DEVICE_EDGES) >= _DEVICE_EDGES_MAX:
                 _DEVICE_EDGES.clear()
-            hit = (*g.get_edges_device(device), torch.from_numpy(g.get_pos()).to(device))
-            _DEVICE_EDGES[key] = hit
-        parts.append(hit)
-        shifts.append(v_shift)
-        v_shift += g.number_of_nodes
-    if not parts:
-        e = torch.empty(0, dtype=torch.int64, device=device)
-        return e, e.clone(), e.clone(), e.clone(), 0
-    counts = torch.tensor([p[0].numel() for p in parts], dtype=torch.int64)
-    n_edges = int(counts.sum())
-    shift = torch.repeat_interleave(torch.tensor(shifts, dtype=torch.int64).to(device), counts.to(device), output_size=n_edges)
-    src = torch.cat([p[0] for p in parts]) + shift
-    dst = torch.cat([p[1] for p in parts]) + shift
-    return src, dst, torch.cat([p[2] for p in parts]), torch.cat([p[3] for p in parts]), v_shift
+            tensors = (*g.get_edges_device(device), torch.from_numpy(g.get_pos()).to(device))
+            hit = _DEVICE_EDGES[key] = (tensors, tuple(t.data_ptr() for t in tensors) + (tensors[0].numel(), tensors[3].numel()))
+        lists.append(hit[0])                              # (kept until the launch: the cache may drop them meanwhile)
+        parts += hit[1]
+        n_edges += hit[1][4]
+        n_nodes += hit[1][5]
+    src, dst, etype = (torch.empty(n_edges, dtype=torch.int64, device=device) for _ in range(3))
+    pos = torch.empty(n_nodes, dtype=torch.int64, device=device)
+    if parts:
+        with torch.cuda.device(device):
+            st = plan_lib().bpt_build_merge_device((ctypes.c_int64 * len(parts))(*parts), len(lists), src.data_ptr(), dst.data_ptr(),
+                                                   etype.data_ptr(), pos.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        if st != 0:
+            raise RuntimeError(f"bpt_build_merge_device: status {st}")
+    return src, dst, etype, pos, n_nodes

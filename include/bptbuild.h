@@ -11,6 +11,12 @@
 extern "C" {
 #endif
 
+/* The block-diagonal merge of graph/lm.py:53-98: parts (host memory) holds six int64 per graph, the device addresses of its src,
+ * dst, etype (n_edges each) and pos (n_nodes), then n_edges and n_nodes; the lists are written one after the other, node ids
+ * shifted by the nodes of the graphs before. */
+int bpt_build_merge_device(const int64_t *parts, int64_t n_parts, int64_t *src, int64_t *dst, int64_t *etype, int64_t *pos,
+                           void *stream);
+
 /* bpt_csr_build_device (bptplan.h) for both sides of a graph in one set of launches: the out-CSR (edges grouped by src) and the
  * in-CSR (by dst) of graph/base.py:71-86.  out_side / in_side: host arrays of the five device pointers (indptr, indices, eid,
  * unit_row, unit_ptr) of each side; sizes and workspace as bpt_csr_device_bounds says.  info: int32[4] = (error, number of

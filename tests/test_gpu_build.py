@@ -68,3 +68,14 @@ def test_groups_at_the_edges_of_their_forms(n, n_index, E, seg, R, order):
         plan = DevicePlan(*tens, n, n_index, DEV, seg, groups=(R, order) if asked_first else None)
         check_base(plan, want, info)
         check_groups(plan.ensure_groups(R, order), groups, E)
+
+
+@pytest.mark.parametrize("n_graphs", [1, 63, 64, 65, 130])
+def test_merge_at_the_edges_of_a_launch(n_graphs):
+    from bpt_amd import graphbuilder as gb
+    rng = np.random.default_rng(n_graphs)
+    graphs = [gb.BinaryPartition(int(L), True, 4, 10) for L in rng.integers(1, 700, n_graphs)] + [gb.FullyConnected(1, True, 2)]
+    want, got = gb.merge_graphs(graphs), gb.merge_graphs_device(graphs, DEV)
+    assert got[4] == want[4]
+    for a, b in zip(got[:4], want[:4]):
+        assert a.dtype == torch.int64 and np.array_equal(a.cpu().numpy(), b)
