@@ -1,8 +1,9 @@
-"""Compiles the three native libraries in-tree:
+"""Compiles the four native libraries in-tree:
 
   bpt_amd/csrc/libbptgraph.so  host C++ (g++)            <- bptgraph.cpp
   bpt_amd/csrc/libbptattn.so   gfx950 HIP (hipcc)        <- bptattn.hip
   bpt_amd/csrc/libbptplan.so   gfx950 HIP (hipcc)        <- bptplan.hip  (plans built on the GPU; rocPRIM headers)
+  bpt_amd/csrc/bptop.so        host C++ (g++, torch)     <- bptop.cpp    (host side of the ops and their autograd; links libbptattn)
 
 hipcc cross-compiles for gfx950 without a GPU.  Run `python -m bpt_amd._build`.
 """
@@ -14,6 +15,7 @@ CSRC = os.path.join(os.path.dirname(os.path.abspath(__file__)), "csrc")
 GRAPH_SO = os.path.join(CSRC, "libbptgraph.so")
 ATTN_SO = os.path.join(CSRC, "libbptattn.so")
 PLAN_SO = os.path.join(CSRC, "libbptplan.so")
+OP_SO = os.path.join(CSRC, "bptop.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = [
@@ -56,8 +58,29 @@ def build_plan(verbose=True):
     return PLAN_SO
 
 
+def build_op(verbose=True):
+    """After build_attn, whose library it links (found beside it at run time)."""
+    import sysconfig
+    import torch
+    from torch.utils import cpp_extension
+    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    include = cpp_extension.include_paths() + [os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-DTORCH_EXTENSION_NAME=bptop",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM"]
+         + [f"-I{p}" for p in include] + [os.path.join(CSRC, "bptop.cpp"), "-o", OP_SO, f"-L{libs}", f"-L{CSRC}",
+                                          "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-ltorch", "-l:libbptattn.so", "-Wl,-rpath,$ORIGIN"], verbose)
+    return OP_SO
+
+
 def build_all(verbose=True):
-    return build_graph(verbose), build_attn(verbose), build_plan(verbose)
+    """The HIP compilations take most of the time and run side by side."""
+    from concurrent.futures import ThreadPoolExecutor
+    with ThreadPoolExecutor(2) as pool:
+        plan = pool.submit(build_plan, verbose)
+        graph, attn = build_graph(verbose), build_attn(verbose)
+        op = build_op(verbose)
+        return graph, attn, plan.result(), op
 
 
 if __name__ == "__main__":

@@ -1,0 +1,323 @@
+// bptop — the host side of a call whose plan is known, in native code: checks, plan lookup, allocation, launch, autograd.
+//
+// A step's kernels take 50 to 300 us, its Python host work took 220 (55 forward, 80 backward, the rest autograd and the hand-over
+// of the interpreter lock to autograd's thread and back): the GPU waited for the host in every case but the largest.  Here the
+// same work is some microseconds a call, and the backward runs on autograd's thread without the interpreter.
+//
+// Nothing is decided here.  bpt_amd/graphop.py chooses kernels and builds plans; each time it has done so it leaves what it
+// chose in the table below (`remember`), under the index tensors' addresses, sizes and versions, the shape and the type.  The
+// plan cache (bpt_amd/plan.py) keeps those index tensors and the plans alive, and drops an entry here when it drops a plan
+// (`forget`); changing a switch clears the table.  A call that is not in the table, or has an argument that a check refuses, goes to
+// the Python function, which raises, or builds, chooses and remembers.  Every call is checked anew.
+#include <torch/extension.h>
+
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+
+#include <array>
+#include <atomic>
+#include <cstring>
+#include <memory>
+#include <mutex>
+#include <optional>
+#include <unordered_map>
+#include <vector>
+
+#include "../../include/bptattn.h"
+
+namespace py = pybind11;
+using at::Tensor;
+
+namespace {
+
+enum Kind { ATTN_FWD = 0, ATTN_BWD = 1 };
+
+constexpr size_t MAX_TENSORS = 8, MAX_EXTRA = 6, MAX_ENTRIES = 512;
+
+struct Key {                          // compared and hashed as bytes: always zeroed first
+    int64_t kind, device;
+    std::array<int64_t, MAX_TENSORS> ptr, numel, version;
+    std::array<int64_t, MAX_EXTRA> extra;
+    bool operator==(const Key &o) const { return std::memcmp(this, &o, sizeof(Key)) == 0; }
+};
+static_assert(sizeof(Key) == 8 * (2 + 3 * MAX_TENSORS + MAX_EXTRA), "no padding");
+
+struct KeyHash {
+    size_t operator()(const Key &k) const {
+        const auto *w = reinterpret_cast<const uint64_t *>(&k);
+        uint64_t h = 0x9E3779B97F4A7C15ull;
+        for (size_t i = 0; i < sizeof(Key) / 8; ++i) {
+            h ^= w[i];
+            h *= 0xBF58476D1CE4E5B9ull;
+            h ^= h >> 29;
+        }
+        return (size_t)h;
+    }
+};
+
+struct Entry {
+    bpt_plan a{}, b{};
+    std::vector<PyObject *> plans;    // owned: what the structs point into lives as long as the entry
+    std::atomic<bool> used{false};
+    ~Entry() {
+        if (plans.empty() || !Py_IsInitialized()) return;
+        py::gil_scoped_acquire gil;
+        for (PyObject *p : plans) Py_DECREF(p);
+    }
+};
+using EntryPtr = std::shared_ptr<Entry>;
+
+std::mutex g_mutex;                   // never held while the interpreter lock is taken
+std::unordered_map<Key, EntryPtr, KeyHash> &table() {
+    static auto *t = new std::unordered_map<Key, EntryPtr, KeyHash>();       // (lives on: entries may outlast static destruction)
+    return *t;
+}
+
+EntryPtr find(const Key &k) {
+    std::lock_guard<std::mutex> lock(g_mutex);
+    auto it = table().find(k);
+    if (it == table().end()) return nullptr;
+    it->second->used.store(true, std::memory_order_relaxed);
+    return it->second;
+}
+
+int dtype_code(at::ScalarType t) { return t == at::kFloat ? BPT_F32 : t == at::kBFloat16 ? BPT_BF16 : t == at::kDouble ? BPT_F64 : -1; }
+
+bool index_ok(const Tensor &t, const at::Device &dev) {
+    return t.scalar_type() == at::kLong && t.dim() == 1 && t.is_cuda() && t.device() == dev && t.is_contiguous() && !t.is_inference();
+}
+
+bool like(const Tensor &t, const Tensor &q) {
+    return t.scalar_type() == q.scalar_type() && t.device() == q.device() && t.is_contiguous();
+}
+
+// false: an index tensor is not what the kernels take
+bool make_key(Key &k, Kind kind, const std::vector<const Tensor *> &index, const at::Device &dev, std::initializer_list<int64_t> extra) {
+    std::memset(static_cast<void *>(&k), 0, sizeof(Key));
+    k.kind = kind;
+    k.device = dev.index();
+    size_t i = 0;
+    for (const Tensor *t : index) {
+        if (!index_ok(*t, dev)) return false;
+        k.ptr[i] = reinterpret_cast<int64_t>(t->data_ptr());
+        k.numel[i] = t->numel();
+        k.version[i++] = (int64_t)t->_version();
+    }
+    i = 0;
+    for (int64_t x : extra) k.extra[i++] = x;
+    return true;
+}
+
+void *stream_of(const at::Device &dev) { return (void *)c10::hip::getCurrentHIPStream(dev.index()).stream(); }
+
+struct Workspace {
+    Tensor t;
+    void *ptr = nullptr;
+    int64_t bytes = 0;
+    Workspace(int op, const bpt_plan *a, const bpt_plan *b, int h, int d, int dt, const Tensor &like) {
+        bytes = bpt_workspace_bytes(op, a, b, h, d, dt);
+        if (bytes > 0) {
+            t = at::empty({bytes}, like.options().dtype(at::kByte));
+            ptr = t.data_ptr();
+        }
+    }
+};
+
+// ---- fused attention -------------------------------------------------------------------------------------------------------
+struct Shape {
+    int64_t nq, nk;
+    int h, d, dt;
+};
+
+bool attention_shape(const Tensor &q, const Tensor &k, const Tensor &v, double p, Shape &s) {
+    if (q.dim() != 3 || k.dim() != 3 || !q.is_cuda() || !q.is_contiguous() || !like(k, q) || !like(v, q)) return false;
+    if (k.size(1) != q.size(1) || k.size(2) != q.size(2) || v.sizes() != k.sizes() || !(p >= 0.0 && p < 1.0)) return false;
+    s = Shape{q.size(0), k.size(0), (int)q.size(1), (int)q.size(2), dtype_code(q.scalar_type())};
+    return s.dt >= 0;
+}
+
+std::optional<std::tuple<Tensor, Tensor>> attention_forward_known(const Tensor &col, const Tensor &indptr, const Tensor &eid, const Tensor &indices,
+                                                                  const Tensor &q, const Tensor &k, const Tensor &v, double scale, double p,
+                                                                  uint64_t seed) {
+    Shape s;
+    if (!attention_shape(q, k, v, p, s) || indices.sizes() != eid.sizes()) return std::nullopt;
+    Key key;
+    if (!make_key(key, ATTN_FWD, {&col, &indptr, &eid, &indices}, q.device(), {s.nq, s.nk, s.h, s.d, s.dt, p > 0.0})) return std::nullopt;
+    const EntryPtr e = find(key);
+    if (!e) return std::nullopt;
+    c10::DeviceGuard guard(q.device());
+    Tensor o = at::empty_like(q), lse = at::empty({s.nq, s.h}, q.options().dtype(at::kFloat));
+    Workspace ws(BPT_OP_ATTN_FWD, &e->a, nullptr, s.h, s.d, s.dt, q);
+    const int st = bpt_attention_forward(&e->a, q.data_ptr(), k.data_ptr(), v.data_ptr(), nullptr, o.data_ptr(), (float *)lse.data_ptr(), ws.ptr,
+                                         ws.bytes, (float)scale, (float)p, seed, s.h, s.d, s.dt, stream_of(q.device()));
+    if (st != BPT_OK) return std::nullopt;                   // (the Python function meets the same status and names it)
+    return std::make_tuple(o, lse);
+}
+
+using Three = std::tuple<Tensor, Tensor, Tensor>;
+
+std::optional<Three> attention_backward_known(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r, const Tensor &indices_r,
+                                              const Tensor &col, const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c,
+                                              const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &o, const Tensor &lse,
+                                              const Tensor &d_o, double scale, double p, uint64_t seed) {
+    Shape s;
+    if (!attention_shape(q, k, v, p, s) || !like(o, q) || !like(d_o, q) || o.sizes() != q.sizes() || d_o.sizes() != q.sizes()) return std::nullopt;
+    if (lse.scalar_type() != at::kFloat || lse.device() != q.device() || !lse.is_contiguous() || lse.dim() != 2 || lse.size(0) != s.nq ||
+        lse.size(1) != s.h)
+        return std::nullopt;
+    if (indices_c.sizes() != eid_c.sizes() || indices_r.sizes() != eid_r.sizes() || eid_r.sizes() != eid_c.sizes()) return std::nullopt;
+    Key key;
+    if (!make_key(key, ATTN_BWD, {&row, &indptr_r, &eid_r, &indices_r, &col, &indptr_c, &eid_c, &indices_c}, q.device(),
+                  {s.nq, s.nk, s.h, s.d, s.dt, p > 0.0}))
+        return std::nullopt;
+    const EntryPtr e = find(key);
+    if (!e) return std::nullopt;
+    c10::DeviceGuard guard(q.device());
+    Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+    Workspace ws(BPT_OP_ATTN_BWD, &e->a, &e->b, s.h, s.d, s.dt, q);
+    const int st = bpt_attention_backward(&e->a, &e->b, q.data_ptr(), k.data_ptr(), v.data_ptr(), nullptr, o.data_ptr(), d_o.data_ptr(),
+                                          (const float *)lse.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), nullptr, ws.ptr, ws.bytes,
+                                          (float)scale, (float)p, seed, s.h, s.d, s.dt, stream_of(q.device()));
+    if (st != BPT_OK) return std::nullopt;
+    return Three{dq, dk, dv};
+}
+
+py::object python(const char *name) { return py::module_::import("bpt_amd.graphop").attr(name); }
+
+// Python's exceptions leave autograd's thread as themselves
+template <typename F> auto with_python(F &&f) {
+    py::gil_scoped_acquire gil;
+    try {
+        return f();
+    } catch (py::error_already_set &e) {
+        e.restore();
+        python_error err;
+        err.persist();
+        throw std::move(err);
+    }
+}
+
+std::tuple<Tensor, Tensor> attention_forward(const Tensor &col, const Tensor &indptr, const Tensor &eid, const Tensor &indices, const Tensor &q,
+                                             const Tensor &k, const Tensor &v, double scale, double p, uint64_t seed) {
+    auto r = attention_forward_known(col, indptr, eid, indices, q, k, v, scale, p, seed);
+    if (!r) r = python("attention_forward")(col, indptr, eid, indices, q, k, v, scale, p, seed).cast<std::tuple<Tensor, Tensor>>();
+    return *r;
+}
+
+// (its forward runs with the interpreter lock held, its backward without)
+struct Attention : torch::autograd::Function<Attention> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r,
+                          const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c,
+                          const Tensor &q, const Tensor &k, const Tensor &v, double scale, double p, int64_t seed) {
+        const auto [o, lse] = attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale, p, (uint64_t)seed);
+        ctx->save_for_backward({row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, o, lse});
+        ctx->saved_data["scale"] = scale;
+        ctx->saved_data["p"] = p;
+        ctx->saved_data["seed"] = seed;
+        return o;
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        const auto t = ctx->get_saved_variables();
+        const double scale = ctx->saved_data["scale"].toDouble(), p = ctx->saved_data["p"].toDouble();
+        const uint64_t seed = (uint64_t)ctx->saved_data["seed"].toInt();
+        const Tensor d_o = grads[0].contiguous();
+        auto r = attention_backward_known(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], t[10], t[11], t[12], d_o, scale, p, seed);
+        if (!r)
+            r = with_python([&] {
+                return python("attention_backward")(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], t[10], t[11], t[12], d_o, scale, p,
+                                                    seed).template cast<Three>();
+            });
+        torch::autograd::variable_list out(14);
+        std::tie(out[8], out[9], out[10]) = *r;
+        return out;
+    }
+};
+
+// op.BPTAttention with the host work in native code: the same call, the same result
+Tensor attention(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r, const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c,
+                 const Tensor &eid_c, const Tensor &indices_c, const Tensor &q, const Tensor &k, const Tensor &v, double scale, double p, uint64_t seed) {
+    if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
+        return Attention::apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale, p, (int64_t)seed);
+    return std::get<0>(attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale, p, seed));
+}
+
+// ---- the table ---------------------------------------------------------------------------------------------------------------
+// `kind`'s choice for these index tensors and numbers: the bpt_plan structs at the addresses a and b (0: none), which point into
+// what `plans` holds.  True if it was taken.
+bool remember(int kind, const std::vector<Tensor> &index, const std::vector<int64_t> &extra, int64_t a, int64_t b, py::tuple plans) {
+    if (index.empty() || index.size() > MAX_TENSORS || extra.size() != MAX_EXTRA || !index[0].defined() || !index[0].is_cuda() || !a) return false;
+    std::vector<const Tensor *> ptrs;
+    for (const Tensor &t : index) ptrs.push_back(&t);
+    Key key;
+    if (!make_key(key, (Kind)kind, ptrs, index[0].device(), {extra[0], extra[1], extra[2], extra[3], extra[4], extra[5]})) return false;
+    auto e = std::make_shared<Entry>();
+    std::memcpy(&e->a, reinterpret_cast<const void *>(a), sizeof(bpt_plan));
+    if (b) std::memcpy(&e->b, reinterpret_cast<const void *>(b), sizeof(bpt_plan));
+    for (auto p : plans) e->plans.push_back(p.inc_ref().ptr());
+    e->used.store(true);
+    std::vector<EntryPtr> dropped;                           // (destroyed behind the lock)
+    {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        if (table().size() >= MAX_ENTRIES) {
+            for (auto &kv : table()) dropped.push_back(std::move(kv.second));
+            table().clear();
+        }
+        EntryPtr &slot = table()[key];
+        dropped.push_back(std::move(slot));
+        slot = e;
+    }
+    return true;
+}
+
+// drops what was chosen with this plan object
+void forget(py::object plan) {
+    std::vector<EntryPtr> dropped;
+    std::lock_guard<std::mutex> lock(g_mutex);
+    for (auto it = table().begin(); it != table().end();) {
+        bool hit = false;
+        for (PyObject *p : it->second->plans) hit = hit || p == plan.ptr();
+        if (hit) {
+            dropped.push_back(std::move(it->second));
+            it = table().erase(it);
+        } else {
+            ++it;
+        }
+    }
+}
+
+void clear() {
+    std::vector<EntryPtr> dropped;
+    std::lock_guard<std::mutex> lock(g_mutex);
+    for (auto &kv : table()) dropped.push_back(std::move(kv.second));
+    table().clear();
+}
+
+// the plan objects whose entries served a call since the last time this was asked
+std::vector<py::object> take_used() {
+    std::vector<EntryPtr> hit;
+    {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        for (auto &kv : table())
+            if (kv.second->used.exchange(false)) hit.push_back(kv.second);
+    }
+    std::vector<py::object> out;
+    for (auto &e : hit)
+        for (PyObject *p : e->plans) out.push_back(py::reinterpret_borrow<py::object>(p));
+    return out;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    m.attr("ATTN_FWD") = (int)ATTN_FWD;
+    m.attr("ATTN_BWD") = (int)ATTN_BWD;
+    m.def("attention", &attention);
+    m.def("attention_forward", &attention_forward_known);
+    m.def("attention_backward", &attention_backward_known);
+    m.def("remember", &remember);
+    m.def("forget", &forget);
+    m.def("clear", &clear);
+    m.def("take_used", &take_used);
+    m.def("plan_bytes", [] { return (int64_t)sizeof(bpt_plan); });
+}

@@ -14,18 +14,24 @@ import collections
 import contextlib
 import ctypes
 import math
+import sys
 import threading
 
 import torch
 
 from ._lib import BPT_ERR_UNSUPPORTED, BptStatusError, PlanStruct, attn_lib, check_attn
+from ._native import native as _native
 from . import plan as _plan
-from .plan import GROUP_ORDER_SRC, TILE_GROUP_R, plan_cache
+from .plan import GROUP_ORDER_SRC, TILE_GROUP_R, PlanCache, plan_cache
 
 __all__ = ["maskedmm_csr_forward", "maskedmm_csr_backward", "node_mul_edge_forward", "node_mul_edge_backward",
            "sparse_softmax_forward", "sparse_softmax_backward", "vector_spmm_forward", "vector_spmm_backward"]
 
 _LIB = attn_lib()          # fail at import time if the HIP library is missing
+if _native.plan_bytes() != ctypes.sizeof(PlanStruct):
+    raise ImportError("bptop was built for another bpt_plan: rebuild with `python -m bpt_amd._build`")
+PlanCache.native = _native
+sys.modules[__name__].__class__ = _plan._Switches
 
 
 class _Settings(collections.namedtuple("_Settings", "use_groups grouped_ops group_rows use_tiles")):
@@ -47,6 +53,7 @@ def _replace_setting(**kw):
     with _SETTINGS_LOCK:
         old = _SETTINGS
         _SETTINGS = old._replace(**kw)
+    _native.clear()                        # (what it serves was chosen under the old settings)
     return old
 
 _DTYPE = {torch.float32: 0, torch.float64: 1, torch.bfloat16: 2}
@@ -511,6 +518,11 @@ def attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale=None, drop
     id, or with bias_by_pair (h, E) with the edges in the order of the numbers attention_pair_rows() gives them (tile
     kernels only)."""
     cfg = _SETTINGS
+    if bias is None:
+        known = _native.attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, 1.0 / math.sqrt(q.size(-1)) if scale is None else float(scale),
+                                          float(dropout_p), int(seed) & (2 ** 64 - 1))
+        if known is not None:
+            return known
     _check_all(col=col, indptr_c=indptr_c, eid_c=eid_c, indices_c=indices_c, q=q, k=k, v=v)
     _check_bias(bias, eid_c.size(0), _hd(q)[0], q.device, cfg, bias_by_pair)
     _same_dtype(q, k, v)
@@ -529,11 +541,12 @@ def attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale=None, drop
     tiles = seg is not None
     if tiles:
         plan = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, None))
-        ref = ctypes.byref(plan.bias_rows(TILE_ROWS)["struct"] if bias_by_pair else plan.ensure_groups(TILE_ROWS)["struct"])
+        struct = plan.bias_rows(TILE_ROWS)["struct"] if bias_by_pair else plan.ensure_groups(TILE_ROWS)["struct"]
     elif not _attention_groups(plan, dropout_p, bias, q, k, cfg):
-        ref = plan.ref
+        struct = plan.struct
     else:
-        ref = ctypes.byref(plan.ensure_groups(_forward_rows(q, h, d, plan, cfg))["struct"])
+        struct = plan.ensure_groups(_forward_rows(q, h, d, plan, cfg))["struct"]
+    ref = ctypes.byref(struct)
     if bias_by_pair and not (tiles and bias is not None):
         raise RuntimeError("bias_by_pair: this call does not run on the tile kernels (ask attention_pair_rows() first)")
     o = torch.empty_like(q)
@@ -544,6 +557,9 @@ def attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale=None, drop
         check_attn(_LIB.bpt_attention_forward(ref, _ptr(q), _ptr(k), _ptr(v), _ptr(bias), _ptr(o), _ptr(lse), _ptr(ws), nws,
                                               scale, float(dropout_p), int(seed) & (2 ** 64 - 1), h, d, dt, _stream()),
                    "attention_forward")
+    if bias is None and cfg is _SETTINGS:
+        _native.remember(_native.ATTN_FWD, [col, indptr_c, eid_c, indices_c], [q.size(0), k.size(0), h, d, dt, int(dropout_p > 0.0)],
+                         ctypes.addressof(struct), 0, (plan,))
     return o, lse
 
 
@@ -553,9 +569,15 @@ def attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, in
     float32 (E, h), or (h, E) with bias_by_pair, the gradient with respect to q.k + bias of every edge and head (= the
     gradient of bias), laid out like bias."""
     cfg = _SETTINGS
+    do = do.contiguous()
+    if bias is None:
+        known = _native.attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, o, lse, do,
+                                           1.0 / math.sqrt(q.size(-1)) if scale is None else float(scale), float(dropout_p),
+                                           int(seed) & (2 ** 64 - 1))
+        if known is not None:
+            return known
     _check_all(row=row, indptr_r=indptr_r, eid_r=eid_r, indices_r=indices_r, col=col, indptr_c=indptr_c,
                eid_c=eid_c, indices_c=indices_c, q=q, k=k, v=v, o=o, lse=lse)
-    do = do.contiguous()
     _same_dtype(q, k, v, o, do)
     h, d = _hd(q)
     _expect_index(eid_c, indices_c)
@@ -582,8 +604,8 @@ def attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, in
         if not (pi.covers_all_edges and po.covers_all_edges):
             return None
         # the destination side writes (p, ds) by its own pair numbers; the source side finds them through its pair mapping
-        return (pi, po, ctypes.byref(pi.bias_rows(TILE_ROWS)["struct"] if bias_by_pair else pi.ensure_groups(TILE_ROWS)["struct"]),
-                ctypes.byref(po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True)))
+        return (pi, po, pi.bias_rows(TILE_ROWS)["struct"] if bias_by_pair else pi.ensure_groups(TILE_ROWS)["struct"],
+                po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True))
 
     # as in attention_forward: the tile plans straight away where the tile kernels are certain
     seg = _tile_seg_without_plan(col, eid_c.size(0), q, k, h, d, dropout_p, bias, cfg) if _tiles_backward(None, q.dtype, bias) else None
@@ -591,17 +613,18 @@ def attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, in
     if chosen is None:
         plan_in = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), prefer_device=on_gpu)
         plan_out = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), prefer_device=on_gpu)
-        in_ref, out_ref = plan_in.ref, plan_out.ref
+        in_struct, out_struct = plan_in.struct, plan_out.struct
         if _attention_groups(plan_in, dropout_p, bias, q, k, cfg) and plan_in.covers_all_edges and plan_out.covers_all_edges:
             if _tiles(q, h, d, plan_in, dropout_p, bias, cfg) and _tiles_backward(plan_in, q.dtype, bias):
                 chosen = tile_plans(_tile_seg_len(plan_in))
             else:
                 R = _group_rows(q, h, d, plan_in, cfg)
-                in_ref = ctypes.byref(plan_in.linked_to(plan_out, R))
-                out_ref = ctypes.byref(plan_out.ensure_groups(R, GROUP_ORDER_SRC)["struct"])
+                in_struct = plan_in.linked_to(plan_out, R)
+                out_struct = plan_out.ensure_groups(R, GROUP_ORDER_SRC)["struct"]
     tiles = chosen is not None
     if tiles:
-        plan_in, plan_out, in_ref, out_ref = chosen
+        plan_in, plan_out, in_struct, out_struct = chosen
+    in_ref, out_ref = ctypes.byref(in_struct), ctypes.byref(out_struct)
     if bias_by_pair and not (tiles and bias is not None):
         raise RuntimeError("bias_by_pair: this call does not run on the tile kernels (ask attention_pair_rows() first)")
     ws, nws = _workspace(OP_ATTN_BWD, plan_in, plan_out, h, d, dt, q.device, plan_ref=in_ref, plan_t_ref=out_ref)
@@ -612,6 +635,10 @@ def attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, in
                    "attention_backward")
     if bias is not None:
         return dq, dk, dv, ds if bias_by_pair else ds[:-1]
+    if cfg is _SETTINGS:
+        _native.remember(_native.ATTN_BWD, [row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c],
+                         [q.size(0), k.size(0), h, d, dt, int(dropout_p > 0.0)], ctypes.addressof(in_struct), ctypes.addressof(out_struct),
+                         (plan_in, plan_out))
     return dq, dk, dv
 
 

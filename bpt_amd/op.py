@@ -8,6 +8,7 @@ import torch
 from torch.autograd import Function
 
 from . import graphop as _g
+from ._native import native as _native
 from .graphop import (maskedmm_csr_backward, maskedmm_csr_forward, node_mul_edge_backward, node_mul_edge_forward,
                       sparse_softmax_backward, sparse_softmax_forward, vector_spmm_backward, vector_spmm_forward)
 
@@ -314,9 +315,14 @@ def bpt_attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices
         h, d = q.size(1), q.size(2)
         hp, dp = padded
         grow = lambda x: torch.nn.functional.pad(x, (0, dp - d, 0, hp - h))
-        o = bpt_attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, grow(q), grow(k), grow(v), scale=scale,
-                          fused=True, dropout_p=dropout_p, seed=seed,
-                          rel_table=None if rel_table is None else torch.nn.functional.pad(rel_table, (0, dp - d)), etype=etype)
+        if dropout_p > 0 and seed is None:
+            seed = int(torch.randint(0, 2 ** 62, (1,)).item())
+        graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
+        if rel_table is None:
+            o = BPTAttention.apply(*graph, grow(q), grow(k), grow(v), scale, float(dropout_p), int(seed or 0))
+        else:
+            o = BPTRelAttention.apply(*graph, grow(q), grow(k), grow(v), scale, float(dropout_p), int(seed or 0),
+                                      torch.nn.functional.pad(rel_table, (0, dp - d)), etype)
         return o[:, :h, :d].contiguous()
     if fused:
         if dropout_p > 0 and seed is None:
@@ -324,8 +330,8 @@ def bpt_attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices
         if rel_table is not None:
             return BPTRelAttention.apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale,
                                          float(dropout_p), int(seed or 0), rel_table, etype)
-        return BPTAttention.apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale,
-                                  float(dropout_p), int(seed or 0))
+        return _native.attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale, float(dropout_p),
+                                 int(seed or 0) & (2 ** 64 - 1))
     e = masked_mm(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, k, q)
     if rel_table is not None:
         e = e + node_mul_edge(col, indptr_c, eid_c, q, edge_type_embedding(rel_table, etype))

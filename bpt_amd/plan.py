@@ -9,7 +9,9 @@ layers, forward and backward) hit the cache.  The cache keeps the key tensors al
 """
 import collections
 import ctypes
+import sys
 import threading
+import types
 
 import numpy as np
 import torch
@@ -214,12 +216,13 @@ class Plan:
     def device_bytes(self):
         """Device memory held by this plan, its row groups and pair mappings (added up again when one of those was added: the cache
         asks every plan it holds whenever a graph is new, which cost 1.1 ms a step with 64 plans of a new graph each)."""
-        parts = (len(self._groups), len(self._links), len(self._bias_rows))
-        if self._bytes is None or self._bytes[0] != parts:
+        parts = len(self._groups) + len(self._links) + len(self._bias_rows)
+        held = self._bytes
+        if held is None or held[0] != parts:
             with self._lock:
-                held = [list(x.values()) for x in (self._groups, self._links, self._bias_rows)]
-            self._bytes = (parts, _tensor_bytes(self._dev) + sum(_tensor_bytes(x) for x in held))
-        return self._bytes[1]
+                values = [list(x.values()) for x in (self._groups, self._links, self._bias_rows)]
+            held = self._bytes = (parts, _tensor_bytes(self._dev) + sum(_tensor_bytes(x) for x in values))
+        return held[1]
 
     _bytes = None
 
@@ -355,6 +358,8 @@ def set_device_build(on):
     degree of DEVICE_BUILD_MIN_DEGREE and DEVICE_BUILD_DENSE_MIN_ROWS rows).  Returns the old setting."""
     global DEVICE_BUILD
     old, DEVICE_BUILD = DEVICE_BUILD, (None if on is None else bool(on))
+    if PlanCache.native is not None:
+        PlanCache.native.clear()
     return old
 
 
@@ -674,15 +679,25 @@ class PlanCache:
         with self._lock:
             return sum(p.device_bytes() + _tensor_bytes(list(t for t in ts if t is not None and t.is_cuda)) for p, ts in self._d.values())
 
+    # the native host path (bpt_amd/_native.py), set by bpt_amd/graphop.py: it serves calls from what was chosen with a plan, so
+    # it says which plans it used when one has to go, and is told which one went
+    native = None
+
     def _evict(self):
         # called with the lock held; the newest entry always stays
-        while len(self._d) > self._cap:
-            self._d.popitem(last=False)
-        if len(self._d) > 1:
-            total = sum(p.device_bytes() for p, _ in self._d.values())
-            while len(self._d) > 1 and total > self._max_bytes:
-                _, (p, _) = self._d.popitem(last=False)
-                total -= p.device_bytes()
+        total = sum(p.device_bytes() for p, _ in self._d.values()) if len(self._d) > 1 else 0
+        if len(self._d) <= self._cap and total <= self._max_bytes:
+            return
+        if self.native is not None and len(self._d) > 1:
+            newest = next(reversed(self._d))
+            used = {id(p) for p in self.native.take_used()}
+            for key in [k for k, (p, _) in self._d.items() if id(p) in used] + [newest]:
+                self._d.move_to_end(key)
+        while len(self._d) > max(self._cap, 1) or (len(self._d) > 1 and total > self._max_bytes):
+            _, (p, _) = self._d.popitem(last=False)
+            total -= p.device_bytes()
+            if self.native is not None:
+                self.native.forget(p)
 
     @staticmethod
     def _key(tensors, n_rows, n_index, seg_len, on_device):
@@ -723,6 +738,8 @@ class PlanCache:
     def clear(self):
         with self._lock:
             self._d.clear()
+            if self.native is not None:
+                self.native.clear()
 
     def held(self):
         """The plans in the cache right now (with the index tensors they were built from), as a list the caller keeps.
@@ -734,3 +751,16 @@ class PlanCache:
 
 
 plan_cache = PlanCache()
+
+
+class _Switches(types.ModuleType):
+    """This module and graphop: an assignment to one of their upper-case switches from outside (tests, measurements) also clears
+    what the native host path keeps of earlier choices."""
+
+    def __setattr__(self, name, value):
+        super().__setattr__(name, value)
+        if name.lstrip("_").isupper() and PlanCache.native is not None:
+            PlanCache.native.clear()
+
+
+sys.modules[__name__].__class__ = _Switches

@@ -1,0 +1,116 @@
+"""The native host path (bpt_amd/csrc/bptop.cpp): a call served from its table gives the bits of the call that was remembered, a
+changed or dropped plan is not served, refused arguments raise as before, threads with streams of their own agree."""
+import threading
+
+import numpy as np
+import pytest
+import torch
+
+from test_gpu_parity import DEV, Case, rand
+
+pytestmark = pytest.mark.gpu
+
+
+def args_of(c):
+    return (*c.out, *c.inn)
+
+
+def step(op, args, q, k, v, do, p=0.0):
+    q, k, v = (x.detach().requires_grad_(True) for x in (q, k, v))
+    o = op.bpt_attention(*args, q, k, v, dropout_p=p, seed=7)
+    return (o.detach(), *torch.autograd.grad(o, (q, k, v), do))
+
+
+def node_tensors(n, dtype=torch.float32, h=8):
+    return tuple(rand((n, h, 64), dtype, s, 1.0 / 8).to(DEV) for s in (1, 2, 3, 4))
+
+
+def same(a, b):
+    return all(torch.equal(x, y) for x, y in zip(a, b))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("p", [0.0, 0.1])
+@pytest.mark.parametrize("gname", ["bpt512_k4", "multigraph"])
+def test_served_calls_equal_the_remembered_one(gname, dtype, p):
+    from bpt_amd import op, plan
+    c = Case(gname)
+    x = node_tensors(c.n, dtype)
+    plan.plan_cache.clear()
+    first = step(op, args_of(c), *x, p)
+    assert plan.PlanCache.native.take_used()
+    assert same(first, step(op, args_of(c), *x, p))
+    assert plan.PlanCache.native.take_used(), "the second call was not served natively"
+    with torch.no_grad():
+        assert torch.equal(first[0], op.bpt_attention(*args_of(c), *x[:3], dropout_p=p, seed=7))
+    plan.plan_cache.clear()
+    assert not plan.PlanCache.native.take_used()
+    assert same(first, step(op, args_of(c), *x, p))
+
+
+def test_changed_graphs_and_dropped_plans_are_not_served():
+    from bpt_amd import op, plan
+    c = Case("bpt512_k4")
+    x = node_tensors(c.n)
+    args = [t.clone() for t in args_of(c)]
+    first = step(op, args, *x)
+    assert same(first, step(op, args, *x))
+    # other neighbours, written into the same memory: every edge's source moved by one node, on both sides
+    src, dst = (np.asarray(c.src) + 1) % c.n, np.asarray(c.dst)
+    from bpt_amd import graphbuilder as gb
+    out_csr, in_csr, ROW, IR, COL, IC = gb.get_csrs(src, dst, c.n)
+    args[7].copy_(in_csr[1].to(DEV))                       # the in-CSR's shape is the same, its columns are not
+    moved = (ROW, IR, out_csr[2], out_csr[1])
+    args[:4] = [t.to(DEV) for t in moved]
+    fresh = [t.clone() for t in args]
+    changed = step(op, args, *x)
+    assert not torch.equal(changed[0], first[0])
+    assert same(changed, step(op, fresh, *x))
+    # a cache of one plan drops one of the two sides all the time
+    old = plan.plan_cache.set_limits(capacity=1)
+    try:
+        assert same(changed, step(op, args, *x)) and same(changed, step(op, args, *x))
+        assert len(plan.plan_cache._d) == 1
+    finally:
+        plan.plan_cache.set_limits(*old)
+
+
+def test_a_known_graph_still_refuses_wrong_arguments():
+    from bpt_amd import graphop, op
+    c = Case("bpt512_k4")
+    q, k, v, do = node_tensors(c.n)
+    step(op, args_of(c), q, k, v, do)
+    for bad in ((q, k[:, :, :32].contiguous(), v), (q, k, v[:-1].contiguous()), (q, k.bfloat16(), v), (q, k.transpose(0, 1).contiguous().transpose(0, 1), v),
+                (q, k.cpu(), v)):
+        with pytest.raises((ValueError, RuntimeError)):
+            op.bpt_attention(*args_of(c), *bad)
+    with pytest.raises((ValueError, RuntimeError)):
+        graphop.attention_forward(*c.inn[:3], c.inn[3][:-1].contiguous(), q, k, v)
+    o, lse = graphop.attention_forward(*c.inn, q, k, v)
+    with pytest.raises(ValueError):
+        graphop.attention_backward(*c.out, *c.inn, q, k, v, o, lse[:-1].contiguous(), do)
+
+
+def test_threads_and_streams():
+    from bpt_amd import op
+    c = Case("bpt512_k4")
+    x = node_tensors(c.n)
+    want = step(op, args_of(c), *x)
+    torch.cuda.synchronize()
+    failures = []
+
+    def work():
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                got = step(op, args_of(c), *x)
+                stream.synchronize()
+                if not same(want, got):
+                    failures.append(1)
+
+    threads = [threading.Thread(target=work) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failures
