@@ -72,6 +72,10 @@ ATTN_API = {
                                                     ctypes.c_uint64] + _tail),
     "bpt_attention_backward": (ctypes.c_int, [_PP, _PP, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp,
                                              c_i64, ctypes.c_float, ctypes.c_float, ctypes.c_uint64] + _tail),
+    "bpt_attention_forward_narrow": (ctypes.c_int, [_PP, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, ctypes.c_float, ctypes.c_float,
+                                                   ctypes.c_uint64, ctypes.c_int] + _tail),
+    "bpt_attention_backward_narrow": (ctypes.c_int, [_PP, _PP, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64,
+                                                    ctypes.c_float, ctypes.c_float, ctypes.c_uint64, ctypes.c_int] + _tail),
 }
 
 c_i32 = ctypes.c_int32

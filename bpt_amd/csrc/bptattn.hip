@@ -187,6 +187,25 @@ __global__ __launch_bounds__(BLOCK) void k_spmm_generic(bpt_plan P, const T *__r
     }
 }
 
+// Heads of fewer than 64 columns (6 x 50, 8 x 40), read and written as they are in memory by the NARROW forms of the tile kernels.
+// The products keep their 64 columns: quad j of a head (the four columns a lane group position stands for) starts at column
+// 4 j, or at d - 4 where that would run over the end of the head.  What a shifted quad repeats of its neighbour, and the quads past
+// the end, count for nothing because the member's operand is zero there (tile_load16, tile_load_row_bf16); results are
+// stored from the quads that start inside the head, a repeated column twice with one value.  No other head's memory is
+// touched, so what stands there does not matter.
+// Against copies padded to 64 columns and 4, 8 or 16 heads (three pads, the output and its gradient, three slices, and the
+// padding heads computed with the rest): 33 765 nodes / 576 k edges at 6 x 50 with dropout, forward and backward,
+// 508 -> 207 us; of that copies 223, the rest two padding heads of eight.
+struct Narrow {
+    int d, heads;              // columns of a head, heads
+    int h;                     // heads the layer is padded to where that shows: dropout keys, lse and workspace rows
+    int slices;                // workgroups per group
+};
+constexpr int NARROW_HW = 2;   // heads per workgroup (6 x 50: three workgroups of two, none of them half empty)
+__device__ __forceinline__ int narrow_col(const Narrow &nw, int quad) { return min(4 * quad, nw.d - 4); }
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));           // such rows start anywhere on 4 bytes
+typedef uint32_t uintx2u __attribute__((ext_vector_type(2), aligned(4)));
+
 // Y[row, :] = sum of the row's partial slots.  Grid (n_heavy, ceil(C / 64), n_out): one block per split
 // row, 64-column strip and output tensor (output z reads its partials n_slots*C further into the
 // workspace).  Wave w adds slots w, w+4, ... (eight independent loads per step); the four wave sums
@@ -246,9 +265,9 @@ template <> __device__ __forceinline__ float4 load4<bf16_t>(const bf16_t *p) {
     const uint2 x = *reinterpret_cast<const uint2 *>(p);
     return make_float4(__uint_as_float(x.x << 16), __uint_as_float(x.x & 0xffff0000u), __uint_as_float(x.y << 16), __uint_as_float(x.y & 0xffff0000u));
 }
-template <typename T>
+template <typename T, bool NARROW = false>
 __device__ __forceinline__ void combine_sum_block4(const int32_t *__restrict__ hv, const float *__restrict__ ws, T *__restrict__ Y, int C,
-                                                   bool accumulate = false, int strip = -1) {
+                                                   bool accumulate = false, int strip = -1, const Narrow &nw = Narrow{}) {
     __shared__ float4 part[WAVES_PER_BLOCK][WAVE];
     const int row = hv[0], s0 = hv[1], ns = hv[2];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -273,6 +292,14 @@ __device__ __forceinline__ void combine_sum_block4(const int32_t *__restrict__ h
         float4 r = part[0][lane];
 #pragma unroll
         for (int i = 1; i < WAVES_PER_BLOCK; ++i) { r.x += part[i][lane].x; r.y += part[i][lane].y; r.z += part[i][lane].z; r.w += part[i][lane].w; }
+        if constexpr (NARROW) {                                   // 64 columns of the partials per head, d of the result
+            const int head = j >> 6, col = j & 63;
+            T *const at = Y + (size_t)row * (nw.heads * nw.d) + head * nw.d + col;
+            const float x[4] = {r.x, r.y, r.z, r.w};
+            for (int e = 0; e < 4; ++e)
+                if (head < nw.heads && col + e < nw.d) Elem<T>::st(at + e, x[e]);
+            return;
+        }
         if (accumulate) {
             const float4 y = load4<T>(Y + (size_t)row * C + j);
             r.x += y.x; r.y += y.y; r.z += y.z; r.w += y.w;
@@ -280,15 +307,16 @@ __device__ __forceinline__ void combine_sum_block4(const int32_t *__restrict__ h
         store4<T>(Y + (size_t)row * C + j, r);
     }
 }
-template <typename T>
+template <typename T, bool NARROW = false>
 __global__ __launch_bounds__(BLOCK) void k_combine_sum3(const int32_t *__restrict__ heavy_a, int n_a, const float *__restrict__ ws_a,
                                                            T *__restrict__ YA, const int32_t *__restrict__ heavy_b,
                                                            const float *__restrict__ ws_b, T *__restrict__ YB0, T *__restrict__ YB1, int C,
-                                                           size_t ws_stride_b) {
+                                                           size_t ws_stride_b, Narrow nw) {
     if ((int)blockIdx.x < n_a) {
-        if (blockIdx.z == 0) combine_sum_block4<T>(heavy_a + 3 * blockIdx.x, ws_a, YA, C);
+        if (blockIdx.z == 0) combine_sum_block4<T, NARROW>(heavy_a + 3 * blockIdx.x, ws_a, YA, C, false, -1, nw);
     } else {
-        combine_sum_block4<T>(heavy_b + 3 * (blockIdx.x - n_a), ws_b + (size_t)blockIdx.z * ws_stride_b, blockIdx.z == 0 ? YB0 : YB1, C);
+        combine_sum_block4<T, NARROW>(heavy_b + 3 * (blockIdx.x - n_a), ws_b + (size_t)blockIdx.z * ws_stride_b, blockIdx.z == 0 ? YB0 : YB1, C,
+                                      false, -1, nw);
     }
 }
 
@@ -918,11 +946,12 @@ __global__ __launch_bounds__(BLOCK) void k_attn_fwd(bpt_plan P, const T *__restr
 // Combine the (m, l, acc) partials of each split row.  Grid (n_heavy, C / 64): one block per split row
 // and 64-column strip; wave w folds slots w, w+4, ... with a running maximum (one pass, eight
 // independent loads per step), then the four wave results are merged in wave order.
-template <typename T, int H, int D>
+template <typename T, int HC, int D, bool NARROW = false>
 __global__ __launch_bounds__(BLOCK) void k_attn_fwd_combine(const int32_t *__restrict__ heavy, const float *__restrict__ ws_acc,
-                                                            const float *__restrict__ ws_ml, T *__restrict__ o, float *__restrict__ lse) {
-    constexpr int C = H * D;
-    static_assert(C % WAVE == 0, "strip width");
+                                                            const float *__restrict__ ws_ml, T *__restrict__ o, float *__restrict__ lse,
+                                                            Narrow nw) {
+    static_assert(HC * D % WAVE == 0, "strip width");
+    const int H = NARROW ? nw.h : HC, C = H * D;                 // (NARROW: one strip per real head)
     __shared__ float pm[WAVES_PER_BLOCK][WAVE], pl[WAVES_PER_BLOCK][WAVE], pa[WAVES_PER_BLOCK][WAVE];
     const int row = heavy[3 * blockIdx.x], s0 = heavy[3 * blockIdx.x + 1], ns = heavy[3 * blockIdx.x + 2];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -974,7 +1003,8 @@ __global__ __launch_bounds__(BLOCK) void k_attn_fwd_combine(const int32_t *__res
             L = fmaf(pl[i][lane], wgt, L);
             A = fmaf(pa[i][lane], wgt, A);
         }
-        Elem<T>::st(o + (size_t)row * C + j, L > 0.f ? A / L : 0.f);
+        if (!NARROW) Elem<T>::st(o + (size_t)row * C + j, L > 0.f ? A / L : 0.f);
+        else if (lane < nw.d) Elem<T>::st(o + (size_t)row * (nw.heads * nw.d) + head * nw.d + lane, L > 0.f ? A / L : 0.f);
         if (j % D == 0) lse[(size_t)row * H + head] = L > 0.f ? Mx + log2f(L) : 0.f;
     }
 }
@@ -1677,21 +1707,27 @@ struct TileCtx {
                                  // products that contract over columns, + 64 t bytes per step), and its columns 4 c .. 4 c + 3
 };
 
-template <typename T, int H, int D, int HW>
-__device__ __forceinline__ bool tile_begin(const bpt_plan &P, TileCtx &t) {
+template <typename T, int H, int D, int HW, bool NARROW = false>
+__device__ __forceinline__ bool tile_begin(const bpt_plan &P, TileCtx &t, const Narrow &nw) {
     static_assert(D == 64 && H % HW == 0 && (sizeof(T) == 4 || sizeof(T) == 2), "64 columns per head: one 16-column slice per lane group");
-    constexpr int HS = H / HW;
+    const int HS = NARROW ? nw.slices : H / HW;
     t.lane = threadIdx.x & (WAVE - 1);
     t.wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     t.c = t.lane & 15;
     t.g = t.lane >> 4;
-    const int x = blockIdx.x & 7, w = (blockIdx.x >> 3) / HS;
+    const int x = blockIdx.x & 7, w = (int)(blockIdx.x >> 3) / HS;
     const int grp = __builtin_amdgcn_readfirstlane(P.grp_chunks[x]) + w;
     if (grp >= __builtin_amdgcn_readfirstlane(P.grp_chunks[x + 1])) return false;
     t.member = reinterpret_cast<const int2 *>(P.grp_members)[(size_t)grp * TILE_R + t.c];
     t.p_begin = __builtin_amdgcn_readfirstlane(P.grp_ptr[grp]);
     t.p_end = __builtin_amdgcn_readfirstlane(P.grp_ptr[grp + 1]);
     t.head = (int)((blockIdx.x >> 3) % HS) * HW + t.wv;
+    if (NARROW) {
+        if (t.head >= nw.heads) return false;
+        t.offa = (uint32_t)(t.head * nw.d * sizeof(T));
+        t.offv = (uint32_t)((t.head * nw.d + narrow_col(nw, t.c)) * sizeof(T));
+        return true;
+    }
     t.offa = (uint32_t)((t.head * D + 4 * t.g) * sizeof(T));
     t.offv = (uint32_t)((t.head * D + 4 * t.c) * sizeof(T));
     return true;
@@ -1731,11 +1767,28 @@ __device__ __forceinline__ void tile_stage_entries(const bpt_plan &P, int2 *lds,
 __device__ __forceinline__ int tile_pair_number(int first, int mask, int c) { return first + __popc((uint32_t)mask & ((1u << c) - 1u)); }
 
 // this lane's 16 columns of a node row (bytes offa + 64 t), as the A or B operand of a product over columns
-__device__ __forceinline__ void tile_load16(const char *row, float (&out)[16]) {
+template <bool NARROW>
+__device__ __forceinline__ void tile_load16(const char *row, float (&out)[16], int g, const Narrow &nw) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-        const float4 x = *reinterpret_cast<const float4 *>(row + 64 * t);
-        out[4 * t] = x.x; out[4 * t + 1] = x.y; out[4 * t + 2] = x.z; out[4 * t + 3] = x.w;
+        if constexpr (NARROW) {
+            const int quad = 4 * (4 * t + g), col = min(quad, nw.d - 4);
+            const floatx4u x = *reinterpret_cast<const floatx4u *>(row + 4 * col);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[4 * t + e] = col + e >= quad ? x[e] : 0.f;
+        } else {
+            const float4 x = *reinterpret_cast<const float4 *>(row + 64 * t);
+            out[4 * t] = x.x; out[4 * t + 1] = x.y; out[4 * t + 2] = x.z; out[4 * t + 3] = x.w;
+        }
+    }
+}
+// this lane's four columns of an entry's row
+template <bool NARROW> __device__ __forceinline__ float4 tile_row4(const char *p) {
+    if constexpr (NARROW) {
+        const floatx4u x = *reinterpret_cast<const floatx4u *>(p);
+        return make_float4(x[0], x[1], x[2], x[3]);
+    } else {
+        return *reinterpret_cast<const float4 *>(p);
     }
 }
 
@@ -1772,28 +1825,33 @@ __device__ __forceinline__ void tile_axpy_upto(const float (&w)[4], const float4
 
 // The members' result rows: whole rows go to `out` (scaled by inv[member] where given), segments of split rows to the
 // workspace in natural column order.
-template <int H, int D, bool SCALE, typename T>
+template <int H, int D, bool SCALE, bool NARROW, typename T>
 __device__ __forceinline__ void tile_store_rows(const TileCtx &t, const floatx4v (&acc)[4], float inv_c, T *__restrict__ out,
-                                                float *__restrict__ ws) {
-    constexpr int C = H * D;
+                                                float *__restrict__ ws, const Narrow &nw) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int m = 4 * t.g + r;                                // the member whose row this lane stores a piece of
         const int row = lane_bcast(t.member.x, m), slot = lane_bcast(t.member.y, m);
         const float inv = SCALE ? lane_bcast(inv_c, m) : 1.f;
-        if (row < 0) continue;
+        if (row < 0 || (NARROW && 4 * t.c >= nw.d)) continue;
         float4 x = make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]);
+        const int col = NARROW ? narrow_col(nw, t.c) : 4 * t.c;
         if (slot < 0) {
             if (SCALE) { x.x *= inv; x.y *= inv; x.z *= inv; x.w *= inv; }
+            T *const at = NARROW ? out + (size_t)row * (uint32_t)(nw.heads * nw.d) + t.head * nw.d + col : out + (size_t)row * (H * D) + t.head * D + col;
             if constexpr (sizeof(T) == 4) {
-                *reinterpret_cast<float4 *>(out + (size_t)row * C + t.head * D + 4 * t.c) = x;
+                if constexpr (NARROW) *reinterpret_cast<floatx4u *>(at) = floatx4u{x.x, x.y, x.z, x.w};
+                else *reinterpret_cast<float4 *>(at) = x;
             } else {
                 const uint2 y = make_uint2(((uint32_t)f32_to_bf16(x.x)) | ((uint32_t)f32_to_bf16(x.y) << 16),
                                ((uint32_t)f32_to_bf16(x.z)) | ((uint32_t)f32_to_bf16(x.w) << 16));
-                *reinterpret_cast<uint2 *>(out + (size_t)row * C + t.head * D + 4 * t.c) = y;
+                if constexpr (NARROW) *reinterpret_cast<uintx2u *>(at) = uintx2u{y.x, y.y};
+                else *reinterpret_cast<uint2 *>(at) = y;
             }
         } else {
-            *reinterpret_cast<float4 *>(ws + (size_t)slot * C + t.head * D + 4 * t.c) = x;
+            float *const at = ws + (size_t)slot * (NARROW ? nw.h * D : H * D) + t.head * D + col;
+            if constexpr (NARROW) *reinterpret_cast<floatx4u *>(at) = floatx4u{x.x, x.y, x.z, x.w};
+            else *reinterpret_cast<float4 *>(at) = x;
         }
     }
 }
@@ -1910,14 +1968,15 @@ __device__ __forceinline__ void tile_walk_first_ahead(int nblk, IssueFirst &&fir
     issue_loads_first();
 }
 
-template <typename T, int H, int D, int HW, bool PIPE, bool DROP, int BIAS>
+template <typename T, int H, int D, int HW, bool PIPE, bool DROP, int BIAS, bool NARROW = false>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE ? 3 : 4))) void k_attn_fwd_tile(
     bpt_plan P, const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v, T *__restrict__ o, float *__restrict__ lse,
     float *__restrict__ ws_acc, float *__restrict__ ws_ml, float scale_log2e, uint32_t drop_thr, uint32_t drop_seed, float drop_inv,
-    const float *__restrict__ bias) {
-    constexpr int C = H * D;
+    const float *__restrict__ bias, Narrow nw) {
+    const int Hs = NARROW ? nw.h : H;                             // heads as lse, workspace and dropout keys count them
+    const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * sizeof(T) : (uint32_t)(H * D * sizeof(T));        // bytes of a node row
     TileCtx t;
-    if (!tile_begin<T, H, D, HW>(P, t)) return;
+    if (!tile_begin<T, H, D, HW, NARROW>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     __shared__ int fst_lds[HW][BIAS == 2 ? TILE_CHUNK : 1];      // the entries' first pair numbers: where a term in pair order sits
     int2 *ent = ent_lds[t.wv];
@@ -1933,9 +1992,9 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
     // The members' q rows are asked for behind the first block's K rows: asked for here, ahead of the loop, they are waited
     // for before the entry list is (one more round trip in front of the K rows).  They stay as they are and the scores are
     // scaled instead, so nothing has to happen to them between their arrival and the first product.
-    const char *const qrow = reinterpret_cast<const char *>(q) + (size_t)max(t.member.x, 0) * (C * sizeof(T)) + t.offa;
+    const char *const qrow = reinterpret_cast<const char *>(q) + (size_t)max(t.member.x, 0) * RB + t.offa;
     constexpr bool AHEAD = !PIPE && !DROP && BIAS == 0;         // (with dropout or the score term the sixteen registers are not there)
-    if constexpr (!AHEAD) tile_load16(qrow, qb);
+    if constexpr (!AHEAD) tile_load16<NARROW>(qrow, qb, g, nw);
     floatx4v acc[4];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
@@ -1954,7 +2013,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
         auto issue_k = [&](Blk &B, int b) {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                B.kq[r] = *reinterpret_cast<const float4 *>(kb + ((uint32_t)ent[TILE_R * b + 4 * r + g].x * (uint32_t)(C * sizeof(T)) + t.offv));
+                B.kq[r] = tile_row4<NARROW>(kb + ((uint32_t)ent[TILE_R * b + 4 * r + g].x * RB + t.offv));
         };
         auto issue_rest = [&](Blk &B, int b) {
             if constexpr (DROP || BIAS == 1) tile_pair_eids(P, p0 + TILE_R * b + g, t.p_end, c, B.xe, 4);
@@ -1968,7 +2027,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
             B.has = ((mk[0] >> c) & 1) | (((mk[1] >> c) & 1) << 1) | (((mk[2] >> c) & 1) << 2) | (((mk[3] >> c) & 1) << 3);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                B.vr[r] = *reinterpret_cast<const float4 *>(vb + ((uint32_t)idxv[r] * (uint32_t)(C * sizeof(T)) + t.offv));
+                B.vr[r] = tile_row4<NARROW>(vb + ((uint32_t)idxv[r] * RB + t.offv));
             if constexpr (BIAS == 1) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, 1>(P, t.head, B.xe[BIAS == 1 ? r : 0], 0)];
@@ -2008,24 +2067,24 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
                 pr[r] = __builtin_amdgcn_exp2f(sc[r] - mref);
                 lrun += pr[r];                                   // the softmax denominator ignores dropout
                 if constexpr (DROP)
-                    pr[r] *= dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)H + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
+                    pr[r] *= dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)Hs + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
             }
             tile_axpy_upto(pr, B.vr, acc, B.nv);
         };
         auto issue = [&](Blk &B, int b) { issue_k(B, b); issue_rest(B, b); };
         if constexpr (!AHEAD) tile_walk<PIPE, Blk>(nblk, issue, compute);
-        else tile_walk_first_ahead<Blk>(nblk, issue_k, issue_rest, compute, [&]() { if (p0 == t.p_begin) tile_load16(qrow, qb); });
+        else tile_walk_first_ahead<Blk>(nblk, issue_k, issue_rest, compute, [&]() { if (p0 == t.p_begin) tile_load16<NARROW>(qrow, qb, g, nw); });
         wave_lds_fence();                                         // the piece is read to the end before the next one is staged
     }
     float lt = lrun + __shfl_xor(lrun, 16);
     lt += __shfl_xor(lt, 32);                                    // denominator of member c, in its four lanes
-    tile_store_rows<H, D, true>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc);
+    tile_store_rows<H, D, true, NARROW>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc, nw);
     if (g == 0 && t.member.x >= 0) {                              // lanes 0 .. 15: one member each
         if (t.member.y < 0) {
-            lse[(size_t)t.member.x * H + t.head] = lt > 0.f ? mref + log2f(lt) : 0.f;
+            lse[(size_t)t.member.x * Hs + t.head] = lt > 0.f ? mref + log2f(lt) : 0.f;
         } else {
-            ws_ml[((size_t)t.member.y * H + t.head) * 2] = mref;
-            ws_ml[((size_t)t.member.y * H + t.head) * 2 + 1] = lt;
+            ws_ml[((size_t)t.member.y * Hs + t.head) * 2] = mref;
+            ws_ml[((size_t)t.member.y * Hs + t.head) * 2 + 1] = lt;
         }
     }
 }
@@ -2042,15 +2101,16 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
 // source side's layout instead (scattered 8-byte stores here, contiguous reads there) cost this kernel a third of its
 // time (126 against 85 us at L = 4096, k = 32); letting the source side recompute p and ds (two more products there,
 // delta (n, H) handed over) measured slower than either on every graph tried.
-template <typename T, int H, int D, int HW, bool PIPE, bool DROP, int BIAS>
+template <typename T, int H, int D, int HW, bool PIPE, bool DROP, int BIAS, bool NARROW = false>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE ? 2 : DROP || BIAS ? 3 : 4))) void k_attn_bwd_dst_tile(
     bpt_plan P, const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v, const T *__restrict__ o,
     const T *__restrict__ d_o, const float *__restrict__ lse, T *__restrict__ dq, float2 *__restrict__ pds, float *__restrict__ ws_dq,
     float scale, float scale_log2e, uint32_t drop_thr, uint32_t drop_seed, float drop_inv, const float *__restrict__ bias,
-    float *__restrict__ ds_out) {
-    constexpr int C = H * D;
+    float *__restrict__ ds_out, Narrow nw) {
+    const int Hs = NARROW ? nw.h : H;
+    const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * sizeof(T) : (uint32_t)(H * D * sizeof(T));
     TileCtx t;
-    if (!tile_begin<T, H, D, HW>(P, t)) return;
+    if (!tile_begin<T, H, D, HW, NARROW>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     __shared__ int fst_lds[HW][TILE_CHUNK];
     int2 *ent = ent_lds[t.wv];
@@ -2062,7 +2122,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
     issue_loads_first();
     const int c = t.c, g = t.g;
     const char *kb = reinterpret_cast<const char *>(k), *vb = reinterpret_cast<const char *>(v);
-    const size_t mrow = (size_t)max(t.member.x, 0) * (C * sizeof(T)) + t.offa;
+    const size_t mrow = (size_t)max(t.member.x, 0) * RB + t.offa;
     float2 *const pds_h = pds + (size_t)t.head * (size_t)P.n_edges;     // this head's part of the scratch
     // the member's dO columns live in LDS (lane-major, read back before every product with them): with them in registers
     // the kernel needs 144 and a SIMD holds three wavefronts, without them 128 and four
@@ -2071,15 +2131,15 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
     float qb[16], delta, lse_c;
     {
         float ob[16], dob[16];
-        tile_load16(reinterpret_cast<const char *>(q) + mrow, qb);
-        tile_load16(reinterpret_cast<const char *>(d_o) + mrow, dob);
-        tile_load16(reinterpret_cast<const char *>(o) + mrow, ob);
+        tile_load16<NARROW>(reinterpret_cast<const char *>(q) + mrow, qb, g, nw);
+        tile_load16<NARROW>(reinterpret_cast<const char *>(d_o) + mrow, dob, g, nw);
+        tile_load16<NARROW>(reinterpret_cast<const char *>(o) + mrow, ob, g, nw);
         float part = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) part = fmaf(dob[i], ob[i], part);
         part += __shfl_xor(part, 16);
         delta = part + __shfl_xor(part, 32);                      // dO . O of member c, this head
-        lse_c = lse[(size_t)max(t.member.x, 0) * H + t.head];
+        lse_c = lse[(size_t)max(t.member.x, 0) * Hs + t.head];
 #pragma unroll
         for (int i = 0; i < 4; ++i) dob_lds[t.wv][i][t.lane] = make_float4(dob[4 * i], dob[4 * i + 1], dob[4 * i + 2], dob[4 * i + 3]);
     }
@@ -2110,10 +2170,10 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
             }
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                B.kc[r] = *reinterpret_cast<const float4 *>(kb + ((uint32_t)idxv[r] * (uint32_t)(C * sizeof(T)) + t.offv));
+                B.kc[r] = tile_row4<NARROW>(kb + ((uint32_t)idxv[r] * RB + t.offv));
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                B.vc[r] = *reinterpret_cast<const float4 *>(vb + ((uint32_t)idxv[r] * (uint32_t)(C * sizeof(T)) + t.offv));
+                B.vc[r] = tile_row4<NARROW>(vb + ((uint32_t)idxv[r] * RB + t.offv));
             if constexpr (BIAS) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], B.pos[r])];
@@ -2142,7 +2202,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
                 float pe = has ? __builtin_amdgcn_exp2f((BIAS ? fmaf(st[r], scale_log2e, B.bz[BIAS ? r : 0] * scale_log2e) : st[r] * scale_log2e) - lse_c) : 0.f;
                 float mt = 1.f;                                   // dropout multiplier of this pair (as in the forward)
                 if constexpr (DROP)
-                    mt = dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)H + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
+                    mt = dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)Hs + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
                 ds[r] = pe * (dp[r] * mt - delta) * scale;
                 pe *= mt;                                         // what multiplies v (forward) and dO (dV)
                 if (has) {
@@ -2155,19 +2215,19 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
         tile_walk<PIPE, Blk>(nblk, issue, compute);
         wave_lds_fence();
     }
-    tile_store_rows<H, D, false>(t, acc, 1.f, dq, ws_dq);
+    tile_store_rows<H, D, false, NARROW>(t, acc, 1.f, dq, ws_dq, nw);
 }
 
 // Backward on tiles, source side (groups of the out-CSR plan: members = source rows, entries = destinations):
 // dk += ds^T q, dv += p^T dO with (p, ds) of every pair fetched from the scratch the destination side filled, at the
 // destination side's pair number that this plan's grp_pairs gives for (entry, member).
-template <typename T, int H, int D, int HW, bool PIPE>
+template <typename T, int H, int D, int HW, bool PIPE, bool NARROW = false>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE ? 3 : 4))) void k_attn_bwd_src_tile(
     bpt_plan P, const T *__restrict__ q, const T *__restrict__ d_o, const float2 *__restrict__ pds, T *__restrict__ dk, T *__restrict__ dv,
-    float *__restrict__ ws_dk, float *__restrict__ ws_dv) {
-    constexpr int C = H * D;
+    float *__restrict__ ws_dk, float *__restrict__ ws_dv, Narrow nw) {
+    const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * sizeof(T) : (uint32_t)(H * D * sizeof(T));
     TileCtx t;
-    if (!tile_begin<T, H, D, HW>(P, t)) return;
+    if (!tile_begin<T, H, D, HW, NARROW>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     int2 *ent = ent_lds[t.wv];
     const int c = t.c, g = t.g;
@@ -2214,9 +2274,9 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
             for (int r = 0; r < 4; ++r) {
                 const int2 en = ent[TILE_R * b + 4 * r + g];
                 B.has |= ((en.y >> c) & 1) << r;
-                const uint32_t off = (uint32_t)en.x * (uint32_t)(C * sizeof(T)) + t.offv;
-                B.qr[r] = *reinterpret_cast<const float4 *>(qb + off);
-                B.dr[r] = *reinterpret_cast<const float4 *>(db + off);
+                const uint32_t off = (uint32_t)en.x * RB + t.offv;
+                B.qr[r] = tile_row4<NARROW>(qb + off);
+                B.dr[r] = tile_row4<NARROW>(db + off);
                 B.w[r] = pds_h[pos[r]];
             }
         };
@@ -2234,8 +2294,8 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
         tile_walk<PIPE, Blk>(nblk, issue, compute);
         wave_lds_fence();
     }
-    tile_store_rows<H, D, false>(t, ak, 1.f, dk, ws_dk);
-    tile_store_rows<H, D, false>(t, av, 1.f, dv, ws_dv);
+    tile_store_rows<H, D, false, NARROW>(t, ak, 1.f, dk, ws_dk, nw);
+    tile_store_rows<H, D, false, NARROW>(t, av, 1.f, dv, ws_dv, nw);
 }
 
 // ---- Dense tiles for bfloat16 rows.  Same walk and the same lane roles as the float32 tile kernels above, on
@@ -2292,9 +2352,31 @@ __device__ __forceinline__ floatx4v tile_dot_bf16(const Bf8 (&a)[2], const Bf8 (
     s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0].v, b[0].v, s, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1].v, b[1].v, s, 0, 0, 0);
 }
-__device__ __forceinline__ void tile_load_row_bf16(const char *p, Bf8 (&out)[2]) {
-    out[0].q = *reinterpret_cast<const uint4 *>(p);
-    out[1].q = *reinterpret_cast<const uint4 *>(p + 16);
+template <bool NARROW>
+__device__ __forceinline__ void tile_load_row_bf16(const char *p, Bf8 (&out)[2], int g, const Narrow &nw) {
+    if constexpr (NARROW) {
+        uint32_t w[8];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {                             // quad 4 g + t; d is even, so a quad is shifted by whole words
+            const int quad = 4 * (4 * g + t), col = min(quad, nw.d - 4);
+            const uintx2u x = *reinterpret_cast<const uintx2u *>(p + 2 * col);
+            w[2 * t] = col >= quad ? x[0] : 0u;
+            w[2 * t + 1] = col + 2 >= quad ? x[1] : 0u;
+        }
+        out[0].q = make_uint4(w[0], w[1], w[2], w[3]);
+        out[1].q = make_uint4(w[4], w[5], w[6], w[7]);
+    } else {
+        out[0].q = *reinterpret_cast<const uint4 *>(p);
+        out[1].q = *reinterpret_cast<const uint4 *>(p + 16);
+    }
+}
+template <bool NARROW> __device__ __forceinline__ uint2 tile_row4_bf16(const char *p) {
+    if constexpr (NARROW) {
+        const uintx2u x = *reinterpret_cast<const uintx2u *>(p);
+        return make_uint2(x[0], x[1]);
+    } else {
+        return *reinterpret_cast<const uint2 *>(p);
+    }
 }
 // As tile_rows_to_operand: the rows of a block's entries, loaded as columns 4 c .. 4 c + 3 of the rows of entries 4 g + r
 // (the sixteen lanes of a lane group read one row's 128 contiguous bytes), turned in a wavefront-private piece of LDS
@@ -2316,14 +2398,15 @@ __device__ __forceinline__ void tile_rows_to_operand_bf16(char *kt, const uint2 
     wave_lds_fence();                                             // (read before the next block's rows are written)
 }
 
-template <int H, int D, int HW, int WPE, bool PIPE, bool DROP, int BIAS>
+template <int H, int D, int HW, int WPE, bool PIPE, bool DROP, int BIAS, bool NARROW = false>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))) void k_attn_fwd_tile_bf16(
     bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, bf16_t *__restrict__ o,
     float *__restrict__ lse, float *__restrict__ ws_acc, float *__restrict__ ws_ml, float scale_log2e, uint32_t drop_thr,
-    uint32_t drop_seed, float drop_inv, const float *__restrict__ bias) {
-    constexpr int RB = H * D * 2;                                 // bytes of a node row
+    uint32_t drop_seed, float drop_inv, const float *__restrict__ bias, Narrow nw) {
+    const int Hs = NARROW ? nw.h : H;                             // heads as lse, workspace and dropout keys count them
+    const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * 2 : (uint32_t)(H * D * 2);                       // bytes of a node row
     TileCtx t;
-    if (!tile_begin<bf16_t, H, D, HW>(P, t)) return;
+    if (!tile_begin<bf16_t, H, D, HW, NARROW>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     __shared__ int fst_lds[HW][BIAS == 2 ? TILE_CHUNK : 1];      // the entries' first pair numbers: where a term in pair order sits
     int2 *ent = ent_lds[t.wv];
@@ -2334,10 +2417,10 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
     issue_loads_first();
     const int c = t.c, g = t.g;
-    const uint32_t offr = (uint32_t)((t.head * D + 16 * g) * 2), offc = (uint32_t)((t.head * D + 4 * c) * 2);
+    const uint32_t offr = NARROW ? t.offa : (uint32_t)((t.head * D + 16 * g) * 2), offc = t.offv;
     const char *kb = reinterpret_cast<const char *>(k), *vb = reinterpret_cast<const char *>(v);
     Bf8 qb[2];
-    tile_load_row_bf16(reinterpret_cast<const char *>(q) + (size_t)max(t.member.x, 0) * RB + offr, qb);
+    tile_load_row_bf16<NARROW>(reinterpret_cast<const char *>(q) + (size_t)max(t.member.x, 0) * RB + offr, qb, g, nw);
     floatx4v acc[4];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
@@ -2358,7 +2441,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             const int4 e23 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g + 2]);
             const int idxv[4] = {e01.x, e01.z, e23.x, e23.z};
 #pragma unroll
-            for (int r = 0; r < 4; ++r) B.kq[r] = *reinterpret_cast<const uint2 *>(kb + ((uint32_t)idxv[r] * (uint32_t)RB + offc));
+            for (int r = 0; r < 4; ++r) B.kq[r] = tile_row4_bf16<NARROW>(kb + ((uint32_t)idxv[r] * RB + offc));
         };
         auto issue_rest = [&](Blk &B, int b) {
             if constexpr (DROP || BIAS == 1) tile_pair_eids(P, p0 + TILE_R * b + 4 * g, t.p_end, c, B.xe);
@@ -2368,7 +2451,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             const int mk[4] = {e01.y, e01.w, e23.y, e23.w};
             B.has = ((mk[0] >> c) & 1) | (((mk[1] >> c) & 1) << 1) | (((mk[2] >> c) & 1) << 2) | (((mk[3] >> c) & 1) << 3);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) B.vr[r] = *reinterpret_cast<const uint2 *>(vb + ((uint32_t)idxv[r] * (uint32_t)RB + offc));
+            for (int r = 0; r < 4; ++r) B.vr[r] = tile_row4_bf16<NARROW>(vb + ((uint32_t)idxv[r] * RB + offc));
             if constexpr (BIAS == 1) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, 1>(P, t.head, B.xe[BIAS == 1 ? r : 0], 0)];
@@ -2408,7 +2491,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
                 pr[r] = __builtin_amdgcn_exp2f(sc[r] - mref);
                 lrun += pr[r];                                   // the softmax denominator ignores dropout
                 if constexpr (DROP)
-                    pr[r] *= dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)H + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
+                    pr[r] *= dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)Hs + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
             }
             Bf4 pa;
             pa.u[0] = pack_bf16(pr[0], pr[1]);
@@ -2422,26 +2505,27 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     }
     float lt = lrun + __shfl_xor(lrun, 16);
     lt += __shfl_xor(lt, 32);
-    tile_store_rows<H, D, true>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc);
+    tile_store_rows<H, D, true, NARROW>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc, nw);
     if (g == 0 && t.member.x >= 0) {
         if (t.member.y < 0) {
-            lse[(size_t)t.member.x * H + t.head] = lt > 0.f ? mref + log2f(lt) : 0.f;
+            lse[(size_t)t.member.x * Hs + t.head] = lt > 0.f ? mref + log2f(lt) : 0.f;
         } else {
-            ws_ml[((size_t)t.member.y * H + t.head) * 2] = mref;
-            ws_ml[((size_t)t.member.y * H + t.head) * 2 + 1] = lt;
+            ws_ml[((size_t)t.member.y * Hs + t.head) * 2] = mref;
+            ws_ml[((size_t)t.member.y * Hs + t.head) * 2 + 1] = lt;
         }
     }
 }
 
-template <int H, int D, int HW, int WPE, bool PIPE, bool DROP, int BIAS>
+template <int H, int D, int HW, int WPE, bool PIPE, bool DROP, int BIAS, bool NARROW = false>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP || BIAS ? WPE - 1 : WPE))) void k_attn_bwd_dst_tile_bf16(
     bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, const bf16_t *__restrict__ o,
     const bf16_t *__restrict__ d_o, const float *__restrict__ lse, bf16_t *__restrict__ dq, uint32_t *__restrict__ pds,
     float *__restrict__ ws_dq, float scale, float scale_log2e, uint32_t drop_thr, uint32_t drop_seed, float drop_inv,
-    const float *__restrict__ bias, float *__restrict__ ds_out) {
-    constexpr int RB = H * D * 2;
+    const float *__restrict__ bias, float *__restrict__ ds_out, Narrow nw) {
+    const int Hs = NARROW ? nw.h : H;
+    const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * 2 : (uint32_t)(H * D * 2);
     TileCtx t;
-    if (!tile_begin<bf16_t, H, D, HW>(P, t)) return;
+    if (!tile_begin<bf16_t, H, D, HW, NARROW>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     __shared__ int fst_lds[HW][TILE_CHUNK];
     int2 *ent = ent_lds[t.wv];
@@ -2452,7 +2536,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
     if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
     issue_loads_first();
     const int c = t.c, g = t.g;
-    const uint32_t offr = (uint32_t)((t.head * D + 16 * g) * 2), offc = (uint32_t)((t.head * D + 4 * c) * 2);
+    const uint32_t offr = NARROW ? t.offa : (uint32_t)((t.head * D + 16 * g) * 2), offc = t.offv;
     const char *kb = reinterpret_cast<const char *>(k), *vb = reinterpret_cast<const char *>(v);
     const size_t mrow = (size_t)max(t.member.x, 0) * RB + offr;
     uint32_t *const pds_h = pds + (size_t)t.head * (size_t)P.n_edges;     // this head's part of the scratch
@@ -2460,9 +2544,9 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
     float delta, lse_c;
     {
         Bf8 ob[2];
-        tile_load_row_bf16(reinterpret_cast<const char *>(q) + mrow, qb);
-        tile_load_row_bf16(reinterpret_cast<const char *>(d_o) + mrow, dob);
-        tile_load_row_bf16(reinterpret_cast<const char *>(o) + mrow, ob);
+        tile_load_row_bf16<NARROW>(reinterpret_cast<const char *>(q) + mrow, qb, g, nw);
+        tile_load_row_bf16<NARROW>(reinterpret_cast<const char *>(d_o) + mrow, dob, g, nw);
+        tile_load_row_bf16<NARROW>(reinterpret_cast<const char *>(o) + mrow, ob, g, nw);
         float part = 0.f;
 #pragma unroll
         for (int h2 = 0; h2 < 2; ++h2) {
@@ -2475,7 +2559,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
         }
         part += __shfl_xor(part, 16);
         delta = part + __shfl_xor(part, 32);                      // dO . O of member c, this head
-        lse_c = lse[(size_t)max(t.member.x, 0) * H + t.head];
+        lse_c = lse[(size_t)max(t.member.x, 0) * Hs + t.head];
     }
     floatx4v acc[4];
 #pragma unroll
@@ -2500,9 +2584,9 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
             B.pos[0] = tile_pair_number(f4.x, e01.y, c); B.pos[1] = tile_pair_number(f4.y, e01.w, c);
             B.pos[2] = tile_pair_number(f4.z, e23.y, c); B.pos[3] = tile_pair_number(f4.w, e23.w, c);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) B.kc[r] = *reinterpret_cast<const uint2 *>(kb + ((uint32_t)idxv[r] * (uint32_t)RB + offc));
+            for (int r = 0; r < 4; ++r) B.kc[r] = tile_row4_bf16<NARROW>(kb + ((uint32_t)idxv[r] * RB + offc));
 #pragma unroll
-            for (int r = 0; r < 4; ++r) B.vc[r] = *reinterpret_cast<const uint2 *>(vb + ((uint32_t)idxv[r] * (uint32_t)RB + offc));
+            for (int r = 0; r < 4; ++r) B.vc[r] = tile_row4_bf16<NARROW>(vb + ((uint32_t)idxv[r] * RB + offc));
             if constexpr (BIAS) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], B.pos[r])];
@@ -2521,7 +2605,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
                 float pe = has ? __builtin_amdgcn_exp2f((BIAS ? st[r] + B.bz[BIAS ? r : 0] : st[r]) * scale_log2e - lse_c) : 0.f;
                 float mt = 1.f;                                   // dropout multiplier of this pair (as in the forward)
                 if constexpr (DROP)
-                    mt = dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)H + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
+                    mt = dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)Hs + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
                 ds[r] = pe * (dp[r] * mt - delta) * scale;
                 pe *= mt;                                         // what multiplies v (forward) and dO (dV)
                 if (has) {
@@ -2537,20 +2621,20 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
         tile_walk<PIPE, Blk>(nblk, issue, compute);
         wave_lds_fence();
     }
-    tile_store_rows<H, D, false>(t, acc, 1.f, dq, ws_dq);
+    tile_store_rows<H, D, false, NARROW>(t, acc, 1.f, dq, ws_dq, nw);
 }
 
-template <int H, int D, int HW, int WPE, bool PIPE>
+template <int H, int D, int HW, int WPE, bool PIPE, bool NARROW = false>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))) void k_attn_bwd_src_tile_bf16(
     bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ d_o, const uint32_t *__restrict__ pds, bf16_t *__restrict__ dk,
-    bf16_t *__restrict__ dv, float *__restrict__ ws_dk, float *__restrict__ ws_dv) {
-    constexpr int RB = H * D * 2;
+    bf16_t *__restrict__ dv, float *__restrict__ ws_dk, float *__restrict__ ws_dv, Narrow nw) {
+    const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * 2 : (uint32_t)(H * D * 2);
     TileCtx t;
-    if (!tile_begin<bf16_t, H, D, HW>(P, t)) return;
+    if (!tile_begin<bf16_t, H, D, HW, NARROW>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     int2 *ent = ent_lds[t.wv];
     const int c = t.c, g = t.g;
-    const uint32_t offc = (uint32_t)((t.head * D + 4 * c) * 2);
+    const uint32_t offc = t.offv;
     const char *qb = reinterpret_cast<const char *>(q), *db = reinterpret_cast<const char *>(d_o);
     const uint32_t *const pds_h = pds + (size_t)t.head * (size_t)P.n_edges;
     floatx4v ak[4], av[4];
@@ -2589,9 +2673,9 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             ahead_of = b + 1;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const uint32_t off = (uint32_t)idxv[r] * (uint32_t)RB + offc;
-                B.qr[r] = *reinterpret_cast<const uint2 *>(qb + off);
-                B.dr[r] = *reinterpret_cast<const uint2 *>(db + off);
+                const uint32_t off = (uint32_t)idxv[r] * RB + offc;
+                B.qr[r] = tile_row4_bf16<NARROW>(qb + off);
+                B.dr[r] = tile_row4_bf16<NARROW>(db + off);
                 B.w[r] = pds_h[pos[r]];
             }
         };
@@ -2608,8 +2692,8 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
         tile_walk<PIPE, Blk>(nblk, issue, compute);
         wave_lds_fence();
     }
-    tile_store_rows<H, D, false>(t, ak, 1.f, dk, ws_dk);
-    tile_store_rows<H, D, false>(t, av, 1.f, dv, ws_dv);
+    tile_store_rows<H, D, false, NARROW>(t, ak, 1.f, dk, ws_dk, nw);
+    tile_store_rows<H, D, false, NARROW>(t, av, 1.f, dv, ws_dv, nw);
 }
 
 // Backward, destination side.  Writes (p, ds) of every pair to pds[(t * H + head)], t = the pair's
@@ -3202,7 +3286,7 @@ __global__ __launch_bounds__(HW * WAVE) void k_rel_bias_tiles(bpt_plan P, const 
     const int n16 = (n_used + 15) & ~15;
     rel_table_to_lds<T>(table, used_types, n_used, rel_lds, REL_LDS_PITCH);
     TileCtx t;
-    const bool mine = tile_begin<T, H, D, HW>(P, t) && t.p_begin < t.p_end;
+    const bool mine = tile_begin<T, H, D, HW>(P, t, Narrow{}) && t.p_begin < t.p_end;
     __syncthreads();
     if (!mine) return;
     float *qt = rel_lds + (size_t)n_used * REL_LDS_PITCH + (size_t)t.wv * n16 * TILE_R;
@@ -4025,7 +4109,7 @@ int run_attn_fwd(const bpt_plan *P, const void *q, const void *k, const void *v,
                 constexpr int HW = H >= 4 ? 4 : H;          // heads per workgroup
 #define LAUNCH_FWD_TILE(PI, DR, BI)                                                                                                  \
     hipLaunchKernelGGL((k_attn_fwd_tile<T, H, D, HW, PI, DR, BI>), dim3(group_grid(P) * (H / HW)), dim3(HW * WAVE), 0, s, *P, (const T *)q, \
-                       (const T *)k, (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed, drop.inv, bias)
+                       (const T *)k, (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed, drop.inv, bias, Narrow{})
                 switch ((drop.thr != 0 ? 1 : 0) + 2 * tile_bias_mode(P, bias)) {
                 case 0: if (tall_tiles(P, H)) LAUNCH_FWD_TILE(true, false, 0); else LAUNCH_FWD_TILE(false, false, 0); break;
                 case 1: LAUNCH_FWD_TILE(false, true, 0); break;
@@ -4044,7 +4128,7 @@ int run_attn_fwd(const bpt_plan *P, const void *q, const void *k, const void *v,
 #define LAUNCH_FWD_TILE(DR, BI)                                                                                                          \
     hipLaunchKernelGGL((k_attn_fwd_tile_bf16<H, D, HW, TILE_BF16_WPE, TILE_BF16_PIPE, DR, BI>), dim3(group_grid(P) * (H / HW)), dim3(HW * WAVE), \
                        0, s, *P, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (bf16_t *)o, lse, ws_acc, ws_ml, scale * LOG2E,   \
-                       drop.thr, drop.seed, drop.inv, bias)
+                       drop.thr, drop.seed, drop.inv, bias, Narrow{})
                 switch ((drop.thr != 0 ? 1 : 0) + 2 * tile_bias_mode(P, bias)) {
                 case 0: LAUNCH_FWD_TILE(false, 0); break;
                 case 1: LAUNCH_FWD_TILE(true, 0); break;
@@ -4095,7 +4179,7 @@ int run_attn_fwd(const bpt_plan *P, const void *q, const void *k, const void *v,
     int st = launch_status();
     if (st != BPT_OK || P->n_heavy == 0) return st;
     hipLaunchKernelGGL((k_attn_fwd_combine<T, H, D>), dim3((int)P->n_heavy, H * D / WAVE), dim3(BLOCK), 0, s, P->heavy,
-                       (const float *)ws_acc, (const float *)ws_ml, (T *)o, lse);
+                       (const float *)ws_acc, (const float *)ws_ml, (T *)o, lse, Narrow{});
     return launch_status();
 }
 
@@ -4119,7 +4203,7 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
 #define LAUNCH_DST_TILE(PI, DR, BI)                                                                                                    \
     hipLaunchKernelGGL((k_attn_bwd_dst_tile<T, H, D, HW, PI, DR, BI>), dim3(group_grid(Pin) * (H / HW)), dim3(HW * WAVE), 0, s, *Pin,     \
                        (const T *)q, (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pds, ws_rows, scale,         \
-                       scale * LOG2E, drop.thr, drop.seed, drop.inv, bias, ds_out)
+                       scale * LOG2E, drop.thr, drop.seed, drop.inv, bias, ds_out, Narrow{})
                 switch ((drop.thr != 0 ? 1 : 0) + 2 * tile_bias_mode(Pin, bias)) {
                 case 0: if (tall_tiles(Pin, H)) LAUNCH_DST_TILE(true, false, 0); else LAUNCH_DST_TILE(false, false, 0); break;
                 case 1: LAUNCH_DST_TILE(false, true, 0); break;
@@ -4136,16 +4220,16 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
                 ProfScope prof(BPT_KERNEL_ATTN_BWD_SRC, s);
                 if (tall_tiles(Pout, H))
                     hipLaunchKernelGGL((k_attn_bwd_src_tile<T, H, D, HW, true>), dim3(group_grid(Pout) * (H / HW)), dim3(HW * WAVE), 0, s, *Pout,
-                                       (const T *)q, (const T *)d_o, (const float2 *)pds, (T *)dk, (T *)dv, ws_dk, ws_dv);
+                                       (const T *)q, (const T *)d_o, (const float2 *)pds, (T *)dk, (T *)dv, ws_dk, ws_dv, Narrow{});
                 else
                     hipLaunchKernelGGL((k_attn_bwd_src_tile<T, H, D, HW, false>), dim3(group_grid(Pout) * (H / HW)), dim3(HW * WAVE), 0, s, *Pout,
-                                       (const T *)q, (const T *)d_o, (const float2 *)pds, (T *)dk, (T *)dv, ws_dk, ws_dv);
+                                       (const T *)q, (const T *)d_o, (const float2 *)pds, (T *)dk, (T *)dv, ws_dk, ws_dv, Narrow{});
             }
             st = launch_status();
             if (st != BPT_OK || Pin->n_heavy + Pout->n_heavy == 0) return st;
             hipLaunchKernelGGL((k_combine_sum3<T>), dim3((int)(Pin->n_heavy + Pout->n_heavy), H * D / (4 * WAVE), 2), dim3(BLOCK), 0, s, Pin->heavy,
                                (int)Pin->n_heavy, (const float *)ws_rows, (T *)dq, Pout->heavy, (const float *)ws_dk, (T *)dk, (T *)dv, H * D,
-                               (size_t)Pout->n_slots * H * D);
+                               (size_t)Pout->n_slots * H * D, Narrow{});
             return launch_status();
         }
     }
@@ -4159,7 +4243,7 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
     hipLaunchKernelGGL((k_attn_bwd_dst_tile_bf16<H, D, HW, TILE_BF16_WPE_DST, TILE_BF16_PIPE, DR, BI>), dim3(group_grid(Pin) * (H / HW)),   \
                        dim3(HW * WAVE), 0, s, *Pin, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (const bf16_t *)o,             \
                        (const bf16_t *)d_o, lse, (bf16_t *)dq, (uint32_t *)ws, ws_rows, scale, scale * LOG2E, drop.thr, drop.seed,          \
-                       drop.inv, bias, ds_out)
+                       drop.inv, bias, ds_out, Narrow{})
                 switch ((drop.thr != 0 ? 1 : 0) + 2 * tile_bias_mode(Pin, bias)) {
                 case 0: LAUNCH_DST_TILE(false, 0); break;
                 case 1: LAUNCH_DST_TILE(true, 0); break;
@@ -4175,13 +4259,13 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
             {
                 ProfScope prof(BPT_KERNEL_ATTN_BWD_SRC, s);
                 hipLaunchKernelGGL((k_attn_bwd_src_tile_bf16<H, D, HW, TILE_BF16_WPE_SRC, TILE_BF16_PIPE>), dim3(group_grid(Pout) * (H / HW)), dim3(HW * WAVE), 0, s,
-                                   *Pout, (const bf16_t *)q, (const bf16_t *)d_o, (const uint32_t *)ws, (bf16_t *)dk, (bf16_t *)dv, ws_dk, ws_dv);
+                                   *Pout, (const bf16_t *)q, (const bf16_t *)d_o, (const uint32_t *)ws, (bf16_t *)dk, (bf16_t *)dv, ws_dk, ws_dv, Narrow{});
             }
             st = launch_status();
             if (st != BPT_OK || Pin->n_heavy + Pout->n_heavy == 0) return st;
             hipLaunchKernelGGL((k_combine_sum3<T>), dim3((int)(Pin->n_heavy + Pout->n_heavy), H * D / (4 * WAVE), 2), dim3(BLOCK), 0, s, Pin->heavy,
                                (int)Pin->n_heavy, (const float *)ws_rows, (T *)dq, Pout->heavy, (const float *)ws_dk, (T *)dk, (T *)dv, H * D,
-                               (size_t)Pout->n_slots * H * D);
+                               (size_t)Pout->n_slots * H * D, Narrow{});
             return launch_status();
         }
     }
@@ -4240,9 +4324,97 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
     // partial rows of dq (destination side) and of dk, dv (source side) in one launch
     hipLaunchKernelGGL((k_combine_sum3<T>), dim3((int)(Pin->n_heavy + Pout->n_heavy), H * D / (4 * WAVE), 2), dim3(BLOCK), 0, s, Pin->heavy,
                        (int)Pin->n_heavy, (const float *)ws_rows, (T *)dq, Pout->heavy, (const float *)ws_dk, (T *)dk, (T *)dv, H * D,
-                       (size_t)Pout->n_slots * H * D);
+                       (size_t)Pout->n_slots * H * D, Narrow{});
     return launch_status();
 }
+
+// ---- heads of fewer than 64 columns ----
+template <typename T> bool narrow_ok(const bpt_plan *P, const Narrow &nw) {
+    return has_tiles(P, nw.h, 64, sizeof(T)) && (P->grp_eids != nullptr);
+}
+
+template <typename T>
+int run_attn_fwd_narrow(const bpt_plan *P, const void *q, const void *k, const void *v, void *o, float *lse, void *ws, float scale, Dropout drop,
+                        const Narrow &nw, hipStream_t s) {
+    if (P->n_items == 0) return BPT_OK;
+    float *ws_acc = (float *)ws, *ws_ml = ws_acc ? ws_acc + (size_t)P->n_slots * nw.h * 64 : nullptr;
+    const dim3 grid(group_grid(P) * nw.slices), block(NARROW_HW * WAVE);
+    {
+        ProfScope prof(BPT_KERNEL_ATTN_FWD, s);
+#define LAUNCH_FWD(DR)                                                                                                                   \
+    do {                                                                                                                                 \
+        if constexpr (sizeof(T) == 4)                                                                                                    \
+            hipLaunchKernelGGL((k_attn_fwd_tile<T, 16, 64, NARROW_HW, false, DR, 0, true>), grid, block, 0, s, *P, (const T *)q, (const T *)k,   \
+                               (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed, drop.inv, (const float *)nullptr, nw); \
+        else                                                                                                                             \
+            hipLaunchKernelGGL((k_attn_fwd_tile_bf16<16, 64, NARROW_HW, TILE_BF16_WPE, false, DR, 0, true>), grid, block, 0, s, *P,              \
+                               (const T *)q, (const T *)k, (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed,       \
+                               drop.inv, (const float *)nullptr, nw);                                                                      \
+    } while (0)
+        if (drop.thr != 0) LAUNCH_FWD(true); else LAUNCH_FWD(false);
+#undef LAUNCH_FWD
+    }
+    const int st = launch_status();
+    if (st != BPT_OK || P->n_heavy == 0) return st;
+    hipLaunchKernelGGL((k_attn_fwd_combine<T, 16, 64, true>), dim3((int)P->n_heavy, nw.heads), dim3(BLOCK), 0, s, P->heavy, (const float *)ws_acc,
+                       (const float *)ws_ml, (T *)o, lse, nw);
+    return launch_status();
+}
+
+template <typename T>
+int run_attn_bwd_narrow(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const void *k, const void *v, const void *o, const void *d_o,
+                        const float *lse, void *dq, void *dk, void *dv, void *ws, float scale, Dropout drop, const Narrow &nw, hipStream_t s) {
+    if (Pin->n_items == 0) return BPT_OK;
+    using pds_t = std::conditional_t<sizeof(T) == 4, float2, uint32_t>;
+    pds_t *pds = (pds_t *)ws;
+    float *ws_dq = (float *)ws + pds_bytes(Pin, Pout, nw.h, 64, sizeof(T)) / 4;
+    float *ws_dk = ws_dq + (size_t)Pin->n_slots * nw.h * 64, *ws_dv = ws_dk + (size_t)Pout->n_slots * nw.h * 64;
+    const dim3 grid(group_grid(Pin) * nw.slices), grid_src(group_grid(Pout) * nw.slices), block(NARROW_HW * WAVE);
+    {
+        ProfScope prof(BPT_KERNEL_ATTN_BWD_DST, s);
+#define LAUNCH_DST(DR)                                                                                                                   \
+    do {                                                                                                                                 \
+        if constexpr (sizeof(T) == 4)                                                                                                    \
+            hipLaunchKernelGGL((k_attn_bwd_dst_tile<T, 16, 64, NARROW_HW, false, DR, 0, true>), grid, block, 0, s, *Pin, (const T *)q,           \
+                               (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pds, ws_dq, scale, scale * LOG2E,       \
+                               drop.thr, drop.seed, drop.inv, (const float *)nullptr, (float *)nullptr, nw);                                \
+        else                                                                                                                             \
+            hipLaunchKernelGGL((k_attn_bwd_dst_tile_bf16<16, 64, NARROW_HW, TILE_BF16_WPE_DST, false, DR, 0, true>), grid, block, 0, s, *Pin,     \
+                               (const T *)q, (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pds, ws_dq, scale,        \
+                               scale * LOG2E, drop.thr, drop.seed, drop.inv, (const float *)nullptr, (float *)nullptr, nw);                 \
+    } while (0)
+        if (drop.thr != 0) LAUNCH_DST(true); else LAUNCH_DST(false);
+#undef LAUNCH_DST
+    }
+    int st = launch_status();
+    if (st != BPT_OK) return st;
+    {
+        ProfScope prof(BPT_KERNEL_ATTN_BWD_SRC, s);
+        if constexpr (sizeof(T) == 4)
+            hipLaunchKernelGGL((k_attn_bwd_src_tile<T, 16, 64, NARROW_HW, false, true>), grid_src, block, 0, s, *Pout, (const T *)q, (const T *)d_o,
+                               pds, (T *)dk, (T *)dv, ws_dk, ws_dv, nw);
+        else
+            hipLaunchKernelGGL((k_attn_bwd_src_tile_bf16<16, 64, NARROW_HW, TILE_BF16_WPE_SRC, false, true>), grid_src, block, 0, s, *Pout,
+                               (const T *)q, (const T *)d_o, pds, (T *)dk, (T *)dv, ws_dk, ws_dv, nw);
+    }
+    st = launch_status();
+    if (st != BPT_OK || Pin->n_heavy + Pout->n_heavy == 0) return st;
+    hipLaunchKernelGGL((k_combine_sum3<T, true>), dim3((int)(Pin->n_heavy + Pout->n_heavy), nw.h * 64 / (4 * WAVE), 2), dim3(BLOCK), 0, s, Pin->heavy,
+                       (int)Pin->n_heavy, (const float *)ws_dq, (T *)dq, Pout->heavy, (const float *)ws_dk, (T *)dk, (T *)dv, nw.h * 64,
+                       (size_t)Pout->n_slots * nw.h * 64, nw);
+    return launch_status();
+}
+
+// heads x d that the NARROW forms take: the padded head count has fused kernels, rows start on 4 bytes, a quad fits a head
+int narrow_shape(int heads, int d, int h, int dtype, Narrow &nw) {
+    if (heads < 1 || d < 1) return BPT_ERR_SHAPE;
+    if (dtype != BPT_F32 && dtype != BPT_BF16) return BPT_ERR_UNSUPPORTED;
+    if (!fast_shape(h, 64, dtype) || heads > h || d < 4 || d > 64 || (dtype == BPT_BF16 && d % 2 != 0)) return BPT_ERR_UNSUPPORTED;
+    nw = Narrow{d, heads, h, (heads + NARROW_HW - 1) / NARROW_HW};
+    return BPT_OK;
+}
+
+inline bool aligned4(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 3) == 0; }
 
 }  // namespace
 
@@ -4592,6 +4764,46 @@ int bpt_attention_backward(const bpt_plan *plan_in, const bpt_plan *plan_out, co
     if (dtype == BPT_BF16) { using T = bf16_t; BPT_FAST_SHAPES_BF16(X) }
 #undef X
     return BPT_ERR_UNSUPPORTED;
+}
+
+int bpt_attention_forward_narrow(const bpt_plan *plan_in, const void *q, const void *k, const void *v, void *o, float *lse, void *workspace,
+                                 int64_t workspace_bytes, float scale, float dropout_p, uint64_t dropout_seed, int heads, int d, int h,
+                                 int dtype, void *stream) {
+    CHECK(check_plan(plan_in, true));
+    Narrow nw;
+    CHECK(narrow_shape(heads, d, h, dtype, nw));
+    if (!q || !k || !v || !o || !lse) return BPT_ERR_NULL;
+    if (!(dropout_p >= 0.f && dropout_p < 1.f)) return BPT_ERR_SIZE;
+    const Dropout drop = make_dropout(dropout_p, dropout_seed);
+    if (!(dtype == BPT_F32 ? narrow_ok<float>(plan_in, nw) : narrow_ok<bf16_t>(plan_in, nw))) return BPT_ERR_UNSUPPORTED;
+    if (!aligned4(q) || !aligned4(k) || !aligned4(v) || !aligned4(o) || !aligned16(workspace)) return BPT_ERR_UNSUPPORTED;
+    const int64_t need = bpt_workspace_bytes(BPT_OP_ATTN_FWD, plan_in, nullptr, h, 64, dtype);
+    if (need > 0 && (!workspace || workspace_bytes < need)) return BPT_ERR_WORKSPACE;
+    hipStream_t s = (hipStream_t)stream;
+    return dtype == BPT_F32 ? run_attn_fwd_narrow<float>(plan_in, q, k, v, o, lse, workspace, scale, drop, nw, s)
+                            : run_attn_fwd_narrow<bf16_t>(plan_in, q, k, v, o, lse, workspace, scale, drop, nw, s);
+}
+
+int bpt_attention_backward_narrow(const bpt_plan *plan_in, const bpt_plan *plan_out, const void *q, const void *k, const void *v, const void *o,
+                                  const void *d_o, const float *lse, void *dq, void *dk, void *dv, void *workspace, int64_t workspace_bytes,
+                                  float scale, float dropout_p, uint64_t dropout_seed, int heads, int d, int h, int dtype, void *stream) {
+    CHECK(check_plan(plan_in, true));
+    CHECK(check_plan(plan_out, true));
+    Narrow nw;
+    CHECK(narrow_shape(heads, d, h, dtype, nw));
+    if (!q || !k || !v || !o || !d_o || !lse || !dq || !dk || !dv) return BPT_ERR_NULL;
+    if (!(dropout_p >= 0.f && dropout_p < 1.f)) return BPT_ERR_SIZE;
+    if (plan_in->n_edges != plan_out->n_edges) return BPT_ERR_PLAN;
+    const Dropout drop = make_dropout(dropout_p, dropout_seed);
+    if (!tiled_backward(plan_in, plan_out, h, 64, dtype == BPT_BF16 ? 2 : 4) || !plan_in->grp_eids) return BPT_ERR_UNSUPPORTED;
+    if (!aligned4(q) || !aligned4(k) || !aligned4(v) || !aligned4(o) || !aligned4(d_o) || !aligned4(dq) || !aligned4(dk) || !aligned4(dv) ||
+        !aligned16(workspace))
+        return BPT_ERR_UNSUPPORTED;
+    const int64_t need = bpt_workspace_bytes(BPT_OP_ATTN_BWD, plan_in, plan_out, h, 64, dtype);
+    if (need > 0 && (!workspace || workspace_bytes < need)) return BPT_ERR_WORKSPACE;
+    hipStream_t s = (hipStream_t)stream;
+    return dtype == BPT_F32 ? run_attn_bwd_narrow<float>(plan_in, plan_out, q, k, v, o, d_o, lse, dq, dk, dv, workspace, scale, drop, nw, s)
+                            : run_attn_bwd_narrow<bf16_t>(plan_in, plan_out, q, k, v, o, d_o, lse, dq, dk, dv, workspace, scale, drop, nw, s);
 }
 
 }  // extern "C"

@@ -31,7 +31,7 @@ using at::Tensor;
 
 namespace {
 
-enum Kind { ATTN_FWD = 0, ATTN_BWD = 1 };
+enum Kind { ATTN_FWD = 0, ATTN_BWD = 1, ATTN_FWD_NARROW = 2, ATTN_BWD_NARROW = 3 };
 
 constexpr size_t MAX_TENSORS = 8, MAX_EXTRA = 6, MAX_ENTRIES = 512;
 
@@ -242,6 +242,100 @@ Tensor attention(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r,
     return std::get<0>(attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale, p, seed));
 }
 
+// ---- fused attention with heads of fewer than 64 columns, h: the heads it is computed as if padded to -------------------------
+std::optional<std::tuple<Tensor, Tensor>> narrow_forward_known(const Tensor &col, const Tensor &indptr, const Tensor &eid, const Tensor &indices,
+                                                               const Tensor &q, const Tensor &k, const Tensor &v, int h, double scale, double p,
+                                                               uint64_t seed) {
+    Shape s;
+    if (!attention_shape(q, k, v, p, s) || indices.sizes() != eid.sizes()) return std::nullopt;
+    Key key;
+    if (!make_key(key, ATTN_FWD_NARROW, {&col, &indptr, &eid, &indices}, q.device(), {s.nq, s.nk, h, s.d, s.dt, s.h})) return std::nullopt;
+    const EntryPtr e = find(key);
+    if (!e) return std::nullopt;
+    c10::DeviceGuard guard(q.device());
+    Tensor o = at::empty_like(q), lse = at::empty({s.nq, h}, q.options().dtype(at::kFloat));
+    Workspace ws(BPT_OP_ATTN_FWD, &e->a, nullptr, h, 64, s.dt, q);
+    const int st = bpt_attention_forward_narrow(&e->a, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), (float *)lse.data_ptr(), ws.ptr,
+                                                ws.bytes, (float)scale, (float)p, seed, s.h, s.d, h, s.dt, stream_of(q.device()));
+    if (st != BPT_OK) return std::nullopt;
+    return std::make_tuple(o, lse);
+}
+
+std::optional<Three> narrow_backward_known(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r, const Tensor &indices_r,
+                                           const Tensor &col, const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c, const Tensor &q,
+                                           const Tensor &k, const Tensor &v, const Tensor &o, const Tensor &lse, const Tensor &d_o, int h,
+                                           double scale, double p, uint64_t seed) {
+    Shape s;
+    if (!attention_shape(q, k, v, p, s) || !like(o, q) || !like(d_o, q) || o.sizes() != q.sizes() || d_o.sizes() != q.sizes()) return std::nullopt;
+    if (lse.scalar_type() != at::kFloat || lse.device() != q.device() || !lse.is_contiguous() || lse.dim() != 2 || lse.size(0) != s.nq ||
+        lse.size(1) != h)
+        return std::nullopt;
+    if (indices_c.sizes() != eid_c.sizes() || indices_r.sizes() != eid_r.sizes() || eid_r.sizes() != eid_c.sizes()) return std::nullopt;
+    Key key;
+    if (!make_key(key, ATTN_BWD_NARROW, {&row, &indptr_r, &eid_r, &indices_r, &col, &indptr_c, &eid_c, &indices_c}, q.device(),
+                  {s.nq, s.nk, h, s.d, s.dt, s.h}))
+        return std::nullopt;
+    const EntryPtr e = find(key);
+    if (!e) return std::nullopt;
+    c10::DeviceGuard guard(q.device());
+    Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
+    Workspace ws(BPT_OP_ATTN_BWD, &e->a, &e->b, h, 64, s.dt, q);
+    const int st = bpt_attention_backward_narrow(&e->a, &e->b, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), d_o.data_ptr(),
+                                                 (const float *)lse.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.ptr, ws.bytes,
+                                                 (float)scale, (float)p, seed, s.h, s.d, h, s.dt, stream_of(q.device()));
+    if (st != BPT_OK) return std::nullopt;
+    return Three{dq, dk, dv};
+}
+
+// The forward is a call of graphop.attention_forward, as that of the padded copies was: q, k, v stand for the padded shape there.
+std::tuple<Tensor, Tensor> narrow_forward(const Tensor &col, const Tensor &indptr, const Tensor &eid, const Tensor &indices, const Tensor &q,
+                                          const Tensor &k, const Tensor &v, int64_t h, double scale, double p, int64_t seed) {
+    const auto meta = at::TensorOptions().dtype(q.dtype()).device(at::kMeta);
+    const Tensor qp = at::empty({q.size(0), h, 64}, meta), kp = at::empty({k.size(0), h, 64}, meta);
+    py::dict kw;
+    kw["narrow"] = py::make_tuple(q, k, v);
+    return python("attention_forward")(col, indptr, eid, indices, qp, kp, kp, scale, p, (uint64_t)seed, **kw).cast<std::tuple<Tensor, Tensor>>();
+}
+
+struct NarrowAttention : torch::autograd::Function<NarrowAttention> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r,
+                          const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c,
+                          const Tensor &q, const Tensor &k, const Tensor &v, int64_t h, double scale, double p, int64_t seed) {
+        const Tensor qc = q.contiguous(), kc = k.contiguous(), vc = v.contiguous();
+        const auto [o, lse] = narrow_forward(col, indptr_c, eid_c, indices_c, qc, kc, vc, h, scale, p, seed);
+        ctx->save_for_backward({row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, qc, kc, vc, o, lse});
+        ctx->saved_data["h"] = h;
+        ctx->saved_data["scale"] = scale;
+        ctx->saved_data["p"] = p;
+        ctx->saved_data["seed"] = seed;
+        return o;
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        const auto t = ctx->get_saved_variables();
+        const double scale = ctx->saved_data["scale"].toDouble(), p = ctx->saved_data["p"].toDouble();
+        const uint64_t seed = (uint64_t)ctx->saved_data["seed"].toInt();
+        const int h = (int)ctx->saved_data["h"].toInt();
+        const Tensor d_o = grads[0].contiguous();
+        auto r = narrow_backward_known(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], t[10], t[11], t[12], d_o, h, scale, p, seed);
+        if (!r)
+            r = with_python([&] {
+                return python("attention_backward_narrow")(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], t[10], t[11], t[12], d_o, h,
+                                                           scale, p, seed).template cast<Three>();
+            });
+        torch::autograd::variable_list out(15);
+        std::tie(out[8], out[9], out[10]) = *r;
+        return out;
+    }
+};
+
+Tensor attention_narrow(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r, const Tensor &indices_r, const Tensor &col,
+                        const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c, const Tensor &q, const Tensor &k, const Tensor &v,
+                        int64_t h, double scale, double p, uint64_t seed) {
+    if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
+        return NarrowAttention::apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, h, scale, p, (int64_t)seed);
+    return std::get<0>(narrow_forward(col, indptr_c, eid_c, indices_c, q.contiguous(), k.contiguous(), v.contiguous(), h, scale, p, (int64_t)seed));
+}
+
 // ---- the table ---------------------------------------------------------------------------------------------------------------
 // `kind`'s choice for these index tensors and numbers: the bpt_plan structs at the addresses a and b (0: none), which point into
 // what `plans` holds.  True if it was taken.
@@ -312,7 +406,11 @@ std::vector<py::object> take_used() {
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.attr("ATTN_FWD") = (int)ATTN_FWD;
     m.attr("ATTN_BWD") = (int)ATTN_BWD;
+    m.attr("ATTN_FWD_NARROW") = (int)ATTN_FWD_NARROW;
+    m.attr("ATTN_BWD_NARROW") = (int)ATTN_BWD_NARROW;
     m.def("attention", &attention);
+    m.def("attention_narrow", &attention_narrow);
+    m.def("attention_forward_narrow", &narrow_forward_known);
     m.def("attention_forward", &attention_forward_known);
     m.def("attention_backward", &attention_backward_known);
     m.def("remember", &remember);

@@ -510,13 +510,110 @@ def _check_bias(bias, n_edges, h, device, cfg, by_pair=False):
         raise RuntimeError("the per-edge score term needs the row-group kernels")
 
 
-def attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale=None, dropout_p=0.0, seed=0, bias=None, bias_by_pair=False):
+def _pad_heads(x, h):
+    """(n, heads, d) zero-padded to (n, h, 64)."""
+    return torch.nn.functional.pad(x, (0, 64 - x.size(2), 0, h - x.size(1)))
+
+
+def _narrow_seg(q, h, n_edges, cfg):
+    """The work-item length of the tile plans of a layer whose rows the kernels for narrow heads take as they are, or None where
+    they do not: heads of 4 to 64 columns, starting on 4 bytes, wherever tiles are the library's choice."""
+    if not (cfg.use_groups and _tiles(q, h, 64, None, 0.0, None, cfg) and 4 <= q.size(2) <= 64 and (q.dtype == torch.float32 or q.size(2) % 2 == 0)
+            and not _FORCE_GENERIC and TILE_BACKWARD is not False):
+        return None
+    if TILE_SEG_LEN is not None:
+        return TILE_SEG_LEN
+    deg = n_edges / max(q.size(0), 1)
+    return 64 if deg < 32 else (128 if deg < 80 else 256)
+
+
+def _attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale, dropout_p, seed):
+    """(o, lse) for heads of fewer than 64 columns: o (n, heads, d), lse (n, h), h the heads the layer is padded to.  On the tile
+    kernels that read the rows as they are, or else on padded copies."""
+    cfg = _SETTINGS
+    seed = int(seed) & (2 ** 64 - 1)
+    known = _native.attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale, dropout_p, seed)
+    if known is not None:
+        return known
+    _check_all(col=col, indptr_c=indptr_c, eid_c=eid_c, indices_c=indices_c, q=q, k=k, v=v)
+    _same_dtype(q, k, v)
+    heads, d = _hd(q)
+    _expect_index(eid_c, indices_c)
+    _expect_shape(k, (k.size(0),) + tuple(q.shape[1:]), "k")
+    _expect_shape(v, k.shape, "v")
+    seg, plan = _narrow_seg(q, h, eid_c.size(0), cfg), None
+    if seg is not None and max(q.size(0), k.size(0)) * h * 64 * q.element_size() < 2 ** 32:
+        plan = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, None))
+    if plan is None or not plan.covers_all_edges:
+        o, lse = attention_forward(col, indptr_c, eid_c, indices_c, _pad_heads(q, h), _pad_heads(k, h), _pad_heads(v, h), scale, dropout_p, seed)
+        return o[:, :heads, :d].contiguous(), lse
+    struct = plan.ensure_groups(TILE_ROWS)["struct"]
+    o = torch.empty_like(q)
+    lse = torch.empty((q.size(0), h), dtype=torch.float32, device=q.device)
+    dt = _dtype(q)
+    ws, nws = _workspace(OP_ATTN_FWD, plan, None, h, 64, dt, q.device)
+    with _on_device_of(q):
+        check_attn(_LIB.bpt_attention_forward_narrow(ctypes.byref(struct), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(ws), nws, scale,
+                                                     float(dropout_p), seed, heads, d, h, dt, _stream()), "attention_forward_narrow")
+    if cfg is _SETTINGS:
+        _native.remember(_native.ATTN_FWD_NARROW, [col, indptr_c, eid_c, indices_c], [q.size(0), k.size(0), h, d, dt, heads],
+                         ctypes.addressof(struct), 0, (plan,))
+    return o, lse
+
+
+def attention_backward_narrow(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, o, lse, do, h, scale, dropout_p, seed):
+    """(dq, dk, dv) of attention_forward(..., narrow=(q, k, v)): the shapes of q, k, v; lse (n, h) as that returned it."""
+    cfg = _SETTINGS
+    _check_all(row=row, indptr_r=indptr_r, eid_r=eid_r, indices_r=indices_r, col=col, indptr_c=indptr_c,
+               eid_c=eid_c, indices_c=indices_c, q=q, k=k, v=v, o=o, lse=lse, do=do)
+    _same_dtype(q, k, v, o, do)
+    heads, d = _hd(q)
+    _expect_index(eid_c, indices_c)
+    _expect_index(eid_r, indices_r)
+    _expect_shape(eid_r, eid_c.shape, "eid_r")
+    _expect_shape(k, (k.size(0),) + tuple(q.shape[1:]), "k")
+    _expect_shape(v, k.shape, "v")
+    _expect_shape(o, q.shape, "o")
+    _expect_shape(do, q.shape, "do")
+    if lse.dtype != torch.float32 or lse.device != q.device:
+        raise ValueError("lse must be the float32 tensor that attention_forward returned")
+    _expect_shape(lse, (q.size(0), h), "lse")
+    seg, pi = _narrow_seg(q, h, eid_c.size(0), cfg), None
+    if seg is not None and max(q.size(0), k.size(0)) * h * 64 * q.element_size() < 2 ** 32:
+        order_src = _plan.tile_order_src(k.size(0), eid_r.size(0))
+        pi = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, None))
+        po = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, order_src))
+    if pi is None or not (pi.covers_all_edges and po.covers_all_edges):
+        grads = attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, *(_pad_heads(x, h) for x in (q, k, v, o)), lse,
+                                   _pad_heads(do, h), scale, dropout_p, seed)
+        return tuple(x[:, :heads, :d].contiguous() for x in grads)
+    in_struct = pi.ensure_groups(TILE_ROWS)["struct"]
+    out_struct = po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True)
+    dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
+    dt = _dtype(q)
+    in_ref, out_ref = ctypes.byref(in_struct), ctypes.byref(out_struct)
+    ws, nws = _workspace(OP_ATTN_BWD, pi, po, h, 64, dt, q.device, plan_ref=in_ref, plan_t_ref=out_ref)
+    with _on_device_of(q):
+        check_attn(_LIB.bpt_attention_backward_narrow(in_ref, out_ref, _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(dq), _ptr(dk),
+                                                      _ptr(dv), _ptr(ws), nws, scale, float(dropout_p), int(seed) & (2 ** 64 - 1), heads, d, h, dt,
+                                                      _stream()), "attention_backward_narrow")
+    if cfg is _SETTINGS:
+        _native.remember(_native.ATTN_BWD_NARROW, [row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c],
+                         [q.size(0), k.size(0), h, d, dt, heads], ctypes.addressof(in_struct), ctypes.addressof(out_struct), (pi, po))
+    return dq, dk, dv
+
+
+def attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale=None, dropout_p=0.0, seed=0, bias=None, bias_by_pair=False, narrow=None):
     """o[dst] = sum over in-edges drop(softmax((q[dst].k[src] + bias[e])*scale)) v[src]; returns (o, lse) with lse
     (n, h) float32 in base-2 units.  Arithmetic of modules/attention.py:66-77 in one pass.  dropout_p > 0
     drops attention probabilities as attention.py:73 does; the mask is a function of (seed, graph), see
     attention_dropout_mask.  bias: None or the float32 score term of rel_bias_forward: (E + 1, h) with its rows by edge
     id, or with bias_by_pair (h, E) with the edges in the order of the numbers attention_pair_rows() gives them (tile
-    kernels only)."""
+    kernels only).
+    narrow=(q, k, v): heads of fewer than 64 columns, (n, heads, d); the q, k, v before it then only stand for the padded shape
+    (attention_padded_shape; tensors of it on the meta device) and o has narrow's shape, lse the padded heads."""
+    if narrow is not None:
+        return _attention_forward_narrow(col, indptr_c, eid_c, indices_c, *narrow, q.size(1), float(scale), float(dropout_p), seed)
     cfg = _SETTINGS
     if bias is None:
         known = _native.attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, 1.0 / math.sqrt(q.size(-1)) if scale is None else float(scale),

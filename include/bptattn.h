@@ -253,6 +253,18 @@ int bpt_attention_forward_noalloc(const bpt_plan *plan_in, const void *q, const 
                                   const float *bias, void *o, float *lse, float scale, float dropout_p,
                                   uint64_t dropout_seed, int h, int d, int dtype, void *stream);
 
+/* bpt_attention_forward / _backward for heads of fewer than 64 columns on tile plans, the rows as they are in memory: q, k, v, o,
+ * d_o, dq, dk, dv (n, heads, d) with d from 4 to 64 (even in bfloat16) on 4-byte addresses.  h: the head count with fused kernels
+ * (4, 8 or 16; 8 or 16 in bfloat16) that the layer is computed as if padded to: lse is (n, h), dropout decides by (seed, edge, head)
+ * as it does there, and the workspace is that of (h, 64).  BPT_ERR_UNSUPPORTED where the kernels do not take the call. */
+int bpt_attention_forward_narrow(const bpt_plan *plan_in, const void *q, const void *k, const void *v, void *o, float *lse,
+                                 void *workspace, int64_t workspace_bytes, float scale, float dropout_p, uint64_t dropout_seed,
+                                 int heads, int d, int h, int dtype, void *stream);
+int bpt_attention_backward_narrow(const bpt_plan *plan_in, const bpt_plan *plan_out, const void *q, const void *k, const void *v,
+                                  const void *o, const void *d_o, const float *lse, void *dq, void *dk, void *dv, void *workspace,
+                                  int64_t workspace_bytes, float scale, float dropout_p, uint64_t dropout_seed, int heads, int d,
+                                  int h, int dtype, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,68 @@
+"""The tile kernels that read heads of fewer than 64 columns as they are in memory, at the widths where quads of four columns end,
+shift or fall away and at head counts that leave a workgroup half empty; against the float64 oracle at the layer's tolerances
+(fp32 outputs rtol / atol 1e-5, gradients rtol 1e-4, bf16 2e-2).  Widths they do not take run on padded copies and are checked with
+them.  What stands behind the last head must not matter: the rows are views into memory full of NaN."""
+import pytest
+import torch
+
+import oracle
+from test_gpu_parity import DEV, GTOL, TOL, Case, close, f64, rand
+
+pytestmark = pytest.mark.gpu
+
+_cases = {}
+
+
+def case(name):
+    if name not in _cases:
+        _cases[name] = Case(name)
+    return _cases[name]
+
+
+def among_nans(x):
+    """x as a contiguous view that starts and ends inside a larger buffer of NaN."""
+    buf = torch.full((x.numel() + 128,), float("nan"), dtype=x.dtype, device=x.device)
+    view = buf[64:64 + x.numel()].view(x.shape)
+    view.copy_(x)
+    return view
+
+
+@pytest.mark.parametrize("gname", ["bpt512_k4", "multigraph"])
+@pytest.mark.parametrize("dtype,h,d", [(torch.float32, 1, 4), (torch.float32, 3, 5), (torch.float32, 4, 6), (torch.float32, 5, 7), (torch.float32, 6, 50),
+                                       (torch.float32, 7, 61), (torch.float32, 9, 63), (torch.float32, 15, 64), (torch.float32, 2, 3),
+                                       (torch.bfloat16, 1, 4), (torch.bfloat16, 5, 6), (torch.bfloat16, 6, 50), (torch.bfloat16, 9, 62),
+                                       (torch.bfloat16, 3, 64), (torch.bfloat16, 6, 51)],
+                         ids=lambda x: str(x).replace("torch.", ""))
+def test_narrow_heads_against_the_oracle(gname, dtype, h, d):
+    from bpt_amd import op
+    c = case(gname)
+    q, k, v, do = (among_nans(rand((c.n, h, d), dtype, s, 1.0 / 8).to(DEV)) for s in (71, 72, 73, 74))
+    for t in (q, k, v):
+        t.requires_grad_(True)
+    o = op.bpt_attention(*c.out, *c.inn, q, k, v)
+    assert o.shape == (c.n, h, d) and o.is_contiguous()
+    grads = torch.autograd.grad(o, (q, k, v), do)
+    ro, ra = oracle.attention_forward(c.csr, f64(q), f64(k), f64(v))
+    want = oracle.attention_backward(c.csr, f64(q), f64(k), f64(v), ra, f64(do))
+    close(o, ro, TOL[dtype], "o")
+    for got, ref, name in zip(grads, want, ("dq", "dk", "dv")):
+        assert got.shape == q.shape
+        close(got, ref, GTOL[dtype], name)
+
+
+@pytest.mark.parametrize("dtype,h,d", [(torch.float32, 6, 50), (torch.float32, 3, 5), (torch.bfloat16, 6, 50)], ids=lambda x: str(x).replace("torch.", ""))
+def test_dropout_of_narrow_heads_is_that_of_the_padded_layer(dtype, h, d):
+    from bpt_amd import graphop, op
+    c = case("bpt512_k4")
+    q, k, v, do = (rand((c.n, h, d), dtype, s, 1.0 / 8).to(DEV) for s in (81, 82, 83, 84))
+    hp = graphop.attention_padded_shape(q)[0]
+    grow = lambda x: torch.nn.functional.pad(x, (0, 64 - d, 0, hp - h))
+    both = []
+    for narrow in (True, False):
+        x = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        rows = x if narrow else [grow(t) for t in x]
+        o = op.bpt_attention(*c.out, *c.inn, *rows, scale=d ** -0.5, dropout_p=0.3, seed=5)[:, :h, :d]
+        both.append((o.detach(), *torch.autograd.grad(o, x, do)))
+    # (the same kernels on the same numbers and zeros: sums over the columns differ in nothing but the zeros' places)
+    for got, want, name in zip(both[0], both[1], ("o", "dq", "dk", "dv")):
+        close(got, f64(want), TOL[dtype] if name == "o" else GTOL[dtype], name)
