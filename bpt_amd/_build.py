@@ -3,7 +3,7 @@
   bpt_amd/csrc/libbptgraph.so  host C++ (g++)            <- bptgraph.cpp
   bpt_amd/csrc/libbptattn.so   gfx950 HIP (hipcc)        <- bptattn.hip
   bpt_amd/csrc/libbptplan.so   gfx950 HIP (hipcc)        <- bptplan.hip  (plans built on the GPU; rocPRIM headers)
-  bpt_amd/csrc/bptop.so        host C++ (g++, torch)     <- bptop.cpp    (host side of the ops and their autograd; links libbptattn)
+  bpt_amd/csrc/bptop.so        host C++ (g++, torch)     <- bptop.cpp    (host side of the ops and their autograd; links both)
 
 hipcc cross-compiles for gfx950 without a GPU.  Run `python -m bpt_amd._build`.
 """
@@ -59,7 +59,7 @@ def build_plan(verbose=True):
 
 
 def build_op(verbose=True):
-    """After build_attn, whose library it links (found beside it at run time)."""
+    """After build_attn and build_plan, whose libraries it links (found beside it at run time)."""
     import sysconfig
     import torch
     from torch.utils import cpp_extension
@@ -69,7 +69,7 @@ def build_op(verbose=True):
     _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-DTORCH_EXTENSION_NAME=bptop",
           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM"]
          + [f"-I{p}" for p in include] + [os.path.join(CSRC, "bptop.cpp"), "-o", OP_SO, f"-L{libs}", f"-L{CSRC}",
-                                          "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-ltorch", "-l:libbptattn.so", "-Wl,-rpath,$ORIGIN"], verbose)
+                                          "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python", "-ltorch", "-l:libbptattn.so", "-l:libbptplan.so", "-Wl,-rpath,$ORIGIN"], verbose)
     return OP_SO
 
 
@@ -79,8 +79,7 @@ def build_all(verbose=True):
     with ThreadPoolExecutor(2) as pool:
         plan = pool.submit(build_plan, verbose)
         graph, attn = build_graph(verbose), build_attn(verbose)
-        op = build_op(verbose)
-        return graph, attn, plan.result(), op
+        return graph, attn, plan.result(), build_op(verbose)
 
 
 if __name__ == "__main__":

@@ -25,6 +25,8 @@
 #include <vector>
 
 #include "../../include/bptattn.h"
+#include "../../include/bptbuild.h"
+#include "../../include/bptplan.h"
 
 namespace py = pybind11;
 using at::Tensor;
@@ -210,7 +212,12 @@ struct Attention : torch::autograd::Function<Attention> {
     static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r,
                           const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c,
                           const Tensor &q, const Tensor &k, const Tensor &v, double scale, double p, int64_t seed) {
-        const auto [o, lse] = attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale, p, (uint64_t)seed);
+        auto r = attention_forward_known(col, indptr_c, eid_c, indices_c, q, k, v, scale, p, (uint64_t)seed);
+        if (!r) {                                             // a new graph: both sides' plans at once
+            python("prepare_training")(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, p);
+            r = attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale, p, (uint64_t)seed);
+        }
+        const auto [o, lse] = *r;
         ctx->save_for_backward({row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, o, lse});
         ctx->saved_data["scale"] = scale;
         ctx->saved_data["p"] = p;
@@ -297,11 +304,21 @@ std::tuple<Tensor, Tensor> narrow_forward(const Tensor &col, const Tensor &indpt
     return python("attention_forward")(col, indptr, eid, indices, qp, kp, kp, scale, p, (uint64_t)seed, **kw).cast<std::tuple<Tensor, Tensor>>();
 }
 
+bool narrow_known(const Tensor &col, const Tensor &indptr, const Tensor &eid, const Tensor &indices, const Tensor &q, const Tensor &k, int64_t h) {
+    Key key;
+    return q.is_cuda() && q.dim() == 3 &&
+           make_key(key, ATTN_FWD_NARROW, {&col, &indptr, &eid, &indices}, q.device(),
+                    {q.size(0), k.size(0), h, q.size(2), dtype_code(q.scalar_type()), q.size(1)}) &&
+           find(key) != nullptr;
+}
+
 struct NarrowAttention : torch::autograd::Function<NarrowAttention> {
     static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r,
                           const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c,
                           const Tensor &q, const Tensor &k, const Tensor &v, int64_t h, double scale, double p, int64_t seed) {
         const Tensor qc = q.contiguous(), kc = k.contiguous(), vc = v.contiguous();
+        if (!narrow_known(col, indptr_c, eid_c, indices_c, qc, kc, h))
+            python("prepare_training")(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, qc, kc, p, h);
         const auto [o, lse] = narrow_forward(col, indptr_c, eid_c, indices_c, qc, kc, vc, h, scale, p, seed);
         ctx->save_for_backward({row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, qc, kc, vc, o, lse});
         ctx->saved_data["h"] = h;
@@ -334,6 +351,122 @@ Tensor attention_narrow(const Tensor &row, const Tensor &indptr_r, const Tensor 
     if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
         return NarrowAttention::apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, h, scale, p, (int64_t)seed);
     return std::get<0>(narrow_forward(col, indptr_c, eid_c, indices_c, q.contiguous(), k.contiguous(), v.contiguous(), h, scale, p, (int64_t)seed));
+}
+
+// ---- tile plans ---------------------------------------------------------------------------------------------------------------
+// The tile plans of one side of a graph or of both (the second linked to the first: what a training step needs), built in shared
+// launches with two waits: one for the counts, one for the finished plans (another stream may use them next).
+struct SideIn {
+    Tensor row, indptr, eid, indices;
+    int64_t n_rows, n_index;
+    int seg_len, by_mask;
+};
+constexpr int PAD_ENTRIES = 8;
+
+void check_build(int st, const char *what) {
+    if (st != BPT_OK) throw std::runtime_error(std::string(what) + ": status " + std::to_string(st));
+}
+
+void wait_for(void *stream) {
+    py::gil_scoped_release nogil;
+    check_build(bpt_build_wait(stream), "bpt_build_wait");
+}
+
+// graphbuilder.get_csrs_device behind its checks: the five arrays of the out- and of the in-side, and (error, units) of each
+std::tuple<std::vector<Tensor>, std::vector<Tensor>, std::vector<int>> build_csrs(const Tensor &src, const Tensor &dst, int64_t n, int chunk) {
+    const int64_t E = src.numel();
+    c10::DeviceGuard guard(src.device());
+    int64_t bounds[2];
+    check_build(bpt_csr_device_bounds(E, n, chunk, bounds), "bpt_csr_device_bounds");
+    std::vector<Tensor> side[2];
+    int64_t *ptr[2][5];
+    for (int i = 0; i < 2; ++i) {
+        int j = 0;
+        for (int64_t size : {n + 1, E, E, bounds[0], bounds[0] + 1}) {
+            side[i].push_back(at::empty({std::max<int64_t>(size, 1)}, src.options()));
+            ptr[i][j] = side[i][j].data_ptr<int64_t>();
+            ++j;
+        }
+    }
+    Tensor ws = at::empty({bounds[1]}, src.options().dtype(at::kByte));
+    Tensor info = at::empty({4}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));      // (written by the last kernel: no copy to wait for)
+    void *stream = stream_of(src.device());
+    check_build(bpt_build_csrs_device(src.const_data_ptr<int64_t>(), dst.const_data_ptr<int64_t>(), E, n, chunk, ptr[0], ptr[1],
+                                      info.data_ptr<int32_t>(), ws.data_ptr(), bounds[1], stream),
+                "bpt_build_csrs_device");
+    wait_for(stream);
+    const int32_t *c = info.data_ptr<int32_t>();
+    return {side[0], side[1], {c[0], c[1], c[2], c[3]}};
+}
+
+// None where the short form does not build them; else (per side: its info block, base arrays, group arrays; the pair mapping of
+// the second side).  A side's info block holds an error where its arrays are malformed (then nothing else is valid).
+py::object build_tile_plans(const std::vector<std::tuple<Tensor, Tensor, Tensor, Tensor, int64_t, int64_t, int, int>> &in) {
+    const int n = (int)in.size();
+    if (n < 1 || n > 2) throw std::invalid_argument("one or two sides");
+    const at::Device dev = std::get<2>(in[0]).device();
+    for (const auto &[row, indptr, eid, indices, n_rows, n_index, seg, mask] : in)
+        for (const Tensor *t : {&row, &indptr, &eid, &indices})
+            if (!index_ok(*t, dev)) return py::none();
+    c10::DeviceGuard guard(dev);
+    const auto i32 = at::TensorOptions().dtype(at::kInt).device(dev);
+    bpt_build_side sides[2] = {};
+    std::vector<std::vector<Tensor>> base(n), groups(n);
+    for (int i = 0; i < n; ++i) {
+        const auto &[row, indptr, eid, indices, n_rows, n_index, seg, mask] = in[i];
+        const int64_t E = eid.numel(), U = row.numel();
+        if (indptr.numel() != U + 1 || indices.numel() != E || n_rows < 0 || n_index < 0 || seg < 1) return py::none();
+        bpt_build_side &s = sides[i];
+        s.n_units = U; s.n_edges = E; s.n_rows = n_rows; s.n_index_nodes = n_index; s.seg_len = seg; s.by_mask = mask;
+    }
+    int64_t bytes = 0;
+    if (bpt_build_tiles_bounds(sides, n, &bytes) != BPT_OK) return py::none();
+    for (int i = 0; i < n; ++i) {
+        const auto &[row, indptr, eid, indices, n_rows, n_index, seg, mask] = in[i];
+        bpt_build_side &s = sides[i];
+        const int64_t E = std::max<int64_t>(s.n_edges, 1), items = std::max<int64_t>(s.n_rows + s.n_edges / seg, 1);
+        base[i] = {at::empty({s.n_rows + 1}, i32), at::empty({E}, i32), at::empty({E}, i32), at::empty({items, 4}, i32), at::empty({items, 2}, i32),
+                   at::empty({std::max<int64_t>(s.n_edges / (seg + 1), 1), 3}, i32), at::empty({16}, i32)};
+        s.row = row.const_data_ptr<int64_t>(); s.indptr_units = indptr.const_data_ptr<int64_t>();
+        s.eid = eid.const_data_ptr<int64_t>(); s.indices = indices.const_data_ptr<int64_t>();
+        int32_t **to[7] = {&s.rowptr, &s.idx32, &s.eid32, &s.items, &s.item_bounds, &s.heavy, &s.info};
+        for (int j = 0; j < 7; ++j) *to[j] = base[i][j].data_ptr<int32_t>();
+    }
+    Tensor ws = at::empty({bytes}, i32.dtype(at::kByte));
+    Tensor counts = at::empty({32 * n}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+    void *stream = stream_of(dev);
+    check_build(bpt_build_tiles_count(sides, n, counts.data_ptr<int32_t>(), ws.data_ptr(), bytes, stream), "bpt_build_tiles_count");
+    wait_for(stream);
+    const int32_t *c = counts.data_ptr<int32_t>();
+    bool good = true;
+    for (int i = 0; i < n; ++i) good = good && c[32 * i] == 0;
+    Tensor pairs, number;
+    if (good) {
+        bpt_build_tiles out[2] = {};
+        const bool link = n == 2 && (c[5] & 1) && (c[37] & 1) && sides[0].n_edges == sides[1].n_edges;
+        for (int i = 0; i < n; ++i) {
+            const int64_t ng = c[32 * i + 16], ne = c[32 * i + 17];
+            groups[i] = {at::empty({ng, 16, 2}, i32), at::empty({ng + 1}, i32), at::empty({ne + 1, 4}, i32), at::empty({sides[i].n_edges}, i32),
+                         at::empty({(ne + PAD_ENTRIES) * 16}, i32), at::empty({9}, i32), at::empty({16}, i32)};
+            int32_t **to[7] = {&out[i].members, &out[i].grp_ptr, &out[i].entries, &out[i].pair_eid, &out[i].grp_eids, &out[i].chunks, &out[i].group_info};
+            for (int j = 0; j < 7; ++j) *to[j] = groups[i][j].data_ptr<int32_t>();
+        }
+        if (link) {
+            number = at::empty({std::max<int64_t>(sides[0].n_edges, 1)}, i32);
+            pairs = at::empty({groups[1][4].numel()}, i32);
+            out[0].number = number.data_ptr<int32_t>();
+        }
+        check_build(bpt_build_tiles_write(sides, n, c, out, PAD_ENTRIES, link ? pairs.data_ptr<int32_t>() : nullptr, ws.data_ptr(), bytes, stream),
+                    "bpt_build_tiles_write");
+        wait_for(stream);
+    }
+    py::list result;
+    for (int i = 0; i < n; ++i) {
+        py::list info;
+        for (int j = 0; j < 32; ++j) info.append(c[32 * i + j]);
+        result.append(py::make_tuple(info, base[i], groups[i]));
+    }
+    return py::make_tuple(result, pairs.defined() ? py::cast(pairs) : py::none());
 }
 
 // ---- the table ---------------------------------------------------------------------------------------------------------------
@@ -413,6 +546,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("attention_forward_narrow", &narrow_forward_known);
     m.def("attention_forward", &attention_forward_known);
     m.def("attention_backward", &attention_backward_known);
+    m.def("build_csrs", &build_csrs);
+    m.def("build_tile_plans", &build_tile_plans);
     m.def("remember", &remember);
     m.def("forget", &forget);
     m.def("clear", &clear);

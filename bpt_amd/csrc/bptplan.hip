@@ -146,10 +146,15 @@ template <int NW> __device__ __forceinline__ int32_t block_excl_sum(int32_t v, i
 }
 
 // counts[side][tile][bin]: how many records of the tile have the digit
+struct RsSizes {
+    int64_t n[2];                                 // records of each side
+};
+
 template <int RS_KPT, class Recs>
-__global__ __launch_bounds__(TPB) void k_rs_count(Recs recs, int64_t n, int shift, int bits, int32_t *counts) {
+__global__ __launch_bounds__(TPB) void k_rs_count(Recs recs, RsSizes sizes, int shift, int bits, int32_t *counts) {
     __shared__ int32_t h[RS_BINS];
     const int bins = 1 << bits, side = blockIdx.y;
+    const int64_t n = sizes.n[side];
     for (int b = threadIdx.x; b < bins; b += TPB) h[b] = 0;
     __syncthreads();
     const int64_t i0 = (int64_t)blockIdx.x * (TPB * RS_KPT);
@@ -209,8 +214,9 @@ __global__ __launch_bounds__(RS_PREFIX_TPB) void k_rs_prefix(int32_t *counts, in
 // on top of its running counts in LDS.
 // SUM: the tile sums up the counts itself (few tiles), else k_rs_prefix has.
 template <int RS_KPT, bool SUM, class Recs, class Out>
-__global__ __launch_bounds__(TPB) void k_rs_scatter(Recs recs, Out out, int64_t n, int shift, int bits, const int32_t *counts,
+__global__ __launch_bounds__(TPB) void k_rs_scatter(Recs recs, Out out, RsSizes sizes, int shift, int bits, const int32_t *counts,
                                                     const int32_t *totals) {
+    const int64_t n = sizes.n[blockIdx.y];
     constexpr int NW = TPB / 64;
     __shared__ int32_t wh[NW][RS_BINS];
     __shared__ int32_t sh[NW + 1];
@@ -305,34 +311,70 @@ struct RsToArrays {
 // largest neighbour; sort by the smallest.
 constexpr int ITEM_ROWS = TPB - 1;    // rows of a block of the first two kernels (one thread more: the end of the last row)
 
-struct BaseWs {
-    int32_t *seen;
-    int4 *totals;                     // per block of ITEM_ROWS rows: items, heavy rows, slots, largest degree
-    int4 *items_tmp;                  // in row order
+struct GroupRec {                     // what a group is known by before the groups are numbered
+    int32_t n_entries, n_pairs, key;            // key: smallest neighbour
+};
+
+// One side's arrays through all the kernels of its plan; up to two sides share the launches (blockIdx.y): most of these kernels
+// take the 3-10 us that any launch over some 10^4 items takes.  Both sides' tile plans and their pair mapping, call to call:
+// 33 765 nodes / 576 k edges 1831 us in library sorts, 481 one side after the other with five waits, 288 together with two.
+struct PlanSide {
+    const int64_t *row, *ipu, *eid, *indices;           // as the caller has them
+    int64_t n_units, n_edges, n_rows, n_index_nodes, max_items;
+    int32_t seg_len;
+    int32_t *rowptr, *idx32, *eid32, *heavy, *info;     // the base plan
+    int4 *items;
+    int2 *bounds;
+    int32_t *seen;                                      // its workspace
+    int4 *totals;                                       // per block of ITEM_ROWS rows: items, heavy rows, slots, largest degree
+    int4 *items_tmp;                                    // in row order
     int2 *bounds_tmp;
-    uint32_t *key[2];
-    int32_t *val[2];
-    int32_t *counts, *bin_totals;
+    // groups
+    int32_t mode, by_work, max_groups;
+    int place_bits, g_bits, key_bits, work_bits;
+    int32_t *jorder;
+    GroupRec *rec;
+    int32_t *loc_group, *loc_work, *loc_prefix;         // groups in locality order
+    int32_t *order, *entry0, *pair0, *chunks;           // final order: group as formed, first entry, first pair
+    uint32_t *word0, *word1;
+    int4 *entries;                                      // parked: neighbour, mask, first pair inside the group
+    int32_t *pairs;                                     // parked: edge ids in pair order
+    int32_t *out_info;
+};
+struct PlanSides {
+    PlanSide side[2];
 };
 
 inline int64_t item_row_blocks(int64_t n_rows) { return (n_rows + ITEM_ROWS) / ITEM_ROWS; }
 
-BaseWs base_layout(Bump &b, int64_t n_rows, int64_t n_edges, int64_t max_items) {
-    BaseWs w;
-    w.seen = b.take<int32_t>(n_edges);
-    w.totals = b.take<int4>(item_row_blocks(n_rows));
-    w.items_tmp = b.take<int4>(max_items);
-    w.bounds_tmp = b.take<int2>(max_items);
+void base_layout(Bump &b, PlanSide &S) {
+    S.seen = b.take<int32_t>(S.n_edges);
+    S.totals = b.take<int4>(item_row_blocks(S.n_rows));
+    S.items_tmp = b.take<int4>(S.max_items);
+    S.bounds_tmp = b.take<int2>(S.max_items);
+}
+
+struct SortWs {                       // the sorts of up to two sides of max_items items
+    uint32_t *key[2];
+    int32_t *val[2];
+    int32_t *counts, *totals;
+};
+SortWs sort_layout(Bump &b, int64_t max_items, int n_sides) {
+    SortWs w;
     for (int i = 0; i < 2; ++i) {
-        w.key[i] = b.take<uint32_t>(max_items);
-        w.val[i] = b.take<int32_t>(max_items);
+        w.key[i] = b.take<uint32_t>(n_sides * max_items);
+        w.val[i] = b.take<int32_t>(n_sides * max_items);
     }
-    w.counts = b.take<int32_t>(rs_tiles(max_items) * RS_BINS);
-    w.bin_totals = b.take<int32_t>(RS_BINS);
+    w.counts = b.take<int32_t>(n_sides * rs_tiles(max_items) * RS_BINS);
+    w.totals = b.take<int32_t>(n_sides * RS_BINS);
     return w;
 }
 
-__global__ void k_plan_clear(int32_t *info, const int64_t *ipu, int64_t n_units, int64_t n_edges) {
+__global__ void k_plan_clear(PlanSides b) {
+    const PlanSide &S = b.side[blockIdx.y];
+    const int64_t *ipu = S.ipu;
+    const int64_t n_units = S.n_units, n_edges = S.n_edges;
+    int32_t *info = S.info;
     if (threadIdx.x != 0) return;
     for (int t = 0; t < 16; ++t) info[t] = 0;
     int err = 0;
@@ -350,10 +392,13 @@ __global__ void k_plan_clear(int32_t *info, const int64_t *ipu, int64_t n_units,
 // Three kinds of blocks: edge slots (indices to 32 bits, eid a permutation?), units (sorted?), rows (rowptr[r] = start of the
 // first unit whose row is >= r, and what the block's rows give).  Malformed arrays set info[BPT_PI_ERR]; what the row blocks
 // then wrote is not used.
-__global__ __launch_bounds__(TPB) void k_plan_narrow(const int64_t *row, const int64_t *ipu, int64_t n_units, const int64_t *eid,
-                                                     const int64_t *indices, int64_t n_edges, int64_t n_rows, int64_t n_index_nodes,
-                                                     int32_t seg_len, unsigned edge_blocks, unsigned unit_blocks, int32_t *info,
-                                                     int32_t *idx32, int32_t *eid32, int32_t *seen, int32_t *rowptr, int4 *totals) {
+__global__ __launch_bounds__(TPB) void k_plan_narrow(PlanSides b, unsigned edge_blocks, unsigned unit_blocks) {
+    const PlanSide &S = b.side[blockIdx.y];
+    const int64_t *row = S.row, *ipu = S.ipu, *eid = S.eid, *indices = S.indices;
+    const int64_t n_units = S.n_units, n_edges = S.n_edges, n_rows = S.n_rows, n_index_nodes = S.n_index_nodes;
+    const int32_t seg_len = S.seg_len;
+    int32_t *info = S.info, *idx32 = S.idx32, *eid32 = S.eid32, *seen = S.seen, *rowptr = S.rowptr;
+    int4 *totals = S.totals;
     if (blockIdx.x < edge_blocks) {
         const int64_t p = (int64_t)blockIdx.x * TPB + threadIdx.x;
         if (p >= n_edges) return;
@@ -383,6 +428,7 @@ __global__ __launch_bounds__(TPB) void k_plan_narrow(const int64_t *row, const i
     __shared__ int32_t sh[TPB / 64 + 1];
     const unsigned blk = blockIdx.x - edge_blocks - unit_blocks;
     const int64_t r = (int64_t)blk * ITEM_ROWS + threadIdx.x;
+    if (blk >= (unsigned)((n_rows + ITEM_ROWS) / ITEM_ROWS)) return;         // (the other side has more rows)
     int32_t at = 0;
     if (r <= n_rows && n_units > 0) {
         int64_t lo = 0, hi = n_units;
@@ -420,18 +466,25 @@ __global__ __launch_bounds__(TPB) void k_plan_narrow(const int64_t *row, const i
 // number in `seen`, and the other slot does not find itself (plain stores and loads: the two kernels 20 us for 576 k edges,
 // with a counter per edge and its clearing 27).
 constexpr int ITEM_FEW = 8;
-__global__ __launch_bounds__(TPB) void k_plan_items(const int32_t *rowptr, int64_t n_rows, int32_t seg_len, const int4 *totals,
-                                                    const int32_t *eid32, const int32_t *seen, int64_t n_edges, unsigned row_blocks,
-                                                    int32_t *info, int4 *items, int32_t *heavy) {
+__global__ __launch_bounds__(TPB) void k_plan_items(PlanSides b, unsigned most_row_blocks) {
+    const PlanSide &S = b.side[blockIdx.y];
+    const int32_t *rowptr = S.rowptr, *eid32 = S.eid32, *seen = S.seen;
+    const int64_t n_rows = S.n_rows, n_edges = S.n_edges;
+    const int32_t seg_len = S.seg_len;
+    const int4 *totals = S.totals;
+    int32_t *info = S.info, *heavy = S.heavy;
+    int4 *items = S.indices ? S.items_tmp : S.items;   // (without indices the items stay in row order, as on the host)
+    const unsigned row_blocks = (unsigned)((n_rows + ITEM_ROWS) / ITEM_ROWS);
     __shared__ int32_t sh[TPB / 64 + 1];
     __shared__ int32_t many[TPB][3];                   // row, first item, first slot
     __shared__ int32_t n_many;
     if (info[BPT_PI_ERR]) return;
-    if (blockIdx.x >= row_blocks) {
-        const int64_t p = (int64_t)(blockIdx.x - row_blocks) * TPB + threadIdx.x;
+    if (blockIdx.x >= most_row_blocks) {
+        const int64_t p = (int64_t)(blockIdx.x - most_row_blocks) * TPB + threadIdx.x;
         if (p < n_edges && seen[eid32[p]] != (int32_t)p) atomicAnd(&info[BPT_PI_FLAGS], ~1);
         return;
     }
+    if (blockIdx.x >= row_blocks) return;
     if (threadIdx.x == 0) n_many = 0;
     const bool last = blockIdx.x == row_blocks - 1;
     int4 part = make_int4(0, 0, 0, 0);
@@ -483,10 +536,14 @@ __global__ __launch_bounds__(TPB) void k_plan_items(const int32_t *rowptr, int64
 
 // smallest and largest neighbour id of every item, sixteen lanes an item; an empty item: its own row id clipped to
 // n_index_nodes, twice
-__global__ __launch_bounds__(TPB) void k_item_bounds(const int4 *items, const int32_t *idx32, const int32_t *info, int64_t max_items,
-                                                     int64_t n_index_nodes, int64_t n_edges, int2 *bounds) {
+__global__ __launch_bounds__(TPB) void k_item_bounds(PlanSides b) {
+    const PlanSide &S = b.side[blockIdx.y];
+    const int32_t *idx32 = S.idx32, *info = S.info;
+    const int64_t n_index_nodes = S.n_index_nodes, n_edges = S.n_edges;
+    const int4 *items = S.indices ? S.items_tmp : S.items;
+    int2 *bounds = S.indices ? S.bounds_tmp : S.bounds;
     const int64_t i = (int64_t)blockIdx.x * (TPB / 16) + (threadIdx.x >> 4);
-    if (i >= max_items || info[BPT_PI_ERR] || i >= info[BPT_PI_N_ITEMS]) return;
+    if (i >= S.max_items || info[BPT_PI_ERR] || i >= info[BPT_PI_N_ITEMS]) return;
     const int4 it = items[i];
     int32_t lo, hi;
     if (it.z > it.y && it.y >= 0 && it.z <= n_edges) {          // (an item list from elsewhere is not trusted with addresses)
@@ -508,27 +565,23 @@ __global__ __launch_bounds__(TPB) void k_item_bounds(const int4 *items, const in
 
 // the items as sort records, by their smallest or largest neighbour; places past the last item sort behind all of them
 struct ItemRecs {
-    const int2 *bounds;
-    const int32_t *info;
-    int largest;
-    uint32_t pad;
-    __device__ uint32_t key(int, int64_t i, bool &) const {
-        if (info[BPT_PI_ERR] || i >= info[BPT_PI_N_ITEMS]) return pad;
-        return (uint32_t)(largest ? bounds[i].y : bounds[i].x);
+    PlanSides b;
+    int largest;                      // by the largest, of the items as sorted by the smallest
+    __device__ uint32_t key(int side, int64_t i, bool &) const {
+        const PlanSide &S = b.side[side];
+        if (S.info[BPT_PI_ERR] || i >= S.info[BPT_PI_N_ITEMS]) return (uint32_t)S.n_index_nodes + 1;
+        return (uint32_t)(largest ? S.bounds[i].y : S.bounds_tmp[i].x);
     }
     __device__ int32_t val(int, int64_t i) const { return (int32_t)i; }
     __device__ void report(int, bool) const {}
 };
 struct ItemsSorted {
-    const int4 *items_tmp;
-    const int2 *bounds_tmp;
-    const int32_t *info;
-    int4 *items;
-    int2 *bounds;
-    __device__ void put(int, int64_t at, uint32_t, int32_t i) const {
-        if (info[BPT_PI_ERR] || i >= info[BPT_PI_N_ITEMS]) return;
-        items[at] = items_tmp[i];
-        if (bounds) bounds[at] = bounds_tmp[i];
+    PlanSides b;
+    __device__ void put(int side, int64_t at, uint32_t, int32_t i) const {
+        const PlanSide &S = b.side[side];
+        if (S.info[BPT_PI_ERR] || i >= S.info[BPT_PI_N_ITEMS]) return;
+        S.items[at] = S.items_tmp[i];
+        if (S.bounds) S.bounds[at] = S.bounds_tmp[i];
     }
 };
 
@@ -870,46 +923,25 @@ constexpr int GRP_MAX_GROUPS = 16384;
 constexpr int GRP_ORDER_TPB = 1024;
 constexpr int GRP_ORDER_LDS = 8192;   // up to so many groups are sorted in LDS, more in global memory
 
-struct GroupRec {                     // what a group is known by before the groups are numbered
-    int32_t n_entries, n_pairs, key;            // key: smallest neighbour
-};
-
-struct ShortWs {
-    uint32_t *key[2];
-    int32_t *val[2];
-    int32_t *counts, *bin_totals, *jorder;
-    GroupRec *rec;
-    int32_t *loc_group, *loc_work, *loc_prefix;       // groups in locality order
-    int32_t *order, *entry0, *pair0, *chunks;         // final order: group as formed, first entry, first pair
-    int4 *entries;                                    // parked: neighbour, mask, first pair inside the group
-    int32_t *pairs;                                   // parked: edge ids in pair order
-};
-
-ShortWs short_layout(Bump &b, int64_t max_items, int64_t max_groups, int64_t n_edges) {
-    ShortWs w;
-    for (int i = 0; i < 2; ++i) {
-        w.key[i] = b.take<uint32_t>(max_items);
-        w.val[i] = b.take<int32_t>(max_items);
-    }
-    w.counts = b.take<int32_t>(rs_tiles(max_items) * RS_BINS);
-    w.bin_totals = b.take<int32_t>(RS_BINS);
-    w.jorder = b.take<int32_t>(max_items);
-    w.rec = b.take<GroupRec>(max_groups);
-    w.loc_group = b.take<int32_t>(max_groups);
-    w.loc_work = b.take<int32_t>(max_groups);
-    w.loc_prefix = b.take<int32_t>(max_groups);
-    w.order = b.take<int32_t>(max_groups);
-    w.entry0 = b.take<int32_t>(max_groups + 1);
-    w.pair0 = b.take<int32_t>(max_groups + 1);
-    w.chunks = b.take<int32_t>(9);
-    w.entries = b.take<int4>(n_edges);
-    w.pairs = b.take<int32_t>(n_edges);
-    return w;
+void short_layout(Bump &b, PlanSide &S) {
+    S.word0 = b.take<uint32_t>(S.max_groups);
+    S.word1 = b.take<uint32_t>(S.max_groups);
+    S.jorder = b.take<int32_t>(S.max_items);
+    S.rec = b.take<GroupRec>(S.max_groups);
+    S.loc_group = b.take<int32_t>(S.max_groups);
+    S.loc_work = b.take<int32_t>(S.max_groups);
+    S.loc_prefix = b.take<int32_t>(S.max_groups);
+    S.order = b.take<int32_t>(S.max_groups);
+    S.entry0 = b.take<int32_t>(S.max_groups + 1);
+    S.pair0 = b.take<int32_t>(S.max_groups + 1);
+    S.chunks = b.take<int32_t>(9);
+    S.entries = b.take<int4>(S.n_edges);
+    S.pairs = b.take<int32_t>(S.n_edges);
 }
 
 struct ItemOrder {                    // last pass of the sort by largest neighbour
-    int32_t *jorder;
-    __device__ void put(int, int64_t at, uint32_t, int32_t i) const { jorder[at] = i; }
+    PlanSides b;
+    __device__ void put(int side, int64_t at, uint32_t, int32_t i) const { b.side[side].jorder[at] = i; }
 };
 
 // The members of a group as formed, and where its results are parked: in the edge slots of its items, which no other group has,
@@ -1035,9 +1067,17 @@ inline __device__ int pow2_at_least(int n) {
 // One group: its records (neighbour, member, place in the member's item) sorted, an entry per neighbour and repeat, the entries
 // in the order asked for, the pairs numbered.  K: 32-bit keys where neighbour, member and place fit.
 template <int CAP, typename K>
-__global__ __launch_bounds__(TPB) void k_group_form(const int4 *items, const int2 *bounds, const int32_t *jorder, const int32_t *idx32,
-                                                    const int32_t *eid32, const int32_t *pinfo, int64_t n_edges, int32_t seg_len, int32_t R,
-                                                    int place_bits, int mode, GroupRec *rec, int4 *entries, int32_t *pairs) {
+__global__ __launch_bounds__(TPB) void k_group_form(PlanSides b, int32_t R) {
+    const PlanSide &S = b.side[blockIdx.y];
+    const int4 *items = S.items;
+    const int2 *bounds = S.bounds;
+    const int32_t *jorder = S.jorder, *idx32 = S.idx32, *eid32 = S.eid32, *pinfo = S.info;
+    const int64_t n_edges = S.n_edges;
+    const int32_t seg_len = S.seg_len;
+    const int place_bits = S.place_bits, mode = S.mode;
+    GroupRec *rec = S.rec;
+    int4 *entries = S.entries;
+    int32_t *pairs = S.pairs;
     // (16 KB for 1024 edges with 32-bit keys: ten workgroups a CU)
     __shared__ K key[CAP];
     __shared__ uint32_t ekey[CAP], emask2[CAP / 2];                 // emask2: two entries' masks a word
@@ -1186,10 +1226,14 @@ template <int NW> __device__ void block_radix_pass(const uint32_t *from, uint32_
 
 // One workgroup numbers the groups: by locality, cut into 8 ranges of equal work, by decreasing work inside a range (or not),
 // and gives every group its place in the arrays.  out_info: the plan's info block and the groups'.
-__global__ __launch_bounds__(GRP_ORDER_TPB) void k_group_order(const GroupRec *rec, const int32_t *pinfo, int32_t R, int by_work, int g_bits,
-                                                               int key_bits, int work_bits, uint32_t *word0, uint32_t *word1, int32_t *loc_group,
-                                                               int32_t *loc_work, int32_t *loc_prefix, int32_t *order, int32_t *entry0,
-                                                               int32_t *pair0, int32_t *chunks, int32_t *out_info) {
+__global__ __launch_bounds__(GRP_ORDER_TPB) void k_group_order(PlanSides b, int32_t R) {
+    const PlanSide &S = b.side[blockIdx.y];
+    const GroupRec *rec = S.rec;
+    const int32_t *pinfo = S.info;
+    const int by_work = S.by_work, g_bits = S.g_bits, key_bits = S.key_bits, work_bits = S.work_bits;
+    uint32_t *word0 = S.word0, *word1 = S.word1;
+    int32_t *loc_group = S.loc_group, *loc_work = S.loc_work, *loc_prefix = S.loc_prefix, *order = S.order, *entry0 = S.entry0, *pair0 = S.pair0,
+            *chunks = S.chunks, *out_info = S.out_info;
     constexpr int NW = GRP_ORDER_TPB / 64;
     __shared__ int32_t wh[NW][RS_BINS];
     __shared__ uint32_t lds0[GRP_ORDER_LDS], lds1[GRP_ORDER_LDS];
@@ -1270,14 +1314,30 @@ __global__ __launch_bounds__(GRP_ORDER_TPB) void k_group_order(const GroupRec *r
 }
 
 // a group's part of the arrays; the block behind the last group writes what stands behind the last entry
-__global__ __launch_bounds__(TPB) void k_group_write(const int4 *items, const int32_t *jorder, const int32_t *pinfo, const GroupRec *rec,
-                                                     const int32_t *order, const int32_t *entry0, const int32_t *pair0, const int32_t *chunks,
-                                                     const int4 *parked, const int32_t *parked_pairs, int64_t n_edges, int32_t R, int32_t n_groups,
-                                                     int32_t n_entries, int32_t max_chunk, int32_t pad_entries, int32_t seg_len, int32_t *members,
-                                                     int32_t *grp_ptr,
-                                                     int4 *entries, int32_t *pair_eid, int32_t *grp_eids, int32_t *out_chunks, int32_t *ginfo) {
+struct GroupsOut {
+    int32_t n_groups, n_entries, max_chunk;
+    int32_t *members, *grp_ptr, *pair_eid, *grp_eids, *chunks, *ginfo;
+    int4 *entries;
+    int32_t *number;                  // per edge: its pair's number (or null)
+};
+struct GroupsOuts {
+    GroupsOut side[2];
+};
+
+__global__ __launch_bounds__(TPB) void k_group_write(PlanSides b, GroupsOuts outs, int32_t R, int32_t pad_entries) {
+    const PlanSide &S = b.side[blockIdx.y];
+    const GroupsOut &O = outs.side[blockIdx.y];
+    const int4 *items = S.items, *parked = S.entries;
+    const int32_t *jorder = S.jorder, *pinfo = S.info, *order = S.order, *entry0 = S.entry0, *pair0 = S.pair0, *chunks = S.chunks,
+                  *parked_pairs = S.pairs;
+    const GroupRec *rec = S.rec;
+    const int64_t n_edges = S.n_edges;
+    const int32_t seg_len = S.seg_len, n_groups = O.n_groups, n_entries = O.n_entries, max_chunk = O.max_chunk;
+    int32_t *members = O.members, *grp_ptr = O.grp_ptr, *pair_eid = O.pair_eid, *grp_eids = O.grp_eids, *out_chunks = O.chunks, *ginfo = O.ginfo;
+    int4 *entries = O.entries;
     const int32_t f = blockIdx.x, tid = threadIdx.x;
-    if (f >= n_groups) {
+    if (f > n_groups) return;                             // (the other side has more)
+    if (f == n_groups) {
         if (tid == 0) {
             grp_ptr[n_groups] = n_entries;
             entries[n_entries] = make_int4(0, 0, 0, 0);
@@ -1303,7 +1363,11 @@ __global__ __launch_bounds__(TPB) void k_group_write(const int4 *items, const in
         e.z += p0;
         entries[e0 + u] = e;
     }
-    for (int x = tid; x < r.n_pairs; x += TPB) pair_eid[p0 + x] = parked_pairs[at.slot(x)];
+    for (int x = tid; x < r.n_pairs; x += TPB) {
+        const int32_t e = parked_pairs[at.slot(x)];
+        pair_eid[p0 + x] = e;
+        if (O.number) O.number[e] = p0 + x;
+    }
     for (int i = tid; i < r.n_entries * R; i += TPB) {
         const int u = i / R, m = i - u * R;
         const int4 e = parked[at.slot(u)];
@@ -1487,6 +1551,21 @@ __global__ __launch_bounds__(TPB) void k_merge(MergeParts m, unsigned edge_block
     int p = 0;
     for (int d = MERGE_PARTS / 2; d > 0; d >>= 1)         // the block's first element: last part that starts at or before it
         if (p + d < m.n && (edges ? m.part[p + d].edge0 : m.part[p + d].node0) <= i) p += d;
+    const int64_t next = p + 1 < m.n ? (edges ? m.part[p + 1].edge0 : m.part[p + 1].node0) : end;
+    const int64_t stop = min(i + TPB * MERGE_PER, end);
+    if (edges && stop <= next) {                          // the whole block in one part: its addresses are the block's
+        const MergePart &a = m.part[p];
+        const int64_t *s0 = a.src - a.edge0, *d0 = a.dst - a.edge0, *e0 = a.etype - a.edge0;
+        int64_t x[MERGE_PER], y[MERGE_PER], z[MERGE_PER];
+        i += threadIdx.x;
+#pragma unroll
+        for (int r = 0; r < MERGE_PER; ++r)
+            if (i + r * TPB < stop) { x[r] = s0[i + r * TPB]; y[r] = d0[i + r * TPB]; z[r] = e0[i + r * TPB]; }
+#pragma unroll
+        for (int r = 0; r < MERGE_PER; ++r)
+            if (i + r * TPB < stop) { src[i + r * TPB] = x[r] + a.node0; dst[i + r * TPB] = y[r] + a.node0; etype[i + r * TPB] = z[r]; }
+        return;
+    }
     i += threadIdx.x;
     for (int r = 0; r < MERGE_PER; ++r, i += TPB) {
         if (i >= end) return;
@@ -1660,72 +1739,179 @@ int sizes_ok(int64_t n_units, int64_t n_edges, int64_t n_rows, int64_t n_index_n
         }                                                                              \
     } while (0)
 
-// one stable sort pass over both sides: counts, prefix, scatter
+// one stable sort pass over one or both sides: counts, prefix, scatter
 template <class Recs, class Out>
-int rs_pass(const Recs &recs, const Out &out, int64_t n, int n_sides, int shift, int bits, int32_t *counts, int32_t *totals, hipStream_t s) {
+int rs_pass(const Recs &recs, const Out &out, const RsSizes &sizes, int n_sides, int shift, int bits, int32_t *counts, int32_t *totals, hipStream_t s) {
+    const int64_t n = n_sides == 2 && sizes.n[1] > sizes.n[0] ? sizes.n[1] : sizes.n[0];
     const dim3 tiles((unsigned)rs_tiles(n), (unsigned)n_sides);
     const int bins = 1 << bits;
     const bool few = rs_per_thread(n) != 8;
-    if (few) hipLaunchKernelGGL((k_rs_count<RS_KPT_FEW, Recs>), tiles, dim3(TPB), 0, s, recs, n, shift, bits, counts);
-    else hipLaunchKernelGGL((k_rs_count<8, Recs>), tiles, dim3(TPB), 0, s, recs, n, shift, bits, counts);
+    if (few) hipLaunchKernelGGL((k_rs_count<RS_KPT_FEW, Recs>), tiles, dim3(TPB), 0, s, recs, sizes, shift, bits, counts);
+    else hipLaunchKernelGGL((k_rs_count<8, Recs>), tiles, dim3(TPB), 0, s, recs, sizes, shift, bits, counts);
     HIP_TRY(hipGetLastError());
     if (few) {
-        hipLaunchKernelGGL((k_rs_scatter<RS_KPT_FEW, true, Recs, Out>), tiles, dim3(TPB), 0, s, recs, out, n, shift, bits, counts, totals);
+        hipLaunchKernelGGL((k_rs_scatter<RS_KPT_FEW, true, Recs, Out>), tiles, dim3(TPB), 0, s, recs, out, sizes, shift, bits, counts, totals);
     } else {
         hipLaunchKernelGGL(k_rs_prefix, dim3((unsigned)((bins + RS_PREFIX_BINS - 1) / RS_PREFIX_BINS), (unsigned)n_sides), dim3(RS_PREFIX_TPB), 0,
                            s, counts, totals, (int64_t)tiles.x, bins);
         HIP_TRY(hipGetLastError());
-        hipLaunchKernelGGL((k_rs_scatter<8, false, Recs, Out>), tiles, dim3(TPB), 0, s, recs, out, n, shift, bits, counts, totals);
+        hipLaunchKernelGGL((k_rs_scatter<8, false, Recs, Out>), tiles, dim3(TPB), 0, s, recs, out, sizes, shift, bits, counts, totals);
     }
     HIP_TRY(hipGetLastError());
     return BPT_OK;
 }
 
-// all passes of a sort of one side: recs to begin with, out at the end
+// all passes of a sort: recs to begin with, out at the end; two arrays of keys and values (n_sides * largest n) in between
 template <class Recs, class Out>
-int rs_sort(const Recs &recs, const Out &out, int64_t n, uint64_t max_key, uint32_t *const key[2], int32_t *const val[2], int32_t *counts,
-            int32_t *totals, hipStream_t s) {
+int rs_sort(const Recs &recs, const Out &out, const RsSizes &sizes, int n_sides, uint64_t max_key, uint32_t *const key[2], int32_t *const val[2],
+            int32_t *counts, int32_t *totals, hipStream_t s) {
+    const int64_t n = n_sides == 2 && sizes.n[1] > sizes.n[0] ? sizes.n[1] : sizes.n[0];
+    if (n == 0) return BPT_OK;
     const RsPasses ps = rs_passes(max_key);
     RsToArrays to[2];
     RsArrays from[2];
     for (int t = 0; t < 2; ++t)
         for (int i = 0; i < 2; ++i) {
-            to[t].k[i] = key[t];
-            to[t].v[i] = val[t];
-            from[t].k[i] = key[t];
-            from[t].v[i] = val[t];
+            to[t].k[i] = key[t] + (i < n_sides ? i : 0) * n;
+            to[t].v[i] = val[t] + (i < n_sides ? i : 0) * n;
+            from[t].k[i] = to[t].k[i];
+            from[t].v[i] = to[t].v[i];
         }
     for (int p = 0; p < ps.n; ++p) {
         const bool first = p == 0, last = p == ps.n - 1;
         const int shift = p * ps.bits;
         int st;
-        if (first && last) st = rs_pass(recs, out, n, 1, shift, ps.bits, counts, totals, s);
-        else if (first) st = rs_pass(recs, to[0], n, 1, shift, ps.bits, counts, totals, s);
-        else if (last) st = rs_pass(from[(p - 1) & 1], out, n, 1, shift, ps.bits, counts, totals, s);
-        else st = rs_pass(from[(p - 1) & 1], to[p & 1], n, 1, shift, ps.bits, counts, totals, s);
+        if (first && last) st = rs_pass(recs, out, sizes, n_sides, shift, ps.bits, counts, totals, s);
+        else if (first) st = rs_pass(recs, to[0], sizes, n_sides, shift, ps.bits, counts, totals, s);
+        else if (last) st = rs_pass(from[(p - 1) & 1], out, sizes, n_sides, shift, ps.bits, counts, totals, s);
+        else st = rs_pass(from[(p - 1) & 1], to[p & 1], sizes, n_sides, shift, ps.bits, counts, totals, s);
         if (st != BPT_OK) return st;
     }
     return BPT_OK;
 }
 
-struct ShortForm {
-    int64_t max_groups;
-    int place_bits, g_bits, work_bits;
-};
-
-// BPT_ERR_UNSUPPORTED where the groups are not built in the short form: a group may hold more edges than fit a workgroup's LDS,
-// or there may be more groups, or wider numbers, than one workgroup sorts as 32-bit words
-int short_form(int64_t max_items, int64_t n_edges, int64_t n_index_nodes, int32_t seg_len, int32_t R, ShortForm &f) {
+// what the kernels need to know of a side's groups, or BPT_ERR_UNSUPPORTED where they are not built in the short form: a group may
+// hold more edges than fit a workgroup's LDS, or there may be more groups, or wider numbers, than one workgroup sorts as
+// 32-bit words
+int short_form(int64_t max_items, int64_t n_edges, int64_t n_index_nodes, int32_t seg_len, int32_t R, int32_t by_mask, PlanSide &S) {
     if (max_items < 0 || n_edges < 0 || n_index_nodes < 0 || max_items >= INT32_MAX || n_edges >= INT32_MAX || n_index_nodes >= INT32_MAX - 1)
         return BPT_ERR_SIZE;
-    if (R < 1 || R > 16 || seg_len < 1) return BPT_ERR_SHAPE;
+    if (R < 1 || R > 16 || seg_len < 1 || by_mask < 0 || (by_mask & 3) > 2 || by_mask > 6) return BPT_ERR_SHAPE;
     if ((n_edges + 8) * R >= INT32_MAX) return BPT_ERR_SIZE;
-    f.max_groups = (max_items + R - 1) / R;
-    if ((int64_t)R * seg_len > GRP_MAX_EDGES || f.max_groups > GRP_MAX_GROUPS) return BPT_ERR_UNSUPPORTED;
-    f.place_bits = (int)bits_for((uint64_t)seg_len - 1);
-    f.g_bits = (int)bits_for((uint64_t)(f.max_groups > 0 ? f.max_groups - 1 : 0));
-    f.work_bits = (int)bits_for((uint64_t)(R == 16 ? 4 * (seg_len + 1) : FIXED_WORK + R * seg_len));
-    if ((int)bits_for((uint64_t)n_index_nodes) + f.g_bits > 32 || 3 + f.work_bits + f.g_bits > 32) return BPT_ERR_UNSUPPORTED;
+    const int64_t max_groups = (max_items + R - 1) / R;
+    if ((int64_t)R * seg_len > GRP_MAX_EDGES || max_groups > GRP_MAX_GROUPS) return BPT_ERR_UNSUPPORTED;
+    S.max_items = max_items;
+    S.n_edges = n_edges;
+    S.n_index_nodes = n_index_nodes;
+    S.seg_len = seg_len;
+    S.mode = by_mask & 3;
+    S.by_work = (by_mask & 4) ? 0 : 1;
+    S.max_groups = (int32_t)max_groups;
+    S.place_bits = (int)bits_for((uint64_t)seg_len - 1);
+    S.g_bits = (int)bits_for((uint64_t)(max_groups > 0 ? max_groups - 1 : 0));
+    S.key_bits = (int)bits_for((uint64_t)n_index_nodes);
+    S.work_bits = (int)bits_for((uint64_t)(R == 16 ? 4 * (seg_len + 1) : FIXED_WORK + R * seg_len));
+    return S.key_bits + S.g_bits > 32 || 3 + S.work_bits + S.g_bits > 32 ? BPT_ERR_UNSUPPORTED : BPT_OK;
+}
+
+int fill_side(const bpt_build_side &side, PlanSide &S) {
+    const int st = sizes_ok(side.n_units, side.n_edges, side.n_rows, side.n_index_nodes, side.seg_len);
+    if (st != BPT_OK) return st;
+    if (!side.rowptr || !side.items || !side.info) return BPT_ERR_NULL;
+    if (side.n_units > 0 && (!side.row || !side.indptr_units)) return BPT_ERR_NULL;
+    if (side.n_edges > 0 && (!side.eid || !side.idx32 || !side.eid32)) return BPT_ERR_NULL;
+    if (side.n_edges / ((int64_t)side.seg_len + 1) > 0 && !side.heavy) return BPT_ERR_NULL;
+    S.max_items = side.n_rows + side.n_edges / side.seg_len;
+    if (S.max_items >= INT32_MAX) return BPT_ERR_SIZE;
+    S.row = side.row;
+    S.ipu = side.indptr_units;
+    S.eid = side.eid;
+    S.indices = side.indices;
+    S.n_units = side.n_units;
+    S.n_edges = side.n_edges;
+    S.n_rows = side.n_rows;
+    S.n_index_nodes = side.n_index_nodes;
+    S.seg_len = side.seg_len;
+    S.rowptr = side.rowptr;
+    S.idx32 = side.idx32;
+    S.eid32 = side.eid32;
+    S.heavy = side.heavy;
+    S.info = side.info;
+    S.items = reinterpret_cast<int4 *>(side.items);
+    S.bounds = reinterpret_cast<int2 *>(side.item_bounds);
+    return BPT_OK;
+}
+
+template <typename F> int64_t most_of(const PlanSides &b, int n_sides, F &&f) {
+    const int64_t x = f(b.side[0]), y = n_sides == 2 ? f(b.side[1]) : 0;
+    return x > y ? x : y;
+}
+
+int base_build(const PlanSides &b, int n_sides, const SortWs &w, hipStream_t s) {
+    const unsigned ns = (unsigned)n_sides;
+    hipLaunchKernelGGL(k_plan_clear, dim3(1, ns), dim3(64), 0, s, b);
+    HIP_TRY(hipGetLastError());
+    const unsigned edge_blocks = blocks_for(most_of(b, n_sides, [](const PlanSide &S) { return S.n_edges; }));
+    const unsigned unit_blocks = blocks_for(most_of(b, n_sides, [](const PlanSide &S) { return S.n_units; }));
+    const unsigned row_blocks = (unsigned)most_of(b, n_sides, [](const PlanSide &S) { return item_row_blocks(S.n_rows); });
+    hipLaunchKernelGGL(k_plan_narrow, dim3(edge_blocks + unit_blocks + row_blocks, ns), dim3(TPB), 0, s, b, edge_blocks, unit_blocks);
+    HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(k_plan_items, dim3(row_blocks + edge_blocks, ns), dim3(TPB), 0, s, b, row_blocks);
+    HIP_TRY(hipGetLastError());
+    const int64_t max_items = most_of(b, n_sides, [](const PlanSide &S) { return S.max_items; });
+    const bool sorted = b.side[0].indices != nullptr;          // (two sides: tiles, which have indices)
+    if (max_items == 0 || (!sorted && !b.side[0].bounds)) return BPT_OK;
+    hipLaunchKernelGGL(k_item_bounds, dim3(blocks_for(max_items * 16), ns), dim3(TPB), 0, s, b);
+    HIP_TRY(hipGetLastError());
+    if (!sorted) return BPT_OK;
+    const int64_t pad = most_of(b, n_sides, [](const PlanSide &S) { return S.n_index_nodes; }) + 1;
+    return rs_sort(ItemRecs{b, 0}, ItemsSorted{b}, RsSizes{{b.side[0].max_items, b.side[1].max_items}}, n_sides, (uint64_t)pad, w.key, w.val, w.counts,
+                   w.totals, s);
+}
+
+int groups_count(const PlanSides &b, int n_sides, int32_t R, const SortWs &w, hipStream_t s) {
+    const unsigned ns = (unsigned)n_sides;
+    const int64_t max_items = most_of(b, n_sides, [](const PlanSide &S) { return S.max_items; });
+    if (max_items > 0) {
+        // the items in the order of their largest neighbour; R consecutive ones are a group
+        const int64_t n_index = most_of(b, n_sides, [](const PlanSide &S) { return S.n_index_nodes; });
+        const int st = rs_sort(ItemRecs{b, 1}, ItemOrder{b}, RsSizes{{b.side[0].max_items, b.side[1].max_items}}, n_sides, (uint64_t)n_index + 1, w.key,
+                               w.val, w.counts, w.totals, s);
+        if (st != BPT_OK) return st;
+        const int64_t place_bits = most_of(b, n_sides, [](const PlanSide &S) { return S.place_bits; });
+        const bool narrow = (int64_t)bits_for((uint64_t)n_index) + 4 + place_bits <= 31;
+        const dim3 grid((unsigned)most_of(b, n_sides, [](const PlanSide &S) { return S.max_groups; }), ns);
+        auto form = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(TPB), 0, s, b, R);
+            return hipGetLastError();
+        };
+        const int64_t cap = R * most_of(b, n_sides, [](const PlanSide &S) { return S.seg_len; });
+        if (narrow) HIP_TRY(cap <= 1024 ? form(k_group_form<1024, uint32_t>) : cap <= 2048 ? form(k_group_form<2048, uint32_t>) : form(k_group_form<4096, uint32_t>));
+        else HIP_TRY(cap <= 1024 ? form(k_group_form<1024, uint64_t>) : cap <= 2048 ? form(k_group_form<2048, uint64_t>) : form(k_group_form<4096, uint64_t>));
+    }
+    hipLaunchKernelGGL(k_group_order, dim3(1, ns), dim3(GRP_ORDER_TPB), 0, s, b, R);
+    HIP_TRY(hipGetLastError());
+    return BPT_OK;
+}
+
+// counts: 16 ints per side, as the groups' info block
+int groups_write(const PlanSides &b, int n_sides, int32_t R, const int32_t *counts, const bpt_build_tiles *out, int32_t pad_entries, hipStream_t s) {
+    if (!counts || !out || pad_entries < 0) return BPT_ERR_NULL;
+    GroupsOuts outs{};
+    int32_t most = 0;
+    for (int i = 0; i < n_sides; ++i) {
+        const PlanSide &S = b.side[i];
+        const bpt_build_tiles &o = out[i];
+        const int32_t ng = counts[16 * i + BPT_GI_N_GROUPS], ne = counts[16 * i + BPT_GI_N_ENTRIES];
+        if (ng < 0 || ng > S.max_groups || ne < 0 || ne > S.n_edges) return BPT_ERR_SIZE;
+        if (!o.grp_ptr || !o.entries || !o.grp_eids || !o.chunks || !o.group_info || (ng > 0 && !o.members) || (S.n_edges > 0 && !o.pair_eid))
+            return BPT_ERR_NULL;
+        outs.side[i] = GroupsOut{ng, ne, counts[16 * i + BPT_GI_MAX_CHUNK], o.members, o.grp_ptr, o.pair_eid, o.grp_eids, o.chunks, o.group_info,
+                                 reinterpret_cast<int4 *>(o.entries), o.number};
+        most = ng > most ? ng : most;
+    }
+    hipLaunchKernelGGL(k_group_write, dim3((unsigned)most + 1, (unsigned)n_sides), dim3(TPB), 0, s, b, outs, R, pad_entries);
+    HIP_TRY(hipGetLastError());
     return BPT_OK;
 }
 
@@ -1742,31 +1928,10 @@ int csr_build(CsrSides g, int n_sides, int64_t n_edges, int64_t n_nodes, int32_t
     Bump bump{(char *)workspace, 0};
     CsrWs w = csr_layout(bump, n_edges, n_nodes, n_sides, g);
     if (workspace_bytes < (int64_t)bump.off) return BPT_ERR_WORKSPACE;
-    if (n_edges > 0) {
-        const RsPasses ps = rs_passes((uint64_t)n_nodes);       // (n_nodes: the key of an edge with a bad id)
-        const CsrEdges edges{g, n_nodes};
-        const CsrSlots slots{g};
-        RsToArrays to[2];
-        RsArrays from[2];
-        for (int t = 0; t < 2; ++t)
-            for (int i = 0; i < 2; ++i) {
-                const int64_t at = (i < n_sides ? i : 0) * n_edges;
-                to[t].k[i] = w.key[t] + at;
-                to[t].v[i] = w.val[t] + at;
-                from[t].k[i] = to[t].k[i];
-                from[t].v[i] = to[t].v[i];
-            }
-        for (int p = 0; p < ps.n; ++p) {
-            const int shift = p * ps.bits;
-            const bool first = p == 0, last = p == ps.n - 1;
-            int st;
-            if (first && last) st = rs_pass(edges, slots, n_edges, n_sides, shift, ps.bits, w.counts, w.totals, s);
-            else if (first) st = rs_pass(edges, to[0], n_edges, n_sides, shift, ps.bits, w.counts, w.totals, s);
-            else if (last) st = rs_pass(from[(p - 1) & 1], slots, n_edges, n_sides, shift, ps.bits, w.counts, w.totals, s);
-            else st = rs_pass(from[(p - 1) & 1], to[p & 1], n_edges, n_sides, shift, ps.bits, w.counts, w.totals, s);
-            if (st != BPT_OK) return st;
-        }
-    }
+    // (n_nodes: the key of an edge with a bad id)
+    const int st = rs_sort(CsrEdges{g, n_nodes}, CsrSlots{g}, RsSizes{{n_edges, n_edges}}, n_sides, (uint64_t)n_nodes, w.key, w.val, w.counts,
+                           w.totals, s);
+    if (st != BPT_OK) return st;
     const dim3 rows((unsigned)((n_nodes + CSR_ROWS) / CSR_ROWS), (unsigned)n_sides);
     hipLaunchKernelGGL(k_csr_rows, rows, dim3(TPB), 0, s, g, n_edges, n_nodes, chunk);
     HIP_TRY(hipGetLastError());
@@ -1888,7 +2053,12 @@ int bpt_plan_device_bounds(int64_t n_units, int64_t n_edges, int64_t n_rows, int
     size_t tmp = 0;
     HIP_TRY(temp_bytes(max_items, max_groups, n_edges, n_rows, &tmp));
     Bump a{nullptr, 0}, b{nullptr, 0}, c{nullptr, 0};
-    base_layout(a, n_rows, n_edges, max_items);
+    PlanSide S{};
+    S.n_edges = n_edges;
+    S.n_rows = n_rows;
+    S.max_items = max_items;
+    base_layout(a, S);
+    sort_layout(a, max_items, 1);
     group_layout(b, max_items, max_groups, n_edges, tmp);
     c.take<int32_t>(n_edges);
     size_t ws = a.off > b.off ? a.off : b.off;
@@ -1912,46 +2082,27 @@ int bpt_build_plan_device(const int64_t *row, const int64_t *indptr_units, int64
                           const int64_t *indices, int64_t n_edges, int64_t n_rows, int64_t n_index_nodes, int32_t seg_len,
                           int32_t *rowptr, int32_t *idx32, int32_t *eid32, int32_t *items, int32_t *heavy, int32_t *item_bounds,
                           int32_t *info, void *workspace, int64_t workspace_bytes, void *stream) {
-    const int st = sizes_ok(n_units, n_edges, n_rows, n_index_nodes, seg_len);
+    bpt_build_side side{row, indptr_units, eid, indices, n_units, n_edges, n_rows, n_index_nodes, seg_len, 0, rowptr, idx32, eid32, items,
+                        item_bounds, heavy, info};
+    PlanSides b{};
+    const int st = fill_side(side, b.side[0]);
     if (st != BPT_OK) return st;
-    if (!rowptr || !items || !info || !workspace) return BPT_ERR_NULL;
-    if (n_units > 0 && (!row || !indptr_units)) return BPT_ERR_NULL;
-    if (n_edges > 0 && (!eid || !idx32 || !eid32)) return BPT_ERR_NULL;
-    const int64_t max_items = n_rows + n_edges / seg_len;
-    if (max_items >= INT32_MAX) return BPT_ERR_SIZE;
-    if (n_edges / ((int64_t)seg_len + 1) > 0 && !heavy) return BPT_ERR_NULL;
+    if (!workspace) return BPT_ERR_NULL;
     Bump bump{(char *)workspace, 0};
-    BaseWs w = base_layout(bump, n_rows, n_edges, max_items);
+    base_layout(bump, b.side[0]);
+    const SortWs w = sort_layout(bump, b.side[0].max_items, 1);
     if (workspace_bytes < (int64_t)bump.off) return BPT_ERR_WORKSPACE;
-    hipStream_t s = (hipStream_t)stream;
-
-    LAUNCH(k_plan_clear, 1, info, indptr_units, n_units, n_edges);
-    const unsigned edge_blocks = blocks_for(n_edges), unit_blocks = blocks_for(n_units), row_blocks = (unsigned)item_row_blocks(n_rows);
-    hipLaunchKernelGGL(k_plan_narrow, dim3(edge_blocks + unit_blocks + row_blocks), dim3(TPB), 0, s, row, indptr_units, n_units, eid, indices,
-                       n_edges, n_rows, n_index_nodes, seg_len, edge_blocks, unit_blocks, info, idx32, eid32, w.seen, rowptr, w.totals);
-    HIP_TRY(hipGetLastError());
-    // without indices the items stay in row order, as on the host
-    int4 *const in_rows = indices ? w.items_tmp : reinterpret_cast<int4 *>(items);
-    int2 *const bounds = reinterpret_cast<int2 *>(item_bounds);
-    hipLaunchKernelGGL(k_plan_items, dim3(row_blocks + edge_blocks), dim3(TPB), 0, s, rowptr, n_rows, seg_len, w.totals, eid32, w.seen, n_edges,
-                       row_blocks, info, in_rows, heavy);
-    HIP_TRY(hipGetLastError());
-    if (max_items == 0 || (!indices && !bounds)) return BPT_OK;
-    LAUNCH(k_item_bounds, max_items * 16, in_rows, idx32, info, max_items, n_index_nodes, n_edges, indices ? w.bounds_tmp : bounds);
-    if (!indices) return BPT_OK;
-    const uint32_t pad = (uint32_t)n_index_nodes + 1;
-    const ItemRecs recs{w.bounds_tmp, info, 0, pad};
-    const ItemsSorted sorted{w.items_tmp, w.bounds_tmp, info, reinterpret_cast<int4 *>(items), bounds};
-    return rs_sort(recs, sorted, max_items, pad, w.key, w.val, w.counts, w.bin_totals, s);
+    return base_build(b, 1, w, (hipStream_t)stream);
 }
 
 int bpt_build_groups_bounds(int64_t max_items, int64_t n_edges, int64_t n_index_nodes, int32_t seg_len, int32_t R, int64_t bounds[1]) {
     if (!bounds) return BPT_ERR_NULL;
-    ShortForm f;
-    const int st = short_form(max_items, n_edges, n_index_nodes, seg_len, R, f);
+    PlanSide S{};
+    const int st = short_form(max_items, n_edges, n_index_nodes, seg_len, R, 0, S);
     if (st != BPT_OK) return st;
     Bump dry{nullptr, 0};
-    short_layout(dry, max_items, f.max_groups, n_edges);
+    short_layout(dry, S);
+    sort_layout(dry, max_items, 1);
     bounds[0] = (int64_t)dry.off + 256;
     return BPT_OK;
 }
@@ -1959,61 +2110,114 @@ int bpt_build_groups_bounds(int64_t max_items, int64_t n_edges, int64_t n_index_
 int bpt_build_groups_count(const int32_t *items, const int32_t *item_bounds, const int32_t *idx32, const int32_t *eid32,
                            const int32_t *plan_info, int64_t max_items, int64_t n_edges, int64_t n_index_nodes, int32_t seg_len, int32_t R,
                            int32_t by_mask, int32_t *out_info, void *workspace, int64_t workspace_bytes, void *stream) {
-    ShortForm f;
-    const int st = short_form(max_items, n_edges, n_index_nodes, seg_len, R, f);
+    PlanSides b{};
+    PlanSide &S = b.side[0];
+    const int st = short_form(max_items, n_edges, n_index_nodes, seg_len, R, by_mask, S);
     if (st != BPT_OK) return st;
-    if (by_mask < 0 || (by_mask & 3) > 2 || by_mask > 6) return BPT_ERR_SHAPE;
     if (!plan_info || !out_info || !workspace || (max_items > 0 && (!items || !item_bounds))) return BPT_ERR_NULL;
     if (n_edges > 0 && (!idx32 || !eid32)) return BPT_ERR_NULL;
+    S.items = (int4 *)items;
+    S.bounds = (int2 *)item_bounds;
+    S.idx32 = (int32_t *)idx32;
+    S.eid32 = (int32_t *)eid32;
+    S.info = (int32_t *)plan_info;
+    S.out_info = out_info;
     Bump bump{(char *)workspace, 0};
-    ShortWs w = short_layout(bump, max_items, f.max_groups, n_edges);
+    short_layout(bump, S);
+    const SortWs w = sort_layout(bump, max_items, 1);
     if (workspace_bytes < (int64_t)bump.off) return BPT_ERR_WORKSPACE;
-    hipStream_t s = (hipStream_t)stream;
-    const int4 *const it = reinterpret_cast<const int4 *>(items);
-    const int2 *const bd = reinterpret_cast<const int2 *>(item_bounds);
-    const int by_work = (by_mask & 4) ? 0 : 1, mode = by_mask & 3;
-    if (max_items > 0) {
-        // the items in the order of their largest neighbour; R consecutive ones are a group
-        const uint32_t pad = (uint32_t)n_index_nodes + 1;
-        const int ss = rs_sort(ItemRecs{bd, plan_info, 1, pad}, ItemOrder{w.jorder}, max_items, pad, w.key, w.val, w.counts,
-                               w.bin_totals, s);
-        if (ss != BPT_OK) return ss;
-        const bool narrow = bits_for((uint64_t)n_index_nodes) + 4 + f.place_bits <= 31;
-        auto form = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, dim3((unsigned)f.max_groups), dim3(TPB), 0, s, it, bd, w.jorder, idx32, eid32, plan_info, n_edges, seg_len, R,
-                               f.place_bits, mode, w.rec, w.entries, w.pairs);
-            return hipGetLastError();
-        };
-        const int cap = R * seg_len;
-        if (narrow) HIP_TRY(cap <= 1024 ? form(k_group_form<1024, uint32_t>) : cap <= 2048 ? form(k_group_form<2048, uint32_t>) : form(k_group_form<4096, uint32_t>));
-        else HIP_TRY(cap <= 1024 ? form(k_group_form<1024, uint64_t>) : cap <= 2048 ? form(k_group_form<2048, uint64_t>) : form(k_group_form<4096, uint64_t>));
-    }
-    // (the words of the groups are sorted in the items' key arrays, which are free again)
-    hipLaunchKernelGGL(k_group_order, dim3(1), dim3(GRP_ORDER_TPB), 0, s, w.rec, plan_info, R, by_work, f.g_bits,
-                       (int)bits_for((uint64_t)n_index_nodes), f.work_bits, w.key[0], w.key[1], w.loc_group, w.loc_work, w.loc_prefix, w.order, w.entry0, w.pair0, w.chunks, out_info);
-    HIP_TRY(hipGetLastError());
-    return BPT_OK;
+    return groups_count(b, 1, R, w, (hipStream_t)stream);
 }
 
 int bpt_build_groups_write(const int32_t *items, const int32_t *plan_info, int64_t max_items, int64_t n_edges, int64_t n_index_nodes,
                            int32_t seg_len, int32_t R, const int32_t *group_counts, int32_t pad_entries, int32_t *members,
                            int32_t *grp_ptr, int32_t *entries, int32_t *pair_eid, int32_t *grp_eids, int32_t *chunks, int32_t *group_info,
                            void *workspace, int64_t workspace_bytes, void *stream) {
-    ShortForm f;
-    const int st = short_form(max_items, n_edges, n_index_nodes, seg_len, R, f);
+    PlanSides b{};
+    PlanSide &S = b.side[0];
+    const int st = short_form(max_items, n_edges, n_index_nodes, seg_len, R, 0, S);
     if (st != BPT_OK) return st;
-    if (!plan_info || !group_counts || !grp_ptr || !entries || !grp_eids || !chunks || !group_info || !workspace) return BPT_ERR_NULL;
-    const int32_t ng = group_counts[BPT_GI_N_GROUPS], ne = group_counts[BPT_GI_N_ENTRIES];
-    if (ng < 0 || ng > f.max_groups || ne < 0 || ne > n_edges || pad_entries < 0) return BPT_ERR_SIZE;
-    if ((ng > 0 && (!items || !members)) || (n_edges > 0 && !pair_eid)) return BPT_ERR_NULL;
+    if (!plan_info || !workspace || (max_items > 0 && !items)) return BPT_ERR_NULL;
+    S.items = (int4 *)items;
+    S.info = (int32_t *)plan_info;
+    const bpt_build_tiles out{members, grp_ptr, entries, pair_eid, grp_eids, chunks, group_info, nullptr};
     Bump bump{(char *)workspace, 0};
-    ShortWs w = short_layout(bump, max_items, f.max_groups, n_edges);
+    short_layout(bump, S);
     if (workspace_bytes < (int64_t)bump.off) return BPT_ERR_WORKSPACE;
+    return groups_write(b, 1, R, group_counts, &out, pad_entries, (hipStream_t)stream);
+}
+
+// where the two calls below put a side's arrays in its part of the workspace
+static int tiles_sides(const bpt_build_side *sides, int n_sides, PlanSides &b, SortWs &w, Bump &bump) {
+    int64_t most = 0;
+    for (int i = 0; i < n_sides; ++i) {
+        const bpt_build_side &side = sides[i];
+        PlanSide &S = b.side[i];
+        int st = fill_side(side, S);
+        if (st != BPT_OK) return st;
+        if (!side.item_bounds && S.max_items > 0) return BPT_ERR_NULL;
+        st = short_form(S.max_items, S.n_edges, S.n_index_nodes, S.seg_len, 16, side.by_mask, S);
+        if (st != BPT_OK) return st;
+        base_layout(bump, S);
+        short_layout(bump, S);
+        most = S.max_items > most ? S.max_items : most;
+    }
+    w = sort_layout(bump, most, n_sides);
+    return BPT_OK;
+}
+
+int bpt_build_tiles_bounds(const bpt_build_side *sides, int n_sides, int64_t bounds[1]) {
+    if (!sides || !bounds || n_sides < 1 || n_sides > 2) return BPT_ERR_NULL;
+    int64_t most = 0;
+    Bump dry{nullptr, 0};
+    for (int i = 0; i < n_sides; ++i) {
+        const bpt_build_side &side = sides[i];
+        int st = sizes_ok(side.n_units, side.n_edges, side.n_rows, side.n_index_nodes, side.seg_len);
+        if (st != BPT_OK) return st;
+        PlanSide S{};
+        S.n_rows = side.n_rows;
+        const int64_t max_items = side.n_rows + side.n_edges / side.seg_len;
+        st = short_form(max_items, side.n_edges, side.n_index_nodes, side.seg_len, 16, side.by_mask, S);
+        if (st != BPT_OK) return st;
+        base_layout(dry, S);
+        short_layout(dry, S);
+        most = max_items > most ? max_items : most;
+    }
+    sort_layout(dry, most, n_sides);
+    bounds[0] = (int64_t)dry.off + 256;
+    return BPT_OK;
+}
+
+int bpt_build_tiles_count(const bpt_build_side *sides, int n_sides, int32_t *out_info, void *workspace, int64_t workspace_bytes, void *stream) {
+    if (!sides || !out_info || !workspace || n_sides < 1 || n_sides > 2) return BPT_ERR_NULL;
+    PlanSides b{};
+    SortWs w;
+    Bump bump{(char *)workspace, 0};
+    int st = tiles_sides(sides, n_sides, b, w, bump);
+    if (st != BPT_OK) return st;
+    if (workspace_bytes < (int64_t)bump.off) return BPT_ERR_WORKSPACE;
+    for (int i = 0; i < n_sides; ++i) b.side[i].out_info = out_info + 32 * i;
+    st = base_build(b, n_sides, w, (hipStream_t)stream);
+    return st != BPT_OK ? st : groups_count(b, n_sides, 16, w, (hipStream_t)stream);
+}
+
+int bpt_build_tiles_write(const bpt_build_side *sides, int n_sides, const int32_t *infos, const bpt_build_tiles *out, int32_t pad_entries,
+                          int32_t *pairs, void *workspace, int64_t workspace_bytes, void *stream) {
+    if (!sides || !infos || !out || !workspace || n_sides < 1 || n_sides > 2) return BPT_ERR_NULL;
+    PlanSides b{};
+    SortWs w;
+    Bump bump{(char *)workspace, 0};
+    int st = tiles_sides(sides, n_sides, b, w, bump);
+    if (st != BPT_OK) return st;
+    if (workspace_bytes < (int64_t)bump.off) return BPT_ERR_WORKSPACE;
+    const int32_t counts[32] = {infos[16], infos[17], infos[18], 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0,
+                                n_sides == 2 ? infos[48] : 0, n_sides == 2 ? infos[49] : 0, n_sides == 2 ? infos[50] : 0};
+    st = groups_write(b, n_sides, 16, counts, out, pad_entries, (hipStream_t)stream);
+    if (st != BPT_OK || !pairs) return st;
+    if (n_sides != 2 || !out[0].number || sides[0].n_edges != sides[1].n_edges) return BPT_ERR_PLAN;
     hipStream_t s = (hipStream_t)stream;
-    hipLaunchKernelGGL(k_group_write, dim3((unsigned)ng + 1), dim3(TPB), 0, s, reinterpret_cast<const int4 *>(items), w.jorder, plan_info, w.rec,
-                       w.order, w.entry0, w.pair0, w.chunks, w.entries, w.pairs, n_edges, R, ng, ne, group_counts[BPT_GI_MAX_CHUNK], pad_entries,
-                       seg_len, members, grp_ptr, reinterpret_cast<int4 *>(entries), pair_eid, grp_eids, chunks, group_info);
-    HIP_TRY(hipGetLastError());
+    const int64_t n_slots = ((int64_t)counts[16 + BPT_GI_N_ENTRIES] + pad_entries) * 16;
+    LAUNCH(k_find_numbers, n_slots, out[1].grp_eids, n_slots, sides[1].n_edges, out[0].number, pairs);
     return BPT_OK;
 }
 

@@ -206,11 +206,9 @@ def get_csrs_bipartite(src, dst, n_src, n_dst, chunk_size=32, as_torch=True):
     if len(src) and (src.min() < 0 or dst.min() < 0 or src.max() >= n_src or dst.max() >= n_dst):
         raise ValueError("node id out of range")
 
-    def side(rows, cols, n_rows):          # stable sort by row = ascending edge id inside a row, as build_csr
-        eid = np.argsort(rows, kind="stable").astype(np.int64)
-        indptr = np.zeros(n_rows + 1, dtype=np.int64)
-        np.cumsum(np.bincount(rows, minlength=n_rows), out=indptr[1:])
-        return indptr, np.ascontiguousarray(cols[eid]), eid
+    def side(rows, cols, n_rows):          # (built over the larger index space: the rows behind n_rows are empty)
+        indptr, indices, eid = build_csr(rows, cols, max(int(n_src), int(n_dst)))
+        return np.ascontiguousarray(indptr[:n_rows + 1]), indices, eid
 
     out_csr = side(src, dst, int(n_src))
     in_csr = side(dst, src, int(n_dst))
@@ -280,39 +278,19 @@ def nli_inter_graph_edges(premise_graphs, hypo_graphs):
 
 def get_csrs_device(src, dst, n_nodes, chunk_size=32):
     """get_csrs for an edge list that already lives on the GPU (int64 CUDA tensors): the same 6-tuple, built there by
-    libbptplan (bpt_build_csrs_device: a stable radix sort by row of both sides at once, binary searches, a prefix sum) and
+    libbptplan (bptop.so calls bpt_build_csrs_device: a stable radix sort by row of both sides at once, binary searches, a prefix sum) and
     bit for bit what get_csrs returns for the same edges.  One synchronisation (the number of units of each side comes back)."""
     import torch
-    from ._lib import plan_lib
+    from ._native import native
     if not (src.is_cuda and dst.is_cuda and src.dtype == torch.int64 and dst.dtype == torch.int64):
         raise ValueError("src and dst must be int64 CUDA tensors")
-    if src.shape != dst.shape or src.dim() != 1:
-        raise ValueError("src and dst must be 1-D tensors of the same length")
-    src, dst = src.contiguous(), dst.contiguous()
-    lib, E, n, dev = plan_lib(), int(src.numel()), int(n_nodes), src.device
-    b = (ctypes.c_int64 * 2)()
-    st = lib.bpt_csr_device_bounds(E, n, int(chunk_size), ctypes.byref(b))
-    if st != 0:
-        raise RuntimeError(f"bpt_csr_device_bounds: status {st}")
-    max_units = int(b[0])
-    with torch.cuda.device(dev):
-        stream = torch.cuda.current_stream().cuda_stream
-        sides = [tuple(torch.empty(max(k, 1), dtype=torch.int64, device=dev) for k in (n + 1, E, E, max_units, max_units + 1))
-                 for _ in range(2)]
-        ptrs = [(ctypes.c_void_p * 5)(*(t.data_ptr() for t in side)) for side in sides]
-        ws = torch.empty(int(b[1]), dtype=torch.uint8, device=dev)
-        info = torch.empty(4, dtype=torch.int32, pin_memory=True)         # (written by the last kernel: no copy to wait for)
-        st = lib.bpt_build_csrs_device(src.data_ptr() if E else None, dst.data_ptr() if E else None, E, n, int(chunk_size),
-                                           ctypes.byref(ptrs[0]), ctypes.byref(ptrs[1]), info.data_ptr(), ws.data_ptr(), ws.numel(), stream)
-        if st != 0:
-            raise RuntimeError(f"bpt_build_csrs_device: status {st}")
-        st = lib.bpt_build_wait(stream)
-        if st != 0:
-            raise RuntimeError(f"bpt_build_wait: status {st}")
-    err_out, n_out, err_in, n_in = info.tolist()
+    if src.shape != dst.shape or src.dim() != 1 or src.device != dst.device:
+        raise ValueError("src and dst must be 1-D tensors of the same length on one device")
+    E = src.numel()
+    out_side, in_side, (err_out, n_out, err_in, n_in) = native.build_csrs(src.contiguous(), dst.contiguous(), int(n_nodes), int(chunk_size))
     if err_out or err_in:
         raise ValueError("bptplan: row id, column id or edge id out of range")
-    (p_out, x_out, e_out, row, row_ptr), (p_in, x_in, e_in, col, col_ptr) = sides
+    (p_out, x_out, e_out, row, row_ptr), (p_in, x_in, e_in, col, col_ptr) = out_side, in_side
     return ((p_out, x_out[:E], e_out[:E]), (p_in, x_in[:E], e_in[:E]), row[:n_out], row_ptr[:n_out + 1], col[:n_in], col_ptr[:n_in + 1])
 
 

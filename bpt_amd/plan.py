@@ -290,6 +290,7 @@ class Plan:
                 st.grp_eids = dev["eids"].data_ptr()
                 hit = {"host": grp, "dev": dev, "struct": st}
                 self._groups[(R, order_mode)] = hit
+                PlanCache.grown += 1
         return hit
 
     def bias_rows(self, R=TILE_GROUP_R):
@@ -306,6 +307,7 @@ class Plan:
                 torch.cuda.current_stream(self.device).synchronize()      # complete before another stream may read it
             with self._lock:
                 self._bias_rows[R] = hit
+                PlanCache.grown += 1
         return hit
 
     def linked_to(self, plan_src, R=GROUP_R, order=None, partner_order=GROUP_ORDER_SRC, pair_numbers=False):
@@ -338,6 +340,7 @@ class Plan:
                 st.grp_pairs = pairs.data_ptr()
                 hit = (st, pairs, plan_src)          # keeps the mapping and the partner alive
                 self._links[key] = hit
+                PlanCache.grown += 1
         return hit[0]
 
 
@@ -449,17 +452,54 @@ class DevicePlan:
             _check_plan(st, "bpt_build_plan_device")
             formed = None if groups is None else self._form_groups(groups[0], self._by_mask(groups[0], groups[1]))
         h = self._info.cpu().tolist() if formed is None else formed["info"]      # the one synchronisation of the build
+        self._describe(h)
+        if formed is not None:
+            self._write_groups(formed)
+
+    @classmethod
+    def tile_plans(cls, sides):
+        """The plans, with their tile groups, of one side of a graph or of both, built together (bpt_build_tiles_count / _write in
+        bptop.so); the second is linked to the first by pair numbers.  sides: (row, indptr, eid, indices, n_rows, n_index_nodes,
+        seg_len, order_mode of the groups).  None where the plans have to be built one by one."""
+        self_of = []
+        for row, indptr, eid, indices, n_rows, n_index_nodes, seg_len, order in sides:
+            self = cls.__new__(cls)
+            self.device, self.seg_len, self.has_indices = eid.device, int(seg_len), True
+            self.n_rows, self.n_edges, self.n_index_nodes = int(n_rows), int(eid.numel()), int(n_index_nodes)
+            self._groups, self._links, self._bias_rows, self._lock = {}, {}, {}, threading.Lock()
+            self._max_items = self.n_rows + self.n_edges // self.seg_len
+            self_of.append((self, self._by_mask(TILE_GROUP_R, order)))
+        built = PlanCache.native.build_tile_plans([(*side[:7], by_mask) for side, (_, by_mask) in zip(sides, self_of)])
+        if built is None:
+            return None
+        arrays, pairs = built
+        for (self, _), (info, base, _) in zip(self_of, arrays):
+            self._info = base[6]
+            self._dev = dict(zip(("rowptr", "idx", "eid", "items", "bounds", "heavy"), base))
+            self._describe(info)                          # (raises where a side is malformed: the groups of neither are there then)
+        for (self, by_mask), (info, _, groups) in zip(self_of, arrays):
+            ng, ne, max_chunk = info[16:19]
+            self._keep_groups(dict(zip(("members", "grp_ptr", "entries", "pair_eid", "eids", "chunks", "ginfo"), groups)), TILE_GROUP_R,
+                              by_mask, ng, ne, max_chunk, wait=False)
+        plans = [self for self, _ in self_of]
+        if pairs is not None:
+            st = PlanStruct.from_buffer_copy(plans[1]._groups[(TILE_GROUP_R, self_of[1][1])]["struct"])
+            st.grp_pairs = pairs.data_ptr()
+            plans[1]._links[(id(plans[0]), TILE_GROUP_R, sides[1][7], sides[0][7], True)] = (st, pairs, plans[0])
+        return plans
+
+    def _describe(self, h):
+        """The plan's numbers and its struct from the info block that came back."""
         if h[0] != 0:
             raise ValueError("bptplan: " + _PLAN_ERRORS.get(h[0], f"error {h[0]}"))
         self.n_items, self.n_heavy, self.n_slots, self.max_degree = h[1], h[2], h[3], h[4]
         self.covers_all_edges = bool(h[5] & 1)
+        d, E = self._dev, self.n_edges
         self.struct = PlanStruct(
             d["rowptr"].data_ptr(), d["idx"].data_ptr() if E else None, d["eid"].data_ptr() if E else None,
             d["items"].data_ptr() if self.n_items else None, d["heavy"].data_ptr() if self.n_heavy else None,
             self.n_rows, E, self.n_items, self.n_heavy, self.n_slots)
         self.struct.n_index_nodes = self.n_index_nodes
-        if formed is not None:
-            self._write_groups(formed)
 
     def _auto_seg_len(self, row, indptr):
         """auto_seg_len on the device: the 90 % quantile of the non-empty rows' degrees."""
@@ -527,7 +567,7 @@ class DevicePlan:
             _check_plan(st, "bpt_build_groups_write")
             return self._keep_groups(dev, R, formed["by_mask"], ng, ne, max_chunk)
 
-    def _keep_groups(self, dev, R, by_mask, ng, ne, max_chunk):
+    def _keep_groups(self, dev, R, by_mask, ng, ne, max_chunk, wait=True):
         st = PlanStruct.from_buffer_copy(self.struct)
         st.grp_members = dev["members"].data_ptr() if ng else None
         st.grp_ptr = dev["grp_ptr"].data_ptr()
@@ -540,7 +580,9 @@ class DevicePlan:
         st.n_grp_entries = ne
         st.grp_eids = dev["eids"].data_ptr()
         hit = _Groups(dev=dev, struct=st, R=R, n_edges=self.n_edges)
-        self._wait()
+        if wait:
+            self._wait()
+            PlanCache.grown += 1
         self._groups[(R, by_mask)] = hit
         return hit
 
@@ -597,6 +639,7 @@ class DevicePlan:
             self._wait()
             with self._lock:
                 self._bias_rows[R] = hit
+                PlanCache.grown += 1
         return hit
 
     def linked_to(self, plan_src, R=GROUP_R, order=None, partner_order=GROUP_ORDER_SRC, pair_numbers=False):
@@ -619,6 +662,7 @@ class DevicePlan:
                     st.grp_pairs = pairs.data_ptr()
                     hit = (st, pairs, plan_src)
                     self._links[key] = hit
+                    PlanCache.grown += 1
                     return hit[0]
                 if pair_numbers:
                     n_slots = mine["dev"]["eids"].numel()
@@ -633,6 +677,7 @@ class DevicePlan:
                     st.grp_pairs = pairs.data_ptr()
                     hit = (st, pairs, plan_src)
                     self._links[key] = hit
+                    PlanCache.grown += 1
                     return hit[0]
                 n_pairs = (mine["struct"].n_grp_entries + GROUP_PAD_ENTRIES) * R
                 pairs = torch.empty((E + GROUP_PAD_ENTRIES) * R, dtype=torch.int32, device=self.device)
@@ -649,6 +694,7 @@ class DevicePlan:
                 st.grp_pairs = pairs.data_ptr()
                 hit = (st, pairs, plan_src)
                 self._links[key] = hit
+                PlanCache.grown += 1
         return hit[0]
 
 
@@ -683,9 +729,21 @@ class PlanCache:
     # it says which plans it used when one has to go, and is told which one went
     native = None
 
+    # how often a plan got groups, a pair mapping or pair-order tables after it was made: the bytes are then counted again
+    grown = 0
+    _total, _counted = 0, 0
+
+    def _insert(self, key, plan, tensors):
+        # called with the lock held
+        old = self._d.pop(key, None)
+        self._d[key] = (plan, tensors)
+        self._total += plan.device_bytes() - (old[0].device_bytes() if old is not None else 0)
+
     def _evict(self):
         # called with the lock held; the newest entry always stays
-        total = sum(p.device_bytes() for p, _ in self._d.values()) if len(self._d) > 1 else 0
+        if self._counted != PlanCache.grown:
+            self._counted, self._total = PlanCache.grown, sum(p.device_bytes() for p, _ in self._d.values())
+        total = self._total
         if len(self._d) <= self._cap and total <= self._max_bytes:
             return
         if self.native is not None and len(self._d) > 1:
@@ -696,6 +754,7 @@ class PlanCache:
         while len(self._d) > max(self._cap, 1) or (len(self._d) > 1 and total > self._max_bytes):
             _, (p, _) = self._d.popitem(last=False)
             total -= p.device_bytes()
+            self._total = total
             if self.native is not None:
                 self.native.forget(p)
 
@@ -731,13 +790,32 @@ class PlanCache:
             ni = n_index_nodes if n_index_nodes is not None else nr
             plan = Plan(row_h, indptr, eid, indices, nr, ni, eid.device, seg_len)
         with self._lock:
-            self._d[key] = (plan, tensors)          # tensors kept alive with the entry
+            self._insert(key, plan, tensors)        # tensors kept alive with the entry
             self._evict()
         return plan
+
+    def put_tile_plans(self, sides):
+        """What get() would build one after the other for a training step on tiles, built together (DevicePlan.tile_plans; sides as
+        there: the in-side, then the out-side), unless one of them is already here or they have to be built one by one."""
+        if self.native is None or DEVICE_BUILD is False or not sides[0][2].is_cuda:
+            return
+        keys = [self._key(side[:4], side[4], side[5], side[6], True) for side in sides]
+        with self._lock:
+            if any(key in self._d for key in keys):
+                return
+        plans = DevicePlan.tile_plans(sides)
+        if plans is None:
+            return
+        self.misses += len(plans)
+        with self._lock:
+            for key, plan, side in zip(keys, plans, sides):
+                self._insert(key, plan, side[:4])
+            self._evict()
 
     def clear(self):
         with self._lock:
             self._d.clear()
+            self._total = 0
             if self.native is not None:
                 self.native.clear()
 

@@ -49,6 +49,26 @@ int bpt_build_groups_write(const int32_t *items, const int32_t *plan_info, int64
                            int32_t *members, int32_t *grp_ptr, int32_t *entries, int32_t *pair_eid, int32_t *grp_eids,
                            int32_t *chunks, int32_t *group_info, void *workspace, int64_t workspace_bytes, void *stream);
 
+/* The tile plans (groups of 16 rows) of one or two sides of a graph in shared launches: base plan, then groups, as the calls above.
+ * bpt_build_tiles_bounds: workspace bytes (from the sizes alone), or BPT_ERR_UNSUPPORTED as bpt_build_groups_bounds.
+ * bpt_build_tiles_count: base plans written, out_info int32[32] per side as bpt_build_groups_count's.  bpt_build_tiles_write: the
+ * arrays of the groups, given those info blocks on the host; with pairs (((n_entries + pad_entries) * 16) int32 of side 1) also the
+ * pair mapping of side 1 to side 0 (bpt_build_pair_numbers), for which out[0].number holds n_edges int32. */
+typedef struct {
+    const int64_t *row, *indptr_units, *eid, *indices;
+    int64_t n_units, n_edges, n_rows, n_index_nodes;
+    int32_t seg_len, by_mask;
+    int32_t *rowptr, *idx32, *eid32, *items, *item_bounds, *heavy, *info;
+} bpt_build_side;
+typedef struct {
+    int32_t *members, *grp_ptr, *entries, *pair_eid, *grp_eids, *chunks, *group_info, *number;
+} bpt_build_tiles;
+int bpt_build_tiles_bounds(const bpt_build_side *sides, int n_sides, int64_t bounds[1]);
+int bpt_build_tiles_count(const bpt_build_side *sides, int n_sides, int32_t *out_info, void *workspace, int64_t workspace_bytes,
+                          void *stream);
+int bpt_build_tiles_write(const bpt_build_side *sides, int n_sides, const int32_t *infos, const bpt_build_tiles *out,
+                          int32_t pad_entries, int32_t *pairs, void *workspace, int64_t workspace_bytes, void *stream);
+
 /* For every (entry, member) of one side's groups (grp_eids_mine, n_slots) the number of the same edge's pair on the other side
  * (pair_eid_theirs, n_edges), 0 where there is none.  number: n_edges int32 of scratch. */
 int bpt_build_pair_numbers(const int32_t *pair_eid_theirs, const int32_t *grp_eids_mine, int64_t n_slots, int64_t n_edges,

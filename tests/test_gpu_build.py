@@ -79,3 +79,49 @@ def test_merge_at_the_edges_of_a_launch(n_graphs):
     assert got[4] == want[4]
     for a, b in zip(got[:4], want[:4]):
         assert a.dtype == torch.int64 and np.array_equal(a.cpu().numpy(), b)
+
+
+@pytest.mark.parametrize("n_src,n_dst,E,seg,orders", [(300, 300, 6000, 64, (None, 0)), (40, 900, 5000, 64, (6, 6)), (900, 40, 5000, 128, (4, 2)),
+                                                      (1, 1, 1, 64, (None, 0)), (5000, 64, 70000, 64, (None, 0))])
+def test_both_sides_built_together(n_src, n_dst, E, seg, orders):
+    """DevicePlan.tile_plans: both sides of a graph in shared launches equal the plans built one by one (the model), the second
+    linked to the first; sides of different sizes share the launches of the larger one."""
+    from bpt_amd import graphbuilder as gb
+    from bpt_amd.plan import DevicePlan, pair_numbers_host
+    rng = np.random.default_rng(E)
+    src, dst = rng.integers(0, n_src, E).astype(np.int64), rng.integers(0, n_dst, E).astype(np.int64)
+    dst[: E // 3] = n_dst // 2
+    if E > 4:
+        src[-3:], dst[-3:] = src[-4], dst[-4]                     # an edge four times
+    out_csr, in_csr, ROW, IR, COL, IC = gb.get_csrs_bipartite(src, dst, n_src, n_dst, as_torch=False)
+    sides = [((COL, IC, in_csr[2], in_csr[1]), n_dst, n_src), ((ROW, IR, out_csr[2], out_csr[1]), n_src, n_dst)]
+    plans = DevicePlan.tile_plans([(*(torch.from_numpy(np.ascontiguousarray(a)).to(DEV) for a in arrs), n, ni, seg, order)
+                                   for (arrs, n, ni), order in zip(sides, orders)])
+    want = []
+    for plan, (arrs, n, ni), order in zip(plans, sides, orders):
+        base, info = model.base_plan(*arrs, n, ni, seg)
+        check_base(plan, base, info)
+        by_mask = plan._by_mask(16, order)
+        want.append(model.group_plan(base, ni, 16, by_mask))
+        hit = plan.ensure_groups(16, order)
+        check_groups(hit, want[-1], E)
+        assert list(plan._groups) == [(16, by_mask)], "the groups were built a second time"
+    st = plans[1].linked_to(plans[0], 16, order=orders[1], partner_order=orders[0], pair_numbers=True)
+    (_, pairs, partner), = plans[1]._links.values()
+    assert partner is plans[0] and st.grp_pairs == pairs.data_ptr()
+    assert np.array_equal(pairs.cpu().numpy(), pair_numbers_host(want[1], want[0], E))
+
+
+def test_malformed_sides_are_refused_together():
+    from bpt_amd import graphbuilder as gb
+    from bpt_amd.plan import DevicePlan
+    src, dst = random_edges(50, 400, False)
+    out_csr, in_csr, ROW, IR, COL, IC = gb.get_csrs(src, dst, 50)
+    good = [tuple(t.to(DEV) for t in side) for side in ((COL, IC, in_csr[2], in_csr[1]), (ROW, IR, out_csr[2], out_csr[1]))]
+    for side in (0, 1):
+        bad = [list(g) for g in good]
+        bad[side][3] = bad[side][3].clone()
+        bad[side][3][7] = 50
+        with pytest.raises(ValueError, match="out of range"):
+            DevicePlan.tile_plans([(*g, 50, 50, 64, None) for g in bad])
+    assert DevicePlan.tile_plans([(*g, 50, 50, 64, None) for g in good])[0].n_rows == 50
