@@ -2306,14 +2306,14 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
 //   LDS, see tile_rows_to_operand_bf16) and loads columns 4 c .. 4 c + 3 of the rows of entries 4 g + r (8 bytes; the B
 //   operand of output columns {4 c + nb} takes element nb of each of the four, packed by byte permutes).
 // Probabilities and ds are rounded to bfloat16 where they enter a product (the softmax denominator is summed unrounded);
-// the scratch between the two backward kernels holds (p, ds) as two bfloat16 in 4 bytes, by head and destination-side pair number.
+// the scratch between the two backward kernels, where there is one, holds (p, ds) as two bfloat16 in 4 bytes, by head and destination-side pair number.
 // The two-stage register pipeline of tile_walk does not pay here: at six wavefronts per SIMD it spills (2.4 x slower),
 // at four it measured 5 to 10 % slower on the sparse graphs and level on the window graph.  Tiles of 32 rows (two member
 // blocks per wavefront on the same loaded rows, three or four wavefronts per SIMD) did not pay either: the entry lists
 // shrink by a third on the destination side but only by an eighth on the source side (L = 8192, k = 4: 67 k -> 46 k and
 // 71 k -> 62 k entries), and the step went from 0.113 to 0.117 ms (32-graph batch 0.177 -> 0.205, window 128 level).
 constexpr bool TILE_BF16_PIPE = false;
-constexpr int TILE_BF16_WPE = 5, TILE_BF16_WPE_DST = 5, TILE_BF16_WPE_SRC = 5;     // wavefronts per SIMD the bfloat16 tile kernels are compiled for
+constexpr int TILE_BF16_WPE = 5, TILE_BF16_WPE_DST = 5, TILE_BF16_WPE_SRC = 5, TILE_BF16_WPE_AGAIN = 4;     // wavefronts per SIMD the bfloat16 tile kernels are compiled for
 typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
 typedef float floatx2v __attribute__((ext_vector_type(2)));
@@ -2516,20 +2516,24 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     }
 }
 
-template <int H, int D, int HW, int WPE, bool PIPE, bool DROP, int BIAS, bool NARROW = false>
+// Destination side.  PDS: (p, ds) of the pairs go to the scratch for the source side that reads them back; otherwise that side
+// forms them again (k_attn_bwd_src_tile_bf16_again) and all it is handed is (lse, delta) of the rows, `stat` (n, H): the
+// segments of a split row write the same values.
+template <int H, int D, int HW, int WPE, bool PIPE, bool DROP, int BIAS, bool PDS, bool NARROW = false>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP || BIAS ? WPE - 1 : WPE))) void k_attn_bwd_dst_tile_bf16(
     bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, const bf16_t *__restrict__ o,
     const bf16_t *__restrict__ d_o, const float *__restrict__ lse, bf16_t *__restrict__ dq, uint32_t *__restrict__ pds,
-    float *__restrict__ ws_dq, float scale, float scale_log2e, uint32_t drop_thr, uint32_t drop_seed, float drop_inv,
+    float2 *__restrict__ stat, float *__restrict__ ws_dq, float scale, float scale_log2e, uint32_t drop_thr, uint32_t drop_seed, float drop_inv,
     const float *__restrict__ bias, float *__restrict__ ds_out, Narrow nw) {
+    static_assert(PDS || BIAS == 0, "the score term's gradient is stored by the pair's position");
     const int Hs = NARROW ? nw.h : H;
     const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * 2 : (uint32_t)(H * D * 2);
     TileCtx t;
     if (!tile_begin<bf16_t, H, D, HW, NARROW>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
-    __shared__ int fst_lds[HW][TILE_CHUNK];
+    __shared__ int fst_lds[HW][PDS ? TILE_CHUNK : 1];
     int2 *ent = ent_lds[t.wv];
-    int *fst = fst_lds[t.wv];
+    int *fst = PDS ? fst_lds[t.wv] : nullptr;
     __shared__ __attribute__((aligned(16))) char kt_lds[HW][TILE_R * TILE_KT_BYTES_BF16];
     char *kt = kt_lds[t.wv];
     TileEntryRegs er;
@@ -2559,14 +2563,18 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
         }
         part += __shfl_xor(part, 16);
         delta = part + __shfl_xor(part, 32);                      // dO . O of member c, this head
-        lse_c = lse[(size_t)max(t.member.x, 0) * Hs + t.head];
+        const size_t at = (size_t)max(t.member.x, 0) * Hs + t.head;
+        lse_c = lse[at];
+        if constexpr (!PDS) {
+            if (g == 0 && t.member.x >= 0) stat[at] = make_float2(lse_c, delta);
+        }
     }
     floatx4v acc[4];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
     struct Blk {
         uint2 kc[4], vc[4];                                       // columns 4 c .. 4 c + 3 of the K / V rows of entries 4 g + r
-        int has, pos[4];                                           // bit r of has: the pair (entry 4 g + r, member c) exists
+        int has, pos[PDS ? 4 : 1];                                 // bit r of has: the pair (entry 4 g + r, member c) exists
         int xe[DROP || BIAS == 1 ? 4 : 1];
         float bz[BIAS ? 4 : 1];
     };
@@ -2578,18 +2586,20 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
             if constexpr (DROP || BIAS == 1) tile_pair_eids(P, p0 + TILE_R * b + 4 * g, t.p_end, c, B.xe);
             const int4 e01 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g]);
             const int4 e23 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g + 2]);
-            const int4 f4 = *reinterpret_cast<const int4 *>(&fst[TILE_R * b + 4 * g]);
             const int idxv[4] = {e01.x, e01.z, e23.x, e23.z};
             B.has = ((e01.y >> c) & 1) | (((e01.w >> c) & 1) << 1) | (((e23.y >> c) & 1) << 2) | (((e23.w >> c) & 1) << 3);
-            B.pos[0] = tile_pair_number(f4.x, e01.y, c); B.pos[1] = tile_pair_number(f4.y, e01.w, c);
-            B.pos[2] = tile_pair_number(f4.z, e23.y, c); B.pos[3] = tile_pair_number(f4.w, e23.w, c);
+            if constexpr (PDS) {
+                const int4 f4 = *reinterpret_cast<const int4 *>(&fst[TILE_R * b + 4 * g]);
+                B.pos[0] = tile_pair_number(f4.x, e01.y, c); B.pos[1] = tile_pair_number(f4.y, e01.w, c);
+                B.pos[2] = tile_pair_number(f4.z, e23.y, c); B.pos[3] = tile_pair_number(f4.w, e23.w, c);
+            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) B.kc[r] = tile_row4_bf16<NARROW>(kb + ((uint32_t)idxv[r] * RB + offc));
 #pragma unroll
             for (int r = 0; r < 4; ++r) B.vc[r] = tile_row4_bf16<NARROW>(vb + ((uint32_t)idxv[r] * RB + offc));
             if constexpr (BIAS) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], B.pos[r])];
+                for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], B.pos[PDS ? r : 0])];
             }
         };
         auto compute = [&](const Blk &B) {
@@ -2608,9 +2618,9 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
                     mt = dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)Hs + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
                 ds[r] = pe * (dp[r] * mt - delta) * scale;
                 pe *= mt;                                         // what multiplies v (forward) and dO (dV)
-                if (has) {
-                    pds_h[B.pos[r]] = pack_bf16(pe, ds[r]);
-                    if constexpr (BIAS) ds_out[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], B.pos[r])] = ds[r];   // dL/d(score before scaling)
+                if (PDS && has) {
+                    pds_h[B.pos[PDS ? r : 0]] = pack_bf16(pe, ds[r]);
+                    if constexpr (BIAS) ds_out[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], B.pos[PDS ? r : 0])] = ds[r];   // dL/d(score before scaling)
                 }
             }
             Bf4 da;
@@ -2694,6 +2704,102 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     }
     tile_store_rows<H, D, false, NARROW>(t, ak, 1.f, dk, ws_dk, nw);
     tile_store_rows<H, D, false, NARROW>(t, av, 1.f, dv, ws_dv, nw);
+}
+
+// Source side without the scratch: p and ds of a block's pairs are formed again from the entries' q and dO rows, which are
+// loaded for the products over the entries anyway and turned in LDS, the members' k and v rows (held as operands) and the
+// entries' (lse, delta), which the destination side leaves in `stat` (n, H).
+// Why: the scratch holds 4 bytes per pair and head, as much as the node tensors on a dense graph, and reading it back is a
+// gather of 4-byte words over 16 to 32 cache lines per instruction.  At L = 32768, k = 8, 16 heads the stores cost the
+// destination side 70 of 295 us and the gathers this side 105 of 370 (the kernels without them, timing only); four more
+// bfloat16 matrix instructions and two turns in LDS per block cost 70: 295 + 370 -> 237 + 315 us, the step 890 -> 782.
+// Both backward kernels together at 8 heads: L = 8192, k = 4 60.8 -> 57.0 us; L = 4096, k = 32 64.7 -> 48.7; window 128 39.7 ->
+// 30.9; L = 32768, k = 2 235 -> 221; 32-graph batch 102.5 -> 99.2; L = 512 and L = 8192 with dropout level.  (6 heads of 50
+// columns with dropout lost 2 %: heads of fewer than 64 columns keep the scratch.)  float32 keeps it too: there the two
+// products are 1024 cycles of the matrix pipeline per block.  118 registers: compiled for four wavefronts per SIMD (for five,
+// with the members' rows in LDS or not, it spills: 658 us; four with them in LDS 316; q rows a block ahead spills too: 346).
+template <int H, int D, int HW, int WPE, bool DROP>
+__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))) void k_attn_bwd_src_tile_bf16_again(
+    bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, const bf16_t *__restrict__ d_o,
+    const float2 *__restrict__ stat, bf16_t *__restrict__ dk, bf16_t *__restrict__ dv, float *__restrict__ ws_dk, float *__restrict__ ws_dv,
+    float scale, float scale_log2e, uint32_t drop_thr, uint32_t drop_seed, float drop_inv) {
+    constexpr uint32_t RB = H * D * 2;
+    const Narrow nw{};
+    TileCtx t;
+    if (!tile_begin<bf16_t, H, D, HW>(P, t, nw)) return;
+    __shared__ int2 ent_lds[HW][TILE_CHUNK];
+    __shared__ __attribute__((aligned(16))) char kt_lds[HW][TILE_R * TILE_KT_BYTES_BF16];
+    __shared__ __attribute__((aligned(16))) float2 stat_lds[HW][TILE_R];
+    int2 *ent = ent_lds[t.wv];
+    char *kt = kt_lds[t.wv];
+    float2 *const st_lds = stat_lds[t.wv];
+    TileEntryRegs er;
+    if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
+    issue_loads_first();
+    const int c = t.c, g = t.g;
+    const uint32_t offr = (uint32_t)((t.head * D + 16 * g) * 2), offc = t.offv;
+    const char *qb = reinterpret_cast<const char *>(q), *db = reinterpret_cast<const char *>(d_o);
+    const size_t mrow = (size_t)max(t.member.x, 0) * RB + offr;
+    const float2 *const stat_h = stat + t.head;
+    Bf8 kb[2], vb[2];
+    tile_load_row_bf16<false>(reinterpret_cast<const char *>(k) + mrow, kb, g, nw);
+    tile_load_row_bf16<false>(reinterpret_cast<const char *>(v) + mrow, vb, g, nw);
+    floatx4v ak[4], av[4];
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) { ak[nb] = floatx4v{0.f, 0.f, 0.f, 0.f}; av[nb] = floatx4v{0.f, 0.f, 0.f, 0.f}; }
+    struct Blk {
+        uint2 qr[4], dr[4];                                       // columns 4 c .. 4 c + 3 of the q / dO rows of entries 4 g + r
+        float2 ld;                                                // (lse, delta) of entry c
+        int has;                                                  // bit r: the pair (entry 4 g + r, member c) exists
+        int xe[DROP ? 4 : 1];
+    };
+    for (int p0 = t.p_begin; p0 < t.p_end; p0 += TILE_CHUNK) {
+        const int cnt = min(TILE_CHUNK, t.p_end - p0), nblk = (cnt + TILE_R - 1) / TILE_R;
+        if (p0 != t.p_begin) tile_ask_entries(P, p0, cnt, t.lane, er);
+        tile_put_entries(er, ent, cnt, t.lane);
+        auto issue = [&](Blk &B, int b) {
+            if constexpr (DROP) tile_pair_eids(P, p0 + TILE_R * b + 4 * g, t.p_end, c, B.xe);
+            const int4 e01 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g]);
+            const int4 e23 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g + 2]);
+            const int idxv[4] = {e01.x, e01.z, e23.x, e23.z};
+            B.has = ((e01.y >> c) & 1) | (((e01.w >> c) & 1) << 1) | (((e23.y >> c) & 1) << 2) | (((e23.w >> c) & 1) << 3);
+            B.ld = stat_h[(size_t)ent[TILE_R * b + c].x * H];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) B.qr[r] = tile_row4_bf16<false>(qb + ((uint32_t)idxv[r] * RB + offc));
+#pragma unroll
+            for (int r = 0; r < 4; ++r) B.dr[r] = tile_row4_bf16<false>(db + ((uint32_t)idxv[r] * RB + offc));
+        };
+        auto compute = [&](const Blk &B) {
+            if (g == 0) st_lds[c] = B.ld;
+            Bf8 row[2];
+            tile_rows_to_operand_bf16(kt, B.qr, c, g, row);
+            const floatx4v l01 = *reinterpret_cast<const floatx4v *>(&st_lds[4 * g]), l23 = *reinterpret_cast<const floatx4v *>(&st_lds[4 * g + 2]);
+            const float lse_e[4] = {l01[0], l01[2], l23[0], l23[2]}, delta_e[4] = {l01[1], l01[3], l23[1], l23[3]};
+            const floatx4v st = tile_dot_bf16(row, kb);
+            tile_rows_to_operand_bf16(kt, B.dr, c, g, row);
+            const floatx4v dp = tile_dot_bf16(row, vb);
+            float pe[4], ds[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const bool has = (B.has >> r) & 1;
+                const float p = has ? __builtin_amdgcn_exp2f(st[r] * scale_log2e - lse_e[r]) : 0.f;
+                float mt = 1.f;                                   // dropout multiplier of this pair (as in the forward)
+                if constexpr (DROP)
+                    mt = dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)H + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
+                ds[r] = has ? p * (dp[r] * mt - delta_e[r]) * scale : 0.f;
+                pe[r] = p * mt;
+            }
+            Bf4 pa, da;
+            da.u[0] = pack_bf16(ds[0], ds[1]); da.u[1] = pack_bf16(ds[2], ds[3]);
+            pa.u[0] = pack_bf16(pe[0], pe[1]); pa.u[1] = pack_bf16(pe[2], pe[3]);
+            tile_axpy_bf16(da, B.qr, ak);
+            tile_axpy_bf16(pa, B.dr, av);
+        };
+        tile_walk<false, Blk>(nblk, issue, compute);
+        wave_lds_fence();
+    }
+    tile_store_rows<H, D, false, false>(t, ak, 1.f, dk, ws_dk, nw);
+    tile_store_rows<H, D, false, false>(t, av, 1.f, dv, ws_dv, nw);
 }
 
 // Backward, destination side.  Writes (p, ds) of every pair to pds[(t * H + head)], t = the pair's
@@ -4090,8 +4196,13 @@ inline bool tiled_backward(const bpt_plan *Pin, const bpt_plan *Pout, int h, int
 inline int64_t pds_bytes(const bpt_plan *Pin, const bpt_plan *Pout, int h, int d, size_t elem) {
     int64_t n = Pin->n_edges;
     if (Pout && grouped_backward(Pin, Pout, h, d, elem)) n = std::max(n, (Pout->n_grp_entries + GRP_PAD_ENTRIES) * Pout->grp_R);
+    if (Pout && elem == 2 && tiled_backward(Pin, Pout, h, d, elem)) n = std::max(n, std::max(Pin->n_rows, Pout->n_index_nodes));   // (lse, delta) of the rows
     return 2 * round16(n * h * 4);
 }
+
+// Whether the source side of the bfloat16 tile kernels forms (p, ds) again instead of reading them back: with a score term
+// it would have to look that up by the pair's position all the same, and the dropout decision needs the pair's edge id.
+inline bool forms_pairs_again(const bpt_plan *Pout, const Dropout &drop, const float *bias) { return !bias && (drop.thr == 0 || Pout->grp_eids); }
 
 // how the tile kernels find the score term: 0 none, 1 by edge id, 2 in the plan's own pair order, head-major
 inline int tile_bias_mode(const bpt_plan *P, const float *bias) { return !bias ? 0 : P->bias_by_pair ? 2 : 1; }
@@ -4235,22 +4346,24 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
     }
     if constexpr (D == 64 && sizeof(T) == 2) {
         if (tiled_backward(Pin, Pout, H, D, sizeof(T)) && ((drop.thr == 0 && !bias) || Pin->grp_eids)) {
+            const bool again = forms_pairs_again(Pout, drop, bias);
             constexpr int HW = H >= 4 ? 4 : H;
             float *ws_dk = ws_rows + (size_t)Pin->n_slots * H * D, *ws_dv = ws_dk + (size_t)Pout->n_slots * H * D;
             {
                 ProfScope prof(BPT_KERNEL_ATTN_BWD_DST, s);
-#define LAUNCH_DST_TILE(DR, BI)                                                                                                          \
-    hipLaunchKernelGGL((k_attn_bwd_dst_tile_bf16<H, D, HW, TILE_BF16_WPE_DST, TILE_BF16_PIPE, DR, BI>), dim3(group_grid(Pin) * (H / HW)),   \
+#define LAUNCH_DST_TILE(DR, BI, PD)                                                                                                      \
+    hipLaunchKernelGGL((k_attn_bwd_dst_tile_bf16<H, D, HW, TILE_BF16_WPE_DST, TILE_BF16_PIPE, DR, BI, PD>), dim3(group_grid(Pin) * (H / HW)), \
                        dim3(HW * WAVE), 0, s, *Pin, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (const bf16_t *)o,             \
-                       (const bf16_t *)d_o, lse, (bf16_t *)dq, (uint32_t *)ws, ws_rows, scale, scale * LOG2E, drop.thr, drop.seed,          \
-                       drop.inv, bias, ds_out, Narrow{})
-                switch ((drop.thr != 0 ? 1 : 0) + 2 * tile_bias_mode(Pin, bias)) {
-                case 0: LAUNCH_DST_TILE(false, 0); break;
-                case 1: LAUNCH_DST_TILE(true, 0); break;
-                case 2: LAUNCH_DST_TILE(false, 1); break;
-                case 3: LAUNCH_DST_TILE(true, 1); break;
-                case 4: LAUNCH_DST_TILE(false, 2); break;
-                default: LAUNCH_DST_TILE(true, 2); break;
+                       (const bf16_t *)d_o, lse, (bf16_t *)dq, (uint32_t *)ws, (float2 *)ws, ws_rows, scale, scale * LOG2E, drop.thr,       \
+                       drop.seed, drop.inv, bias, ds_out, Narrow{})
+                switch (again ? (drop.thr != 0 ? 7 : 6) : (drop.thr != 0 ? 1 : 0) + 2 * tile_bias_mode(Pin, bias)) {
+                case 6: LAUNCH_DST_TILE(false, 0, false); break;
+                case 7: LAUNCH_DST_TILE(true, 0, false); break;
+                case 1: LAUNCH_DST_TILE(true, 0, true); break;
+                case 2: LAUNCH_DST_TILE(false, 1, true); break;
+                case 3: LAUNCH_DST_TILE(true, 1, true); break;
+                case 4: LAUNCH_DST_TILE(false, 2, true); break;
+                default: LAUNCH_DST_TILE(true, 2, true); break;
                 }
 #undef LAUNCH_DST_TILE
             }
@@ -4258,8 +4371,16 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
             if (st != BPT_OK) return st;
             {
                 ProfScope prof(BPT_KERNEL_ATTN_BWD_SRC, s);
-                hipLaunchKernelGGL((k_attn_bwd_src_tile_bf16<H, D, HW, TILE_BF16_WPE_SRC, TILE_BF16_PIPE>), dim3(group_grid(Pout) * (H / HW)), dim3(HW * WAVE), 0, s,
-                                   *Pout, (const bf16_t *)q, (const bf16_t *)d_o, (const uint32_t *)ws, (bf16_t *)dk, (bf16_t *)dv, ws_dk, ws_dv, Narrow{});
+#define LAUNCH_SRC_AGAIN(DR)                                                                                                             \
+    hipLaunchKernelGGL((k_attn_bwd_src_tile_bf16_again<H, D, HW, TILE_BF16_WPE_AGAIN, DR>), dim3(group_grid(Pout) * (H / HW)), dim3(HW * WAVE), 0, s, \
+                       *Pout, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (const bf16_t *)d_o, (const float2 *)ws, (bf16_t *)dk, \
+                       (bf16_t *)dv, ws_dk, ws_dv, scale, scale * LOG2E, drop.thr, drop.seed, drop.inv)
+                if (again && drop.thr != 0) LAUNCH_SRC_AGAIN(true);
+                else if (again) LAUNCH_SRC_AGAIN(false);
+                else
+                    hipLaunchKernelGGL((k_attn_bwd_src_tile_bf16<H, D, HW, TILE_BF16_WPE_SRC, TILE_BF16_PIPE>), dim3(group_grid(Pout) * (H / HW)), dim3(HW * WAVE), 0, s,
+                                       *Pout, (const bf16_t *)q, (const bf16_t *)d_o, (const uint32_t *)ws, (bf16_t *)dk, (bf16_t *)dv, ws_dk, ws_dv, Narrow{});
+#undef LAUNCH_SRC_AGAIN
             }
             st = launch_status();
             if (st != BPT_OK || Pin->n_heavy + Pout->n_heavy == 0) return st;
@@ -4379,9 +4500,9 @@ int run_attn_bwd_narrow(const bpt_plan *Pin, const bpt_plan *Pout, const void *q
                                (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pds, ws_dq, scale, scale * LOG2E,       \
                                drop.thr, drop.seed, drop.inv, (const float *)nullptr, (float *)nullptr, nw);                                \
         else                                                                                                                             \
-            hipLaunchKernelGGL((k_attn_bwd_dst_tile_bf16<16, 64, NARROW_HW, TILE_BF16_WPE_DST, false, DR, 0, true>), grid, block, 0, s, *Pin,     \
-                               (const T *)q, (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pds, ws_dq, scale,        \
-                               scale * LOG2E, drop.thr, drop.seed, drop.inv, (const float *)nullptr, (float *)nullptr, nw);                 \
+            hipLaunchKernelGGL((k_attn_bwd_dst_tile_bf16<16, 64, NARROW_HW, TILE_BF16_WPE_DST, false, DR, 0, true, true>), grid, block, 0, s, *Pin, \
+                               (const T *)q, (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pds, (float2 *)nullptr, ws_dq, \
+                               scale, scale * LOG2E, drop.thr, drop.seed, drop.inv, (const float *)nullptr, (float *)nullptr, nw);          \
     } while (0)
         if (drop.thr != 0) LAUNCH_DST(true); else LAUNCH_DST(false);
 #undef LAUNCH_DST
