@@ -2221,8 +2221,24 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
 // Backward on tiles, source side (groups of the out-CSR plan: members = source rows, entries = destinations):
 // dk += ds^T q, dv += p^T dO with (p, ds) of every pair fetched from the scratch the destination side filled, at the
 // destination side's pair number that this plan's grp_pairs gives for (entry, member).
-template <typename T, int H, int D, int HW, bool PIPE, bool NARROW = false>
-__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE ? 3 : 4))) void k_attn_bwd_src_tile(
+//
+// A lane asks for the pairs of ONE entry (destination) with four neighbouring members, not of one member with four entries:
+// the destination side numbers the pairs of a tile by its entries, which are this side's members, so lanes c, the
+// destinations of a block, mostly read one run of 8 bytes each per member instead of 16 places 8 bytes x (members per entry)
+// apart, and the four positions are one load.  The block of (p, ds) is turned in LDS on the way into the products, which also
+// frees its registers: the next block's (p, ds) are asked for behind this block's rows and the positions of the one after that,
+// so neither is waited for, in 117 registers (two sets of (p, ds) in registers: 128 and 44 bytes spilled, 89 -> 100 us for the
+// 32-graph batch).  The first positions leave with the entry list.  8 heads, before -> now: L = 32768, k = 4 218 -> 210 us;
+// L = 4096, k = 32 54.1 -> 52.2; window 128 27.2 -> 25.6 (before: rows read a block ahead at three wavefronts per SIMD, which is
+// not needed any more); 6 heads of 50 columns 68.5 -> 65.6; 32-graph batch and L = 8192, k = 4 level.
+constexpr int TILE_WT_STRIDE = 18;                                // float2 per entry: 16 members + 2 (writes and reads spread over the banks)
+typedef int intx4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void tile_pair_positions(const bpt_plan &P, int entry, int g, int (&pos)[4]) {
+    const intx4u x = *reinterpret_cast<const intx4u *>(P.grp_pairs + (size_t)entry * TILE_R + 4 * g);
+    pos[0] = x[0]; pos[1] = x[1]; pos[2] = x[2]; pos[3] = x[3];
+}
+template <typename T, int H, int D, int HW, bool NARROW = false>
+__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_attn_bwd_src_tile(
     bpt_plan P, const T *__restrict__ q, const T *__restrict__ d_o, const float2 *__restrict__ pds, T *__restrict__ dk, T *__restrict__ dv,
     float *__restrict__ ws_dk, float *__restrict__ ws_dv, Narrow nw) {
     const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * sizeof(T) : (uint32_t)(H * D * sizeof(T));
@@ -2230,6 +2246,8 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
     if (!tile_begin<T, H, D, HW, NARROW>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     int2 *ent = ent_lds[t.wv];
+    __shared__ __attribute__((aligned(16))) float2 wt_lds[HW][TILE_R * TILE_WT_STRIDE];
+    float2 *const wt = wt_lds[t.wv];
     const int c = t.c, g = t.g;
     const char *qb = reinterpret_cast<const char *>(q), *db = reinterpret_cast<const char *>(d_o);
     const float2 *const pds_h = pds + (size_t)t.head * (size_t)P.n_edges;
@@ -2240,36 +2258,33 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
     // the steps past the end of the group's list (half of a group's last block on average) can be left out.
     struct Blk {
         float4 qr[4], dr[4];
-        float2 w[4];
         int has, nv;                                              // bit r of has: the pair (entry 4 r + g, member c) exists; nv: entries of the block that exist
     };
+    TileEntryRegs er;
+    if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
+    int pos[4];
+    float2 w[4];                                                  // (p, ds) of the pairs (entry c, member 4 g + r) of the next block
+    auto positions = [&](int first_entry) { tile_pair_positions(P, min(first_entry + c, t.p_end - 1), g, pos); };
+    if (t.p_end > t.p_begin) positions(t.p_begin);
+    issue_loads_first();
     for (int p0 = t.p_begin; p0 < t.p_end; p0 += TILE_CHUNK) {
         const int cnt = min(TILE_CHUNK, t.p_end - p0), nblk = (cnt + TILE_R - 1) / TILE_R;
-        tile_stage_entries(P, ent, p0, cnt, t.lane);
-        // Where this lane's four pairs of block b sit in the scratch (positions past the group's end are read at its last
-        // entry: their masks are empty).  They are fetched one block ahead, so that the (p, ds) loads of a block leave
-        // together with its row loads instead of one round trip later.
-        auto positions = [&](int b, int (&pos)[4]) {
+        if (p0 != t.p_begin) tile_ask_entries(P, p0, cnt, t.lane, er);
+        tile_put_entries(er, ent, cnt, t.lane);
+        if (p0 == t.p_begin) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) pos[r] = P.grp_pairs[(size_t)min(p0 + TILE_R * b + 4 * r + g, t.p_end - 1) * TILE_R + c];
+            for (int r = 0; r < 4; ++r) w[r] = pds_h[pos[r]];
+            positions(p0 + TILE_R);
+        }
+        auto put_pairs = [&]() {
+            floatx4v *const wp = reinterpret_cast<floatx4v *>(wt + c * TILE_WT_STRIDE + 4 * g);
+            wp[0] = floatx4v{w[0].x, w[0].y, w[1].x, w[1].y};
+            wp[1] = floatx4v{w[2].x, w[2].y, w[3].x, w[3].y};
+            wave_lds_fence();
         };
-        int pos_ahead[4], ahead_of = -1;                          // the positions of block ahead_of
-        auto issue = [&](Blk &B, int b) {
+        auto issue_rows = [&](Blk &B, int b) {
             B.nv = min(TILE_R, cnt - TILE_R * b);
             B.has = 0;
-            int pos[4];
-            if constexpr (PIPE) {                                 // (rows are read a block ahead there, and registers are short)
-                positions(b, pos);
-            } else {
-                if (b == ahead_of) {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) pos[r] = pos_ahead[r];
-                } else {
-                    positions(b, pos);
-                }
-                if (b + 1 < nblk) positions(b + 1, pos_ahead);
-                ahead_of = b + 1;
-            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int2 en = ent[TILE_R * b + 4 * r + g];
@@ -2277,21 +2292,35 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
                 const uint32_t off = (uint32_t)en.x * RB + t.offv;
                 B.qr[r] = tile_row4<NARROW>(qb + off);
                 B.dr[r] = tile_row4<NARROW>(db + off);
-                B.w[r] = pds_h[pos[r]];
             }
         };
         auto compute = [&](const Blk &B) {
             float pe[4], ds[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
+                const float2 w = wt[(4 * r + g) * TILE_WT_STRIDE + c];
                 const bool has = (B.has >> r) & 1;              // the scratch of pairs that do not exist is not initialised
-                pe[r] = has ? B.w[r].x : 0.f;
-                ds[r] = has ? B.w[r].y : 0.f;
+                pe[r] = has ? w.x : 0.f;
+                ds[r] = has ? w.y : 0.f;
             }
+            wave_lds_fence();                                     // (read before the next block's are written)
             tile_axpy_upto(ds, B.qr, ak, B.nv);
             tile_axpy_upto(pe, B.dr, av, B.nv);
         };
-        tile_walk<PIPE, Blk>(nblk, issue, compute);
+        for (int b = 0; b < nblk; ++b) {
+            Blk B;
+            issue_rows(B, b);
+            issue_loads_first();
+            put_pairs();
+            if (p0 + TILE_R * (b + 1) < t.p_end) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) w[r] = pds_h[pos[r]];
+                positions(p0 + TILE_R * (b + 2));
+            }
+            issue_loads_first();
+            compute(B);
+            issue_loads_first();
+        }
         wave_lds_fence();
     }
     tile_store_rows<H, D, false, NARROW>(t, ak, 1.f, dk, ws_dk, nw);
@@ -2634,6 +2663,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
     tile_store_rows<H, D, false, NARROW>(t, acc, 1.f, dq, ws_dq, nw);
 }
 
+constexpr int TILE_WT_STRIDE_BF16 = 20;
 template <int H, int D, int HW, int WPE, bool PIPE, bool NARROW = false>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))) void k_attn_bwd_src_tile_bf16(
     bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ d_o, const uint32_t *__restrict__ pds, bf16_t *__restrict__ dk,
@@ -2643,6 +2673,8 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     if (!tile_begin<bf16_t, H, D, HW, NARROW>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     int2 *ent = ent_lds[t.wv];
+    __shared__ __attribute__((aligned(16))) uint32_t wt_lds[HW][TILE_R * TILE_WT_STRIDE_BF16];    // (turned as in the float32 kernel)
+    uint32_t *const wt = wt_lds[t.wv];
     const int c = t.c, g = t.g;
     const uint32_t offc = t.offv;
     const char *qb = reinterpret_cast<const char *>(q), *db = reinterpret_cast<const char *>(d_o);
@@ -2652,7 +2684,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     for (int nb = 0; nb < 4; ++nb) { ak[nb] = floatx4v{0.f, 0.f, 0.f, 0.f}; av[nb] = floatx4v{0.f, 0.f, 0.f, 0.f}; }
     struct Blk {
         uint2 qr[4], dr[4];
-        uint32_t w[4];
+        uint32_t w[4];                                            // (p, ds) of the pairs (entry c, member 4 g + r)
         int has;                                                  // bit r: the pair (entry 4 g + r, member c) exists
     };
     for (int p0 = t.p_begin; p0 < t.p_end; p0 += TILE_CHUNK) {
@@ -2662,10 +2694,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
         // (p, ds) loads leave with the row loads; positions past the group's end are read at its last entry: their masks are
         // empty.  The four registers this takes are why the kernel is compiled for five wavefronts per SIMD, not six: with
         // six it spills and loses what the prefetch gains)
-        auto positions = [&](int b, int (&pos)[4]) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) pos[r] = P.grp_pairs[(size_t)min(p0 + TILE_R * b + 4 * g + r, t.p_end - 1) * TILE_R + c];
-        };
+        auto positions = [&](int b, int (&pos)[4]) { tile_pair_positions(P, min(p0 + TILE_R * b + c, t.p_end - 1), g, pos); };
         int pos_ahead[4], ahead_of = -1;
         auto issue = [&](Blk &B, int b) {
             const int4 e01 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g]);
@@ -2690,9 +2719,14 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             }
         };
         auto compute = [&](const Blk &B) {
+            *reinterpret_cast<uintx4v *>(wt + c * TILE_WT_STRIDE_BF16 + 4 * g) = uintx4v{B.w[0], B.w[1], B.w[2], B.w[3]};
+            wave_lds_fence();
             uint32_t w[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) w[r] = ((B.has >> r) & 1) ? B.w[r] : 0u;     // the scratch of pairs that do not exist is not initialised
+            for (int r = 0; r < 4; ++r) w[r] = wt[(4 * g + r) * TILE_WT_STRIDE_BF16 + c];
+            wave_lds_fence();                                     // (read before the next block's are written)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) w[r] = ((B.has >> r) & 1) ? w[r] : 0u;       // the scratch of pairs that do not exist is not initialised
             Bf4 pa, da;
             pa.u[0] = pack_lo16(w[0], w[1]); pa.u[1] = pack_lo16(w[2], w[3]);
             da.u[0] = pack_hi16(w[0], w[1]); da.u[1] = pack_hi16(w[2], w[3]);
@@ -4329,12 +4363,8 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
             if (st != BPT_OK) return st;
             {
                 ProfScope prof(BPT_KERNEL_ATTN_BWD_SRC, s);
-                if (tall_tiles(Pout, H))
-                    hipLaunchKernelGGL((k_attn_bwd_src_tile<T, H, D, HW, true>), dim3(group_grid(Pout) * (H / HW)), dim3(HW * WAVE), 0, s, *Pout,
-                                       (const T *)q, (const T *)d_o, (const float2 *)pds, (T *)dk, (T *)dv, ws_dk, ws_dv, Narrow{});
-                else
-                    hipLaunchKernelGGL((k_attn_bwd_src_tile<T, H, D, HW, false>), dim3(group_grid(Pout) * (H / HW)), dim3(HW * WAVE), 0, s, *Pout,
-                                       (const T *)q, (const T *)d_o, (const float2 *)pds, (T *)dk, (T *)dv, ws_dk, ws_dv, Narrow{});
+                hipLaunchKernelGGL((k_attn_bwd_src_tile<T, H, D, HW>), dim3(group_grid(Pout) * (H / HW)), dim3(HW * WAVE), 0, s, *Pout,
+                                   (const T *)q, (const T *)d_o, (const float2 *)pds, (T *)dk, (T *)dv, ws_dk, ws_dv, Narrow{});
             }
             st = launch_status();
             if (st != BPT_OK || Pin->n_heavy + Pout->n_heavy == 0) return st;
@@ -4512,7 +4542,7 @@ int run_attn_bwd_narrow(const bpt_plan *Pin, const bpt_plan *Pout, const void *q
     {
         ProfScope prof(BPT_KERNEL_ATTN_BWD_SRC, s);
         if constexpr (sizeof(T) == 4)
-            hipLaunchKernelGGL((k_attn_bwd_src_tile<T, 16, 64, NARROW_HW, false, true>), grid_src, block, 0, s, *Pout, (const T *)q, (const T *)d_o,
+            hipLaunchKernelGGL((k_attn_bwd_src_tile<T, 16, 64, NARROW_HW, true>), grid_src, block, 0, s, *Pout, (const T *)q, (const T *)d_o,
                                pds, (T *)dk, (T *)dv, ws_dk, ws_dv, nw);
         else
             hipLaunchKernelGGL((k_attn_bwd_src_tile_bf16<16, 64, NARROW_HW, TILE_BF16_WPE_SRC, false, true>), grid_src, block, 0, s, *Pout,
