@@ -1692,6 +1692,7 @@ constexpr int TILE_R = 16;
 constexpr int TILE_CHUNK = 128;                     // entries staged in LDS at a time = 8 blocks
 
 typedef float floatx4v __attribute__((ext_vector_type(4)));
+typedef uint32_t uintx2v __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ float lane_bcast(float x, int src_lane) {
     return __int_as_float(__builtin_amdgcn_ds_bpermute(src_lane << 2, __float_as_int(x)));
@@ -1824,7 +1825,12 @@ __device__ __forceinline__ void tile_axpy_upto(const float (&w)[4], const float4
 }
 
 // The members' result rows: whole rows go to `out` (scaled by inv[member] where given), segments of split rows to the
-// workspace in natural column order.
+// workspace in natural column order.  Whole rows are written past the L2 (non-temporal): this kernel does not read them again,
+// and written the ordinary way they push out the neighbours' rows that the other tiles of the XCD are about to read.  Sum of a
+// training step's kernels, new inputs every pass, before -> now: 32-graph batch float32 284 -> 274 us (forward 76 -> 70.5),
+// L = 8192 float32 161 -> 157, bfloat16 91 -> 85.5 (forward 21.8 -> 19.2), L = 32768, k = 4 649 -> 632, window 128 97 -> 94.5;
+// L = 512 level.  The same on the stores of (p, ds), which the source side reads soon, or on its loads of them: 47 -> 50.5 and
+// 47 -> 55 us for the source side of L = 8192; on the loads of the members' rows: destination side 58 -> 61.6.
 template <int H, int D, bool SCALE, bool NARROW, typename T>
 __device__ __forceinline__ void tile_store_rows(const TileCtx &t, const floatx4v (&acc)[4], float inv_c, T *__restrict__ out,
                                                 float *__restrict__ ws, const Narrow &nw) {
@@ -1841,12 +1847,12 @@ __device__ __forceinline__ void tile_store_rows(const TileCtx &t, const floatx4v
             T *const at = NARROW ? out + (size_t)row * (uint32_t)(nw.heads * nw.d) + t.head * nw.d + col : out + (size_t)row * (H * D) + t.head * D + col;
             if constexpr (sizeof(T) == 4) {
                 if constexpr (NARROW) *reinterpret_cast<floatx4u *>(at) = floatx4u{x.x, x.y, x.z, x.w};
-                else *reinterpret_cast<float4 *>(at) = x;
+                else __builtin_nontemporal_store(floatx4v{x.x, x.y, x.z, x.w}, reinterpret_cast<floatx4v *>(at));
             } else {
                 const uint2 y = make_uint2(((uint32_t)f32_to_bf16(x.x)) | ((uint32_t)f32_to_bf16(x.y) << 16),
                                ((uint32_t)f32_to_bf16(x.z)) | ((uint32_t)f32_to_bf16(x.w) << 16));
                 if constexpr (NARROW) *reinterpret_cast<uintx2u *>(at) = uintx2u{y.x, y.y};
-                else *reinterpret_cast<uint2 *>(at) = y;
+                else __builtin_nontemporal_store(uintx2v{y.x, y.y}, reinterpret_cast<uintx2v *>(at));
             }
         } else {
             float *const at = ws + (size_t)slot * (NARROW ? nw.h * D : H * D) + t.head * D + col;
@@ -2412,7 +2418,6 @@ template <bool NARROW> __device__ __forceinline__ uint2 tile_row4_bf16(const cha
 // into the operand of the products over the columns (lane (c, g): columns 16 g .. 16 g + 15 of the row of entry c).
 // Rows of TILE_KT_BYTES_BF16 = 128 + 16 bytes: the sixteen rows of a read fall on different banks.
 constexpr int TILE_KT_BYTES_BF16 = 144;
-typedef uint32_t uintx2v __attribute__((ext_vector_type(2)));
 typedef uint32_t uintx4v __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void tile_rows_to_operand_bf16(char *kt, const uint2 (&rows)[4], int c, int g, Bf8 (&out)[2]) {
 #pragma unroll
