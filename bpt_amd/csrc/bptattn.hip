@@ -3203,16 +3203,58 @@ __global__ __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(grp_wpe<T,
     }
 }
 
+// Sums, over the LPH neighbouring lanes of a head, of R values per lane, with the results spread over the lanes: a step over a
+// pair of lanes halves the values a lane carries as long as it carries more than one (the other half goes to its partner),
+// 12 + 6 + 3 instructions for 8 values over 8 lanes where 8 sums in every lane are 24.  Lanes are paired by the DPP patterns
+// there are: mirrored within 16 and within 8, then exchanged in steps of 2 and 1.  Steps run from the widest pattern down;
+// those that come before the last log2(R) add without halving.
+template <int CTRL, int N> __device__ __forceinline__ void sum_halve(float (&x)[N], bool upper) {
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+        const float keep = upper ? x[N / 2 + i] : x[i], give = upper ? x[i] : x[N / 2 + i];
+        x[i] = keep + dpp_mov<CTRL>(give);
+    }
+}
+template <int LPH, int R> __device__ __forceinline__ float sum_scatter(float (&x)[R], int lane) {
+    static_assert((LPH == 8 || LPH == 16) && (R == 4 || R == 8), "eight or sixteen lanes per head, four or eight values");
+    if constexpr (LPH == 16) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) x[i] += dpp_mov<0x140>(x[i]);
+    }
+    float y[4];
+    if constexpr (R == 8) {
+        sum_halve<0x141, 8>(x, (lane & 4) != 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[i] = x[i];
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[i] = x[i] + dpp_mov<0x141>(x[i]);
+    }
+    sum_halve<0x4E, 4>(y, (lane & 2) != 0);
+    float z[2] = {y[0], y[1]};
+    sum_halve<0xB1, 2>(z, (lane & 1) != 0);
+    return z[0];
+}
+// which of the R values sum_scatter leaves in this lane; -1 where a lane further left has it too
+template <int LPH, int R> __device__ __forceinline__ int sum_scatter_index(int lane) {
+    const int l = lane % LPH;
+    return l >= R ? -1 : l;
+}
+
 // y[eid, head] = <A[row, head, :], B[idx, head, :]> for every edge: the row-group form of k_sddmm_fast.  The
 // members' A rows stay in registers, B[idx] is loaded once per entry and every member that has the edge takes its
 // dot products with it; the edge id of (entry, member) comes from grp_eids.  TABLE: B is a (n, D) table whose rows
 // all heads share (the rel_pos score term q[row] . table[idx], written as float32).
+// All R products of an entry are formed (60 % of them belong to an edge at L = 8192, k = 4) and their sums over the head's lanes
+// are spread over those lanes, so an entry is one store from all lanes, with the edge ids loaded a batch ahead.  One full sum,
+// one edge id read across lanes and one 32-byte store per edge, with a branch around each, took 45 us at L = 8192, k = 4, 8
+// heads float32 (two calls a training step 90.9 us), this form 37.5 (75.0); 16 heads L = 2048 43 for two, L = 512 29.
 template <typename T, int H, int D, int R, int HS, bool TABLE = false, typename YT = T>
 __global__ __launch_bounds__(WAVE) void k_sddmm_grp(bpt_plan P, const T *__restrict__ A, const T *__restrict__ B, YT *__restrict__ y) {
     constexpr int HL = H / HS, CF = H * D;                  // heads of this wavefront's slice; elements of a full row
     using L = Lay<T, HL, D>;
     constexpr int EPL = L::EPL, GRP_BATCH = 2;
-    static_assert(H % HS == 0 && R % 4 == 0, "edge ids come four members per vector");
+    static_assert(H % HS == 0, "whole heads per slice");
     GroupHead<R> gh;
     if (!fetch_group<R, HS>(P, gh)) return;
     const int slice = group_slice<R, HS>(), coff = slice * HL * D;
@@ -3220,28 +3262,25 @@ __global__ __launch_bounds__(WAVE) void k_sddmm_grp(bpt_plan P, const T *__restr
     const uint32_t loff = (uint32_t)((coff + L::off(lane, 0)) * sizeof(T));
     const uint32_t toff = (uint32_t)((lane % L::LPH) * L::VE * sizeof(T));      // the lane's columns inside a table row
     const int4 *entries = reinterpret_cast<const int4 *>(P.grp_entries);
-    const int4 *eids4 = reinterpret_cast<const int4 *>(P.grp_eids);
+    const int member = sum_scatter_index<L::LPH, R>(lane);         // whose product this lane ends up with (-1: another lane has it too)
     float a[R][EPL];
 #pragma unroll
     for (int m = 0; m < R; ++m) load_row32<T, HL, D, CF>(A, (uint32_t)max(gh.rows[m], 0), loff, a[m]);
     struct Batch {
         RawRow<T, HL, D> br[GRP_BATCH];
-        int mk[GRP_BATCH], pz[GRP_BATCH];
+        int mk[GRP_BATCH], edge[GRP_BATCH];
     };
     for (int p0 = gh.begin; p0 < gh.end; p0 += GRP_CHUNK) {
         const int cnt = min(GRP_CHUNK, gh.end - p0);
         // lanes past the end repeat the last entry with an empty mask
         int4 ent = entries[p0 + min(lane, cnt - 1)];
         ent.y = lane < cnt ? ent.y : 0;
-        int4 xe[R / 4];                                     // edge ids of the lane's entry, four members per vector
-#pragma unroll
-        for (int c = 0; c < R / 4; ++c) xe[c] = eids4[(size_t)(p0 + min(lane, cnt - 1)) * (R / 4) + c];
         auto load_batch = [&](Batch &Bt, int b) {
 #pragma unroll
             for (int e = 0; e < GRP_BATCH; ++e) {
                 const uint32_t src = (uint32_t)__builtin_amdgcn_readlane(ent.x, b + e);
                 Bt.mk[e] = __builtin_amdgcn_readlane(ent.y, b + e);
-                Bt.pz[e] = b + e;
+                Bt.edge[e] = P.grp_eids[(size_t)(p0 + min(b + e, cnt - 1)) * R + max(member, 0)];
                 if constexpr (TABLE) load_row32_raw<T, HL, D, D>(B, src, toff, Bt.br[e]);
                 else load_row32_raw<T, HL, D, CF>(B, src, loff, Bt.br[e]);
             }
@@ -3251,16 +3290,11 @@ __global__ __launch_bounds__(WAVE) void k_sddmm_grp(bpt_plan P, const T *__restr
             for (int e = 0; e < GRP_BATCH; ++e) {
                 float bv[EPL];
                 unpack_row<T, HL, D>(Bt.br[e], bv);
+                float x[R];
 #pragma unroll
-                for (int m = 0; m < R; ++m) {
-                    if ((Bt.mk[e] >> m) & 1) {
-                        const float s = head_sum<L::LPH>(dot_n<EPL>(a[m], bv));
-                        const int4 &x = xe[m / 4];
-                        const int held = (m & 3) == 0 ? x.x : (m & 3) == 1 ? x.y : (m & 3) == 2 ? x.z : x.w;
-                        const uint32_t edge = (uint32_t)__builtin_amdgcn_readlane(held, Bt.pz[e]);
-                        if (lane % L::LPH == 0) Elem<YT>::st(y + (size_t)edge * H + head, s);
-                    }
-                }
+                for (int m = 0; m < R; ++m) x[m] = dot_n<EPL>(a[m], bv);
+                const float s = sum_scatter<L::LPH, R>(x, lane);
+                if (member >= 0 && ((Bt.mk[e] >> member) & 1)) Elem<YT>::st(y + (size_t)(uint32_t)Bt.edge[e] * H + head, s);
             }
         };
         // two-stage software pipeline as in the fused kernels (unconditional loads; look-ahead past the end re-reads
