@@ -241,10 +241,19 @@ struct Attention : torch::autograd::Function<Attention> {
     }
 };
 
+// Through the autograd function also where a tangent of forward-mode differentiation is carried: the function refuses it, the bare
+// forward would drop it.
+bool differentiated(const Tensor &q, const Tensor &k, const Tensor &v) {
+    if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) return true;
+    for (const Tensor *t : {&q, &k, &v})
+        if (t->_fw_grad(/*level=*/0).defined()) return true;
+    return false;
+}
+
 // op.BPTAttention with the host work in native code: the same call, the same result
 Tensor attention(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r, const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c,
                  const Tensor &eid_c, const Tensor &indices_c, const Tensor &q, const Tensor &k, const Tensor &v, double scale, double p, uint64_t seed) {
-    if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
+    if (differentiated(q, k, v))
         return Attention::apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale, p, (int64_t)seed);
     return std::get<0>(attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale, p, seed));
 }
@@ -348,7 +357,7 @@ struct NarrowAttention : torch::autograd::Function<NarrowAttention> {
 Tensor attention_narrow(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r, const Tensor &indices_r, const Tensor &col,
                         const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c, const Tensor &q, const Tensor &k, const Tensor &v,
                         int64_t h, double scale, double p, uint64_t seed) {
-    if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad()))
+    if (differentiated(q, k, v))
         return NarrowAttention::apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, h, scale, p, (int64_t)seed);
     return std::get<0>(narrow_forward(col, indptr_c, eid_c, indices_c, q.contiguous(), k.contiguous(), v.contiguous(), h, scale, p, (int64_t)seed));
 }

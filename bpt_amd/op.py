@@ -318,9 +318,12 @@ def bpt_attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices
         if dropout_p > 0 and seed is None:
             seed = int(torch.randint(0, 2 ** 62, (1,)).item())
         graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
+        grow = lambda x: torch.nn.functional.pad(x, (0, dp - d, 0, hp - h))
+        if rel_table is None and torch.jit.is_tracing():    # (a trace records the Python function, not what the native one launches)
+            o = BPTAttention.apply(*graph, grow(q), grow(k), grow(v), scale, float(dropout_p), int(seed or 0))
+            return o[:, :h, :d].contiguous()
         if rel_table is None:
             return _native.attention_narrow(*graph, q, k, v, hp, scale, float(dropout_p), int(seed or 0) & (2 ** 64 - 1))
-        grow = lambda x: torch.nn.functional.pad(x, (0, dp - d, 0, hp - h))
         o = BPTRelAttention.apply(*graph, grow(q), grow(k), grow(v), scale, float(dropout_p), int(seed or 0),
                                   torch.nn.functional.pad(rel_table, (0, dp - d)), etype)
         return o[:, :h, :d].contiguous()
@@ -330,6 +333,9 @@ def bpt_attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices
         if rel_table is not None:
             return BPTRelAttention.apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale,
                                          float(dropout_p), int(seed or 0), rel_table, etype)
+        if torch.jit.is_tracing():
+            return BPTAttention.apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale,
+                                      float(dropout_p), int(seed or 0))
         return _native.attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale, float(dropout_p),
                                  int(seed or 0) & (2 ** 64 - 1))
     e = masked_mm(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, k, q)

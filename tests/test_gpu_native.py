@@ -114,3 +114,20 @@ def test_threads_and_streams():
     for t in threads:
         t.join()
     assert not failures
+
+
+@pytest.mark.parametrize("h,d", [(8, 64), (6, 50)])
+def test_transforms_that_need_the_autograd_function(h, d):
+    """A tangent is refused, not dropped, also where no gradient is asked for; a trace runs the layer again on other inputs."""
+    import torch.autograd.forward_ad as forward_ad
+    from bpt_amd import op
+    c = Case("bpt512_k4")
+    q, k, v = (rand((c.n, h, d), torch.float32, s).to(DEV) for s in (1, 2, 3))
+    op.bpt_attention(*args_of(c), q, k, v)
+    with forward_ad.dual_level():
+        for no_grad in (False, True):
+            with torch.set_grad_enabled(not no_grad), pytest.raises(RuntimeError):
+                op.bpt_attention(*args_of(c), q, forward_ad.make_dual(k, q), v)
+    traced = torch.jit.trace(lambda x: op.bpt_attention(*args_of(c), x, k, v), (q,), check_trace=False)
+    other = v.clone()
+    torch.testing.assert_close(traced(other), op.bpt_attention(*args_of(c), other, k, v), rtol=1e-5, atol=1e-6)
