@@ -303,6 +303,12 @@ std::optional<Three> narrow_backward_known(const Tensor &row, const Tensor &indp
     return Three{dq, dk, dv};
 }
 
+// a contiguous tensor that starts on 4 bytes, as the kernels' loads need (a bfloat16 view may start on 2)
+Tensor rows(const Tensor &x) {
+    Tensor y = x.contiguous();
+    return y.is_cuda() && (reinterpret_cast<uintptr_t>(y.data_ptr()) & 3) ? y.clone() : y;
+}
+
 // The forward is a call of graphop.attention_forward, as that of the padded copies was: q, k, v stand for the padded shape there.
 std::tuple<Tensor, Tensor> narrow_forward(const Tensor &col, const Tensor &indptr, const Tensor &eid, const Tensor &indices, const Tensor &q,
                                           const Tensor &k, const Tensor &v, int64_t h, double scale, double p, int64_t seed) {
@@ -325,7 +331,7 @@ struct NarrowAttention : torch::autograd::Function<NarrowAttention> {
     static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r,
                           const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c,
                           const Tensor &q, const Tensor &k, const Tensor &v, int64_t h, double scale, double p, int64_t seed) {
-        const Tensor qc = q.contiguous(), kc = k.contiguous(), vc = v.contiguous();
+        const Tensor qc = rows(q), kc = rows(k), vc = rows(v);
         if (!narrow_known(col, indptr_c, eid_c, indices_c, qc, kc, h))
             python("prepare_training")(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, qc, kc, p, h);
         const auto [o, lse] = narrow_forward(col, indptr_c, eid_c, indices_c, qc, kc, vc, h, scale, p, seed);
@@ -341,7 +347,7 @@ struct NarrowAttention : torch::autograd::Function<NarrowAttention> {
         const double scale = ctx->saved_data["scale"].toDouble(), p = ctx->saved_data["p"].toDouble();
         const uint64_t seed = (uint64_t)ctx->saved_data["seed"].toInt();
         const int h = (int)ctx->saved_data["h"].toInt();
-        const Tensor d_o = grads[0].contiguous();
+        const Tensor d_o = rows(grads[0]);
         auto r = narrow_backward_known(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], t[10], t[11], t[12], d_o, h, scale, p, seed);
         if (!r)
             r = with_python([&] {
@@ -359,7 +365,7 @@ Tensor attention_narrow(const Tensor &row, const Tensor &indptr_r, const Tensor 
                         int64_t h, double scale, double p, uint64_t seed) {
     if (differentiated(q, k, v))
         return NarrowAttention::apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, h, scale, p, (int64_t)seed);
-    return std::get<0>(narrow_forward(col, indptr_c, eid_c, indices_c, q.contiguous(), k.contiguous(), v.contiguous(), h, scale, p, (int64_t)seed));
+    return std::get<0>(narrow_forward(col, indptr_c, eid_c, indices_c, rows(q), rows(k), rows(v), h, scale, p, (int64_t)seed));
 }
 
 // ---- tile plans ---------------------------------------------------------------------------------------------------------------

@@ -66,3 +66,24 @@ def test_dropout_of_narrow_heads_is_that_of_the_padded_layer(dtype, h, d):
     # (the same kernels on the same numbers and zeros: sums over the columns differ in nothing but the zeros' places)
     for got, want, name in zip(both[0], both[1], ("o", "dq", "dk", "dv")):
         close(got, f64(want), TOL[dtype] if name == "o" else GTOL[dtype], name)
+
+
+@pytest.mark.parametrize("p", [0.0, 0.1])
+@pytest.mark.parametrize("d", [50, 64])
+def test_bfloat16_rows_that_start_on_two_bytes(d, p):
+    """Views one element into their memory, the incoming gradient among them: the bits of the same values from their own memory."""
+    from bpt_amd import op
+    c = case("bpt512_k4")                                     # (with dropout: the kernels that read the rows as they are, whatever the size)
+    x = [rand((c.n, 6, d), torch.bfloat16, s, 1.0 / 8).to(DEV) for s in (91, 92, 93, 94)]
+
+    def shifted(t):
+        view = torch.zeros(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+        return view.copy_(t)
+
+    def step(q, k, v, do):
+        q, k, v = (t.detach().requires_grad_(True) for t in (q, k, v))
+        o = op.bpt_attention(*c.out, *c.inn, q, k, v, dropout_p=p, seed=3)
+        return (o.detach(), *torch.autograd.grad(o, (q, k, v), do))
+
+    for want, got in zip(step(*x), step(*map(shifted, x))):
+        assert torch.equal(want, got)
