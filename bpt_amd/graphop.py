@@ -515,16 +515,20 @@ def _pad_heads(x, h):
     return torch.nn.functional.pad(x, (0, 64 - x.size(2), 0, h - x.size(1)))
 
 
-def _narrow_seg(q, h, n_edges, cfg):
+def _narrow_seg(units, q, k, h, n_edges, dropout_p, cfg):
     """The work-item length of the tile plans of a layer whose rows the kernels for narrow heads take as they are, or None where
-    they do not: heads of 4 to 64 columns, starting on 4 bytes, wherever tiles are the library's choice."""
-    if not (cfg.use_groups and _tiles(q, h, 64, None, 0.0, None, cfg) and 4 <= q.size(2) <= 64 and (q.dtype == torch.float32 or q.size(2) % 2 == 0)
-            and not _FORCE_GENERIC and TILE_BACKWARD is not False):
+    they do not: heads of 4 to 64 columns, starting on 4 bytes, wherever the padded layer takes tiles without a plan to look
+    at.  Smaller graphs stay on padded copies and the kernels that walk single rows, though tiles would be faster there too
+    (6 heads of 50, 603 nodes, forward and backward: 105 us against 240): a row kernel keeps its probabilities in float32 where a
+    bfloat16 tile rounds them, and an infinite row reaches its neighbours only and not the other rows of a tile."""
+    if not (4 <= q.size(2) <= 64 and (q.dtype == torch.float32 or q.size(2) % 2 == 0) and not _FORCE_GENERIC and TILE_BACKWARD is not False):
         return None
-    if TILE_SEG_LEN is not None:
-        return TILE_SEG_LEN
-    deg = n_edges / max(q.size(0), 1)
-    return 64 if deg < 32 else (128 if deg < 80 else 256)
+    return _tile_seg_without_plan(units, n_edges, q, k, h, 64, dropout_p, None, cfg)
+
+
+def attention_reads_narrow(col, eid_c, q, k, h, dropout_p):
+    """True if the layer of q's heads of fewer than 64 columns, h of them when padded, runs on the kernels that read its rows as they are."""
+    return _narrow_seg(col, q, k, h, eid_c.size(0), dropout_p, _SETTINGS) is not None
 
 
 def _attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale, dropout_p, seed):
@@ -541,8 +545,8 @@ def _attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale
     _expect_index(eid_c, indices_c)
     _expect_shape(k, (k.size(0),) + tuple(q.shape[1:]), "k")
     _expect_shape(v, k.shape, "v")
-    seg, plan = _narrow_seg(q, h, eid_c.size(0), cfg), None
-    if seg is not None and max(q.size(0), k.size(0)) * h * 64 * q.element_size() < 2 ** 32:
+    seg, plan = _narrow_seg(col, q, k, h, eid_c.size(0), dropout_p, cfg), None
+    if seg is not None:
         plan = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, None))
     if plan is None or not plan.covers_all_edges:
         o, lse = attention_forward(col, indptr_c, eid_c, indices_c, _pad_heads(q, h), _pad_heads(k, h), _pad_heads(v, h), scale, dropout_p, seed)
@@ -578,8 +582,8 @@ def attention_backward_narrow(row, indptr_r, eid_r, indices_r, col, indptr_c, ei
     if lse.dtype != torch.float32 or lse.device != q.device:
         raise ValueError("lse must be the float32 tensor that attention_forward returned")
     _expect_shape(lse, (q.size(0), h), "lse")
-    seg, pi = _narrow_seg(q, h, eid_c.size(0), cfg), None
-    if seg is not None and max(q.size(0), k.size(0)) * h * 64 * q.element_size() < 2 ** 32:
+    seg, pi = _narrow_seg(col, q, k, h, eid_c.size(0), dropout_p, cfg), None
+    if seg is not None:
         order_src = _plan.tile_order_src(k.size(0), eid_r.size(0))
         pi = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, None))
         po = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, order_src))
@@ -751,7 +755,7 @@ def prepare_training(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indi
     if max(q.size(0), k.size(0)) * h * d * q.element_size() >= 2 ** 32 or not _tiles_backward(None, q.dtype, None):
         return
     if narrow_h is not None:
-        seg = _narrow_seg(q, h, eid_c.size(0), cfg)
+        seg = _narrow_seg(col, q, k, h, eid_c.size(0), dropout_p, cfg)
     else:
         seg = _tile_seg_without_plan(col, eid_c.size(0), q, k, h, d, dropout_p, None, cfg) if attention_supported(q) else None
     if seg is not None:

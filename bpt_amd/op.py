@@ -311,19 +311,20 @@ def bpt_attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices
         padded = _g.attention_padded_shape(q)
     if fused and padded is not None:
         # heads of fewer than 64 columns (6 x 50, 8 x 40 in the reference's configs), computed as (h', 64) with the scale of the real d:
-        # by kernels that read the rows as they are, with the rel_pos term on zero-padded copies (the pads and the slice are
-        # ordinary differentiable torch ops)
+        # by kernels that read the rows as they are (attention_reads_narrow), else and with the rel_pos term on zero-padded copies (the
+        # pads and the slice are ordinary differentiable torch ops)
         h, d = q.size(1), q.size(2)
         hp, dp = padded
         if dropout_p > 0 and seed is None:
             seed = int(torch.randint(0, 2 ** 62, (1,)).item())
         graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
         grow = lambda x: torch.nn.functional.pad(x, (0, dp - d, 0, hp - h))
-        if rel_table is None and torch.jit.is_tracing():    # (a trace records the Python function, not what the native one launches)
+        if rel_table is None:
+            # (a trace records the Python function, not what the native one launches)
+            if not torch.jit.is_tracing() and _g.attention_reads_narrow(col, eid_c, q, k, hp, dropout_p):
+                return _native.attention_narrow(*graph, q, k, v, hp, scale, float(dropout_p), int(seed or 0) & (2 ** 64 - 1))
             o = BPTAttention.apply(*graph, grow(q), grow(k), grow(v), scale, float(dropout_p), int(seed or 0))
             return o[:, :h, :d].contiguous()
-        if rel_table is None:
-            return _native.attention_narrow(*graph, q, k, v, hp, scale, float(dropout_p), int(seed or 0) & (2 ** 64 - 1))
         o = BPTRelAttention.apply(*graph, grow(q), grow(k), grow(v), scale, float(dropout_p), int(seed or 0),
                                   torch.nn.functional.pad(rel_table, (0, dp - d)), etype)
         return o[:, :h, :d].contiguous()

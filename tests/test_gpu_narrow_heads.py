@@ -33,8 +33,9 @@ def among_nans(x):
                                        (torch.bfloat16, 1, 4), (torch.bfloat16, 5, 6), (torch.bfloat16, 6, 50), (torch.bfloat16, 9, 62),
                                        (torch.bfloat16, 3, 64), (torch.bfloat16, 6, 51)],
                          ids=lambda x: str(x).replace("torch.", ""))
-def test_narrow_heads_against_the_oracle(gname, dtype, h, d):
-    from bpt_amd import op
+def test_narrow_heads_against_the_oracle(gname, dtype, h, d, monkeypatch):
+    from bpt_amd import graphop, op
+    monkeypatch.setattr(graphop, "_MIN_GROUP_ITEMS", 0)       # (tiles whatever the graph's size)
     c = case(gname)
     q, k, v, do = (among_nans(rand((c.n, h, d), dtype, s, 1.0 / 8).to(DEV)) for s in (71, 72, 73, 74))
     for t in (q, k, v):
@@ -87,3 +88,26 @@ def test_bfloat16_rows_that_start_on_two_bytes(d, p):
 
     for want, got in zip(step(*x), step(*map(shifted, x))):
         assert torch.equal(want, got)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_small_graphs_keep_the_row_kernels(dtype):
+    """A layer too small for tiles takes its padded form's kernels: the bits of the padded layer, and a row that is not finite
+    reaches its neighbours and no one else."""
+    from bpt_amd import graphbuilder as gb, op
+    g = gb.BinaryPartition(300, True, 4, 10)
+    src, dst, _, _, n = gb.merge_graphs_device([g, g], torch.device(DEV))
+    out_csr, in_csr, row, ir, col, ic = gb.get_csrs_device(src, dst, n)
+    graph = (row, ir, out_csr[2], out_csr[1], col, ic, in_csr[2], in_csr[1])
+    assert col.numel() < 1536
+    q, k, v, do = (rand((n, 6, 50), dtype, s, 1.0 / 8).to(DEV) for s in (61, 62, 63, 64))
+    q[5] = float("inf")
+    grow = lambda x: torch.nn.functional.pad(x, (0, 14, 0, 2))
+    both = []
+    for rows in (lambda x: x, grow):
+        x = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        o = op.bpt_attention(*graph, *map(rows, x), scale=50 ** -0.5)[:, :6, :50]
+        both.append((o.detach(), *torch.autograd.grad(o, x, do)))
+    for got, want in zip(*both):
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+        assert not got[n // 2:].isnan().any()                  # the second graph
