@@ -1099,7 +1099,7 @@ __global__ __launch_bounds__(TPB) void k_group_form(PlanSides b, int32_t R) {
             k = ((K)(uint32_t)idx32[at.begin[m] + place] << (place_bits + 4)) | (K)((m << place_bits) | place);
         }
         key[t] = k;
-        if (2 * t < n + 1) emask2[t] = 0;
+        if (2 * t < n) emask2[t] = 0;                               // (a full group: CAP / 2 words, all there are)
     }
     __syncthreads();
     lds_sort<TPB, K>(key, P);
