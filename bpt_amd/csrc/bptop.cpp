@@ -6,8 +6,9 @@
 //
 // Nothing is decided here.  bpt_amd/graphop.py chooses kernels and builds plans; each time it has done so it leaves what it
 // chose in the table below (`remember`), under the index tensors' addresses, sizes and versions, the shape and the type.  The
-// plan cache (bpt_amd/plan.py) keeps those index tensors and the plans alive, and drops an entry here when it drops a plan
-// (`forget`); changing a switch clears the table.  A call that is not in the table, or has an argument that a check refuses, goes to
+// plan cache (bpt_amd/plan.py) lets an entry in only while it holds the entry's plans, and drops the entry when it drops one of
+// them (`forget`); an entry holds its index tensors too, so that their addresses mean nothing else as long as it stands.
+// Changing a switch clears the table.  A call that is not in the table, or has an argument that a check refuses, goes to
 // the Python function, which raises, or builds, chooses and remembers.  Every call is checked anew.
 #include <torch/extension.h>
 
@@ -61,6 +62,7 @@ struct KeyHash {
 struct Entry {
     bpt_plan a{}, b{};
     std::vector<PyObject *> plans;    // owned: what the structs point into lives as long as the entry
+    std::vector<Tensor> index;        // whose addresses the key holds: they are not given to other tensors meanwhile
     std::atomic<bool> used{false};
     ~Entry() {
         if (plans.empty() || !Py_IsInitialized()) return;
@@ -497,6 +499,7 @@ bool remember(int kind, const std::vector<Tensor> &index, const std::vector<int6
     std::memcpy(&e->a, reinterpret_cast<const void *>(a), sizeof(bpt_plan));
     if (b) std::memcpy(&e->b, reinterpret_cast<const void *>(b), sizeof(bpt_plan));
     for (auto p : plans) e->plans.push_back(p.inc_ref().ptr());
+    e->index = index;
     e->used.store(true);
     std::vector<EntryPtr> dropped;                           // (destroyed behind the lock)
     {

@@ -560,8 +560,8 @@ def _attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale
         check_attn(_LIB.bpt_attention_forward_narrow(ctypes.byref(struct), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(ws), nws, scale,
                                                      float(dropout_p), seed, heads, d, h, dt, _stream()), "attention_forward_narrow")
     if cfg is _SETTINGS:
-        _native.remember(_native.ATTN_FWD_NARROW, [col, indptr_c, eid_c, indices_c], [q.size(0), k.size(0), h, d, dt, heads],
-                         ctypes.addressof(struct), 0, (plan,))
+        plan_cache.remember((plan,), _native.ATTN_FWD_NARROW, [col, indptr_c, eid_c, indices_c], [q.size(0), k.size(0), h, d, dt, heads],
+                            ctypes.addressof(struct), 0)
     return o, lse
 
 
@@ -602,8 +602,8 @@ def attention_backward_narrow(row, indptr_r, eid_r, indices_r, col, indptr_c, ei
                                                       _ptr(dv), _ptr(ws), nws, scale, float(dropout_p), int(seed) & (2 ** 64 - 1), heads, d, h, dt,
                                                       _stream()), "attention_backward_narrow")
     if cfg is _SETTINGS:
-        _native.remember(_native.ATTN_BWD_NARROW, [row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c],
-                         [q.size(0), k.size(0), h, d, dt, heads], ctypes.addressof(in_struct), ctypes.addressof(out_struct), (pi, po))
+        plan_cache.remember((pi, po), _native.ATTN_BWD_NARROW, [row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c],
+                            [q.size(0), k.size(0), h, d, dt, heads], ctypes.addressof(in_struct), ctypes.addressof(out_struct))
     return dq, dk, dv
 
 
@@ -659,8 +659,8 @@ def attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale=None, drop
                                               scale, float(dropout_p), int(seed) & (2 ** 64 - 1), h, d, dt, _stream()),
                    "attention_forward")
     if bias is None and cfg is _SETTINGS:
-        _native.remember(_native.ATTN_FWD, [col, indptr_c, eid_c, indices_c], [q.size(0), k.size(0), h, d, dt, int(dropout_p > 0.0)],
-                         ctypes.addressof(struct), 0, (plan,))
+        plan_cache.remember((plan,), _native.ATTN_FWD, [col, indptr_c, eid_c, indices_c], [q.size(0), k.size(0), h, d, dt, int(dropout_p > 0.0)],
+                            ctypes.addressof(struct), 0)
     return o, lse
 
 
@@ -737,9 +737,8 @@ def attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, in
     if bias is not None:
         return dq, dk, dv, ds if bias_by_pair else ds[:-1]
     if cfg is _SETTINGS:
-        _native.remember(_native.ATTN_BWD, [row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c],
-                         [q.size(0), k.size(0), h, d, dt, int(dropout_p > 0.0)], ctypes.addressof(in_struct), ctypes.addressof(out_struct),
-                         (plan_in, plan_out))
+        plan_cache.remember((plan_in, plan_out), _native.ATTN_BWD, [row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c],
+                            [q.size(0), k.size(0), h, d, dt, int(dropout_p > 0.0)], ctypes.addressof(in_struct), ctypes.addressof(out_struct))
     return dq, dk, dv
 
 

@@ -734,10 +734,16 @@ class PlanCache:
     _total, _counted = 0, 0
 
     def _insert(self, key, plan, tensors):
-        # called with the lock held
-        old = self._d.pop(key, None)
+        # called with the lock held, for a key that is not here
         self._d[key] = (plan, tensors)
-        self._total += plan.device_bytes() - (old[0].device_bytes() if old is not None else 0)
+        self._total += plan.device_bytes()
+
+    def remember(self, plans, *choice):
+        """native.remember(*choice, plans): what was chosen with these plans, as long as all of them are here.  Another thread may
+        have dropped one since the caller got it; nobody would tell the native host path when its index tensors go."""
+        with self._lock:
+            if all(any(p is plan for p, _ in reversed(self._d.values())) for plan in plans):
+                self.native.remember(*choice, plans)
 
     def _evict(self):
         # called with the lock held; the newest entry always stays
@@ -790,6 +796,9 @@ class PlanCache:
             ni = n_index_nodes if n_index_nodes is not None else nr
             plan = Plan(row_h, indptr, eid, indices, nr, ni, eid.device, seg_len)
         with self._lock:
+            hit = self._d.get(key)
+            if hit is not None:                     # (another thread built it meanwhile, and streams may be using it: that one stays)
+                return hit[0]
             self._insert(key, plan, tensors)        # tensors kept alive with the entry
             self._evict()
         return plan
@@ -808,6 +817,8 @@ class PlanCache:
             return
         self.misses += len(plans)
         with self._lock:
+            if any(key in self._d for key in keys):
+                return                              # (as in get: another thread's stay)
             for key, plan, side in zip(keys, plans, sides):
                 self._insert(key, plan, side[:4])
             self._evict()

@@ -116,6 +116,63 @@ def test_threads_and_streams():
     assert not failures
 
 
+@pytest.mark.parametrize("tiles", [False, True], ids=["by-size", "tiles"])
+def test_threads_that_build_the_same_graph_at_once(tiles, monkeypatch):
+    """From an empty cache, every thread on a stream of its own; then another graph of the same sizes, in memory that the first one's
+    index tensors may have left."""
+    from bpt_amd import graphbuilder as gb, graphop, op, plan
+    if tiles:
+        monkeypatch.setattr(graphop, "_MIN_GROUP_ITEMS", 0)
+    c = Case("bpt512_k4")
+    x = node_tensors(c.n)
+    want = [step(op, args_of(c), *x)]
+    out_csr, in_csr, ROW, IR, COL, IC = gb.get_csrs((np.asarray(c.src) + 1) % c.n, np.asarray(c.dst), c.n)
+    other = tuple(t.to(DEV) for t in (ROW, IR, out_csr[2], out_csr[1], COL, IC, in_csr[2], in_csr[1]))
+    want.append(step(op, other, *x))
+    torch.cuda.synchronize()
+    failures = []
+
+    def work(args, expected, start):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            start.wait()
+            for _ in range(2):
+                got = step(op, args, *x)
+                stream.synchronize()
+                if not same(expected, got):
+                    failures.append(1)
+
+    for i in range(12):
+        plan.plan_cache.clear()
+        args = [t.clone() for t in (args_of(c), other)[i % 2]]
+        torch.cuda.synchronize()
+        start = threading.Barrier(4)
+        threads = [threading.Thread(target=work, args=(args, want[i % 2], start)) for _ in range(4)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        torch.cuda.synchronize()
+        del args
+    assert not failures
+
+
+def test_an_entry_holds_its_index_tensors():
+    """Their addresses are the key: nothing else may come to lie there while the entry stands."""
+    import ctypes
+    from bpt_amd import graphop, plan
+    native = plan.PlanCache.native
+    native.clear()
+    struct, before = graphop.PlanStruct(), torch.cuda.memory_allocated()
+    index = [torch.zeros(1 << 20, dtype=torch.int64, device=DEV) for _ in range(4)]
+    held = torch.cuda.memory_allocated()
+    assert native.remember(native.ATTN_FWD, index, [1, 1, 8, 64, 0, 0], ctypes.addressof(struct), 0, (object(),))
+    del index
+    assert torch.cuda.memory_allocated() == held
+    native.clear()
+    assert torch.cuda.memory_allocated() == before
+
+
 @pytest.mark.parametrize("h,d", [(8, 64), (6, 50)])
 def test_transforms_that_need_the_autograd_function(h, d):
     """A tangent is refused, not dropped, also where no gradient is asked for; a trace runs the layer again on other inputs."""
