@@ -73,6 +73,7 @@ struct Entry {
 using EntryPtr = std::shared_ptr<Entry>;
 
 std::mutex g_mutex;                   // never held while the interpreter lock is taken
+int64_t g_generation = 0;             // (under g_mutex) how often the table was cleared
 std::unordered_map<Key, EntryPtr, KeyHash> &table() {
     static auto *t = new std::unordered_map<Key, EntryPtr, KeyHash>();       // (lives on: entries may outlast static destruction)
     return *t;
@@ -488,8 +489,9 @@ py::object build_tile_plans(const std::vector<std::tuple<Tensor, Tensor, Tensor,
 
 // ---- the table ---------------------------------------------------------------------------------------------------------------
 // `kind`'s choice for these index tensors and numbers: the bpt_plan structs at the addresses a and b (0: none), which point into
-// what `plans` holds.  True if it was taken.
-bool remember(int kind, const std::vector<Tensor> &index, const std::vector<int64_t> &extra, int64_t a, int64_t b, py::tuple plans) {
+// what `plans` holds.  generation: what generation() said before the choice was begun; a table that was cleared since does not take
+// it, since a switch may have changed under it.  True if it was taken.
+bool remember(int64_t generation, int kind, const std::vector<Tensor> &index, const std::vector<int64_t> &extra, int64_t a, int64_t b, py::tuple plans) {
     if (index.empty() || index.size() > MAX_TENSORS || extra.size() != MAX_EXTRA || !index[0].defined() || !index[0].is_cuda() || !a) return false;
     std::vector<const Tensor *> ptrs;
     for (const Tensor &t : index) ptrs.push_back(&t);
@@ -504,6 +506,7 @@ bool remember(int kind, const std::vector<Tensor> &index, const std::vector<int6
     std::vector<EntryPtr> dropped;                           // (destroyed behind the lock)
     {
         std::lock_guard<std::mutex> lock(g_mutex);
+        if (generation != g_generation) return false;
         if (table().size() >= MAX_ENTRIES) {
             for (auto &kv : table()) dropped.push_back(std::move(kv.second));
             table().clear();
@@ -534,8 +537,14 @@ void forget(py::object plan) {
 void clear() {
     std::vector<EntryPtr> dropped;
     std::lock_guard<std::mutex> lock(g_mutex);
+    ++g_generation;
     for (auto &kv : table()) dropped.push_back(std::move(kv.second));
     table().clear();
+}
+
+int64_t generation() {
+    std::lock_guard<std::mutex> lock(g_mutex);
+    return g_generation;
 }
 
 // the plan objects whose entries served a call since the last time this was asked
@@ -569,6 +578,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("remember", &remember);
     m.def("forget", &forget);
     m.def("clear", &clear);
+    m.def("generation", &generation);
     m.def("take_used", &take_used);
     m.def("plan_bytes", [] { return (int64_t)sizeof(bpt_plan); });
 }

@@ -534,11 +534,11 @@ def attention_reads_narrow(col, eid_c, q, k, h, dropout_p):
 def _attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale, dropout_p, seed):
     """(o, lse) for heads of fewer than 64 columns: o (n, heads, d), lse (n, h), h the heads the layer is padded to.  On the tile
     kernels that read the rows as they are, or else on padded copies."""
-    cfg = _SETTINGS
     seed = int(seed) & (2 ** 64 - 1)
     known = _native.attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale, dropout_p, seed)
     if known is not None:
         return known
+    generation, cfg = _native.generation(), _SETTINGS
     _check_all(col=col, indptr_c=indptr_c, eid_c=eid_c, indices_c=indices_c, q=q, k=k, v=v)
     _same_dtype(q, k, v)
     heads, d = _hd(q)
@@ -559,15 +559,14 @@ def _attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale
     with _on_device_of(q):
         check_attn(_LIB.bpt_attention_forward_narrow(ctypes.byref(struct), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(ws), nws, scale,
                                                      float(dropout_p), seed, heads, d, h, dt, _stream()), "attention_forward_narrow")
-    if cfg is _SETTINGS:
-        plan_cache.remember((plan,), _native.ATTN_FWD_NARROW, [col, indptr_c, eid_c, indices_c], [q.size(0), k.size(0), h, d, dt, heads],
-                            ctypes.addressof(struct), 0)
+    plan_cache.remember((plan,), generation, _native.ATTN_FWD_NARROW, [col, indptr_c, eid_c, indices_c],
+                        [q.size(0), k.size(0), h, d, dt, heads], ctypes.addressof(struct), 0)
     return o, lse
 
 
 def attention_backward_narrow(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, o, lse, do, h, scale, dropout_p, seed):
     """(dq, dk, dv) of attention_forward(..., narrow=(q, k, v)): the shapes of q, k, v; lse (n, h) as that returned it."""
-    cfg = _SETTINGS
+    generation, cfg = _native.generation(), _SETTINGS
     _check_all(row=row, indptr_r=indptr_r, eid_r=eid_r, indices_r=indices_r, col=col, indptr_c=indptr_c,
                eid_c=eid_c, indices_c=indices_c, q=q, k=k, v=v, o=o, lse=lse, do=do)
     _same_dtype(q, k, v, o, do)
@@ -601,9 +600,8 @@ def attention_backward_narrow(row, indptr_r, eid_r, indices_r, col, indptr_c, ei
         check_attn(_LIB.bpt_attention_backward_narrow(in_ref, out_ref, _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(dq), _ptr(dk),
                                                       _ptr(dv), _ptr(ws), nws, scale, float(dropout_p), int(seed) & (2 ** 64 - 1), heads, d, h, dt,
                                                       _stream()), "attention_backward_narrow")
-    if cfg is _SETTINGS:
-        plan_cache.remember((pi, po), _native.ATTN_BWD_NARROW, [row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c],
-                            [q.size(0), k.size(0), h, d, dt, heads], ctypes.addressof(in_struct), ctypes.addressof(out_struct))
+    plan_cache.remember((pi, po), generation, _native.ATTN_BWD_NARROW, [row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c],
+                        [q.size(0), k.size(0), h, d, dt, heads], ctypes.addressof(in_struct), ctypes.addressof(out_struct))
     return dq, dk, dv
 
 
@@ -618,12 +616,12 @@ def attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale=None, drop
     (attention_padded_shape; tensors of it on the meta device) and o has narrow's shape, lse the padded heads."""
     if narrow is not None:
         return _attention_forward_narrow(col, indptr_c, eid_c, indices_c, *narrow, q.size(1), float(scale), float(dropout_p), seed)
-    cfg = _SETTINGS
     if bias is None:
         known = _native.attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, 1.0 / math.sqrt(q.size(-1)) if scale is None else float(scale),
                                           float(dropout_p), int(seed) & (2 ** 64 - 1))
         if known is not None:
             return known
+    generation, cfg = _native.generation(), _SETTINGS
     _check_all(col=col, indptr_c=indptr_c, eid_c=eid_c, indices_c=indices_c, q=q, k=k, v=v)
     _check_bias(bias, eid_c.size(0), _hd(q)[0], q.device, cfg, bias_by_pair)
     _same_dtype(q, k, v)
@@ -658,9 +656,9 @@ def attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale=None, drop
         check_attn(_LIB.bpt_attention_forward(ref, _ptr(q), _ptr(k), _ptr(v), _ptr(bias), _ptr(o), _ptr(lse), _ptr(ws), nws,
                                               scale, float(dropout_p), int(seed) & (2 ** 64 - 1), h, d, dt, _stream()),
                    "attention_forward")
-    if bias is None and cfg is _SETTINGS:
-        plan_cache.remember((plan,), _native.ATTN_FWD, [col, indptr_c, eid_c, indices_c], [q.size(0), k.size(0), h, d, dt, int(dropout_p > 0.0)],
-                            ctypes.addressof(struct), 0)
+    if bias is None:
+        plan_cache.remember((plan,), generation, _native.ATTN_FWD, [col, indptr_c, eid_c, indices_c],
+                            [q.size(0), k.size(0), h, d, dt, int(dropout_p > 0.0)], ctypes.addressof(struct), 0)
     return o, lse
 
 
@@ -669,7 +667,6 @@ def attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, in
     """(dq, dk, dv) of attention_forward (same dropout_p, seed, bias and bias_by_pair).  With bias a fourth result: ds,
     float32 (E, h), or (h, E) with bias_by_pair, the gradient with respect to q.k + bias of every edge and head (= the
     gradient of bias), laid out like bias."""
-    cfg = _SETTINGS
     do = do.contiguous()
     if bias is None:
         known = _native.attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, o, lse, do,
@@ -677,6 +674,7 @@ def attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, in
                                            int(seed) & (2 ** 64 - 1))
         if known is not None:
             return known
+    generation, cfg = _native.generation(), _SETTINGS
     _check_all(row=row, indptr_r=indptr_r, eid_r=eid_r, indices_r=indices_r, col=col, indptr_c=indptr_c,
                eid_c=eid_c, indices_c=indices_c, q=q, k=k, v=v, o=o, lse=lse)
     _same_dtype(q, k, v, o, do)
@@ -736,9 +734,8 @@ def attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, in
                    "attention_backward")
     if bias is not None:
         return dq, dk, dv, ds if bias_by_pair else ds[:-1]
-    if cfg is _SETTINGS:
-        plan_cache.remember((plan_in, plan_out), _native.ATTN_BWD, [row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c],
-                            [q.size(0), k.size(0), h, d, dt, int(dropout_p > 0.0)], ctypes.addressof(in_struct), ctypes.addressof(out_struct))
+    plan_cache.remember((plan_in, plan_out), generation, _native.ATTN_BWD, [row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c],
+                        [q.size(0), k.size(0), h, d, dt, int(dropout_p > 0.0)], ctypes.addressof(in_struct), ctypes.addressof(out_struct))
     return dq, dk, dv
 
 

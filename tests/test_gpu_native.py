@@ -157,6 +157,37 @@ def test_threads_that_build_the_same_graph_at_once(tiles, monkeypatch):
     assert not failures
 
 
+@pytest.mark.parametrize("h,d", [(8, 64), (6, 50)])
+@pytest.mark.parametrize("when", ["get", "remember"])
+def test_a_choice_made_before_a_switch_changed_is_not_remembered(when, h, d, monkeypatch):
+    """Another thread changes a switch or a setting between the moment a call looks and the moment its choice is put into the table."""
+    from bpt_amd import graphop, op, plan
+    monkeypatch.setattr(graphop, "_MIN_GROUP_ITEMS", 0)
+    c = Case("bpt512_k4")
+    x = tuple(rand((c.n, h, d), torch.float32, s, 1.0 / 8).to(DEV) for s in (1, 2, 3, 4))
+    native = plan.PlanCache.native
+    original = getattr(plan.plan_cache, when)
+    for change in (lambda: graphop.set_tiles(False), lambda: setattr(graphop, "_MIN_GROUP_ITEMS", 10 ** 9)):
+        def meanwhile(*args, **kw):
+            if when == "remember":
+                change()
+                return original(*args, **kw)
+            result = original(*args, **kw)
+            change()
+            return result
+
+        plan.plan_cache.clear()
+        setattr(plan.plan_cache, when, meanwhile)
+        try:
+            step(op, args_of(c), *x)
+            served = native.take_used()              # (before the switches are put back, which clears the table)
+        finally:
+            delattr(plan.plan_cache, when)
+            graphop.set_tiles(True)
+            graphop._MIN_GROUP_ITEMS = 0
+        assert not served
+
+
 def test_an_entry_holds_its_index_tensors():
     """Their addresses are the key: nothing else may come to lie there while the entry stands."""
     import ctypes
@@ -166,7 +197,7 @@ def test_an_entry_holds_its_index_tensors():
     struct, before = graphop.PlanStruct(), torch.cuda.memory_allocated()
     index = [torch.zeros(1 << 20, dtype=torch.int64, device=DEV) for _ in range(4)]
     held = torch.cuda.memory_allocated()
-    assert native.remember(native.ATTN_FWD, index, [1, 1, 8, 64, 0, 0], ctypes.addressof(struct), 0, (object(),))
+    assert native.remember(native.generation(), native.ATTN_FWD, index, [1, 1, 8, 64, 0, 0], ctypes.addressof(struct), 0, (object(),))
     del index
     assert torch.cuda.memory_allocated() == held
     native.clear()

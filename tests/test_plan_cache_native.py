@@ -13,7 +13,7 @@ class Native:
     def __init__(self):
         self.table = {}
 
-    def remember(self, kind, index, extra, a, b, plans):
+    def remember(self, generation, kind, index, extra, a, b, plans):
         self.table[kind, tuple(id(t) for t in index)] = plans
 
     def forget(self, plan):
@@ -47,7 +47,7 @@ def cache(monkeypatch):
 
 
 def choice(index):
-    return 0, list(index), [0] * 6, 1, 0
+    return 0, 0, list(index), [0] * 6, 1, 0
 
 
 def test_a_plan_in_the_cache_is_remembered(cache):
