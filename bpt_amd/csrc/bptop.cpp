@@ -16,6 +16,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 
+#include <algorithm>
 #include <array>
 #include <atomic>
 #include <cstring>
@@ -36,7 +37,7 @@ namespace {
 
 enum Kind { ATTN_FWD = 0, ATTN_BWD = 1, ATTN_FWD_NARROW = 2, ATTN_BWD_NARROW = 3 };
 
-constexpr size_t MAX_TENSORS = 8, MAX_EXTRA = 6, MAX_ENTRIES = 512;
+constexpr size_t MAX_TENSORS = 8, MAX_EXTRA = 7, MAX_ENTRIES = 512;
 
 struct Key {                          // compared and hashed as bytes: always zeroed first
     int64_t kind, device;
@@ -268,7 +269,8 @@ std::optional<std::tuple<Tensor, Tensor>> narrow_forward_known(const Tensor &col
     Shape s;
     if (!attention_shape(q, k, v, p, s) || indices.sizes() != eid.sizes()) return std::nullopt;
     Key key;
-    if (!make_key(key, ATTN_FWD_NARROW, {&col, &indptr, &eid, &indices}, q.device(), {s.nq, s.nk, h, s.d, s.dt, s.h})) return std::nullopt;
+    if (!make_key(key, ATTN_FWD_NARROW, {&col, &indptr, &eid, &indices}, q.device(), {s.nq, s.nk, h, s.d, s.dt, p > 0.0, s.h}))
+        return std::nullopt;
     const EntryPtr e = find(key);
     if (!e) return std::nullopt;
     c10::DeviceGuard guard(q.device());
@@ -292,7 +294,7 @@ std::optional<Three> narrow_backward_known(const Tensor &row, const Tensor &indp
     if (indices_c.sizes() != eid_c.sizes() || indices_r.sizes() != eid_r.sizes() || eid_r.sizes() != eid_c.sizes()) return std::nullopt;
     Key key;
     if (!make_key(key, ATTN_BWD_NARROW, {&row, &indptr_r, &eid_r, &indices_r, &col, &indptr_c, &eid_c, &indices_c}, q.device(),
-                  {s.nq, s.nk, h, s.d, s.dt, s.h}))
+                  {s.nq, s.nk, h, s.d, s.dt, p > 0.0, s.h}))
         return std::nullopt;
     const EntryPtr e = find(key);
     if (!e) return std::nullopt;
@@ -322,11 +324,12 @@ std::tuple<Tensor, Tensor> narrow_forward(const Tensor &col, const Tensor &indpt
     return python("attention_forward")(col, indptr, eid, indices, qp, kp, kp, scale, p, (uint64_t)seed, **kw).cast<std::tuple<Tensor, Tensor>>();
 }
 
-bool narrow_known(const Tensor &col, const Tensor &indptr, const Tensor &eid, const Tensor &indices, const Tensor &q, const Tensor &k, int64_t h) {
+bool narrow_known(const Tensor &col, const Tensor &indptr, const Tensor &eid, const Tensor &indices, const Tensor &q, const Tensor &k, int64_t h,
+                  double p) {
     Key key;
     return q.is_cuda() && q.dim() == 3 &&
            make_key(key, ATTN_FWD_NARROW, {&col, &indptr, &eid, &indices}, q.device(),
-                    {q.size(0), k.size(0), h, q.size(2), dtype_code(q.scalar_type()), q.size(1)}) &&
+                    {q.size(0), k.size(0), h, q.size(2), dtype_code(q.scalar_type()), p > 0.0, q.size(1)}) &&
            find(key) != nullptr;
 }
 
@@ -335,7 +338,7 @@ struct NarrowAttention : torch::autograd::Function<NarrowAttention> {
                           const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c,
                           const Tensor &q, const Tensor &k, const Tensor &v, int64_t h, double scale, double p, int64_t seed) {
         const Tensor qc = rows(q), kc = rows(k), vc = rows(v);
-        if (!narrow_known(col, indptr_c, eid_c, indices_c, qc, kc, h))
+        if (!narrow_known(col, indptr_c, eid_c, indices_c, qc, kc, h, p))
             python("prepare_training")(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, qc, kc, p, h);
         const auto [o, lse] = narrow_forward(col, indptr_c, eid_c, indices_c, qc, kc, vc, h, scale, p, seed);
         ctx->save_for_backward({row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, qc, kc, vc, o, lse});
@@ -492,11 +495,12 @@ py::object build_tile_plans(const std::vector<std::tuple<Tensor, Tensor, Tensor,
 // what `plans` holds.  generation: what generation() said before the choice was begun; a table that was cleared since does not take
 // it, since a switch may have changed under it.  True if it was taken.
 bool remember(int64_t generation, int kind, const std::vector<Tensor> &index, const std::vector<int64_t> &extra, int64_t a, int64_t b, py::tuple plans) {
-    if (index.empty() || index.size() > MAX_TENSORS || extra.size() != MAX_EXTRA || !index[0].defined() || !index[0].is_cuda() || !a) return false;
+    if (index.empty() || index.size() > MAX_TENSORS || extra.size() > MAX_EXTRA || !index[0].defined() || !index[0].is_cuda() || !a) return false;
     std::vector<const Tensor *> ptrs;
     for (const Tensor &t : index) ptrs.push_back(&t);
     Key key;
-    if (!make_key(key, (Kind)kind, ptrs, index[0].device(), {extra[0], extra[1], extra[2], extra[3], extra[4], extra[5]})) return false;
+    if (!make_key(key, (Kind)kind, ptrs, index[0].device(), {})) return false;
+    std::copy(extra.begin(), extra.end(), key.extra.begin());
     auto e = std::make_shared<Entry>();
     std::memcpy(&e->a, reinterpret_cast<const void *>(a), sizeof(bpt_plan));
     if (b) std::memcpy(&e->b, reinterpret_cast<const void *>(b), sizeof(bpt_plan));

@@ -560,7 +560,7 @@ def _attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale
         check_attn(_LIB.bpt_attention_forward_narrow(ctypes.byref(struct), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(ws), nws, scale,
                                                      float(dropout_p), seed, heads, d, h, dt, _stream()), "attention_forward_narrow")
     plan_cache.remember((plan,), generation, _native.ATTN_FWD_NARROW, [col, indptr_c, eid_c, indices_c],
-                        [q.size(0), k.size(0), h, d, dt, heads], ctypes.addressof(struct), 0)
+                        [q.size(0), k.size(0), h, d, dt, int(dropout_p > 0.0), heads], ctypes.addressof(struct), 0)
     return o, lse
 
 
@@ -601,7 +601,7 @@ def attention_backward_narrow(row, indptr_r, eid_r, indices_r, col, indptr_c, ei
                                                       _ptr(dv), _ptr(ws), nws, scale, float(dropout_p), int(seed) & (2 ** 64 - 1), heads, d, h, dt,
                                                       _stream()), "attention_backward_narrow")
     plan_cache.remember((pi, po), generation, _native.ATTN_BWD_NARROW, [row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c],
-                        [q.size(0), k.size(0), h, d, dt, heads], ctypes.addressof(in_struct), ctypes.addressof(out_struct))
+                        [q.size(0), k.size(0), h, d, dt, int(dropout_p > 0.0), heads], ctypes.addressof(in_struct), ctypes.addressof(out_struct))
     return dq, dk, dv
 
 

@@ -111,3 +111,26 @@ def test_small_graphs_keep_the_row_kernels(dtype):
     for got, want in zip(*both):
         assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
         assert not got[n // 2:].isnan().any()                  # the second graph
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+def test_a_small_layer_is_the_same_after_one_with_dropout(dtype):
+    """Dropout puts a small layer on tiles; the layer without it keeps the row kernels, whichever call came first."""
+    from bpt_amd import graphbuilder as gb, graphop, plan
+    g = gb.BinaryPartition(300, True, 4, 10)
+    src, dst, _, _, n = gb.merge_graphs_device([g], torch.device(DEV))
+    out_csr, in_csr, row, ir, col, ic = gb.get_csrs_device(src, dst, n)
+    out, inn = (row, ir, out_csr[2], out_csr[1]), (col, ic, in_csr[2], in_csr[1])
+    q, k, v, do = (rand((n, 6, 50), dtype, s, 1.0 / 8).to(DEV) for s in (51, 52, 53, 54))
+    q[5] = float("inf")
+    stand_in = torch.empty(n, 8, 64, dtype=dtype, device="meta")
+
+    def layer(p):
+        o, lse = graphop.attention_forward(*inn, stand_in, stand_in, stand_in, 50 ** -0.5, p, 3, narrow=(q, k, v))
+        return (o, lse[:, :6], *graphop.attention_backward_narrow(*out, *inn, q, k, v, o, lse, do, 8, 50 ** -0.5, p, 3))
+
+    plan.plan_cache.clear()
+    cold = layer(0.0)
+    layer(0.1)
+    for got, want in zip(layer(0.0), cold):
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
