@@ -190,9 +190,10 @@ __global__ __launch_bounds__(BLOCK) void k_spmm_generic(bpt_plan P, const T *__r
 // Heads of fewer than 64 columns (6 x 50, 8 x 40), read and written as they are in memory by the NARROW forms of the tile kernels.
 // The products keep their 64 columns: quad j of a head (the four columns a lane group position stands for) starts at column
 // 4 j, or at d - 4 where that would run over the end of the head.  What a shifted quad repeats of its neighbour, and the quads past
-// the end, count for nothing because the member's operand is zero there (tile_load16, tile_load_row_bf16); results are
-// stored from the quads that start inside the head, a repeated column twice with one value.  No other head's memory is
-// touched, so what stands there does not matter.
+// the end, are zero in both operands of the products over the columns (the members': tile_load16, tile_load_row_bf16; the
+// entries': tile_rows_to_operand): a masking -inf in one of the last columns counts once, as in a zero-padded head, where
+// zero in one operand alone would make it NaN.  Results are stored from the quads that start inside the head, a repeated column
+// twice with one value.  No other head's memory is touched, so what stands there does not matter.
 // Against copies padded to 64 columns and 4, 8 or 16 heads (three pads, the output and its gradient, three slices, and the
 // padding heads computed with the rest): 33 765 nodes / 576 k edges at 6 x 50 with dropout, forward and backward,
 // 508 -> 207 us; of that copies 223, the rest two padding heads of eight.
@@ -203,6 +204,10 @@ struct Narrow {
 };
 constexpr int NARROW_HW = 2;   // heads per workgroup (6 x 50: three workgroups of two, none of them half empty)
 __device__ __forceinline__ int narrow_col(const Narrow &nw, int quad) { return min(4 * quad, nw.d - 4); }
+// whether column e of the quad as loaded is one that the quad before has (or, past the end of the head, any): 4 quad > d - 4 + e
+template <bool NARROW> __device__ __forceinline__ bool narrow_again(const Narrow &nw, int quad, int e) {
+    return NARROW && quad > (nw.d - 4 + e) >> 2;
+}
 typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));           // such rows start anywhere on 4 bytes
 typedef uint32_t uintx2u __attribute__((ext_vector_type(2), aligned(4)));
 
@@ -1889,10 +1894,13 @@ __device__ __forceinline__ uint32_t tile_bias_at(const bpt_plan &P, int head, in
 // instead of one.  So the rows are loaded once, in the first layout, and turned in a wavefront-private piece of LDS:
 // rows of TILE_KT_STRIDE floats (64 + 4: the sixteen rows of a read fall on different banks).
 constexpr int TILE_KT_STRIDE = 68;
-__device__ __forceinline__ void tile_rows_to_operand(float *kt, const float4 (&rows)[4], int c, int g, float (&out)[16]) {
+template <bool NARROW>
+__device__ __forceinline__ void tile_rows_to_operand(float *kt, const float4 (&rows)[4], int c, int g, float (&out)[16], const Narrow &nw) {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-        *reinterpret_cast<floatx4v *>(kt + (4 * r + g) * TILE_KT_STRIDE + 4 * c) = floatx4v{rows[r].x, rows[r].y, rows[r].z, rows[r].w};
+        *reinterpret_cast<floatx4v *>(kt + (4 * r + g) * TILE_KT_STRIDE + 4 * c) =
+            floatx4v{narrow_again<NARROW>(nw, c, 0) ? 0.f : rows[r].x, narrow_again<NARROW>(nw, c, 1) ? 0.f : rows[r].y,
+                     narrow_again<NARROW>(nw, c, 2) ? 0.f : rows[r].z, narrow_again<NARROW>(nw, c, 3) ? 0.f : rows[r].w};
     wave_lds_fence();
     const float *src = kt + tile_entry_of_row(c) * TILE_KT_STRIDE + 4 * g;
 #pragma unroll
@@ -2045,7 +2053,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
         };
         auto compute = [&](const Blk &B) {
             float kr[16];
-            tile_rows_to_operand(kt, B.kq, c, g, kr);
+            tile_rows_to_operand<NARROW>(kt, B.kq, c, g, kr, nw);
             const floatx4v st = tile_dot(kr, qb);
             float sc[4];
 #pragma unroll
@@ -2189,11 +2197,11 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
             floatx4v st;
             {
                 float kr[16];
-                tile_rows_to_operand(kt, B.kc, c, g, kr);
+                tile_rows_to_operand<NARROW>(kt, B.kc, c, g, kr, nw);
                 st = tile_dot(kr, qb);
             }
             float va[16];
-            tile_rows_to_operand(kt, B.vc, c, g, va);
+            tile_rows_to_operand<NARROW>(kt, B.vc, c, g, va, nw);
             float dob[16];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -2419,9 +2427,12 @@ template <bool NARROW> __device__ __forceinline__ uint2 tile_row4_bf16(const cha
 // Rows of TILE_KT_BYTES_BF16 = 128 + 16 bytes: the sixteen rows of a read fall on different banks.
 constexpr int TILE_KT_BYTES_BF16 = 144;
 typedef uint32_t uintx4v __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void tile_rows_to_operand_bf16(char *kt, const uint2 (&rows)[4], int c, int g, Bf8 (&out)[2]) {
+template <bool NARROW>
+__device__ __forceinline__ void tile_rows_to_operand_bf16(char *kt, const uint2 (&rows)[4], int c, int g, Bf8 (&out)[2], const Narrow &nw) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) *reinterpret_cast<uintx2v *>(kt + (4 * g + r) * TILE_KT_BYTES_BF16 + 8 * c) = uintx2v{rows[r].x, rows[r].y};
+    for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<uintx2v *>(kt + (4 * g + r) * TILE_KT_BYTES_BF16 + 8 * c) =           // (d is even: words are whole)
+            uintx2v{narrow_again<NARROW>(nw, c, 0) ? 0u : rows[r].x, narrow_again<NARROW>(nw, c, 2) ? 0u : rows[r].y};
     wave_lds_fence();
     const char *src = kt + c * TILE_KT_BYTES_BF16 + 32 * g;
 #pragma unroll
@@ -2499,7 +2510,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
         };
         auto compute = [&](const Blk &B) {
             Bf8 kr[2];
-            tile_rows_to_operand_bf16(kt, B.kq, c, g, kr);
+            tile_rows_to_operand_bf16<NARROW>(kt, B.kq, c, g, kr, nw);
             const floatx4v st = tile_dot_bf16(kr, qb);
             float sc[4];
 #pragma unroll
@@ -2638,9 +2649,9 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
         };
         auto compute = [&](const Blk &B) {
             Bf8 kr[2];
-            tile_rows_to_operand_bf16(kt, B.kc, c, g, kr);
+            tile_rows_to_operand_bf16<NARROW>(kt, B.kc, c, g, kr, nw);
             const floatx4v st = tile_dot_bf16(kr, qb);
-            tile_rows_to_operand_bf16(kt, B.vc, c, g, kr);
+            tile_rows_to_operand_bf16<NARROW>(kt, B.vc, c, g, kr, nw);
             const floatx4v dp = tile_dot_bf16(kr, dob);
             float ds[4];
 #pragma unroll
@@ -2811,11 +2822,11 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
         auto compute = [&](const Blk &B) {
             if (g == 0) st_lds[c] = B.ld;
             Bf8 row[2];
-            tile_rows_to_operand_bf16(kt, B.qr, c, g, row);
+            tile_rows_to_operand_bf16<false>(kt, B.qr, c, g, row, nw);
             const floatx4v l01 = *reinterpret_cast<const floatx4v *>(&st_lds[4 * g]), l23 = *reinterpret_cast<const floatx4v *>(&st_lds[4 * g + 2]);
             const float lse_e[4] = {l01[0], l01[2], l23[0], l23[2]}, delta_e[4] = {l01[1], l01[3], l23[1], l23[3]};
             const floatx4v st = tile_dot_bf16(row, kb);
-            tile_rows_to_operand_bf16(kt, B.dr, c, g, row);
+            tile_rows_to_operand_bf16<false>(kt, B.dr, c, g, row, nw);
             const floatx4v dp = tile_dot_bf16(row, vb);
             float pe[4], ds[4];
 #pragma unroll

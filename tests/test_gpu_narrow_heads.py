@@ -134,3 +134,31 @@ def test_a_small_layer_is_the_same_after_one_with_dropout(dtype):
     layer(0.1)
     for got, want in zip(layer(0.0), cold):
         assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
+@pytest.mark.parametrize("p", [0.0, 0.1])
+@pytest.mark.parametrize("dtype,h,d", [(torch.float32, 8, 40), (torch.float32, 6, 50), (torch.float32, 5, 51), (torch.float32, 3, 5), (torch.bfloat16, 8, 40),
+                                       (torch.bfloat16, 6, 50)], ids=lambda x: str(x).replace("torch.", ""))
+def test_a_mask_column_of_minus_infinity(dtype, h, d, p, monkeypatch):
+    """-inf in one of the last columns of some key rows, where the query rows hold one: their edges have probability zero, and what is
+    finite, infinite or NaN is what it is on the padded layer's tiles."""
+    from bpt_amd import graphop, op
+    monkeypatch.setattr(graphop, "_MIN_GROUP_ITEMS", 0)       # (tiles whatever the graph's size)
+    c = case("bpt512_k4")
+    q, k, v, do = (rand((c.n, h, d), dtype, s, 1.0 / 8).to(DEV) for s in (41, 42, 43, 44))
+    hp = graphop.attention_padded_shape(q)[0]
+    grow = lambda x: torch.nn.functional.pad(x, (0, 64 - d, 0, hp - h))
+    masked = torch.arange(0, c.n, 7, device=DEV)
+    for col in range(d - 4, d):
+        qm, km = q.clone(), k.clone()
+        qm[..., col], km[..., col] = 1.0, 0.0
+        km[masked, :, col] = float("-inf")
+        both = []
+        for narrow in (True, False):
+            x = [t.detach().requires_grad_(True) for t in (qm, km, v)]
+            o = op.bpt_attention(*c.out, *c.inn, *(x if narrow else [grow(t) for t in x]), scale=d ** -0.5, dropout_p=p, seed=5)[:, :h, :d]
+            both.append((o.detach(), *torch.autograd.grad(o, x, do)))
+        assert both[1][0].isfinite().all() and not both[0][3][masked].any()
+        for got, want, name in zip(both[0], both[1], ("o", "dq", "dk", "dv")):
+            assert torch.equal(got.isfinite(), want.isfinite()) and torch.equal(got.isnan(), want.isnan()), name
+            close(got.nan_to_num(), f64(want.nan_to_num()), TOL[dtype] if name == "o" else GTOL[dtype], name)
