@@ -805,14 +805,18 @@ class PlanCache:
 
     def put_tile_plans(self, sides):
         """What get() would build one after the other for a training step on tiles, built together (DevicePlan.tile_plans; sides as
-        there: the in-side, then the out-side), unless one of them is already here or they have to be built one by one."""
+        there: the in-side, then the out-side), unless one of them is already here or they have to be built one by one.  A side that is
+        malformed is refused where it is asked for: a forward never asks for the out-side."""
         if self.native is None or DEVICE_BUILD is False or not sides[0][2].is_cuda:
             return
         keys = [self._key(side[:4], side[4], side[5], side[6], True) for side in sides]
         with self._lock:
             if any(key in self._d for key in keys):
                 return
-        plans = DevicePlan.tile_plans(sides)
+        try:
+            plans = DevicePlan.tile_plans(sides)
+        except ValueError:
+            plans = None
         if plans is None:
             return
         self.misses += len(plans)

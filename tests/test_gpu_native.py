@@ -91,6 +91,31 @@ def test_a_known_graph_still_refuses_wrong_arguments():
         graphop.attention_backward(*c.out, *c.inn, q, k, v, o, lse[:-1].contiguous(), do)
 
 
+@pytest.mark.parametrize("h,d", [(8, 64), (6, 50)])
+def test_a_malformed_out_side_is_refused_by_the_backward(h, d, monkeypatch):
+    """The forward reads the in-side alone, also where both sides' plans are built with it."""
+    from bpt_amd import graphop, op, plan
+    monkeypatch.setattr(graphop, "_MIN_GROUP_ITEMS", 0)
+    c = Case("bpt512_k4")
+    q, k, v, do = (rand((c.n, h, d), torch.float32, s, 1.0 / 8).to(DEV) for s in (1, 2, 3, 4))
+    q.requires_grad_(True)
+    plan.plan_cache.clear()
+    with torch.no_grad():
+        want = op.bpt_attention(*args_of(c), q, k, v)
+    for side, place in ((0, 3), (1, 7)):
+        args = [t.clone() for t in args_of(c)]
+        args[place][5] = c.n                                  # (a column that is no node: the builder's check refuses it)
+        plan.plan_cache.clear()
+        if side == 1:
+            with pytest.raises(ValueError, match="out of range"):
+                op.bpt_attention(*args, q, k, v)
+            continue
+        o = op.bpt_attention(*args, q, k, v)
+        assert torch.equal(o, want)
+        with pytest.raises(ValueError, match="out of range"):
+            torch.autograd.grad(o, q, do)
+
+
 def test_threads_and_streams():
     from bpt_amd import op
     c = Case("bpt512_k4")
