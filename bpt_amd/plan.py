@@ -461,6 +461,7 @@ class DevicePlan:
         """The plans, with their tile groups, of one side of a graph or of both, built together (bpt_build_tiles_count / _write in
         bptop.so); the second is linked to the first by pair numbers.  sides: (row, indptr, eid, indices, n_rows, n_index_nodes,
         seg_len, order_mode of the groups).  None where the plans have to be built one by one."""
+        from ._native import native
         self_of = []
         for row, indptr, eid, indices, n_rows, n_index_nodes, seg_len, order in sides:
             self = cls.__new__(cls)
@@ -469,7 +470,7 @@ class DevicePlan:
             self._groups, self._links, self._bias_rows, self._lock = {}, {}, {}, threading.Lock()
             self._max_items = self.n_rows + self.n_edges // self.seg_len
             self_of.append((self, self._by_mask(TILE_GROUP_R, order)))
-        built = PlanCache.native.build_tile_plans([(*side[:7], by_mask) for side, (_, by_mask) in zip(sides, self_of)])
+        built = native.build_tile_plans([(*side[:7], by_mask) for side, (_, by_mask) in zip(sides, self_of)])
         if built is None:
             return None
         arrays, pairs = built

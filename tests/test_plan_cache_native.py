@@ -1,6 +1,10 @@
 """What the plan cache (bpt_amd/plan.py) tells the native host path, whose table answers calls by the addresses of their index tensors:
 an entry is let in only while its plans are in the cache, and a plan that other threads may have taken from the cache is not
 replaced.  CPU only: the native side is a stub, other threads' doings are put where they would fall."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -130,3 +134,11 @@ def test_two_threads_that_build_both_sides_share_the_first(cache, monkeypatch):
     monkeypatch.setattr(plan_mod.DevicePlan, "tile_plans", staticmethod(tile_plans))
     cache.put_tile_plans(sides)
     assert len(built) == 2 and [p for p, _ in cache._d.values()] == built[1] and cache._total == 2
+
+
+def test_joint_plans_without_the_ops():
+    """DevicePlan.tile_plans where nothing has imported the ops: tensors that are not on a GPU are left to the other builders."""
+    code = ("import sys, torch; from bpt_amd.plan import DevicePlan; t = torch.zeros(2, dtype=torch.int64); "
+            "assert 'bpt_amd.graphop' not in sys.modules; assert DevicePlan.tile_plans([(t[:1], t, t[:1], t[:1], 1, 1, 64, None)]) is None")
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    subprocess.run([sys.executable, "-c", code], cwd=root, check=True)
