@@ -307,8 +307,16 @@ def merge_graphs(graphs):
     return cat(src), cat(dst), cat(et), cat(pos), v_shift
 
 
-_DEVICE_EDGES = {}           # (graph class, constructor arguments, device) -> (src, dst, etype, pos) device tensors and their part record
+_DEVICE_EDGES = {}           # (_edges_key of the graph, device) -> (src, dst, etype, pos) device tensors and their part record
 _DEVICE_EDGES_MAX = 4096
+
+
+def _edges_key(g):
+    """What a graph's edge list is a function of: its class and constructor arguments, as pickling has them (a subclass may have
+    more of them; the classes here are asked without the call, some 0.3 us a graph)."""
+    if type(g) in (BinaryPartition, FullyConnected, OpenAISparse):
+        return type(g), g._length, g._triu, g._a, g._b
+    return (type(g), *g.__reduce__()[1])
 
 
 def merge_graphs_device(graphs, device):
@@ -323,7 +331,7 @@ def merge_graphs_device(graphs, device):
         device = torch.device("cuda", torch.cuda.current_device())
     parts, lists, n_edges, n_nodes = [], [], 0, 0
     for g in graphs:
-        key = (type(g), g._length, g._triu, g._a, g._b, device)
+        key = (_edges_key(g), device)
         hit = _DEVICE_EDGES.get(key)
         if hit is None:
             if len(_DEVICE_EDGES) >= _DEVICE_EDGES_MAX:

@@ -81,6 +81,46 @@ def test_merge_at_the_edges_of_a_launch(n_graphs):
         assert a.dtype == torch.int64 and np.array_equal(a.cpu().numpy(), b)
 
 
+def test_merge_keeps_graphs_apart_that_a_subclass_tells_apart():
+    """A subclass with a constructor argument of its own, and a class that only has what the merge calls."""
+    from bpt_amd import graphbuilder as gb
+
+    class Without(gb.BinaryPartition):                            # leaves out the edges of some types
+        def __init__(self, length, types):
+            super().__init__(length, True, 4, 10)
+            self.types = types
+
+        def __reduce__(self):
+            return Without, (self._length, self.types)
+
+        def get_edges_device(self, device, v_shift=0):
+            src, dst, etype = super().get_edges_device(device, v_shift)
+            keep = ~torch.isin(etype, torch.tensor(self.types, device=device))
+            return src[keep], dst[keep], etype[keep]
+
+    class Chain:
+        number_of_nodes = 4
+
+        def __reduce__(self):
+            return Chain, ()
+
+        def get_edges_device(self, device):
+            i = torch.arange(3, device=device)
+            return i, i + 1, torch.zeros_like(i)
+
+        def get_pos(self):
+            return np.arange(4)
+
+    plain, some, more = gb.BinaryPartition(30, True, 4, 10), Without(30, (0,)), Without(30, (0, 1))
+    n = plain.number_of_nodes
+    src, dst, etype, pos, nodes = gb.merge_graphs_device([plain, some, more, Chain()], DEV)
+    _, _, want = plain.get_edges()
+    want = [want, want[want > 0], want[want > 1], np.zeros(3, dtype=np.int64)]
+    assert nodes == 3 * n + 4 and pos.numel() == nodes
+    assert np.array_equal(etype.cpu().numpy(), np.concatenate(want))
+    assert src[-3:].tolist() == [3 * n, 3 * n + 1, 3 * n + 2] and dst[-1].item() == 3 * n + 3
+
+
 @pytest.mark.parametrize("n_src,n_dst,E,seg,orders", [(300, 300, 6000, 64, (None, 0)), (40, 900, 5000, 64, (6, 6)), (900, 40, 5000, 128, (4, 2)),
                                                       (1, 1, 1, 64, (None, 0)), (5000, 64, 70000, 64, (None, 0))])
 def test_both_sides_built_together(n_src, n_dst, E, seg, orders):
