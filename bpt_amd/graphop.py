@@ -154,7 +154,7 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None and t.numel() else None
 
 
-def _workspace(op, plan, plan_t, h, d, dt, device, plan_ref=None, plan_t_ref=None):
+def _workspace(op, plan, plan_t, h, d, dt, device, plan_ref=None, plan_t_ref=None, keep=True):
     if plan_t_ref is None and plan_t is not None:
         plan_t_ref = plan_t.ref
     n = _LIB.bpt_workspace_bytes(op, plan.ref if plan_ref is None else plan_ref, plan_t_ref, h, d, dt)
@@ -162,13 +162,16 @@ def _workspace(op, plan, plan_t, h, d, dt, device, plan_ref=None, plan_t_ref=Non
         raise RuntimeError("bpt_workspace_bytes failed")
     if n == 0:
         return None, 0
-    return _scratch(n, device), n
+    return _scratch(n, device) if keep else torch.empty(n, dtype=torch.uint8, device=device), n
 
 
 # Workspaces are kept per (device, stream) and grown on demand: calls on one stream are ordered, so the next call may
-# overwrite what the previous one left there, and a step no longer asks the allocator for tens of MB per call (after
+# overwrite what the previous one left there, and a step does not ask the allocator for tens of MB per call (after
 # torch.cuda.empty_cache() such requests were measured at 0.16 ms each, GPU idle).  Under stream capture the buffer comes
 # from the capture's own pool as before.  release_workspaces() gives the memory back.
+# Fused attention without a score term keeps none: from its second call on a graph it is served by the native host path, which
+# asks the allocator (the same block comes back call after call), and what the first call had left here would lie idle beside it
+# (422 MB at L = 32768, k = 8, 16 heads).
 _SCRATCH = {}
 _SCRATCH_LOCK = threading.Lock()
 KEEP_WORKSPACES = True
@@ -555,7 +558,7 @@ def _attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale
     o = torch.empty_like(q)
     lse = torch.empty((q.size(0), h), dtype=torch.float32, device=q.device)
     dt = _dtype(q)
-    ws, nws = _workspace(OP_ATTN_FWD, plan, None, h, 64, dt, q.device)
+    ws, nws = _workspace(OP_ATTN_FWD, plan, None, h, 64, dt, q.device, keep=False)
     with _on_device_of(q):
         check_attn(_LIB.bpt_attention_forward_narrow(ctypes.byref(struct), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(ws), nws, scale,
                                                      float(dropout_p), seed, heads, d, h, dt, _stream()), "attention_forward_narrow")
@@ -595,7 +598,7 @@ def attention_backward_narrow(row, indptr_r, eid_r, indices_r, col, indptr_c, ei
     dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
     dt = _dtype(q)
     in_ref, out_ref = ctypes.byref(in_struct), ctypes.byref(out_struct)
-    ws, nws = _workspace(OP_ATTN_BWD, pi, po, h, 64, dt, q.device, plan_ref=in_ref, plan_t_ref=out_ref)
+    ws, nws = _workspace(OP_ATTN_BWD, pi, po, h, 64, dt, q.device, plan_ref=in_ref, plan_t_ref=out_ref, keep=False)
     with _on_device_of(q):
         check_attn(_LIB.bpt_attention_backward_narrow(in_ref, out_ref, _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(do), _ptr(lse), _ptr(dq), _ptr(dk),
                                                       _ptr(dv), _ptr(ws), nws, scale, float(dropout_p), int(seed) & (2 ** 64 - 1), heads, d, h, dt,
@@ -651,7 +654,7 @@ def attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale=None, drop
     o = torch.empty_like(q)
     lse = torch.empty((q.size(0), h), dtype=torch.float32, device=q.device)
     dt = _dtype(q)
-    ws, nws = _workspace(OP_ATTN_FWD, plan, None, h, d, dt, q.device)
+    ws, nws = _workspace(OP_ATTN_FWD, plan, None, h, d, dt, q.device, keep=bias is not None)
     with _on_device_of(q):
         check_attn(_LIB.bpt_attention_forward(ref, _ptr(q), _ptr(k), _ptr(v), _ptr(bias), _ptr(o), _ptr(lse), _ptr(ws), nws,
                                               scale, float(dropout_p), int(seed) & (2 ** 64 - 1), h, d, dt, _stream()),
@@ -726,7 +729,7 @@ def attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, in
     in_ref, out_ref = ctypes.byref(in_struct), ctypes.byref(out_struct)
     if bias_by_pair and not (tiles and bias is not None):
         raise RuntimeError("bias_by_pair: this call does not run on the tile kernels (ask attention_pair_rows() first)")
-    ws, nws = _workspace(OP_ATTN_BWD, plan_in, plan_out, h, d, dt, q.device, plan_ref=in_ref, plan_t_ref=out_ref)
+    ws, nws = _workspace(OP_ATTN_BWD, plan_in, plan_out, h, d, dt, q.device, plan_ref=in_ref, plan_t_ref=out_ref, keep=bias is not None)
     with _on_device_of(q):
         check_attn(_LIB.bpt_attention_backward(in_ref, out_ref, _ptr(q), _ptr(k), _ptr(v), _ptr(bias), _ptr(o), _ptr(do),
                                                _ptr(lse), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(ds), _ptr(ws), nws,

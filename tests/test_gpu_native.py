@@ -182,6 +182,32 @@ def test_threads_that_build_the_same_graph_at_once(tiles, monkeypatch):
     assert not failures
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("h,d", [(8, 64), (6, 50)])
+def test_no_workspace_lies_idle_beside_that_of_served_calls(h, d, dtype):
+    """What a step leaves allocated is its plans, from the first call on; with a score term, whose calls are never served natively, one
+    workspace is kept."""
+    from bpt_amd import graphbuilder as gb, graphop, op, plan
+    g = gb.BinaryPartition(2048, False, 4, 10)
+    src, dst, etype, _, n = gb.merge_graphs_device([g], torch.device(DEV))
+    out_csr, in_csr, row, ir, col, ic = gb.get_csrs_device(src, dst, n)
+    args = (row, ir, out_csr[2], out_csr[1], col, ic, in_csr[2], in_csr[1])
+    x = tuple(rand((n, h, d), dtype, s, 1.0 / 8).to(DEV) for s in (1, 2, 3, 4))
+    plan.plan_cache.clear()
+    graphop.release_workspaces()
+    held = []
+    for _ in range(3):
+        step(op, args, *x)
+        held.append(torch.cuda.memory_allocated())
+    assert not graphop._SCRATCH and held[0] == held[1] == held[2]
+    if d == 64:
+        q = x[0].clone().requires_grad_(True)
+        o = op.bpt_attention(*args, q, *x[1:3], rel_table=torch.zeros(1000, d, dtype=dtype, device=DEV), etype=etype)
+        torch.autograd.grad(o, q, x[3])
+        assert len(graphop._SCRATCH) == 1
+    graphop.release_workspaces()
+
+
 @pytest.mark.parametrize("h,d", [(8, 64), (6, 50)])
 @pytest.mark.parametrize("when", ["get", "remember"])
 def test_a_choice_made_before_a_switch_changed_is_not_remembered(when, h, d, monkeypatch):
