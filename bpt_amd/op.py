@@ -281,6 +281,12 @@ def edge_type_embedding(table, etype):
     return EdgeTypeEmbedding.apply(table, etype, _type_csr(etype, table.size(0)))
 
 
+def _served_natively(graph):
+    """Whether bptop.so's function may take the call: a trace records the Python function, not what the native one launches, and a
+    caller that only wants a forward may leave the out-CSR side out (None), which is no tensor to it."""
+    return graph[0] is not None and graph[1] is not None and graph[2] is not None and graph[3] is not None and not torch.jit.is_tracing()
+
+
 def bpt_attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale=None, fused=None,
                   dropout_p=0.0, seed=None, rel_table=None, etype=None):
     """Attention over the graph: (ROW, INDPTR_R, out_eid, out_idx) is the out-CSR side (rows =
@@ -320,8 +326,7 @@ def bpt_attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices
         graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
         grow = lambda x: torch.nn.functional.pad(x, (0, dp - d, 0, hp - h))
         if rel_table is None:
-            # (a trace records the Python function, not what the native one launches)
-            if not torch.jit.is_tracing() and _g.attention_reads_narrow(col, eid_c, q, k, hp, dropout_p):
+            if _served_natively(graph) and _g.attention_reads_narrow(col, eid_c, q, k, hp, dropout_p):
                 return _native.attention_narrow(*graph, q, k, v, hp, scale, float(dropout_p), int(seed or 0) & (2 ** 64 - 1))
             o = BPTAttention.apply(*graph, grow(q), grow(k), grow(v), scale, float(dropout_p), int(seed or 0))
             return o[:, :h, :d].contiguous()
@@ -334,7 +339,7 @@ def bpt_attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices
         if rel_table is not None:
             return BPTRelAttention.apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale,
                                          float(dropout_p), int(seed or 0), rel_table, etype)
-        if torch.jit.is_tracing():
+        if not _served_natively((row, indptr_r, eid_r, indices_r)):
             return BPTAttention.apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale,
                                       float(dropout_p), int(seed or 0))
         return _native.attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale, float(dropout_p),

@@ -116,6 +116,25 @@ def test_a_malformed_out_side_is_refused_by_the_backward(h, d, monkeypatch):
             torch.autograd.grad(o, q, do)
 
 
+@pytest.mark.parametrize("h,d", [(8, 64), (6, 50)])
+def test_a_forward_does_without_the_out_side(h, d, monkeypatch):
+    """None in place of the out-CSR's tensors: only a backward reads them, also where gradients are recorded."""
+    from bpt_amd import graphop, op, plan
+    monkeypatch.setattr(graphop, "_MIN_GROUP_ITEMS", 0)
+    c = Case("bpt512_k4")
+    q, k, v, do = (rand((c.n, h, d), torch.float32, s, 1.0 / 8).to(DEV) for s in (1, 2, 3, 4))
+    with torch.no_grad():
+        want = op.bpt_attention(*args_of(c), q, k, v)
+    for known in (False, True):
+        if not known:
+            plan.plan_cache.clear()
+        with torch.no_grad():
+            got = op.bpt_attention(None, None, None, None, *c.inn, q, k, v)
+        o = op.bpt_attention(None, None, None, None, *c.inn, q.detach().requires_grad_(True), k, v)
+        torch.testing.assert_close(got, want, rtol=1e-5, atol=1e-6)
+        torch.testing.assert_close(o, want, rtol=1e-5, atol=1e-6)
+
+
 def test_threads_and_streams():
     from bpt_amd import op
     c = Case("bpt512_k4")
