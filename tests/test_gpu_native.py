@@ -1,6 +1,7 @@
 """The native host path (bpt_amd/csrc/bptop.cpp): a call served from its table gives the bits of the call that was remembered, a
 changed or dropped plan is not served, refused arguments raise as before, threads with streams of their own agree."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -201,6 +202,16 @@ def test_threads_that_build_the_same_graph_at_once(tiles, monkeypatch):
     assert not failures
 
 
+def allocated_at_rest():
+    """Bytes allocated once autograd's thread has let go of the last step (it drops its reference to the gradients after handing them
+    over, which the caller does not wait for)."""
+    seen = []
+    for _ in range(25):
+        seen.append(torch.cuda.memory_allocated())
+        time.sleep(0.002)
+    return min(seen)
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 @pytest.mark.parametrize("h,d", [(8, 64), (6, 50)])
 def test_no_workspace_lies_idle_beside_that_of_served_calls(h, d, dtype):
@@ -217,7 +228,7 @@ def test_no_workspace_lies_idle_beside_that_of_served_calls(h, d, dtype):
     held = []
     for _ in range(3):
         step(op, args, *x)
-        held.append(torch.cuda.memory_allocated())
+        held.append(allocated_at_rest())
     assert not graphop._SCRATCH and held[0] == held[1] == held[2]
     if d == 64:
         q = x[0].clone().requires_grad_(True)
