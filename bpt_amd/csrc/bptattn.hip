@@ -4275,12 +4275,17 @@ inline bool tiled_backward(const bpt_plan *Pin, const bpt_plan *Pout, int h, int
     return has_tiles(Pin, h, d, elem) && has_tiles(Pout, h, d, elem) && Pout->grp_pairs;
 }
 
-// float2 (p, ds) scratch of the fused backward: one per (entry, member) of the source-side groups (plus the
-// look-ahead padding) for the row-group kernels, one per edge for the per-row and the tile kernels
-inline int64_t pds_bytes(const bpt_plan *Pin, const bpt_plan *Pout, int h, int d, size_t elem) {
+// What the two backward kernels hand each other.  float2 (p, ds): one per (entry, member) of the source-side groups (plus the
+// look-ahead padding) for the row-group kernels, one per edge for the per-row and the float32 tile kernels.  bfloat16 tiles: (p, ds)
+// in four bytes per edge, or (lse, delta) of the rows where the source side forms the pairs again, which `plain` calls (64-column
+// rows, no score term) always do if the plan has its edge ids: L = 32768, k = 8, 16 heads 8.4 MB, where the pairs would be 211.
+inline int64_t pds_bytes(const bpt_plan *Pin, const bpt_plan *Pout, int h, int d, size_t elem, bool plain) {
     int64_t n = Pin->n_edges;
+    if (Pout && elem == 2 && tiled_backward(Pin, Pout, h, d, elem)) {
+        const int64_t rows = std::max(Pin->n_rows, Pout->n_index_nodes) * h * 8;
+        return round16(plain && Pout->grp_eids ? rows : std::max(rows, n * h * 4));
+    }
     if (Pout && grouped_backward(Pin, Pout, h, d, elem)) n = std::max(n, (Pout->n_grp_entries + GRP_PAD_ENTRIES) * Pout->grp_R);
-    if (Pout && elem == 2 && tiled_backward(Pin, Pout, h, d, elem)) n = std::max(n, std::max(Pin->n_rows, Pout->n_index_nodes));   // (lse, delta) of the rows
     return 2 * round16(n * h * 4);
 }
 
@@ -4384,7 +4389,7 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
                  float *ds_out, hipStream_t s) {
     if (Pin->n_items == 0) return BPT_OK;
     const bool grouped = grouped_backward(Pin, Pout, H, D, sizeof(T));
-    const int64_t pbytes = pds_bytes(Pin, Pout, H, D, sizeof(T));
+    const int64_t pbytes = pds_bytes(Pin, Pout, H, D, sizeof(T), !bias);
     float *pbuf = (float *)ws;                                   // per-row kernels: p (E, H) then ds (E, H)
     float *dsbuf = pbuf + pbytes / 8;
     float2 *pds = (float2 *)ws;                                  // row-group kernels: interleaved (p, ds)
@@ -4568,7 +4573,7 @@ int run_attn_bwd_narrow(const bpt_plan *Pin, const bpt_plan *Pout, const void *q
     if (Pin->n_items == 0) return BPT_OK;
     using pds_t = std::conditional_t<sizeof(T) == 4, float2, uint32_t>;
     pds_t *pds = (pds_t *)ws;
-    float *ws_dq = (float *)ws + pds_bytes(Pin, Pout, nw.h, 64, sizeof(T)) / 4;
+    float *ws_dq = (float *)ws + pds_bytes(Pin, Pout, nw.h, 64, sizeof(T), false) / 4;
     float *ws_dk = ws_dq + (size_t)Pin->n_slots * nw.h * 64, *ws_dv = ws_dk + (size_t)Pout->n_slots * nw.h * 64;
     const dim3 grid(group_grid(Pin) * nw.slices), grid_src(group_grid(Pout) * nw.slices), block(NARROW_HW * WAVE);
     {
@@ -4711,9 +4716,10 @@ int64_t bpt_workspace_bytes(int op, const bpt_plan *plan, const bpt_plan *plan_t
         case BPT_OP_ATTN_FWD: return round16(s0 * (C + 2 * h) * 4);
         case BPT_OP_SOFTMAX_FWD: return WAVE % h == 0 ? round16(s0 * h * 2 * a) : 0;      // (m, s) of every segment and head
         case BPT_OP_SOFTMAX_BWD: return WAVE % h == 0 ? round16(s0 * h * a) : 0;
-        case BPT_OP_ATTN_BWD: {
+        case BPT_OP_ATTN_BWD:
+        case BPT_OP_ATTN_BWD_PLAIN: {
             // partial rows of dq, then of dk and dv (the three are merged by one launch after the source-side kernel)
-            return pds_bytes(plan, plan_t, h, d, dtype == BPT_BF16 ? 2 : 4) + round16((s0 + 2 * s1) * C * 4);
+            return pds_bytes(plan, plan_t, h, d, dtype == BPT_BF16 ? 2 : 4, op == BPT_OP_ATTN_BWD_PLAIN) + round16((s0 + 2 * s1) * C * 4);
         }
         default: return -1;
     }
@@ -4956,7 +4962,7 @@ int bpt_attention_backward(const bpt_plan *plan_in, const bpt_plan *plan_out, co
     if (!fast_shape(h, d, dtype) || !aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(o) || !aligned16(d_o) ||
         !aligned16(dq) || !aligned16(dk) || !aligned16(dv) || !aligned16(workspace))
         return BPT_ERR_UNSUPPORTED;
-    const int64_t need = bpt_workspace_bytes(BPT_OP_ATTN_BWD, plan_in, plan_out, h, d, dtype);
+    const int64_t need = bpt_workspace_bytes(bias ? BPT_OP_ATTN_BWD : BPT_OP_ATTN_BWD_PLAIN, plan_in, plan_out, h, d, dtype);
     if (need > 0 && (!workspace || workspace_bytes < need)) return BPT_ERR_WORKSPACE;
     hipStream_t s = (hipStream_t)stream;
 #define X(HH, DD) \

@@ -181,7 +181,7 @@ std::optional<Three> attention_backward_known(const Tensor &row, const Tensor &i
     if (!e) return std::nullopt;
     c10::DeviceGuard guard(q.device());
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v);
-    Workspace ws(BPT_OP_ATTN_BWD, &e->a, &e->b, s.h, s.d, s.dt, q);
+    Workspace ws(BPT_OP_ATTN_BWD_PLAIN, &e->a, &e->b, s.h, s.d, s.dt, q);
     const int st = bpt_attention_backward(&e->a, &e->b, q.data_ptr(), k.data_ptr(), v.data_ptr(), nullptr, o.data_ptr(), d_o.data_ptr(),
                                           (const float *)lse.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), nullptr, ws.ptr, ws.bytes,
                                           (float)scale, (float)p, seed, s.h, s.d, s.dt, stream_of(q.device()));

@@ -58,6 +58,7 @@ def _replace_setting(**kw):
 
 _DTYPE = {torch.float32: 0, torch.float64: 1, torch.bfloat16: 2}
 OP_MASKEDMM_BWD, OP_NME_BWD, OP_SPMM_FWD, OP_SPMM_BWD, OP_ATTN_FWD, OP_ATTN_BWD, OP_SOFTMAX_FWD, OP_SOFTMAX_BWD = 1, 2, 3, 4, 5, 6, 7, 8
+OP_ATTN_BWD_PLAIN = 9        # OP_ATTN_BWD without a score term, on rows of 64 columns as they are
 
 
 def _check_input(t, name):
@@ -171,7 +172,7 @@ def _workspace(op, plan, plan_t, h, d, dt, device, plan_ref=None, plan_t_ref=Non
 # from the capture's own pool as before.  release_workspaces() gives the memory back.
 # Fused attention without a score term keeps none: from its second call on a graph it is served by the native host path, which
 # asks the allocator (the same block comes back call after call), and what the first call had left here would lie idle beside it
-# (422 MB at L = 32768, k = 8, 16 heads).
+# (422 MB at L = 32768, k = 8, 16 heads in float32).
 _SCRATCH = {}
 _SCRATCH_LOCK = threading.Lock()
 KEEP_WORKSPACES = True
@@ -729,7 +730,8 @@ def attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, in
     in_ref, out_ref = ctypes.byref(in_struct), ctypes.byref(out_struct)
     if bias_by_pair and not (tiles and bias is not None):
         raise RuntimeError("bias_by_pair: this call does not run on the tile kernels (ask attention_pair_rows() first)")
-    ws, nws = _workspace(OP_ATTN_BWD, plan_in, plan_out, h, d, dt, q.device, plan_ref=in_ref, plan_t_ref=out_ref, keep=bias is not None)
+    ws, nws = _workspace(OP_ATTN_BWD_PLAIN if bias is None else OP_ATTN_BWD, plan_in, plan_out, h, d, dt, q.device, plan_ref=in_ref,
+                         plan_t_ref=out_ref, keep=bias is not None)
     with _on_device_of(q):
         check_attn(_LIB.bpt_attention_backward(in_ref, out_ref, _ptr(q), _ptr(k), _ptr(v), _ptr(bias), _ptr(o), _ptr(do),
                                                _ptr(lse), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(ds), _ptr(ws), nws,

@@ -102,10 +102,12 @@ int64_t bpt_plan_struct_bytes(void);
 
 const char *bpt_strerror(int status);
 
-/* Bytes of workspace the call needs (0 possible).  op: one of the BPT_OP_* below. */
+/* Bytes of workspace the call needs (0 possible).  op: one of the BPT_OP_* below.  BPT_OP_ATTN_BWD covers every form of the fused
+ * backward; BPT_OP_ATTN_BWD_PLAIN is bpt_attention_backward without a score term, which needs no more and in bfloat16 much less. */
 enum {
     BPT_OP_MASKEDMM_BWD = 1, BPT_OP_NODE_MUL_EDGE_BWD = 2, BPT_OP_SPMM_FWD = 3, BPT_OP_SPMM_BWD = 4,
-    BPT_OP_ATTN_FWD = 5, BPT_OP_ATTN_BWD = 6, BPT_OP_SOFTMAX_FWD = 7, BPT_OP_SOFTMAX_BWD = 8
+    BPT_OP_ATTN_FWD = 5, BPT_OP_ATTN_BWD = 6, BPT_OP_SOFTMAX_FWD = 7, BPT_OP_SOFTMAX_BWD = 8,
+    BPT_OP_ATTN_BWD_PLAIN = 9
 };
 int64_t bpt_workspace_bytes(int op, const bpt_plan *plan, const bpt_plan *plan_t, int h, int d, int dtype);
 

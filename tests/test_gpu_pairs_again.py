@@ -54,3 +54,33 @@ def test_pairs_formed_again_match_the_oracle(name, heads, dropout):
     for got, want, what in ((qd.grad, rdq, "dq"), (kd.grad, rdk, "dk"), (vd.grad, rdv, "dv")):
         # a row of dk or dv sums up to `n` rounded terms: the absolute part grows with the square root of their number
         check(got, want, dict(rtol=2e-2, atol=2e-2 * max(1.0, (len(src) / 16) ** 0.5)), what)
+
+
+@pytest.mark.parametrize("dropout", [0.0, 0.25])
+@pytest.mark.parametrize("rel", [False, True], ids=["plain", "rel"])
+@pytest.mark.parametrize("name", ["sparse", "17", "300"])
+def test_the_backward_stays_inside_its_workspace(name, rel, dropout, monkeypatch):
+    """The workspace holds (lse, delta) of the rows without a score term and (p, ds) of the pairs with one, and the split rows' sums."""
+    from bpt_amd import graphbuilder as gb
+    from bpt_amd import graphop, op
+    from bpt_amd.plan import plan_cache
+    src, dst, n_k, n_q = graph(name)
+    out_csr, in_csr, ROW, IR, COL, IC = gb.get_csrs_bipartite(src, dst, n_k, n_q)
+    args = tuple(x.to(DEV) for x in (ROW, IR, out_csr[2], out_csr[1], COL, IC, in_csr[2], in_csr[1]))
+    q, k, v = (torch.randn(n, 8, 64, device=DEV).to(torch.bfloat16).requires_grad_(True) for n in (n_q, n_k, n_k))
+    real, behind = graphop._workspace, []
+
+    def with_a_mark_behind(*a, **kw):
+        n = real(*a, **kw)[1]
+        buf = torch.full((n + 65536,), 0x5A, dtype=torch.uint8, device=DEV)
+        behind.append(buf[n:])
+        return (buf, n) if n else (None, 0)
+
+    monkeypatch.setattr(graphop, "_workspace", with_a_mark_behind)
+    plan_cache.clear()
+    rel_kw = dict(rel_table=torch.randn(5, 64, device=DEV).to(torch.bfloat16), etype=torch.arange(len(src), device=DEV) % 5) if rel else {}
+    with forced_tiles(64):
+        o = op.bpt_attention(*args, q, k, v, fused=True, dropout_p=dropout, seed=77, **rel_kw)
+        o.backward(torch.randn_like(o))
+    torch.cuda.synchronize()
+    assert len(behind) >= 2 and all(bool((x == 0x5A).all()) for x in behind)

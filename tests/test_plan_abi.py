@@ -101,6 +101,27 @@ def test_error_strings_and_argument_errors_without_gpu():
     assert plib.bpt_graph_fill_device(2, 8, 1, 4, 5, 0, None, 0, None, None, None, None) == -2                # c > stride
 
 
+@pytest.mark.parametrize("n_rows,n_edges", [(65535, 3290000), (900, 40)])
+def test_workspace_of_the_bf16_tile_backward_is_sized_by_the_path_that_runs(n_rows, n_edges):
+    """Without a score term the two kernels hand each other (lse, delta) of the rows, 8 bytes a row and head; with one, or on heads of
+    fewer than 64 columns, (p, ds) of the pairs, 4 bytes a pair and head.  Partial rows of split rows come on top."""
+    lib, h, slots = _lib.attn_lib(), 16, 48
+    here = ctypes.create_string_buffer(16)                       # (stands for device memory: the sizes only are looked at)
+    st = _lib.PlanStruct()
+    st.n_rows = st.n_index_nodes = n_rows
+    st.n_edges, st.n_items, st.n_heavy, st.n_slots = n_edges, n_rows + 24, 24, slots
+    st.n_groups, st.grp_R, st.grp_max_chunk, st.n_grp_entries = n_rows // 16 + 1, 16, n_rows // 16 + 1, n_edges
+    for name in ("grp_members", "grp_ptr", "grp_entries", "grp_pairs", "grp_chunks", "grp_eids"):
+        setattr(st, name, ctypes.addressof(here))
+    size = lambda op, dtype: lib.bpt_workspace_bytes(op, ctypes.byref(st), ctypes.byref(st), h, 64, dtype)
+    partial, rows, pairs = 3 * slots * h * 64 * 4, n_rows * h * 8, n_edges * h * 4
+    assert size(9, 2) == rows + partial
+    assert size(6, 2) == max(rows, pairs) + partial
+    assert size(9, 0) == size(6, 0) == 2 * pairs + partial
+    st.grp_eids = None                                           # (a call with dropout then needs the pairs)
+    assert size(9, 2) == max(rows, pairs) + partial
+
+
 def _bpt_csr(L, triu, step):
     g = gb.BinaryPartition(L, triu, step, 10)
     src, dst, _ = g.get_edges()
