@@ -196,7 +196,8 @@ __global__ __launch_bounds__(BLOCK) void k_spmm_generic(bpt_plan P, const T *__r
 // twice with one value.  No other head's memory is touched, so what stands there does not matter.
 // Against copies padded to 64 columns and 4, 8 or 16 heads (three pads, the output and its gradient, three slices, and the
 // padding heads computed with the rest): 33 765 nodes / 576 k edges at 6 x 50 with dropout, forward and backward,
-// 508 -> 207 us; of that copies 223, the rest two padding heads of eight.
+// 508 -> 266 us, of which 60 are plain copies of q, k, v and o for the backward (bptop.cpp, own_rows); of the 508 copies were
+// 223, the rest two padding heads of eight.
 struct Narrow {
     int d, heads;              // columns of a head, heads
     int h;                     // heads the layer is padded to where that shows: dropout keys, lse and workspace rows

@@ -314,6 +314,14 @@ Tensor rows(const Tensor &x) {
     return y.is_cuda() && (reinterpret_cast<uintptr_t>(y.data_ptr()) & 3) ? y.clone() : y;
 }
 
+// The same in memory that is nobody else's.  A backward needs the rows as the forward saw them, and a layer on padded copies let
+// its caller write to q, k, v and o after the forward (an activation or a residual in place); so does this one.  The four copies
+// take 60 of 266 us at 33 765 nodes, 6 x 50 float32 with dropout, forward and backward.
+Tensor own_rows(const Tensor &x) {
+    Tensor y = rows(x);
+    return y.is_alias_of(x) ? y.clone() : y;
+}
+
 // The forward is a call of graphop.attention_forward, as that of the padded copies was: q, k, v stand for the padded shape there.
 std::tuple<Tensor, Tensor> narrow_forward(const Tensor &col, const Tensor &indptr, const Tensor &eid, const Tensor &indices, const Tensor &q,
                                           const Tensor &k, const Tensor &v, int64_t h, double scale, double p, int64_t seed) {
@@ -337,11 +345,11 @@ struct NarrowAttention : torch::autograd::Function<NarrowAttention> {
     static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r,
                           const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c,
                           const Tensor &q, const Tensor &k, const Tensor &v, int64_t h, double scale, double p, int64_t seed) {
-        const Tensor qc = rows(q), kc = rows(k), vc = rows(v);
+        const Tensor qc = own_rows(q), kc = own_rows(k), vc = own_rows(v);
         if (!narrow_known(col, indptr_c, eid_c, indices_c, qc, kc, h, p))
             python("prepare_training")(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, qc, kc, p, h);
         const auto [o, lse] = narrow_forward(col, indptr_c, eid_c, indices_c, qc, kc, vc, h, scale, p, seed);
-        ctx->save_for_backward({row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, qc, kc, vc, o, lse});
+        ctx->save_for_backward({row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, qc, kc, vc, o.clone(), lse});
         ctx->saved_data["h"] = h;
         ctx->saved_data["scale"] = scale;
         ctx->saved_data["p"] = p;

@@ -162,3 +162,24 @@ def test_a_mask_column_of_minus_infinity(dtype, h, d, p, monkeypatch):
         for got, want, name in zip(both[0], both[1], ("o", "dq", "dk", "dv")):
             assert torch.equal(got.isfinite(), want.isfinite()) and torch.equal(got.isnan(), want.isnan()), name
             close(got.nan_to_num(), f64(want.nan_to_num()), TOL[dtype] if name == "o" else GTOL[dtype], name)
+
+
+@pytest.mark.parametrize("tiles", [True, False], ids=["tiles", "by-size"])
+@pytest.mark.parametrize("dtype,h,d", [(torch.float32, 6, 50), (torch.float32, 3, 5), (torch.bfloat16, 6, 50), (torch.bfloat16, 3, 64)],
+                         ids=lambda x: str(x).replace("torch.", ""))
+def test_rows_and_result_may_be_written_to_after_the_forward(dtype, h, d, tiles, monkeypatch):
+    """As on padded copies: the gradients are those of the values that the forward saw."""
+    from bpt_amd import graphop, op
+    if tiles:
+        monkeypatch.setattr(graphop, "_MIN_GROUP_ITEMS", 0)
+    c = case("bpt512_k4")
+    leaves = [rand((c.n, h, d), dtype, s, 1.0 / 8).to(DEV).requires_grad_(True) for s in (21, 22, 23)]
+    do = rand((c.n, h, d), dtype, 24, 1.0 / 8).to(DEV)
+    want = torch.autograd.grad(op.bpt_attention(*c.out, *c.inn, *leaves), leaves, 2 * do)
+    q, k, v = (x * 1 for x in leaves)
+    o = op.bpt_attention(*c.out, *c.inn, q, k, v)
+    for x in (q, k, v):
+        x.add_(1.0)
+    o.mul_(2.0)
+    for got, ref in zip(torch.autograd.grad(o, leaves, do), want):
+        assert torch.equal(got, ref)
