@@ -307,7 +307,7 @@ def merge_graphs(graphs):
     return cat(src), cat(dst), cat(et), cat(pos), v_shift
 
 
-_DEVICE_EDGES = {}           # (_edges_key of the graph, device) -> (src, dst, etype, pos) device tensors and their part record
+_DEVICE_EDGES = {}           # (_edges_key of the graph, device) -> (src, dst, etype, pos) device tensors, nodes, _addresses
 _DEVICE_EDGES_MAX = 4096
 
 
@@ -317,6 +317,27 @@ def _edges_key(g):
     if type(g) in (BinaryPartition, FullyConnected, OpenAISparse):
         return type(g), g._length, g._triu, g._a, g._b
     return (type(g), *g.__reduce__()[1])
+
+
+def _addresses(tensors, n_nodes, device):
+    """What bpt_build_merge_device is told of a graph: the addresses of its lists, its edges and nodes.  None where that would
+    not describe them (a class of the caller's with lists of another type, layout, length or device)."""
+    if device.type != "cuda" or any(str(t.dtype) != "torch.int64" or t.dim() != 1 or not t.is_contiguous() or t.device != device for t in tensors):
+        return None
+    n_edges = tensors[0].numel()
+    if tensors[1].numel() != n_edges or tensors[2].numel() != n_edges or tensors[3].numel() != n_nodes:
+        return None
+    return tuple(t.data_ptr() for t in tensors) + (n_edges, n_nodes)
+
+
+def _concatenated(lists, nodes, device):
+    """merge_graphs_device by torch's concatenations, for lists that have no _addresses."""
+    import torch
+    counts = torch.tensor([tensors[0].numel() for tensors in lists], dtype=torch.int64)
+    shifts = torch.from_numpy(np.cumsum([0] + nodes[:-1], dtype=np.int64))
+    shift = torch.repeat_interleave(shifts.to(device), counts.to(device), output_size=int(counts.sum()))
+    src, dst, etype, pos = (torch.cat(ts) for ts in zip(*lists))
+    return src + shift, dst + shift, etype, pos, sum(nodes)
 
 
 def merge_graphs_device(graphs, device):
@@ -329,24 +350,25 @@ def merge_graphs_device(graphs, device):
     device = torch.device(device)
     if device.type == "cuda" and device.index is None:
         device = torch.device("cuda", torch.cuda.current_device())
-    parts, lists, n_edges, n_nodes = [], [], 0, 0
+    hits = []                                             # (kept until the launch: the cache may drop them meanwhile)
     for g in graphs:
         key = (_edges_key(g), device)
         hit = _DEVICE_EDGES.get(key)
         if hit is None:
             if len(_DEVICE_EDGES) >= _DEVICE_EDGES_MAX:
                 _DEVICE_EDGES.clear()
-            tensors = (*g.get_edges_device(device), torch.from_numpy(g.get_pos()).to(device))
-            hit = _DEVICE_EDGES[key] = (tensors, tuple(t.data_ptr() for t in tensors) + (tensors[0].numel(), tensors[3].numel()))
-        lists.append(hit[0])                              # (kept until the launch: the cache may drop them meanwhile)
-        parts += hit[1]
-        n_edges += hit[1][4]
-        n_nodes += hit[1][5]
+            tensors, nodes = (*g.get_edges_device(device), torch.from_numpy(g.get_pos()).to(device)), g.number_of_nodes
+            hit = _DEVICE_EDGES[key] = (tensors, nodes, _addresses(tensors, nodes, device))
+        hits.append(hit)
+    if any(hit[2] is None for hit in hits):
+        return _concatenated([hit[0] for hit in hits], [hit[1] for hit in hits], device)
+    parts = [x for hit in hits for x in hit[2]]
+    n_edges, n_nodes = sum(parts[4::6]), sum(parts[5::6])
     src, dst, etype = (torch.empty(n_edges, dtype=torch.int64, device=device) for _ in range(3))
     pos = torch.empty(n_nodes, dtype=torch.int64, device=device)
     if parts:
         with torch.cuda.device(device):
-            st = plan_lib().bpt_build_merge_device((ctypes.c_int64 * len(parts))(*parts), len(lists), src.data_ptr(), dst.data_ptr(),
+            st = plan_lib().bpt_build_merge_device((ctypes.c_int64 * len(parts))(*parts), len(hits), src.data_ptr(), dst.data_ptr(),
                                                    etype.data_ptr(), pos.data_ptr(), torch.cuda.current_stream().cuda_stream)
         if st != 0:
             raise RuntimeError(f"bpt_build_merge_device: status {st}")

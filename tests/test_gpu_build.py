@@ -121,6 +121,34 @@ def test_merge_keeps_graphs_apart_that_a_subclass_tells_apart():
     assert src[-3:].tolist() == [3 * n, 3 * n + 1, 3 * n + 2] and dst[-1].item() == 3 * n + 3
 
 
+@pytest.mark.parametrize("dtype,step,more", [(torch.int32, 1, 0), (torch.int64, 2, 0), (torch.int64, 1, 3)])
+def test_merge_with_lists_that_the_launch_cannot_read(dtype, step, more):
+    """A class of the caller's with 32-bit lists, strided views or positions of another length, beside an ordinary graph."""
+    from bpt_amd import graphbuilder as gb
+
+    class Chain:
+        number_of_nodes = 5
+
+        def __reduce__(self):
+            return Chain, (dtype, step, more)
+
+        def get_edges_device(self, device):
+            i = torch.arange(4, device=device).repeat_interleave(step).to(dtype)[::step]
+            return i, i + 1, i
+
+        def get_pos(self):
+            return np.arange(5 + more)
+
+    plain = gb.BinaryPartition(30, True, 4, 10)
+    n, (src, dst, etype), pos = plain.number_of_nodes, plain.get_edges(), plain.get_pos()
+    got = gb.merge_graphs_device([Chain(), plain, Chain()], DEV)
+    i = np.arange(4)
+    want = ([i, src + 5, i + 5 + n], [i + 1, dst + 5, i + 6 + n], [i, etype, i], [np.arange(5 + more), pos, np.arange(5 + more)])
+    assert got[4] == n + 10
+    for a, b in zip(got[:4], want):
+        assert a.dtype == torch.int64 and np.array_equal(a.cpu().numpy(), np.concatenate(b))
+
+
 @pytest.mark.parametrize("n_src,n_dst,E,seg,orders", [(300, 300, 6000, 64, (None, 0)), (40, 900, 5000, 64, (6, 6)), (900, 40, 5000, 128, (4, 2)),
                                                       (1, 1, 1, 64, (None, 0)), (5000, 64, 70000, 64, (None, 0))])
 def test_both_sides_built_together(n_src, n_dst, E, seg, orders):

@@ -208,3 +208,31 @@ def test_inter_graph_edges_follow_the_reference_construction():
     assert len(pairs) == len(s2) and all((b, a) in pairs for a, b in pairs)                  # two-way, no duplicates
     v0 = prem[0].number_of_nodes
     assert (0, v0) in pairs and (v0 + 2, 3) in pairs and (4, v0) not in pairs                  # node 4 is a span node
+
+
+@pytest.mark.parametrize("dtype,step,more", [("int64", 1, 0), ("int32", 1, 0), ("int64", 2, 0), ("int64", 1, 3)])
+def test_merge_of_lists_that_are_no_plain_int64_arrays(dtype, step, more):
+    """A class of the caller's may keep its lists in another type or as a strided view, and its positions may be of another length:
+    what would make their addresses and sizes say something else goes through concatenations (on the CPU all of it does)."""
+    torch = pytest.importorskip("torch")
+
+    class Chain:
+        def __init__(self, length):
+            self.number_of_nodes = length
+
+        def __reduce__(self):
+            return Chain, (self.number_of_nodes, dtype, step, more)
+
+        def get_edges_device(self, device):
+            i = torch.arange(step * (self.number_of_nodes - 1), dtype=getattr(torch, dtype), device=device)[::step]
+            return i // step, torch.div(i, step, rounding_mode="floor") + 1, i
+
+        def get_pos(self):
+            return np.arange(self.number_of_nodes + more)
+
+    src, dst, etype, pos, n = gb.merge_graphs_device([Chain(4), Chain(7), Chain(1)], "cpu")
+    assert n == 12 and src.dtype == dst.dtype == torch.int64
+    assert src.tolist() == [0, 1, 2] + list(range(4, 10)) and dst.tolist() == [1, 2, 3] + list(range(5, 11))
+    assert etype.tolist() == [step * i for i in [0, 1, 2, 0, 1, 2, 3, 4, 5]]
+    assert pos.tolist() == [i for k in (4, 7, 1) for i in range(k + more)]
+    assert gb._addresses((src, dst, etype, pos), n, torch.device("cpu")) is None
