@@ -183,3 +183,36 @@ def test_rows_and_result_may_be_written_to_after_the_forward(dtype, h, d, tiles,
     o.mul_(2.0)
     for got, ref in zip(torch.autograd.grad(o, leaves, do), want):
         assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("dtype,h,d", [(torch.float32, 6, 50), (torch.bfloat16, 8, 40)], ids=lambda x: str(x).replace("torch.", ""))
+def test_graph_replay_of_a_training_step_equals_eager(dtype, h, d):
+    """A captured forward and backward holds the copies of the rows and of the result, too: replayed on new values, with eager work in
+    between, it gives the eager step's bits."""
+    from bpt_amd import graphop, op
+    c = case("bpt512_k4")
+    q, k, v, do = (rand((c.n, h, d), dtype, s, 1.0 / 8).to(DEV) for s in (31, 32, 33, 34))
+    assert graphop.attention_reads_narrow(c.inn[0], c.inn[2], q, k, graphop.attention_padded_shape(q)[0], 0.1)
+
+    def step():
+        x = [t.detach().requires_grad_(True) for t in (q, k, v)]
+        o = op.bpt_attention(*c.out, *c.inn, *x, dropout_p=0.1, seed=5)
+        return (o.detach(), *torch.autograd.grad(o, x, do))
+
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):                              # plans are built and cached before the capture
+        for _ in range(2):
+            step()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step()
+    for rep in range(4):
+        for t in (q, k, v, do):
+            t.mul_(-0.5).add_(0.01 * rep)
+        want = step()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for got, ref, name in zip(captured, want, ("o", "dq", "dk", "dv")):
+            assert torch.equal(got, ref), f"replay {rep}: {name}"
