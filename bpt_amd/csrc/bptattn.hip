@@ -1708,16 +1708,18 @@ __device__ __forceinline__ int lane_bcast(int x, int src_lane) { return __builti
 // Common start of the tile kernels.  HW heads (= wavefronts) per workgroup: workgroup b handles head slice
 // (b / 8) % (H / HW) of group (b / 8) / (H / HW) of XCD b % 8's range.
 struct TileCtx {
-    int lane, wv, c, g, head, p_begin, p_end;
+    int lane, wv, c, g, head, p_begin, p_end, part;
     int2 member;                 // (row, slot) of member c
     uint32_t offa, offv;         // byte offsets of this lane inside a node row: its 16-column slice of the head (operands of the
                                  // products that contract over columns, + 64 t bytes per step), and its columns 4 c .. 4 c + 3
 };
 
-template <typename T, int H, int D, int HW, bool NARROW = false>
+template <typename T, int H, int D, int HW, bool NARROW = false, int SP = 1>
 __device__ __forceinline__ bool tile_begin(const bpt_plan &P, TileCtx &t, const Narrow &nw) {
-    static_assert(D == 64 && H % HW == 0 && (sizeof(T) == 4 || sizeof(T) == 2), "64 columns per head: one 16-column slice per lane group");
-    const int HS = NARROW ? nw.slices : H / HW;
+    static_assert(D == 64 && (H * SP) % HW == 0 && HW % SP == 0 && (sizeof(T) == 4 || sizeof(T) == 2), "64 columns per head: one 16-column slice per lane group");
+    static_assert(!NARROW || SP == 1 || SP == HW, "heads a workgroup has past the last one leave its barrier alone");
+    constexpr int HEADS = HW / SP;
+    const int HS = NARROW ? nw.slices : H / HEADS;
     t.lane = threadIdx.x & (WAVE - 1);
     t.wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     t.c = t.lane & 15;
@@ -1728,7 +1730,13 @@ __device__ __forceinline__ bool tile_begin(const bpt_plan &P, TileCtx &t, const 
     t.member = reinterpret_cast<const int2 *>(P.grp_members)[(size_t)grp * TILE_R + t.c];
     t.p_begin = __builtin_amdgcn_readfirstlane(P.grp_ptr[grp]);
     t.p_end = __builtin_amdgcn_readfirstlane(P.grp_ptr[grp + 1]);
-    t.head = (int)((blockIdx.x >> 3) % HS) * HW + t.wv;
+    t.part = SP > 1 ? t.wv / HEADS : 0;
+    if constexpr (SP > 1) {
+        const int per = ((t.p_end - t.p_begin + TILE_R * SP - 1) / (TILE_R * SP)) * TILE_R;
+        t.p_begin = min(t.p_begin + t.part * per, t.p_end);
+        t.p_end = min(t.p_begin + per, t.p_end);
+    }
+    t.head = (int)((blockIdx.x >> 3) % HS) * HEADS + (SP > 1 ? t.wv % HEADS : t.wv);
     if (NARROW) {
         if (t.head >= nw.heads) return false;
         t.offa = (uint32_t)(t.head * nw.d * sizeof(T));
@@ -1775,18 +1783,22 @@ __device__ __forceinline__ int tile_pair_number(int first, int mask, int c) { re
 
 // this lane's 16 columns of a node row (bytes offa + 64 t), as the A or B operand of a product over columns
 template <bool NARROW>
+__device__ __forceinline__ floatx4v tile_load4(const char *row, int t, int g, const Narrow &nw) {      // the four of step t
+    if constexpr (NARROW) {
+        const int quad = 4 * (4 * t + g), col = min(quad, nw.d - 4);
+        const floatx4u x = *reinterpret_cast<const floatx4u *>(row + 4 * col);
+        return floatx4v{col >= quad ? x[0] : 0.f, col + 1 >= quad ? x[1] : 0.f, col + 2 >= quad ? x[2] : 0.f, col + 3 >= quad ? x[3] : 0.f};
+    } else {
+        return *reinterpret_cast<const floatx4v *>(row + 64 * t);
+    }
+}
+template <bool NARROW>
 __device__ __forceinline__ void tile_load16(const char *row, float (&out)[16], int g, const Narrow &nw) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-        if constexpr (NARROW) {
-            const int quad = 4 * (4 * t + g), col = min(quad, nw.d - 4);
-            const floatx4u x = *reinterpret_cast<const floatx4u *>(row + 4 * col);
+        const floatx4v x = tile_load4<NARROW>(row, t, g, nw);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) out[4 * t + e] = col + e >= quad ? x[e] : 0.f;
-        } else {
-            const float4 x = *reinterpret_cast<const float4 *>(row + 64 * t);
-            out[4 * t] = x.x; out[4 * t + 1] = x.y; out[4 * t + 2] = x.z; out[4 * t + 3] = x.w;
-        }
+        for (int e = 0; e < 4; ++e) out[4 * t + e] = x[e];
     }
 }
 // this lane's four columns of an entry's row
@@ -1838,33 +1850,107 @@ __device__ __forceinline__ void tile_axpy_upto(const float (&w)[4], const float4
 // L = 512 level.  The same on the stores of (p, ds), which the source side reads soon, or on its loads of them: 47 -> 50.5 and
 // 47 -> 55 us for the source side of L = 8192; on the loads of the members' rows: destination side 58 -> 61.6.
 template <int H, int D, bool SCALE, bool NARROW, typename T>
+__device__ __forceinline__ void tile_store_row(const TileCtx &t, int r, float4 x, float inv_c, T *__restrict__ out, float *__restrict__ ws,
+                                               const Narrow &nw) {
+    const int m = 4 * t.g + r;                                    // the member whose row this lane stores a piece of
+    const int row = lane_bcast(t.member.x, m), slot = lane_bcast(t.member.y, m);
+    const float inv = SCALE ? lane_bcast(inv_c, m) : 1.f;
+    if (row < 0 || (NARROW && 4 * t.c >= nw.d)) return;
+    const int col = NARROW ? narrow_col(nw, t.c) : 4 * t.c;
+    if (slot < 0) {
+        if (SCALE) { x.x *= inv; x.y *= inv; x.z *= inv; x.w *= inv; }
+        T *const at = NARROW ? out + (size_t)row * (uint32_t)(nw.heads * nw.d) + t.head * nw.d + col : out + (size_t)row * (H * D) + t.head * D + col;
+        if constexpr (sizeof(T) == 4) {
+            if constexpr (NARROW) *reinterpret_cast<floatx4u *>(at) = floatx4u{x.x, x.y, x.z, x.w};
+            else __builtin_nontemporal_store(floatx4v{x.x, x.y, x.z, x.w}, reinterpret_cast<floatx4v *>(at));
+        } else {
+            const uint2 y = make_uint2(((uint32_t)f32_to_bf16(x.x)) | ((uint32_t)f32_to_bf16(x.y) << 16),
+                           ((uint32_t)f32_to_bf16(x.z)) | ((uint32_t)f32_to_bf16(x.w) << 16));
+            if constexpr (NARROW) *reinterpret_cast<uintx2u *>(at) = uintx2u{y.x, y.y};
+            else __builtin_nontemporal_store(uintx2v{y.x, y.y}, reinterpret_cast<uintx2v *>(at));
+        }
+    } else {
+        float *const at = ws + (size_t)slot * (NARROW ? nw.h * D : H * D) + t.head * D + col;
+        if constexpr (NARROW) *reinterpret_cast<floatx4u *>(at) = floatx4u{x.x, x.y, x.z, x.w};
+        else *reinterpret_cast<float4 *>(at) = x;
+    }
+}
+template <int H, int D, bool SCALE, bool NARROW, typename T>
 __device__ __forceinline__ void tile_store_rows(const TileCtx &t, const floatx4v (&acc)[4], float inv_c, T *__restrict__ out,
                                                 float *__restrict__ ws, const Narrow &nw) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int m = 4 * t.g + r;                                // the member whose row this lane stores a piece of
-        const int row = lane_bcast(t.member.x, m), slot = lane_bcast(t.member.y, m);
-        const float inv = SCALE ? lane_bcast(inv_c, m) : 1.f;
-        if (row < 0 || (NARROW && 4 * t.c >= nw.d)) continue;
-        float4 x = make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]);
-        const int col = NARROW ? narrow_col(nw, t.c) : 4 * t.c;
-        if (slot < 0) {
-            if (SCALE) { x.x *= inv; x.y *= inv; x.z *= inv; x.w *= inv; }
-            T *const at = NARROW ? out + (size_t)row * (uint32_t)(nw.heads * nw.d) + t.head * nw.d + col : out + (size_t)row * (H * D) + t.head * D + col;
-            if constexpr (sizeof(T) == 4) {
-                if constexpr (NARROW) *reinterpret_cast<floatx4u *>(at) = floatx4u{x.x, x.y, x.z, x.w};
-                else __builtin_nontemporal_store(floatx4v{x.x, x.y, x.z, x.w}, reinterpret_cast<floatx4v *>(at));
-            } else {
-                const uint2 y = make_uint2(((uint32_t)f32_to_bf16(x.x)) | ((uint32_t)f32_to_bf16(x.y) << 16),
-                               ((uint32_t)f32_to_bf16(x.z)) | ((uint32_t)f32_to_bf16(x.w) << 16));
-                if constexpr (NARROW) *reinterpret_cast<uintx2u *>(at) = uintx2u{y.x, y.y};
-                else __builtin_nontemporal_store(uintx2v{y.x, y.y}, reinterpret_cast<uintx2v *>(at));
-            }
+    for (int r = 0; r < 4; ++r)
+        tile_store_row<H, D, SCALE, NARROW>(t, r, make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]), inv_c, out, ws, nw);
+}
+
+// SP > 1: SP wavefronts of a workgroup share a tile and head, each walks a contiguous SP-th of the tile's blocks (tile_begin),
+// and what they have summed up meets in LDS: every wavefront leaves its accumulators in its own piece, [r][lane] so that
+// the 16-byte accesses of a wavefront are contiguous, and after one barrier adds up and stores the members 4 g + r of its
+// 4 / SP registers r.  Parts are added in their order: the same bits on every run.
+constexpr int TILE_PART_FLOATS = TILE_R * 64;                     // accumulators of a wavefront
+__device__ __forceinline__ void tile_park(float *part, const floatx4v (&acc)[4], int lane) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        *reinterpret_cast<floatx4v *>(part + (r * WAVE + lane) * 4) = floatx4v{acc[0][r], acc[1][r], acc[2][r], acc[3][r]};
+}
+// sum over the parts of register r, part s (`stride` floats after part s - 1) weighted with wgt[s] of the lane's member
+template <int SP, bool WEIGHTED>
+__device__ __forceinline__ float4 tile_meet(const float *part0, int stride, int r, const TileCtx &t, const float (&wgt)[SP]) {
+    float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int s = 0; s < SP; ++s) {
+        const floatx4v y = *reinterpret_cast<const floatx4v *>(part0 + s * stride + (r * WAVE + t.lane) * 4);
+        if constexpr (WEIGHTED) {
+            const float w = lane_bcast(wgt[s], 4 * t.g + r);
+            x.x = fmaf(w, y[0], x.x); x.y = fmaf(w, y[1], x.y); x.z = fmaf(w, y[2], x.z); x.w = fmaf(w, y[3], x.w);
         } else {
-            float *const at = ws + (size_t)slot * (NARROW ? nw.h * D : H * D) + t.head * D + col;
-            if constexpr (NARROW) *reinterpret_cast<floatx4u *>(at) = floatx4u{x.x, x.y, x.z, x.w};
-            else *reinterpret_cast<float4 *>(at) = x;
+            x.x += y[0]; x.y += y[1]; x.z += y[2]; x.w += y[3];
         }
+    }
+    return x;
+}
+// the same for a kernel without weights: parked accumulators of the SP parts -> result rows
+template <int SP, int H, int D, bool NARROW, typename T>
+__device__ __forceinline__ void tile_meet_and_store(const float *part0, int stride, const TileCtx &t, T *__restrict__ out, float *__restrict__ ws,
+                                                    const Narrow &nw) {
+    constexpr int RS = 4 / SP;
+    const float none[SP] = {};
+#pragma unroll
+    for (int i = 0; i < RS; ++i) {
+        const int r = t.part * RS + i;
+        tile_store_row<H, D, false, NARROW>(t, r, tile_meet<SP, false>(part0, stride, r, t, none), 1.f, out, ws, nw);
+    }
+}
+// ... and for the forward: with the parts' exponent references and denominators (left behind the accumulators by member)
+constexpr int TILE_PART_FWD_FLOATS = TILE_PART_FLOATS + 2 * TILE_R;
+template <int SP, int H, int D, bool NARROW, typename T>
+__device__ __forceinline__ void tile_meet_forward(float *mine, const float *part0, int stride, const TileCtx &t, const floatx4v (&acc)[4], float &mref,
+                                                  float &lt, T *__restrict__ out, float *__restrict__ ws, const Narrow &nw) {
+    constexpr int RS = 4 / SP;
+    tile_park(mine, acc, t.lane);
+    if (t.g == 0) {
+        mine[TILE_PART_FLOATS + 2 * t.c] = mref;
+        mine[TILE_PART_FLOATS + 2 * t.c + 1] = lt;
+    }
+    __syncthreads();
+    float wgt[SP], l = 0.f, M = M_INIT_LOG2;
+#pragma unroll
+    for (int s = 0; s < SP; ++s) {
+        wgt[s] = part0[s * stride + TILE_PART_FLOATS + 2 * t.c];
+        M = fmaxf(M, wgt[s]);
+    }
+#pragma unroll
+    for (int s = 0; s < SP; ++s) {
+        wgt[s] = __builtin_amdgcn_exp2f(wgt[s] - M);
+        l = fmaf(wgt[s], part0[s * stride + TILE_PART_FLOATS + 2 * t.c + 1], l);
+    }
+    mref = M;
+    lt = l;
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+    for (int i = 0; i < RS; ++i) {
+        const int r = t.part * RS + i;
+        tile_store_row<H, D, true, NARROW>(t, r, tile_meet<SP, true>(part0, stride, r, t, wgt), inv, out, ws, nw);
     }
 }
 
@@ -1912,36 +1998,21 @@ __device__ __forceinline__ void tile_rows_to_operand(float *kt, const float4 (&r
     wave_lds_fence();                                             // (read before the next block's rows are written)
 }
 
-// PIPE: the rows of the next block are loaded while one is used (two-stage register pipeline).  Pays on graphs with few,
-// tall tiles (a dense window graph: 9 blocks per tile, two wavefronts per SIMD in all), costs a wavefront per SIMD:
-// at L = 8192, k = 4 (1217 tiles of 4 blocks) the forward takes 47 us with it and 44 without.
-// Other forms measured there and dropped: groups of 32 rows (two member blocks per wavefront sharing the K / V
+// Block after block, a block's loads ahead of its products.  Forms measured at L = 8192, k = 4 (1217 tiles of 4 blocks) and
+// dropped: the rows of the next block loaded while one is used (a two-stage register pipeline: 47 us against 44, a wavefront
+// per SIMD fewer; on few, tall tiles it was the better form until the parts of a tile came to be walked side by side, see
+// tile_parts), groups of 32 rows (two member blocks per wavefront sharing the K / V
 // registers: a third fewer rows through the L1s, two or three wavefronts per SIMD, 56 us; two wavefronts per head in step
 // on the same entries, one member block each, so that the L1 fetches a row once: 60 us: the time follows the number
 // of 16 x 16 blocks, 4716 against 6324, not the bytes), five or six wavefronts per SIMD by spilling (53 / 85 us).
-template <bool PIPE, typename Blk, typename Issue, typename Compute>
+template <typename Blk, typename Issue, typename Compute>
 __device__ __forceinline__ void tile_walk(int nblk, Issue &&issue, Compute &&compute) {
-    if constexpr (PIPE) {
-        Blk A, B;
-        issue(A, 0);
-        for (int b = 0; b < nblk; b += 2) {
-            issue(B, min(b + 1, nblk - 1));                       // past the end: the last block again, not used
-            issue_loads_first();
-            compute(A);
-            issue_loads_first();
-            issue(A, min(b + 2, nblk - 1));
-            issue_loads_first();
-            if (b + 1 < nblk) compute(B);
-            issue_loads_first();
-        }
-    } else {
-        for (int b = 0; b < nblk; ++b) {
-            Blk A;
-            issue(A, b);
-            issue_loads_first();
-            compute(A);
-            issue_loads_first();
-        }
+    for (int b = 0; b < nblk; ++b) {
+        Blk A;
+        issue(A, b);
+        issue_loads_first();
+        compute(A);
+        issue_loads_first();
     }
 }
 
@@ -1983,20 +2054,20 @@ __device__ __forceinline__ void tile_walk_first_ahead(int nblk, IssueFirst &&fir
     issue_loads_first();
 }
 
-template <typename T, int H, int D, int HW, bool PIPE, bool DROP, int BIAS, bool NARROW = false>
-__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE ? 3 : 4))) void k_attn_fwd_tile(
+template <typename T, int H, int D, int HW, bool DROP, int BIAS, bool NARROW = false, int SP = 1>
+__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_attn_fwd_tile(
     bpt_plan P, const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v, T *__restrict__ o, float *__restrict__ lse,
     float *__restrict__ ws_acc, float *__restrict__ ws_ml, float scale_log2e, uint32_t drop_thr, uint32_t drop_seed, float drop_inv,
     const float *__restrict__ bias, Narrow nw) {
     const int Hs = NARROW ? nw.h : H;                             // heads as lse, workspace and dropout keys count them
     const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * sizeof(T) : (uint32_t)(H * D * sizeof(T));        // bytes of a node row
     TileCtx t;
-    if (!tile_begin<T, H, D, HW, NARROW>(P, t, nw)) return;
+    if (!tile_begin<T, H, D, HW, NARROW, SP>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     __shared__ int fst_lds[HW][BIAS == 2 ? TILE_CHUNK : 1];      // the entries' first pair numbers: where a term in pair order sits
     int2 *ent = ent_lds[t.wv];
     int *fst = BIAS == 2 ? fst_lds[t.wv] : nullptr;
-    __shared__ float kt_lds[HW][TILE_R * TILE_KT_STRIDE];
+    __shared__ __attribute__((aligned(16))) float kt_lds[HW][TILE_R * TILE_KT_STRIDE];
     float *kt = kt_lds[t.wv];
     TileEntryRegs er;
     if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
@@ -2008,7 +2079,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
     // for before the entry list is (one more round trip in front of the K rows).  They stay as they are and the scores are
     // scaled instead, so nothing has to happen to them between their arrival and the first product.
     const char *const qrow = reinterpret_cast<const char *>(q) + (size_t)max(t.member.x, 0) * RB + t.offa;
-    constexpr bool AHEAD = !PIPE && !DROP && BIAS == 0;         // (with dropout or the score term the sixteen registers are not there)
+    constexpr bool AHEAD = !DROP && BIAS == 0;         // (with dropout or the score term the sixteen registers are not there)
     if constexpr (!AHEAD) tile_load16<NARROW>(qrow, qb, g, nw);
     floatx4v acc[4];
 #pragma unroll
@@ -2087,13 +2158,19 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
             tile_axpy_upto(pr, B.vr, acc, B.nv);
         };
         auto issue = [&](Blk &B, int b) { issue_k(B, b); issue_rest(B, b); };
-        if constexpr (!AHEAD) tile_walk<PIPE, Blk>(nblk, issue, compute);
+        if constexpr (!AHEAD) tile_walk<Blk>(nblk, issue, compute);
         else tile_walk_first_ahead<Blk>(nblk, issue_k, issue_rest, compute, [&]() { if (p0 == t.p_begin) tile_load16<NARROW>(qrow, qb, g, nw); });
         wave_lds_fence();                                         // the piece is read to the end before the next one is staged
     }
     float lt = lrun + __shfl_xor(lrun, 16);
     lt += __shfl_xor(lt, 32);                                    // denominator of member c, in its four lanes
-    tile_store_rows<H, D, true, NARROW>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc, nw);
+    if constexpr (SP > 1) {
+        static_assert(TILE_PART_FWD_FLOATS <= TILE_R * TILE_KT_STRIDE, "a part fits its wavefront's piece");
+        tile_meet_forward<SP, H, D, NARROW>(kt, kt_lds[t.wv % (HW / SP)], (HW / SP) * TILE_R * TILE_KT_STRIDE, t, acc, mref, lt, o, ws_acc, nw);
+        if (t.part != 0) return;
+    } else {
+        tile_store_rows<H, D, true, NARROW>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc, nw);
+    }
     if (g == 0 && t.member.x >= 0) {                              // lanes 0 .. 15: one member each
         if (t.member.y < 0) {
             lse[(size_t)t.member.x * Hs + t.head] = lt > 0.f ? mref + log2f(lt) : 0.f;
@@ -2116,8 +2193,8 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
 // source side's layout instead (scattered 8-byte stores here, contiguous reads there) cost this kernel a third of its
 // time (126 against 85 us at L = 4096, k = 32); letting the source side recompute p and ds (two more products there,
 // delta (n, H) handed over) measured slower than either on every graph tried.
-template <typename T, int H, int D, int HW, bool PIPE, bool DROP, int BIAS, bool NARROW = false>
-__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE ? 2 : DROP || BIAS ? 3 : 4))) void k_attn_bwd_dst_tile(
+template <typename T, int H, int D, int HW, bool DROP, int BIAS, bool NARROW = false, int SP = 1>
+__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP || BIAS ? 3 : 4))) void k_attn_bwd_dst_tile(
     bpt_plan P, const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v, const T *__restrict__ o,
     const T *__restrict__ d_o, const float *__restrict__ lse, T *__restrict__ dq, float2 *__restrict__ pds, float *__restrict__ ws_dq,
     float scale, float scale_log2e, uint32_t drop_thr, uint32_t drop_seed, float drop_inv, const float *__restrict__ bias,
@@ -2125,12 +2202,12 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
     const int Hs = NARROW ? nw.h : H;
     const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * sizeof(T) : (uint32_t)(H * D * sizeof(T));
     TileCtx t;
-    if (!tile_begin<T, H, D, HW, NARROW>(P, t, nw)) return;
+    if (!tile_begin<T, H, D, HW, NARROW, SP>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     __shared__ int fst_lds[HW][TILE_CHUNK];
     int2 *ent = ent_lds[t.wv];
     int *fst = fst_lds[t.wv];
-    __shared__ float kt_lds[HW][TILE_R * TILE_KT_STRIDE];
+    __shared__ __attribute__((aligned(16))) float kt_lds[HW][TILE_R * TILE_KT_STRIDE];
     float *kt = kt_lds[t.wv];
     TileEntryRegs er;
     if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
@@ -2141,10 +2218,46 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
     float2 *const pds_h = pds + (size_t)t.head * (size_t)P.n_edges;     // this head's part of the scratch
     // the member's dO columns live in LDS (lane-major, read back before every product with them): with them in registers
     // the kernel needs 144 and a SIMD holds three wavefronts, without them 128 and four
-    __shared__ float4 dob_lds[HW][4][WAVE];
+    __shared__ floatx4v dob_lds[HW / SP][4][WAVE];
+    floatx4v(&dob_h)[4][WAVE] = dob_lds[t.wv % (HW / SP)];
     // (q stays as it is and the scores are scaled, as in the forward: the same roundings in both)
     float qb[16], delta, lse_c;
-    {
+    if constexpr (SP > 1) {
+        // each part reads its 4 / SP steps of the members' rows for all of them
+        __shared__ floatx4v q_lds[HW / SP][4][WAVE];
+        __shared__ float delta_lds[HW][TILE_R];
+        floatx4v(&q_h)[4][WAVE] = q_lds[t.wv % (HW / SP)];
+        constexpr int TS = 4 / SP;
+        floatx4v xq[TS], xd[TS], xo[TS];
+#pragma unroll
+        for (int i = 0; i < TS; ++i) {
+            const int at = t.part * TS + i;
+            xq[i] = tile_load4<NARROW>(reinterpret_cast<const char *>(q) + mrow, at, g, nw);
+            xd[i] = tile_load4<NARROW>(reinterpret_cast<const char *>(d_o) + mrow, at, g, nw);
+            xo[i] = tile_load4<NARROW>(reinterpret_cast<const char *>(o) + mrow, at, g, nw);
+        }
+        lse_c = lse[(size_t)max(t.member.x, 0) * Hs + t.head];
+        float part = 0.f;
+#pragma unroll
+        for (int i = 0; i < TS; ++i) {
+            q_h[t.part * TS + i][t.lane] = xq[i];
+            dob_h[t.part * TS + i][t.lane] = xd[i];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) part = fmaf(xd[i][e], xo[i][e], part);
+        }
+        part += __shfl_xor(part, 16);
+        part += __shfl_xor(part, 32);
+        if (g == 0) delta_lds[t.wv][c] = part;
+        __syncthreads();
+        delta = 0.f;
+#pragma unroll
+        for (int i = 0; i < SP; ++i) delta += delta_lds[i * (HW / SP) + t.wv % (HW / SP)][c];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const floatx4v x = q_h[i][t.lane];
+            qb[4 * i] = x[0]; qb[4 * i + 1] = x[1]; qb[4 * i + 2] = x[2]; qb[4 * i + 3] = x[3];
+        }
+    } else {
         float ob[16], dob[16];
         tile_load16<NARROW>(reinterpret_cast<const char *>(q) + mrow, qb, g, nw);
         tile_load16<NARROW>(reinterpret_cast<const char *>(d_o) + mrow, dob, g, nw);
@@ -2156,7 +2269,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
         delta = part + __shfl_xor(part, 32);                      // dO . O of member c, this head
         lse_c = lse[(size_t)max(t.member.x, 0) * Hs + t.head];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dob_lds[t.wv][i][t.lane] = make_float4(dob[4 * i], dob[4 * i + 1], dob[4 * i + 2], dob[4 * i + 3]);
+        for (int i = 0; i < 4; ++i) dob_h[i][t.lane] = floatx4v{dob[4 * i], dob[4 * i + 1], dob[4 * i + 2], dob[4 * i + 3]};
     }
     floatx4v acc[4];
 #pragma unroll
@@ -2206,8 +2319,8 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
             float dob[16];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float4 x = dob_lds[t.wv][i][t.lane];
-                dob[4 * i] = x.x; dob[4 * i + 1] = x.y; dob[4 * i + 2] = x.z; dob[4 * i + 3] = x.w;
+                const floatx4v x = dob_h[i][t.lane];
+                dob[4 * i] = x[0]; dob[4 * i + 1] = x[1]; dob[4 * i + 2] = x[2]; dob[4 * i + 3] = x[3];
             }
             const floatx4v dp = tile_dot(va, dob);
             float ds[4];
@@ -2227,10 +2340,16 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(PIPE 
             }
             tile_axpy_upto(ds, B.kc, acc, B.nv);
         };
-        tile_walk<PIPE, Blk>(nblk, issue, compute);
+        tile_walk<Blk>(nblk, issue, compute);
         wave_lds_fence();
     }
-    tile_store_rows<H, D, false, NARROW>(t, acc, 1.f, dq, ws_dq, nw);
+    if constexpr (SP > 1) {
+        tile_park(kt, acc, t.lane);
+        __syncthreads();
+        tile_meet_and_store<SP, H, D, NARROW>(kt_lds[t.wv % (HW / SP)], (HW / SP) * TILE_R * TILE_KT_STRIDE, t, dq, ws_dq, nw);
+    } else {
+        tile_store_rows<H, D, false, NARROW>(t, acc, 1.f, dq, ws_dq, nw);
+    }
 }
 
 // Backward on tiles, source side (groups of the out-CSR plan: members = source rows, entries = destinations):
@@ -2252,17 +2371,19 @@ __device__ __forceinline__ void tile_pair_positions(const bpt_plan &P, int entry
     const intx4u x = *reinterpret_cast<const intx4u *>(P.grp_pairs + (size_t)entry * TILE_R + 4 * g);
     pos[0] = x[0]; pos[1] = x[1]; pos[2] = x[2]; pos[3] = x[3];
 }
-template <typename T, int H, int D, int HW, bool NARROW = false>
+template <typename T, int H, int D, int HW, bool NARROW = false, int SP = 1>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_attn_bwd_src_tile(
     bpt_plan P, const T *__restrict__ q, const T *__restrict__ d_o, const float2 *__restrict__ pds, T *__restrict__ dk, T *__restrict__ dv,
     float *__restrict__ ws_dk, float *__restrict__ ws_dv, Narrow nw) {
     const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * sizeof(T) : (uint32_t)(H * D * sizeof(T));
     TileCtx t;
-    if (!tile_begin<T, H, D, HW, NARROW>(P, t, nw)) return;
-    __shared__ int2 ent_lds[HW][TILE_CHUNK];
-    int2 *ent = ent_lds[t.wv];
-    __shared__ __attribute__((aligned(16))) float2 wt_lds[HW][TILE_R * TILE_WT_STRIDE];
-    float2 *const wt = wt_lds[t.wv];
+    if (!tile_begin<T, H, D, HW, NARROW, SP>(P, t, nw)) return;
+    // a wavefront's piece: its entry list and its block of (p, ds), afterwards (SP > 1) what it has summed up
+    constexpr int ENT = TILE_CHUNK * 2, LIVE = ENT + TILE_R * TILE_WT_STRIDE * 2, PIECE = SP > 1 ? 2 * TILE_PART_FLOATS : LIVE;
+    static_assert(PIECE >= LIVE, "the lists fit");
+    __shared__ __attribute__((aligned(16))) float piece[HW][PIECE];
+    int2 *ent = reinterpret_cast<int2 *>(piece[t.wv]);
+    float2 *const wt = reinterpret_cast<float2 *>(piece[t.wv] + ENT);
     const int c = t.c, g = t.g;
     const char *qb = reinterpret_cast<const char *>(q), *db = reinterpret_cast<const char *>(d_o);
     const float2 *const pds_h = pds + (size_t)t.head * (size_t)P.n_edges;
@@ -2338,8 +2459,18 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
         }
         wave_lds_fence();
     }
-    tile_store_rows<H, D, false, NARROW>(t, ak, 1.f, dk, ws_dk, nw);
-    tile_store_rows<H, D, false, NARROW>(t, av, 1.f, dv, ws_dv, nw);
+    if constexpr (SP > 1) {
+        constexpr int NEXT = (HW / SP) * PIECE;
+        tile_park(piece[t.wv], ak, t.lane);
+        tile_park(piece[t.wv] + TILE_PART_FLOATS, av, t.lane);
+        __syncthreads();
+        const float *const part0 = piece[t.wv % (HW / SP)];
+        tile_meet_and_store<SP, H, D, NARROW>(part0, NEXT, t, dk, ws_dk, nw);
+        tile_meet_and_store<SP, H, D, NARROW>(part0 + TILE_PART_FLOATS, NEXT, t, dv, ws_dv, nw);
+    } else {
+        tile_store_rows<H, D, false, NARROW>(t, ak, 1.f, dk, ws_dk, nw);
+        tile_store_rows<H, D, false, NARROW>(t, av, 1.f, dv, ws_dv, nw);
+    }
 }
 
 // ---- Dense tiles for bfloat16 rows.  Same walk and the same lane roles as the float32 tile kernels above, on
@@ -2351,12 +2482,11 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
 //   operand of output columns {4 c + nb} takes element nb of each of the four, packed by byte permutes).
 // Probabilities and ds are rounded to bfloat16 where they enter a product (the softmax denominator is summed unrounded);
 // the scratch between the two backward kernels, where there is one, holds (p, ds) as two bfloat16 in 4 bytes, by head and destination-side pair number.
-// The two-stage register pipeline of tile_walk does not pay here: at six wavefronts per SIMD it spills (2.4 x slower),
+// A two-stage register pipeline does not pay here: at six wavefronts per SIMD it spills (2.4 x slower),
 // at four it measured 5 to 10 % slower on the sparse graphs and level on the window graph.  Tiles of 32 rows (two member
 // blocks per wavefront on the same loaded rows, three or four wavefronts per SIMD) did not pay either: the entry lists
 // shrink by a third on the destination side but only by an eighth on the source side (L = 8192, k = 4: 67 k -> 46 k and
 // 71 k -> 62 k entries), and the step went from 0.113 to 0.117 ms (32-graph batch 0.177 -> 0.205, window 128 level).
-constexpr bool TILE_BF16_PIPE = false;
 constexpr int TILE_BF16_WPE = 5, TILE_BF16_WPE_DST = 5, TILE_BF16_WPE_SRC = 5, TILE_BF16_WPE_AGAIN = 4;     // wavefronts per SIMD the bfloat16 tile kernels are compiled for
 typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
@@ -2444,7 +2574,8 @@ __device__ __forceinline__ void tile_rows_to_operand_bf16(char *kt, const uint2 
     wave_lds_fence();                                             // (read before the next block's rows are written)
 }
 
-template <int H, int D, int HW, int WPE, bool PIPE, bool DROP, int BIAS, bool NARROW = false>
+constexpr int TILE_KT_FLOATS_BF16 = TILE_R * TILE_KT_BYTES_BF16 / 4;
+template <int H, int D, int HW, int WPE, bool DROP, int BIAS, bool NARROW = false, int SP = 1>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))) void k_attn_fwd_tile_bf16(
     bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, bf16_t *__restrict__ o,
     float *__restrict__ lse, float *__restrict__ ws_acc, float *__restrict__ ws_ml, float scale_log2e, uint32_t drop_thr,
@@ -2452,13 +2583,15 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     const int Hs = NARROW ? nw.h : H;                             // heads as lse, workspace and dropout keys count them
     const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * 2 : (uint32_t)(H * D * 2);                       // bytes of a node row
     TileCtx t;
-    if (!tile_begin<bf16_t, H, D, HW, NARROW>(P, t, nw)) return;
+    if (!tile_begin<bf16_t, H, D, HW, NARROW, SP>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     __shared__ int fst_lds[HW][BIAS == 2 ? TILE_CHUNK : 1];      // the entries' first pair numbers: where a term in pair order sits
     int2 *ent = ent_lds[t.wv];
     int *fst = BIAS == 2 ? fst_lds[t.wv] : nullptr;
-    __shared__ __attribute__((aligned(16))) char kt_lds[HW][TILE_R * TILE_KT_BYTES_BF16];
-    char *kt = kt_lds[t.wv];
+    constexpr int PIECE = SP > 1 ? TILE_PART_FWD_FLOATS : TILE_KT_FLOATS_BF16;
+    static_assert(PIECE >= TILE_KT_FLOATS_BF16, "the rows fit");
+    __shared__ __attribute__((aligned(16))) float piece[HW][PIECE];
+    char *kt = reinterpret_cast<char *>(piece[t.wv]);
     TileEntryRegs er;
     if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
     issue_loads_first();
@@ -2545,13 +2678,18 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             tile_axpy_bf16(pa, B.vr, acc);
         };
         auto issue = [&](Blk &B, int b) { issue_k(B, b); issue_rest(B, b); };
-        if constexpr (PIPE || DROP || BIAS != 0) tile_walk<PIPE, Blk>(nblk, issue, compute);      // (the K rows ahead: eight registers more)
+        if constexpr (DROP || BIAS != 0) tile_walk<Blk>(nblk, issue, compute);      // (the K rows ahead: eight registers more)
         else tile_walk_first_ahead<Blk>(nblk, issue_k, issue_rest, compute, []() {});
         wave_lds_fence();
     }
     float lt = lrun + __shfl_xor(lrun, 16);
     lt += __shfl_xor(lt, 32);
-    tile_store_rows<H, D, true, NARROW>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc, nw);
+    if constexpr (SP > 1) {
+        tile_meet_forward<SP, H, D, NARROW>(piece[t.wv], piece[t.wv % (HW / SP)], (HW / SP) * PIECE, t, acc, mref, lt, o, ws_acc, nw);
+        if (t.part != 0) return;
+    } else {
+        tile_store_rows<H, D, true, NARROW>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc, nw);
+    }
     if (g == 0 && t.member.x >= 0) {
         if (t.member.y < 0) {
             lse[(size_t)t.member.x * Hs + t.head] = lt > 0.f ? mref + log2f(lt) : 0.f;
@@ -2565,7 +2703,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
 // Destination side.  PDS: (p, ds) of the pairs go to the scratch for the source side that reads them back; otherwise that side
 // forms them again (k_attn_bwd_src_tile_bf16_again) and all it is handed is (lse, delta) of the rows, `stat` (n, H): the
 // segments of a split row write the same values.
-template <int H, int D, int HW, int WPE, bool PIPE, bool DROP, int BIAS, bool PDS, bool NARROW = false>
+template <int H, int D, int HW, int WPE, bool DROP, int BIAS, bool PDS, bool NARROW = false, int SP = 1>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP || BIAS ? WPE - 1 : WPE))) void k_attn_bwd_dst_tile_bf16(
     bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, const bf16_t *__restrict__ o,
     const bf16_t *__restrict__ d_o, const float *__restrict__ lse, bf16_t *__restrict__ dq, uint32_t *__restrict__ pds,
@@ -2575,13 +2713,15 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
     const int Hs = NARROW ? nw.h : H;
     const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * 2 : (uint32_t)(H * D * 2);
     TileCtx t;
-    if (!tile_begin<bf16_t, H, D, HW, NARROW>(P, t, nw)) return;
+    if (!tile_begin<bf16_t, H, D, HW, NARROW, SP>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     __shared__ int fst_lds[HW][PDS ? TILE_CHUNK : 1];
     int2 *ent = ent_lds[t.wv];
     int *fst = PDS ? fst_lds[t.wv] : nullptr;
-    __shared__ __attribute__((aligned(16))) char kt_lds[HW][TILE_R * TILE_KT_BYTES_BF16];
-    char *kt = kt_lds[t.wv];
+    constexpr int PIECE = SP > 1 ? TILE_PART_FLOATS : TILE_KT_FLOATS_BF16;
+    static_assert(PIECE >= TILE_KT_FLOATS_BF16, "the rows fit");
+    __shared__ __attribute__((aligned(16))) float piece[HW][PIECE];
+    char *kt = reinterpret_cast<char *>(piece[t.wv]);
     TileEntryRegs er;
     if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
     issue_loads_first();
@@ -2612,7 +2752,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
         const size_t at = (size_t)max(t.member.x, 0) * Hs + t.head;
         lse_c = lse[at];
         if constexpr (!PDS) {
-            if (g == 0 && t.member.x >= 0) stat[at] = make_float2(lse_c, delta);
+            if (g == 0 && t.part == 0 && t.member.x >= 0) stat[at] = make_float2(lse_c, delta);
         }
     }
     floatx4v acc[4];
@@ -2674,24 +2814,31 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
             da.u[1] = pack_bf16(ds[2], ds[3]);
             tile_axpy_bf16(da, B.kc, acc);
         };
-        tile_walk<PIPE, Blk>(nblk, issue, compute);
+        tile_walk<Blk>(nblk, issue, compute);
         wave_lds_fence();
     }
-    tile_store_rows<H, D, false, NARROW>(t, acc, 1.f, dq, ws_dq, nw);
+    if constexpr (SP > 1) {
+        tile_park(piece[t.wv], acc, t.lane);
+        __syncthreads();
+        tile_meet_and_store<SP, H, D, NARROW>(piece[t.wv % (HW / SP)], (HW / SP) * PIECE, t, dq, ws_dq, nw);
+    } else {
+        tile_store_rows<H, D, false, NARROW>(t, acc, 1.f, dq, ws_dq, nw);
+    }
 }
 
 constexpr int TILE_WT_STRIDE_BF16 = 20;
-template <int H, int D, int HW, int WPE, bool PIPE, bool NARROW = false>
+template <int H, int D, int HW, int WPE, bool NARROW = false, int SP = 1>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))) void k_attn_bwd_src_tile_bf16(
     bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ d_o, const uint32_t *__restrict__ pds, bf16_t *__restrict__ dk,
     bf16_t *__restrict__ dv, float *__restrict__ ws_dk, float *__restrict__ ws_dv, Narrow nw) {
     const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * 2 : (uint32_t)(H * D * 2);
     TileCtx t;
-    if (!tile_begin<bf16_t, H, D, HW, NARROW>(P, t, nw)) return;
-    __shared__ int2 ent_lds[HW][TILE_CHUNK];
-    int2 *ent = ent_lds[t.wv];
-    __shared__ __attribute__((aligned(16))) uint32_t wt_lds[HW][TILE_R * TILE_WT_STRIDE_BF16];    // (turned as in the float32 kernel)
-    uint32_t *const wt = wt_lds[t.wv];
+    if (!tile_begin<bf16_t, H, D, HW, NARROW, SP>(P, t, nw)) return;
+    constexpr int ENT = TILE_CHUNK * 2, LIVE = ENT + TILE_R * TILE_WT_STRIDE_BF16, PIECE = SP > 1 ? 2 * TILE_PART_FLOATS : LIVE;
+    static_assert(PIECE >= LIVE, "the lists fit");
+    __shared__ __attribute__((aligned(16))) float piece[HW][PIECE];
+    int2 *ent = reinterpret_cast<int2 *>(piece[t.wv]);
+    uint32_t *const wt = reinterpret_cast<uint32_t *>(piece[t.wv] + ENT);         // (turned as in the float32 kernel)
     const int c = t.c, g = t.g;
     const uint32_t offc = t.offv;
     const char *qb = reinterpret_cast<const char *>(q), *db = reinterpret_cast<const char *>(d_o);
@@ -2750,11 +2897,21 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             tile_axpy_bf16(da, B.qr, ak);
             tile_axpy_bf16(pa, B.dr, av);
         };
-        tile_walk<PIPE, Blk>(nblk, issue, compute);
+        tile_walk<Blk>(nblk, issue, compute);
         wave_lds_fence();
     }
-    tile_store_rows<H, D, false, NARROW>(t, ak, 1.f, dk, ws_dk, nw);
-    tile_store_rows<H, D, false, NARROW>(t, av, 1.f, dv, ws_dv, nw);
+    if constexpr (SP > 1) {
+        constexpr int NEXT = (HW / SP) * PIECE;
+        tile_park(piece[t.wv], ak, t.lane);
+        tile_park(piece[t.wv] + TILE_PART_FLOATS, av, t.lane);
+        __syncthreads();
+        const float *const part0 = piece[t.wv % (HW / SP)];
+        tile_meet_and_store<SP, H, D, NARROW>(part0, NEXT, t, dk, ws_dk, nw);
+        tile_meet_and_store<SP, H, D, NARROW>(part0 + TILE_PART_FLOATS, NEXT, t, dv, ws_dv, nw);
+    } else {
+        tile_store_rows<H, D, false, NARROW>(t, ak, 1.f, dk, ws_dk, nw);
+        tile_store_rows<H, D, false, NARROW>(t, av, 1.f, dv, ws_dv, nw);
+    }
 }
 
 // Source side without the scratch: p and ds of a block's pairs are formed again from the entries' q and dO rows, which are
@@ -2769,7 +2926,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
 // columns with dropout lost 2 %: heads of fewer than 64 columns keep the scratch.)  float32 keeps it too: there the two
 // products are 1024 cycles of the matrix pipeline per block.  118 registers: compiled for four wavefronts per SIMD (for five,
 // with the members' rows in LDS or not, it spills: 658 us; four with them in LDS 316; q rows a block ahead spills too: 346).
-template <int H, int D, int HW, int WPE, bool DROP>
+template <int H, int D, int HW, int WPE, bool DROP, int SP = 1>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))) void k_attn_bwd_src_tile_bf16_again(
     bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, const bf16_t *__restrict__ d_o,
     const float2 *__restrict__ stat, bf16_t *__restrict__ dk, bf16_t *__restrict__ dv, float *__restrict__ ws_dk, float *__restrict__ ws_dv,
@@ -2777,13 +2934,14 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     constexpr uint32_t RB = H * D * 2;
     const Narrow nw{};
     TileCtx t;
-    if (!tile_begin<bf16_t, H, D, HW>(P, t, nw)) return;
-    __shared__ int2 ent_lds[HW][TILE_CHUNK];
-    __shared__ __attribute__((aligned(16))) char kt_lds[HW][TILE_R * TILE_KT_BYTES_BF16];
-    __shared__ __attribute__((aligned(16))) float2 stat_lds[HW][TILE_R];
-    int2 *ent = ent_lds[t.wv];
-    char *kt = kt_lds[t.wv];
-    float2 *const st_lds = stat_lds[t.wv];
+    if (!tile_begin<bf16_t, H, D, HW, false, SP>(P, t, nw)) return;
+    // a wavefront's piece: its entry list, the rows being turned, the entries' (lse, delta); afterwards (SP > 1) what it has summed up
+    constexpr int ENT = TILE_CHUNK * 2, LIVE = ENT + TILE_KT_FLOATS_BF16 + 2 * TILE_R, PIECE = SP > 1 ? 2 * TILE_PART_FLOATS : LIVE;
+    static_assert(PIECE >= LIVE, "the lists fit");
+    __shared__ __attribute__((aligned(16))) float piece[HW][PIECE];
+    int2 *ent = reinterpret_cast<int2 *>(piece[t.wv]);
+    char *kt = reinterpret_cast<char *>(piece[t.wv] + ENT);
+    float2 *const st_lds = reinterpret_cast<float2 *>(piece[t.wv] + ENT + TILE_KT_FLOATS_BF16);
     TileEntryRegs er;
     if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
     issue_loads_first();
@@ -2846,11 +3004,21 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             tile_axpy_bf16(da, B.qr, ak);
             tile_axpy_bf16(pa, B.dr, av);
         };
-        tile_walk<false, Blk>(nblk, issue, compute);
+        tile_walk<Blk>(nblk, issue, compute);
         wave_lds_fence();
     }
-    tile_store_rows<H, D, false, false>(t, ak, 1.f, dk, ws_dk, nw);
-    tile_store_rows<H, D, false, false>(t, av, 1.f, dv, ws_dv, nw);
+    if constexpr (SP > 1) {
+        constexpr int NEXT = (HW / SP) * PIECE;
+        tile_park(piece[t.wv], ak, t.lane);
+        tile_park(piece[t.wv] + TILE_PART_FLOATS, av, t.lane);
+        __syncthreads();
+        const float *const part0 = piece[t.wv % (HW / SP)];
+        tile_meet_and_store<SP, H, D, false>(part0, NEXT, t, dk, ws_dk, nw);
+        tile_meet_and_store<SP, H, D, false>(part0 + TILE_PART_FLOATS, NEXT, t, dv, ws_dv, nw);
+    } else {
+        tile_store_rows<H, D, false, false>(t, ak, 1.f, dk, ws_dk, nw);
+        tile_store_rows<H, D, false, false>(t, av, 1.f, dv, ws_dv, nw);
+    }
 }
 
 // Backward, destination side.  Writes (p, ds) of every pair to pds[(t * H + head)], t = the pair's
@@ -4217,10 +4385,32 @@ inline bool has_tiles(const bpt_plan *P, int h, int d, size_t elem) {
            fits32(std::max(P->n_rows, P->n_index_nodes), (int64_t)h * d * (int64_t)elem);
 }
 
-// Few and tall tiles (fewer wavefronts than three per SIMD, six or more blocks each on average): the kernels then read one
-// block ahead in registers instead of counting on other wavefronts to cover the loads.
-inline bool tall_tiles(const bpt_plan *P, int h) {
-    return P->n_groups * h < 3 * 1024 && P->n_grp_entries >= 6 * TILE_R * P->n_groups;
+// Over how many wavefronts (1, 2 or 4) of a workgroup the blocks of a tile are spread.  A launch has 1024 SIMDs to fill, and one
+// that does not lasts as long as its longest chain of blocks: each part's chain is a half or a quarter as long.  What
+// the parts cost is the tile's header, read by each of them, and the meeting in LDS, so with more wavefronts than fill the chip
+// a part has to keep enough blocks.  float32, 8 heads, forward / destination side / source side, one part -> two -> four:
+//   584 wavefronts of 4 to 9 blocks (L = 512)           10.3 / 13.8 / 16.4 -> 8.0 / 10.8 / 10.9 -> 8.0 / 9.6 / 8.6 us
+//   1032 of 9 (window of 128, L = 2048)                 20.5 / 29.8 / 17.0 -> 15.7 / 21.3 / 13.7 -> 14.5 / 19.4 / 13.8
+//   1448 of 3 (L = 1400, k = 4)                         11.9 / 16.3 / 11.3 -> 11.4 / 14.3 / 10.2 -> 12.8 / 16.6 / 11.7
+//   2056 of 9 (window of 128, L = 4096)                 25.2 / 38.6 / 25.1 -> 20.8 / 30.7 / 21.3 -> 22.9 / 32.5 / 22.3
+//   2096 of 3 (16 heads, L = 1024, k = 4)               12.8 / 19.2 / 13.9 -> 13.4 / 19.6 / 15.0 -> 14.8 / 20.6 / 14.8
+//   2072 of 4 / 2168 of 5 (L = 2048, k = 8)             16.8 / 26.1 / 19.0 -> 14.4 / 21.4 / 18.2 -> 15.8 / 22.4 / 17.5
+//   4112 of 9 (window of 128, L = 8192)                 33.3 / 56.6 / 48.4 -> 32.3 / 53.1 / 35.5 -> 37.0 / 58.3 / 38.6
+//   4160 of 5 / 4448 of 8 (L = 4096, k = 4, both ways)  24.0 / 37.6 / 37.0 -> 24.4 / 39.4 / 35.3 -> 27.8 / 42.4 / 37.1
+//   8080 of 16 / 8072 of 9 (window of 256, L = 8192)    91.0 / 142 / 93.8  -> 93.2 / 140 / 85.0  -> 101 / 149 / 88.6
+//   8256 of 5 (window of 64, L = 16384)                 46.5 / 72.1 / 51.4 -> 49.6 / 72.2 / 50.1 -> 57.4 / 84.7 / 61.6
+// bfloat16, whose blocks are shorter against their headers:
+//   584 of 3 (L = 512)      5.8 / 6.6 / 8.1 -> 5.1 / 6.0 / 6.4 -> 5.0 / 6.4 / 5.5;    1048 of 3    6.6 / 7.5 / 8.5 -> 6.4 / 7.6 / 8.4 -> 6.9 / 9.2 / 9.1
+//   1032 of 9              11.4 / 12.9 / 12.0 -> 9.0 / 11.2 / 10.0 -> 8.3 / 10.1 / 10.4;  2056 of 9   13.1 / 14.8 / 14.8 -> 11.8 / 14.0 / 14.4 -> 12.8 / 18.7 / 15.8
+//   4112 of 9              18.3 / 21.0 / 22.1 -> 17.8 / 23.8 / 22.3 -> 20.1 / 30.3 / 27.1
+inline int tile_parts(const bpt_plan *P, int heads, size_t elem) {
+    const int64_t wavefronts = P->n_groups * heads, blocks = P->n_grp_entries / TILE_R;
+    auto pays = [&](int parts) {
+        const int64_t w = wavefronts * parts, each = blocks / std::max<int64_t>(P->n_groups * parts, 1);      // (blocks of a part, rounded down)
+        if (elem == 2) return w <= 2400 || (parts == 2 && w <= 4608 && each >= 4);
+        return w <= 3072 || (w <= 6144 && each >= 2) || (parts == 2 && w <= 16384 && each >= 4);
+    };
+    return pays(4) ? 4 : pays(2) ? 2 : 1;
 }
 
 bool spmm_grp_ok(const bpt_plan *P, int h, int d, int dtype) {
@@ -4308,28 +4498,17 @@ int run_attn_fwd(const bpt_plan *P, const void *q, const void *k, const void *v,
         if constexpr (D == 64 && sizeof(T) == 4) {
             if (has_tiles(P, H, D, sizeof(T)) && ((drop.thr == 0 && !bias) || P->grp_eids)) {
                 constexpr int HW = H >= 4 ? 4 : H;          // heads per workgroup
-#define LAUNCH_FWD_TILE(PI, DR, BI)                                                                                                  \
-    hipLaunchKernelGGL((k_attn_fwd_tile<T, H, D, HW, PI, DR, BI>), dim3(group_grid(P) * (H / HW)), dim3(HW * WAVE), 0, s, *P, (const T *)q, \
-                       (const T *)k, (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed, drop.inv, bias, Narrow{})
-                switch ((drop.thr != 0 ? 1 : 0) + 2 * tile_bias_mode(P, bias)) {
-                case 0: if (tall_tiles(P, H)) LAUNCH_FWD_TILE(true, false, 0); else LAUNCH_FWD_TILE(false, false, 0); break;
-                case 1: LAUNCH_FWD_TILE(false, true, 0); break;
-                case 2: LAUNCH_FWD_TILE(false, false, 1); break;
-                case 3: LAUNCH_FWD_TILE(false, true, 1); break;
-                case 4: LAUNCH_FWD_TILE(false, false, 2); break;
-                default: LAUNCH_FWD_TILE(false, true, 2); break;
-                }
-#undef LAUNCH_FWD_TILE
-                goto launched;
-            }
-        }
-        if constexpr (D == 64 && sizeof(T) == 2) {
-            if (has_tiles(P, H, D, sizeof(T)) && ((drop.thr == 0 && !bias) || P->grp_eids)) {
-                constexpr int HW = H >= 4 ? 4 : H;
-#define LAUNCH_FWD_TILE(DR, BI)                                                                                                          \
-    hipLaunchKernelGGL((k_attn_fwd_tile_bf16<H, D, HW, TILE_BF16_WPE, TILE_BF16_PIPE, DR, BI>), dim3(group_grid(P) * (H / HW)), dim3(HW * WAVE), \
-                       0, s, *P, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (bf16_t *)o, lse, ws_acc, ws_ml, scale * LOG2E,   \
-                       drop.thr, drop.seed, drop.inv, bias, Narrow{})
+                const int parts = tile_parts(P, H, sizeof(T));
+#define LAUNCH_FWD_TILE_PARTS(DR, BI, SP)                                                                                            \
+    hipLaunchKernelGGL((k_attn_fwd_tile<T, H, D, HW, DR, BI, false, SP>), dim3(group_grid(P) * (H * SP / HW)), dim3(HW * WAVE), 0, s, *P, \
+                       (const T *)q, (const T *)k, (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed, drop.inv, bias, \
+                       Narrow{})
+#define LAUNCH_FWD_TILE(DR, BI)                                                                                                      \
+    do {                                                                                                                             \
+        if (parts == 4) LAUNCH_FWD_TILE_PARTS(DR, BI, 4);                                                                            \
+        else if (parts == 2) LAUNCH_FWD_TILE_PARTS(DR, BI, 2);                                                                       \
+        else LAUNCH_FWD_TILE_PARTS(DR, BI, 1);                                                                                       \
+    } while (0)
                 switch ((drop.thr != 0 ? 1 : 0) + 2 * tile_bias_mode(P, bias)) {
                 case 0: LAUNCH_FWD_TILE(false, 0); break;
                 case 1: LAUNCH_FWD_TILE(true, 0); break;
@@ -4339,6 +4518,34 @@ int run_attn_fwd(const bpt_plan *P, const void *q, const void *k, const void *v,
                 default: LAUNCH_FWD_TILE(true, 2); break;
                 }
 #undef LAUNCH_FWD_TILE
+#undef LAUNCH_FWD_TILE_PARTS
+                goto launched;
+            }
+        }
+        if constexpr (D == 64 && sizeof(T) == 2) {
+            if (has_tiles(P, H, D, sizeof(T)) && ((drop.thr == 0 && !bias) || P->grp_eids)) {
+                constexpr int HW = H >= 4 ? 4 : H;
+                const int parts = tile_parts(P, H, sizeof(T));
+#define LAUNCH_FWD_TILE_PARTS(DR, BI, SP)                                                                                                \
+    hipLaunchKernelGGL((k_attn_fwd_tile_bf16<H, D, HW, TILE_BF16_WPE, DR, BI, false, SP>), dim3(group_grid(P) * (H * SP / HW)), \
+                       dim3(HW * WAVE), 0, s, *P, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (bf16_t *)o, lse, ws_acc, ws_ml, \
+                       scale * LOG2E, drop.thr, drop.seed, drop.inv, bias, Narrow{})
+#define LAUNCH_FWD_TILE(DR, BI)                                                                                                          \
+    do {                                                                                                                                 \
+        if (parts == 4) LAUNCH_FWD_TILE_PARTS(DR, BI, 4);                                                                                \
+        else if (parts == 2) LAUNCH_FWD_TILE_PARTS(DR, BI, 2);                                                                           \
+        else LAUNCH_FWD_TILE_PARTS(DR, BI, 1);                                                                                           \
+    } while (0)
+                switch ((drop.thr != 0 ? 1 : 0) + 2 * tile_bias_mode(P, bias)) {
+                case 0: LAUNCH_FWD_TILE(false, 0); break;
+                case 1: LAUNCH_FWD_TILE(true, 0); break;
+                case 2: LAUNCH_FWD_TILE(false, 1); break;
+                case 3: LAUNCH_FWD_TILE(true, 1); break;
+                case 4: LAUNCH_FWD_TILE(false, 2); break;
+                default: LAUNCH_FWD_TILE(true, 2); break;
+                }
+#undef LAUNCH_FWD_TILE
+#undef LAUNCH_FWD_TILE_PARTS
                 goto launched;
             }
         }
@@ -4401,26 +4608,40 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
             float *ws_dk = ws_rows + (size_t)Pin->n_slots * H * D, *ws_dv = ws_dk + (size_t)Pout->n_slots * H * D;
             {
                 ProfScope prof(BPT_KERNEL_ATTN_BWD_DST, s);
-#define LAUNCH_DST_TILE(PI, DR, BI)                                                                                                    \
-    hipLaunchKernelGGL((k_attn_bwd_dst_tile<T, H, D, HW, PI, DR, BI>), dim3(group_grid(Pin) * (H / HW)), dim3(HW * WAVE), 0, s, *Pin,     \
-                       (const T *)q, (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pds, ws_rows, scale,         \
+                const int parts = tile_parts(Pin, H, sizeof(T));
+#define LAUNCH_DST_TILE_PARTS(DR, BI, SP)                                                                                              \
+    hipLaunchKernelGGL((k_attn_bwd_dst_tile<T, H, D, HW, DR, BI, false, SP>), dim3(group_grid(Pin) * (H * SP / HW)), dim3(HW * WAVE), 0, s, \
+                       *Pin, (const T *)q, (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pds, ws_rows, scale,    \
                        scale * LOG2E, drop.thr, drop.seed, drop.inv, bias, ds_out, Narrow{})
+#define LAUNCH_DST_TILE(DR, BI)                                                                                                        \
+    do {                                                                                                                               \
+        if (parts == 4) LAUNCH_DST_TILE_PARTS(DR, BI, 4);                                                                              \
+        else if (parts == 2) LAUNCH_DST_TILE_PARTS(DR, BI, 2);                                                                         \
+        else LAUNCH_DST_TILE_PARTS(DR, BI, 1);                                                                                         \
+    } while (0)
                 switch ((drop.thr != 0 ? 1 : 0) + 2 * tile_bias_mode(Pin, bias)) {
-                case 0: if (tall_tiles(Pin, H)) LAUNCH_DST_TILE(true, false, 0); else LAUNCH_DST_TILE(false, false, 0); break;
-                case 1: LAUNCH_DST_TILE(false, true, 0); break;
-                case 2: LAUNCH_DST_TILE(false, false, 1); break;
-                case 3: LAUNCH_DST_TILE(false, true, 1); break;
-                case 4: LAUNCH_DST_TILE(false, false, 2); break;
-                default: LAUNCH_DST_TILE(false, true, 2); break;
+                case 0: LAUNCH_DST_TILE(false, 0); break;
+                case 1: LAUNCH_DST_TILE(true, 0); break;
+                case 2: LAUNCH_DST_TILE(false, 1); break;
+                case 3: LAUNCH_DST_TILE(true, 1); break;
+                case 4: LAUNCH_DST_TILE(false, 2); break;
+                default: LAUNCH_DST_TILE(true, 2); break;
                 }
 #undef LAUNCH_DST_TILE
+#undef LAUNCH_DST_TILE_PARTS
             }
             int st = launch_status();
             if (st != BPT_OK) return st;
             {
                 ProfScope prof(BPT_KERNEL_ATTN_BWD_SRC, s);
-                hipLaunchKernelGGL((k_attn_bwd_src_tile<T, H, D, HW>), dim3(group_grid(Pout) * (H / HW)), dim3(HW * WAVE), 0, s, *Pout,
-                                   (const T *)q, (const T *)d_o, (const float2 *)pds, (T *)dk, (T *)dv, ws_dk, ws_dv, Narrow{});
+#define LAUNCH_SRC_TILE(SP)                                                                                                              \
+    hipLaunchKernelGGL((k_attn_bwd_src_tile<T, H, D, HW, false, SP>), dim3(group_grid(Pout) * (H * SP / HW)), dim3(HW * WAVE), 0, s, *Pout,  \
+                       (const T *)q, (const T *)d_o, (const float2 *)pds, (T *)dk, (T *)dv, ws_dk, ws_dv, Narrow{})
+                const int parts = tile_parts(Pout, H, sizeof(T));
+                if (parts == 4) LAUNCH_SRC_TILE(4);
+                else if (parts == 2) LAUNCH_SRC_TILE(2);
+                else LAUNCH_SRC_TILE(1);
+#undef LAUNCH_SRC_TILE
             }
             st = launch_status();
             if (st != BPT_OK || Pin->n_heavy + Pout->n_heavy == 0) return st;
@@ -4437,11 +4658,18 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
             float *ws_dk = ws_rows + (size_t)Pin->n_slots * H * D, *ws_dv = ws_dk + (size_t)Pout->n_slots * H * D;
             {
                 ProfScope prof(BPT_KERNEL_ATTN_BWD_DST, s);
-#define LAUNCH_DST_TILE(DR, BI, PD)                                                                                                      \
-    hipLaunchKernelGGL((k_attn_bwd_dst_tile_bf16<H, D, HW, TILE_BF16_WPE_DST, TILE_BF16_PIPE, DR, BI, PD>), dim3(group_grid(Pin) * (H / HW)), \
-                       dim3(HW * WAVE), 0, s, *Pin, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (const bf16_t *)o,             \
+                const int parts = tile_parts(Pin, H, sizeof(T));
+#define LAUNCH_DST_TILE_PARTS(DR, BI, PD, SP)                                                                                            \
+    hipLaunchKernelGGL((k_attn_bwd_dst_tile_bf16<H, D, HW, TILE_BF16_WPE_DST, DR, BI, PD, false, SP>),                       \
+                       dim3(group_grid(Pin) * (H * SP / HW)), dim3(HW * WAVE), 0, s, *Pin, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (const bf16_t *)o,             \
                        (const bf16_t *)d_o, lse, (bf16_t *)dq, (uint32_t *)ws, (float2 *)ws, ws_rows, scale, scale * LOG2E, drop.thr,       \
                        drop.seed, drop.inv, bias, ds_out, Narrow{})
+#define LAUNCH_DST_TILE(DR, BI, PD)                                                                                                      \
+    do {                                                                                                                                 \
+        if (parts == 4) LAUNCH_DST_TILE_PARTS(DR, BI, PD, 4);                                                                            \
+        else if (parts == 2) LAUNCH_DST_TILE_PARTS(DR, BI, PD, 2);                                                                       \
+        else LAUNCH_DST_TILE_PARTS(DR, BI, PD, 1);                                                                                       \
+    } while (0)
                 switch (again ? (drop.thr != 0 ? 7 : 6) : (drop.thr != 0 ? 1 : 0) + 2 * tile_bias_mode(Pin, bias)) {
                 case 6: LAUNCH_DST_TILE(false, 0, false); break;
                 case 7: LAUNCH_DST_TILE(true, 0, false); break;
@@ -4452,21 +4680,33 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
                 default: LAUNCH_DST_TILE(true, 2, true); break;
                 }
 #undef LAUNCH_DST_TILE
+#undef LAUNCH_DST_TILE_PARTS
             }
             int st = launch_status();
             if (st != BPT_OK) return st;
             {
                 ProfScope prof(BPT_KERNEL_ATTN_BWD_SRC, s);
-#define LAUNCH_SRC_AGAIN(DR)                                                                                                             \
-    hipLaunchKernelGGL((k_attn_bwd_src_tile_bf16_again<H, D, HW, TILE_BF16_WPE_AGAIN, DR>), dim3(group_grid(Pout) * (H / HW)), dim3(HW * WAVE), 0, s, \
-                       *Pout, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (const bf16_t *)d_o, (const float2 *)ws, (bf16_t *)dk, \
-                       (bf16_t *)dv, ws_dk, ws_dv, scale, scale * LOG2E, drop.thr, drop.seed, drop.inv)
-                if (again && drop.thr != 0) LAUNCH_SRC_AGAIN(true);
-                else if (again) LAUNCH_SRC_AGAIN(false);
-                else
-                    hipLaunchKernelGGL((k_attn_bwd_src_tile_bf16<H, D, HW, TILE_BF16_WPE_SRC, TILE_BF16_PIPE>), dim3(group_grid(Pout) * (H / HW)), dim3(HW * WAVE), 0, s,
-                                       *Pout, (const bf16_t *)q, (const bf16_t *)d_o, (const uint32_t *)ws, (bf16_t *)dk, (bf16_t *)dv, ws_dk, ws_dv, Narrow{});
-#undef LAUNCH_SRC_AGAIN
+                const int parts = tile_parts(Pout, H, sizeof(T));
+#define LAUNCH_SRC_AGAIN_PARTS(DR, SP)                                                                                                   \
+    hipLaunchKernelGGL((k_attn_bwd_src_tile_bf16_again<H, D, HW, TILE_BF16_WPE_AGAIN, DR, SP>), dim3(group_grid(Pout) * (H * SP / HW)),      \
+                       dim3(HW * WAVE), 0, s, *Pout, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (const bf16_t *)d_o,         \
+                       (const float2 *)ws, (bf16_t *)dk, (bf16_t *)dv, ws_dk, ws_dv, scale, scale * LOG2E, drop.thr, drop.seed, drop.inv)
+#define LAUNCH_SRC_PDS(SP)                                                                                                               \
+    hipLaunchKernelGGL((k_attn_bwd_src_tile_bf16<H, D, HW, TILE_BF16_WPE_SRC, false, SP>), dim3(group_grid(Pout) * (H * SP / HW)), \
+                       dim3(HW * WAVE), 0, s, *Pout, (const bf16_t *)q, (const bf16_t *)d_o, (const uint32_t *)ws, (bf16_t *)dk, (bf16_t *)dv, \
+                       ws_dk, ws_dv, Narrow{})
+#define LAUNCH_SRC_TILE(SP)                                                                                                              \
+    do {                                                                                                                                 \
+        if (again && drop.thr != 0) LAUNCH_SRC_AGAIN_PARTS(true, SP);                                                                    \
+        else if (again) LAUNCH_SRC_AGAIN_PARTS(false, SP);                                                                               \
+        else LAUNCH_SRC_PDS(SP);                                                                                                         \
+    } while (0)
+                if (parts == 4) LAUNCH_SRC_TILE(4);
+                else if (parts == 2) LAUNCH_SRC_TILE(2);
+                else LAUNCH_SRC_TILE(1);
+#undef LAUNCH_SRC_TILE
+#undef LAUNCH_SRC_PDS
+#undef LAUNCH_SRC_AGAIN_PARTS
             }
             st = launch_status();
             if (st != BPT_OK || Pin->n_heavy + Pout->n_heavy == 0) return st;
@@ -4540,25 +4780,40 @@ template <typename T> bool narrow_ok(const bpt_plan *P, const Narrow &nw) {
     return has_tiles(P, nw.h, 64, sizeof(T)) && (P->grp_eids != nullptr);
 }
 
+// a tile in parts: one head a workgroup, so that no wavefront of it lies past the last head
+inline Narrow narrow_parts(Narrow nw, int parts) {
+    if (parts > 1) nw.slices = nw.heads;
+    return nw;
+}
+
 template <typename T>
 int run_attn_fwd_narrow(const bpt_plan *P, const void *q, const void *k, const void *v, void *o, float *lse, void *ws, float scale, Dropout drop,
                         const Narrow &nw, hipStream_t s) {
     if (P->n_items == 0) return BPT_OK;
     float *ws_acc = (float *)ws, *ws_ml = ws_acc ? ws_acc + (size_t)P->n_slots * nw.h * 64 : nullptr;
-    const dim3 grid(group_grid(P) * nw.slices), block(NARROW_HW * WAVE);
+    const int parts = tile_parts(P, nw.heads, sizeof(T));
+    const Narrow np = narrow_parts(nw, parts);
+    const dim3 grid(group_grid(P) * np.slices), block((parts == 1 ? NARROW_HW : parts) * WAVE);
     {
         ProfScope prof(BPT_KERNEL_ATTN_FWD, s);
-#define LAUNCH_FWD(DR)                                                                                                                   \
+#define LAUNCH_FWD_PARTS(DR, HW, SP)                                                                                                     \
     do {                                                                                                                                 \
         if constexpr (sizeof(T) == 4)                                                                                                    \
-            hipLaunchKernelGGL((k_attn_fwd_tile<T, 16, 64, NARROW_HW, false, DR, 0, true>), grid, block, 0, s, *P, (const T *)q, (const T *)k,   \
-                               (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed, drop.inv, (const float *)nullptr, nw); \
+            hipLaunchKernelGGL((k_attn_fwd_tile<T, 16, 64, HW, DR, 0, true, SP>), grid, block, 0, s, *P, (const T *)q, (const T *)k,         \
+                               (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed, drop.inv, (const float *)nullptr, np); \
         else                                                                                                                             \
-            hipLaunchKernelGGL((k_attn_fwd_tile_bf16<16, 64, NARROW_HW, TILE_BF16_WPE, false, DR, 0, true>), grid, block, 0, s, *P,              \
+            hipLaunchKernelGGL((k_attn_fwd_tile_bf16<16, 64, HW, TILE_BF16_WPE, DR, 0, true, SP>), grid, block, 0, s, *P,                    \
                                (const T *)q, (const T *)k, (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed,       \
-                               drop.inv, (const float *)nullptr, nw);                                                                      \
+                               drop.inv, (const float *)nullptr, np);                                                                      \
+    } while (0)
+#define LAUNCH_FWD(DR)                                                                                                                   \
+    do {                                                                                                                                 \
+        if (parts == 4) LAUNCH_FWD_PARTS(DR, 4, 4);                                                                                      \
+        else if (parts == 2) LAUNCH_FWD_PARTS(DR, 2, 2);                                                                                 \
+        else LAUNCH_FWD_PARTS(DR, NARROW_HW, 1);                                                                                         \
     } while (0)
         if (drop.thr != 0) LAUNCH_FWD(true); else LAUNCH_FWD(false);
+#undef LAUNCH_FWD_PARTS
 #undef LAUNCH_FWD
     }
     const int st = launch_status();
@@ -4576,33 +4831,50 @@ int run_attn_bwd_narrow(const bpt_plan *Pin, const bpt_plan *Pout, const void *q
     pds_t *pds = (pds_t *)ws;
     float *ws_dq = (float *)ws + pds_bytes(Pin, Pout, nw.h, 64, sizeof(T), false) / 4;
     float *ws_dk = ws_dq + (size_t)Pin->n_slots * nw.h * 64, *ws_dv = ws_dk + (size_t)Pout->n_slots * nw.h * 64;
-    const dim3 grid(group_grid(Pin) * nw.slices), grid_src(group_grid(Pout) * nw.slices), block(NARROW_HW * WAVE);
+    const int parts = tile_parts(Pin, nw.heads, sizeof(T)), parts_src = tile_parts(Pout, nw.heads, sizeof(T));
+    const Narrow np = narrow_parts(nw, parts), np_src = narrow_parts(nw, parts_src);
+    const dim3 grid(group_grid(Pin) * np.slices), block((parts == 1 ? NARROW_HW : parts) * WAVE);
+    const dim3 grid_src(group_grid(Pout) * np_src.slices), block_src((parts_src == 1 ? NARROW_HW : parts_src) * WAVE);
     {
         ProfScope prof(BPT_KERNEL_ATTN_BWD_DST, s);
-#define LAUNCH_DST(DR)                                                                                                                   \
+#define LAUNCH_DST_PARTS(DR, HW, SP)                                                                                                     \
     do {                                                                                                                                 \
         if constexpr (sizeof(T) == 4)                                                                                                    \
-            hipLaunchKernelGGL((k_attn_bwd_dst_tile<T, 16, 64, NARROW_HW, false, DR, 0, true>), grid, block, 0, s, *Pin, (const T *)q,           \
+            hipLaunchKernelGGL((k_attn_bwd_dst_tile<T, 16, 64, HW, DR, 0, true, SP>), grid, block, 0, s, *Pin, (const T *)q,                 \
                                (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pds, ws_dq, scale, scale * LOG2E,       \
-                               drop.thr, drop.seed, drop.inv, (const float *)nullptr, (float *)nullptr, nw);                                \
+                               drop.thr, drop.seed, drop.inv, (const float *)nullptr, (float *)nullptr, np);                                \
         else                                                                                                                             \
-            hipLaunchKernelGGL((k_attn_bwd_dst_tile_bf16<16, 64, NARROW_HW, TILE_BF16_WPE_DST, false, DR, 0, true, true>), grid, block, 0, s, *Pin, \
+            hipLaunchKernelGGL((k_attn_bwd_dst_tile_bf16<16, 64, HW, TILE_BF16_WPE_DST, DR, 0, true, true, SP>), grid, block, 0, s, *Pin,    \
                                (const T *)q, (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pds, (float2 *)nullptr, ws_dq, \
-                               scale, scale * LOG2E, drop.thr, drop.seed, drop.inv, (const float *)nullptr, (float *)nullptr, nw);          \
+                               scale, scale * LOG2E, drop.thr, drop.seed, drop.inv, (const float *)nullptr, (float *)nullptr, np);          \
+    } while (0)
+#define LAUNCH_DST(DR)                                                                                                                   \
+    do {                                                                                                                                 \
+        if (parts == 4) LAUNCH_DST_PARTS(DR, 4, 4);                                                                                      \
+        else if (parts == 2) LAUNCH_DST_PARTS(DR, 2, 2);                                                                                 \
+        else LAUNCH_DST_PARTS(DR, NARROW_HW, 1);                                                                                         \
     } while (0)
         if (drop.thr != 0) LAUNCH_DST(true); else LAUNCH_DST(false);
+#undef LAUNCH_DST_PARTS
 #undef LAUNCH_DST
     }
     int st = launch_status();
     if (st != BPT_OK) return st;
     {
         ProfScope prof(BPT_KERNEL_ATTN_BWD_SRC, s);
-        if constexpr (sizeof(T) == 4)
-            hipLaunchKernelGGL((k_attn_bwd_src_tile<T, 16, 64, NARROW_HW, true>), grid_src, block, 0, s, *Pout, (const T *)q, (const T *)d_o,
-                               pds, (T *)dk, (T *)dv, ws_dk, ws_dv, nw);
-        else
-            hipLaunchKernelGGL((k_attn_bwd_src_tile_bf16<16, 64, NARROW_HW, TILE_BF16_WPE_SRC, false, true>), grid_src, block, 0, s, *Pout,
-                               (const T *)q, (const T *)d_o, pds, (T *)dk, (T *)dv, ws_dk, ws_dv, nw);
+#define LAUNCH_SRC(HW, SP)                                                                                                               \
+    do {                                                                                                                                 \
+        if constexpr (sizeof(T) == 4)                                                                                                    \
+            hipLaunchKernelGGL((k_attn_bwd_src_tile<T, 16, 64, HW, true, SP>), grid_src, block_src, 0, s, *Pout, (const T *)q, (const T *)d_o, \
+                               pds, (T *)dk, (T *)dv, ws_dk, ws_dv, np_src);                                                               \
+        else                                                                                                                             \
+            hipLaunchKernelGGL((k_attn_bwd_src_tile_bf16<16, 64, HW, TILE_BF16_WPE_SRC, true, SP>), grid_src, block_src, 0, s, *Pout,        \
+                               (const T *)q, (const T *)d_o, pds, (T *)dk, (T *)dv, ws_dk, ws_dv, np_src);                                  \
+    } while (0)
+        if (parts_src == 4) LAUNCH_SRC(4, 4);
+        else if (parts_src == 2) LAUNCH_SRC(2, 2);
+        else LAUNCH_SRC(NARROW_HW, 1);
+#undef LAUNCH_SRC
     }
     st = launch_status();
     if (st != BPT_OK || Pin->n_heavy + Pout->n_heavy == 0) return st;
