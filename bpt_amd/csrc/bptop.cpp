@@ -384,7 +384,7 @@ Tensor attention_narrow(const Tensor &row, const Tensor &indptr_r, const Tensor 
 
 // ---- tile plans ---------------------------------------------------------------------------------------------------------------
 // The tile plans of one side of a graph or of both (the second linked to the first: what a training step needs), built in shared
-// launches with two waits: one for the counts, one for the finished plans (another stream may use them next).
+// launches.  One wait, for the counts; the caller waits for the finished plans before anybody else may use them.
 struct SideIn {
     Tensor row, indptr, eid, indices;
     int64_t n_rows, n_index;
@@ -487,7 +487,6 @@ py::object build_tile_plans(const std::vector<std::tuple<Tensor, Tensor, Tensor,
         }
         check_build(bpt_build_tiles_write(sides, n, c, out, PAD_ENTRIES, link ? pairs.data_ptr<int32_t>() : nullptr, ws.data_ptr(), bytes, stream),
                     "bpt_build_tiles_write");
-        wait_for(stream);
     }
     py::list result;
     for (int i = 0; i < n; ++i) {

@@ -746,9 +746,11 @@ def attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, in
 
 def prepare_training(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p=0.0, narrow_h=None):
     """Builds the plans that a forward and a backward of this layer are going to ask for together, where both run on tiles and
-    neither plan is in the cache (a new graph: two waits for the GPU instead of five, half of the launches).  A convenience: what
-    is not built here is built when it is asked for.  narrow_h: heads that attention_padded_shape pads to."""
-    cfg = _SETTINGS
+    neither plan is in the cache (a new graph: two waits for the GPU instead of five, half of the launches).  What attention_forward
+    and attention_backward would choose with them is remembered at once, so that both passes are served by the native host path
+    (the backward would else run here, on autograd's thread, which waits for the interpreter to be handed over).  A convenience:
+    what is not built here is built when it is asked for.  narrow_h: heads that attention_padded_shape pads to."""
+    generation, cfg = _native.generation(), _SETTINGS
     graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
     if q.dim() != 3 or not q.is_cuda or any(t.dim() != 1 or t.dtype != torch.int64 or t.device != q.device or not t.is_contiguous() for t in graph):
         return
@@ -759,9 +761,22 @@ def prepare_training(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indi
         seg = _narrow_seg(col, q, k, h, eid_c.size(0), dropout_p, cfg)
     else:
         seg = _tile_seg_without_plan(col, eid_c.size(0), q, k, h, d, dropout_p, None, cfg) if attention_supported(q) else None
-    if seg is not None:
-        plan_cache.put_tile_plans([(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg, None),
-                                   (row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg, _plan.tile_order_src(k.size(0), eid_r.size(0)))])
+    if seg is None:
+        return
+    order_src = _plan.tile_order_src(k.size(0), eid_r.size(0))
+    if not plan_cache.put_tile_plans([(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg, None),
+                                      (row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg, order_src)]):
+        return
+    pi = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, None))
+    po = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, order_src))
+    if not (pi.covers_all_edges and po.covers_all_edges):
+        return
+    fwd, bwd = (_native.ATTN_FWD, _native.ATTN_BWD) if narrow_h is None else (_native.ATTN_FWD_NARROW, _native.ATTN_BWD_NARROW)
+    numbers = [q.size(0), k.size(0), h, q.size(2), _dtype(q), int(dropout_p > 0.0)] + ([] if narrow_h is None else [q.size(1)])
+    in_struct = pi.ensure_groups(TILE_ROWS)["struct"]
+    out_struct = po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True)
+    plan_cache.remember((pi,), generation, fwd, list(graph[4:]), numbers, ctypes.addressof(in_struct), 0)
+    plan_cache.remember((pi, po), generation, bwd, list(graph), numbers, ctypes.addressof(in_struct), ctypes.addressof(out_struct))
 
 
 def _pair_order(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p):

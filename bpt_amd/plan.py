@@ -487,6 +487,7 @@ class DevicePlan:
             st = PlanStruct.from_buffer_copy(plans[1]._groups[(TILE_GROUP_R, self_of[1][1])]["struct"])
             st.grp_pairs = pairs.data_ptr()
             plans[1]._links[(id(plans[0]), TILE_GROUP_R, sides[1][7], sides[0][7], True)] = (st, pairs, plans[0])
+        plans[0]._wait()                                  # (the last kernels ran beside all this)
         return plans
 
     def _describe(self, h):
@@ -807,26 +808,28 @@ class PlanCache:
     def put_tile_plans(self, sides):
         """What get() would build one after the other for a training step on tiles, built together (DevicePlan.tile_plans; sides as
         there: the in-side, then the out-side), unless one of them is already here or they have to be built one by one.  A side that is
-        malformed is refused where it is asked for: a forward never asks for the out-side."""
+        malformed is refused where it is asked for: a forward never asks for the out-side.  True if the plans are here now because of
+        this call."""
         if self.native is None or DEVICE_BUILD is False or not sides[0][2].is_cuda:
-            return
+            return False
         keys = [self._key(side[:4], side[4], side[5], side[6], True) for side in sides]
         with self._lock:
             if any(key in self._d for key in keys):
-                return
+                return False
         try:
             plans = DevicePlan.tile_plans(sides)
         except ValueError:
             plans = None
         if plans is None:
-            return
+            return False
         self.misses += len(plans)
         with self._lock:
             if any(key in self._d for key in keys):
-                return                              # (as in get: another thread's stay)
+                return False                        # (as in get: another thread's stay)
             for key, plan, side in zip(keys, plans, sides):
                 self._insert(key, plan, side[:4])
             self._evict()
+        return True
 
     def clear(self):
         with self._lock:

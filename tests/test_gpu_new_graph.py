@@ -1,0 +1,53 @@
+"""A training call on a graph nobody has seen: both sides' plans are built with it and what both passes take is remembered, so
+that the backward of that very call is served by the native host path; results are those of the Python functions."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def new_graph(lengths, device=DEV):
+    from bpt_amd import graphbuilder as gb
+    src, dst, _, _, n = gb.merge_graphs_device([gb.BinaryPartition(m, True, 4, 10) for m in lengths], torch.device(device))
+    out_csr, in_csr, row, ir, col, ic = gb.get_csrs_device(src, dst, n)
+    return (row, ir, out_csr[2], out_csr[1], col, ic, in_csr[2], in_csr[1]), n
+
+
+@pytest.mark.parametrize("heads,d,dtype,p", [(8, 64, torch.float32, 0.0), (16, 64, torch.bfloat16, 0.1), (6, 50, torch.float32, 0.1)])
+def test_first_backward_of_a_new_graph_is_served_natively(heads, d, dtype, p, monkeypatch):
+    from bpt_amd import graphop, op, plan
+    plan.plan_cache.clear()
+    args, n = new_graph([700, 300, 65])
+    gen = torch.Generator(device=DEV).manual_seed(5)
+    q, k, v, do = (torch.randn(n, heads, d, generator=gen, device=DEV).to(dtype) for _ in range(4))
+    leaves = [x.requires_grad_(True) for x in (q, k, v)]
+    o = op.bpt_attention(*args, *leaves, dropout_p=p, seed=3)
+
+    def not_here(*a, **kw):
+        raise AssertionError("the backward went through Python")
+
+    with monkeypatch.context() as m:
+        m.setattr(graphop, "attention_backward", not_here)
+        m.setattr(graphop, "attention_backward_narrow", not_here)
+        first = (o.detach(),) + torch.autograd.grad(o, leaves, do)
+    # the same through plans that are built one by one when they are asked for
+    plan.plan_cache.clear()
+    monkeypatch.setattr(graphop, "prepare_training", lambda *a, **kw: None)
+    o = op.bpt_attention(*args, *leaves, dropout_p=p, seed=3)
+    for name, a, b in zip(("o", "dq", "dk", "dv"), first, (o.detach(),) + torch.autograd.grad(o, leaves, do)):
+        assert torch.equal(a, b), name
+
+
+def test_a_malformed_out_side_is_refused_by_the_backward_only():
+    from bpt_amd import op, plan
+    plan.plan_cache.clear()
+    args, n = new_graph([700, 300, 65])
+    bad = list(args)
+    bad[3] = args[3].clone()
+    bad[3][5] = n + 7                                              # an out-side neighbour that does not exist
+    q, k, v = (torch.randn(n, 8, 64, device=DEV, requires_grad=True) for _ in range(3))
+    o = op.bpt_attention(*bad, q, k, v)
+    with pytest.raises(ValueError):
+        o.sum().backward()
