@@ -631,6 +631,216 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_bwd_seg_finish(bpt_plan P, co
     }
 }
 
+// The same for 4, 8 or 16 heads in float32 or bfloat16 with four heads a lane (16 bytes of a float32 record): 8 Q lanes an item,
+// Q = H / 4, so a wavefront works on 8 / Q items at a time and an item of 64 edges is read with eight loads in flight a lane.  The
+// kernels above give every item a wavefront, in 2.1 rounds of wavefronts at L = 8192, k = 4, and three memory instructions to every
+// 64 / H slots of a row of 5 as of 64.  Two launches: the first finishes whole rows and leaves (m, s) of the segments of split rows, the
+// second forms a split row's result from its segments and its edges, several blocks a row.  8 heads, 430 k edges, 16 383 rows:
+// forward 20.2 + 4.4 + 9.2 -> 15.3 + 8.0 us, backward 19.1 + 4.9 + 11.3 -> 19.8 + 8.0: what is left are the 128-byte lines around the
+// 32-byte records (208 k lines a tensor where 108 k would hold them: an in-row's edge ids are neighbours by twos).
+template <typename T> struct Quad;                    // four neighbouring heads
+template <> struct Quad<float> {
+    static __device__ __forceinline__ void ld(const float *p, float (&v)[4]) {
+        const float4 x = *reinterpret_cast<const float4 *>(p);
+        v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+    }
+    static __device__ __forceinline__ void st(float *p, const float (&v)[4]) { *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]); }
+};
+template <> struct Quad<bf16_t> {
+    static __device__ __forceinline__ void ld(const bf16_t *p, float (&v)[4]) {
+        const uint2 x = *reinterpret_cast<const uint2 *>(p);
+        v[0] = __uint_as_float(x.x << 16); v[1] = __uint_as_float(x.x & 0xffff0000u);
+        v[2] = __uint_as_float(x.y << 16); v[3] = __uint_as_float(x.y & 0xffff0000u);
+    }
+    static __device__ __forceinline__ void st(bf16_t *p, const float (&v)[4]) {
+        *reinterpret_cast<uint2 *>(p) = make_uint2((uint32_t)f32_to_bf16(v[0]) | ((uint32_t)f32_to_bf16(v[1]) << 16),
+                                                   (uint32_t)f32_to_bf16(v[2]) | ((uint32_t)f32_to_bf16(v[3]) << 16));
+    }
+};
+
+// over the slots of an item: the 8 Q lanes that share it, those of one quad of heads
+template <int Q, bool IS_MAX> __device__ __forceinline__ void quad_reduce(float (&v)[4]) {
+#pragma unroll
+    for (int off = Q; off < 8 * Q; off <<= 1)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float o = __shfl_xor(v[i], off);
+            v[i] = IS_MAX ? (v[i] > o ? v[i] : o) : v[i] + o;
+        }
+}
+
+// an item for every 8 Q lanes: eight slots a load, QUAD_U loads in flight (64 slots: an item of the usual length at once)
+constexpr int QUAD_SLOTS = 8, QUAD_U = 8;
+template <int Q> __device__ __forceinline__ bool fetch_quad_item(const bpt_plan &P, Item &it) {
+    const int64_t w = ((int64_t)xcd_contiguous_block() * BLOCK + threadIdx.x) / (QUAD_SLOTS * Q);
+    if (w >= P.n_items) return false;
+    const int4 v = reinterpret_cast<const int4 *>(P.items)[w];
+    it = Item{v.x, v.y, v.z, v.w};
+    return true;
+}
+// ids of this lane's slots p, p + step, ...: -1 past the end of the range
+template <int U> __device__ __forceinline__ void quad_eids(const bpt_plan &P, int p, int step, int end, int (&e)[U]) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) e[u] = p + u * step < end ? P.eid[p + u * step] : -1;
+}
+
+template <typename T, int Q>
+__global__ __launch_bounds__(BLOCK) void k_softmax_fwd_quads(bpt_plan P, const T *__restrict__ x, T *__restrict__ y, float *__restrict__ seg) {
+    constexpr int H = 4 * Q, SL = QUAD_SLOTS, U = QUAD_U;
+    Item it;
+    if (!fetch_quad_item<Q>(P, it)) return;
+    const int lane = threadIdx.x % (SL * Q), q4 = 4 * (lane % Q), p0 = it.begin + lane / Q;
+    const bool once = it.end - it.begin <= U * SL;
+    int e[U];
+    float v[U][4], m[4] = {-1e9f, -1e9f, -1e9f, -1e9f}, s[4] = {0.f, 0.f, 0.f, 0.f};
+    auto load = [&](int p) {
+        quad_eids<U>(P, p, SL, it.end, e);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            v[u][0] = v[u][1] = v[u][2] = v[u][3] = -INFINITY;
+            if (e[u] >= 0) Quad<T>::ld(x + (size_t)e[u] * H + q4, v[u]);
+        }
+    };
+    for (int p = p0; p < it.end || p == p0; p += U * SL) {
+        load(p);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) m[i] = v[u][i] > m[i] ? v[u][i] : m[i];
+    }
+    quad_reduce<Q, true>(m);
+    for (int p = p0; p < it.end || p == p0; p += U * SL) {
+        if (!once) load(p);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { v[u][i] = expf(v[u][i] - m[i]); s[i] += v[u][i]; }       // exp(-inf) = 0 for the empty slots
+    }
+    quad_reduce<Q, false>(s);
+    if (it.slot >= 0) {
+        if (lane < Q) {
+            float *o = seg + ((size_t)it.slot * H + q4) * 2;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { o[2 * i] = m[i]; o[2 * i + 1] = s[i]; }
+        }
+        return;
+    }
+    for (int p = p0; p < it.end; p += U * SL) {
+        if (!once) {
+            load(p);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[u][i] = expf(v[u][i] - m[i]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (e[u] < 0) continue;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[u][i] = v[u][i] / s[i];
+            Quad<T>::st(y + (size_t)e[u] * H + q4, v[u]);
+        }
+    }
+}
+
+template <typename T, int Q>
+__global__ __launch_bounds__(BLOCK) void k_softmax_bwd_quads(bpt_plan P, const T *__restrict__ y, const T *__restrict__ dy, T *__restrict__ dx,
+                                                             float *__restrict__ seg) {
+    constexpr int H = 4 * Q, SL = QUAD_SLOTS, U = QUAD_U;
+    Item it;
+    if (!fetch_quad_item<Q>(P, it)) return;
+    const int lane = threadIdx.x % (SL * Q), q4 = 4 * (lane % Q), p0 = it.begin + lane / Q;
+    const bool once = it.end - it.begin <= U * SL;
+    int e[U];
+    float yv[U][4], dv[U][4], s[4] = {0.f, 0.f, 0.f, 0.f};
+    auto load = [&](int p) {
+        quad_eids<U>(P, p, SL, it.end, e);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) yv[u][i] = dv[u][i] = 0.f;
+            if (e[u] >= 0) {
+                Quad<T>::ld(y + (size_t)e[u] * H + q4, yv[u]);
+                Quad<T>::ld(dy + (size_t)e[u] * H + q4, dv[u]);
+            }
+        }
+    };
+    for (int p = p0; p < it.end || p == p0; p += U * SL) {
+        load(p);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[i] += dv[u][i] * yv[u][i];
+    }
+    quad_reduce<Q, false>(s);
+    if (it.slot >= 0) {
+        if (lane < Q) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) seg[(size_t)it.slot * H + q4 + i] = s[i];
+        }
+        return;
+    }
+    for (int p = p0; p < it.end; p += U * SL) {
+        if (!once) load(p);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (e[u] < 0) continue;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dv[u][i] = dv[u][i] * yv[u][i] - s[i] * yv[u][i];
+            Quad<T>::st(dx + (size_t)e[u] * H + q4, dv[u]);
+        }
+    }
+}
+
+// Split rows, second launch: block (i, j) is the j-th of gridDim.y blocks of split row i.  Every block reduces the row's segments
+// by itself (16 bytes a segment and head at most: they come from the L2), then writes its share of the row's edges.
+template <typename T, int Q, bool FWD>
+__global__ __launch_bounds__(BLOCK) void k_softmax_split_quads(bpt_plan P, const T *__restrict__ x, const T *__restrict__ dy, T *__restrict__ y,
+                                                               const float *__restrict__ seg) {
+    constexpr int H = 4 * Q, SL = BLOCK / Q, U = 4;               // slots of a load of the block
+    __shared__ float smem[WAVES_PER_BLOCK * WAVE];
+    __shared__ float of_head[2][H];
+    const int row = P.heavy[3 * blockIdx.x], s0 = P.heavy[3 * blockIdx.x + 1], ns = P.heavy[3 * blockIdx.x + 2];
+    const int h = threadIdx.x % H, j0 = threadIdx.x / H, nj = BLOCK / H;
+    const int begin = P.rowptr[row], deg = P.rowptr[row + 1] - begin;
+    const int per = (deg + (int)gridDim.y - 1) / (int)gridDim.y, first = begin + (int)blockIdx.y * per, end = min(first + per, begin + deg);
+    if constexpr (FWD) {
+        float m = -1e9f, s = 0.f;
+        for (int j = j0; j < ns; j += nj) { const float v = seg[((size_t)(s0 + j) * H + h) * 2]; m = v > m ? v : m; }
+        m = head_reduce<float, WAVES_PER_BLOCK, true>(m, H, h, smem);
+        for (int j = j0; j < ns; j += nj) s += seg[((size_t)(s0 + j) * H + h) * 2 + 1] * expf(seg[((size_t)(s0 + j) * H + h) * 2] - m);
+        s = head_reduce<float, WAVES_PER_BLOCK, false>(s, H, h, smem);
+        if (threadIdx.x < H) { of_head[0][h] = m; of_head[1][h] = s; }
+    } else {
+        float s = 0.f;
+        for (int j = j0; j < ns; j += nj) s += seg[(size_t)(s0 + j) * H + h];
+        s = head_reduce<float, WAVES_PER_BLOCK, false>(s, H, h, smem);
+        if (threadIdx.x < H) of_head[0][h] = s;
+    }
+    __syncthreads();
+    const int q4 = 4 * ((int)threadIdx.x % Q);
+    float a[4], b[4], v[U][4], d[U][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { a[i] = of_head[0][q4 + i]; b[i] = FWD ? of_head[1][q4 + i] : 0.f; }
+    int e[U];
+    for (int p = first + (int)threadIdx.x / Q; p < end; p += U * SL) {
+        quad_eids<U>(P, p, SL, end, e);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (e[u] >= 0) {
+                Quad<T>::ld(x + (size_t)e[u] * H + q4, v[u]);
+                if constexpr (!FWD) Quad<T>::ld(dy + (size_t)e[u] * H + q4, d[u]);
+            }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (e[u] < 0) continue;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[u][i] = FWD ? expf(v[u][i] - a[i]) / b[i] : v[u][i] * (d[u][i] - a[i]);
+            Quad<T>::st(y + (size_t)e[u] * H + q4, v[u]);
+        }
+    }
+}
+
 // ------------------------------------------------------------------------------------------
 // fast family: compile-time (H, D), f32 / bf16
 // ------------------------------------------------------------------------------------------
@@ -3997,10 +4207,43 @@ int run_spmm_generic(const bpt_plan *P, const void *W, const void *X, void *Y, v
     return launch_status();
 }
 
+// blocks of k_softmax_split_quads a split row: the longest are many times the average (16 of 127 segments at L = 8192)
+inline unsigned softmax_split_blocks(const bpt_plan *P) {
+    return (unsigned)std::min<int64_t>(64, std::max<int64_t>(16, P->n_slots / P->n_heavy));
+}
+inline unsigned softmax_item_blocks(const bpt_plan *P, int q) { return (unsigned)((P->n_items * QUAD_SLOTS * q + BLOCK - 1) / BLOCK); }
+
+template <typename T, int Q>
+int run_softmax_fwd_quads(const bpt_plan *P, const void *x, void *y, void *ws, hipStream_t s) {
+    hipLaunchKernelGGL((k_softmax_fwd_quads<T, Q>), dim3(softmax_item_blocks(P, Q)), dim3(BLOCK), 0, s, *P, (const T *)x, (T *)y, (float *)ws);
+    const int st = launch_status();
+    if (st != BPT_OK || P->n_heavy == 0) return st;
+    hipLaunchKernelGGL((k_softmax_split_quads<T, Q, true>), dim3((int)P->n_heavy, softmax_split_blocks(P)), dim3(BLOCK), 0, s, *P, (const T *)x,
+                       (const T *)nullptr, (T *)y, (const float *)ws);
+    return launch_status();
+}
+template <typename T, int Q>
+int run_softmax_bwd_quads(const bpt_plan *P, const void *y, const void *dy, void *dx, void *ws, hipStream_t s) {
+    hipLaunchKernelGGL((k_softmax_bwd_quads<T, Q>), dim3(softmax_item_blocks(P, Q)), dim3(BLOCK), 0, s, *P, (const T *)y, (const T *)dy, (T *)dx, (float *)ws);
+    const int st = launch_status();
+    if (st != BPT_OK || P->n_heavy == 0) return st;
+    hipLaunchKernelGGL((k_softmax_split_quads<T, Q, false>), dim3((int)P->n_heavy, softmax_split_blocks(P)), dim3(BLOCK), 0, s, *P, (const T *)y,
+                       (const T *)dy, (T *)dx, (const float *)ws);
+    return launch_status();
+}
+// four heads are one load: 4, 8 or 16 heads of float32 or bfloat16 in tensors that start on 16 bytes (8 would do for bfloat16)
+template <typename T> bool softmax_quads(int h, const void *a, const void *b, const void *c) {
+    return sizeof(T) != 8 && (h == 4 || h == 8 || h == 16) && aligned16(a) && aligned16(b) && aligned16(c);
+}
+
 template <typename T>
 int run_softmax_fwd(const bpt_plan *P, const void *x, void *y, void *ws, int h, hipStream_t s) {
     using acc_t = typename Elem<T>::acc_t;
     if (P->n_items == 0) return BPT_OK;
+    if constexpr (sizeof(T) != 8) {
+        if (softmax_quads<T>(h, x, y, nullptr))
+            return h == 4 ? run_softmax_fwd_quads<T, 1>(P, x, y, ws, s) : h == 8 ? run_softmax_fwd_quads<T, 2>(P, x, y, ws, s) : run_softmax_fwd_quads<T, 4>(P, x, y, ws, s);
+    }
     if (WAVE % h == 0) {       // heads side by side; split rows in three steps over their segments
         acc_t *seg = P->n_heavy > 0 ? (acc_t *)ws : nullptr;
         hipLaunchKernelGGL((k_softmax_fwd_heads<T, 1>), dim3(grid_for(P)), dim3(BLOCK), 0, s, *P, (const T *)x, (T *)y, h, seg);
@@ -4023,6 +4266,10 @@ template <typename T>
 int run_softmax_bwd(const bpt_plan *P, const void *y, const void *dy, void *dx, void *ws, int h, hipStream_t s) {
     using acc_t = typename Elem<T>::acc_t;
     if (P->n_items == 0) return BPT_OK;
+    if constexpr (sizeof(T) != 8) {
+        if (softmax_quads<T>(h, y, dy, dx))
+            return h == 4 ? run_softmax_bwd_quads<T, 1>(P, y, dy, dx, ws, s) : h == 8 ? run_softmax_bwd_quads<T, 2>(P, y, dy, dx, ws, s) : run_softmax_bwd_quads<T, 4>(P, y, dy, dx, ws, s);
+    }
     if (WAVE % h == 0) {       // heads side by side; split rows in three steps over their segments
         acc_t *seg = P->n_heavy > 0 ? (acc_t *)ws : nullptr;
         hipLaunchKernelGGL((k_softmax_bwd_heads<T, 1>), dim3(grid_for(P)), dim3(BLOCK), 0, s, *P, (const T *)y, (const T *)dy, (T *)dx, h, seg);
