@@ -972,6 +972,44 @@ __device__ __forceinline__ void issue_loads_first() { __builtin_amdgcn_sched_bar
 // weight loads for the fast SpMM: the unfused API passes T-typed edge data, the fused backward f32
 template <typename WT> __device__ __forceinline__ float ld_w(const WT *p) { return Elem<WT>::ld(p); }
 
+// NW wavefronts (a workgroup) share an item: each takes whole batches of its edges, as many as the others, and the sums meet in
+// LDS.  False: no such item (the whole workgroup).  parts: how many wavefronts have edges (one at least).
+template <int NW, int BATCH> __device__ __forceinline__ bool fetch_item_part(const bpt_plan &P, Item &it, int &part, int &parts) {
+    part = 0;
+    parts = 1;
+    if constexpr (NW == 1) return fetch_item(P, it);
+    const int w = xcd_contiguous_block();
+    if (w >= (int)P.n_items) return false;
+    const int4 v = reinterpret_cast<const int4 *>(P.items)[w];
+    it.row = __builtin_amdgcn_readfirstlane(v.x);
+    it.begin = __builtin_amdgcn_readfirstlane(v.y);
+    it.end = __builtin_amdgcn_readfirstlane(v.z);
+    it.slot = __builtin_amdgcn_readfirstlane(v.w);
+    const int deg = it.end - it.begin, per = (deg + NW * BATCH - 1) / (NW * BATCH) * BATCH;
+    part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    parts = max(1, (deg + max(per, 1) - 1) / max(per, 1));
+    it.begin = min(it.begin + part * per, it.end);
+    it.end = min(it.begin + per, it.end);
+    return true;
+}
+
+// the wavefronts' sums of one item in the first wavefront, in their order; the others are done.  By the whole workgroup.
+template <int NW, int N> __device__ __forceinline__ bool parts_meet(float (&acc)[N], int part, int parts, int lane) {
+    if constexpr (NW > 1) {
+        __shared__ float held[NW - 1][N][WAVE];
+        if (part > 0 && part < parts) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) held[part - 1][i][lane] = acc[i];
+        }
+        __syncthreads();
+        if (part > 0) return false;
+        for (int w = 0; w < parts - 1; ++w)
+#pragma unroll
+            for (int i = 0; i < N; ++i) acc[i] += held[w][i][lane];
+    }
+    return true;
+}
+
 // y[eid[p], head] = A[row, head, :] . B[idx[p], head, :]   (MODE 1: . B[eid[p], :], B an (E, D) edge feature;
 // MODE 2: . B[idx[p], :], B a (n_index, D) table shared by the heads).  YT: element type of y.
 template <typename T, int H, int D, int BATCH, int MODE = 0, typename YT = T>
@@ -1009,13 +1047,14 @@ __global__ __launch_bounds__(BLOCK) void k_sddmm_fast(bpt_plan P, const T *__res
 
 // Y0[row] = sum_p W0[eid[p], head] * X0[idx[p]]  (and the same with W1, X1 -> Y1 when NOUT == 2);
 // MODE 1: * X0[eid[p], :], X0 an (E, D) edge feature shared by the heads
-template <typename T, typename WT, int H, int D, int BATCH, int NOUT, int MODE = 0>
-__global__ __launch_bounds__(BLOCK) void k_spmm_fast(bpt_plan P, const WT *__restrict__ W0, const T *__restrict__ X0, T *__restrict__ Y0,
+template <typename T, typename WT, int H, int D, int BATCH, int NOUT, int MODE = 0, int NW = 1>
+__global__ __launch_bounds__(NW == 1 ? BLOCK : NW * WAVE) void k_spmm_fast(bpt_plan P, const WT *__restrict__ W0, const T *__restrict__ X0, T *__restrict__ Y0,
                                                      const WT *__restrict__ W1, const T *__restrict__ X1, T *__restrict__ Y1,
                                                      float *__restrict__ ws0, float *__restrict__ ws1) {
     using L = Lay<T, H, D>;
     Item it;
-    if (!fetch_item(P, it)) return;
+    int part, parts;
+    if (!fetch_item_part<NW, BATCH>(P, it, part, parts)) return;
     const int lane = threadIdx.x & 63, head = lane / L::LPH;
     float acc0[L::EPL], acc1[L::EPL];
 #pragma unroll
@@ -1050,6 +1089,20 @@ __global__ __launch_bounds__(BLOCK) void k_spmm_fast(bpt_plan P, const WT *__res
                     if constexpr (NOUT == 2) acc1[i] = fmaf(w1[e], x1[e][i], acc1[i]);
                 }
             }
+        }
+    }
+    if constexpr (NW > 1) {
+        float both[NOUT * L::EPL];
+#pragma unroll
+        for (int i = 0; i < L::EPL; ++i) {
+            both[i] = acc0[i];
+            if constexpr (NOUT == 2) both[L::EPL + i] = acc1[i];
+        }
+        if (!parts_meet<NW>(both, part, parts, lane)) return;
+#pragma unroll
+        for (int i = 0; i < L::EPL; ++i) {
+            acc0[i] = both[i];
+            if constexpr (NOUT == 2) acc1[i] = both[L::EPL + i];
         }
     }
     if (it.slot < 0) {
@@ -1097,14 +1150,15 @@ __global__ __launch_bounds__(BLOCK) void k_nme_dB_fast(bpt_plan P, const T *__re
 }
 
 // Fused forward: per destination row, online softmax over the in-edges in batches of BATCH.
-// Scores are kept in base-2 units (q is pre-multiplied by scale*log2(e)).
-template <typename T, int H, int D, int BATCH>
-__global__ __launch_bounds__(BLOCK) void k_attn_fwd(bpt_plan P, const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v,
+// Scores are kept in base-2 units (q is pre-multiplied by scale*log2(e)).  NW: wavefronts a row (row_parts).
+template <typename T, int H, int D, int BATCH, int NW = 1>
+__global__ __launch_bounds__(NW == 1 ? BLOCK : NW * WAVE) void k_attn_fwd(bpt_plan P, const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v,
                                                     T *__restrict__ o, float *__restrict__ lse, float *__restrict__ ws_acc,
                                                     float *__restrict__ ws_ml, float scale_log2e) {
     using L = Lay<T, H, D>;
     Item it;
-    if (!fetch_item(P, it)) return;
+    int part, parts;
+    if (!fetch_item_part<NW, BATCH>(P, it, part, parts)) return;
     const int lane = threadIdx.x & 63, head = lane / L::LPH;
     float qv[L::EPL], acc[L::EPL];
     load_row<T, H, D>(q + (size_t)it.row * L::C, lane, qv);
@@ -1141,6 +1195,25 @@ __global__ __launch_bounds__(BLOCK) void k_attn_fwd(bpt_plan P, const T *__restr
 #pragma unroll
                 for (int i = 0; i < L::EPL; ++i) acc[i] = fmaf(pe, vv[e][i], acc[i]);
             }
+            m = mx;
+        }
+    }
+    if constexpr (NW > 1) {
+        __shared__ float held[NW - 1][L::EPL + 2][WAVE];
+        if (part > 0 && part < parts) {
+#pragma unroll
+            for (int i = 0; i < L::EPL; ++i) held[part - 1][i][lane] = acc[i];
+            held[part - 1][L::EPL][lane] = m;
+            held[part - 1][L::EPL + 1][lane] = l;
+        }
+        __syncthreads();
+        if (part > 0) return;
+        for (int w = 0; w < parts - 1; ++w) {
+            const float mw = held[w][L::EPL][lane], mx = fmaxf(m, mw);
+            const float a = __builtin_amdgcn_exp2f(m - mx), b = __builtin_amdgcn_exp2f(mw - mx);
+            l = fmaf(b, held[w][L::EPL + 1][lane], a * l);
+#pragma unroll
+            for (int i = 0; i < L::EPL; ++i) acc[i] = fmaf(b, held[w][i][lane], a * acc[i]);
             m = mx;
         }
     }
@@ -1227,14 +1300,15 @@ __global__ __launch_bounds__(BLOCK) void k_attn_fwd_combine(const int32_t *__res
 
 // Fused backward, destination side: recompute p from lse, delta = dO.O, ds = p*(dO.v - delta)*scale,
 // dQ[row] = sum ds*k; p and ds go to (E, H) f32 buffers addressed by edge id for the source-side pass.
-template <typename T, int H, int D, int BATCH>
-__global__ __launch_bounds__(BLOCK) void k_attn_bwd_dst(bpt_plan P, const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v,
+template <typename T, int H, int D, int BATCH, int NW = 1>
+__global__ __launch_bounds__(NW == 1 ? BLOCK : NW * WAVE) void k_attn_bwd_dst(bpt_plan P, const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v,
                                                         const T *__restrict__ o, const T *__restrict__ d_o, const float *__restrict__ lse,
                                                         T *__restrict__ dq, float *__restrict__ pbuf, float *__restrict__ dsbuf,
                                                         float *__restrict__ ws_dq, float scale, float scale_log2e) {
     using L = Lay<T, H, D>;
     Item it;
-    if (!fetch_item(P, it)) return;
+    int part, parts;
+    if (!fetch_item_part<NW, BATCH>(P, it, part, parts)) return;
     const int lane = threadIdx.x & 63, head = lane / L::LPH;
     float qv[L::EPL], dov[L::EPL], dqa[L::EPL];
     float delta;
@@ -1280,6 +1354,7 @@ __global__ __launch_bounds__(BLOCK) void k_attn_bwd_dst(bpt_plan P, const T *__r
             }
         }
     }
+    if (!parts_meet<NW>(dqa, part, parts, lane)) return;
     if (it.slot < 0) store_row<T, H, D>(dq + (size_t)it.row * L::C, lane, dqa);
     else store_row_ws<T, H, D>(ws_dq + (size_t)it.slot * L::C, lane, dqa);
 }
@@ -4318,6 +4393,13 @@ int spmm_edge_generic(const bpt_plan *P, const void *W, const void *X, void *Y, 
 }
 
 // ---- fast launchers ----
+// Wavefronts a work item for the kernels that walk single rows.  They run graphs of fewer than 1536 items, and there a launch lasts
+// as long as its longest item: 16 batches of four edges one after the other, each a round trip to memory.  Forward / destination
+// side / source side, one -> four -> eight wavefronts an item, us: L = 64 (127 items) 9.4 / 13.7 / 7.2 -> 4.7 / 6.4 / 4.2 -> 4.8 / 5.6 / 4.2;
+// L = 256, k = 16 (539) 11.1 / 16.6 / 14.4 -> 9.2 / 11.7 / 11.6 -> 8.2 / 9.4 / 10.8; bfloat16, L = 256 (516) 12.2 / 16.9 / 15.5 -> 6.0 / 7.3 /
+// 7.4 -> 5.6 / 6.6 / 7.4; L = 400 (816) 11.4 / 16.6 / 13.8 -> 7.9 / 10.0 / 11.0 -> 9.0 / 10.4 / 10.5; L = 700, k = 1 (1434) 15.7 / 21.2 /
+// 15.0 -> 10.1 / 12.0 / 12.2 -> 11.3 / 12.8 / 12.6.  Larger launches fill the GPU with a wavefront an item.
+inline int row_parts(const bpt_plan *P) { return P->n_items <= 640 ? 8 : P->n_items <= 2048 ? 4 : 1; }
 template <typename T, int H, int D>
 int run_sddmm_fast(const bpt_plan *P, const void *A, const void *B, void *y, hipStream_t s) {
     if (P->n_items == 0) return BPT_OK;
@@ -4332,8 +4414,16 @@ int run_spmm_fast(const bpt_plan *P, const void *W0, const void *X0, void *Y0, c
     float *ws1 = ws ? ws + (size_t)P->n_slots * H * D : nullptr;
     {
         ProfScope prof(NOUT == 2 ? BPT_KERNEL_ATTN_BWD_SRC : -1, s);
-        hipLaunchKernelGGL((k_spmm_fast<T, WT, H, D, FAST_BATCH, NOUT>), dim3(grid_for(P)), dim3(BLOCK), 0, s, *P, (const WT *)W0,
-                           (const T *)X0, (T *)Y0, (const WT *)W1, (const T *)X1, (T *)Y1, ws, ws1);
+#define LAUNCH_SPMM(NW)                                                                                                                  \
+    hipLaunchKernelGGL((k_spmm_fast<T, WT, H, D, FAST_BATCH, NOUT, 0, NW>), dim3(NW == 1 ? grid_for(P) : (int)P->n_items),                    \
+                       dim3(NW == 1 ? BLOCK : NW * WAVE), 0, s, *P, (const WT *)W0, (const T *)X0, (T *)Y0, (const WT *)W1, (const T *)X1, \
+                       (T *)Y1, ws, ws1)
+        switch (row_parts(P)) {
+        case 8: LAUNCH_SPMM(8); break;
+        case 4: LAUNCH_SPMM(4); break;
+        default: LAUNCH_SPMM(1); break;
+        }
+#undef LAUNCH_SPMM
     }
     int st = launch_status();
     if (st != BPT_OK || P->n_heavy == 0) return st;
@@ -4826,8 +4916,15 @@ int run_attn_fwd(const bpt_plan *P, const void *q, const void *k, const void *v,
 #undef LAUNCH_FWD
 #undef LAUNCH_FWD_MFMA
         } else {
-            hipLaunchKernelGGL((k_attn_fwd<T, H, D, FAST_BATCH>), dim3(grid_for(P)), dim3(BLOCK), 0, s, *P, (const T *)q, (const T *)k,
-                               (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E);
+#define LAUNCH_FWD_ROWS(NW)                                                                                                           \
+    hipLaunchKernelGGL((k_attn_fwd<T, H, D, FAST_BATCH, NW>), dim3(NW == 1 ? grid_for(P) : (int)P->n_items), dim3(NW == 1 ? BLOCK : NW * WAVE), \
+                       0, s, *P, (const T *)q, (const T *)k, (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E)
+            switch (row_parts(P)) {
+            case 8: LAUNCH_FWD_ROWS(8); break;
+            case 4: LAUNCH_FWD_ROWS(4); break;
+            default: LAUNCH_FWD_ROWS(1); break;
+            }
+#undef LAUNCH_FWD_ROWS
         }
     launched:;
     }
@@ -4984,9 +5081,16 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
             }
 #undef LAUNCH_DST
         } else {
-            hipLaunchKernelGGL((k_attn_bwd_dst<T, H, D, FAST_BATCH>), dim3(grid_for(Pin)), dim3(BLOCK), 0, s, *Pin, (const T *)q,
-                               (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pbuf, dsbuf, ws_rows, scale,
-                               scale * LOG2E);
+#define LAUNCH_DST_ROWS(NW)                                                                                                              \
+    hipLaunchKernelGGL((k_attn_bwd_dst<T, H, D, FAST_BATCH, NW>), dim3(NW == 1 ? grid_for(Pin) : (int)Pin->n_items),                         \
+                       dim3(NW == 1 ? BLOCK : NW * WAVE), 0, s, *Pin, (const T *)q, (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, \
+                       (T *)dq, pbuf, dsbuf, ws_rows, scale, scale * LOG2E)
+            switch (row_parts(Pin)) {
+            case 8: LAUNCH_DST_ROWS(8); break;
+            case 4: LAUNCH_DST_ROWS(4); break;
+            default: LAUNCH_DST_ROWS(1); break;
+            }
+#undef LAUNCH_DST_ROWS
         }
     }
     int st = launch_status();
