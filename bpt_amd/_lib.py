@@ -74,6 +74,8 @@ ATTN_API = {
                                              c_i64, ctypes.c_float, ctypes.c_float, ctypes.c_uint64] + _tail),
     "bpt_attention_forward_narrow": (ctypes.c_int, [_PP, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, ctypes.c_float, ctypes.c_float,
                                                    ctypes.c_uint64, ctypes.c_int] + _tail),
+    "bpt_attention_forward_narrow_keep": (ctypes.c_int, [_PP, c_vp, c_vp, c_vp, c_vp, c_vp, ctypes.POINTER(c_vp * 4), c_i64, c_i64, c_vp, c_i64,
+                                                        ctypes.c_float, ctypes.c_float, ctypes.c_uint64, ctypes.c_int] + _tail),
     "bpt_attention_backward_narrow": (ctypes.c_int, [_PP, _PP, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64,
                                                     ctypes.c_float, ctypes.c_float, ctypes.c_uint64, ctypes.c_int] + _tail),
 }

@@ -196,13 +196,76 @@ __global__ __launch_bounds__(BLOCK) void k_spmm_generic(bpt_plan P, const T *__r
 // twice with one value.  No other head's memory is touched, so what stands there does not matter.
 // Against copies padded to 64 columns and 4, 8 or 16 heads (three pads, the output and its gradient, three slices, and the
 // padding heads computed with the rest): 33 765 nodes / 576 k edges at 6 x 50 with dropout, forward and backward,
-// 508 -> 266 us, of which 60 are plain copies of q, k, v and o for the backward (bptop.cpp, own_rows); of the 508 copies were
-// 223, the rest two padding heads of eight.
+// 508 -> 253 us, of which 38 are copies of q, k, v and o for the backward (Keep); of the 508 copies were 223, the rest two
+// padding heads of eight.
 struct Narrow {
     int d, heads;              // columns of a head, heads
     int h;                     // heads the layer is padded to where that shows: dropout keys, lse and workspace rows
     int slices;                // workgroups per group
 };
+
+// Copies that a NARROW forward writes beside its result, for a backward whose caller may have written to the rows in the meantime:
+// q, k and v by workgroups of the forward's own launch that do nothing else, spread evenly between those of the tiles, and the
+// result where it is stored.  The forward waits for its gathers and products and leaves much of the memory's rate unused.  Training
+// pass at 33 765 nodes, 6 x 50 float32 with dropout: 265.1 us with four copies of their own behind the forward (62 us of them),
+// 252.7 so, 215 with none; the copying workgroups first or last, or with loads past the L2, 253.8 to 256.5; stored the ordinary way,
+// into the L2 that the tiles' rows want, 265.
+struct Keep {
+    const char *src[3];
+    char *dst[3];              // on 16 bytes; null: no copy of this one (bytes = 0)
+    int64_t bytes[3];
+    int per_xcd;               // copying workgroups per XCD
+    void *o;                   // second copy of the result, or null
+};
+constexpr int KEEP_CHUNK = 16384;          // bytes a workgroup copies
+
+typedef float floatx4k __attribute__((ext_vector_type(4), aligned(4)));
+typedef float floatx4n __attribute__((ext_vector_type(4)));
+// What workgroup blockIdx.x of a launch with copying workgroups among it is to do: the number of its tile workgroup, or -1 after it
+// has copied its chunk.
+template <int THREADS> __device__ __forceinline__ int keep_or_tile(const Keep &keep) {
+    if (keep.per_xcd == 0) return (int)blockIdx.x;
+    const uint32_t x = blockIdx.x & 7, w = blockIdx.x >> 3, all = gridDim.x >> 3, c = (uint32_t)keep.per_xcd;
+    const uint32_t before = (uint32_t)((uint64_t)w * c / all), upto = (uint32_t)((uint64_t)(w + 1) * c / all);
+    if (before == upto) return (int)((w - before) * 8 + x);
+    // (chosen by conditions, not by an index: indexed, the arguments would be copied to scratch memory by every wavefront)
+    int64_t at = (int64_t)(before * 8 + x) * KEEP_CHUNK, left = keep.bytes[0];
+    const char *src = keep.src[0];
+    char *dst = keep.dst[0];
+#pragma unroll
+    for (int i = 1; i < 3; ++i) {
+        const int64_t past = at - (left + KEEP_CHUNK - 1) / KEEP_CHUNK * KEEP_CHUNK;
+        if (past >= 0) { at = past; left = keep.bytes[i]; src = keep.src[i]; dst = keep.dst[i]; }
+        else break;
+    }
+    src += at;
+    dst += at;
+    left -= at;
+    constexpr int U = 4;                                          // loads in flight
+    const floatx4k *from = reinterpret_cast<const floatx4k *>(src) + threadIdx.x;
+    floatx4n *to = reinterpret_cast<floatx4n *>(dst) + threadIdx.x;
+    const int n = (int)min((int64_t)KEEP_CHUNK, max(left, (int64_t)0)) / 16;       // whole 16-byte pieces
+    if (n == KEEP_CHUNK / 16) {
+#pragma unroll 1
+        for (int i = 0; i < KEEP_CHUNK / 16; i += U * THREADS) {
+            floatx4k v[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[u] = from[i + u * THREADS];
+#pragma unroll
+            for (int u = 0; u < U; ++u) __builtin_nontemporal_store(floatx4n{v[u][0], v[u][1], v[u][2], v[u][3]}, to + (i + u * THREADS));
+        }
+        return -1;
+    }
+    // the last chunk of a tensor, and what is left of no whole number of 16 bytes (up to seven bfloat16)
+#pragma unroll 1
+    for (int i = threadIdx.x; i < n; i += THREADS) {
+        const floatx4k v = reinterpret_cast<const floatx4k *>(src)[i];
+        reinterpret_cast<floatx4n *>(dst)[i] = floatx4n{v[0], v[1], v[2], v[3]};
+    }
+    const int64_t end = 16 * (int64_t)n + 2 * (int)threadIdx.x;
+    if (end + 2 <= left) *reinterpret_cast<uint16_t *>(dst + end) = *reinterpret_cast<const uint16_t *>(src + end);
+    return -1;
+}
 constexpr int NARROW_HW = 2;   // heads per workgroup (6 x 50: three workgroups of two, none of them half empty)
 __device__ __forceinline__ int narrow_col(const Narrow &nw, int quad) { return min(4 * quad, nw.d - 4); }
 // whether column e of the quad as loaded is one that the quad before has (or, past the end of the head, any): 4 quad > d - 4 + e
@@ -1238,7 +1301,7 @@ __global__ __launch_bounds__(NW == 1 ? BLOCK : NW * WAVE) void k_attn_fwd(bpt_pl
 template <typename T, int HC, int D, bool NARROW = false>
 __global__ __launch_bounds__(BLOCK) void k_attn_fwd_combine(const int32_t *__restrict__ heavy, const float *__restrict__ ws_acc,
                                                             const float *__restrict__ ws_ml, T *__restrict__ o, float *__restrict__ lse,
-                                                            Narrow nw) {
+                                                            Narrow nw, T *__restrict__ o_keep = nullptr) {
     static_assert(HC * D % WAVE == 0, "strip width");
     const int H = NARROW ? nw.h : HC, C = H * D;                 // (NARROW: one strip per real head)
     __shared__ float pm[WAVES_PER_BLOCK][WAVE], pl[WAVES_PER_BLOCK][WAVE], pa[WAVES_PER_BLOCK][WAVE];
@@ -1293,7 +1356,10 @@ __global__ __launch_bounds__(BLOCK) void k_attn_fwd_combine(const int32_t *__res
             A = fmaf(pa[i][lane], wgt, A);
         }
         if (!NARROW) Elem<T>::st(o + (size_t)row * C + j, L > 0.f ? A / L : 0.f);
-        else if (lane < nw.d) Elem<T>::st(o + (size_t)row * (nw.heads * nw.d) + head * nw.d + lane, L > 0.f ? A / L : 0.f);
+        else if (lane < nw.d) {
+            Elem<T>::st(o + (size_t)row * (nw.heads * nw.d) + head * nw.d + lane, L > 0.f ? A / L : 0.f);
+            if (o_keep) Elem<T>::st(o_keep + (size_t)row * (nw.heads * nw.d) + head * nw.d + lane, L > 0.f ? A / L : 0.f);
+        }
         if (j % D == 0) lse[(size_t)row * H + head] = L > 0.f ? Mx + log2f(L) : 0.f;
     }
 }
@@ -2000,7 +2066,7 @@ struct TileCtx {
 };
 
 template <typename T, int H, int D, int HW, bool NARROW = false, int SP = 1>
-__device__ __forceinline__ bool tile_begin(const bpt_plan &P, TileCtx &t, const Narrow &nw) {
+__device__ __forceinline__ bool tile_begin(const bpt_plan &P, TileCtx &t, const Narrow &nw, unsigned block = blockIdx.x) {
     static_assert(D == 64 && (H * SP) % HW == 0 && HW % SP == 0 && (sizeof(T) == 4 || sizeof(T) == 2), "64 columns per head: one 16-column slice per lane group");
     static_assert(!NARROW || SP == 1 || SP == HW, "heads a workgroup has past the last one leave its barrier alone");
     constexpr int HEADS = HW / SP;
@@ -2009,7 +2075,7 @@ __device__ __forceinline__ bool tile_begin(const bpt_plan &P, TileCtx &t, const 
     t.wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     t.c = t.lane & 15;
     t.g = t.lane >> 4;
-    const int x = blockIdx.x & 7, w = (int)(blockIdx.x >> 3) / HS;
+    const int x = block & 7, w = (int)(block >> 3) / HS;
     const int grp = __builtin_amdgcn_readfirstlane(P.grp_chunks[x]) + w;
     if (grp >= __builtin_amdgcn_readfirstlane(P.grp_chunks[x + 1])) return false;
     t.member = reinterpret_cast<const int2 *>(P.grp_members)[(size_t)grp * TILE_R + t.c];
@@ -2021,7 +2087,7 @@ __device__ __forceinline__ bool tile_begin(const bpt_plan &P, TileCtx &t, const 
         t.p_begin = min(t.p_begin + t.part * per, t.p_end);
         t.p_end = min(t.p_begin + per, t.p_end);
     }
-    t.head = (int)((blockIdx.x >> 3) % HS) * HEADS + (SP > 1 ? t.wv % HEADS : t.wv);
+    t.head = (int)((block >> 3) % HS) * HEADS + (SP > 1 ? t.wv % HEADS : t.wv);
     if (NARROW) {
         if (t.head >= nw.heads) return false;
         t.offa = (uint32_t)(t.head * nw.d * sizeof(T));
@@ -2136,7 +2202,7 @@ __device__ __forceinline__ void tile_axpy_upto(const float (&w)[4], const float4
 // 47 -> 55 us for the source side of L = 8192; on the loads of the members' rows: destination side 58 -> 61.6.
 template <int H, int D, bool SCALE, bool NARROW, typename T>
 __device__ __forceinline__ void tile_store_row(const TileCtx &t, int r, float4 x, float inv_c, T *__restrict__ out, float *__restrict__ ws,
-                                               const Narrow &nw) {
+                                               const Narrow &nw, T *__restrict__ also = nullptr) {      // also (NARROW): second copy of whole rows
     const int m = 4 * t.g + r;                                    // the member whose row this lane stores a piece of
     const int row = lane_bcast(t.member.x, m), slot = lane_bcast(t.member.y, m);
     const float inv = SCALE ? lane_bcast(inv_c, m) : 1.f;
@@ -2146,13 +2212,17 @@ __device__ __forceinline__ void tile_store_row(const TileCtx &t, int r, float4 x
         if (SCALE) { x.x *= inv; x.y *= inv; x.z *= inv; x.w *= inv; }
         T *const at = NARROW ? out + (size_t)row * (uint32_t)(nw.heads * nw.d) + t.head * nw.d + col : out + (size_t)row * (H * D) + t.head * D + col;
         if constexpr (sizeof(T) == 4) {
-            if constexpr (NARROW) *reinterpret_cast<floatx4u *>(at) = floatx4u{x.x, x.y, x.z, x.w};
-            else __builtin_nontemporal_store(floatx4v{x.x, x.y, x.z, x.w}, reinterpret_cast<floatx4v *>(at));
+            if constexpr (NARROW) {
+                *reinterpret_cast<floatx4u *>(at) = floatx4u{x.x, x.y, x.z, x.w};
+                if (also) *reinterpret_cast<floatx4u *>(also + (at - out)) = floatx4u{x.x, x.y, x.z, x.w};
+            } else __builtin_nontemporal_store(floatx4v{x.x, x.y, x.z, x.w}, reinterpret_cast<floatx4v *>(at));
         } else {
             const uint2 y = make_uint2(((uint32_t)f32_to_bf16(x.x)) | ((uint32_t)f32_to_bf16(x.y) << 16),
                            ((uint32_t)f32_to_bf16(x.z)) | ((uint32_t)f32_to_bf16(x.w) << 16));
-            if constexpr (NARROW) *reinterpret_cast<uintx2u *>(at) = uintx2u{y.x, y.y};
-            else __builtin_nontemporal_store(uintx2v{y.x, y.y}, reinterpret_cast<uintx2v *>(at));
+            if constexpr (NARROW) {
+                *reinterpret_cast<uintx2u *>(at) = uintx2u{y.x, y.y};
+                if (also) *reinterpret_cast<uintx2u *>(also + (at - out)) = uintx2u{y.x, y.y};
+            } else __builtin_nontemporal_store(uintx2v{y.x, y.y}, reinterpret_cast<uintx2v *>(at));
         }
     } else {
         float *const at = ws + (size_t)slot * (NARROW ? nw.h * D : H * D) + t.head * D + col;
@@ -2162,10 +2232,10 @@ __device__ __forceinline__ void tile_store_row(const TileCtx &t, int r, float4 x
 }
 template <int H, int D, bool SCALE, bool NARROW, typename T>
 __device__ __forceinline__ void tile_store_rows(const TileCtx &t, const floatx4v (&acc)[4], float inv_c, T *__restrict__ out,
-                                                float *__restrict__ ws, const Narrow &nw) {
+                                                float *__restrict__ ws, const Narrow &nw, T *__restrict__ also = nullptr) {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-        tile_store_row<H, D, SCALE, NARROW>(t, r, make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]), inv_c, out, ws, nw);
+        tile_store_row<H, D, SCALE, NARROW>(t, r, make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]), inv_c, out, ws, nw, also);
 }
 
 // SP > 1: SP wavefronts of a workgroup share a tile and head, each walks a contiguous SP-th of the tile's blocks (tile_begin),
@@ -2210,7 +2280,8 @@ __device__ __forceinline__ void tile_meet_and_store(const float *part0, int stri
 constexpr int TILE_PART_FWD_FLOATS = TILE_PART_FLOATS + 2 * TILE_R;
 template <int SP, int H, int D, bool NARROW, typename T>
 __device__ __forceinline__ void tile_meet_forward(float *mine, const float *part0, int stride, const TileCtx &t, const floatx4v (&acc)[4], float &mref,
-                                                  float &lt, T *__restrict__ out, float *__restrict__ ws, const Narrow &nw) {
+                                                  float &lt, T *__restrict__ out, float *__restrict__ ws, const Narrow &nw,
+                                                  T *__restrict__ also) {
     constexpr int RS = 4 / SP;
     tile_park(mine, acc, t.lane);
     if (t.g == 0) {
@@ -2235,7 +2306,7 @@ __device__ __forceinline__ void tile_meet_forward(float *mine, const float *part
 #pragma unroll
     for (int i = 0; i < RS; ++i) {
         const int r = t.part * RS + i;
-        tile_store_row<H, D, true, NARROW>(t, r, tile_meet<SP, true>(part0, stride, r, t, wgt), inv, out, ws, nw);
+        tile_store_row<H, D, true, NARROW>(t, r, tile_meet<SP, true>(part0, stride, r, t, wgt), inv, out, ws, nw, also);
     }
 }
 
@@ -2343,11 +2414,15 @@ template <typename T, int H, int D, int HW, bool DROP, int BIAS, bool NARROW = f
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) void k_attn_fwd_tile(
     bpt_plan P, const T *__restrict__ q, const T *__restrict__ k, const T *__restrict__ v, T *__restrict__ o, float *__restrict__ lse,
     float *__restrict__ ws_acc, float *__restrict__ ws_ml, float scale_log2e, uint32_t drop_thr, uint32_t drop_seed, float drop_inv,
-    const float *__restrict__ bias, Narrow nw) {
+    const float *__restrict__ bias, Narrow nw, Keep keep) {
     const int Hs = NARROW ? nw.h : H;                             // heads as lse, workspace and dropout keys count them
     const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * sizeof(T) : (uint32_t)(H * D * sizeof(T));        // bytes of a node row
+    int block = (int)blockIdx.x;
+    if constexpr (NARROW) block = keep_or_tile<HW * WAVE>(keep);
+    if (NARROW && block < 0) return;
+    T *const o_keep = NARROW ? reinterpret_cast<T *>(keep.o) : nullptr;
     TileCtx t;
-    if (!tile_begin<T, H, D, HW, NARROW, SP>(P, t, nw)) return;
+    if (!tile_begin<T, H, D, HW, NARROW, SP>(P, t, nw, (unsigned)block)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     __shared__ int fst_lds[HW][BIAS == 2 ? TILE_CHUNK : 1];      // the entries' first pair numbers: where a term in pair order sits
     int2 *ent = ent_lds[t.wv];
@@ -2451,10 +2526,10 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
     lt += __shfl_xor(lt, 32);                                    // denominator of member c, in its four lanes
     if constexpr (SP > 1) {
         static_assert(TILE_PART_FWD_FLOATS <= TILE_R * TILE_KT_STRIDE, "a part fits its wavefront's piece");
-        tile_meet_forward<SP, H, D, NARROW>(kt, kt_lds[t.wv % (HW / SP)], (HW / SP) * TILE_R * TILE_KT_STRIDE, t, acc, mref, lt, o, ws_acc, nw);
+        tile_meet_forward<SP, H, D, NARROW>(kt, kt_lds[t.wv % (HW / SP)], (HW / SP) * TILE_R * TILE_KT_STRIDE, t, acc, mref, lt, o, ws_acc, nw, o_keep);
         if (t.part != 0) return;
     } else {
-        tile_store_rows<H, D, true, NARROW>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc, nw);
+        tile_store_rows<H, D, true, NARROW>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc, nw, o_keep);
     }
     if (g == 0 && t.member.x >= 0) {                              // lanes 0 .. 15: one member each
         if (t.member.y < 0) {
@@ -2864,11 +2939,15 @@ template <int H, int D, int HW, int WPE, bool DROP, int BIAS, bool NARROW = fals
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))) void k_attn_fwd_tile_bf16(
     bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, bf16_t *__restrict__ o,
     float *__restrict__ lse, float *__restrict__ ws_acc, float *__restrict__ ws_ml, float scale_log2e, uint32_t drop_thr,
-    uint32_t drop_seed, float drop_inv, const float *__restrict__ bias, Narrow nw) {
+    uint32_t drop_seed, float drop_inv, const float *__restrict__ bias, Narrow nw, Keep keep) {
     const int Hs = NARROW ? nw.h : H;                             // heads as lse, workspace and dropout keys count them
     const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * 2 : (uint32_t)(H * D * 2);                       // bytes of a node row
+    int block = (int)blockIdx.x;
+    if constexpr (NARROW) block = keep_or_tile<HW * WAVE>(keep);
+    if (NARROW && block < 0) return;
+    bf16_t *const o_keep = NARROW ? reinterpret_cast<bf16_t *>(keep.o) : nullptr;
     TileCtx t;
-    if (!tile_begin<bf16_t, H, D, HW, NARROW, SP>(P, t, nw)) return;
+    if (!tile_begin<bf16_t, H, D, HW, NARROW, SP>(P, t, nw, (unsigned)block)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     __shared__ int fst_lds[HW][BIAS == 2 ? TILE_CHUNK : 1];      // the entries' first pair numbers: where a term in pair order sits
     int2 *ent = ent_lds[t.wv];
@@ -2970,10 +3049,10 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     float lt = lrun + __shfl_xor(lrun, 16);
     lt += __shfl_xor(lt, 32);
     if constexpr (SP > 1) {
-        tile_meet_forward<SP, H, D, NARROW>(piece[t.wv], piece[t.wv % (HW / SP)], (HW / SP) * PIECE, t, acc, mref, lt, o, ws_acc, nw);
+        tile_meet_forward<SP, H, D, NARROW>(piece[t.wv], piece[t.wv % (HW / SP)], (HW / SP) * PIECE, t, acc, mref, lt, o, ws_acc, nw, o_keep);
         if (t.part != 0) return;
     } else {
-        tile_store_rows<H, D, true, NARROW>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc, nw);
+        tile_store_rows<H, D, true, NARROW>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc, nw, o_keep);
     }
     if (g == 0 && t.member.x >= 0) {
         if (t.member.y < 0) {
@@ -4839,7 +4918,7 @@ int run_attn_fwd(const bpt_plan *P, const void *q, const void *k, const void *v,
 #define LAUNCH_FWD_TILE_PARTS(DR, BI, SP)                                                                                            \
     hipLaunchKernelGGL((k_attn_fwd_tile<T, H, D, HW, DR, BI, false, SP>), dim3(group_grid(P) * (H * SP / HW)), dim3(HW * WAVE), 0, s, *P, \
                        (const T *)q, (const T *)k, (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed, drop.inv, bias, \
-                       Narrow{})
+                       Narrow{}, Keep{})
 #define LAUNCH_FWD_TILE(DR, BI)                                                                                                      \
     do {                                                                                                                             \
         if (parts == 4) LAUNCH_FWD_TILE_PARTS(DR, BI, 4);                                                                            \
@@ -4866,7 +4945,7 @@ int run_attn_fwd(const bpt_plan *P, const void *q, const void *k, const void *v,
 #define LAUNCH_FWD_TILE_PARTS(DR, BI, SP)                                                                                                \
     hipLaunchKernelGGL((k_attn_fwd_tile_bf16<H, D, HW, TILE_BF16_WPE, DR, BI, false, SP>), dim3(group_grid(P) * (H * SP / HW)), \
                        dim3(HW * WAVE), 0, s, *P, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (bf16_t *)o, lse, ws_acc, ws_ml, \
-                       scale * LOG2E, drop.thr, drop.seed, drop.inv, bias, Narrow{})
+                       scale * LOG2E, drop.thr, drop.seed, drop.inv, bias, Narrow{}, Keep{})
 #define LAUNCH_FWD_TILE(DR, BI)                                                                                                          \
     do {                                                                                                                                 \
         if (parts == 4) LAUNCH_FWD_TILE_PARTS(DR, BI, 4);                                                                                \
@@ -4931,7 +5010,7 @@ int run_attn_fwd(const bpt_plan *P, const void *q, const void *k, const void *v,
     int st = launch_status();
     if (st != BPT_OK || P->n_heavy == 0) return st;
     hipLaunchKernelGGL((k_attn_fwd_combine<T, H, D>), dim3((int)P->n_heavy, H * D / WAVE), dim3(BLOCK), 0, s, P->heavy,
-                       (const float *)ws_acc, (const float *)ws_ml, (T *)o, lse, Narrow{});
+                       (const float *)ws_acc, (const float *)ws_ml, (T *)o, lse, Narrow{}, (T *)nullptr);
     return launch_status();
 }
 
@@ -5139,23 +5218,23 @@ inline Narrow narrow_parts(Narrow nw, int parts) {
 
 template <typename T>
 int run_attn_fwd_narrow(const bpt_plan *P, const void *q, const void *k, const void *v, void *o, float *lse, void *ws, float scale, Dropout drop,
-                        const Narrow &nw, hipStream_t s) {
-    if (P->n_items == 0) return BPT_OK;
+                        const Narrow &nw, const Keep &keep, hipStream_t s) {
     float *ws_acc = (float *)ws, *ws_ml = ws_acc ? ws_acc + (size_t)P->n_slots * nw.h * 64 : nullptr;
     const int parts = tile_parts(P, nw.heads, sizeof(T));
     const Narrow np = narrow_parts(nw, parts);
-    const dim3 grid(group_grid(P) * np.slices), block((parts == 1 ? NARROW_HW : parts) * WAVE);
+    const dim3 grid(group_grid(P) * np.slices + 8 * keep.per_xcd), block((parts == 1 ? NARROW_HW : parts) * WAVE);
+    if (grid.x == 0) return BPT_OK;
     {
         ProfScope prof(BPT_KERNEL_ATTN_FWD, s);
 #define LAUNCH_FWD_PARTS(DR, HW, SP)                                                                                                     \
     do {                                                                                                                                 \
         if constexpr (sizeof(T) == 4)                                                                                                    \
             hipLaunchKernelGGL((k_attn_fwd_tile<T, 16, 64, HW, DR, 0, true, SP>), grid, block, 0, s, *P, (const T *)q, (const T *)k,         \
-                               (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed, drop.inv, (const float *)nullptr, np); \
+                               (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed, drop.inv, (const float *)nullptr, np, keep); \
         else                                                                                                                             \
             hipLaunchKernelGGL((k_attn_fwd_tile_bf16<16, 64, HW, TILE_BF16_WPE, DR, 0, true, SP>), grid, block, 0, s, *P,                    \
                                (const T *)q, (const T *)k, (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed,       \
-                               drop.inv, (const float *)nullptr, np);                                                                      \
+                               drop.inv, (const float *)nullptr, np, keep);                                                                \
     } while (0)
 #define LAUNCH_FWD(DR)                                                                                                                   \
     do {                                                                                                                                 \
@@ -5170,7 +5249,7 @@ int run_attn_fwd_narrow(const bpt_plan *P, const void *q, const void *k, const v
     const int st = launch_status();
     if (st != BPT_OK || P->n_heavy == 0) return st;
     hipLaunchKernelGGL((k_attn_fwd_combine<T, 16, 64, true>), dim3((int)P->n_heavy, nw.heads), dim3(BLOCK), 0, s, P->heavy, (const float *)ws_acc,
-                       (const float *)ws_ml, (T *)o, lse, nw);
+                       (const float *)ws_ml, (T *)o, lse, nw, (T *)keep.o);
     return launch_status();
 }
 
@@ -5597,22 +5676,45 @@ int bpt_attention_backward(const bpt_plan *plan_in, const bpt_plan *plan_out, co
     return BPT_ERR_UNSUPPORTED;
 }
 
-int bpt_attention_forward_narrow(const bpt_plan *plan_in, const void *q, const void *k, const void *v, void *o, float *lse, void *workspace,
-                                 int64_t workspace_bytes, float scale, float dropout_p, uint64_t dropout_seed, int heads, int d, int h,
-                                 int dtype, void *stream) {
+int bpt_attention_forward_narrow_keep(const bpt_plan *plan_in, const void *q, const void *k, const void *v, void *o, float *lse, void *const keep[4],
+                                      int64_t n_q, int64_t n_k, void *workspace, int64_t workspace_bytes, float scale, float dropout_p,
+                                      uint64_t dropout_seed, int heads, int d, int h, int dtype, void *stream) {
     CHECK(check_plan(plan_in, true));
     Narrow nw;
     CHECK(narrow_shape(heads, d, h, dtype, nw));
-    if (!q || !k || !v || !o || !lse) return BPT_ERR_NULL;
+    if (!q || !k || !v || !o || !lse || !keep) return BPT_ERR_NULL;
     if (!(dropout_p >= 0.f && dropout_p < 1.f)) return BPT_ERR_SIZE;
     const Dropout drop = make_dropout(dropout_p, dropout_seed);
     if (!(dtype == BPT_F32 ? narrow_ok<float>(plan_in, nw) : narrow_ok<bf16_t>(plan_in, nw))) return BPT_ERR_UNSUPPORTED;
     if (!aligned4(q) || !aligned4(k) || !aligned4(v) || !aligned4(o) || !aligned16(workspace)) return BPT_ERR_UNSUPPORTED;
     const int64_t need = bpt_workspace_bytes(BPT_OP_ATTN_FWD, plan_in, nullptr, h, 64, dtype);
     if (need > 0 && (!workspace || workspace_bytes < need)) return BPT_ERR_WORKSPACE;
+    if (n_q < 0 || n_k < 0 || (keep[3] && !aligned4(keep[3]))) return BPT_ERR_SIZE;
+    Keep kp{};
+    int64_t chunks = 0;
+    const void *const from[3] = {q, k, v};
+    for (int i = 0; i < 3; ++i) {
+        if (!keep[i]) continue;
+        if (!aligned16(keep[i])) return BPT_ERR_UNSUPPORTED;
+        kp.src[i] = (const char *)from[i];
+        kp.dst[i] = (char *)keep[i];
+        kp.bytes[i] = (i == 0 ? n_q : n_k) * heads * d * (dtype == BPT_F32 ? 4 : 2);
+        chunks += (kp.bytes[i] + KEEP_CHUNK - 1) / KEEP_CHUNK;
+    }
+    if (chunks >= (1 << 27)) return BPT_ERR_SIZE;
+    kp.per_xcd = (int)((chunks + 7) / 8);
+    kp.o = keep[3];
     hipStream_t s = (hipStream_t)stream;
-    return dtype == BPT_F32 ? run_attn_fwd_narrow<float>(plan_in, q, k, v, o, lse, workspace, scale, drop, nw, s)
-                            : run_attn_fwd_narrow<bf16_t>(plan_in, q, k, v, o, lse, workspace, scale, drop, nw, s);
+    return dtype == BPT_F32 ? run_attn_fwd_narrow<float>(plan_in, q, k, v, o, lse, workspace, scale, drop, nw, kp, s)
+                            : run_attn_fwd_narrow<bf16_t>(plan_in, q, k, v, o, lse, workspace, scale, drop, nw, kp, s);
+}
+
+int bpt_attention_forward_narrow(const bpt_plan *plan_in, const void *q, const void *k, const void *v, void *o, float *lse, void *workspace,
+                                 int64_t workspace_bytes, float scale, float dropout_p, uint64_t dropout_seed, int heads, int d, int h,
+                                 int dtype, void *stream) {
+    void *const none[4] = {};
+    return bpt_attention_forward_narrow_keep(plan_in, q, k, v, o, lse, none, 0, 0, workspace, workspace_bytes, scale, dropout_p, dropout_seed, heads, d,
+                                             h, dtype, stream);
 }
 
 int bpt_attention_backward_narrow(const bpt_plan *plan_in, const bpt_plan *plan_out, const void *q, const void *k, const void *v, const void *o,

@@ -263,11 +263,20 @@ Tensor attention(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r,
 }
 
 // ---- fused attention with heads of fewer than 64 columns, h: the heads it is computed as if padded to -------------------------
+// keep: tensors that become copies of q, k, v and of the result (graphop._attention_forward_narrow)
+using Copies = std::array<std::optional<Tensor>, 4>;
+
 std::optional<std::tuple<Tensor, Tensor>> narrow_forward_known(const Tensor &col, const Tensor &indptr, const Tensor &eid, const Tensor &indices,
                                                                const Tensor &q, const Tensor &k, const Tensor &v, int h, double scale, double p,
-                                                               uint64_t seed) {
+                                                               uint64_t seed, const Copies &keep) {
     Shape s;
     if (!attention_shape(q, k, v, p, s) || indices.sizes() != eid.sizes()) return std::nullopt;
+    void *copies[4] = {};
+    for (size_t i = 0; i < 4; ++i) {
+        if (!keep[i]) continue;
+        if (!like(*keep[i], q) || keep[i]->sizes() != (i == 1 || i == 2 ? k : q).sizes()) return std::nullopt;
+        copies[i] = keep[i]->data_ptr();
+    }
     Key key;
     if (!make_key(key, ATTN_FWD_NARROW, {&col, &indptr, &eid, &indices}, q.device(), {s.nq, s.nk, h, s.d, s.dt, p > 0.0, s.h}))
         return std::nullopt;
@@ -276,8 +285,9 @@ std::optional<std::tuple<Tensor, Tensor>> narrow_forward_known(const Tensor &col
     c10::DeviceGuard guard(q.device());
     Tensor o = at::empty_like(q), lse = at::empty({s.nq, h}, q.options().dtype(at::kFloat));
     Workspace ws(BPT_OP_ATTN_FWD, &e->a, nullptr, h, 64, s.dt, q);
-    const int st = bpt_attention_forward_narrow(&e->a, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), (float *)lse.data_ptr(), ws.ptr,
-                                                ws.bytes, (float)scale, (float)p, seed, s.h, s.d, h, s.dt, stream_of(q.device()));
+    const int st = bpt_attention_forward_narrow_keep(&e->a, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), (float *)lse.data_ptr(), copies,
+                                                     s.nq, s.nk, ws.ptr, ws.bytes, (float)scale, (float)p, seed, s.h, s.d, h, s.dt,
+                                                     stream_of(q.device()));
     if (st != BPT_OK) return std::nullopt;
     return std::make_tuple(o, lse);
 }
@@ -314,21 +324,22 @@ Tensor rows(const Tensor &x) {
     return y.is_cuda() && (reinterpret_cast<uintptr_t>(y.data_ptr()) & 3) ? y.clone() : y;
 }
 
-// The same in memory that is nobody else's.  A backward needs the rows as the forward saw them, and a layer on padded copies let
-// its caller write to q, k, v and o after the forward (an activation or a residual in place); so does this one.  The four copies
-// take 60 of 266 us at 33 765 nodes, 6 x 50 float32 with dropout, forward and backward.
-Tensor own_rows(const Tensor &x) {
-    Tensor y = rows(x);
-    return y.is_alias_of(x) ? y.clone() : y;
+// Memory for a copy of rows(x) that is nobody else's, where rows(x) is not one already.  A backward needs the rows as the forward saw
+// them, and a layer on padded copies let its caller write to q, k, v and o after the forward (an activation or a residual in
+// place); so does this one.  The forward's launches fill the copies.
+std::optional<Tensor> room_for_copy(const Tensor &x, const Tensor &rows_of_x) {
+    if (!rows_of_x.is_alias_of(x)) return std::nullopt;
+    return at::empty_like(rows_of_x);
 }
 
 // The forward is a call of graphop.attention_forward, as that of the padded copies was: q, k, v stand for the padded shape there.
 std::tuple<Tensor, Tensor> narrow_forward(const Tensor &col, const Tensor &indptr, const Tensor &eid, const Tensor &indices, const Tensor &q,
-                                          const Tensor &k, const Tensor &v, int64_t h, double scale, double p, int64_t seed) {
+                                          const Tensor &k, const Tensor &v, int64_t h, double scale, double p, int64_t seed, const Copies &keep) {
     const auto meta = at::TensorOptions().dtype(q.dtype()).device(at::kMeta);
     const Tensor qp = at::empty({q.size(0), h, 64}, meta), kp = at::empty({k.size(0), h, 64}, meta);
     py::dict kw;
     kw["narrow"] = py::make_tuple(q, k, v);
+    kw["keep"] = py::make_tuple(keep[0], keep[1], keep[2], keep[3]);
     return python("attention_forward")(col, indptr, eid, indices, qp, kp, kp, scale, p, (uint64_t)seed, **kw).cast<std::tuple<Tensor, Tensor>>();
 }
 
@@ -345,11 +356,13 @@ struct NarrowAttention : torch::autograd::Function<NarrowAttention> {
     static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r,
                           const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c,
                           const Tensor &q, const Tensor &k, const Tensor &v, int64_t h, double scale, double p, int64_t seed) {
-        const Tensor qc = own_rows(q), kc = own_rows(k), vc = own_rows(v);
-        if (!narrow_known(col, indptr_c, eid_c, indices_c, qc, kc, h, p))
-            python("prepare_training")(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, qc, kc, p, h);
-        const auto [o, lse] = narrow_forward(col, indptr_c, eid_c, indices_c, qc, kc, vc, h, scale, p, seed);
-        ctx->save_for_backward({row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, qc, kc, vc, o.clone(), lse});
+        const Tensor qr = rows(q), kr = rows(k), vr = rows(v);
+        if (!narrow_known(col, indptr_c, eid_c, indices_c, qr, kr, h, p))
+            python("prepare_training")(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, qr, kr, p, h);
+        const Copies keep{room_for_copy(q, qr), room_for_copy(k, kr), room_for_copy(v, vr), at::empty_like(qr)};
+        const auto [o, lse] = narrow_forward(col, indptr_c, eid_c, indices_c, qr, kr, vr, h, scale, p, seed, keep);
+        ctx->save_for_backward({row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, keep[0].value_or(qr), keep[1].value_or(kr),
+                                keep[2].value_or(vr), *keep[3], lse});
         ctx->saved_data["h"] = h;
         ctx->saved_data["scale"] = scale;
         ctx->saved_data["p"] = p;
@@ -379,7 +392,7 @@ Tensor attention_narrow(const Tensor &row, const Tensor &indptr_r, const Tensor 
                         int64_t h, double scale, double p, uint64_t seed) {
     if (differentiated(q, k, v))
         return NarrowAttention::apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, h, scale, p, (int64_t)seed);
-    return std::get<0>(narrow_forward(col, indptr_c, eid_c, indices_c, rows(q), rows(k), rows(v), h, scale, p, (int64_t)seed));
+    return std::get<0>(narrow_forward(col, indptr_c, eid_c, indices_c, rows(q), rows(k), rows(v), h, scale, p, (int64_t)seed, Copies{}));
 }
 
 // ---- tile plans ---------------------------------------------------------------------------------------------------------------

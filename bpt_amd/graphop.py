@@ -535,11 +535,13 @@ def attention_reads_narrow(col, eid_c, q, k, h, dropout_p):
     return _narrow_seg(col, q, k, h, eid_c.size(0), dropout_p, _SETTINGS) is not None
 
 
-def _attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale, dropout_p, seed):
+def _attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale, dropout_p, seed, keep=None):
     """(o, lse) for heads of fewer than 64 columns: o (n, heads, d), lse (n, h), h the heads the layer is padded to.  On the tile
-    kernels that read the rows as they are, or else on padded copies."""
+    kernels that read the rows as they are, or else on padded copies.  keep: None or four tensors like q, k, v and o (None: not
+    this one) that become copies of them, on the tile kernels in the same launch."""
     seed = int(seed) & (2 ** 64 - 1)
-    known = _native.attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale, dropout_p, seed)
+    keep = (None,) * 4 if keep is None else tuple(keep)
+    known = _native.attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale, dropout_p, seed, keep)
     if known is not None:
         return known
     generation, cfg = _native.generation(), _SETTINGS
@@ -554,15 +556,25 @@ def _attention_forward_narrow(col, indptr_c, eid_c, indices_c, q, k, v, h, scale
         plan = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, None))
     if plan is None or not plan.covers_all_edges:
         o, lse = attention_forward(col, indptr_c, eid_c, indices_c, _pad_heads(q, h), _pad_heads(k, h), _pad_heads(v, h), scale, dropout_p, seed)
-        return o[:, :heads, :d].contiguous(), lse
+        o = o[:, :heads, :d].contiguous()
+        for held, x in zip(keep, (q, k, v, o)):
+            if held is not None:
+                held.copy_(x)
+        return o, lse
+    for held, x in zip(keep, (q, k, v, q)):
+        if held is not None:
+            _check_input(held, "keep")
+            _same_dtype(q, held)
+            _expect_shape(held, x.shape, "keep")
     struct = plan.ensure_groups(TILE_ROWS)["struct"]
     o = torch.empty_like(q)
     lse = torch.empty((q.size(0), h), dtype=torch.float32, device=q.device)
     dt = _dtype(q)
     ws, nws = _workspace(OP_ATTN_FWD, plan, None, h, 64, dt, q.device, keep=False)
     with _on_device_of(q):
-        check_attn(_LIB.bpt_attention_forward_narrow(ctypes.byref(struct), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse), _ptr(ws), nws, scale,
-                                                     float(dropout_p), seed, heads, d, h, dt, _stream()), "attention_forward_narrow")
+        check_attn(_LIB.bpt_attention_forward_narrow_keep(ctypes.byref(struct), _ptr(q), _ptr(k), _ptr(v), _ptr(o), _ptr(lse),
+                                                          ctypes.byref((ctypes.c_void_p * 4)(*map(_ptr, keep))), q.size(0), k.size(0), _ptr(ws), nws,
+                                                          scale, float(dropout_p), seed, heads, d, h, dt, _stream()), "attention_forward_narrow")
     plan_cache.remember((plan,), generation, _native.ATTN_FWD_NARROW, [col, indptr_c, eid_c, indices_c],
                         [q.size(0), k.size(0), h, d, dt, int(dropout_p > 0.0), heads], ctypes.addressof(struct), 0)
     return o, lse
@@ -609,7 +621,8 @@ def attention_backward_narrow(row, indptr_r, eid_r, indices_r, col, indptr_c, ei
     return dq, dk, dv
 
 
-def attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale=None, dropout_p=0.0, seed=0, bias=None, bias_by_pair=False, narrow=None):
+def attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale=None, dropout_p=0.0, seed=0, bias=None, bias_by_pair=False, narrow=None,
+                      keep=None):
     """o[dst] = sum over in-edges drop(softmax((q[dst].k[src] + bias[e])*scale)) v[src]; returns (o, lse) with lse
     (n, h) float32 in base-2 units.  Arithmetic of modules/attention.py:66-77 in one pass.  dropout_p > 0
     drops attention probabilities as attention.py:73 does; the mask is a function of (seed, graph), see
@@ -617,9 +630,10 @@ def attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale=None, drop
     id, or with bias_by_pair (h, E) with the edges in the order of the numbers attention_pair_rows() gives them (tile
     kernels only).
     narrow=(q, k, v): heads of fewer than 64 columns, (n, heads, d); the q, k, v before it then only stand for the padded shape
-    (attention_padded_shape; tensors of it on the meta device) and o has narrow's shape, lse the padded heads."""
+    (attention_padded_shape; tensors of it on the meta device) and o has narrow's shape, lse the padded heads; keep as
+    _attention_forward_narrow takes it."""
     if narrow is not None:
-        return _attention_forward_narrow(col, indptr_c, eid_c, indices_c, *narrow, q.size(1), float(scale), float(dropout_p), seed)
+        return _attention_forward_narrow(col, indptr_c, eid_c, indices_c, *narrow, q.size(1), float(scale), float(dropout_p), seed, keep)
     if bias is None:
         known = _native.attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, 1.0 / math.sqrt(q.size(-1)) if scale is None else float(scale),
                                           float(dropout_p), int(seed) & (2 ** 64 - 1))

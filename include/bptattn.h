@@ -262,6 +262,12 @@ int bpt_attention_forward_noalloc(const bpt_plan *plan_in, const void *q, const 
 int bpt_attention_forward_narrow(const bpt_plan *plan_in, const void *q, const void *k, const void *v, void *o, float *lse,
                                  void *workspace, int64_t workspace_bytes, float scale, float dropout_p, uint64_t dropout_seed,
                                  int heads, int d, int h, int dtype, void *stream);
+/* The same, and copies of q, k, v and of the result as well (keep: four device pointers, the first three on 16 bytes and outside of
+ * what they are copies of; NULL: no copy of that one), written by the same launches.  n_q, n_k: rows of q and of k, v. */
+int bpt_attention_forward_narrow_keep(const bpt_plan *plan_in, const void *q, const void *k, const void *v, void *o, float *lse,
+                                      void *const keep[4], int64_t n_q, int64_t n_k, void *workspace, int64_t workspace_bytes,
+                                      float scale, float dropout_p, uint64_t dropout_seed, int heads, int d, int h, int dtype,
+                                      void *stream);
 int bpt_attention_backward_narrow(const bpt_plan *plan_in, const bpt_plan *plan_out, const void *q, const void *k, const void *v,
                                   const void *o, const void *d_o, const float *lse, void *dq, void *dk, void *dv, void *workspace,
                                   int64_t workspace_bytes, float scale, float dropout_p, uint64_t dropout_seed, int heads, int d,
