@@ -783,8 +783,8 @@ def prepare_training(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indi
         return
     pi = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, None))
     po = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, order_src))
-    if not (pi.covers_all_edges and po.covers_all_edges):
-        return
+    if not (pi.covers_all_edges and po.covers_all_edges) or TILE_BACKWARD is not None:
+        return                       # (with the hook set the passes choose for themselves)
     fwd, bwd = (_native.ATTN_FWD, _native.ATTN_BWD) if narrow_h is None else (_native.ATTN_FWD_NARROW, _native.ATTN_BWD_NARROW)
     numbers = [q.size(0), k.size(0), h, q.size(2), _dtype(q), int(dropout_p > 0.0)] + ([] if narrow_h is None else [q.size(1)])
     in_struct = pi.ensure_groups(TILE_ROWS)["struct"]

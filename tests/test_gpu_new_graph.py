@@ -51,3 +51,18 @@ def test_a_malformed_out_side_is_refused_by_the_backward_only():
     o = op.bpt_attention(*bad, q, k, v)
     with pytest.raises(ValueError):
         o.sum().backward()
+
+
+@pytest.mark.parametrize("tiles", [False, True])
+def test_a_forced_backward_is_chosen_by_the_backward(tiles, monkeypatch):
+    """Nothing is remembered ahead while TILE_BACKWARD is set: the first backward reads it."""
+    from bpt_amd import graphop, op, plan
+    monkeypatch.setattr(graphop, "TILE_BACKWARD", tiles)
+    plan.plan_cache.clear()
+    args, n = new_graph([700, 300, 65])
+    q, k, v = (torch.randn(n, 8, 64, device=DEV, requires_grad=True) for _ in range(3))
+    here, real = [], graphop.attention_backward
+    monkeypatch.setattr(graphop, "attention_backward", lambda *a, **kw: here.append(1) or real(*a, **kw))
+    op.bpt_attention(*args, q, k, v).sum().backward()
+    plan.plan_cache.clear()
+    assert here
