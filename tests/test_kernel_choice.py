@@ -53,6 +53,18 @@ def test_segment_length_of_the_tile_plans_follows_the_mean_degree():
     assert graphop._tile_seg_len(fake_plan(4097, 524224)) == 256           # 128
 
 
+def test_segment_length_of_two_node_sets_counts_half_of_the_rows():
+    """Sentences attending to others: 26 edges a node are 52 a token; both ways of asking agree."""
+    two = SimpleNamespace(n_rows=6905, n_index_nodes=6838, n_edges=176728, n_items=6905)
+    q, k, units = torch.empty(6905, 8, 64), torch.empty(6838, 8, 64), torch.empty(7000, dtype=torch.int64)
+    for n_edges, want in ((6905 * 16 - 1, 64), (6905 * 16, 128), (176728, 128), (6905 * 40 - 1, 128), (6905 * 40, 256)):
+        two.n_edges = n_edges
+        assert graphop._tile_seg_len(two) == want
+        assert graphop._tile_seg_without_plan(units, n_edges, q, k, 8, 64, 0.0, None, graphop._SETTINGS) == want
+    same = SimpleNamespace(n_rows=6905, n_index_nodes=6905, n_edges=176728, n_items=6905)
+    assert graphop._tile_seg_len(same) == 64
+
+
 def test_choice_of_the_tile_kernels_without_a_plan_to_look_at():
     """_tile_seg_without_plan: the same answers as the rules that look at a plan wherever it gives one, None elsewhere."""
     cfg = graphop._SETTINGS
