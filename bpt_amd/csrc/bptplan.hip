@@ -334,9 +334,8 @@ struct PlanSide {
     int place_bits, g_bits, key_bits, work_bits;
     int32_t *jorder;
     GroupRec *rec;
-    int32_t *loc_group, *loc_work, *loc_prefix;         // groups in locality order
     int32_t *order, *entry0, *pair0, *chunks;           // final order: group as formed, first entry, first pair
-    uint32_t *word0, *word1;
+    int4 *placed;                                       // groups in locality order: word of the final order, entries, pairs, group
     int4 *entries;                                      // parked: neighbour, mask, first pair inside the group
     int32_t *pairs;                                     // parked: edge ids in pair order
     int32_t *out_info;
@@ -915,22 +914,16 @@ __global__ void k_edge_ids(const uint64_t *skey, const int32_t *slot_of, const i
 // The same groups as above for groups whose edges fit a workgroup's LDS (at most GRP_MAX_EDGES) and at most GRP_MAX_GROUPS of
 // them, which are the plans of graphs up to some 10^5 nodes.  A group's records never meet another group's, so the device-wide
 // sorts of all edges (fifty launches a side) become one workgroup per group that sorts its 200-1000 records in LDS and forms
-// the entries, their order and the pair numbers there; one workgroup then numbers the groups; after the caller has read the
+// the entries, their order and the pair numbers there; two small launches then number the groups; after the caller has read the
 // two counts and allocated exactly, every group writes its part of the arrays.  33 765 nodes / 576 k edges, base plan and tiles of
 // one side, call to call: 868 -> 227 us (65 535 / 3.3 M: 1690 -> 384, 1 023 / 17 k: 504 -> 165, mostly launches and the waits).
 constexpr int GRP_MAX_EDGES = 4096;
 constexpr int GRP_MAX_GROUPS = 16384;
-constexpr int GRP_ORDER_TPB = 1024;
-constexpr int GRP_ORDER_LDS = 8192;   // up to so many groups are sorted in LDS, more in global memory
 
 void short_layout(Bump &b, PlanSide &S) {
-    S.word0 = b.take<uint32_t>(S.max_groups);
-    S.word1 = b.take<uint32_t>(S.max_groups);
+    S.placed = b.take<int4>(S.max_groups);
     S.jorder = b.take<int32_t>(S.max_items);
     S.rec = b.take<GroupRec>(S.max_groups);
-    S.loc_group = b.take<int32_t>(S.max_groups);
-    S.loc_work = b.take<int32_t>(S.max_groups);
-    S.loc_prefix = b.take<int32_t>(S.max_groups);
     S.order = b.take<int32_t>(S.max_groups);
     S.entry0 = b.take<int32_t>(S.max_groups + 1);
     S.pair0 = b.take<int32_t>(S.max_groups + 1);
@@ -1183,134 +1176,208 @@ __global__ __launch_bounds__(TPB) void k_group_form(PlanSides b, int32_t R) {
     if (tid == 0) rec[g] = GroupRec{n_ent, n, smallest};
 }
 
-// One stable pass over n <= GRP_MAX_GROUPS words by one workgroup, from -> to (LDS or global memory); a wavefront owns a
-// contiguous part.  (A bitonic sort of the words in LDS took 73 us for 2200 groups, four passes and the rest 28.)
-template <int NW> __device__ void block_radix_pass(const uint32_t *from, uint32_t *to, int n, int shift, int bits, int32_t (*wh)[RS_BINS], int32_t *sh) {
-    const int bins = 1 << bits, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int per = ((n + NW * 64 - 1) / (NW * 64)) * 64, w0 = wave * per, w1 = min(w0 + per, n);
-    for (int b = threadIdx.x; b < NW * RS_BINS; b += NW * 64) wh[b / RS_BINS][b % RS_BINS] = 0;
-    __syncthreads();
-    for (int i = w0 + lane; i < w1; i += 64) atomicAdd(&wh[wave][(from[i] >> shift) & (uint32_t)(bins - 1)], 1);
-    __syncthreads();
-    int32_t sum = 0, all;
-    const int bin = threadIdx.x;
-    if (bin < bins)
-        for (int w = 0; w < NW; ++w) sum += wh[w][bin];
-    int32_t at = block_excl_sum<NW>(sum, sh, all);
-    if (bin < bins)
-        for (int w = 0; w < NW; ++w) {
-            const int32_t c = wh[w][bin];
-            wh[w][bin] = at;
-            at += c;
+// The groups' numbers: by locality (smallest neighbour, then as formed), cut into 8 ranges of equal work, by decreasing work inside
+// a range (or not); with them every group's place in the arrays.  Two launches of comparisons of every group with every other one
+// (the second: of its range): what a group is told apart by is a word that no other group has, its place is the number of smaller
+// words, and what it starts at is the sum over those.  A workgroup places GRP_PLACE groups, GRP_EACH of them a thread; 64 threads
+// share the others out.  Bound up to some 2000 groups by the latency of the launches and of reading the records, above by the
+// comparisons.  Groups of both sides, us: 131 12, 1072 13, 2200 16.6, 4352 27, 8768 58, 13477 97 (one workgroup a side that sorted the
+// words by radix passes in LDS: 12, 20, 28.6, 32, 67, 101).
+constexpr int GRP_PLACE_TPB = 1024;
+constexpr int GRP_EACH = 2;
+constexpr int GRP_PLACE = 16 * GRP_EACH;      // groups of a workgroup
+constexpr int GRP_PLACE_WAVES = GRP_PLACE_TPB / 64;
+// A thread meets at most a 64th of the groups, each of which has at most GRP_MAX_EDGES entries and less than twice that as its
+// work: number and sum of the smaller ones share a word, one addition for both.
+constexpr int GRP_SUM_BITS = 22;
+static_assert(GRP_MAX_GROUPS / 64 * (2 * GRP_MAX_EDGES) < 1 << GRP_SUM_BITS && GRP_MAX_GROUPS / 64 < 1 << (32 - GRP_SUM_BITS), "a thread's sums");
+
+struct GroupSums {                    // over the groups with a smaller word; all: of the a of all groups
+    int32_t place, a, b, all;
+};
+// The sums over a workgroup's threads; base: of what is smaller than all of its groups.  Valid in the first GRP_PLACE threads.
+template <bool TWO>
+__device__ GroupSums add_up(const uint32_t *sum, const uint32_t *b, GroupSums base) {
+    __shared__ int32_t part[GRP_PLACE_WAVES][GRP_PLACE][TWO ? 3 : 2], part_base[GRP_PLACE_WAVES][4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int m = 1; m < 64; m <<= 1) {
+        base.all += __shfl_xor(base.all, m, 64);
+        if constexpr (TWO) {
+            base.place += __shfl_xor(base.place, m, 64);
+            base.a += __shfl_xor(base.a, m, 64);
+            base.b += __shfl_xor(base.b, m, 64);
         }
-    __syncthreads();
-    const uint64_t below = (uint64_t(1) << lane) - 1;
-    for (int i0 = w0; i0 < w1; i0 += 64) {
-        const bool on = i0 + lane < w1;
-        const uint32_t key = on ? from[i0 + lane] : 0u;
-        const int d = (int)((key >> shift) & (uint32_t)(bins - 1));
-        uint64_t peers = __ballot(on);
-        for (int b = 0; b < bits; ++b) {
-            const bool bit = (d >> b) & 1;
-            const uint64_t m = __ballot(bit);
-            peers &= bit ? m : ~m;
+    }
+    if (lane == 0) {
+        part_base[wave][0] = base.place;
+        part_base[wave][1] = base.a;
+        part_base[wave][2] = base.b;
+        part_base[wave][3] = base.all;
+    }
+#pragma unroll
+    for (int e = 0; e < GRP_EACH; ++e) {
+        int32_t place = (int32_t)(sum[e] >> GRP_SUM_BITS), a = (int32_t)(sum[e] & ((1u << GRP_SUM_BITS) - 1u)), b_here = TWO ? (int32_t)b[e] : 0;
+        for (int m = 16; m < 64; m <<= 1) {
+            place += __shfl_xor(place, m, 64);
+            a += __shfl_xor(a, m, 64);
+            if constexpr (TWO) b_here += __shfl_xor(b_here, m, 64);
         }
-        const int32_t start = wh[wave][d];
-        wave_lds_order();
-        if (on && (peers & below) == 0) wh[wave][d] = start + __popcll(peers);
-        wave_lds_order();
-        if (on) to[start + __popcll(peers & below)] = key;
+        if (lane < 16) {
+            part[wave][16 * e + lane][0] = place;
+            part[wave][16 * e + lane][1] = a;
+            if constexpr (TWO) part[wave][16 * e + lane][2] = b_here;
+        }
     }
     __syncthreads();
+    GroupSums r{0, 0, 0, 0};
+    if (tid < GRP_PLACE)
+        for (int w = 0; w < GRP_PLACE_WAVES; ++w) {
+            r.place += part[w][tid][0] + part_base[w][0];
+            r.a += part[w][tid][1] + part_base[w][1];
+            if constexpr (TWO) r.b += part[w][tid][2] + part_base[w][2];
+            r.all += part_base[w][3];
+        }
+    return r;
 }
 
-// One workgroup numbers the groups: by locality, cut into 8 ranges of equal work, by decreasing work inside a range (or not),
-// and gives every group its place in the arrays.  out_info: the plan's info block and the groups'.
-__global__ __launch_bounds__(GRP_ORDER_TPB) void k_group_order(PlanSides b, int32_t R) {
+// locality order: a group's record goes to its place there, with the word that says its final place: (range, decreasing work or
+// nothing, place by locality)
+__global__ __launch_bounds__(GRP_PLACE_TPB) void k_group_place(PlanSides b, int32_t R) {
     const PlanSide &S = b.side[blockIdx.y];
     const GroupRec *rec = S.rec;
-    const int32_t *pinfo = S.info;
-    const int by_work = S.by_work, g_bits = S.g_bits, key_bits = S.key_bits, work_bits = S.work_bits;
-    uint32_t *word0 = S.word0, *word1 = S.word1;
-    int32_t *loc_group = S.loc_group, *loc_work = S.loc_work, *loc_prefix = S.loc_prefix, *order = S.order, *entry0 = S.entry0, *pair0 = S.pair0,
-            *chunks = S.chunks, *out_info = S.out_info;
-    constexpr int NW = GRP_ORDER_TPB / 64;
-    __shared__ int32_t wh[NW][RS_BINS];
-    __shared__ uint32_t lds0[GRP_ORDER_LDS], lds1[GRP_ORDER_LDS];
-    __shared__ int32_t sh[NW + 1], cut[9];
-    const int tid = threadIdx.x, ng = n_groups_of(pinfo, R);
-    const uint32_t g_mask = (1u << g_bits) - 1u;
-    uint32_t *from = ng <= GRP_ORDER_LDS ? lds0 : word0, *to = ng <= GRP_ORDER_LDS ? lds1 : word1;
-    auto sort = [&](int bits) {                           // the words by their `bits` bits above the group's number
-        const int passes = (bits + RS_MAX_BITS - 1) / RS_MAX_BITS, step = (bits + passes - 1) / passes;
-        for (int p = 0; p < passes; ++p) {
-            block_radix_pass<NW>(from, to, ng, g_bits + p * step, min(step, bits - p * step), wh, sh);
-            uint32_t *t = from; from = to; to = t;
-        }
-    };
-    for (int g = tid; g < ng; g += GRP_ORDER_TPB) from[g] = ((uint32_t)rec[g].key << g_bits) | (uint32_t)g;
-    __syncthreads();
-    sort(key_bits);
-    int64_t total = 0;
-    for (int l0 = 0; l0 < ng; l0 += GRP_ORDER_TPB) {
-        const int l = l0 + tid;
-        int32_t work = 0, in_round;
-        if (l < ng) {
-            const int32_t g = (int32_t)(from[l] & g_mask);
-            work = R == 16 ? 4 * ((rec[g].n_entries + R - 1) / R + 1) : FIXED_WORK + rec[g].n_pairs;
-            loc_group[l] = g;
-            loc_work[l] = work;
-        }
-        const int32_t before = block_excl_sum<NW>(work, sh, in_round);
-        if (l < ng) loc_prefix[l] = (int32_t)total + before;
-        total += in_round;
+    const int g_bits = S.g_bits, work_bits = S.work_bits, by_work = S.by_work;
+    const int ng = n_groups_of(S.info, R), g0 = blockIdx.x * GRP_PLACE, tid = threadIdx.x;
+    if (g0 >= ng) return;
+    __shared__ uint2 word_work[2 * GRP_PLACE_TPB];                // word; 1 and the work
+    auto work_of = [&](const GroupRec &r) { return R == 16 ? 4 * ((r.n_entries + R - 1) / R + 1) : FIXED_WORK + r.n_pairs; };
+    auto word_of = [&](const GroupRec &r, int g) { return ((uint32_t)r.key << g_bits) | (uint32_t)g; };
+    uint32_t mine[GRP_EACH], sum[GRP_EACH];
+#pragma unroll
+    for (int e = 0; e < GRP_EACH; ++e) {
+        const int g = g0 + 16 * e + (tid & 15);
+        mine[e] = g < ng ? word_of(rec[g], g) : 0u;
+        sum[e] = 0;
     }
-    __syncthreads();
-    // cut[x] = number of groups whose midpoint lies before x/8 of the total: the midpoints ascend, so the group that crosses says so
-    if (tid <= 8) cut[tid] = tid == 0 ? 0 : ng;
-    __syncthreads();
-    for (int l = tid; l < ng; l += GRP_ORDER_TPB) {
-        const int64_t mid = (int64_t)loc_prefix[l] + loc_work[l] / 2, prev = l > 0 ? (int64_t)loc_prefix[l - 1] + loc_work[l - 1] / 2 : -1;
-        for (int x = 1; x <= 7; ++x)
-            if (mid >= total * x / 8 && prev < total * x / 8) cut[x] = l;
-    }
-    __syncthreads();
-    if (tid <= 8) chunks[tid] = cut[tid];
-    if (by_work) {
-        const uint32_t w_max = (1u << work_bits) - 1u;
-        for (int l = tid; l < ng; l += GRP_ORDER_TPB) {
-            uint32_t c = 0;
-            for (int x = 1; x <= 7; ++x) c += cut[x] <= l ? 1u : 0u;
-            from[l] = (((c << work_bits) | (w_max - (uint32_t)loc_work[l])) << g_bits) | (uint32_t)l;
+    GroupSums base{0, 0, 0, 0};
+    for (int t0 = 0; t0 < ng; t0 += 2 * GRP_PLACE_TPB) {
+        const int n = min(2 * GRP_PLACE_TPB, ng - t0);
+        __syncthreads();
+        for (int t = tid; t < n; t += GRP_PLACE_TPB) {
+            const GroupRec r = rec[t0 + t];
+            const int32_t work = work_of(r);
+            word_work[t] = make_uint2(word_of(r, t0 + t), (1u << GRP_SUM_BITS) + (uint32_t)work);
+            base.all += work;
         }
         __syncthreads();
-        sort(3 + work_bits);
-    }
-    int32_t n_entries = 0, n_pairs = 0;
-    for (int f0 = 0; f0 < ng; f0 += GRP_ORDER_TPB) {
-        const int f = f0 + tid;
-        int32_t ne = 0, np = 0, round_e, round_p;
-        if (f < ng) {
-            const int32_t g = loc_group[by_work ? (int)(from[f] & g_mask) : f];
-            order[f] = g;
-            ne = rec[g].n_entries;
-            np = rec[g].n_pairs;
+#pragma unroll 8
+        for (int t = tid >> 4; t < n; t += GRP_PLACE_TPB / 16) {
+            const uint2 x = word_work[t];
+#pragma unroll
+            for (int e = 0; e < GRP_EACH; ++e) sum[e] += x.x < mine[e] ? x.y : 0u;
         }
-        const int32_t e0 = n_entries + block_excl_sum<NW>(ne, sh, round_e), p0 = n_pairs + block_excl_sum<NW>(np, sh, round_p);
-        if (f < ng) {
-            entry0[f] = e0;
-            pair0[f] = p0;
+    }
+    const GroupSums at = add_up<false>(sum, nullptr, base);
+    const int g = g0 + tid;
+    if (tid >= GRP_PLACE || g >= ng) return;
+    // range: how many of the points 1/8 ... 7/8 of the total lie at or before the group's midpoint
+    const GroupRec r = rec[g];
+    const int32_t work = work_of(r);
+    const int64_t mid = (int64_t)at.a + work / 2, total = at.all;
+    uint32_t range = 0;
+    for (int x = 1; x <= 7; ++x) range += mid >= total * x / 8 ? 1u : 0u;
+    const uint32_t down = by_work ? ((1u << work_bits) - 1u) - (uint32_t)work : 0u;
+    S.placed[at.place] = make_int4((int)((((range << work_bits) | down) << g_bits) | (uint32_t)at.place), r.n_entries, r.n_pairs, g);
+}
+
+// final order, and every group's first entry and pair.  The ranges are runs of the locality order: a workgroup adds up what lies in
+// the ranges before its groups' and compares inside theirs.  The last workgroup writes the ranges' bounds and the plan's and the
+// groups' info blocks.
+__global__ __launch_bounds__(GRP_PLACE_TPB) void k_group_order(PlanSides b, int32_t R) {
+    const PlanSide &S = b.side[blockIdx.y];
+    const int4 *placed = S.placed;
+    const int32_t *pinfo = S.info;
+    const int range_at = S.work_bits + S.g_bits;
+    const int ng = n_groups_of(pinfo, R), tid = threadIdx.x;
+    auto range_of = [&](int l) { return (int)((uint32_t)placed[l].x >> range_at); };
+    if (blockIdx.x == gridDim.x - 1) {
+        int32_t *chunks = S.chunks, *out_info = S.out_info;
+        __shared__ int32_t cut[9], entries[GRP_PLACE_WAVES];
+        if (tid < 9) cut[tid] = tid == 0 ? 0 : ng;
+        __syncthreads();
+        int32_t n_entries = 0;
+        for (int l = tid; l < ng; l += GRP_PLACE_TPB) {
+            const int from = l > 0 ? range_of(l - 1) : 0, to = range_of(l);
+            for (int x = from + 1; x <= to; ++x) cut[x] = l;
+            n_entries += placed[l].y;
         }
-        n_entries += round_e;
-        n_pairs += round_p;
+        for (int m = 1; m < 64; m <<= 1) n_entries += __shfl_xor(n_entries, m, 64);
+        if ((tid & 63) == 0) entries[tid >> 6] = n_entries;
+        __syncthreads();
+        if (tid < 9) chunks[tid] = cut[tid];
+        if (tid < 16) out_info[tid] = pinfo[tid];
+        if (tid > 0) return;
+        for (int w = 1; w < GRP_PLACE_WAVES; ++w) n_entries += entries[w];
+        int32_t most = 0;
+        for (int x = 0; x < 8; ++x) most = max(most, cut[x + 1] - cut[x]);
+        S.entry0[ng] = n_entries;
+        for (int i = 0; i < 16; ++i) out_info[16 + i] = i == BPT_GI_N_GROUPS ? ng : i == BPT_GI_N_ENTRIES ? n_entries : i == BPT_GI_MAX_CHUNK ? most : 0;
+        return;
     }
-    if (tid < 16) out_info[tid] = pinfo[tid];
-    if (tid == 0) {
-        entry0[ng] = n_entries;
-        int32_t mx = 0;
-        for (int x = 0; x < 8; ++x) mx = max(mx, cut[x + 1] - cut[x]);
-        for (int i = 0; i < 16; ++i) out_info[16 + i] = i == BPT_GI_N_GROUPS ? ng : i == BPT_GI_N_ENTRIES ? n_entries : i == BPT_GI_MAX_CHUNK ? mx : 0;
+    const int l0 = blockIdx.x * GRP_PLACE;
+    if (l0 >= ng) return;
+    const int first = range_of(l0), last = range_of(min(l0 + GRP_PLACE, ng) - 1);
+    __shared__ uint2 word_entries[2 * GRP_PLACE_TPB];             // word; 1 and the entries
+    __shared__ uint32_t n_pairs[2 * GRP_PLACE_TPB];
+    uint32_t mine[GRP_EACH], sum[GRP_EACH], pairs[GRP_EACH];
+#pragma unroll
+    for (int e = 0; e < GRP_EACH; ++e) {
+        const int l = l0 + 16 * e + (tid & 15);
+        mine[e] = l < ng ? (uint32_t)placed[l].x : 0u;
+        sum[e] = pairs[e] = 0;
     }
+    GroupSums base{0, 0, 0, 0};
+    for (int t0 = 0; t0 < ng; t0 += 2 * GRP_PLACE_TPB) {
+        int lo = 0, hi = 0;                                       // of these: in the ranges before, in those and the groups' own
+        for (int u = 0; u < 2; ++u) {
+            const int t = u * GRP_PLACE_TPB + tid;
+            bool before = false, own = false;
+            if (t0 + t < ng) {
+                const int4 x = placed[t0 + t];
+                const int range = (int)((uint32_t)x.x >> range_at);
+                before = range < first;
+                own = range >= first && range <= last;
+                if (before) {
+                    base.place += 1;
+                    base.a += x.y;
+                    base.b += x.z;
+                }
+                if (own) {
+                    word_entries[t] = make_uint2((uint32_t)x.x, (1u << GRP_SUM_BITS) + (uint32_t)x.y);
+                    n_pairs[t] = (uint32_t)x.z;
+                }
+            }
+            const int n_before = __syncthreads_count(before), n_own = __syncthreads_count(own);
+            lo += n_before;
+            hi += n_before + n_own;
+        }
+        for (int t = lo + (tid >> 4); t < hi; t += GRP_PLACE_TPB / 16) {
+            const uint2 x = word_entries[t];
+            const uint32_t p = n_pairs[t];
+#pragma unroll
+            for (int e = 0; e < GRP_EACH; ++e) {
+                const bool less = x.x < mine[e];
+                sum[e] += less ? x.y : 0u;
+                pairs[e] += less ? p : 0u;
+            }
+        }
+        __syncthreads();
+        if (hi < min(2 * GRP_PLACE_TPB, ng - t0)) break;          // the rest lies in later ranges
+    }
+    const GroupSums at = add_up<true>(sum, pairs, base);
+    if (tid >= GRP_PLACE || l0 + tid >= ng) return;
+    S.order[at.place] = placed[l0 + tid].w;
+    S.entry0[at.place] = at.a;
+    S.pair0[at.place] = at.b;
 }
 
 // a group's part of the arrays; the block behind the last group writes what stands behind the last entry
@@ -1791,8 +1858,8 @@ int rs_sort(const Recs &recs, const Out &out, const RsSizes &sizes, int n_sides,
 }
 
 // what the kernels need to know of a side's groups, or BPT_ERR_UNSUPPORTED where they are not built in the short form: a group may
-// hold more edges than fit a workgroup's LDS, or there may be more groups, or wider numbers, than one workgroup sorts as
-// 32-bit words
+// hold more edges than fit a workgroup's LDS, or there may be more groups than it pays to compare with each other, or numbers that
+// don't fit 32-bit words
 int short_form(int64_t max_items, int64_t n_edges, int64_t n_index_nodes, int32_t seg_len, int32_t R, int32_t by_mask, PlanSide &S) {
     if (max_items < 0 || n_edges < 0 || n_index_nodes < 0 || max_items >= INT32_MAX || n_edges >= INT32_MAX || n_index_nodes >= INT32_MAX - 1)
         return BPT_ERR_SIZE;
@@ -1889,7 +1956,13 @@ int groups_count(const PlanSides &b, int n_sides, int32_t R, const SortWs &w, hi
         if (narrow) HIP_TRY(cap <= 1024 ? form(k_group_form<1024, uint32_t>) : cap <= 2048 ? form(k_group_form<2048, uint32_t>) : form(k_group_form<4096, uint32_t>));
         else HIP_TRY(cap <= 1024 ? form(k_group_form<1024, uint64_t>) : cap <= 2048 ? form(k_group_form<2048, uint64_t>) : form(k_group_form<4096, uint64_t>));
     }
-    hipLaunchKernelGGL(k_group_order, dim3(1, ns), dim3(GRP_ORDER_TPB), 0, s, b, R);
+    const int64_t max_groups = most_of(b, n_sides, [](const PlanSide &S) { return S.max_groups; });
+    const unsigned places = (unsigned)((max_groups + GRP_PLACE - 1) / GRP_PLACE);
+    if (places > 0) {
+        hipLaunchKernelGGL(k_group_place, dim3(places, ns), dim3(GRP_PLACE_TPB), 0, s, b, R);
+        HIP_TRY(hipGetLastError());
+    }
+    hipLaunchKernelGGL(k_group_order, dim3(places + 1, ns), dim3(GRP_PLACE_TPB), 0, s, b, R);
     HIP_TRY(hipGetLastError());
     return BPT_OK;
 }
