@@ -788,8 +788,10 @@ def prepare_training(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indi
     fwd, bwd = (_native.ATTN_FWD, _native.ATTN_BWD) if narrow_h is None else (_native.ATTN_FWD_NARROW, _native.ATTN_BWD_NARROW)
     numbers = [q.size(0), k.size(0), h, q.size(2), _dtype(q), int(dropout_p > 0.0)] + ([] if narrow_h is None else [q.size(1)])
     in_struct = pi.ensure_groups(TILE_ROWS)["struct"]
-    out_struct = po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True)
     plan_cache.remember((pi,), generation, fwd, list(graph[4:]), numbers, ctypes.addressof(in_struct), 0)
+    if po.n_edges != pi.n_edges:
+        return                       # (two different graphs: the backward, which asks for the out-side, is the one to refuse them)
+    out_struct = po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True)
     plan_cache.remember((pi, po), generation, bwd, list(graph), numbers, ctypes.addressof(in_struct), ctypes.addressof(out_struct))
 
 

@@ -53,6 +53,23 @@ def test_a_malformed_out_side_is_refused_by_the_backward_only():
         o.sum().backward()
 
 
+@pytest.mark.parametrize("heads,d", [(8, 64), (6, 50)])
+def test_an_out_side_of_another_graph_is_refused_by_the_backward_only(heads, d):
+    """Each side is sound by itself, but they have different numbers of edges: a forward never asks for the out-side."""
+    from bpt_amd import op, plan
+    args, n = new_graph([700, 300, 65])
+    other, m = new_graph([700, 300, 64])
+    assert m < n and args[2].numel() != other[2].numel()
+    q, k, v = (torch.randn(n, heads, d, device=DEV, requires_grad=True) for _ in range(3))
+    plan.plan_cache.clear()
+    want = op.bpt_attention(*args, q, k, v)
+    plan.plan_cache.clear()
+    o = op.bpt_attention(*other[:4], *args[4:], q, k, v)
+    assert torch.equal(o, want)
+    with pytest.raises(ValueError):
+        o.sum().backward()
+
+
 @pytest.mark.parametrize("tiles", [False, True])
 def test_a_forced_backward_is_chosen_by_the_backward(tiles, monkeypatch):
     """Nothing is remembered ahead while TILE_BACKWARD is set: the first backward reads it."""
