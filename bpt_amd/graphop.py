@@ -778,11 +778,11 @@ def prepare_training(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indi
     if seg is None:
         return
     order_src = _plan.tile_order_src(k.size(0), eid_r.size(0))
-    if not plan_cache.put_tile_plans([(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg, None),
-                                      (row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg, order_src)]):
+    plans = plan_cache.put_tile_plans([(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg, None),
+                                       (row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg, order_src)])
+    if plans is None:
         return
-    pi = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, None))
-    po = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, order_src))
+    pi, po = plans
     if not (pi.covers_all_edges and po.covers_all_edges) or TILE_BACKWARD is not None:
         return                       # (with the hook set the passes choose for themselves)
     fwd, bwd = (_native.ATTN_FWD, _native.ATTN_BWD) if narrow_h is None else (_native.ATTN_FWD_NARROW, _native.ATTN_BWD_NARROW)

@@ -808,28 +808,28 @@ class PlanCache:
     def put_tile_plans(self, sides):
         """What get() would build one after the other for a training step on tiles, built together (DevicePlan.tile_plans; sides as
         there: the in-side, then the out-side), unless one of them is already here or they have to be built one by one.  A side that is
-        malformed is refused where it is asked for: a forward never asks for the out-side.  True if the plans are here now because of
-        this call."""
+        malformed is refused where it is asked for: a forward never asks for the out-side.  The plans, which the cache may have had no
+        room for, or None where this call has not built them."""
         if self.native is None or DEVICE_BUILD is False or not sides[0][2].is_cuda:
-            return False
+            return None
         keys = [self._key(side[:4], side[4], side[5], side[6], True) for side in sides]
         with self._lock:
             if any(key in self._d for key in keys):
-                return False
+                return None
         try:
             plans = DevicePlan.tile_plans(sides)
         except ValueError:
             plans = None
         if plans is None:
-            return False
+            return None
         self.misses += len(plans)
         with self._lock:
             if any(key in self._d for key in keys):
-                return False                        # (as in get: another thread's stay)
+                return None                         # (as in get: another thread's stay)
             for key, plan, side in zip(keys, plans, sides):
                 self._insert(key, plan, side[:4])
             self._evict()
-        return True
+        return plans
 
     def clear(self):
         with self._lock:

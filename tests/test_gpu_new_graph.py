@@ -70,6 +70,34 @@ def test_an_out_side_of_another_graph_is_refused_by_the_backward_only(heads, d):
         o.sum().backward()
 
 
+@pytest.mark.parametrize("limits", [dict(capacity=1), dict(max_bytes=0)])
+def test_a_cache_too_small_for_both_sides_builds_neither_again(limits):
+    """Both sides are built together once; what the cache has no room for is built where a pass asks for it, as ever."""
+    from bpt_amd import graphop, op, plan
+    args, n = new_graph([700, 300, 65])
+    leaves = [torch.randn(n, 8, 64, device=DEV, requires_grad=True) for _ in range(3)]
+
+    def step():
+        o = op.bpt_attention(*args, *leaves)
+        return (o.detach(),) + torch.autograd.grad(o.sum(), leaves)
+
+    plan.plan_cache.clear()
+    want = step()
+    old = plan.plan_cache.set_limits(**limits)
+    try:
+        plan.plan_cache.clear()
+        built = plan.plan_cache.misses
+        graphop.prepare_training(*args, *leaves[:2])
+        assert plan.plan_cache.misses == built + 2 and len(plan.plan_cache._d) == 1
+        plan.plan_cache.clear()
+        got = step()
+    finally:
+        plan.plan_cache.set_limits(*old)
+        plan.plan_cache.clear()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("tiles", [False, True])
 def test_a_forced_backward_is_chosen_by_the_backward(tiles, monkeypatch):
     """Nothing is remembered ahead while TILE_BACKWARD is set: the first backward reads it."""
