@@ -99,6 +99,7 @@ BUILD_API = {
     "bpt_build_csrs_device": (ctypes.c_int, [c_vp, c_vp, c_i64, c_i64, c_i32, ctypes.POINTER(c_vp * 5), ctypes.POINTER(c_vp * 5), c_vp,
                                              c_vp, c_i64, c_vp]),
     "bpt_build_merge_device": (ctypes.c_int, [c_vp, c_i64, c_vp, c_vp, c_vp, c_vp, c_vp]),
+    "bpt_build_count_rows": (ctypes.c_int, [ctypes.POINTER(c_vp * 2), ctypes.POINTER(c_vp * 2), ctypes.POINTER(c_i64 * 2), ctypes.c_int, c_vp, c_vp]),
     "bpt_build_wait": (ctypes.c_int, [c_vp]),
     "bpt_build_plan_device": (ctypes.c_int, [c_vp, c_vp, c_i64, c_vp, c_vp, c_i64, c_i64, c_i64, c_i32,
                                              c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_vp, c_i64, c_vp]),

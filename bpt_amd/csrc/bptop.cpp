@@ -441,6 +441,31 @@ std::tuple<std::vector<Tensor>, std::vector<Tensor>, std::vector<int>> build_csr
     return {side[0], side[1], {c[0], c[1], c[2], c[3]}};
 }
 
+// how many rows of one or two CSR sides (their units' rows and pointers) have edges; one wait
+std::vector<int64_t> count_rows(const std::vector<std::tuple<Tensor, Tensor>> &in) {
+    const int n = (int)in.size();
+    if (n < 1 || n > 2) throw std::invalid_argument("one or two sides");
+    const at::Device dev = std::get<0>(in[0]).device();
+    const int64_t *row[2] = {}, *indptr[2] = {};
+    int64_t units[2] = {};
+    for (int i = 0; i < n; ++i) {
+        const auto &[r, p] = in[i];
+        if (!index_ok(r, dev) || !index_ok(p, dev) || p.numel() != r.numel() + 1)
+            throw std::invalid_argument("row and indptr: contiguous int64 on one GPU, one indptr more than rows");
+        row[i] = r.const_data_ptr<int64_t>();
+        indptr[i] = p.const_data_ptr<int64_t>();
+        units[i] = r.numel();
+    }
+    c10::DeviceGuard guard(dev);
+    Tensor parts = at::empty({n * BPT_COUNT_PARTS}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+    void *stream = stream_of(dev);
+    check_build(bpt_build_count_rows(row, indptr, units, n, parts.data_ptr<int32_t>(), stream), "bpt_build_count_rows");
+    wait_for(stream);
+    std::vector<int64_t> counts(n, 0);
+    for (int i = 0; i < n * BPT_COUNT_PARTS; ++i) counts[i / BPT_COUNT_PARTS] += parts.data_ptr<int32_t>()[i];
+    return counts;
+}
+
 // None where the short form does not build them; else (per side: its info block, base arrays, group arrays; the pair mapping of
 // the second side).  A side's info block holds an error where its arrays are malformed (then nothing else is valid).
 py::object build_tile_plans(const std::vector<std::tuple<Tensor, Tensor, Tensor, Tensor, int64_t, int64_t, int, int>> &in) {
@@ -599,6 +624,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("attention_backward", &attention_backward_known);
     m.def("build_csrs", &build_csrs);
     m.def("build_tile_plans", &build_tile_plans);
+    m.def("count_rows", &count_rows);
     m.def("remember", &remember);
     m.def("forget", &forget);
     m.def("clear", &clear);

@@ -1176,6 +1176,30 @@ __global__ __launch_bounds__(TPB) void k_group_form(PlanSides b, int32_t R) {
     if (tid == 0) rec[g] = GroupRec{n_ent, n, smallest};
 }
 
+// Rows that have edges: a row counts at its first unit that is not empty.  Bound by the latency of one launch (a side's units are some
+// 100 KB), so every workgroup leaves its own count for the host to add up, and nothing is cleared or added across workgroups.
+struct UnitSide {
+    const int64_t *row, *indptr;
+    int32_t n;
+};
+struct UnitSides {
+    UnitSide side[2];
+};
+__global__ __launch_bounds__(TPB) void k_count_rows(UnitSides b, int32_t *counts) {
+    const UnitSide &S = b.side[blockIdx.y];
+    __shared__ int32_t sh[TPB / 64 + 1];
+    int32_t mine = 0, all;
+    for (int64_t u = blockIdx.x * TPB + threadIdx.x; u < S.n; u += gridDim.x * TPB) {
+        if (S.indptr[u + 1] <= S.indptr[u]) continue;
+        const int64_t r = S.row[u];
+        int64_t v = u;                                            // back over the row's empty units
+        while (v > 0 && S.row[v - 1] == r && S.indptr[v] <= S.indptr[v - 1]) --v;
+        mine += v == 0 || S.row[v - 1] != r;
+    }
+    block_excl_sum<TPB / 64>(mine, sh, all);
+    if (threadIdx.x == 0) counts[blockIdx.y * BPT_COUNT_PARTS + blockIdx.x] = all;
+}
+
 // The groups' numbers: by locality (smallest neighbour, then as formed), cut into 8 ranges of equal work, by decreasing work inside
 // a range (or not); with them every group's place in the arrays.  Two launches of comparisons of every group with every other one
 // (the second: of its range): what a group is told apart by is a word that no other group has, its place is the number of smaller
@@ -2016,6 +2040,21 @@ int csr_build(CsrSides g, int n_sides, int64_t n_edges, int64_t n_nodes, int32_t
 }  // namespace
 
 extern "C" {
+
+int bpt_build_count_rows(const int64_t *const row[2], const int64_t *const indptr_units[2], const int64_t n_units[2], int n_sides, int32_t *counts,
+                         void *stream) {
+    if (n_sides < 1 || n_sides > 2) return BPT_ERR_SHAPE;
+    if (!row || !indptr_units || !n_units || !counts) return BPT_ERR_NULL;
+    UnitSides b{};
+    for (int i = 0; i < n_sides; ++i) {
+        if (n_units[i] < 0 || n_units[i] >= INT32_MAX) return BPT_ERR_SIZE;
+        if (n_units[i] > 0 && (!row[i] || !indptr_units[i])) return BPT_ERR_NULL;
+        b.side[i] = UnitSide{row[i], indptr_units[i], (int32_t)n_units[i]};
+    }
+    hipLaunchKernelGGL(k_count_rows, dim3(BPT_COUNT_PARTS, n_sides), dim3(TPB), 0, (hipStream_t)stream, b, counts);
+    HIP_TRY(hipGetLastError());
+    return BPT_OK;
+}
 
 int bpt_build_wait(void *stream) {
     HIP_TRY(hipStreamSynchronize((hipStream_t)stream));

@@ -976,16 +976,18 @@ def _tile_seg_len(plan):
 
 
 def _tile_seg_of(n_edges, n_rows, n_index_nodes):
-    """Edges per work item of the plans the tile kernels walk (TILE_SEG_LEN overrides when set), by the average row.  Two different
-    node sets are sentences that attend to others: the inner nodes of their trees, half of all nodes, have no edges, and every
-    other row has as many as the other sentence has tokens, none far above the average.  The average there is over half of the
-    rows; cut at 64, a third of them was split, written in float32 parts and added up by two more launches.  Kernels of a
-    training pass, 8 x 64 float32, 64 pairs of up to 96 tokens: 63.3 us at 64, 50.8 at 128.  (Graphs of one node set have a few
-    long rows among many short ones and lose by longer items: 33 598 nodes, 17 edges a row, 257 us at 64, 270 at 128.)"""
+    """Edges per work item of the plans the tile kernels walk (TILE_SEG_LEN overrides when set): plan.tile_seg_len by the average row.
+    In a graph of two node sets rows without edges are common, and what counts is the average over the others: of sentences that
+    attend to other sentences half of the nodes, the inner ones of their trees, have no edges, and the tokens' rows, as
+    long as the other sentence, would be cut at 64 by an average over all of them.  Kernels of a training pass, 8 x 64 float32, 64
+    pairs of up to 96 tokens: 63.3 us at 64, 50.8 at 128.  Such a plan counts its rows with edges when it is built (SEG_BY_ROWS, 15 us
+    of the 800 that the first pass takes): the sizes at hand here do not tell that graph from one whose rows all have edges, which
+    loses by items of twice its average (41 to 62 edges a row on 8000 to 12 000 rows, a few of some thousand, items of 128 | 256: float32
+    239 | 255, 234 | 254, 209 | 223 us, bfloat16 117 | 121, 114 | 138, 103 | 120; at 16 to 27 edges a row 64 and 128 are level within
+    4 %).  Equal counts are taken for one node set, where every row has edges (a new batch of such graphs would wait for nothing)."""
     if TILE_SEG_LEN is not None:
         return TILE_SEG_LEN
-    deg = n_edges / max(n_rows, 1) * (1 if n_rows == n_index_nodes else 2)
-    return 64 if deg < 32 else (128 if deg < 80 else 256)
+    return _plan.tile_seg_len(n_edges, n_rows) if n_rows == n_index_nodes else _plan.SEG_BY_ROWS
 
 
 def set_tiles(on):

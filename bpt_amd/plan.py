@@ -19,6 +19,7 @@ import torch
 from ._lib import BPT_ERR_UNSUPPORTED, PlanInfo, PlanStruct, check_graph, graph_lib, plan_lib
 
 DEFAULT_SEG_LEN = None  # edges per work item: None = chosen per plan by auto_seg_len
+SEG_BY_ROWS = -1        # what a caller of PlanCache asks for: tile_seg_len by the rows that have edges, counted when the plan is built
 FORCE_SEG_LEN = None    # testing hook: when set, replaces the automatic choice for plans built from now on
 GROUP_R = 4            # default rows per group (the row-group kernels exist for 4 and, float32 with h <= 8 and h*d <= 512, 8)
 GROUP_WINDOW = 32      # how many following items the greedy grouping examines per group
@@ -93,6 +94,29 @@ def auto_seg_len(row, indptr, n_rows):
         return 64
     q90 = float(np.quantile(deg, 0.9))
     return 64 if q90 <= 64 else (128 if q90 <= 128 else 256)
+
+
+def tile_seg_len(n_edges, n_rows):
+    """Edges per work item of a plan that the tile kernels walk, by the average row of n_rows.  Shorter items leave no tile much longer
+    than the others, longer ones leave more rows whole: a row that is cut is written in float32 parts and added up by a launch
+    more."""
+    deg = n_edges / max(n_rows, 1)
+    return 64 if deg < 32 else (128 if deg < 80 else 256)
+
+
+def rows_with_edges(sides):
+    """How many rows of each of one or two CSR sides (row, indptr) have an edge: on the GPU one launch and one wait for both."""
+    if not all(len(indptr) == len(row) + 1 for row, indptr in sides):
+        return [0] * len(sides)                     # malformed: whoever builds the plan says so
+    if sides[0][0].is_cuda:
+        from ._native import native
+        return native.count_rows(list(sides))
+    return [int(torch.unique_consecutive(row[indptr[1:] > indptr[:-1]]).numel()) for row, indptr in sides]
+
+
+def seg_lens_by_rows(sides):
+    """tile_seg_len of each of the sides (row, indptr, n_edges) by its rows with edges."""
+    return [tile_seg_len(side[2], n) for side, n in zip(sides, rows_with_edges([side[:2] for side in sides]))]
 
 
 def build_plan_host(row, indptr, eid, indices, n_rows, n_index_nodes, seg_len=DEFAULT_SEG_LEN):
@@ -775,7 +799,7 @@ class PlanCache:
         """n_rows None: as many rows as `row` mentions (ops that only produce edge outputs).  prefer_device: build on the GPU
         whatever the graph's size, unless set_device_build() fixed the place (the tile kernels ask for this: the GPU
         builder's groups of 16 run them as fast or faster on every graph measured).  groups = (R, order_mode): row groups the caller
-        asks the plan for next; a plan built on the GPU for this call forms them along with it."""
+        asks the plan for next; a plan built on the GPU for this call forms them along with it.  seg_len may be SEG_BY_ROWS."""
         tensors = (row, indptr, eid, indices)
         on_device = _build_on_device(eid, n_rows) or bool(prefer_device and DEVICE_BUILD is None and eid.is_cuda and n_rows is not None)
         key = self._key(tensors, n_rows, n_index_nodes, seg_len, on_device)
@@ -788,6 +812,8 @@ class PlanCache:
                     self._evict()                   # row groups and pair mappings are added to plans after insertion
                 return hit[0]
         self.misses += 1
+        if seg_len == SEG_BY_ROWS:
+            seg_len, = seg_lens_by_rows([(row, indptr, eid.numel())])
         if on_device:
             nr = n_rows if n_rows is not None else (int(row[-1]) + 1 if row.numel() else 0)
             ni = n_index_nodes if n_index_nodes is not None else nr
@@ -816,8 +842,13 @@ class PlanCache:
         with self._lock:
             if any(key in self._d for key in keys):
                 return None
+        if sides[0][6] == SEG_BY_ROWS:
+            seg_lens = seg_lens_by_rows([(side[0], side[1], side[2].numel()) for side in sides])
+            built_of = [(*side[:6], seg_len, side[7]) for side, seg_len in zip(sides, seg_lens)]
+        else:
+            built_of = sides
         try:
-            plans = DevicePlan.tile_plans(sides)
+            plans = DevicePlan.tile_plans(built_of)
         except ValueError:
             plans = None
         if plans is None:

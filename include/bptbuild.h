@@ -74,6 +74,13 @@ int bpt_build_tiles_write(const bpt_build_side *sides, int n_sides, const int32_
 int bpt_build_pair_numbers(const int32_t *pair_eid_theirs, const int32_t *grp_eids_mine, int64_t n_slots, int64_t n_edges,
                            int32_t *number, int32_t *pairs, void *stream);
 
+/* How many rows of one or two CSR sides have edges (what the length of the work items of a graph of two node sets goes by): side s
+ * has n_units[s] units, sorted by row, a row's one after the other.  counts: BPT_COUNT_PARTS int32 a side in memory the device can
+ * write (pinned host memory saves the caller a copy); their sum is the number.  Rows are compared, not used as an index: any value does. */
+#define BPT_COUNT_PARTS 64
+int bpt_build_count_rows(const int64_t *const row[2], const int64_t *const indptr_units[2], const int64_t n_units[2], int n_sides,
+                         int32_t *counts, void *stream);
+
 /* Waits until everything enqueued on the stream has run (for a caller that reads an info block in pinned host memory). */
 int bpt_build_wait(void *stream);
 

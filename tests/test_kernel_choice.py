@@ -53,16 +53,32 @@ def test_segment_length_of_the_tile_plans_follows_the_mean_degree():
     assert graphop._tile_seg_len(fake_plan(4097, 524224)) == 256           # 128
 
 
-def test_segment_length_of_two_node_sets_counts_half_of_the_rows():
-    """Sentences attending to others: 26 edges a node are 52 a token; both ways of asking agree."""
+def test_segment_length_of_two_node_sets_is_left_to_the_plan():
+    """The sizes of a graph of two node sets do not say how many of its rows have edges; both ways of asking agree."""
     two = SimpleNamespace(n_rows=6905, n_index_nodes=6838, n_edges=176728, n_items=6905)
-    q, k, units = torch.empty(6905, 8, 64), torch.empty(6838, 8, 64), torch.empty(7000, dtype=torch.int64)
-    for n_edges, want in ((6905 * 16 - 1, 64), (6905 * 16, 128), (176728, 128), (6905 * 40 - 1, 128), (6905 * 40, 256)):
-        two.n_edges = n_edges
-        assert graphop._tile_seg_len(two) == want
-        assert graphop._tile_seg_without_plan(units, n_edges, q, k, 8, 64, 0.0, None, graphop._SETTINGS) == want
+    q, k, units = torch.empty(6905, 8, 64), torch.empty(6838, 8, 64), torch.empty(6900, dtype=torch.int64)
+    assert graphop._tile_seg_len(two) == plan.SEG_BY_ROWS
+    assert graphop._tile_seg_without_plan(units, 176728, q, k, 8, 64, 0.0, None, graphop._SETTINGS) == plan.SEG_BY_ROWS
     same = SimpleNamespace(n_rows=6905, n_index_nodes=6905, n_edges=176728, n_items=6905)
     assert graphop._tile_seg_len(same) == 64
+
+
+def test_segment_length_by_the_rows_that_have_edges():
+    """Of 1000 rows every second or every one has 20, 40 or 100 edges, in units of up to 32 and as a plain CSR with its empty rows."""
+    for edges, step, want in ((20, 1, 64), (20, 2, 64), (40, 1, 128), (40, 2, 128), (100, 1, 256), (100, 2, 256)):
+        rows = torch.arange(0, 1000, step)
+        ends = torch.arange(32, edges + 32, 32).clamp(max=edges)
+        row = rows.repeat_interleave(len(ends))
+        indptr = torch.cat([torch.zeros(1, dtype=torch.int64), (torch.arange(len(rows))[:, None] * edges + ends[None]).reshape(-1)])
+        plain = torch.zeros(1001, dtype=torch.int64)
+        plain[rows + 1] = edges
+        for r, ip in ((row, indptr), (torch.arange(1000), plain.cumsum(0))):
+            assert plan.rows_with_edges([(r, ip)]) == [len(rows)]
+            assert plan.seg_lens_by_rows([(r, ip, len(rows) * edges)] * 2) == [want] * 2
+    assert plan.tile_seg_len(176728, 6905) == 64                           # 26 edges a node, but 51 a row with edges
+    none = torch.zeros(0, dtype=torch.int64)
+    assert plan.seg_lens_by_rows([(none, none.new_zeros(1), 0)] * 2) == [64, 64]
+    assert plan.rows_with_edges([(none, none)]) == [0]                     # (refused by the plan's validation, not here)
 
 
 def test_choice_of_the_tile_kernels_without_a_plan_to_look_at():
