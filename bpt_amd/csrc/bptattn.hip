@@ -4472,13 +4472,28 @@ int spmm_edge_generic(const bpt_plan *P, const void *W, const void *X, void *Y, 
 }
 
 // ---- fast launchers ----
-// Wavefronts a work item for the kernels that walk single rows.  They run graphs of fewer than 1536 items, and there a launch lasts
+// Wavefronts a work item for the kernels that walk single rows.  The fused kernels walk them on graphs of fewer than 1536 items (with
+// row groups switched off: on any), the separate operators' SpMM where it is handed a plan without groups.  There a launch lasts
 // as long as its longest item: 16 batches of four edges one after the other, each a round trip to memory.  Forward / destination
-// side / source side, one -> four -> eight wavefronts an item, us: L = 64 (127 items) 9.4 / 13.7 / 7.2 -> 4.7 / 6.4 / 4.2 -> 4.8 / 5.6 / 4.2;
-// L = 256, k = 16 (539) 11.1 / 16.6 / 14.4 -> 9.2 / 11.7 / 11.6 -> 8.2 / 9.4 / 10.8; bfloat16, L = 256 (516) 12.2 / 16.9 / 15.5 -> 6.0 / 7.3 /
-// 7.4 -> 5.6 / 6.6 / 7.4; L = 400 (816) 11.4 / 16.6 / 13.8 -> 7.9 / 10.0 / 11.0 -> 9.0 / 10.4 / 10.5; L = 700, k = 1 (1434) 15.7 / 21.2 /
-// 15.0 -> 10.1 / 12.0 / 12.2 -> 11.3 / 12.8 / 12.6.  Larger launches fill the GPU with a wavefront an item.
-inline int row_parts(const bpt_plan *P) { return P->n_items <= 640 ? 8 : P->n_items <= 2048 ? 4 : 1; }
+// side / source side, one -> four -> eight wavefronts an item, 8 x 64 float32 unless said otherwise, us:
+//   127 items (L = 64)                  9.4 / 13.7 / 7.2  -> 4.7 / 6.4 / 4.2   -> 4.8 / 5.6 / 4.2;   SpMM 7.5 -> 4.0 -> 3.8
+//   539 (L = 256, k = 16)              11.1 / 16.6 / 14.4 -> 9.2 / 11.7 / 11.6 -> 8.2 / 9.4 / 10.8;  bfloat16 12.2 / 16.9 / 15.5 -> 6.0 / 7.3 / 7.4 -> 5.6 / 6.6 / 7.4
+//   816 (L = 400)                      11.4 / 16.6 / 13.8 -> 7.9 / 10.0 / 11.0 -> 9.0 / 10.4 / 10.5; SpMM 10.8 -> 6.7 -> 6.7
+//   1434 (L = 700, k = 1)              15.7 / 21.2 / 15.0 -> 10.1 / 12.0 / 12.2 -> 11.3 / 12.8 / 12.6; SpMM 11.6 -> 7.9 -> 7.1
+//   2050 (L = 1000, k = 1, no groups)  16.8 / 22.2 / 17.9 -> 11.0 / 14.0 / 13.6 -> 14.1 / 17.0 / 15.4; SpMM 11.6 -> 8.4 -> 8.2
+// Larger launches fill the GPU with a wavefront an item.  Rows of 1024 columns take twice the registers and the LDS: eight
+// wavefronts an item of them are one round of the chip up to 256 items, beyond it four are faster.  16 x 64:
+//   268 (L = 130, k = 4)               16.3 / 22.7 / 16.7 -> 7.9 / 10.4 / 9.3   -> 8.2 / 10.2 / 9.4;   bfloat16 16.4 / 21.3 / 19.6 -> 7.6 / 9.6 / 8.7 -> 8.3 / 8.7 / 11.4
+//   324 (L = 160, k = 4)               15.7 / 22.1 / 18.1 -> 8.5 / 10.2 / 13.1  -> 10.2 / 12.0 / 12.6; bfloat16 16.0 / 20.7 / 19.8 -> 7.6 / 9.6 / 11.5 -> 10.5 / 10.8 / 12.2
+//   585 (L = 256, k = 16, both ways)   18.7 / 26.8 / 23.4 -> 18.6 / 21.2 / 19.4 -> 22.3 / 24.3 / 21.2
+// A float32 forward of 512 columns or more that already has a wavefront for each of the 1024 SIMDs and 25 edges or more an
+// item waits for the rate of its loads, not for one item: one -> four, 8 x 64 and 16 x 64, 983 items of 25 790 edges 11.7 -> 12.4 and 19.1 ->
+// 21.0; 957 of 32 613 12.0 -> 12.2 and 19.7 -> 20.4; (1018 of 23 540 11.3 -> 11.2 and 18.2 -> 18.7; 756 items 11.2 -> 10.4 and 18.6 -> 17.1).
+inline int row_parts(const bpt_plan *P, int columns, bool forward_f32 = false) {
+    if (P->n_items <= (columns > 512 ? 288 : 640)) return 8;
+    if (forward_f32 && columns >= 512 && P->n_items > 800 && P->n_items <= 1024 && P->n_edges >= 25000) return 1;
+    return P->n_items <= 2048 ? 4 : 1;
+}
 template <typename T, int H, int D>
 int run_sddmm_fast(const bpt_plan *P, const void *A, const void *B, void *y, hipStream_t s) {
     if (P->n_items == 0) return BPT_OK;
@@ -4497,7 +4512,7 @@ int run_spmm_fast(const bpt_plan *P, const void *W0, const void *X0, void *Y0, c
     hipLaunchKernelGGL((k_spmm_fast<T, WT, H, D, FAST_BATCH, NOUT, 0, NW>), dim3(NW == 1 ? grid_for(P) : (int)P->n_items),                    \
                        dim3(NW == 1 ? BLOCK : NW * WAVE), 0, s, *P, (const WT *)W0, (const T *)X0, (T *)Y0, (const WT *)W1, (const T *)X1, \
                        (T *)Y1, ws, ws1)
-        switch (row_parts(P)) {
+        switch (row_parts(P, H * D)) {
         case 8: LAUNCH_SPMM(8); break;
         case 4: LAUNCH_SPMM(4); break;
         default: LAUNCH_SPMM(1); break;
@@ -4998,7 +5013,7 @@ int run_attn_fwd(const bpt_plan *P, const void *q, const void *k, const void *v,
 #define LAUNCH_FWD_ROWS(NW)                                                                                                           \
     hipLaunchKernelGGL((k_attn_fwd<T, H, D, FAST_BATCH, NW>), dim3(NW == 1 ? grid_for(P) : (int)P->n_items), dim3(NW == 1 ? BLOCK : NW * WAVE), \
                        0, s, *P, (const T *)q, (const T *)k, (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E)
-            switch (row_parts(P)) {
+            switch (row_parts(P, H * D, sizeof(T) == 4)) {
             case 8: LAUNCH_FWD_ROWS(8); break;
             case 4: LAUNCH_FWD_ROWS(4); break;
             default: LAUNCH_FWD_ROWS(1); break;
@@ -5164,7 +5179,7 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
     hipLaunchKernelGGL((k_attn_bwd_dst<T, H, D, FAST_BATCH, NW>), dim3(NW == 1 ? grid_for(Pin) : (int)Pin->n_items),                         \
                        dim3(NW == 1 ? BLOCK : NW * WAVE), 0, s, *Pin, (const T *)q, (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, \
                        (T *)dq, pbuf, dsbuf, ws_rows, scale, scale * LOG2E)
-            switch (row_parts(Pin)) {
+            switch (row_parts(Pin, H * D)) {
             case 8: LAUNCH_DST_ROWS(8); break;
             case 4: LAUNCH_DST_ROWS(4); break;
             default: LAUNCH_DST_ROWS(1); break;
@@ -5397,6 +5412,15 @@ int bpt_gather_probe(const void *region, int64_t region_bytes, int waves_per_cu,
     default: return BPT_ERR_SIZE;
     }
     return launch_status();
+}
+
+int bpt_wavefronts_per_item(const bpt_plan *plan, int kernel, int h, int d, int dtype) {
+    if (!plan) return BPT_ERR_NULL;
+    if (kernel < BPT_KERNEL_ATTN_FWD || kernel > BPT_KERNEL_ATTN_BWD_SRC || h < 1 || d < 1) return BPT_ERR_SHAPE;
+    if (dtype != BPT_F32 && dtype != BPT_BF16) return BPT_ERR_DTYPE;
+    const size_t elem = dtype == BPT_F32 ? 4 : 2;
+    if (has_tiles(plan, h, d, elem)) return tile_parts(plan, h, elem);
+    return row_parts(plan, h * d, kernel == BPT_KERNEL_ATTN_FWD && dtype == BPT_F32);
 }
 
 int bpt_profile_kernel(int which, void *start_event, void *stop_event) {

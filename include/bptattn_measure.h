@@ -9,6 +9,8 @@
 
 #include <stdint.h>
 
+#include "bptattn.h"
+
 #ifdef __cplusplus
 extern "C" {
 #endif
@@ -21,6 +23,11 @@ int bpt_set_force_generic(int on);
  * the launch stream, so a benchmark can time one kernel with HIP events; 0 switches it off. */
 enum { BPT_KERNEL_NONE = 0, BPT_KERNEL_ATTN_FWD = 1, BPT_KERNEL_ATTN_BWD_DST = 2, BPT_KERNEL_ATTN_BWD_SRC = 3 };
 int bpt_profile_kernel(int which, void *start_event, void *stop_event);
+
+/* How many wavefronts share a work item (a plan without groups) or a tile and head (a plan with groups of 16 rows, d = 64; heads
+ * of fewer columns are asked for with their own number and d = 64 too) in `kernel`, one of BPT_KERNEL_ATTN_*: the choice by
+ * sizes that the launch makes.  For tests of that choice; negative: bpt_status. */
+int bpt_wavefronts_per_item(const bpt_plan *plan, int kernel, int h, int d, int dtype);
 
 /* Measurement aid (no counterpart in the reference): launches a kernel in which waves_per_cu wavefronts per compute unit
  * (a multiple of 4, at most 64) each read `iters` batches of in_flight (2, 4 or 8) pseudo-random 1 KB rows of `region`

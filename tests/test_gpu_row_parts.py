@@ -1,6 +1,8 @@
 """The kernels that walk single rows, with four or eight wavefronts a work item (small graphs): rows of every length around a batch
 and around a wavefront's share, split rows, rows without edges, against the float64 oracle; one path for each size of graph, the
 same bits on every run; an infinite row reaches its neighbours and nobody else."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -14,7 +16,9 @@ DEGREES = [0, 1, 2, 3, 4, 5, 7, 8, 9, 12, 13, 15, 16, 17, 20, 28, 29, 31, 32, 33
 def graph(n):
     from bpt_amd import graphbuilder as gb
     rng = np.random.default_rng(n)
-    deg = np.array([DEGREES[i % len(DEGREES)] for i in range(n)]) if n <= 128 else np.minimum([DEGREES[i % len(DEGREES)] for i in range(n)], 40)
+    deg = np.array([DEGREES[i % len(DEGREES)] for i in range(n)])
+    if n not in (33, 128, 800):                                   # (800: the long rows that a float32 forward gives one wavefront each)
+        deg = np.minimum(deg, 40)
     dst = np.repeat(np.arange(n), deg)
     src = rng.integers(1, n, len(dst))                            # (node 0 is nobody's neighbour)
     perm = rng.permutation(len(dst))
@@ -23,12 +27,12 @@ def graph(n):
     return src, dst, tuple(x.to(DEV) for x in (ROW, IR, out_csr[2], out_csr[1], COL, IC, in_csr[2], in_csr[1]))
 
 
-@pytest.mark.parametrize("n", [33, 128, 600, 700, 1000])
+@pytest.mark.parametrize("n", [33, 128, 600, 700, 800, 1000])
 @pytest.mark.parametrize("heads,d,dtype", [(8, 64, torch.float32), (16, 64, torch.float32), (4, 64, torch.float32), (8, 32, torch.float32), (8, 64, torch.bfloat16),
                                            (16, 64, torch.bfloat16)])
 def test_small_graphs_match_the_oracle(n, heads, d, dtype):
     from oracle import torch_ops
-    from bpt_amd import op, plan
+    from bpt_amd import _lib, op, plan
     plan.plan_cache.clear()
     src, dst, args = graph(n)
     gen = torch.Generator().manual_seed(13)
@@ -41,6 +45,9 @@ def test_small_graphs_match_the_oracle(n, heads, d, dtype):
     for a, b in zip(*runs):
         assert torch.equal(a, b)
     items = [p.n_items for p, _ in plan.plan_cache._d.values()]
+    lib, struct = _lib.attn_lib(), next(iter(plan.plan_cache._d.values()))[0].struct
+    want_parts = 8 if n < 289 or (n == 600 and heads * d <= 512) else 1 if n == 800 and dtype == torch.float32 and heads * d >= 512 else 4
+    assert lib.bpt_wavefronts_per_item(ctypes.byref(struct), 1, heads, d, 0 if dtype == torch.float32 else 2) == want_parts
     assert max(items) < 1536 and not any(p._groups for p, _ in plan.plan_cache._d.values())       # (rows, not groups of rows)
     f64 = lambda x: x.detach().cpu().double()
     want = torch_ops.attention_fwd_bwd(torch.from_numpy(src), torch.from_numpy(dst), f64(q), f64(k), f64(v), f64(do))

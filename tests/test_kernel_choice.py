@@ -1,11 +1,12 @@
 """Which kernel family a call takes is decided on the host from the plan's sizes and the dtype (graphop._tiles,
 _tiles_backward, _tile_seg_len, and _tile_seg_without_plan where no plan is needed to decide) and where a plan is built from its size and the caller's preference
 (plan._build_on_device, PlanCache.get(prefer_device=...)).  CPU only: the rules are plain functions of sizes."""
+import ctypes
 from types import SimpleNamespace
 
 import torch
 
-from bpt_amd import graphop, plan
+from bpt_amd import _lib, graphop, plan
 
 
 def fake_plan(n_rows, n_edges):
@@ -192,3 +193,32 @@ def test_order_of_the_destination_side_tile_groups():
     assert p.ensure_groups(plan.TILE_GROUP_R) is not a
     chunks = np.asarray(a["host"]["chunks"])
     assert chunks[0] == 0 and chunks[-1] == len(a["host"]["grp_ptr"]) - 1
+
+
+FWD, DST, SRC, F32, BF16 = 1, 2, 3, 0, 2                                    # bptattn_measure.h, bptattn.h
+
+
+def test_wavefronts_of_a_row():
+    """Kernels that walk single rows: eight, four or one wavefront an item.  Rows of 1024 columns are shared by eight up to
+    288 items only (585 items, forward: 22.3 us with eight, 18.7 with one), and a float32 forward with a wavefront for nearly every
+    SIMD and many edges an item takes one."""
+    lib = _lib.attn_lib()
+
+    def parts(n_items, n_edges, kernel, h, d, dtype):
+        p = _lib.PlanStruct()
+        p.n_rows, p.n_items, p.n_edges = n_items, n_items, n_edges
+        return lib.bpt_wavefronts_per_item(ctypes.byref(p), kernel, h, d, dtype)
+
+    for kernel in (FWD, DST, SRC):
+        for dtype in (F32, BF16):
+            for h, d, most in ((4, 64, 640), (8, 64, 640), (8, 32, 640), (16, 64, 288)):
+                assert [parts(n, 20000, kernel, h, d, dtype) for n in (1, most, most + 1, 801, 1024, 2048, 2049)] == [8, 8, 4, 4, 4, 4, 1]
+            for h, d in ((4, 64), (8, 32), (8, 64), (16, 64)):
+                want = 1 if kernel == FWD and dtype == F32 and h * d >= 512 else 4
+                for n, e in ((801, 25000), (1024, 25000), (1024, 60000)):
+                    assert parts(n, e, kernel, h, d, dtype) == want
+                for n, e in ((800, 25000), (1025, 25000), (1024, 24999)):
+                    assert parts(n, e, kernel, h, d, dtype) == 4
+    for bad in ((0, 8, 64, F32), (4, 8, 64, F32), (FWD, 0, 64, F32), (FWD, 8, 0, F32), (FWD, 8, 64, 1), (FWD, 8, 64, 9)):
+        assert lib.bpt_wavefronts_per_item(ctypes.byref(_lib.PlanStruct()), *bad) < 0
+    assert lib.bpt_wavefronts_per_item(None, FWD, 8, 64, F32) < 0
