@@ -4834,12 +4834,25 @@ inline bool has_tiles(const bpt_plan *P, int h, int d, size_t elem) {
 //   584 of 3 (L = 512)      5.8 / 6.6 / 8.1 -> 5.1 / 6.0 / 6.4 -> 5.0 / 6.4 / 5.5;    1048 of 3    6.6 / 7.5 / 8.5 -> 6.4 / 7.6 / 8.4 -> 6.9 / 9.2 / 9.1
 //   1032 of 9              11.4 / 12.9 / 12.0 -> 9.0 / 11.2 / 10.0 -> 8.3 / 10.1 / 10.4;  2056 of 9   13.1 / 14.8 / 14.8 -> 11.8 / 14.0 / 14.4 -> 12.8 / 18.7 / 15.8
 //   4112 of 9              18.3 / 21.0 / 22.1 -> 17.8 / 23.8 / 22.3 -> 20.1 / 30.3 / 27.1
-inline int tile_parts(const bpt_plan *P, int heads, size_t elem) {
+// The same line holds with dropout, the score term and narrow heads (one head a workgroup in parts, two otherwise); float32:
+//   L = 512, dropout                10.9 / 13.6 / 15.6 -> 7.9 / 10.2 / 10.4  -> 7.8 / 10.3 / 9.1;   term and dropout 11.8 / 16.5 / 16.2 -> 8.6 / 12.3 / 10.5 -> 8.0 / 11.9 / 8.2
+//   window 128, L = 4096, dropout   27.9 / 39.4 / 24.5 -> 22.3 / 35.6 / 20.9 -> 25.0 / 37.2 / 22.6; 6 x 50 with dropout 34.8 / 37.8 / 21.7 -> 26.6 / 28.0 / 20.8 -> 26.8 / 30.9 / 19.9
+//   L = 4096, k = 32, dropout       39.5 / 56.2 / 48.2 -> 34.8 / 54.5 / 43.6 -> 40.1 / 61.7 / 46.8; term and dropout 43.0 / 64.8 / 49.2 -> 37.5 / 63.9 / 45.1 -> 42.0 / 72.0 / 48.6
+//                                   6 x 50 with dropout 55.9 / 59.4 / 42.7 -> 33.5 / 44.1 / 34.5 -> 38.4 / 49.3 / 37.4
+//   L = 8192, k = 4 (one part)      35.8 / 55.6 / 38.3 -> 38.9 / 62.7 / 40.6;  6 x 50 with dropout 44.3 / 46.2 / 36.2 -> 47.0 / 50.1 / 38.4
+// bfloat16, dropout: L = 512 7.2 / 7.9 / 13.4 -> 5.9 / 6.6 / 9.7 -> 5.6 / 6.7 / 6.7; window 128, L = 4096 15.4 / 16.2 / 15.6 -> 12.5 / 14.7 / 15.0 -> 13.9 /
+// 19.3 / 16.4; 6 x 50 there 19.2 / 21.3 / 13.0 -> 14.4 / 17.3 / 12.8 -> 15.3 / 18.9 / 12.6.  Of 290 kernels of a hundred graphs drawn at random over all
+// of these the rule slowed one by more than 1 % against one part (a window of 52, forward 16.9 -> 17.8).
+// Two parts of launches that fill the chip about twice (6500 to 8192 wavefronts) pay on the source side (window 256, above) and with dropout
+// (forward there 108.2 -> 106.8), not for a float32 forward without: L = 7000, k = 32 51.7 -> 53.9, L = 6000, k = 64 63.5 -> 66.0, window 128, L =
+// 16000 61.1 -> 63.1, window 256 90.8 -> 92.4 (plain_forward; below, 5600 to 6300 wavefronts 42.7 -> 42.9, 46.2 -> 45.7, 48.4 -> 47.0).
+inline int tile_parts(const bpt_plan *P, int heads, size_t elem, bool plain_forward = false) {
     const int64_t wavefronts = P->n_groups * heads, blocks = P->n_grp_entries / TILE_R;
+    const int64_t most = plain_forward ? 13000 : 16384;
     auto pays = [&](int parts) {
         const int64_t w = wavefronts * parts, each = blocks / std::max<int64_t>(P->n_groups * parts, 1);      // (blocks of a part, rounded down)
         if (elem == 2) return w <= 2400 || (parts == 2 && w <= 4608 && each >= 4);
-        return w <= 3072 || (w <= 6144 && each >= 2) || (parts == 2 && w <= 16384 && each >= 4);
+        return w <= 3072 || (w <= 6144 && each >= 2) || (parts == 2 && w <= most && each >= 4);
     };
     return pays(4) ? 4 : pays(2) ? 2 : 1;
 }
@@ -4929,7 +4942,7 @@ int run_attn_fwd(const bpt_plan *P, const void *q, const void *k, const void *v,
         if constexpr (D == 64 && sizeof(T) == 4) {
             if (has_tiles(P, H, D, sizeof(T)) && ((drop.thr == 0 && !bias) || P->grp_eids)) {
                 constexpr int HW = H >= 4 ? 4 : H;          // heads per workgroup
-                const int parts = tile_parts(P, H, sizeof(T));
+                const int parts = tile_parts(P, H, sizeof(T), drop.thr == 0 && !bias);
 #define LAUNCH_FWD_TILE_PARTS(DR, BI, SP)                                                                                            \
     hipLaunchKernelGGL((k_attn_fwd_tile<T, H, D, HW, DR, BI, false, SP>), dim3(group_grid(P) * (H * SP / HW)), dim3(HW * WAVE), 0, s, *P, \
                        (const T *)q, (const T *)k, (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed, drop.inv, bias, \
@@ -5419,7 +5432,7 @@ int bpt_wavefronts_per_item(const bpt_plan *plan, int kernel, int h, int d, int 
     if (kernel < BPT_KERNEL_ATTN_FWD || kernel > BPT_KERNEL_ATTN_BWD_SRC || h < 1 || d < 1) return BPT_ERR_SHAPE;
     if (dtype != BPT_F32 && dtype != BPT_BF16) return BPT_ERR_DTYPE;
     const size_t elem = dtype == BPT_F32 ? 4 : 2;
-    if (has_tiles(plan, h, d, elem)) return tile_parts(plan, h, elem);
+    if (has_tiles(plan, h, d, elem)) return tile_parts(plan, h, elem, kernel == BPT_KERNEL_ATTN_FWD);
     return row_parts(plan, h * d, kernel == BPT_KERNEL_ATTN_FWD && dtype == BPT_F32);
 }
 

@@ -26,7 +26,7 @@ int bpt_profile_kernel(int which, void *start_event, void *stop_event);
 
 /* How many wavefronts share a work item (a plan without groups) or a tile and head (a plan with groups of 16 rows, d = 64; heads
  * of fewer columns are asked for with their own number and d = 64 too) in `kernel`, one of BPT_KERNEL_ATTN_*: the choice by
- * sizes that the launch makes.  For tests of that choice; negative: bpt_status. */
+ * sizes that the launch makes for a layer without dropout and score term.  For tests of that choice; negative: bpt_status. */
 int bpt_wavefronts_per_item(const bpt_plan *plan, int kernel, int h, int d, int dtype);
 
 /* Measurement aid (no counterpart in the reference): launches a kernel in which waves_per_cu wavefronts per compute unit

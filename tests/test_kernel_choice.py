@@ -222,3 +222,29 @@ def test_wavefronts_of_a_row():
     for bad in ((0, 8, 64, F32), (4, 8, 64, F32), (FWD, 0, 64, F32), (FWD, 8, 0, F32), (FWD, 8, 64, 1), (FWD, 8, 64, 9)):
         assert lib.bpt_wavefronts_per_item(ctypes.byref(_lib.PlanStruct()), *bad) < 0
     assert lib.bpt_wavefronts_per_item(None, FWD, 8, 64, F32) < 0
+
+
+def test_wavefronts_of_a_tile_and_head():
+    """Dense tiles: four, two or one wavefront a tile and head, by the wavefronts of the launch and the blocks each keeps; a float32
+    forward stops at 6500 wavefronts (L = 7000, k = 32: 51.7 us with one, 53.9 with two), the backward at 8192."""
+    lib = _lib.attn_lib()
+
+    def parts(n_groups, blocks, kernel, h=8, dtype=F32):
+        p = _lib.PlanStruct()
+        p.n_rows = p.n_items = 16 * n_groups
+        p.n_index_nodes = p.n_rows
+        p.grp_R, p.n_groups, p.grp_max_chunk, p.n_grp_entries = 16, n_groups, n_groups, 16 * n_groups * blocks
+        p.grp_members = p.grp_ptr = p.grp_entries = p.grp_chunks = 16          # (looked at for null only)
+        return lib.bpt_wavefronts_per_item(ctypes.byref(p), kernel, h, 64, dtype)
+
+    for kernel in (FWD, DST, SRC):
+        # float32: wavefronts 8 n_groups
+        assert [parts(n, 1, kernel) for n in (1, 96, 97, 192, 193)] == [4, 4, 2, 2, 1]
+        assert [parts(n, 4, kernel) for n in (193, 384, 385)] == [2, 2, 1]
+        assert [parts(n, 8, kernel) for n in (192, 193, 384, 385, 812)] == [4, 2, 2, 2, 2]
+        assert parts(813, 8, kernel) == parts(1024, 8, kernel) == (1 if kernel == FWD else 2)
+        assert parts(1025, 8, kernel) == 1 and parts(812, 7, kernel) == 1
+        assert [parts(n, 8, kernel, h=16) for n in (96, 97, 406, 513)] == [4, 2, 2, 1]
+        # bfloat16
+        assert [parts(n, 1, kernel, dtype=BF16) for n in (75, 76, 150, 151)] == [4, 2, 2, 1]
+        assert [parts(n, 8, kernel, dtype=BF16) for n in (150, 151, 288, 289)] == [2, 2, 2, 1]
