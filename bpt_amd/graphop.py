@@ -782,7 +782,9 @@ def prepare_training(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indi
                                        (row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg, order_src)])
     if plans is None:
         return
-    pi, po = plans
+    # (through the cache, as every other call: what stands there now is what the passes are going to find)
+    pi = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, None), built=plans[0])
+    po = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg_len=seg, prefer_device=True, groups=(TILE_ROWS, order_src), built=plans[1])
     if not (pi.covers_all_edges and po.covers_all_edges) or TILE_BACKWARD is not None:
         return                       # (with the hook set the passes choose for themselves)
     fwd, bwd = (_native.ATTN_FWD, _native.ATTN_BWD) if narrow_h is None else (_native.ATTN_FWD_NARROW, _native.ATTN_BWD_NARROW)

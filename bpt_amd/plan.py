@@ -795,11 +795,12 @@ class PlanCache:
         return tuple((t.data_ptr(), t.numel(), t._version, t.device) if t is not None else None
                      for t in tensors) + (n_rows, n_index, seg_len, on_device)
 
-    def get(self, row, indptr, eid, indices, n_rows=None, n_index_nodes=None, seg_len=DEFAULT_SEG_LEN, prefer_device=False, groups=None):
+    def get(self, row, indptr, eid, indices, n_rows=None, n_index_nodes=None, seg_len=DEFAULT_SEG_LEN, prefer_device=False, groups=None, built=None):
         """n_rows None: as many rows as `row` mentions (ops that only produce edge outputs).  prefer_device: build on the GPU
         whatever the graph's size, unless set_device_build() fixed the place (the tile kernels ask for this: the GPU
         builder's groups of 16 run them as fast or faster on every graph measured).  groups = (R, order_mode): row groups the caller
-        asks the plan for next; a plan built on the GPU for this call forms them along with it.  seg_len may be SEG_BY_ROWS."""
+        asks the plan for next; a plan built on the GPU for this call forms them along with it.  seg_len may be SEG_BY_ROWS.  built: what
+        put_tile_plans has just returned for the same arguments, taken where the cache had no room for it."""
         tensors = (row, indptr, eid, indices)
         on_device = _build_on_device(eid, n_rows) or bool(prefer_device and DEVICE_BUILD is None and eid.is_cuda and n_rows is not None)
         key = self._key(tensors, n_rows, n_index_nodes, seg_len, on_device)
@@ -811,6 +812,8 @@ class PlanCache:
                 if self.hits % 64 == 0:
                     self._evict()                   # row groups and pair mappings are added to plans after insertion
                 return hit[0]
+        if built is not None:
+            return built
         self.misses += 1
         if seg_len == SEG_BY_ROWS:
             seg_len, = seg_lens_by_rows([(row, indptr, eid.numel())])
