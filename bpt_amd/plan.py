@@ -815,6 +815,8 @@ class PlanCache:
         if built is not None:
             return built
         self.misses += 1
+        # (the GPU builder and the count of rows read 64-bit numbers; the host builder takes any)
+        row, indptr, eid, indices = (t if t is None or t.dtype == torch.int64 else t.to(torch.int64) for t in tensors)
         if seg_len == SEG_BY_ROWS:
             seg_len, = seg_lens_by_rows([(row, indptr, eid.numel())])
         if on_device:

@@ -94,3 +94,26 @@ def test_rows_with_edges_are_counted(n):
     assert plan.rows_with_edges(sides) == want
     assert plan.rows_with_edges(sides[:1]) == want[:1]
     assert plan.rows_with_edges([tuple(t.cpu() for t in side) for side in sides]) == want
+
+
+@pytest.mark.parametrize("heads,d", [(8, 64), (6, 50)])
+@pytest.mark.parametrize("n_q,n_k", [(3200, 3201), (3200, 3200)])
+def test_index_tensors_of_32_bits(n_q, n_k, heads, d):
+    """Widened for the plans that are built on the GPU, as the host builder widens them: the same results."""
+    from bpt_amd import graphbuilder as gb
+    from bpt_amd import op, plan
+    rng = np.random.default_rng(7)
+    dst = np.repeat(np.arange(n_q), 12).astype(np.int64)
+    out_csr, in_csr, row, ir, col, ic = gb.get_csrs_bipartite(rng.integers(0, n_k, len(dst)), dst, n_k, n_q)
+    args = tuple(x.to(DEV) for x in (row, ir, out_csr[2], out_csr[1], col, ic, in_csr[2], in_csr[1]))
+    gen = torch.Generator().manual_seed(47)
+    q, do = (torch.randn(n_q, heads, d, generator=gen).to(DEV) for _ in range(2))
+    k, v = (torch.randn(n_k, heads, d, generator=gen).to(DEV) for _ in range(2))
+    leaves = [x.requires_grad_(True) for x in (q, k, v)]
+    runs = []
+    for graph in (args, tuple(t.to(torch.int32) for t in args)):
+        plan.plan_cache.clear()
+        o = op.bpt_attention(*graph, *leaves)
+        runs.append((o.detach(),) + torch.autograd.grad(o, leaves, do))
+    for a, b in zip(*runs):
+        assert torch.equal(a, b)
