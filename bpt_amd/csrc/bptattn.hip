@@ -2833,6 +2833,223 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
     }
 }
 
+// ---- The separate operators on tiles, float32: Y[row] = sum of W[eid, head] X[idx] and y[eid, head] = <A[row, head, :], B[idx, head, :]>
+// on the tile walk above, one of its products each.  Beside the rows, what these kernels move is the (n_edges, H) edge tensor, found by
+// the edge ids of a block's pairs (grp_eids): a record of H floats per edge, of which a wavefront, one head, wants four bytes.  So
+// the wavefronts of a workgroup share them (SHARED): each reads or writes a quarter of a block's pairs (half with two heads a
+// workgroup) with all the workgroup's heads in one 16-byte access, and they meet in LDS, one barrier a block.  Every wavefront for
+// itself: the texture addresser works through 64 places per instruction, four instructions a block and head.
+// 8 heads, per launch without merges, row groups of 8 -> each for itself -> shared: L = 8192, k = 4 SpMM 33.9 -> 31 -> 26.6 (out-CSR) and 33 ->
+// 27 -> 22.6 us (in-CSR), SDDMM 32.5 -> 27.7 -> 23.4 and 31.5 -> 28 -> 21.6; 32-graph batch SpMM 43 -> 40 -> 34, SDDMM 43 -> 41 -> 34;
+// window 128 SpMM 38 -> 17 to 23 -> 12 to 19, SDDMM 29 -> 19 to 23 -> 15 to 18.  What bounds them now: at L = 8192 the node rows read and
+// written by themselves are 13 us at the rate of a large copy, the products 7; the rest is the tiles' first loads and the edge tensor's places.
+template <int HW> struct HeadPack;
+template <> struct HeadPack<4> { typedef floatx4v vec; };
+template <> struct HeadPack<2> { typedef float vec __attribute__((ext_vector_type(2))); };
+
+// The sums of a tile again, pair by pair.  A product over a block multiplies the weight 0 of a pair that does not exist with the row's
+// columns: a row that is not finite reaches members that do not have it.  A wavefront whose sums are not all finite comes here, where
+// only pairs that exist are added, so that such a row reaches its own neighbours and no others.
+template <bool NARROW>
+__device__ __forceinline__ void spmm_tile_by_pairs(const bpt_plan &P, const TileCtx &t, const float *Wh, uint32_t WH, const char *xb, uint32_t RB, floatx4v (&acc)[4]) {
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
+    for (int p = t.p_begin; p < t.p_end; ++p) {
+        const int4 en = reinterpret_cast<const int4 *>(P.grp_entries)[p];
+        const float4 x = tile_row4<NARROW>(xb + ((uint32_t)en.x * RB + t.offv));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int m = 4 * t.g + r;                            // accumulators: register r of every lane belongs to member 4 g + r
+            if (!((en.y >> m) & 1)) continue;
+            const float w = Wh[(size_t)(uint32_t)P.grp_eids[(size_t)p * TILE_R + m] * WH];
+            acc[0][r] = fmaf(w, x.x, acc[0][r]); acc[1][r] = fmaf(w, x.y, acc[1][r]); acc[2][r] = fmaf(w, x.z, acc[2][r]); acc[3][r] = fmaf(w, x.w, acc[3][r]);
+        }
+    }
+}
+
+template <int H, int D, int HW, bool SHARED, bool NARROW = false, int SP = 1>
+__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(SP > 1 ? 5 : 6))) void k_spmm_tile(
+    bpt_plan P, const float *__restrict__ W, const float *__restrict__ X, float *__restrict__ Y, float *__restrict__ ws, Narrow nw) {
+    static_assert(SP == 1 || !SHARED, "the parts of a tile have blocks of their own: no barrier a block");
+    using vec = typename HeadPack<SHARED ? HW : 2>::vec;
+    constexpr int RW = SHARED ? 4 / HW : 4;                       // registers r (entries 4 r + g of a block) that a wavefront fetches weights of
+    const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * 4 : (uint32_t)(H * D * 4), WH = NARROW ? (uint32_t)nw.heads : (uint32_t)H;
+    TileCtx t;
+    if (!tile_begin<float, H, D, HW, NARROW, SP>(P, t, nw)) return;
+    constexpr int ENT = TILE_CHUNK * 2, PIECE = SP > 1 ? TILE_PART_FLOATS : ENT;
+    static_assert(PIECE >= ENT, "the list fits");
+    __shared__ __attribute__((aligned(16))) float piece[HW][PIECE];
+    __shared__ float wt[SHARED ? 2 : 1][SHARED ? HW : 1][SHARED ? 4 * WAVE : 1];         // this block's weights and the next one's: [head][r][lane]
+    int2 *ent = reinterpret_cast<int2 *>(piece[t.wv]);
+    const int c = t.c, g = t.g, r0 = SHARED ? t.wv * RW : 0;
+    const char *xb = reinterpret_cast<const char *>(X);
+    const float *const Wh = W + t.head - (SHARED ? t.wv : 0);
+    floatx4v acc[4];
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
+    TileEntryRegs er;
+    if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
+    // the edge ids of a block's pairs are asked for two blocks ahead, the weights one block ahead
+    int xe[RW];
+    float w[SHARED ? 1 : 4];
+    vec wv[SHARED ? RW : 1];
+    auto edges = [&](int first_entry) {
+#pragma unroll
+        for (int i = 0; i < RW; ++i) xe[i] = P.grp_eids[(size_t)min(first_entry + 4 * (r0 + i) + g, t.p_end - 1) * TILE_R + c];
+    };
+    auto weights = [&]() {                                        // (n_edges: the pair does not exist)
+#pragma unroll
+        for (int i = 0; i < RW; ++i) {
+            const bool there = (uint32_t)xe[i] < (uint32_t)P.n_edges;
+            const float *const at = Wh + (size_t)((uint32_t)xe[i] * WH);
+            if constexpr (SHARED) {
+#pragma unroll
+                for (int k = 0; k < HW; ++k) wv[i][k] = 0.f;
+                if (there) wv[i] = *reinterpret_cast<const vec *>(at);
+            } else {
+                w[i] = 0.f;
+                if (there) w[i] = *at;
+            }
+        }
+    };
+    int stage = 0;
+    auto put = [&]() {
+        if constexpr (SHARED) {
+#pragma unroll
+            for (int i = 0; i < RW; ++i)
+#pragma unroll
+                for (int k = 0; k < HW; ++k) wt[stage][k][WAVE * (r0 + i) + t.lane] = wv[i][k];
+        }
+    };
+    if (t.p_end > t.p_begin) edges(t.p_begin);
+    issue_loads_first();
+    for (int p0 = t.p_begin; p0 < t.p_end; p0 += TILE_CHUNK) {
+        const int cnt = min(TILE_CHUNK, t.p_end - p0), nblk = (cnt + TILE_R - 1) / TILE_R;
+        if (p0 != t.p_begin) tile_ask_entries(P, p0, cnt, t.lane, er);
+        tile_put_entries(er, ent, cnt, t.lane);
+        if (p0 == t.p_begin) {
+            weights();
+            edges(p0 + TILE_R);
+            put();
+        }
+        for (int b = 0; b < nblk; ++b) {
+            if constexpr (SHARED) __syncthreads();                // (the other stage is read to the end too)
+            const int nv = min(TILE_R, cnt - TILE_R * b);
+            int has = 0;
+            float4 xr[4];
+            float wc[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int2 en = ent[TILE_R * b + 4 * r + g];
+                has |= ((en.y >> c) & 1) << r;
+                xr[r] = tile_row4<NARROW>(xb + ((uint32_t)en.x * RB + t.offv));
+                if constexpr (!SHARED) wc[r] = w[r];
+            }
+            issue_loads_first();
+            const bool more = p0 + TILE_R * (b + 1) < t.p_end;
+            if (more) {
+                weights();
+                edges(p0 + TILE_R * (b + 2));
+            }
+            issue_loads_first();
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if constexpr (SHARED) wc[r] = wt[stage][t.wv][WAVE * r + t.lane];
+                wc[r] = ((has >> r) & 1) ? wc[r] : 0.f;
+            }
+            tile_axpy_upto(wc, xr, acc, nv);
+            issue_loads_first();
+            stage ^= SHARED ? 1 : 0;
+            if (more) put();
+        }
+        wave_lds_fence();                                         // the piece is read to the end before the next one is staged
+    }
+    float zero = 0.f;                                             // 0 times a sum is 0 unless the sum is not finite
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) zero = fmaf(acc[nb][r], 0.f, zero);
+    if (__builtin_amdgcn_ballot_w64(!(zero == 0.f)) != 0) spmm_tile_by_pairs<NARROW>(P, t, W + t.head, WH, xb, RB, acc);
+    if constexpr (SP > 1) {
+        tile_park(piece[t.wv], acc, t.lane);
+        __syncthreads();
+        tile_meet_and_store<SP, H, D, NARROW>(piece[t.wv % (HW / SP)], (HW / SP) * PIECE, t, Y, ws, nw);
+    } else {
+        tile_store_rows<H, D, false, NARROW>(t, acc, 1.f, Y, ws, nw);
+    }
+}
+
+template <int H, int D, int HW, bool SHARED, bool NARROW = false, int SP = 1>
+__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(5))) void k_sddmm_tile(
+    bpt_plan P, const float *__restrict__ A, const float *__restrict__ B, float *__restrict__ y, Narrow nw) {
+    static_assert(SP == 1 || !SHARED, "the parts of a tile have blocks of their own: no barrier a block");
+    using vec = typename HeadPack<SHARED ? HW : 2>::vec;
+    constexpr int RW = SHARED ? 4 / HW : 4;
+    const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * 4 : (uint32_t)(H * D * 4), WH = NARROW ? (uint32_t)nw.heads : (uint32_t)H;
+    TileCtx t;
+    if (!tile_begin<float, H, D, HW, NARROW, SP>(P, t, nw)) return;
+    __shared__ int2 ent_lds[HW][TILE_CHUNK];
+    __shared__ __attribute__((aligned(16))) float kt_lds[HW][TILE_R * TILE_KT_STRIDE];
+    __shared__ float wt[SHARED ? 2 : 1][SHARED ? HW : 1][SHARED ? 4 * WAVE : 1];
+    int2 *ent = ent_lds[t.wv];
+    float *kt = kt_lds[t.wv];
+    const int c = t.c, g = t.g, r0 = SHARED ? t.wv * RW : 0;
+    TileEntryRegs er;
+    if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
+    issue_loads_first();
+    const char *bb = reinterpret_cast<const char *>(B);
+    const char *const arow = reinterpret_cast<const char *>(A) + (size_t)max(t.member.x, 0) * RB + t.offa;
+    float *const yh = y + t.head - (SHARED ? t.wv : 0);
+    float ab[16];
+    int stage = 0;
+    struct Blk {
+        float4 rows[4];
+        int xe[RW];                                               // edge ids of the pairs that this lane stores (n_edges or more: none)
+    };
+    for (int p0 = t.p_begin; p0 < t.p_end; p0 += TILE_CHUNK) {
+        const int cnt = min(TILE_CHUNK, t.p_end - p0), nblk = (cnt + TILE_R - 1) / TILE_R;
+        if (p0 != t.p_begin) tile_ask_entries(P, p0, cnt, t.lane, er);
+        tile_put_entries(er, ent, cnt, t.lane);
+        auto issue = [&](Blk &K, int b) {
+#pragma unroll
+            for (int i = 0; i < RW; ++i) {
+                const int e = p0 + TILE_R * b + 4 * (r0 + i) + g;
+                const int id = P.grp_eids[(size_t)min(e, t.p_end - 1) * TILE_R + c];
+                K.xe[i] = e < t.p_end ? id : -1;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) K.rows[r] = tile_row4<NARROW>(bb + ((uint32_t)ent[TILE_R * b + 4 * r + g].x * RB + t.offv));
+        };
+        auto rest = [](Blk &, int) {};
+        auto compute = [&](const Blk &K) {
+            float kr[16];
+            tile_rows_to_operand<NARROW>(kt, K.rows, c, g, kr, nw);
+            const floatx4v st = tile_dot(kr, ab);
+            if constexpr (SHARED) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) wt[stage][t.wv][WAVE * r + t.lane] = st[r];
+                __syncthreads();                                  // (the stage before this one is read to the end too)
+            }
+#pragma unroll
+            for (int i = 0; i < RW; ++i) {
+                if ((uint32_t)K.xe[i] >= (uint32_t)P.n_edges) continue;
+                float *const at = yh + (size_t)((uint32_t)K.xe[i] * WH);
+                if constexpr (SHARED) {
+                    vec x;
+#pragma unroll
+                    for (int k = 0; k < HW; ++k) x[k] = wt[stage][k][WAVE * (r0 + i) + t.lane];
+                    *reinterpret_cast<vec *>(at) = x;
+                } else {
+                    *at = st[i];
+                }
+            }
+            stage ^= SHARED ? 1 : 0;
+        };
+        tile_walk_first_ahead<Blk>(nblk, issue, rest, compute, [&]() { if (p0 == t.p_begin) tile_load16<NARROW>(arow, ab, g, nw); });
+        wave_lds_fence();
+    }
+}
+
 // ---- Dense tiles for bfloat16 rows.  Same walk and the same lane roles as the float32 tile kernels above, on
 // v_mfma_f32_16x16x32_bf16 (products over the 64 columns: two instructions) and v_mfma_f32_16x16x16_bf16 (products over
 // the 16 entries of a block: one instruction per four output columns), float32 accumulation:
@@ -4741,7 +4958,11 @@ int spmm_fast(const bpt_plan *P, const void *W, const void *Xp, void *Y, void *w
 // SDDMM / SpMM with automatic family choice
 bool spmm_grp_ok(const bpt_plan *P, int h, int d, int dtype);
 int sddmm_grp(const bpt_plan *P, const void *A, const void *B, void *y, int h, int d, int dtype, hipStream_t s);
+bool product_tiles_ok(const bpt_plan *P, int h, int d, int dtype);
+int sddmm_tile(const bpt_plan *P, const void *A, const void *B, void *y, int h, int d, hipStream_t s);
+int spmm_tile(const bpt_plan *P, const void *W, const void *X, void *Y, void *ws, int h, int d, hipStream_t s);
 int sddmm(const bpt_plan *P, const void *A, const void *B, void *y, int h, int d, int dtype, hipStream_t s) {
+    if (product_tiles_ok(P, h, d, dtype)) return sddmm_tile(P, A, B, y, h, d, s);
     if (fast_shape(h, d, dtype) && aligned16(A) && aligned16(B)) {
         if (spmm_grp_ok(P, h, d, dtype)) return sddmm_grp(P, A, B, y, h, d, dtype, s);
         return sddmm_fast(P, A, B, y, h, d, dtype, s);
@@ -4750,6 +4971,7 @@ int sddmm(const bpt_plan *P, const void *A, const void *B, void *y, int h, int d
 }
 int spmm_grp(const bpt_plan *P, const void *W, const void *X, void *Y, void *ws, int h, int d, int dtype, hipStream_t s, int accumulate = 0);
 int spmm(const bpt_plan *P, const void *W, const void *X, void *Y, void *ws, int h, int d, int dtype, hipStream_t s) {
+    if (product_tiles_ok(P, h, d, dtype) && aligned16(ws)) return spmm_tile(P, W, X, Y, ws, h, d, s);
     if (fast_shape(h, d, dtype) && aligned16(X) && aligned16(Y) && aligned16(ws)) {
         // a plan that carries row groups and their edge ids: one row load per entry instead of one per edge
         if (spmm_grp_ok(P, h, d, dtype)) return spmm_grp(P, W, X, Y, ws, h, d, dtype, s);
@@ -4759,6 +4981,7 @@ int spmm(const bpt_plan *P, const void *W, const void *X, void *Y, void *ws, int
 }
 
 inline int64_t round16(int64_t b) { return (b + 15) & ~(int64_t)15; }
+inline int product_tile_heads(int h) { return (h + 3) & ~3; }        // heads of a partial row of the separate operators on tiles, 64 columns each
 
 // dropout of the fused path: threshold on the 32-bit hash (0 = off), seed, 1 / (1 - p)
 struct Dropout {
@@ -4855,6 +5078,94 @@ inline int tile_parts(const bpt_plan *P, int heads, size_t elem, bool plain_forw
         return w <= 3072 || (w <= 6144 && each >= 2) || (parts == 2 && w <= most && each >= 4);
     };
     return pays(4) ? 4 : pays(2) ? 2 : 1;
+}
+
+// a tile in parts: one head a workgroup, so that no wavefront of it lies past the last head
+inline Narrow narrow_parts(Narrow nw, int parts) {
+    if (parts > 1) nw.slices = nw.heads;
+    return nw;
+}
+
+// The separate operators on tiles: float32, groups of 16 rows with their edge ids.  Heads of 64 columns, 4, 8 or 16 of them, whose rows
+// lie on 16 bytes, take the kernels of those shapes, all others of 4 to 64 columns the narrow ones (rows on 4 bytes).
+bool product_tiles_ok(const bpt_plan *P, int h, int d, int dtype) {
+    return dtype == BPT_F32 && !g_force_generic.load(std::memory_order_relaxed) && P->n_edges > 0 && P->grp_eids && d >= 4 && d <= 64 && h <= 16 &&
+           P->n_groups > 0 && P->grp_R == TILE_R && P->grp_members && P->grp_ptr && P->grp_entries && P->grp_chunks && P->grp_max_chunk > 0 &&
+           8 * P->grp_max_chunk >= P->n_groups && P->n_grp_entries >= 0 && fits32(std::max(P->n_rows, P->n_index_nodes), (int64_t)h * d * 4) &&
+           fits32(P->n_edges, h);
+}
+inline Narrow product_narrow(int h, int d) { return Narrow{d, h, product_tile_heads(h), (h + NARROW_HW - 1) / NARROW_HW}; }
+
+template <int H>
+int run_spmm_tile(const bpt_plan *P, const float *W, const float *X, float *Y, float *ws, hipStream_t s) {
+    const int parts = tile_parts(P, H, 4);
+#define LAUNCH(SH, SP) \
+    hipLaunchKernelGGL((k_spmm_tile<H, 64, 4, SH, false, SP>), dim3(group_grid(P) * (H * SP / 4)), dim3(4 * WAVE), 0, s, *P, W, X, Y, ws, Narrow{})
+    if (parts == 4) LAUNCH(false, 4);
+    else if (parts == 2) LAUNCH(false, 2);
+    else if (aligned16(W)) LAUNCH(true, 1);
+    else LAUNCH(false, 1);
+#undef LAUNCH
+    const int st = launch_status();
+    if (st != BPT_OK || P->n_heavy == 0) return st;
+    hipLaunchKernelGGL((k_combine_sum_v4<float>), dim3((int)P->n_heavy, H * 64 / (4 * WAVE), 1), dim3(BLOCK), 0, s, P->heavy, (const float *)ws, Y,
+                       (float *)nullptr, H * 64, (size_t)0);
+    return launch_status();
+}
+int spmm_tile(const bpt_plan *P, const void *W_, const void *X_, void *Y_, void *ws_, int h, int d, hipStream_t s) {
+    const float *W = (const float *)W_, *X = (const float *)X_;
+    float *Y = (float *)Y_, *ws = (float *)ws_;
+    if (d == 64 && aligned16(X) && aligned16(Y)) {
+        if (h == 4) return run_spmm_tile<4>(P, W, X, Y, ws, s);
+        if (h == 8) return run_spmm_tile<8>(P, W, X, Y, ws, s);
+        if (h == 16) return run_spmm_tile<16>(P, W, X, Y, ws, s);
+    }
+    const int parts = tile_parts(P, h, 4);
+    const Narrow nw = narrow_parts(product_narrow(h, d), parts);
+#define LAUNCH(HW, SH, SP) \
+    hipLaunchKernelGGL((k_spmm_tile<16, 64, HW, SH, true, SP>), dim3(group_grid(P) * nw.slices), dim3(HW * WAVE), 0, s, *P, W, X, Y, ws, nw)
+    if (parts == 4) LAUNCH(4, false, 4);
+    else if (parts == 2) LAUNCH(2, false, 2);
+    else if (h % NARROW_HW == 0 && (reinterpret_cast<uintptr_t>(W) & 7u) == 0) LAUNCH(NARROW_HW, true, 1);
+    else LAUNCH(NARROW_HW, false, 1);
+#undef LAUNCH
+    const int st = launch_status();
+    if (st != BPT_OK || P->n_heavy == 0) return st;
+    hipLaunchKernelGGL((k_combine_sum3<float, true>), dim3((int)P->n_heavy, nw.h * 64 / (4 * WAVE), 1), dim3(BLOCK), 0, s, P->heavy, (int)P->n_heavy,
+                       (const float *)ws, Y, (const int32_t *)nullptr, (const float *)nullptr, (float *)nullptr, (float *)nullptr, nw.h * 64, (size_t)0, nw);
+    return launch_status();
+}
+
+template <int H>
+int run_sddmm_tile(const bpt_plan *P, const float *A, const float *B, float *y, hipStream_t s) {
+    const int parts = tile_parts(P, H, 4);
+#define LAUNCH(SH, SP) \
+    hipLaunchKernelGGL((k_sddmm_tile<H, 64, 4, SH, false, SP>), dim3(group_grid(P) * (H * SP / 4)), dim3(4 * WAVE), 0, s, *P, A, B, y, Narrow{})
+    if (parts == 4) LAUNCH(false, 4);
+    else if (parts == 2) LAUNCH(false, 2);
+    else if (aligned16(y)) LAUNCH(true, 1);
+    else LAUNCH(false, 1);
+#undef LAUNCH
+    return launch_status();
+}
+int sddmm_tile(const bpt_plan *P, const void *A_, const void *B_, void *y_, int h, int d, hipStream_t s) {
+    const float *A = (const float *)A_, *B = (const float *)B_;
+    float *y = (float *)y_;
+    if (d == 64 && aligned16(A) && aligned16(B)) {
+        if (h == 4) return run_sddmm_tile<4>(P, A, B, y, s);
+        if (h == 8) return run_sddmm_tile<8>(P, A, B, y, s);
+        if (h == 16) return run_sddmm_tile<16>(P, A, B, y, s);
+    }
+    const int parts = tile_parts(P, h, 4);
+    const Narrow nw = narrow_parts(product_narrow(h, d), parts);
+#define LAUNCH(HW, SH, SP) \
+    hipLaunchKernelGGL((k_sddmm_tile<16, 64, HW, SH, true, SP>), dim3(group_grid(P) * nw.slices), dim3(HW * WAVE), 0, s, *P, A, B, y, nw)
+    if (parts == 4) LAUNCH(4, false, 4);
+    else if (parts == 2) LAUNCH(2, false, 2);
+    else if (h % NARROW_HW == 0 && (reinterpret_cast<uintptr_t>(y) & 7u) == 0) LAUNCH(NARROW_HW, true, 1);
+    else LAUNCH(NARROW_HW, false, 1);
+#undef LAUNCH
+    return launch_status();
 }
 
 bool spmm_grp_ok(const bpt_plan *P, int h, int d, int dtype) {
@@ -5238,12 +5549,6 @@ template <typename T> bool narrow_ok(const bpt_plan *P, const Narrow &nw) {
     return has_tiles(P, nw.h, 64, sizeof(T)) && (P->grp_eids != nullptr);
 }
 
-// a tile in parts: one head a workgroup, so that no wavefront of it lies past the last head
-inline Narrow narrow_parts(Narrow nw, int parts) {
-    if (parts > 1) nw.slices = nw.heads;
-    return nw;
-}
-
 template <typename T>
 int run_attn_fwd_narrow(const bpt_plan *P, const void *q, const void *k, const void *v, void *o, float *lse, void *ws, float scale, Dropout drop,
                         const Narrow &nw, const Keep &keep, hipStream_t s) {
@@ -5448,11 +5753,15 @@ int64_t bpt_workspace_bytes(int op, const bpt_plan *plan, const bpt_plan *plan_t
     if (!plan || h < 1 || d < 1) return -1;
     const int64_t C = (int64_t)h * d, a = (int64_t)acc_size(dtype);
     const int64_t s0 = plan->n_slots, s1 = plan_t ? plan_t->n_slots : 0;
+    // partial rows of a SpMM on this plan (on tiles: whole heads of 64 columns)
+    auto rows = [&](const bpt_plan *P) {
+        return P ? round16(P->n_slots * std::max(C, product_tiles_ok(P, h, d, dtype) ? (int64_t)product_tile_heads(h) * 64 : 0) * a) : 0;
+    };
     switch (op) {
-        case BPT_OP_MASKEDMM_BWD: return round16((s0 > s1 ? s0 : s1) * C * a);
-        case BPT_OP_NODE_MUL_EDGE_BWD:
-        case BPT_OP_SPMM_FWD: return round16(s0 * C * a);
-        case BPT_OP_SPMM_BWD: return round16(s1 * C * a);
+        case BPT_OP_MASKEDMM_BWD: return std::max(rows(plan), rows(plan_t));
+        case BPT_OP_NODE_MUL_EDGE_BWD: return round16(s0 * C * a);
+        case BPT_OP_SPMM_FWD: return rows(plan);
+        case BPT_OP_SPMM_BWD: return rows(plan_t);
         case BPT_OP_ATTN_FWD: return round16(s0 * (C + 2 * h) * 4);
         case BPT_OP_SOFTMAX_FWD: return WAVE % h == 0 ? round16(s0 * h * 2 * a) : 0;      // (m, s) of every segment and head
         case BPT_OP_SOFTMAX_BWD: return WAVE % h == 0 ? round16(s0 * h * a) : 0;

@@ -199,13 +199,37 @@ def release_workspaces():
         _SCRATCH.clear()
 
 
-def _spmm_ref(plan, x, h, d, cfg):
-    """The plan to hand a SpMM- or SDDMM-shaped op: with row groups (one load of a neighbour row per group entry instead of one
+def _spmm_struct(plan, x, h, d, cfg):
+    """The plan struct to hand a SpMM- or SDDMM-shaped op: with row groups (one load of a neighbour row per group entry instead of one
     per edge) where the row-group kernels apply, else the plain plan."""
     if not (cfg.use_groups and cfg.grouped_ops and attention_supported(x) and plan.covers_all_edges and plan.has_indices
             and plan.n_edges > 0 and max(plan.n_rows, plan.n_index_nodes) * h * d * x.element_size() < 2 ** 32):
-        return plan.ref
-    return ctypes.byref(plan.ensure_groups(_group_rows(x, h, d, plan, cfg), GROUP_ORDER_SRC)["struct"])
+        return plan.struct
+    return plan.ensure_groups(_group_rows(x, h, d, plan, cfg), GROUP_ORDER_SRC)["struct"]
+
+
+def _product_tiles(n_edges, n_rows, n_index_nodes, x, h, d, cfg):
+    """Whether a SpMM- or SDDMM-shaped op takes the tile kernels if its plan covers every edge (_product_plan says why)."""
+    return (cfg.use_groups and cfg.grouped_ops and cfg.use_tiles and cfg.group_rows is None and not _FORCE_GENERIC and x.dim() == 3
+            and x.dtype == torch.float32 and 4 <= d <= 64 and h <= 16 and n_edges > 0 and n_rows == n_index_nodes
+            and n_rows * h * d * 4 < 2 ** 32 and n_edges * h < 2 ** 32)
+
+
+def _product_plan(row, indptr, eid, indices, n_rows, n_index_nodes, x, h, d, cfg, order=None):
+    """(plan, the struct to hand over) for a SpMM- or SDDMM-shaped op over one CSR side: tiles for float32 rows of 4 to 64
+    columns a head and up to 16 heads of a graph of one node set, built on the GPU, else _spmm_struct's choice.  Both products of
+    a tile's blocks go to the matrix cores, a row is loaded once per 16 rows instead of 8 or 4, and heads that no other
+    specialised kernel has are read as they are: L = 8192, k = 4, 8 x 64, per launch 33 -> 22 to 27 us (comment at k_spmm_tile), and the plans of a
+    new graph take 0.6 ms instead of the 22 of the host's row groups.  A SpMM into another number of rows stays with the row groups: the CSR
+    of the edge types (n_rows) has few rows of some hundred edges with no neighbours in common.  order: of the groups, as ensure_groups
+    takes it; the tile plans of the fused attention are taken where they are there."""
+    if indices is not None and _product_tiles(eid.numel(), n_rows, n_index_nodes, x, h, d, cfg):
+        plan = plan_cache.get(row, indptr, eid, indices, n_rows, n_index_nodes, seg_len=_tile_seg_of(eid.numel(), n_rows, n_index_nodes),
+                              prefer_device=True, groups=(TILE_ROWS, order))
+        if plan.covers_all_edges:
+            return plan, plan.ensure_groups(TILE_ROWS, order)["struct"]
+    plan = plan_cache.get(row, indptr, eid, indices, n_rows, n_index_nodes)
+    return plan, _spmm_struct(plan, x, h, d, cfg)
 
 
 def _edge_out(plan, shape, like):
@@ -221,11 +245,12 @@ def maskedmm_csr_forward(row, indptr, eid, indices, A, B):
     h, d = _hd(A)
     _expect_index(eid, indices)
     _expect_shape(B, (B.size(0),) + tuple(A.shape[1:]), "B")
-    plan = plan_cache.get(row, indptr, eid, indices, A.size(0), B.size(0))
+    # (the rows here are the edges' sources, as in the source side of the fused backward)
+    plan, struct = _product_plan(row, indptr, eid, indices, A.size(0), B.size(0), A, h, d, cfg, _plan.tile_order_src(A.size(0), eid.size(0)))
     e = eid.size(0)
     y = _edge_out(plan, (e,) if A.dim() == 2 else (e, h), A)
     with _on_device_of(A):
-        check_attn(_LIB.bpt_maskedmm_csr_forward(_spmm_ref(plan, A, h, d, cfg), _ptr(A), _ptr(B), _ptr(y), h, d, _dtype(A), _stream()),
+        check_attn(_LIB.bpt_maskedmm_csr_forward(ctypes.byref(struct), _ptr(A), _ptr(B), _ptr(y), h, d, _dtype(A), _stream()),
                    "maskedmm_csr_forward")
     return y
 
@@ -243,13 +268,14 @@ def maskedmm_csr_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c,
     _expect_shape(B, (B.size(0),) + tuple(A.shape[1:]), "B")
     _expect_shape(eid_c, eid_r.shape, "eid_c")
     _expect_edges(dy, eid_r.size(0), h, "dy", A.dim() == 2)
-    plan_r = plan_cache.get(row, indptr_r, eid_r, indices_r, A.size(0), B.size(0))
-    plan_c = plan_cache.get(col, indptr_c, eid_c, indices_c, B.size(0), A.size(0))
+    plan_r, struct_r = _product_plan(row, indptr_r, eid_r, indices_r, A.size(0), B.size(0), A, h, d, cfg, _plan.tile_order_src(A.size(0), eid_r.size(0)))
+    plan_c, struct_c = _product_plan(col, indptr_c, eid_c, indices_c, B.size(0), A.size(0), A, h, d, cfg)
     dA, dB = torch.empty_like(A), torch.empty_like(B)
     dt = _dtype(A)
-    ws, nws = _workspace(OP_MASKEDMM_BWD, plan_r, plan_c, h, d, dt, A.device)
+    ref_r, ref_c = ctypes.byref(struct_r), ctypes.byref(struct_c)
+    ws, nws = _workspace(OP_MASKEDMM_BWD, plan_r, plan_c, h, d, dt, A.device, plan_ref=ref_r, plan_t_ref=ref_c)
     with _on_device_of(A):
-        check_attn(_LIB.bpt_maskedmm_csr_backward(_spmm_ref(plan_r, A, h, d, cfg), _spmm_ref(plan_c, A, h, d, cfg), _ptr(A), _ptr(B), _ptr(dy), _ptr(dA), _ptr(dB),
+        check_attn(_LIB.bpt_maskedmm_csr_backward(ref_r, ref_c, _ptr(A), _ptr(B), _ptr(dy), _ptr(dA), _ptr(dB),
                                                   _ptr(ws), nws, h, d, dt, _stream()), "maskedmm_csr_backward")
     return [dA, dB]
 
@@ -296,7 +322,7 @@ def sparse_softmax_forward(row, indptr, eid, x):
     _expect_index(eid, None)
     if x.dim() not in (1, 2) or x.size(0) != eid.size(0):
         raise ValueError(f"x must be ({eid.size(0)},) or ({eid.size(0)}, h), got {tuple(x.shape)}")
-    plan = plan_cache.get(row, indptr, eid, None, None, None)
+    plan = plan_cache.get(row, indptr, eid, None, None, None, prefer_device=True)
     y = (torch.empty_like if plan.covers_all_edges else torch.zeros_like)(x)
     ws, nws = _workspace(OP_SOFTMAX_FWD, plan, None, _edge_h(x), 1, _dtype(x), x.device)
     with _on_device_of(x):
@@ -313,7 +339,7 @@ def sparse_softmax_backward(row, indptr, eid, y, dy):
     if y.dim() not in (1, 2) or y.size(0) != eid.size(0):
         raise ValueError(f"y must be ({eid.size(0)},) or ({eid.size(0)}, h), got {tuple(y.shape)}")
     _expect_shape(dy, y.shape, "dy")
-    plan = plan_cache.get(row, indptr, eid, None, None, None)
+    plan = plan_cache.get(row, indptr, eid, None, None, None, prefer_device=True)
     dx = (torch.empty_like if plan.covers_all_edges else torch.zeros_like)(dy)
     ws, nws = _workspace(OP_SOFTMAX_BWD, plan, None, _edge_h(dy), 1, _dtype(y), y.device)
     with _on_device_of(y):
@@ -337,14 +363,20 @@ def vector_spmm_forward(row, indptr, eid, indices, edata, x, *, n_rows=None, out
     _expect_index(eid, indices)
     _expect_edges(edata, eid.size(0), h, "edata", x.dim() == 2)
     n_out = x.size(0) if n_rows is None else int(n_rows)
-    plan = plan_cache.get(row, indptr, eid, indices, n_out, x.size(0))
+    square = out is None and n_rows is None
+    if square:
+        plan, struct = _product_plan(row, indptr, eid, indices, n_out, x.size(0), x, h, d, cfg)
+    else:
+        plan = plan_cache.get(row, indptr, eid, indices, n_out, x.size(0))
     y = torch.empty_like(x) if n_rows is None else torch.empty((n_out,) + tuple(x.shape[1:]), dtype=x.dtype, device=x.device)
     dt = _dtype(x)
-    ws, nws = _workspace(OP_SPMM_FWD, plan, None, h, d, dt, x.device)
+    ws, nws = _workspace(OP_SPMM_FWD, plan, None, h, d, dt, x.device, plan_ref=ctypes.byref(struct) if square else None)
     if out is not None and (out.shape != y.shape or out.dtype != y.dtype or out.device != y.device or not out.is_contiguous()):
         raise ValueError("out must be a contiguous tensor of the result's shape, dtype and device")
     with _on_device_of(x):
-        ref = _spmm_ref(plan, x, h, d, cfg)
+        if not square:
+            struct = _spmm_struct(plan, x, h, d, cfg)
+        ref = ctypes.byref(struct)
         if out is not None:
             st = _LIB.bpt_vector_spmm_accumulate(ref, _ptr(edata), _ptr(x), _ptr(out), _ptr(ws), nws, h, d, dt, _stream())
             if st == 0:
@@ -370,14 +402,15 @@ def vector_spmm_backward(row, indptr, eid, indices, col, indptr_t, eid_t, indice
     _expect_edges(edata, eid.size(0), h, "edata", x.dim() == 2)
     # y = dy may have another number of rows than x (a rectangular operator: attention to a memory of another length)
     _expect_shape(dy, (dy.size(0),) + tuple(x.shape[1:]), "dy")
-    plan = plan_cache.get(row, indptr, eid, indices, dy.size(0), x.size(0))
-    plan_t = plan_cache.get(col, indptr_t, eid_t, indices_t, x.size(0), dy.size(0))
+    plan, struct = _product_plan(row, indptr, eid, indices, dy.size(0), x.size(0), x, h, d, cfg)
+    plan_t, struct_t = _product_plan(col, indptr_t, eid_t, indices_t, x.size(0), dy.size(0), x, h, d, cfg, _plan.tile_order_src(x.size(0), eid.size(0)))
     dedata = (torch.empty_like if plan.covers_all_edges else torch.zeros_like)(edata)
     dx = torch.empty_like(x)
     dt = _dtype(x)
-    ws, nws = _workspace(OP_SPMM_BWD, plan, plan_t, h, d, dt, x.device)
+    ref, ref_t = ctypes.byref(struct), ctypes.byref(struct_t)
+    ws, nws = _workspace(OP_SPMM_BWD, plan, plan_t, h, d, dt, x.device, plan_ref=ref, plan_t_ref=ref_t)
     with _on_device_of(x):
-        check_attn(_LIB.bpt_vector_spmm_backward(_spmm_ref(plan, x, h, d, cfg), _spmm_ref(plan_t, x, h, d, cfg), _ptr(edata), _ptr(dy), _ptr(x), _ptr(dedata), _ptr(dx),
+        check_attn(_LIB.bpt_vector_spmm_backward(ref, ref_t, _ptr(edata), _ptr(dy), _ptr(x), _ptr(dedata), _ptr(dx),
                                                  _ptr(ws), nws, h, d, dt, _stream()), "vector_spmm_backward")
     return [dedata, dx]
 
@@ -438,7 +471,7 @@ def rel_bias_forward(col, indptr_c, eid_c, type_slot, q, table, used_types=None,
         if by_pair:
             raise ValueError("by_pair needs used_types")
         plan = plan_cache.get(col, indptr_c, eid_c, type_slot, q.size(0), table.size(0))
-        ref, n_used = _spmm_ref(plan, q, h, d, cfg), 0
+        ref, n_used = ctypes.byref(_spmm_struct(plan, q, h, d, cfg)), 0
     bias = (torch.empty if plan.covers_all_edges else torch.zeros)((h, E) if by_pair else (E + 1, h), dtype=torch.float32, device=q.device)
     if not by_pair and (used_types is None or not plan.n_items):
         bias[E].zero_()                     # (the kernel of the other form clears the spare row itself)

@@ -802,7 +802,7 @@ class PlanCache:
         asks the plan for next; a plan built on the GPU for this call forms them along with it.  seg_len may be SEG_BY_ROWS.  built: what
         put_tile_plans has just returned for the same arguments, taken where the cache had no room for it."""
         tensors = (row, indptr, eid, indices)
-        on_device = _build_on_device(eid, n_rows) or bool(prefer_device and DEVICE_BUILD is None and eid.is_cuda and n_rows is not None)
+        on_device = _build_on_device(eid, n_rows) or bool(prefer_device and DEVICE_BUILD is None and eid.is_cuda)
         key = self._key(tensors, n_rows, n_index_nodes, seg_len, on_device)
         with self._lock:
             hit = self._d.get(key)
@@ -819,8 +819,8 @@ class PlanCache:
         row, indptr, eid, indices = (t if t is None or t.dtype == torch.int64 else t.to(torch.int64) for t in tensors)
         if seg_len == SEG_BY_ROWS:
             seg_len, = seg_lens_by_rows([(row, indptr, eid.numel())])
-        if on_device:
-            nr = n_rows if n_rows is not None else (int(row[-1]) + 1 if row.numel() else 0)
+        nr = n_rows if n_rows is not None or not on_device else (int(row[-1]) + 1 if row.numel() else 0)
+        if on_device and 0 <= nr < 2 ** 31 - 1:         # (a last row that is no row: the host builder says so)
             ni = n_index_nodes if n_index_nodes is not None else nr
             plan = DevicePlan(row, indptr, eid, indices, nr, ni, eid.device, seg_len, groups=groups)
         else:

@@ -102,6 +102,8 @@ int64_t bpt_plan_struct_bytes(void);
 
 const char *bpt_strerror(int status);
 
+/* float32 calls of the SDDMM- and SpMM-shaped ops on a plan with grp_R = 16 and grp_eids take the tile kernels whatever h <= 16 and 4 <= d <= 64
+ * are; their workspace holds partial rows of whole heads of 64 columns, so ask bpt_workspace_bytes with the plan of the call. */
 /* Bytes of workspace the call needs (0 possible).  op: one of the BPT_OP_* below.  BPT_OP_ATTN_BWD covers every form of the fused
  * backward; BPT_OP_ATTN_BWD_PLAIN is bpt_attention_backward without a score term, which needs no more and in bfloat16 much less. */
 enum {
