@@ -35,7 +35,7 @@ using at::Tensor;
 
 namespace {
 
-enum Kind { ATTN_FWD = 0, ATTN_BWD = 1, ATTN_FWD_NARROW = 2, ATTN_BWD_NARROW = 3 };
+enum Kind { ATTN_FWD = 0, ATTN_BWD = 1, ATTN_FWD_NARROW = 2, ATTN_BWD_NARROW = 3, MM_FWD = 4, MM_BWD = 5, SPMM_FWD = 6, SPMM_BWD = 7, SOFTMAX = 8 };
 
 constexpr size_t MAX_TENSORS = 8, MAX_EXTRA = 7, MAX_ENTRIES = 512;
 
@@ -247,17 +247,16 @@ struct Attention : torch::autograd::Function<Attention> {
 
 // Through the autograd function also where a tangent of forward-mode differentiation is carried: the function refuses it, the bare
 // forward would drop it.
-bool differentiated(const Tensor &q, const Tensor &k, const Tensor &v) {
-    if (at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad())) return true;
-    for (const Tensor *t : {&q, &k, &v})
-        if (t->_fw_grad(/*level=*/0).defined()) return true;
+bool differentiated(std::initializer_list<const Tensor *> tensors) {
+    for (const Tensor *t : tensors)
+        if ((at::GradMode::is_enabled() && t->requires_grad()) || t->_fw_grad(/*level=*/0).defined()) return true;
     return false;
 }
 
 // op.BPTAttention with the host work in native code: the same call, the same result
 Tensor attention(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r, const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c,
                  const Tensor &eid_c, const Tensor &indices_c, const Tensor &q, const Tensor &k, const Tensor &v, double scale, double p, uint64_t seed) {
-    if (differentiated(q, k, v))
+    if (differentiated({&q, &k, &v}))
         return Attention::apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale, p, (int64_t)seed);
     return std::get<0>(attention_forward(col, indptr_c, eid_c, indices_c, q, k, v, scale, p, seed));
 }
@@ -390,9 +389,202 @@ struct NarrowAttention : torch::autograd::Function<NarrowAttention> {
 Tensor attention_narrow(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r, const Tensor &indices_r, const Tensor &col,
                         const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c, const Tensor &q, const Tensor &k, const Tensor &v,
                         int64_t h, double scale, double p, uint64_t seed) {
-    if (differentiated(q, k, v))
+    if (differentiated({&q, &k, &v}))
         return NarrowAttention::apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, h, scale, p, (int64_t)seed);
     return std::get<0>(narrow_forward(col, indptr_c, eid_c, indices_c, rows(q), rows(k), rows(v), h, scale, p, (int64_t)seed, Copies{}));
+}
+
+// ---- the separate operators (modules/op.py:10-58 of the reference) -----------------------------------------------------------
+// masked_mm, sparse_softmax and vec_spmm of (n, h, d) rows and (E, h) edge tensors whose plans are known and cover every edge.  A
+// training pass through the chain cost the host 325 us in Python, at L = 512 as at L = 8192: three calls of its autograd functions,
+// and their backwards on autograd's thread, which has to be handed the interpreter for each.
+using Two = std::tuple<Tensor, Tensor>;
+
+bool rows_of_heads(const Tensor &a) { return a.dim() == 3 && a.is_cuda() && a.is_contiguous() && dtype_code(a.scalar_type()) >= 0; }
+bool same_heads(const Tensor &b, const Tensor &a) { return b.dim() == 3 && like(b, a) && b.size(1) == a.size(1) && b.size(2) == a.size(2); }
+bool per_edge(const Tensor &e, const Tensor &a, const Tensor &eid) {
+    return e.dim() == 2 && like(e, a) && e.size(0) == eid.numel() && e.size(1) == a.size(1);
+}
+
+std::optional<Tensor> masked_mm_known(const Tensor &row, const Tensor &indptr, const Tensor &eid, const Tensor &indices, const Tensor &a, const Tensor &b) {
+    if (!rows_of_heads(a) || !same_heads(b, a) || indices.sizes() != eid.sizes()) return std::nullopt;
+    const int h = (int)a.size(1), d = (int)a.size(2), dt = dtype_code(a.scalar_type());
+    Key key;
+    if (!make_key(key, MM_FWD, {&row, &indptr, &eid, &indices}, a.device(), {a.size(0), b.size(0), h, d, dt})) return std::nullopt;
+    const EntryPtr e = find(key);
+    if (!e) return std::nullopt;
+    c10::DeviceGuard guard(a.device());
+    Tensor y = at::empty({eid.numel(), h}, a.options());
+    if (bpt_maskedmm_csr_forward(&e->a, a.data_ptr(), b.data_ptr(), y.data_ptr(), h, d, dt, stream_of(a.device())) != BPT_OK) return std::nullopt;
+    return y;
+}
+
+std::optional<Two> masked_mm_backward_known(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r, const Tensor &indices_r, const Tensor &col,
+                                            const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c, const Tensor &a, const Tensor &b,
+                                            const Tensor &dy) {
+    if (!rows_of_heads(a) || !same_heads(b, a) || indices_r.sizes() != eid_r.sizes() || indices_c.sizes() != eid_c.sizes() ||
+        eid_c.sizes() != eid_r.sizes() || !per_edge(dy, a, eid_r))
+        return std::nullopt;
+    const int h = (int)a.size(1), d = (int)a.size(2), dt = dtype_code(a.scalar_type());
+    Key key;
+    if (!make_key(key, MM_BWD, {&row, &indptr_r, &eid_r, &indices_r, &col, &indptr_c, &eid_c, &indices_c}, a.device(), {a.size(0), b.size(0), h, d, dt}))
+        return std::nullopt;
+    const EntryPtr e = find(key);
+    if (!e) return std::nullopt;
+    c10::DeviceGuard guard(a.device());
+    Tensor da = at::empty_like(a), db = at::empty_like(b);
+    Workspace ws(BPT_OP_MASKEDMM_BWD, &e->a, &e->b, h, d, dt, a);
+    if (bpt_maskedmm_csr_backward(&e->a, &e->b, a.data_ptr(), b.data_ptr(), dy.data_ptr(), da.data_ptr(), db.data_ptr(), ws.ptr, ws.bytes, h, d, dt,
+                                  stream_of(a.device())) != BPT_OK)
+        return std::nullopt;
+    return Two{da, db};
+}
+
+std::optional<Tensor> softmax_known(const Tensor &row, const Tensor &indptr, const Tensor &eid, const Tensor &x, const Tensor *dy) {
+    // forward of x, or with dy the backward of the probabilities x
+    if (x.dim() != 2 || !x.is_cuda() || !x.is_contiguous() || dtype_code(x.scalar_type()) < 0 || x.size(0) != eid.numel()) return std::nullopt;
+    if (dy && (!like(*dy, x) || dy->sizes() != x.sizes())) return std::nullopt;
+    const int h = (int)x.size(1), dt = dtype_code(x.scalar_type());
+    Key key;
+    if (!make_key(key, SOFTMAX, {&row, &indptr, &eid}, x.device(), {h, dt})) return std::nullopt;
+    const EntryPtr e = find(key);
+    if (!e) return std::nullopt;
+    c10::DeviceGuard guard(x.device());
+    Tensor y = at::empty_like(x);
+    Workspace ws(dy ? BPT_OP_SOFTMAX_BWD : BPT_OP_SOFTMAX_FWD, &e->a, nullptr, h, 1, dt, x);
+    const int st = dy ? bpt_sparse_softmax_backward(&e->a, x.data_ptr(), dy->data_ptr(), y.data_ptr(), ws.ptr, ws.bytes, h, dt, stream_of(x.device()))
+                      : bpt_sparse_softmax_forward(&e->a, x.data_ptr(), y.data_ptr(), ws.ptr, ws.bytes, h, dt, stream_of(x.device()));
+    if (st != BPT_OK) return std::nullopt;
+    return y;
+}
+
+std::optional<Tensor> vec_spmm_known(const Tensor &row, const Tensor &indptr, const Tensor &eid, const Tensor &indices, const Tensor &w, const Tensor &x) {
+    if (!rows_of_heads(x) || !per_edge(w, x, eid) || indices.sizes() != eid.sizes()) return std::nullopt;
+    const int h = (int)x.size(1), d = (int)x.size(2), dt = dtype_code(x.scalar_type());
+    Key key;
+    if (!make_key(key, SPMM_FWD, {&row, &indptr, &eid, &indices}, x.device(), {x.size(0), h, d, dt})) return std::nullopt;
+    const EntryPtr e = find(key);
+    if (!e) return std::nullopt;
+    c10::DeviceGuard guard(x.device());
+    Tensor y = at::empty_like(x);
+    Workspace ws(BPT_OP_SPMM_FWD, &e->a, nullptr, h, d, dt, x);
+    if (bpt_vector_spmm_forward(&e->a, w.data_ptr(), x.data_ptr(), y.data_ptr(), ws.ptr, ws.bytes, h, d, dt, stream_of(x.device())) != BPT_OK)
+        return std::nullopt;
+    return y;
+}
+
+std::optional<Two> vec_spmm_backward_known(const Tensor &row, const Tensor &indptr, const Tensor &eid, const Tensor &indices, const Tensor &col,
+                                           const Tensor &indptr_t, const Tensor &eid_t, const Tensor &indices_t, const Tensor &w, const Tensor &dy,
+                                           const Tensor &x) {
+    if (!rows_of_heads(x) || !per_edge(w, x, eid) || !same_heads(dy, x) || dy.size(0) != x.size(0) || indices.sizes() != eid.sizes() ||
+        indices_t.sizes() != eid_t.sizes() || eid_t.sizes() != eid.sizes())
+        return std::nullopt;
+    const int h = (int)x.size(1), d = (int)x.size(2), dt = dtype_code(x.scalar_type());
+    Key key;
+    if (!make_key(key, SPMM_BWD, {&row, &indptr, &eid, &indices, &col, &indptr_t, &eid_t, &indices_t}, x.device(), {x.size(0), h, d, dt})) return std::nullopt;
+    const EntryPtr e = find(key);
+    if (!e) return std::nullopt;
+    c10::DeviceGuard guard(x.device());
+    Tensor dw = at::empty_like(w), dx = at::empty_like(x);
+    Workspace ws(BPT_OP_SPMM_BWD, &e->a, &e->b, h, d, dt, x);
+    if (bpt_vector_spmm_backward(&e->a, &e->b, w.data_ptr(), dy.data_ptr(), x.data_ptr(), dw.data_ptr(), dx.data_ptr(), ws.ptr, ws.bytes, h, d, dt,
+                                 stream_of(x.device())) != BPT_OK)
+        return std::nullopt;
+    return Two{dw, dx};
+}
+
+struct MaskedMM : torch::autograd::Function<MaskedMM> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r,
+                          const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c,
+                          const Tensor &a, const Tensor &b) {
+        ctx->save_for_backward({row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, a, b});
+        auto r = masked_mm_known(row, indptr_r, eid_r, indices_r, a, b);
+        if (!r) {                                             // a new graph: both sides' plans at once
+            python("prepare_products")(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, a, b);
+            r = python("maskedmm_csr_forward")(row, indptr_r, eid_r, indices_r, a, b).cast<Tensor>();
+        }
+        return *r;
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        const auto t = ctx->get_saved_variables();
+        const Tensor dy = grads[0].contiguous();
+        auto r = masked_mm_backward_known(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], dy);
+        if (!r)
+            r = with_python([&] {
+                const auto two = python("maskedmm_csr_backward")(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], dy)
+                                     .template cast<std::vector<Tensor>>();
+                return Two{two[0], two[1]};
+            });
+        torch::autograd::variable_list out(10);
+        std::tie(out[8], out[9]) = *r;
+        return out;
+    }
+};
+
+struct EdgeSoftmax : torch::autograd::Function<EdgeSoftmax> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &row, const Tensor &indptr, const Tensor &eid, const Tensor &x) {
+        auto y = softmax_known(row, indptr, eid, x, nullptr);
+        if (!y) y = python("sparse_softmax_forward")(row, indptr, eid, x).cast<Tensor>();
+        ctx->save_for_backward({row, indptr, eid, *y});
+        return *y;
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        const auto t = ctx->get_saved_variables();
+        const Tensor dy = grads[0].contiguous();
+        auto dx = softmax_known(t[0], t[1], t[2], t[3], &dy);
+        if (!dx) dx = with_python([&] { return python("sparse_softmax_backward")(t[0], t[1], t[2], t[3], dy).template cast<Tensor>(); });
+        return {Tensor(), Tensor(), Tensor(), *dx};
+    }
+};
+
+struct VecSpmm : torch::autograd::Function<VecSpmm> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &row, const Tensor &indptr, const Tensor &eid, const Tensor &indices,
+                          const Tensor &col, const Tensor &indptr_t, const Tensor &eid_t, const Tensor &indices_t, const Tensor &w, const Tensor &x) {
+        ctx->save_for_backward({row, indptr, eid, indices, col, indptr_t, eid_t, indices_t, w, x});
+        auto y = vec_spmm_known(row, indptr, eid, indices, w, x);
+        if (!y) y = python("vector_spmm_forward")(row, indptr, eid, indices, w, x).cast<Tensor>();
+        return *y;
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        const auto t = ctx->get_saved_variables();
+        const Tensor dy = grads[0].contiguous();
+        auto r = vec_spmm_backward_known(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], dy, t[9]);
+        if (!r)
+            r = with_python([&] {
+                const auto two = python("vector_spmm_backward")(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], dy, t[9])
+                                     .template cast<std::vector<Tensor>>();
+                return Two{two[0], two[1]};
+            });
+        torch::autograd::variable_list out(10);
+        std::tie(out[8], out[9]) = *r;
+        return out;
+    }
+};
+
+Tensor masked_mm(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r, const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c,
+                 const Tensor &eid_c, const Tensor &indices_c, const Tensor &a, const Tensor &b) {
+    if (differentiated({&a, &b})) return MaskedMM::apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, a, b);
+    auto y = masked_mm_known(row, indptr_r, eid_r, indices_r, a, b);
+    if (!y) {
+        python("prepare_products")(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, a, b);
+        y = python("maskedmm_csr_forward")(row, indptr_r, eid_r, indices_r, a, b).cast<Tensor>();
+    }
+    return *y;
+}
+
+Tensor sparse_softmax(const Tensor &row, const Tensor &indptr, const Tensor &eid, const Tensor &x) {
+    if (differentiated({&x})) return EdgeSoftmax::apply(row, indptr, eid, x);
+    auto y = softmax_known(row, indptr, eid, x, nullptr);
+    if (!y) y = python("sparse_softmax_forward")(row, indptr, eid, x).cast<Tensor>();
+    return *y;
+}
+
+Tensor vec_spmm(const Tensor &row, const Tensor &indptr, const Tensor &eid, const Tensor &indices, const Tensor &col, const Tensor &indptr_t,
+                const Tensor &eid_t, const Tensor &indices_t, const Tensor &w, const Tensor &x) {
+    if (differentiated({&w, &x})) return VecSpmm::apply(row, indptr, eid, indices, col, indptr_t, eid_t, indices_t, w, x);
+    auto y = vec_spmm_known(row, indptr, eid, indices, w, x);
+    if (!y) y = python("vector_spmm_forward")(row, indptr, eid, indices, w, x).cast<Tensor>();
+    return *y;
 }
 
 // ---- tile plans ---------------------------------------------------------------------------------------------------------------
@@ -617,6 +809,14 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.attr("ATTN_BWD") = (int)ATTN_BWD;
     m.attr("ATTN_FWD_NARROW") = (int)ATTN_FWD_NARROW;
     m.attr("ATTN_BWD_NARROW") = (int)ATTN_BWD_NARROW;
+    m.attr("MM_FWD") = (int)MM_FWD;
+    m.attr("MM_BWD") = (int)MM_BWD;
+    m.attr("SPMM_FWD") = (int)SPMM_FWD;
+    m.attr("SPMM_BWD") = (int)SPMM_BWD;
+    m.attr("SOFTMAX") = (int)SOFTMAX;
+    m.def("masked_mm", &masked_mm);
+    m.def("sparse_softmax", &sparse_softmax);
+    m.def("vec_spmm", &vec_spmm);
     m.def("attention", &attention);
     m.def("attention_narrow", &attention_narrow);
     m.def("attention_forward_narrow", &narrow_forward_known);

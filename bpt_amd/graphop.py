@@ -215,6 +215,27 @@ def _product_tiles(n_edges, n_rows, n_index_nodes, x, h, d, cfg):
             and n_rows * h * d * 4 < 2 ** 32 and n_edges * h < 2 ** 32)
 
 
+def prepare_products(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, A, B):
+    """Builds the two sides' tile plans together that masked_mm, vec_spmm and their backwards are going to ask for, where neither is in
+    the cache (a new graph).  A convenience, as prepare_training: what is not built here is built when it is asked for."""
+    cfg = _SETTINGS
+    graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
+    if any(t.dim() != 1 or t.dtype != torch.int64 or t.device != A.device or not t.is_contiguous() for t in graph) or not A.is_cuda:
+        return
+    n = A.size(0)
+    if A.dim() != 3 or not _product_tiles(eid_r.numel(), n, B.size(0), A, A.size(1), A.size(2), cfg):
+        return
+    seg = _tile_seg_of(eid_r.numel(), n, n)
+    plan_cache.put_tile_plans([(col, indptr_c, eid_c, indices_c, n, n, seg, None),
+                               (row, indptr_r, eid_r, indices_r, n, n, seg, _plan.tile_order_src(n, eid_r.numel()))])
+
+
+def _remember_op(plans, generation, kind, index, numbers, struct, struct_t=None):
+    """Leaves the choice of one of the separate operators to the native host path, which takes plans that cover every edge."""
+    if all(p.covers_all_edges and p.n_edges > 0 for p in plans):
+        plan_cache.remember(plans, generation, kind, index, numbers, ctypes.addressof(struct), 0 if struct_t is None else ctypes.addressof(struct_t))
+
+
 def _product_plan(row, indptr, eid, indices, n_rows, n_index_nodes, x, h, d, cfg, order=None):
     """(plan, the struct to hand over) for a SpMM- or SDDMM-shaped op over one CSR side: tiles for float32 rows of 4 to 64
     columns a head and up to 16 heads of a graph of one node set, built on the GPU, else _spmm_struct's choice.  Both products of
@@ -239,7 +260,7 @@ def _edge_out(plan, shape, like):
 
 def maskedmm_csr_forward(row, indptr, eid, indices, A, B):
     """y[eid[p]] = <A[row], B[indices[p]]> per head (graphop.cpp:16-31, graphop_kernel.cu:269-304)."""
-    cfg = _SETTINGS
+    generation, cfg = _native.generation(), _SETTINGS
     _check_all(row=row, indptr=indptr, eid=eid, indices=indices, A=A, B=B)
     _same_dtype(A, B)
     h, d = _hd(A)
@@ -252,12 +273,14 @@ def maskedmm_csr_forward(row, indptr, eid, indices, A, B):
     with _on_device_of(A):
         check_attn(_LIB.bpt_maskedmm_csr_forward(ctypes.byref(struct), _ptr(A), _ptr(B), _ptr(y), h, d, _dtype(A), _stream()),
                    "maskedmm_csr_forward")
+    if A.dim() == 3:
+        _remember_op((plan,), generation, _native.MM_FWD, [row, indptr, eid, indices], [A.size(0), B.size(0), h, d, _dtype(A)], struct)
     return y
 
 
 def maskedmm_csr_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, A, B, dy):
     """[dA, dB] (graphop.cpp:108-139, graphop_kernel.cu:355-409)."""
-    cfg = _SETTINGS
+    generation, cfg = _native.generation(), _SETTINGS
     _check_all(row=row, indptr_r=indptr_r, eid_r=eid_r, indices_r=indices_r, col=col, indptr_c=indptr_c,
                eid_c=eid_c, indices_c=indices_c, A=A, B=B)
     dy = dy.contiguous()
@@ -277,6 +300,9 @@ def maskedmm_csr_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c,
     with _on_device_of(A):
         check_attn(_LIB.bpt_maskedmm_csr_backward(ref_r, ref_c, _ptr(A), _ptr(B), _ptr(dy), _ptr(dA), _ptr(dB),
                                                   _ptr(ws), nws, h, d, dt, _stream()), "maskedmm_csr_backward")
+    if A.dim() == 3:
+        _remember_op((plan_r, plan_c), generation, _native.MM_BWD, [row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c],
+                     [A.size(0), B.size(0), h, d, dt], struct_r, struct_c)
     return [dA, dB]
 
 
@@ -318,6 +344,7 @@ def node_mul_edge_backward(row, indptr, eid, A, B, dy):
 
 def sparse_softmax_forward(row, indptr, eid, x):
     """softmax of x over the slots of each row (graphop.cpp:59-71, graphop_kernel.cu:411-463)."""
+    generation = _native.generation()
     _check_all(row=row, indptr=indptr, eid=eid, x=x)
     _expect_index(eid, None)
     if x.dim() not in (1, 2) or x.size(0) != eid.size(0):
@@ -328,11 +355,14 @@ def sparse_softmax_forward(row, indptr, eid, x):
     with _on_device_of(x):
         check_attn(_LIB.bpt_sparse_softmax_forward(plan.ref, _ptr(x), _ptr(y), _ptr(ws), nws, _edge_h(x), _dtype(x), _stream()),
                    "sparse_softmax_forward")
+    if x.dim() == 2:
+        _remember_op((plan,), generation, _native.SOFTMAX, [row, indptr, eid], [x.size(1), _dtype(x)], plan.struct)
     return y
 
 
 def sparse_softmax_backward(row, indptr, eid, y, dy):
     """dx = y * (dy - sum_row dy*y) (graphop.cpp:163-177, graphop_kernel.cu:465-507)."""
+    generation = _native.generation()
     _check_all(row=row, indptr=indptr, eid=eid, y=y, dy=dy)
     _same_dtype(y, dy)
     _expect_index(eid, None)
@@ -346,6 +376,8 @@ def sparse_softmax_backward(row, indptr, eid, y, dy):
         check_attn(_LIB.bpt_sparse_softmax_backward(plan.ref, _ptr(y), _ptr(dy), _ptr(dx), _ptr(ws), nws, _edge_h(dy), _dtype(y),
                                                     _stream()),
                    "sparse_softmax_backward")
+    if y.dim() == 2:
+        _remember_op((plan,), generation, _native.SOFTMAX, [row, indptr, eid], [y.size(1), _dtype(y)], plan.struct)
     return dx
 
 
@@ -356,7 +388,7 @@ def vector_spmm_forward(row, indptr, eid, indices, edata, x, *, n_rows=None, out
     rectangular operator, used for the segment sums of the relative-position table's gradient.
     out (keyword only, not in the reference): a contiguous tensor of y's shape that the sum is ADDED to and that is
     returned (in the kernel's store where the row-group kernels apply, else by a separate addition)."""
-    cfg = _SETTINGS
+    generation, cfg = _native.generation(), _SETTINGS
     _check_all(row=row, indptr=indptr, eid=eid, indices=indices, edata=edata, x=x)
     _same_dtype(edata, x)
     h, d = _hd(x)
@@ -385,12 +417,14 @@ def vector_spmm_forward(row, indptr, eid, indices, edata, x, *, n_rows=None, out
                 check_attn(st, "vector_spmm_accumulate")
         check_attn(_LIB.bpt_vector_spmm_forward(ref, _ptr(edata), _ptr(x), _ptr(y), _ptr(ws), nws, h, d, dt, _stream()),
                    "vector_spmm_forward")
+    if square and x.dim() == 3 and edata.dim() == 2:
+        _remember_op((plan,), generation, _native.SPMM_FWD, [row, indptr, eid, indices], [x.size(0), h, d, dt], struct)
     return y if out is None else out.add_(y)
 
 
 def vector_spmm_backward(row, indptr, eid, indices, col, indptr_t, eid_t, indices_t, edata, dy, x):
     """[dedata, dx] (graphop.cpp:190-214, graphop_kernel.cu:544-600; dx over all units of the transposed side)."""
-    cfg = _SETTINGS
+    generation, cfg = _native.generation(), _SETTINGS
     _check_all(row=row, indptr=indptr, eid=eid, indices=indices, col=col, indptr_t=indptr_t, eid_t=eid_t,
                indices_t=indices_t, edata=edata, x=x)
     dy = dy.contiguous()
@@ -408,10 +442,14 @@ def vector_spmm_backward(row, indptr, eid, indices, col, indptr_t, eid_t, indice
     dx = torch.empty_like(x)
     dt = _dtype(x)
     ref, ref_t = ctypes.byref(struct), ctypes.byref(struct_t)
+    square = x.dim() == 3 and dy.size(0) == x.size(0) and edata.dim() == 2
     ws, nws = _workspace(OP_SPMM_BWD, plan, plan_t, h, d, dt, x.device, plan_ref=ref, plan_t_ref=ref_t)
     with _on_device_of(x):
         check_attn(_LIB.bpt_vector_spmm_backward(ref, ref_t, _ptr(edata), _ptr(dy), _ptr(x), _ptr(dedata), _ptr(dx),
                                                  _ptr(ws), nws, h, d, dt, _stream()), "vector_spmm_backward")
+    if square:
+        _remember_op((plan, plan_t), generation, _native.SPMM_BWD, [row, indptr, eid, indices, col, indptr_t, eid_t, indices_t],
+                     [x.size(0), h, d, dt], struct, struct_t)
     return [dedata, dx]
 
 

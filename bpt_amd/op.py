@@ -205,11 +205,21 @@ def _rel_type_rows(aux, etype, col, indptr_c, eid_c, n_types):
     return aux["type_rows"]
 
 
+def _native_takes(*tensors):
+    """Whether bptop.so's function may take a call of one of the separate operators: a trace and the transforms of torch.func work on the
+    Python functions, and None (a side that only a backward would read) is no tensor to it."""
+    return not torch.jit.is_tracing() and not torch._C._are_functorch_transforms_active() and all(t is not None for t in tensors)
+
+
 def sparse_softmax(row, indptr, eid, x):
+    if _native_takes(row, indptr, eid, x):
+        return _native.sparse_softmax(row, indptr, eid, x)
     return SparseSoftmax.apply(row, indptr, eid, x)
 
 
 def masked_mm(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, A, B):
+    if _native_takes(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, A, B):
+        return _native.masked_mm(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, A, B)
     return MaskedMMCSR.apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, A, B)
 
 
@@ -218,6 +228,8 @@ def node_mul_edge(row, indptr, eid, A, B):
 
 
 def vec_spmm(row, indptr, eid, indices, col, ptr_t, eid_t, indices_t, edata, x, n_rows=None):
+    if n_rows is None and _native_takes(row, indptr, eid, indices, col, ptr_t, eid_t, indices_t, edata, x):
+        return _native.vec_spmm(row, indptr, eid, indices, col, ptr_t, eid_t, indices_t, edata, x)
     return VectorSPMM.apply(row, indptr, eid, indices, col, ptr_t, eid_t, indices_t, edata, x, n_rows)
 
 

@@ -1,0 +1,89 @@
+"""The native host path of masked_mm, sparse_softmax and vec_spmm: the results and gradients of the autograd functions it stands for, bit for
+bit, on a first call and on later ones; what the functions refuse is refused, what they hold is held."""
+import math
+
+import pytest
+import torch
+
+from test_gpu_product_tiles import DEV, rand, sides
+
+pytestmark = pytest.mark.gpu
+
+
+def chain(ops, s, q, k, v):
+    e = ops[0](*s.out, *s.inn, k, q)
+    a = ops[1](*s.inn[:3], e / math.sqrt(q.size(-1)))
+    return ops[2](*s.inn, *s.out, a, v)
+
+
+@pytest.mark.parametrize("dtype,h,d", [(torch.float32, 8, 64), (torch.float32, 6, 50), (torch.bfloat16, 8, 64), (torch.float64, 3, 10)],
+                         ids=lambda x: str(x).replace("torch.", ""))
+@pytest.mark.parametrize("name", ["bpt512", "multigraph"])
+def test_same_bits_as_the_autograd_functions(name, dtype, h, d):
+    from bpt_amd import graphop, op, plan
+    s = sides(name)
+    x = [rand((s.n, h, d), i).to(dtype).requires_grad_(True) for i in (1, 2, 3)]
+    do = rand((s.n, h, d), 4).to(dtype)
+    plan.plan_cache.clear()
+    native = plan.PlanCache.native
+
+    def run(ops):
+        o = chain(ops, s, *x)
+        return (o.detach(),) + torch.autograd.grad(o, x, do)
+
+    functions = (op.MaskedMMCSR.apply, op.SparseSoftmax.apply, op.VectorSPMM.apply)
+    calls = (op.masked_mm, op.sparse_softmax, op.vec_spmm)
+    want = run(functions)
+    plan.plan_cache.clear()
+    first = run(calls)
+    native.take_used()
+    second = run(calls)
+    assert native.take_used()                                     # served from the table
+    with torch.no_grad():
+        third = chain(calls, s, *x)
+    assert torch.equal(third, want[0])
+    for a, b, c in zip(want, first, second):
+        assert torch.equal(a, b) and torch.equal(a, c)
+    old = graphop.set_tiles(False)                                # a switch: what was chosen under the other one is not used
+    try:
+        assert not native.take_used()
+        off = run(calls)
+        assert all(torch.equal(a, b) for a, b in zip(off, run(functions)))
+    finally:
+        graphop.set_tiles(old)
+
+
+def test_refused_and_held_as_by_the_autograd_functions():
+    import torch.autograd.forward_ad as forward_ad
+    from bpt_amd import op
+    s = sides("bpt512")
+    q, k, v = (rand((s.n, 8, 64), i) for i in (1, 2, 3))
+    calls = (op.masked_mm, op.sparse_softmax, op.vec_spmm)
+    chain(calls, s, q, k, v)
+    chain(calls, s, q, k, v)
+    with forward_ad.dual_level():
+        for no_grad in (False, True):
+            with torch.set_grad_enabled(not no_grad), pytest.raises(RuntimeError):
+                op.masked_mm(*s.out, *s.inn, forward_ad.make_dual(k, q), q)
+            with torch.set_grad_enabled(not no_grad), pytest.raises(RuntimeError):
+                op.vec_spmm(*s.inn, *s.out, rand((s.E, 8), 5), forward_ad.make_dual(v, q))
+            with torch.set_grad_enabled(not no_grad), pytest.raises(RuntimeError):
+                op.sparse_softmax(*s.inn[:3], forward_ad.make_dual(rand((s.E, 8), 5), rand((s.E, 8), 6)))
+    with pytest.raises(RuntimeError):
+        torch.func.grad(lambda x: op.masked_mm(*s.out, *s.inn, x, q).sum())(k)
+    with pytest.raises(RuntimeError):
+        op.masked_mm(*s.out, *s.inn, k.cpu(), q.cpu())
+    with pytest.raises(RuntimeError):
+        op.masked_mm(*s.out, *s.inn, k.transpose(0, 1), q.transpose(0, 1))
+    with pytest.raises(ValueError):
+        op.vec_spmm(*s.inn, *s.out, rand((s.E - 1, 8), 5), v)
+    packed = []
+    x = v.clone().requires_grad_(True)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: packed.append(t) or t, lambda t: t):
+        o = op.vec_spmm(*s.inn, *s.out, rand((s.E, 8), 5), x)
+    assert any(t.shape == v.shape for t in packed)
+    o = op.vec_spmm(*s.inn, *s.out, rand((s.E, 8), 5), x)
+    with torch.no_grad():
+        x += 1
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(o, x, q)
