@@ -2057,6 +2057,43 @@ constexpr int TILE_CHUNK = 128;                     // entries staged in LDS at 
 typedef float floatx4v __attribute__((ext_vector_type(4)));
 typedef uint32_t uintx2v __attribute__((ext_vector_type(2)));
 
+typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
+typedef float floatx2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+    union { bf16x2v v; uint32_t u; } r;
+    r.v = __builtin_convertvector(floatx2v{lo, hi}, bf16x2v);      // round to nearest even
+    return r.u;
+}
+
+// What a tile costs beside its blocks - sums and maxima over lane groups, the rows it stores, masks - is kept to few vector instructions:
+// float32 products (v_mfma_f32_16x16x4) and vector arithmetic do not run side by side on a SIMD, whichever wavefronts they come from (a
+// wavefront of each takes the sum of their times: 288 + 351 -> 628 cycles; bfloat16 16 x 16 x 32 products 145 + 345 -> 405).  Lane groups
+// are swapped instead of looked up through the LDS crossbar, masks are one bit field extract and one and, a member's row or slot is one
+// word, rows go to 32-bit offsets from a uniform base, bfloat16 is rounded by the hardware and sums that are still zero are not rescaled;
+// the float32 destination side reads masks and pair numbers back from LDS and no longer spills.  Same results to the bit.  Kernels before ->
+// after, forward / destination / source side: bfloat16, L = 8192, k = 4 18.5 / 25.6 / 29.2 -> 17.1 / 24.6 / 26.5 us, 16 heads at L = 32768, k = 8
+// 185 / 241 / 339 -> 184 / 240 / 333; float32, L = 8192 35.3 / 59.3 / 42.8 -> 34.1 / 58.1 / 40.9, 32-graph batch 68.6 / 105.1 / 89.4 -> 67.0 / 101.6 / 87.4.
+// x of the lanes c, 16 + c, 32 + c and 48 + c, combined, in all four of them
+__device__ __forceinline__ float groups_sum(float x) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+__device__ __forceinline__ float groups_max(float x) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    x = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+// x where bit `bit` of the mask is set, -inf (0) where it is not
+__device__ __forceinline__ float where_pair(int mask, int bit, float x) {
+    const int m = __builtin_amdgcn_sbfe(mask, bit, 1);
+    return __int_as_float((__float_as_int(x) & m) | (0xff800000 & ~m));
+}
+__device__ __forceinline__ float where_pair_or_zero(int mask, int bit, float x) {
+    return __int_as_float(__float_as_int(x) & __builtin_amdgcn_sbfe(mask, bit, 1));
+}
 __device__ __forceinline__ float lane_bcast(float x, int src_lane) {
     return __int_as_float(__builtin_amdgcn_ds_bpermute(src_lane << 2, __float_as_int(x)));
 }
@@ -2206,42 +2243,47 @@ __device__ __forceinline__ void tile_axpy_upto(const float (&w)[4], const float4
 // L = 8192 float32 161 -> 157, bfloat16 91 -> 85.5 (forward 21.8 -> 19.2), L = 32768, k = 4 649 -> 632, window 128 97 -> 94.5;
 // L = 512 level.  The same on the stores of (p, ds), which the source side reads soon, or on its loads of them: 47 -> 50.5 and
 // 47 -> 55 us for the source side of L = 8192; on the loads of the members' rows: destination side 58 -> 61.6.
+// where: per member, its row, -1 where there is none, -2 - slot for a segment of a split row (tile_where of lane c for member c)
+__device__ __forceinline__ int tile_where(int2 member) { return member.x < 0 ? -1 : member.y < 0 ? member.x : -2 - member.y; }
 template <int H, int D, bool SCALE, bool NARROW, typename T>
 __device__ __forceinline__ void tile_store_row(const TileCtx &t, int r, float4 x, float inv_c, T *__restrict__ out, float *__restrict__ ws,
-                                               const Narrow &nw, T *__restrict__ also = nullptr) {      // also (NARROW): second copy of whole rows
+                                               const Narrow &nw, int where, T *__restrict__ also = nullptr) {      // also (NARROW): second copy of whole rows
     const int m = 4 * t.g + r;                                    // the member whose row this lane stores a piece of
-    const int row = lane_bcast(t.member.x, m), slot = lane_bcast(t.member.y, m);
+    int at = lane_bcast(where, m);
     const float inv = SCALE ? lane_bcast(inv_c, m) : 1.f;
-    if (row < 0 || (NARROW && 4 * t.c >= nw.d)) return;
+    if (NARROW && 4 * t.c >= nw.d) at = -1;
     const int col = NARROW ? narrow_col(nw, t.c) : 4 * t.c;
-    if (slot < 0) {
+    if (at >= 0) {
         if (SCALE) { x.x *= inv; x.y *= inv; x.z *= inv; x.w *= inv; }
-        T *const at = NARROW ? out + (size_t)row * (uint32_t)(nw.heads * nw.d) + t.head * nw.d + col : out + (size_t)row * (H * D) + t.head * D + col;
+        // (node tensors end before 4 GiB)
+        const uint32_t off = NARROW ? ((uint32_t)at * (uint32_t)(nw.heads * nw.d) + (uint32_t)(t.head * nw.d + col)) * (uint32_t)sizeof(T)
+                                    : (uint32_t)at * (uint32_t)(H * D * sizeof(T)) + t.offv;
+        char *const to = reinterpret_cast<char *>(out) + off;
         if constexpr (sizeof(T) == 4) {
             if constexpr (NARROW) {
-                *reinterpret_cast<floatx4u *>(at) = floatx4u{x.x, x.y, x.z, x.w};
-                if (also) *reinterpret_cast<floatx4u *>(also + (at - out)) = floatx4u{x.x, x.y, x.z, x.w};
-            } else __builtin_nontemporal_store(floatx4v{x.x, x.y, x.z, x.w}, reinterpret_cast<floatx4v *>(at));
+                *reinterpret_cast<floatx4u *>(to) = floatx4u{x.x, x.y, x.z, x.w};
+                if (also) *reinterpret_cast<floatx4u *>(reinterpret_cast<char *>(also) + off) = floatx4u{x.x, x.y, x.z, x.w};
+            } else __builtin_nontemporal_store(floatx4v{x.x, x.y, x.z, x.w}, reinterpret_cast<floatx4v *>(to));
         } else {
-            const uint2 y = make_uint2(((uint32_t)f32_to_bf16(x.x)) | ((uint32_t)f32_to_bf16(x.y) << 16),
-                           ((uint32_t)f32_to_bf16(x.z)) | ((uint32_t)f32_to_bf16(x.w) << 16));
+            const uint2 y = make_uint2(pack_bf16(x.x, x.y), pack_bf16(x.z, x.w));
             if constexpr (NARROW) {
-                *reinterpret_cast<uintx2u *>(at) = uintx2u{y.x, y.y};
-                if (also) *reinterpret_cast<uintx2u *>(also + (at - out)) = uintx2u{y.x, y.y};
-            } else __builtin_nontemporal_store(uintx2v{y.x, y.y}, reinterpret_cast<uintx2v *>(at));
+                *reinterpret_cast<uintx2u *>(to) = uintx2u{y.x, y.y};
+                if (also) *reinterpret_cast<uintx2u *>(reinterpret_cast<char *>(also) + off) = uintx2u{y.x, y.y};
+            } else __builtin_nontemporal_store(uintx2v{y.x, y.y}, reinterpret_cast<uintx2v *>(to));
         }
-    } else {
-        float *const at = ws + (size_t)slot * (NARROW ? nw.h * D : H * D) + t.head * D + col;
-        if constexpr (NARROW) *reinterpret_cast<floatx4u *>(at) = floatx4u{x.x, x.y, x.z, x.w};
-        else *reinterpret_cast<float4 *>(at) = x;
+    } else if (at < -1) {
+        float *const to = ws + (size_t)(-2 - at) * (NARROW ? nw.h * D : H * D) + t.head * D + col;
+        if constexpr (NARROW) *reinterpret_cast<floatx4u *>(to) = floatx4u{x.x, x.y, x.z, x.w};
+        else *reinterpret_cast<float4 *>(to) = x;
     }
 }
 template <int H, int D, bool SCALE, bool NARROW, typename T>
 __device__ __forceinline__ void tile_store_rows(const TileCtx &t, const floatx4v (&acc)[4], float inv_c, T *__restrict__ out,
                                                 float *__restrict__ ws, const Narrow &nw, T *__restrict__ also = nullptr) {
+    const int where = tile_where(t.member);
 #pragma unroll
     for (int r = 0; r < 4; ++r)
-        tile_store_row<H, D, SCALE, NARROW>(t, r, make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]), inv_c, out, ws, nw, also);
+        tile_store_row<H, D, SCALE, NARROW>(t, r, make_float4(acc[0][r], acc[1][r], acc[2][r], acc[3][r]), inv_c, out, ws, nw, where, also);
 }
 
 // SP > 1: SP wavefronts of a workgroup share a tile and head, each walks a contiguous SP-th of the tile's blocks (tile_begin),
@@ -2279,7 +2321,7 @@ __device__ __forceinline__ void tile_meet_and_store(const float *part0, int stri
 #pragma unroll
     for (int i = 0; i < RS; ++i) {
         const int r = t.part * RS + i;
-        tile_store_row<H, D, false, NARROW>(t, r, tile_meet<SP, false>(part0, stride, r, t, none), 1.f, out, ws, nw);
+        tile_store_row<H, D, false, NARROW>(t, r, tile_meet<SP, false>(part0, stride, r, t, none), 1.f, out, ws, nw, tile_where(t.member));
     }
 }
 // ... and for the forward: with the parts' exponent references and denominators (left behind the accumulators by member)
@@ -2312,7 +2354,7 @@ __device__ __forceinline__ void tile_meet_forward(float *mine, const float *part
 #pragma unroll
     for (int i = 0; i < RS; ++i) {
         const int r = t.part * RS + i;
-        tile_store_row<H, D, true, NARROW>(t, r, tile_meet<SP, true>(part0, stride, r, t, wgt), inv, out, ws, nw, also);
+        tile_store_row<H, D, true, NARROW>(t, r, tile_meet<SP, true>(part0, stride, r, t, wgt), inv, out, ws, nw, tile_where(t.member), also);
     }
 }
 
@@ -2445,16 +2487,19 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
     // for before the entry list is (one more round trip in front of the K rows).  They stay as they are and the scores are
     // scaled instead, so nothing has to happen to them between their arrival and the first product.
     const char *const qrow = reinterpret_cast<const char *>(q) + (size_t)max(t.member.x, 0) * RB + t.offa;
-    constexpr bool AHEAD = !DROP && BIAS == 0;         // (with dropout or the score term the sixteen registers are not there)
+    // (with the score term the sixteen registers are not there; with dropout they just are, and it does not pay: L = 8192 level, 6 x 50
+    // with dropout 97.7 -> 100 us)
+    constexpr bool AHEAD = !DROP && BIAS == 0;
     if constexpr (!AHEAD) tile_load16<NARROW>(qrow, qb, g, nw);
     floatx4v acc[4];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
     float mref = M_INIT_LOG2, lrun = 0.f;
+    bool fresh = true;                                            // nothing has been summed up yet
     struct Blk {
         float4 kq[4];                                             // columns 4 c .. 4 c + 3 of the K rows of entries 4 r + g
         float4 vr[4];
-        int has, nv;                                              // bit r of has: the pair (entry 4 r + g, member c) exists; nv: entries of the block that exist
+        int mk[4], nv;                                            // bit c of mk[r]: the pair (entry 4 r + g, member c) exists; nv: entries of the block that exist
         int xe[DROP || BIAS == 1 ? 4 : 1];
         float bz[BIAS ? 4 : 1];
     };
@@ -2470,13 +2515,12 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
         auto issue_rest = [&](Blk &B, int b) {
             if constexpr (DROP || BIAS == 1) tile_pair_eids(P, p0 + TILE_R * b + g, t.p_end, c, B.xe, 4);
             B.nv = min(TILE_R, cnt - TILE_R * b);
-            int idxv[4], mk[4];
+            int idxv[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int2 en = ent[TILE_R * b + 4 * r + g];
-                idxv[r] = en.x; mk[r] = en.y;
+                idxv[r] = en.x; B.mk[r] = en.y;
             }
-            B.has = ((mk[0] >> c) & 1) | (((mk[1] >> c) & 1) << 1) | (((mk[2] >> c) & 1) << 2) | (((mk[3] >> c) & 1) << 3);
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 B.vr[r] = tile_row4<NARROW>(vb + ((uint32_t)idxv[r] * RB + t.offv));
@@ -2486,7 +2530,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
             }
             if constexpr (BIAS == 2) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, 2>(P, t.head, 0, tile_pair_number(fst[TILE_R * b + 4 * r + g], mk[r], c))];
+                for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, 2>(P, t.head, 0, tile_pair_number(fst[TILE_R * b + 4 * r + g], B.mk[r], c))];
             }
         };
         auto compute = [&](const Blk &B) {
@@ -2496,23 +2540,24 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
             float sc[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r)
-                sc[r] = ((B.has >> r) & 1) ? (BIAS ? fmaf(st[r], scale_log2e, B.bz[BIAS ? r : 0] * scale_log2e) : st[r] * scale_log2e) : -INFINITY;
+                sc[r] = where_pair(B.mk[r], c, BIAS ? fmaf(st[r], scale_log2e, B.bz[BIAS ? r : 0] * scale_log2e) : st[r] * scale_log2e);
             const float mb = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
             if (__builtin_amdgcn_ballot_w64(mb > mref + MFMA_TAU) != 0) {
-                float gm = fmaxf(mb, __shfl_xor(mb, 16));
-                gm = fmaxf(gm, __shfl_xor(gm, 32));              // over the four lanes of member c
-                const float mn = fmaxf(mref, gm);
+                const float mn = fmaxf(mref, groups_max(mb));    // over the four lanes of member c
                 const float al = __builtin_amdgcn_exp2f(mref - mn);
                 mref = mn;
-                lrun *= al;
-                // register r' of the accumulators belongs to member 4 g + r': its factor sits in lane 4 g + r'
+                if (!fresh) {
+                    lrun *= al;
+                    // register r' of the accumulators belongs to member 4 g + r': its factor sits in lane 4 g + r'
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float a = lane_bcast(al, 4 * g + r);
+                    for (int r = 0; r < 4; ++r) {
+                        const float a = lane_bcast(al, 4 * g + r);
 #pragma unroll
-                    for (int nb = 0; nb < 4; ++nb) acc[nb][r] *= a;
+                        for (int nb = 0; nb < 4; ++nb) acc[nb][r] *= a;
+                    }
                 }
             }
+            fresh = false;
             float pr[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -2528,8 +2573,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
         else tile_walk_first_ahead<Blk>(nblk, issue_k, issue_rest, compute, [&]() { if (p0 == t.p_begin) tile_load16<NARROW>(qrow, qb, g, nw); });
         wave_lds_fence();                                         // the piece is read to the end before the next one is staged
     }
-    float lt = lrun + __shfl_xor(lrun, 16);
-    lt += __shfl_xor(lt, 32);                                    // denominator of member c, in its four lanes
+    float lt = groups_sum(lrun);                                 // denominator of member c, in its four lanes
     if constexpr (SP > 1) {
         static_assert(TILE_PART_FWD_FLOATS <= TILE_R * TILE_KT_STRIDE, "a part fits its wavefront's piece");
         tile_meet_forward<SP, H, D, NARROW>(kt, kt_lds[t.wv % (HW / SP)], (HW / SP) * TILE_R * TILE_KT_STRIDE, t, acc, mref, lt, o, ws_acc, nw, o_keep);
@@ -2550,8 +2594,8 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
 // Backward on tiles, destination side: per block the scores and dO . v of all 16 x 16 pairs (two products over the
 // columns, the K and V rows turned in LDS from the layout they are loaded in), p = 2^(s - lse),
 // ds = p (dO . v - delta) scale, dq += ds K (third product, on the K rows as loaded).  With dropout or a score term the
-// kernel is compiled for three wavefronts per SIMD: at four it keeps the members' q rows in scratch memory and reads
-// them back for every block (83 against 58 us with dropout at L = 8192, k = 4).
+// kernel is compiled for three wavefronts per SIMD or more: held to four it kept the members' q rows in scratch memory and reads
+// them back for every block (83 against 58 us with dropout at L = 8192, k = 4; with dropout alone four fit by themselves since).
 // (p, ds) of the pairs that exist go to a scratch in THIS side's order, compact:
 // pds[head * n_edges + t] for the pair number t of (entry, member) = the entry's first pair + the rank of the member in
 // its mask, so the lanes of an entry write one contiguous run and the runs of consecutive entries follow each other.  The
@@ -2611,8 +2655,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
 #pragma unroll
             for (int e = 0; e < 4; ++e) part = fmaf(xd[i][e], xo[i][e], part);
         }
-        part += __shfl_xor(part, 16);
-        part += __shfl_xor(part, 32);
+        part = groups_sum(part);
         if (g == 0) delta_lds[t.wv][c] = part;
         __syncthreads();
         delta = 0.f;
@@ -2631,8 +2674,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
         float part = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) part = fmaf(dob[i], ob[i], part);
-        part += __shfl_xor(part, 16);
-        delta = part + __shfl_xor(part, 32);                      // dO . O of member c, this head
+        delta = groups_sum(part);                                 // dO . O of member c, this head
         lse_c = lse[(size_t)max(t.member.x, 0) * Hs + t.head];
 #pragma unroll
         for (int i = 0; i < 4; ++i) dob_h[i][t.lane] = floatx4v{dob[4 * i], dob[4 * i + 1], dob[4 * i + 2], dob[4 * i + 3]};
@@ -2642,7 +2684,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
     for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
     struct Blk {
         float4 kc[4], vc[4];                                      // columns 4 c .. 4 c + 3 of the K / V rows of entries 4 r + g
-        int pos[4], has, nv;                                       // bit r of has: the pair (entry 4 r + g, member c) exists; nv: entries of the block that exist
+        int b, nv;                                                // which block of the piece; entries of it that exist
         int xe[DROP || BIAS == 1 ? 4 : 1];
         float bz[BIAS ? 4 : 1];
     };
@@ -2652,16 +2694,11 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
         tile_put_entries(er, ent, cnt, t.lane, fst);
         auto issue = [&](Blk &B, int b) {
             if constexpr (DROP || BIAS == 1) tile_pair_eids(P, p0 + TILE_R * b + g, t.p_end, c, B.xe, 4);
+            B.b = b;
             B.nv = min(TILE_R, cnt - TILE_R * b);
             int idxv[4];
-            B.has = 0;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int2 en = ent[TILE_R * b + 4 * r + g];
-                idxv[r] = en.x;
-                B.has |= ((en.y >> c) & 1) << r;
-                B.pos[r] = tile_pair_number(fst[TILE_R * b + 4 * r + g], en.y, c);
-            }
+            for (int r = 0; r < 4; ++r) idxv[r] = ent[TILE_R * b + 4 * r + g].x;
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 B.kc[r] = tile_row4<NARROW>(kb + ((uint32_t)idxv[r] * RB + t.offv));
@@ -2670,10 +2707,20 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
                 B.vc[r] = tile_row4<NARROW>(vb + ((uint32_t)idxv[r] * RB + t.offv));
             if constexpr (BIAS) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], B.pos[r])];
+                for (int r = 0; r < 4; ++r) {
+                    const int at = TILE_R * b + 4 * r + g;
+                    B.bz[r] = bias[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], BIAS == 2 ? tile_pair_number(fst[at], ent[at].y, c) : 0)];
+                }
             }
         };
         auto compute = [&](const Blk &B) {
+            int mask[4], number[4];                               // (read here, not kept from the block's issue on)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int at = TILE_R * B.b + 4 * r + g;
+                mask[r] = ent[at].y;
+                number[r] = tile_pair_number(fst[at], mask[r], c);
+            }
             floatx4v st;
             {
                 float kr[16];
@@ -2692,16 +2739,15 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
             float ds[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const bool has = (B.has >> r) & 1;
-                float pe = has ? __builtin_amdgcn_exp2f((BIAS ? fmaf(st[r], scale_log2e, B.bz[BIAS ? r : 0] * scale_log2e) : st[r] * scale_log2e) - lse_c) : 0.f;
+                float pe = where_pair_or_zero(mask[r], c, __builtin_amdgcn_exp2f((BIAS ? fmaf(st[r], scale_log2e, B.bz[BIAS ? r : 0] * scale_log2e) : st[r] * scale_log2e) - lse_c));
                 float mt = 1.f;                                   // dropout multiplier of this pair (as in the forward)
                 if constexpr (DROP)
                     mt = dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)Hs + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
                 ds[r] = pe * (dp[r] * mt - delta) * scale;
                 pe *= mt;                                         // what multiplies v (forward) and dO (dV)
-                if (has) {
-                    pds_h[B.pos[r]] = make_float2(pe, ds[r]);
-                    if constexpr (BIAS) ds_out[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], B.pos[r])] = ds[r];   // dL/d(score before scaling)
+                if ((mask[r] >> c) & 1) {
+                    pds_h[(uint32_t)number[r]] = make_float2(pe, ds[r]);
+                    if constexpr (BIAS) ds_out[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], number[r])] = ds[r];   // dL/d(score before scaling)
                 }
             }
             tile_axpy_upto(ds, B.kc, acc, B.nv);
@@ -2760,7 +2806,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
     // the steps past the end of the group's list (half of a group's last block on average) can be left out.
     struct Blk {
         float4 qr[4], dr[4];
-        int has, nv;                                              // bit r of has: the pair (entry 4 r + g, member c) exists; nv: entries of the block that exist
+        int mk[4], nv;                                            // bit c of mk[r]: the pair (entry 4 r + g, member c) exists; nv: entries of the block that exist
     };
     TileEntryRegs er;
     if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
@@ -2775,7 +2821,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
         tile_put_entries(er, ent, cnt, t.lane);
         if (p0 == t.p_begin) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) w[r] = pds_h[pos[r]];
+            for (int r = 0; r < 4; ++r) w[r] = pds_h[(uint32_t)pos[r]];
             positions(p0 + TILE_R);
         }
         auto put_pairs = [&]() {
@@ -2786,11 +2832,10 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
         };
         auto issue_rows = [&](Blk &B, int b) {
             B.nv = min(TILE_R, cnt - TILE_R * b);
-            B.has = 0;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int2 en = ent[TILE_R * b + 4 * r + g];
-                B.has |= ((en.y >> c) & 1) << r;
+                B.mk[r] = en.y;
                 const uint32_t off = (uint32_t)en.x * RB + t.offv;
                 B.qr[r] = tile_row4<NARROW>(qb + off);
                 B.dr[r] = tile_row4<NARROW>(db + off);
@@ -2801,9 +2846,8 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float2 w = wt[(4 * r + g) * TILE_WT_STRIDE + c];
-                const bool has = (B.has >> r) & 1;              // the scratch of pairs that do not exist is not initialised
-                pe[r] = has ? w.x : 0.f;
-                ds[r] = has ? w.y : 0.f;
+                pe[r] = where_pair_or_zero(B.mk[r], c, w.x);      // the scratch of pairs that do not exist is not initialised
+                ds[r] = where_pair_or_zero(B.mk[r], c, w.y);
             }
             wave_lds_fence();                                     // (read before the next block's are written)
             tile_axpy_upto(ds, B.qr, ak, B.nv);
@@ -2816,7 +2860,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
             put_pairs();
             if (p0 + TILE_R * (b + 1) < t.p_end) {
 #pragma unroll
-                for (int r = 0; r < 4; ++r) w[r] = pds_h[pos[r]];
+                for (int r = 0; r < 4; ++r) w[r] = pds_h[(uint32_t)pos[r]];
                 positions(p0 + TILE_R * (b + 2));
             }
             issue_loads_first();
@@ -2941,13 +2985,13 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(SP > 
         for (int b = 0; b < nblk; ++b) {
             if constexpr (SHARED) __syncthreads();                // (the other stage is read to the end too)
             const int nv = min(TILE_R, cnt - TILE_R * b);
-            int has = 0;
+            int mk[4];
             float4 xr[4];
             float wc[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int2 en = ent[TILE_R * b + 4 * r + g];
-                has |= ((en.y >> c) & 1) << r;
+                mk[r] = en.y;
                 xr[r] = tile_row4<NARROW>(xb + ((uint32_t)en.x * RB + t.offv));
                 if constexpr (!SHARED) wc[r] = w[r];
             }
@@ -2961,7 +3005,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(SP > 
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 if constexpr (SHARED) wc[r] = wt[stage][t.wv][WAVE * r + t.lane];
-                wc[r] = ((has >> r) & 1) ? wc[r] : 0.f;
+                wc[r] = where_pair_or_zero(mk[r], c, wc[r]);
             }
             tile_axpy_upto(wc, xr, acc, nv);
             issue_loads_first();
@@ -3072,17 +3116,10 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(5))) 
 // 71 k -> 62 k entries), and the step went from 0.113 to 0.117 ms (32-graph batch 0.177 -> 0.205, window 128 level).
 constexpr int TILE_BF16_WPE = 5, TILE_BF16_WPE_DST = 5, TILE_BF16_WPE_SRC = 5, TILE_BF16_WPE_AGAIN = 4;     // wavefronts per SIMD the bfloat16 tile kernels are compiled for
 typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
-typedef float floatx2v __attribute__((ext_vector_type(2)));
 typedef short shortx4v __attribute__((ext_vector_type(4)));
 union Bf8 { bf16x8v v; uint4 q; };
 union Bf4 { shortx4v v; uint32_t u[2]; };
 
-__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
-    union { bf16x2v v; uint32_t u; } r;
-    r.v = __builtin_convertvector(floatx2v{lo, hi}, bf16x2v);      // round to nearest even
-    return r.u;
-}
 __device__ __forceinline__ uint32_t pack_lo16(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100u); }   // (a.lo, b.lo)
 __device__ __forceinline__ uint32_t pack_hi16(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }   // (a.hi, b.hi)
 
@@ -3191,10 +3228,11 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
     float mref = M_INIT_LOG2, lrun = 0.f;
+    bool fresh = true;                                            // nothing has been summed up yet
     struct Blk {
         uint2 kq[4];                                              // columns 4 c .. 4 c + 3 of the K rows of entries 4 g + r
         uint2 vr[4];
-        int has;                                                  // bit r: the pair (entry 4 g + r, member c) exists
+        int mk[4];                                                // bit c of mk[r]: the pair (entry 4 g + r, member c) exists
         int xe[DROP || BIAS == 1 ? 4 : 1];
         float bz[BIAS ? 4 : 1];
     };
@@ -3214,8 +3252,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             const int4 e01 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g]);
             const int4 e23 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g + 2]);
             const int idxv[4] = {e01.x, e01.z, e23.x, e23.z};
-            const int mk[4] = {e01.y, e01.w, e23.y, e23.w};
-            B.has = ((mk[0] >> c) & 1) | (((mk[1] >> c) & 1) << 1) | (((mk[2] >> c) & 1) << 2) | (((mk[3] >> c) & 1) << 3);
+            B.mk[0] = e01.y; B.mk[1] = e01.w; B.mk[2] = e23.y; B.mk[3] = e23.w;
 #pragma unroll
             for (int r = 0; r < 4; ++r) B.vr[r] = tile_row4_bf16<NARROW>(vb + ((uint32_t)idxv[r] * RB + offc));
             if constexpr (BIAS == 1) {
@@ -3226,7 +3263,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
                 const int4 f4 = *reinterpret_cast<const int4 *>(&fst[TILE_R * b + 4 * g]);
                 const int fv[4] = {f4.x, f4.y, f4.z, f4.w};
 #pragma unroll
-                for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, 2>(P, t.head, 0, tile_pair_number(fv[r], mk[r], c))];
+                for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, 2>(P, t.head, 0, tile_pair_number(fv[r], B.mk[r], c))];
             }
         };
         auto compute = [&](const Blk &B) {
@@ -3235,22 +3272,23 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             const floatx4v st = tile_dot_bf16(kr, qb);
             float sc[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) sc[r] = ((B.has >> r) & 1) ? (BIAS ? st[r] + B.bz[BIAS ? r : 0] : st[r]) * scale_log2e : -INFINITY;
+            for (int r = 0; r < 4; ++r) sc[r] = where_pair(B.mk[r], c, (BIAS ? st[r] + B.bz[BIAS ? r : 0] : st[r]) * scale_log2e);
             const float mb = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
             if (__builtin_amdgcn_ballot_w64(mb > mref + MFMA_TAU) != 0) {
-                float gm = fmaxf(mb, __shfl_xor(mb, 16));
-                gm = fmaxf(gm, __shfl_xor(gm, 32));              // over the four lanes of member c
-                const float mn = fmaxf(mref, gm);
+                const float mn = fmaxf(mref, groups_max(mb));    // over the four lanes of member c
                 const float al = __builtin_amdgcn_exp2f(mref - mn);
                 mref = mn;
-                lrun *= al;
+                if (!fresh) {
+                    lrun *= al;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float a = lane_bcast(al, 4 * g + r);
+                    for (int r = 0; r < 4; ++r) {
+                        const float a = lane_bcast(al, 4 * g + r);
 #pragma unroll
-                    for (int nb = 0; nb < 4; ++nb) acc[nb][r] *= a;
+                        for (int nb = 0; nb < 4; ++nb) acc[nb][r] *= a;
+                    }
                 }
             }
+            fresh = false;
             float pr[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -3269,8 +3307,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
         else tile_walk_first_ahead<Blk>(nblk, issue_k, issue_rest, compute, []() {});
         wave_lds_fence();
     }
-    float lt = lrun + __shfl_xor(lrun, 16);
-    lt += __shfl_xor(lt, 32);
+    float lt = groups_sum(lrun);
     if constexpr (SP > 1) {
         tile_meet_forward<SP, H, D, NARROW>(piece[t.wv], piece[t.wv % (HW / SP)], (HW / SP) * PIECE, t, acc, mref, lt, o, ws_acc, nw, o_keep);
         if (t.part != 0) return;
@@ -3334,8 +3371,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
                 part = fmaf(__uint_as_float(a[i] & 0xffff0000u), __uint_as_float(b[i] & 0xffff0000u), part);
             }
         }
-        part += __shfl_xor(part, 16);
-        delta = part + __shfl_xor(part, 32);                      // dO . O of member c, this head
+        delta = groups_sum(part);                                 // dO . O of member c, this head
         const size_t at = (size_t)max(t.member.x, 0) * Hs + t.head;
         lse_c = lse[at];
         if constexpr (!PDS) {
@@ -3347,7 +3383,8 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
     for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
     struct Blk {
         uint2 kc[4], vc[4];                                       // columns 4 c .. 4 c + 3 of the K / V rows of entries 4 g + r
-        int has, pos[PDS ? 4 : 1];                                 // bit r of has: the pair (entry 4 g + r, member c) exists
+        int mk[4];                                                // bit c of mk[r]: the pair (entry 4 g + r, member c) exists
+        uint32_t pos[PDS ? 4 : 1];
         int xe[DROP || BIAS == 1 ? 4 : 1];
         float bz[BIAS ? 4 : 1];
     };
@@ -3360,7 +3397,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
             const int4 e01 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g]);
             const int4 e23 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g + 2]);
             const int idxv[4] = {e01.x, e01.z, e23.x, e23.z};
-            B.has = ((e01.y >> c) & 1) | (((e01.w >> c) & 1) << 1) | (((e23.y >> c) & 1) << 2) | (((e23.w >> c) & 1) << 3);
+            B.mk[0] = e01.y; B.mk[1] = e01.w; B.mk[2] = e23.y; B.mk[3] = e23.w;
             if constexpr (PDS) {
                 const int4 f4 = *reinterpret_cast<const int4 *>(&fst[TILE_R * b + 4 * g]);
                 B.pos[0] = tile_pair_number(f4.x, e01.y, c); B.pos[1] = tile_pair_number(f4.y, e01.w, c);
@@ -3384,14 +3421,13 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
             float ds[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const bool has = (B.has >> r) & 1;
-                float pe = has ? __builtin_amdgcn_exp2f((BIAS ? st[r] + B.bz[BIAS ? r : 0] : st[r]) * scale_log2e - lse_c) : 0.f;
+                float pe = where_pair_or_zero(B.mk[r], c, __builtin_amdgcn_exp2f((BIAS ? st[r] + B.bz[BIAS ? r : 0] : st[r]) * scale_log2e - lse_c));
                 float mt = 1.f;                                   // dropout multiplier of this pair (as in the forward)
                 if constexpr (DROP)
                     mt = dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)Hs + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
                 ds[r] = pe * (dp[r] * mt - delta) * scale;
                 pe *= mt;                                         // what multiplies v (forward) and dO (dV)
-                if (PDS && has) {
+                if (PDS && ((B.mk[r] >> c) & 1)) {
                     pds_h[B.pos[PDS ? r : 0]] = pack_bf16(pe, ds[r]);
                     if constexpr (BIAS) ds_out[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], B.pos[PDS ? r : 0])] = ds[r];   // dL/d(score before scaling)
                 }
@@ -3436,7 +3472,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     struct Blk {
         uint2 qr[4], dr[4];
         uint32_t w[4];                                            // (p, ds) of the pairs (entry c, member 4 g + r)
-        int has;                                                  // bit r: the pair (entry 4 g + r, member c) exists
+        int mk[4];                                                // bit c of mk[r]: the pair (entry 4 g + r, member c) exists
     };
     for (int p0 = t.p_begin; p0 < t.p_end; p0 += TILE_CHUNK) {
         const int cnt = min(TILE_CHUNK, t.p_end - p0), nblk = (cnt + TILE_R - 1) / TILE_R;
@@ -3451,7 +3487,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             const int4 e01 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g]);
             const int4 e23 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g + 2]);
             const int idxv[4] = {e01.x, e01.z, e23.x, e23.z};
-            B.has = ((e01.y >> c) & 1) | (((e01.w >> c) & 1) << 1) | (((e23.y >> c) & 1) << 2) | (((e23.w >> c) & 1) << 3);
+            B.mk[0] = e01.y; B.mk[1] = e01.w; B.mk[2] = e23.y; B.mk[3] = e23.w;
             int pos[4];
             if (b == ahead_of) {
 #pragma unroll
@@ -3466,7 +3502,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
                 const uint32_t off = (uint32_t)idxv[r] * RB + offc;
                 B.qr[r] = tile_row4_bf16<NARROW>(qb + off);
                 B.dr[r] = tile_row4_bf16<NARROW>(db + off);
-                B.w[r] = pds_h[pos[r]];
+                B.w[r] = pds_h[(uint32_t)pos[r]];
             }
         };
         auto compute = [&](const Blk &B) {
@@ -3477,7 +3513,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             for (int r = 0; r < 4; ++r) w[r] = wt[(4 * g + r) * TILE_WT_STRIDE_BF16 + c];
             wave_lds_fence();                                     // (read before the next block's are written)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) w[r] = ((B.has >> r) & 1) ? w[r] : 0u;       // the scratch of pairs that do not exist is not initialised
+            for (int r = 0; r < 4; ++r) w[r] &= (uint32_t)__builtin_amdgcn_sbfe(B.mk[r], c, 1);       // the scratch of pairs that do not exist is not initialised
             Bf4 pa, da;
             pa.u[0] = pack_lo16(w[0], w[1]); pa.u[1] = pack_lo16(w[2], w[3]);
             da.u[0] = pack_hi16(w[0], w[1]); da.u[1] = pack_hi16(w[2], w[3]);
@@ -3546,7 +3582,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     struct Blk {
         uint2 qr[4], dr[4];                                       // columns 4 c .. 4 c + 3 of the q / dO rows of entries 4 g + r
         float2 ld;                                                // (lse, delta) of entry c
-        int has;                                                  // bit r: the pair (entry 4 g + r, member c) exists
+        int mk[4];                                                // bit c of mk[r]: the pair (entry 4 g + r, member c) exists
         int xe[DROP ? 4 : 1];
     };
     for (int p0 = t.p_begin; p0 < t.p_end; p0 += TILE_CHUNK) {
@@ -3558,7 +3594,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             const int4 e01 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g]);
             const int4 e23 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g + 2]);
             const int idxv[4] = {e01.x, e01.z, e23.x, e23.z};
-            B.has = ((e01.y >> c) & 1) | (((e01.w >> c) & 1) << 1) | (((e23.y >> c) & 1) << 2) | (((e23.w >> c) & 1) << 3);
+            B.mk[0] = e01.y; B.mk[1] = e01.w; B.mk[2] = e23.y; B.mk[3] = e23.w;
             B.ld = stat_h[(size_t)ent[TILE_R * b + c].x * H];
 #pragma unroll
             for (int r = 0; r < 4; ++r) B.qr[r] = tile_row4_bf16<false>(qb + ((uint32_t)idxv[r] * RB + offc));
@@ -3577,12 +3613,11 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             float pe[4], ds[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const bool has = (B.has >> r) & 1;
-                const float p = has ? __builtin_amdgcn_exp2f(st[r] * scale_log2e - lse_e[r]) : 0.f;
+                const float p = where_pair_or_zero(B.mk[r], c, __builtin_amdgcn_exp2f(st[r] * scale_log2e - lse_e[r]));
                 float mt = 1.f;                                   // dropout multiplier of this pair (as in the forward)
                 if constexpr (DROP)
                     mt = dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)H + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
-                ds[r] = has ? p * (dp[r] * mt - delta_e[r]) * scale : 0.f;
+                ds[r] = where_pair_or_zero(B.mk[r], c, p * (dp[r] * mt - delta_e[r]) * scale);
                 pe[r] = p * mt;
             }
             Bf4 pa, da;
