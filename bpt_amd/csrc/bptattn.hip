@@ -2594,8 +2594,8 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
 // Backward on tiles, destination side: per block the scores and dO . v of all 16 x 16 pairs (two products over the
 // columns, the K and V rows turned in LDS from the layout they are loaded in), p = 2^(s - lse),
 // ds = p (dO . v - delta) scale, dq += ds K (third product, on the K rows as loaded).  With dropout or a score term the
-// kernel is compiled for three wavefronts per SIMD or more: held to four it kept the members' q rows in scratch memory and reads
-// them back for every block (83 against 58 us with dropout at L = 8192, k = 4; with dropout alone four fit by themselves since).
+// kernel is compiled for three wavefronts per SIMD: at four it keeps the members' q rows in scratch memory and reads
+// them back for every block (83 against 58 us with dropout at L = 8192, k = 4).
 // (p, ds) of the pairs that exist go to a scratch in THIS side's order, compact:
 // pds[head * n_edges + t] for the pair number t of (entry, member) = the entry's first pair + the rank of the member in
 // its mask, so the lanes of an entry write one contiguous run and the runs of consecutive entries follow each other.  The
@@ -3104,16 +3104,14 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(5))) 
 // v_mfma_f32_16x16x32_bf16 (products over the 64 columns: two instructions) and v_mfma_f32_16x16x16_bf16 (products over
 // the 16 entries of a block: one instruction per four output columns), float32 accumulation:
 //   lane (c, g) holds columns 16 g .. 16 g + 15 of the row of entry c (32 contiguous bytes; slot j of step t of the product
-//   stands for column 16 g + 8 t + j in both operands; the members' rows are loaded that way, the entries' rows turned in
-//   LDS, see tile_rows_to_operand_bf16) and loads columns 4 c .. 4 c + 3 of the rows of entries 4 g + r (8 bytes; the B
-//   operand of output columns {4 c + nb} takes element nb of each of the four, packed by byte permutes).
+//   stands for column 16 g + 8 t + j in both operands).
+// Heads of 64 columns: rows go through LDS for both kinds of product (k_attn_fwd_rows_bf16, k_attn_bwd_dst_rows_bf16,
+// k_attn_bwd_src_tile_bf16_again; tile_ask_rows_bf16 says why), the next block's asked for while this one's are used.  Narrower heads, and
+// the source side that reads (p, ds) back: a lane loads columns 4 c .. 4 c + 3 of the rows of entries 4 g + r (8 bytes; the B
+// operand of output columns {4 c + nb} takes element nb of each of the four, packed by byte permutes), and the entries' rows
+// are turned in LDS for the products over the columns (tile_rows_to_operand_bf16).
 // Probabilities and ds are rounded to bfloat16 where they enter a product (the softmax denominator is summed unrounded);
 // the scratch between the two backward kernels, where there is one, holds (p, ds) as two bfloat16 in 4 bytes, by head and destination-side pair number.
-// A two-stage register pipeline does not pay here: at six wavefronts per SIMD it spills (2.4 x slower),
-// at four it measured 5 to 10 % slower on the sparse graphs and level on the window graph.  Tiles of 32 rows (two member
-// blocks per wavefront on the same loaded rows, three or four wavefronts per SIMD) did not pay either: the entry lists
-// shrink by a third on the destination side but only by an eighth on the source side (L = 8192, k = 4: 67 k -> 46 k and
-// 71 k -> 62 k entries), and the step went from 0.113 to 0.117 ms (32-graph batch 0.177 -> 0.205, window 128 level).
 constexpr int TILE_BF16_WPE = 5, TILE_BF16_WPE_DST = 5, TILE_BF16_WPE_SRC = 5, TILE_BF16_WPE_AGAIN = 4;     // wavefronts per SIMD the bfloat16 tile kernels are compiled for
 typedef __bf16 bf16x8v __attribute__((ext_vector_type(8)));
 typedef short shortx4v __attribute__((ext_vector_type(4)));
@@ -3146,23 +3144,17 @@ __device__ __forceinline__ floatx4v tile_dot_bf16(const Bf8 (&a)[2], const Bf8 (
     s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0].v, b[0].v, s, 0, 0, 0);
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[1].v, b[1].v, s, 0, 0, 0);
 }
-template <bool NARROW>
 __device__ __forceinline__ void tile_load_row_bf16(const char *p, Bf8 (&out)[2], int g, const Narrow &nw) {
-    if constexpr (NARROW) {
-        uint32_t w[8];
+    uint32_t w[8];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {                             // quad 4 g + t; d is even, so a quad is shifted by whole words
-            const int quad = 4 * (4 * g + t), col = min(quad, nw.d - 4);
-            const uintx2u x = *reinterpret_cast<const uintx2u *>(p + 2 * col);
-            w[2 * t] = col >= quad ? x[0] : 0u;
-            w[2 * t + 1] = col + 2 >= quad ? x[1] : 0u;
-        }
-        out[0].q = make_uint4(w[0], w[1], w[2], w[3]);
-        out[1].q = make_uint4(w[4], w[5], w[6], w[7]);
-    } else {
-        out[0].q = *reinterpret_cast<const uint4 *>(p);
-        out[1].q = *reinterpret_cast<const uint4 *>(p + 16);
+    for (int t = 0; t < 4; ++t) {                                 // quad 4 g + t; d is even, so a quad is shifted by whole words
+        const int quad = 4 * (4 * g + t), col = min(quad, nw.d - 4);
+        const uintx2u x = *reinterpret_cast<const uintx2u *>(p + 2 * col);
+        w[2 * t] = col >= quad ? x[0] : 0u;
+        w[2 * t + 1] = col + 2 >= quad ? x[1] : 0u;
     }
+    out[0].q = make_uint4(w[0], w[1], w[2], w[3]);
+    out[1].q = make_uint4(w[4], w[5], w[6], w[7]);
 }
 template <bool NARROW> __device__ __forceinline__ uint2 tile_row4_bf16(const char *p) {
     if constexpr (NARROW) {
@@ -3178,12 +3170,11 @@ template <bool NARROW> __device__ __forceinline__ uint2 tile_row4_bf16(const cha
 // Rows of TILE_KT_BYTES_BF16 = 128 + 16 bytes: the sixteen rows of a read fall on different banks.
 constexpr int TILE_KT_BYTES_BF16 = 144;
 typedef uint32_t uintx4v __attribute__((ext_vector_type(4)));
-template <bool NARROW>
 __device__ __forceinline__ void tile_rows_to_operand_bf16(char *kt, const uint2 (&rows)[4], int c, int g, Bf8 (&out)[2], const Narrow &nw) {
 #pragma unroll
     for (int r = 0; r < 4; ++r)
         *reinterpret_cast<uintx2v *>(kt + (4 * g + r) * TILE_KT_BYTES_BF16 + 8 * c) =           // (d is even: words are whole)
-            uintx2v{narrow_again<NARROW>(nw, c, 0) ? 0u : rows[r].x, narrow_again<NARROW>(nw, c, 2) ? 0u : rows[r].y};
+            uintx2v{narrow_again<true>(nw, c, 0) ? 0u : rows[r].x, narrow_again<true>(nw, c, 2) ? 0u : rows[r].y};
     wave_lds_fence();
     const char *src = kt + c * TILE_KT_BYTES_BF16 + 32 * g;
 #pragma unroll
@@ -3195,23 +3186,412 @@ __device__ __forceinline__ void tile_rows_to_operand_bf16(char *kt, const uint2 
 }
 
 constexpr int TILE_KT_FLOATS_BF16 = TILE_R * TILE_KT_BYTES_BF16 / 4;
-template <int H, int D, int HW, int WPE, bool DROP, int BIAS, bool NARROW = false, int SP = 1>
-__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))) void k_attn_fwd_tile_bf16(
+// Rows of 64 columns, 16 bytes a lane: lane l asks for piece l % 8 of rows l / 8 and 8 + l / 8 of sixteen, puts them into LDS as
+// above, and both kinds of product read them there: the products over the columns the row of entry c, the sums over the
+// entries their columns, transposed (tile_axpy_rows_bf16), so that the registers are free for the next block's rows.
+//
+// What bounds the bfloat16 kernels is the texture addresser, which takes a vector memory instruction four lanes at a time: 16 cycles
+// for one whose neighbouring lanes read on in a line, whatever a lane reads of it, 64 where each lane's line is another
+// (busy 77 % of all three kernels at 16 heads, L = 32768, k = 8).  Rows of eight bytes a lane took twice the instructions, members' rows
+// read row by lane four times the cycles, (lse, delta) of a block's entries read by all 64 lanes as many as its rows.  So: rows, members'
+// rows and results in 16 bytes a lane, along the rows; single words of a row by one lane group.  Nothing else helped the source side there:
+// its rows a block ahead through LDS but 8 bytes a lane 333 -> 343 us; 16 bytes a lane 315; the members and (lse, delta) too 303;
+// free of bank conflicts in LDS 281 to 290.  Kernels before -> after, forward / destination / source side: 16 heads at L = 32768, k = 8 184 / 240 / 333
+// -> 162 / 208 / 285 us, 8 heads at L = 8192, k = 4 17.1 / 24.6 / 26.5 -> 16.4 / 22.8 / 23.6.  Training passes: window of 64 at L = 16384,
+// 16 heads 163.5 -> 139.8, 32-graph batch 152 -> 139.8, L = 16384, k = 8 180 -> 158, with dropout at L = 32768, k = 8 818 -> 760.
+__device__ __forceinline__ void tile_ask_rows_bf16(const char *base, const uint32_t (&off)[2], uintx4v (&rows)[2]) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r) rows[r] = *reinterpret_cast<const uintx4v *>(base + off[r]);
+}
+// In LDS such rows lie 128 bytes apart, piece j of row e at place j ^ piece_turn(e): two rows of a write, the sixteen rows of an operand's
+// read and the eight rows of a transposed read (32 lanes of 8 bytes, two pieces a row) fall on different banks.
+constexpr int TILE_ROWS_FLOATS_BF16 = TILE_R * 32;
+__device__ __forceinline__ int piece_turn(int e) { return (e & 6) | (e >> 3); }
+__device__ __forceinline__ void tile_put_rows_bf16(char *kt, const uintx4v (&rows)[2], int lane) {
+    const int at = (lane >> 3) * 128 + 16 * ((lane & 7) ^ piece_turn(lane >> 3));
+    *reinterpret_cast<uintx4v *>(kt + at) = rows[0];
+    *reinterpret_cast<uintx4v *>(kt + (at ^ 16) + 1024) = rows[1];
+}
+__device__ __forceinline__ void tile_operand_bf16(const char *kt, int c, int g, Bf8 (&out)[2]) {
+    const int at = c * 128 + 16 * ((2 * g) ^ piece_turn(c));
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const uintx4v x = *reinterpret_cast<const uintx4v *>(kt + (at ^ (16 * i)));
+        out[i].q = make_uint4(x[0], x[1], x[2], x[3]);
+    }
+}
+// byte offsets of this lane's pieces of the members' rows / of the rows of the sixteen entries at `ent`
+__device__ __forceinline__ uint32_t tile_piece_at(const TileCtx &t) { return (uint32_t)(t.head * 128 + 16 * (t.lane & 7)); }
+template <uint32_t RB> __device__ __forceinline__ void tile_member_offsets(const TileCtx &t, uint32_t (&off)[2]) {
+    const int row = max(t.member.x, 0);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) off[r] = (uint32_t)lane_bcast(row, 8 * r + (t.lane >> 3)) * RB + tile_piece_at(t);
+}
+template <uint32_t RB> __device__ __forceinline__ void tile_entry_offsets(const TileCtx &t, const int2 *ent, uint32_t (&off)[2]) {
+#pragma unroll
+    for (int r = 0; r < 2; ++r) off[r] = (uint32_t)ent[8 * r + (t.lane >> 3)].x * RB + tile_piece_at(t);
+}
+// masks of entries 4 g .. 4 g + 3
+__device__ __forceinline__ void tile_masks(const int2 *ent, int g, int (&mk)[4]) {
+    const int4 e01 = *reinterpret_cast<const int4 *>(&ent[4 * g]), e23 = *reinterpret_cast<const int4 *>(&ent[4 * g + 2]);
+    mk[0] = e01.y; mk[1] = e01.w; mk[2] = e23.y; mk[3] = e23.w;
+}
+// acc += w^T rows, by column: lane (c, g), register r of acc[nb] = column 16 nb + 4 g + r of member c
+__device__ __forceinline__ void tile_axpy_rows_bf16(const Bf4 &w, const char *kt, int c, int g, floatx4v (&acc)[4]) {
+    // sixteen lanes read four rows of sixteen columns and are given one column of the four each
+    const int e = 4 * g + (c >> 2), at = e * 128 + 16 * (((c >> 1) & 1) ^ piece_turn(e)) + 8 * (c & 1);
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) {
+        const shortx4v cols = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) shortx4v *)(kt + (at ^ (32 * nb))));
+        acc[nb] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(cols, w.v, acc[nb], 0, 0, 0);
+    }
+}
+// Such sums through LDS (TILE_R * TILE_TURN_STRIDE floats): into the tile kernels' other order (lane (c, g), register r: columns 4 c .. 4 c + 3
+// of member 4 g + r), or to where the members' rows go.
+constexpr int TILE_TURN_STRIDE = 68;
+__device__ __forceinline__ void tile_put_sums(float *sh, const floatx4v (&acc)[4], int c, int g) {
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) *reinterpret_cast<floatx4v *>(sh + c * TILE_TURN_STRIDE + 16 * nb + 4 * g) = acc[nb];
+    wave_lds_fence();
+}
+__device__ __forceinline__ void tile_sums_by_row(float *sh, floatx4v (&acc)[4], int c, int g) {
+    tile_put_sums(sh, acc, c, g);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const floatx4v x = *reinterpret_cast<const floatx4v *>(sh + (4 * g + r) * TILE_TURN_STRIDE + 4 * c);
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) acc[nb][r] = x[nb];
+    }
+    wave_lds_fence();
+}
+template <int H, int D>
+__device__ __forceinline__ void tile_store_sums(const TileCtx &t, float *sh, const floatx4v (&acc)[4], bf16_t *__restrict__ out, float *__restrict__ ws) {
+    tile_put_sums(sh, acc, t.c, t.g);
+    const int where = tile_where(t.member);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const int m = 8 * r + (t.lane >> 3), at = lane_bcast(where, m);
+        const floatx4v *const from = reinterpret_cast<const floatx4v *>(sh + m * TILE_TURN_STRIDE + 8 * (t.lane & 7));
+        const floatx4v x = from[0], y = from[1];
+        if (at >= 0) {                                            // (node tensors end before 4 GiB)
+            char *const to = reinterpret_cast<char *>(out) + ((uint32_t)at * (uint32_t)(H * D * 2) + tile_piece_at(t));
+            __builtin_nontemporal_store(uintx4v{pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3]), pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3])},
+                                        reinterpret_cast<uintx4v *>(to));
+        } else if (at < -1) {
+            floatx4v *const to = reinterpret_cast<floatx4v *>(ws + (size_t)(-2 - at) * (H * D) + t.head * D + 8 * (t.lane & 7));
+            to[0] = x;
+            to[1] = y;
+        }
+    }
+    wave_lds_fence();
+}
+
+template <int H, int D, int HW, int WPE, bool DROP, int BIAS, int SP>
+__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP || BIAS ? WPE - 1 : WPE))) void k_attn_fwd_rows_bf16(
     bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, bf16_t *__restrict__ o,
     float *__restrict__ lse, float *__restrict__ ws_acc, float *__restrict__ ws_ml, float scale_log2e, uint32_t drop_thr,
-    uint32_t drop_seed, float drop_inv, const float *__restrict__ bias, Narrow nw, Keep keep) {
-    const int Hs = NARROW ? nw.h : H;                             // heads as lse, workspace and dropout keys count them
-    const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * 2 : (uint32_t)(H * D * 2);                       // bytes of a node row
-    int block = (int)blockIdx.x;
-    if constexpr (NARROW) block = keep_or_tile<HW * WAVE>(keep);
-    if (NARROW && block < 0) return;
-    bf16_t *const o_keep = NARROW ? reinterpret_cast<bf16_t *>(keep.o) : nullptr;
+    uint32_t drop_seed, float drop_inv, const float *__restrict__ bias) {
+    constexpr uint32_t RB = H * D * 2;
+    const Narrow nw{};
     TileCtx t;
-    if (!tile_begin<bf16_t, H, D, HW, NARROW, SP>(P, t, nw, (unsigned)block)) return;
+    if (!tile_begin<bf16_t, H, D, HW, false, SP>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
     __shared__ int fst_lds[HW][BIAS == 2 ? TILE_CHUNK : 1];      // the entries' first pair numbers: where a term in pair order sits
     int2 *ent = ent_lds[t.wv];
     int *fst = BIAS == 2 ? fst_lds[t.wv] : nullptr;
+    constexpr int PIECE = 2 * TILE_ROWS_FLOATS_BF16 + 4 * TILE_R;      // (the turned sums' rows are longer)
+    static_assert(PIECE >= TILE_PART_FWD_FLOATS && PIECE >= TILE_R * TILE_TURN_STRIDE, "parts and turned sums fit the rows' piece");
+    __shared__ __attribute__((aligned(16))) float piece[HW][PIECE];
+    char *const k_lds = reinterpret_cast<char *>(piece[t.wv]), *const v_lds = k_lds + 4 * TILE_ROWS_FLOATS_BF16;
+    TileEntryRegs er;
+    if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
+    issue_loads_first();
+    const int c = t.c, g = t.g;
+    const char *kb = reinterpret_cast<const char *>(k), *vb = reinterpret_cast<const char *>(v);
+    uintx4v qr[2];
+    {
+        uint32_t off[2];
+        tile_member_offsets<RB>(t, off);
+        tile_ask_rows_bf16(reinterpret_cast<const char *>(q), off, qr);
+    }
+    issue_loads_first();
+    Bf8 qb[2];
+    floatx4v acc[4];
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
+    float mref = M_INIT_LOG2, lrun = 0.f;
+    bool fresh = true;                                            // nothing has been summed up yet
+    struct Blk {
+        uintx4v kr[2], vr[2];
+        int xe[DROP || BIAS == 1 ? 4 : 1];
+        float bz[BIAS ? 4 : 1];
+    };
+    for (int p0 = t.p_begin; p0 < t.p_end; p0 += TILE_CHUNK) {
+        const int cnt = min(TILE_CHUNK, t.p_end - p0), nblk = (cnt + TILE_R - 1) / TILE_R;
+        if (p0 != t.p_begin) tile_ask_entries(P, p0, cnt, t.lane, er);
+        tile_put_entries(er, ent, cnt, t.lane, fst);
+        auto issue = [&](Blk &B, int b) {
+            if constexpr (DROP || BIAS == 1) tile_pair_eids(P, p0 + TILE_R * b + 4 * g, t.p_end, c, B.xe);
+            uint32_t off[2];
+            tile_entry_offsets<RB>(t, ent + TILE_R * b, off);
+            tile_ask_rows_bf16(kb, off, B.kr);
+            tile_ask_rows_bf16(vb, off, B.vr);
+            if constexpr (BIAS == 1) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, 1>(P, t.head, B.xe[BIAS == 1 ? r : 0], 0)];
+            }
+            if constexpr (BIAS == 2) {
+                int mk[4];
+                tile_masks(ent + TILE_R * b, g, mk);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, 2>(P, t.head, 0, tile_pair_number(fst[TILE_R * b + 4 * g + r], mk[r], c))];
+            }
+        };
+        Blk B;
+        issue(B, 0);
+        issue_loads_first();
+        if (p0 == t.p_begin) {
+            tile_put_rows_bf16(k_lds, qr, t.lane);
+            wave_lds_fence();
+            tile_operand_bf16(k_lds, c, g, qb);
+            wave_lds_fence();
+        }
+        for (int b = 0; b < nblk; ++b) {
+            int mk[4], xe[DROP ? 4 : 1];
+            float bz[BIAS ? 4 : 1];
+            tile_masks(ent + TILE_R * b, g, mk);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if constexpr (DROP) xe[DROP ? r : 0] = B.xe[DROP ? r : 0];
+                if constexpr (BIAS) bz[BIAS ? r : 0] = B.bz[BIAS ? r : 0];
+            }
+            tile_put_rows_bf16(k_lds, B.kr, t.lane);
+            tile_put_rows_bf16(v_lds, B.vr, t.lane);
+            wave_lds_fence();
+            if (b + 1 < nblk) issue(B, b + 1);
+            issue_loads_first();
+            Bf8 kr[2];
+            tile_operand_bf16(k_lds, c, g, kr);
+            const floatx4v st = tile_dot_bf16(kr, qb);
+            float sc[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sc[r] = where_pair(mk[r], c, (BIAS ? st[r] + bz[BIAS ? r : 0] : st[r]) * scale_log2e);
+            const float mb = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
+            if (__builtin_amdgcn_ballot_w64(mb > mref + MFMA_TAU) != 0) {
+                const float mn = fmaxf(mref, groups_max(mb));    // over the four lanes of member c
+                const float al = __builtin_amdgcn_exp2f(mref - mn);
+                mref = mn;
+                if (!fresh) {
+                    lrun *= al;
+#pragma unroll
+                    for (int nb = 0; nb < 4; ++nb) acc[nb] *= al;
+                }
+            }
+            fresh = false;
+            float pr[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                pr[r] = __builtin_amdgcn_exp2f(sc[r] - mref);
+                lrun += pr[r];                                   // the softmax denominator ignores dropout
+                if constexpr (DROP)
+                    pr[r] *= dropout_keep((uint32_t)xe[DROP ? r : 0] * (uint32_t)H + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
+            }
+            Bf4 pa;
+            pa.u[0] = pack_bf16(pr[0], pr[1]);
+            pa.u[1] = pack_bf16(pr[2], pr[3]);
+            tile_axpy_rows_bf16(pa, v_lds, c, g, acc);
+            wave_lds_fence();                                     // (read before the next block's are written)
+            issue_loads_first();
+        }
+    }
+    float lt = groups_sum(lrun);
+    if constexpr (SP > 1) {
+        tile_sums_by_row(piece[t.wv], acc, c, g);
+        tile_meet_forward<SP, H, D, false>(piece[t.wv], piece[t.wv % (HW / SP)], (HW / SP) * PIECE, t, acc, mref, lt, o, ws_acc, nw, static_cast<bf16_t *>(nullptr));
+        if (t.part != 0) return;
+    } else {
+        if (t.member.y < 0) {                                     // (segments of a split row are stored as summed up)
+            const float inv = lt > 0.f ? 1.f / lt : 0.f;
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) acc[nb] *= inv;
+        }
+        tile_store_sums<H, D>(t, piece[t.wv], acc, o, ws_acc);
+    }
+    if (g == 0 && t.member.x >= 0) {
+        if (t.member.y < 0) {
+            lse[(size_t)t.member.x * H + t.head] = lt > 0.f ? mref + log2f(lt) : 0.f;
+        } else {
+            ws_ml[((size_t)t.member.y * H + t.head) * 2] = mref;
+            ws_ml[((size_t)t.member.y * H + t.head) * 2 + 1] = lt;
+        }
+    }
+}
+
+// Destination side.  PDS: (p, ds) of the pairs go to the scratch for the source side that reads them back; otherwise that side
+// forms them again (k_attn_bwd_src_tile_bf16_again) and all it is handed is (lse, delta) of the rows, `stat` (n, H): the
+// segments of a split row write the same values.
+template <int H, int D, int HW, int WPE, bool DROP, int BIAS, bool PDS, int SP>
+__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP || BIAS ? WPE - 1 : WPE))) void k_attn_bwd_dst_rows_bf16(
+    bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, const bf16_t *__restrict__ o,
+    const bf16_t *__restrict__ d_o, const float *__restrict__ lse, bf16_t *__restrict__ dq, uint32_t *__restrict__ pds,
+    float2 *__restrict__ stat, float *__restrict__ ws_dq, float scale, float scale_log2e, uint32_t drop_thr, uint32_t drop_seed, float drop_inv,
+    const float *__restrict__ bias, float *__restrict__ ds_out) {
+    static_assert(PDS || BIAS == 0, "the score term's gradient is stored by the pair's position");
+    constexpr uint32_t RB = H * D * 2;
+    const Narrow nw{};
+    TileCtx t;
+    if (!tile_begin<bf16_t, H, D, HW, false, SP>(P, t, nw)) return;
+    __shared__ int2 ent_lds[HW][TILE_CHUNK];
+    __shared__ int fst_lds[HW][PDS ? TILE_CHUNK : 1];
+    int2 *ent = ent_lds[t.wv];
+    int *fst = PDS ? fst_lds[t.wv] : nullptr;
+    constexpr int PIECE = 2 * TILE_ROWS_FLOATS_BF16 + 4 * TILE_R;      // (the turned sums' rows are longer)
+    static_assert(PIECE >= TILE_PART_FLOATS && PIECE >= TILE_R * TILE_TURN_STRIDE, "parts and turned sums fit the rows' piece");
+    __shared__ __attribute__((aligned(16))) float piece[HW][PIECE];
+    char *const k_lds = reinterpret_cast<char *>(piece[t.wv]), *const v_lds = k_lds + 4 * TILE_ROWS_FLOATS_BF16;
+    TileEntryRegs er;
+    if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
+    issue_loads_first();
+    const int c = t.c, g = t.g;
+    const char *kb = reinterpret_cast<const char *>(k), *vb = reinterpret_cast<const char *>(v);
+    uint32_t *const pds_h = pds + (size_t)t.head * (size_t)P.n_edges;     // this head's part of the scratch
+    Bf8 qb[2], dob[2];
+    float delta, lse_c;
+    {
+        uint32_t off[2];
+        tile_member_offsets<RB>(t, off);
+        uintx4v qr[2], dr[2], orow[2];
+        tile_ask_rows_bf16(reinterpret_cast<const char *>(d_o), off, dr);
+        tile_ask_rows_bf16(reinterpret_cast<const char *>(o), off, orow);
+        tile_ask_rows_bf16(reinterpret_cast<const char *>(q), off, qr);
+        const size_t at = (size_t)max(t.member.x, 0) * H + t.head;
+        lse_c = g == 0 ? lse[at] : 0.f;
+        float part[2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            part[r] = 0.f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                part[r] = fmaf(__uint_as_float(dr[r][i] << 16), __uint_as_float(orow[r][i] << 16), part[r]);
+                part[r] = fmaf(__uint_as_float(dr[r][i] & 0xffff0000u), __uint_as_float(orow[r][i] & 0xffff0000u), part[r]);
+            }
+            part[r] = head_sum<8>(part[r]);                       // dO . O of member 8 r + l / 8, this head
+        }
+        tile_put_rows_bf16(k_lds, qr, t.lane);
+        tile_put_rows_bf16(v_lds, dr, t.lane);
+        wave_lds_fence();
+        tile_operand_bf16(k_lds, c, g, qb);
+        tile_operand_bf16(v_lds, c, g, dob);
+        wave_lds_fence();
+        const float d0 = lane_bcast(part[0], 8 * (c & 7)), d1 = lane_bcast(part[1], 8 * (c & 7));
+        delta = c < 8 ? d0 : d1;
+        if constexpr (!PDS) {
+            if (g == 0 && t.part == 0 && t.member.x >= 0) stat[at] = make_float2(lse_c, delta);
+        }
+        lse_c = lane_bcast(lse_c, c);
+    }
+    floatx4v acc[4];
+#pragma unroll
+    for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
+    struct Blk {
+        uintx4v kr[2], vr[2];
+        int xe[DROP || BIAS == 1 ? 4 : 1];
+        float bz[BIAS ? 4 : 1];
+    };
+    for (int p0 = t.p_begin; p0 < t.p_end; p0 += TILE_CHUNK) {
+        const int cnt = min(TILE_CHUNK, t.p_end - p0), nblk = (cnt + TILE_R - 1) / TILE_R;
+        if (p0 != t.p_begin) tile_ask_entries(P, p0, cnt, t.lane, er);
+        tile_put_entries(er, ent, cnt, t.lane, fst);
+        auto numbers = [&](int b, const int (&mk)[4], uint32_t (&pos)[4]) {
+            const int4 f4 = *reinterpret_cast<const int4 *>(&fst[TILE_R * b + 4 * g]);
+            pos[0] = tile_pair_number(f4.x, mk[0], c); pos[1] = tile_pair_number(f4.y, mk[1], c);
+            pos[2] = tile_pair_number(f4.z, mk[2], c); pos[3] = tile_pair_number(f4.w, mk[3], c);
+        };
+        auto issue = [&](Blk &B, int b) {
+            if constexpr (DROP || BIAS == 1) tile_pair_eids(P, p0 + TILE_R * b + 4 * g, t.p_end, c, B.xe);
+            uint32_t off[2];
+            tile_entry_offsets<RB>(t, ent + TILE_R * b, off);
+            tile_ask_rows_bf16(kb, off, B.kr);
+            tile_ask_rows_bf16(vb, off, B.vr);
+            if constexpr (BIAS) {
+                int mk[4];
+                uint32_t pos[4];
+                tile_masks(ent + TILE_R * b, g, mk);
+                numbers(b, mk, pos);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], pos[r])];
+            }
+        };
+        Blk B;
+        issue(B, 0);
+        for (int b = 0; b < nblk; ++b) {
+            int mk[4], xe[DROP || BIAS == 1 ? 4 : 1];
+            float bz[BIAS ? 4 : 1];
+            uint32_t pos[4];
+            tile_masks(ent + TILE_R * b, g, mk);
+            if constexpr (PDS) numbers(b, mk, pos);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if constexpr (DROP || BIAS == 1) xe[DROP || BIAS == 1 ? r : 0] = B.xe[DROP || BIAS == 1 ? r : 0];
+                if constexpr (BIAS) bz[BIAS ? r : 0] = B.bz[BIAS ? r : 0];
+            }
+            tile_put_rows_bf16(k_lds, B.kr, t.lane);
+            tile_put_rows_bf16(v_lds, B.vr, t.lane);
+            wave_lds_fence();
+            if (b + 1 < nblk) issue(B, b + 1);
+            issue_loads_first();
+            Bf8 row[2];
+            tile_operand_bf16(k_lds, c, g, row);
+            const floatx4v st = tile_dot_bf16(row, qb);
+            tile_operand_bf16(v_lds, c, g, row);
+            const floatx4v dp = tile_dot_bf16(row, dob);
+            float ds[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                float pe = where_pair_or_zero(mk[r], c, __builtin_amdgcn_exp2f((BIAS ? st[r] + bz[BIAS ? r : 0] : st[r]) * scale_log2e - lse_c));
+                float mt = 1.f;                                   // dropout multiplier of this pair (as in the forward)
+                if constexpr (DROP)
+                    mt = dropout_keep((uint32_t)xe[DROP ? r : 0] * (uint32_t)H + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
+                ds[r] = pe * (dp[r] * mt - delta) * scale;
+                pe *= mt;                                         // what multiplies v (forward) and dO (dV)
+                if (PDS && ((mk[r] >> c) & 1)) {
+                    pds_h[pos[r]] = pack_bf16(pe, ds[r]);
+                    if constexpr (BIAS) ds_out[tile_bias_at<H, BIAS>(P, t.head, xe[BIAS == 1 ? r : 0], pos[r])] = ds[r];   // dL/d(score before scaling)
+                }
+            }
+            Bf4 da;
+            da.u[0] = pack_bf16(ds[0], ds[1]);
+            da.u[1] = pack_bf16(ds[2], ds[3]);
+            tile_axpy_rows_bf16(da, k_lds, c, g, acc);
+            wave_lds_fence();                                     // (read before the next block's are written)
+            issue_loads_first();
+        }
+    }
+    if constexpr (SP > 1) {
+        tile_sums_by_row(piece[t.wv], acc, c, g);
+        tile_park(piece[t.wv], acc, t.lane);
+        __syncthreads();
+        tile_meet_and_store<SP, H, D, false>(piece[t.wv % (HW / SP)], (HW / SP) * PIECE, t, dq, ws_dq, nw);
+    } else {
+        tile_store_sums<H, D>(t, piece[t.wv], acc, dq, ws_dq);
+    }
+}
+
+// Heads of fewer than 64 columns (their rows on 4 bytes): rows of 8 bytes a lane, kept in registers.
+template <int H, int D, int HW, int WPE, bool DROP, int SP>
+__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))) void k_attn_fwd_tile_bf16(
+    bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, bf16_t *__restrict__ o,
+    float *__restrict__ lse, float *__restrict__ ws_acc, float *__restrict__ ws_ml, float scale_log2e, uint32_t drop_thr,
+    uint32_t drop_seed, float drop_inv, Narrow nw, Keep keep) {
+    const int Hs = nw.h;                                          // heads as lse, workspace and dropout keys count them
+    const uint32_t RB = (uint32_t)(nw.heads * nw.d) * 2;          // bytes of a node row
+    const int block = keep_or_tile<HW * WAVE>(keep);
+    if (block < 0) return;
+    bf16_t *const o_keep = reinterpret_cast<bf16_t *>(keep.o);
+    TileCtx t;
+    if (!tile_begin<bf16_t, H, D, HW, true, SP>(P, t, nw, (unsigned)block)) return;
+    __shared__ int2 ent_lds[HW][TILE_CHUNK];
+    int2 *ent = ent_lds[t.wv];
     constexpr int PIECE = SP > 1 ? TILE_PART_FWD_FLOATS : TILE_KT_FLOATS_BF16;
     static_assert(PIECE >= TILE_KT_FLOATS_BF16, "the rows fit");
     __shared__ __attribute__((aligned(16))) float piece[HW][PIECE];
@@ -3220,10 +3600,10 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
     issue_loads_first();
     const int c = t.c, g = t.g;
-    const uint32_t offr = NARROW ? t.offa : (uint32_t)((t.head * D + 16 * g) * 2), offc = t.offv;
+    const uint32_t offr = t.offa, offc = t.offv;
     const char *kb = reinterpret_cast<const char *>(k), *vb = reinterpret_cast<const char *>(v);
     Bf8 qb[2];
-    tile_load_row_bf16<NARROW>(reinterpret_cast<const char *>(q) + (size_t)max(t.member.x, 0) * RB + offr, qb, g, nw);
+    tile_load_row_bf16(reinterpret_cast<const char *>(q) + (size_t)max(t.member.x, 0) * RB + offr, qb, g, nw);
     floatx4v acc[4];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
@@ -3233,46 +3613,35 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
         uint2 kq[4];                                              // columns 4 c .. 4 c + 3 of the K rows of entries 4 g + r
         uint2 vr[4];
         int mk[4];                                                // bit c of mk[r]: the pair (entry 4 g + r, member c) exists
-        int xe[DROP || BIAS == 1 ? 4 : 1];
-        float bz[BIAS ? 4 : 1];
+        int xe[DROP ? 4 : 1];
     };
     for (int p0 = t.p_begin; p0 < t.p_end; p0 += TILE_CHUNK) {
         const int cnt = min(TILE_CHUNK, t.p_end - p0), nblk = (cnt + TILE_R - 1) / TILE_R;
         if (p0 != t.p_begin) tile_ask_entries(P, p0, cnt, t.lane, er);
-        tile_put_entries(er, ent, cnt, t.lane, fst);
+        tile_put_entries(er, ent, cnt, t.lane);
         auto issue_k = [&](Blk &B, int b) {
             const int4 e01 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g]);
             const int4 e23 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g + 2]);
             const int idxv[4] = {e01.x, e01.z, e23.x, e23.z};
 #pragma unroll
-            for (int r = 0; r < 4; ++r) B.kq[r] = tile_row4_bf16<NARROW>(kb + ((uint32_t)idxv[r] * RB + offc));
+            for (int r = 0; r < 4; ++r) B.kq[r] = tile_row4_bf16<true>(kb + ((uint32_t)idxv[r] * RB + offc));
         };
         auto issue_rest = [&](Blk &B, int b) {
-            if constexpr (DROP || BIAS == 1) tile_pair_eids(P, p0 + TILE_R * b + 4 * g, t.p_end, c, B.xe);
+            if constexpr (DROP) tile_pair_eids(P, p0 + TILE_R * b + 4 * g, t.p_end, c, B.xe);
             const int4 e01 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g]);
             const int4 e23 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g + 2]);
             const int idxv[4] = {e01.x, e01.z, e23.x, e23.z};
             B.mk[0] = e01.y; B.mk[1] = e01.w; B.mk[2] = e23.y; B.mk[3] = e23.w;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) B.vr[r] = tile_row4_bf16<NARROW>(vb + ((uint32_t)idxv[r] * RB + offc));
-            if constexpr (BIAS == 1) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, 1>(P, t.head, B.xe[BIAS == 1 ? r : 0], 0)];
-            }
-            if constexpr (BIAS == 2) {
-                const int4 f4 = *reinterpret_cast<const int4 *>(&fst[TILE_R * b + 4 * g]);
-                const int fv[4] = {f4.x, f4.y, f4.z, f4.w};
-#pragma unroll
-                for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, 2>(P, t.head, 0, tile_pair_number(fv[r], B.mk[r], c))];
-            }
+            for (int r = 0; r < 4; ++r) B.vr[r] = tile_row4_bf16<true>(vb + ((uint32_t)idxv[r] * RB + offc));
         };
         auto compute = [&](const Blk &B) {
             Bf8 kr[2];
-            tile_rows_to_operand_bf16<NARROW>(kt, B.kq, c, g, kr, nw);
+            tile_rows_to_operand_bf16(kt, B.kq, c, g, kr, nw);
             const floatx4v st = tile_dot_bf16(kr, qb);
             float sc[4];
 #pragma unroll
-            for (int r = 0; r < 4; ++r) sc[r] = where_pair(B.mk[r], c, (BIAS ? st[r] + B.bz[BIAS ? r : 0] : st[r]) * scale_log2e);
+            for (int r = 0; r < 4; ++r) sc[r] = where_pair(B.mk[r], c, st[r] * scale_log2e);
             const float mb = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
             if (__builtin_amdgcn_ballot_w64(mb > mref + MFMA_TAU) != 0) {
                 const float mn = fmaxf(mref, groups_max(mb));    // over the four lanes of member c
@@ -3303,16 +3672,16 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
             tile_axpy_bf16(pa, B.vr, acc);
         };
         auto issue = [&](Blk &B, int b) { issue_k(B, b); issue_rest(B, b); };
-        if constexpr (DROP || BIAS != 0) tile_walk<Blk>(nblk, issue, compute);      // (the K rows ahead: eight registers more)
+        if constexpr (DROP) tile_walk<Blk>(nblk, issue, compute);      // (the K rows ahead: eight registers more)
         else tile_walk_first_ahead<Blk>(nblk, issue_k, issue_rest, compute, []() {});
         wave_lds_fence();
     }
     float lt = groups_sum(lrun);
     if constexpr (SP > 1) {
-        tile_meet_forward<SP, H, D, NARROW>(piece[t.wv], piece[t.wv % (HW / SP)], (HW / SP) * PIECE, t, acc, mref, lt, o, ws_acc, nw, o_keep);
+        tile_meet_forward<SP, H, D, true>(piece[t.wv], piece[t.wv % (HW / SP)], (HW / SP) * PIECE, t, acc, mref, lt, o, ws_acc, nw, o_keep);
         if (t.part != 0) return;
     } else {
-        tile_store_rows<H, D, true, NARROW>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc, nw, o_keep);
+        tile_store_rows<H, D, true, true>(t, acc, lt > 0.f ? 1.f / lt : 0.f, o, ws_acc, nw, o_keep);
     }
     if (g == 0 && t.member.x >= 0) {
         if (t.member.y < 0) {
@@ -3324,24 +3693,20 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     }
 }
 
-// Destination side.  PDS: (p, ds) of the pairs go to the scratch for the source side that reads them back; otherwise that side
-// forms them again (k_attn_bwd_src_tile_bf16_again) and all it is handed is (lse, delta) of the rows, `stat` (n, H): the
-// segments of a split row write the same values.
-template <int H, int D, int HW, int WPE, bool DROP, int BIAS, bool PDS, bool NARROW = false, int SP = 1>
-__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP || BIAS ? WPE - 1 : WPE))) void k_attn_bwd_dst_tile_bf16(
+// Destination side of such heads: (p, ds) of the pairs go to the scratch.
+template <int H, int D, int HW, int WPE, bool DROP, int SP>
+__global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP ? WPE - 1 : WPE))) void k_attn_bwd_dst_tile_bf16(
     bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, const bf16_t *__restrict__ o,
     const bf16_t *__restrict__ d_o, const float *__restrict__ lse, bf16_t *__restrict__ dq, uint32_t *__restrict__ pds,
-    float2 *__restrict__ stat, float *__restrict__ ws_dq, float scale, float scale_log2e, uint32_t drop_thr, uint32_t drop_seed, float drop_inv,
-    const float *__restrict__ bias, float *__restrict__ ds_out, Narrow nw) {
-    static_assert(PDS || BIAS == 0, "the score term's gradient is stored by the pair's position");
-    const int Hs = NARROW ? nw.h : H;
-    const uint32_t RB = NARROW ? (uint32_t)(nw.heads * nw.d) * 2 : (uint32_t)(H * D * 2);
+    float *__restrict__ ws_dq, float scale, float scale_log2e, uint32_t drop_thr, uint32_t drop_seed, float drop_inv, Narrow nw) {
+    const int Hs = nw.h;
+    const uint32_t RB = (uint32_t)(nw.heads * nw.d) * 2;
     TileCtx t;
-    if (!tile_begin<bf16_t, H, D, HW, NARROW, SP>(P, t, nw)) return;
+    if (!tile_begin<bf16_t, H, D, HW, true, SP>(P, t, nw)) return;
     __shared__ int2 ent_lds[HW][TILE_CHUNK];
-    __shared__ int fst_lds[HW][PDS ? TILE_CHUNK : 1];
+    __shared__ int fst_lds[HW][TILE_CHUNK];
     int2 *ent = ent_lds[t.wv];
-    int *fst = PDS ? fst_lds[t.wv] : nullptr;
+    int *fst = fst_lds[t.wv];
     constexpr int PIECE = SP > 1 ? TILE_PART_FLOATS : TILE_KT_FLOATS_BF16;
     static_assert(PIECE >= TILE_KT_FLOATS_BF16, "the rows fit");
     __shared__ __attribute__((aligned(16))) float piece[HW][PIECE];
@@ -3350,7 +3715,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
     if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
     issue_loads_first();
     const int c = t.c, g = t.g;
-    const uint32_t offr = NARROW ? t.offa : (uint32_t)((t.head * D + 16 * g) * 2), offc = t.offv;
+    const uint32_t offr = t.offa, offc = t.offv;
     const char *kb = reinterpret_cast<const char *>(k), *vb = reinterpret_cast<const char *>(v);
     const size_t mrow = (size_t)max(t.member.x, 0) * RB + offr;
     uint32_t *const pds_h = pds + (size_t)t.head * (size_t)P.n_edges;     // this head's part of the scratch
@@ -3358,9 +3723,9 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
     float delta, lse_c;
     {
         Bf8 ob[2];
-        tile_load_row_bf16<NARROW>(reinterpret_cast<const char *>(q) + mrow, qb, g, nw);
-        tile_load_row_bf16<NARROW>(reinterpret_cast<const char *>(d_o) + mrow, dob, g, nw);
-        tile_load_row_bf16<NARROW>(reinterpret_cast<const char *>(o) + mrow, ob, g, nw);
+        tile_load_row_bf16(reinterpret_cast<const char *>(q) + mrow, qb, g, nw);
+        tile_load_row_bf16(reinterpret_cast<const char *>(d_o) + mrow, dob, g, nw);
+        tile_load_row_bf16(reinterpret_cast<const char *>(o) + mrow, ob, g, nw);
         float part = 0.f;
 #pragma unroll
         for (int h2 = 0; h2 < 2; ++h2) {
@@ -3372,11 +3737,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
             }
         }
         delta = groups_sum(part);                                 // dO . O of member c, this head
-        const size_t at = (size_t)max(t.member.x, 0) * Hs + t.head;
-        lse_c = lse[at];
-        if constexpr (!PDS) {
-            if (g == 0 && t.part == 0 && t.member.x >= 0) stat[at] = make_float2(lse_c, delta);
-        }
+        lse_c = lse[(size_t)max(t.member.x, 0) * Hs + t.head];
     }
     floatx4v acc[4];
 #pragma unroll
@@ -3384,53 +3745,43 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
     struct Blk {
         uint2 kc[4], vc[4];                                       // columns 4 c .. 4 c + 3 of the K / V rows of entries 4 g + r
         int mk[4];                                                // bit c of mk[r]: the pair (entry 4 g + r, member c) exists
-        uint32_t pos[PDS ? 4 : 1];
-        int xe[DROP || BIAS == 1 ? 4 : 1];
-        float bz[BIAS ? 4 : 1];
+        uint32_t pos[4];
+        int xe[DROP ? 4 : 1];
     };
     for (int p0 = t.p_begin; p0 < t.p_end; p0 += TILE_CHUNK) {
         const int cnt = min(TILE_CHUNK, t.p_end - p0), nblk = (cnt + TILE_R - 1) / TILE_R;
         if (p0 != t.p_begin) tile_ask_entries(P, p0, cnt, t.lane, er);
         tile_put_entries(er, ent, cnt, t.lane, fst);
         auto issue = [&](Blk &B, int b) {
-            if constexpr (DROP || BIAS == 1) tile_pair_eids(P, p0 + TILE_R * b + 4 * g, t.p_end, c, B.xe);
+            if constexpr (DROP) tile_pair_eids(P, p0 + TILE_R * b + 4 * g, t.p_end, c, B.xe);
             const int4 e01 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g]);
             const int4 e23 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g + 2]);
             const int idxv[4] = {e01.x, e01.z, e23.x, e23.z};
             B.mk[0] = e01.y; B.mk[1] = e01.w; B.mk[2] = e23.y; B.mk[3] = e23.w;
-            if constexpr (PDS) {
-                const int4 f4 = *reinterpret_cast<const int4 *>(&fst[TILE_R * b + 4 * g]);
-                B.pos[0] = tile_pair_number(f4.x, e01.y, c); B.pos[1] = tile_pair_number(f4.y, e01.w, c);
-                B.pos[2] = tile_pair_number(f4.z, e23.y, c); B.pos[3] = tile_pair_number(f4.w, e23.w, c);
-            }
+            const int4 f4 = *reinterpret_cast<const int4 *>(&fst[TILE_R * b + 4 * g]);
+            B.pos[0] = tile_pair_number(f4.x, e01.y, c); B.pos[1] = tile_pair_number(f4.y, e01.w, c);
+            B.pos[2] = tile_pair_number(f4.z, e23.y, c); B.pos[3] = tile_pair_number(f4.w, e23.w, c);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) B.kc[r] = tile_row4_bf16<NARROW>(kb + ((uint32_t)idxv[r] * RB + offc));
+            for (int r = 0; r < 4; ++r) B.kc[r] = tile_row4_bf16<true>(kb + ((uint32_t)idxv[r] * RB + offc));
 #pragma unroll
-            for (int r = 0; r < 4; ++r) B.vc[r] = tile_row4_bf16<NARROW>(vb + ((uint32_t)idxv[r] * RB + offc));
-            if constexpr (BIAS) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) B.bz[r] = bias[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], B.pos[PDS ? r : 0])];
-            }
+            for (int r = 0; r < 4; ++r) B.vc[r] = tile_row4_bf16<true>(vb + ((uint32_t)idxv[r] * RB + offc));
         };
         auto compute = [&](const Blk &B) {
             Bf8 kr[2];
-            tile_rows_to_operand_bf16<NARROW>(kt, B.kc, c, g, kr, nw);
+            tile_rows_to_operand_bf16(kt, B.kc, c, g, kr, nw);
             const floatx4v st = tile_dot_bf16(kr, qb);
-            tile_rows_to_operand_bf16<NARROW>(kt, B.vc, c, g, kr, nw);
+            tile_rows_to_operand_bf16(kt, B.vc, c, g, kr, nw);
             const floatx4v dp = tile_dot_bf16(kr, dob);
             float ds[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                float pe = where_pair_or_zero(B.mk[r], c, __builtin_amdgcn_exp2f((BIAS ? st[r] + B.bz[BIAS ? r : 0] : st[r]) * scale_log2e - lse_c));
+                float pe = where_pair_or_zero(B.mk[r], c, __builtin_amdgcn_exp2f(st[r] * scale_log2e - lse_c));
                 float mt = 1.f;                                   // dropout multiplier of this pair (as in the forward)
                 if constexpr (DROP)
                     mt = dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)Hs + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
                 ds[r] = pe * (dp[r] * mt - delta) * scale;
                 pe *= mt;                                         // what multiplies v (forward) and dO (dV)
-                if (PDS && ((B.mk[r] >> c) & 1)) {
-                    pds_h[B.pos[PDS ? r : 0]] = pack_bf16(pe, ds[r]);
-                    if constexpr (BIAS) ds_out[tile_bias_at<H, BIAS>(P, t.head, B.xe[BIAS == 1 ? r : 0], B.pos[PDS ? r : 0])] = ds[r];   // dL/d(score before scaling)
-                }
+                if ((B.mk[r] >> c) & 1) pds_h[B.pos[r]] = pack_bf16(pe, ds[r]);
             }
             Bf4 da;
             da.u[0] = pack_bf16(ds[0], ds[1]);
@@ -3443,9 +3794,9 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
     if constexpr (SP > 1) {
         tile_park(piece[t.wv], acc, t.lane);
         __syncthreads();
-        tile_meet_and_store<SP, H, D, NARROW>(piece[t.wv % (HW / SP)], (HW / SP) * PIECE, t, dq, ws_dq, nw);
+        tile_meet_and_store<SP, H, D, true>(piece[t.wv % (HW / SP)], (HW / SP) * PIECE, t, dq, ws_dq, nw);
     } else {
-        tile_store_rows<H, D, false, NARROW>(t, acc, 1.f, dq, ws_dq, nw);
+        tile_store_rows<H, D, false, true>(t, acc, 1.f, dq, ws_dq, nw);
     }
 }
 
@@ -3547,8 +3898,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
 // Both backward kernels together at 8 heads: L = 8192, k = 4 60.8 -> 57.0 us; L = 4096, k = 32 64.7 -> 48.7; window 128 39.7 ->
 // 30.9; L = 32768, k = 2 235 -> 221; 32-graph batch 102.5 -> 99.2; L = 512 and L = 8192 with dropout level.  (6 heads of 50
 // columns with dropout lost 2 %: heads of fewer than 64 columns keep the scratch.)  float32 keeps it too: there the two
-// products are 1024 cycles of the matrix pipeline per block.  118 registers: compiled for four wavefronts per SIMD (for five,
-// with the members' rows in LDS or not, it spills: 658 us; four with them in LDS 316; q rows a block ahead spills too: 346).
+// products are 1024 cycles of the matrix pipeline per block.  122 registers: compiled for four wavefronts per SIMD.
 template <int H, int D, int HW, int WPE, bool DROP, int SP = 1>
 __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))) void k_attn_bwd_src_tile_bf16_again(
     bpt_plan P, const bf16_t *__restrict__ q, const bf16_t *__restrict__ k, const bf16_t *__restrict__ v, const bf16_t *__restrict__ d_o,
@@ -3559,30 +3909,38 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
     TileCtx t;
     if (!tile_begin<bf16_t, H, D, HW, false, SP>(P, t, nw)) return;
     // a wavefront's piece: its entry list, the rows being turned, the entries' (lse, delta); afterwards (SP > 1) what it has summed up
-    constexpr int ENT = TILE_CHUNK * 2, LIVE = ENT + TILE_KT_FLOATS_BF16 + 2 * TILE_R, PIECE = SP > 1 ? 2 * TILE_PART_FLOATS : LIVE;
-    static_assert(PIECE >= LIVE, "the lists fit");
+    constexpr int ENT = TILE_CHUNK * 2, ROWS = 2 * TILE_ROWS_FLOATS_BF16 + 4 * TILE_R, LIVE = ENT + ROWS + 2 * TILE_R, PIECE = SP > 1 ? 2 * TILE_PART_FLOATS : LIVE;
+    static_assert(PIECE >= LIVE && ROWS >= TILE_R * TILE_TURN_STRIDE, "the lists and the turned sums fit");
     __shared__ __attribute__((aligned(16))) float piece[HW][PIECE];
     int2 *ent = reinterpret_cast<int2 *>(piece[t.wv]);
-    char *kt = reinterpret_cast<char *>(piece[t.wv] + ENT);
-    float2 *const st_lds = reinterpret_cast<float2 *>(piece[t.wv] + ENT + TILE_KT_FLOATS_BF16);
+    char *const q_lds = reinterpret_cast<char *>(piece[t.wv] + ENT), *const d_lds = q_lds + 4 * TILE_ROWS_FLOATS_BF16;
+    float2 *const st_lds = reinterpret_cast<float2 *>(piece[t.wv] + ENT + ROWS);
     TileEntryRegs er;
     if (t.p_end > t.p_begin) tile_ask_entries(P, t.p_begin, min(TILE_CHUNK, t.p_end - t.p_begin), t.lane, er);
     issue_loads_first();
     const int c = t.c, g = t.g;
-    const uint32_t offr = (uint32_t)((t.head * D + 16 * g) * 2), offc = t.offv;
     const char *qb = reinterpret_cast<const char *>(q), *db = reinterpret_cast<const char *>(d_o);
-    const size_t mrow = (size_t)max(t.member.x, 0) * RB + offr;
     const float2 *const stat_h = stat + t.head;
     Bf8 kb[2], vb[2];
-    tile_load_row_bf16<false>(reinterpret_cast<const char *>(k) + mrow, kb, g, nw);
-    tile_load_row_bf16<false>(reinterpret_cast<const char *>(v) + mrow, vb, g, nw);
+    {
+        uint32_t off[2];
+        uintx4v kr[2], vr[2];
+        tile_member_offsets<RB>(t, off);
+        tile_ask_rows_bf16(reinterpret_cast<const char *>(k), off, kr);
+        tile_ask_rows_bf16(reinterpret_cast<const char *>(v), off, vr);
+        tile_put_rows_bf16(q_lds, kr, t.lane);
+        tile_put_rows_bf16(d_lds, vr, t.lane);
+        wave_lds_fence();
+        tile_operand_bf16(q_lds, c, g, kb);
+        tile_operand_bf16(d_lds, c, g, vb);
+        wave_lds_fence();
+    }
     floatx4v ak[4], av[4];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) { ak[nb] = floatx4v{0.f, 0.f, 0.f, 0.f}; av[nb] = floatx4v{0.f, 0.f, 0.f, 0.f}; }
     struct Blk {
-        uint2 qr[4], dr[4];                                       // columns 4 c .. 4 c + 3 of the q / dO rows of entries 4 g + r
-        float2 ld;                                                // (lse, delta) of entry c
-        int mk[4];                                                // bit c of mk[r]: the pair (entry 4 g + r, member c) exists
+        uintx4v qr[2], dr[2];
+        float2 ld;                                                // (lse, delta) of entry c, in the first lane group
         int xe[DROP ? 4 : 1];
     };
     for (int p0 = t.p_begin; p0 < t.p_end; p0 += TILE_CHUNK) {
@@ -3591,45 +3949,55 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
         tile_put_entries(er, ent, cnt, t.lane);
         auto issue = [&](Blk &B, int b) {
             if constexpr (DROP) tile_pair_eids(P, p0 + TILE_R * b + 4 * g, t.p_end, c, B.xe);
-            const int4 e01 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g]);
-            const int4 e23 = *reinterpret_cast<const int4 *>(&ent[TILE_R * b + 4 * g + 2]);
-            const int idxv[4] = {e01.x, e01.z, e23.x, e23.z};
-            B.mk[0] = e01.y; B.mk[1] = e01.w; B.mk[2] = e23.y; B.mk[3] = e23.w;
-            B.ld = stat_h[(size_t)ent[TILE_R * b + c].x * H];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) B.qr[r] = tile_row4_bf16<false>(qb + ((uint32_t)idxv[r] * RB + offc));
-#pragma unroll
-            for (int r = 0; r < 4; ++r) B.dr[r] = tile_row4_bf16<false>(db + ((uint32_t)idxv[r] * RB + offc));
+            if (g == 0) B.ld = stat_h[(size_t)ent[TILE_R * b + c].x * H];
+            uint32_t off[2];
+            tile_entry_offsets<RB>(t, ent + TILE_R * b, off);
+            tile_ask_rows_bf16(qb, off, B.qr);
+            tile_ask_rows_bf16(db, off, B.dr);
         };
-        auto compute = [&](const Blk &B) {
+        Blk B;
+        issue(B, 0);
+        for (int b = 0; b < nblk; ++b) {
+            int mk[4], xe[DROP ? 4 : 1];
+            tile_masks(ent + TILE_R * b, g, mk);
+#pragma unroll
+            for (int r = 0; r < (DROP ? 4 : 0); ++r) xe[r] = B.xe[r];
+            tile_put_rows_bf16(q_lds, B.qr, t.lane);
+            tile_put_rows_bf16(d_lds, B.dr, t.lane);
             if (g == 0) st_lds[c] = B.ld;
+            wave_lds_fence();
+            if (b + 1 < nblk) issue(B, b + 1);
+            issue_loads_first();
             Bf8 row[2];
-            tile_rows_to_operand_bf16<false>(kt, B.qr, c, g, row, nw);
+            tile_operand_bf16(q_lds, c, g, row);
+            const floatx4v st = tile_dot_bf16(row, kb);
             const floatx4v l01 = *reinterpret_cast<const floatx4v *>(&st_lds[4 * g]), l23 = *reinterpret_cast<const floatx4v *>(&st_lds[4 * g + 2]);
             const float lse_e[4] = {l01[0], l01[2], l23[0], l23[2]}, delta_e[4] = {l01[1], l01[3], l23[1], l23[3]};
-            const floatx4v st = tile_dot_bf16(row, kb);
-            tile_rows_to_operand_bf16<false>(kt, B.dr, c, g, row, nw);
+            tile_operand_bf16(d_lds, c, g, row);
             const floatx4v dp = tile_dot_bf16(row, vb);
             float pe[4], ds[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float p = where_pair_or_zero(B.mk[r], c, __builtin_amdgcn_exp2f(st[r] * scale_log2e - lse_e[r]));
+                const float p = where_pair_or_zero(mk[r], c, __builtin_amdgcn_exp2f(st[r] * scale_log2e - lse_e[r]));
                 float mt = 1.f;                                   // dropout multiplier of this pair (as in the forward)
                 if constexpr (DROP)
-                    mt = dropout_keep((uint32_t)B.xe[DROP ? r : 0] * (uint32_t)H + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
-                ds[r] = where_pair_or_zero(B.mk[r], c, p * (dp[r] * mt - delta_e[r]) * scale);
+                    mt = dropout_keep((uint32_t)xe[DROP ? r : 0] * (uint32_t)H + (uint32_t)t.head, drop_seed, drop_thr, drop_inv);
+                ds[r] = where_pair_or_zero(mk[r], c, p * (dp[r] * mt - delta_e[r]) * scale);
                 pe[r] = p * mt;
             }
             Bf4 pa, da;
             da.u[0] = pack_bf16(ds[0], ds[1]); da.u[1] = pack_bf16(ds[2], ds[3]);
             pa.u[0] = pack_bf16(pe[0], pe[1]); pa.u[1] = pack_bf16(pe[2], pe[3]);
-            tile_axpy_bf16(da, B.qr, ak);
-            tile_axpy_bf16(pa, B.dr, av);
-        };
-        tile_walk<Blk>(nblk, issue, compute);
-        wave_lds_fence();
+            tile_axpy_rows_bf16(da, q_lds, c, g, ak);
+            tile_axpy_rows_bf16(pa, d_lds, c, g, av);
+            wave_lds_fence();                                     // (read before the next block's are written)
+            issue_loads_first();
+        }
     }
+    float *const turn = reinterpret_cast<float *>(q_lds);
     if constexpr (SP > 1) {
+        tile_sums_by_row(turn, ak, c, g);
+        tile_sums_by_row(turn, av, c, g);
         constexpr int NEXT = (HW / SP) * PIECE;
         tile_park(piece[t.wv], ak, t.lane);
         tile_park(piece[t.wv] + TILE_PART_FLOATS, av, t.lane);
@@ -3638,8 +4006,8 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(WPE))
         tile_meet_and_store<SP, H, D, false>(part0, NEXT, t, dk, ws_dk, nw);
         tile_meet_and_store<SP, H, D, false>(part0 + TILE_PART_FLOATS, NEXT, t, dv, ws_dv, nw);
     } else {
-        tile_store_rows<H, D, false, false>(t, ak, 1.f, dk, ws_dk, nw);
-        tile_store_rows<H, D, false, false>(t, av, 1.f, dv, ws_dv, nw);
+        tile_store_sums<H, D>(t, turn, ak, dk, ws_dk);
+        tile_store_sums<H, D>(t, turn, av, dv, ws_dv);
     }
 }
 
@@ -5323,9 +5691,9 @@ int run_attn_fwd(const bpt_plan *P, const void *q, const void *k, const void *v,
                 constexpr int HW = H >= 4 ? 4 : H;
                 const int parts = tile_parts(P, H, sizeof(T));
 #define LAUNCH_FWD_TILE_PARTS(DR, BI, SP)                                                                                                \
-    hipLaunchKernelGGL((k_attn_fwd_tile_bf16<H, D, HW, TILE_BF16_WPE, DR, BI, false, SP>), dim3(group_grid(P) * (H * SP / HW)), \
+    hipLaunchKernelGGL((k_attn_fwd_rows_bf16<H, D, HW, TILE_BF16_WPE, DR, BI, SP>), dim3(group_grid(P) * (H * SP / HW)), \
                        dim3(HW * WAVE), 0, s, *P, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (bf16_t *)o, lse, ws_acc, ws_ml, \
-                       scale * LOG2E, drop.thr, drop.seed, drop.inv, bias, Narrow{}, Keep{})
+                       scale * LOG2E, drop.thr, drop.seed, drop.inv, bias)
 #define LAUNCH_FWD_TILE(DR, BI)                                                                                                          \
     do {                                                                                                                                 \
         if (parts == 4) LAUNCH_FWD_TILE_PARTS(DR, BI, 4);                                                                                \
@@ -5463,10 +5831,10 @@ int run_attn_bwd(const bpt_plan *Pin, const bpt_plan *Pout, const void *q, const
                 ProfScope prof(BPT_KERNEL_ATTN_BWD_DST, s);
                 const int parts = tile_parts(Pin, H, sizeof(T));
 #define LAUNCH_DST_TILE_PARTS(DR, BI, PD, SP)                                                                                            \
-    hipLaunchKernelGGL((k_attn_bwd_dst_tile_bf16<H, D, HW, TILE_BF16_WPE_DST, DR, BI, PD, false, SP>),                       \
+    hipLaunchKernelGGL((k_attn_bwd_dst_rows_bf16<H, D, HW, TILE_BF16_WPE_DST, DR, BI, PD, SP>),                              \
                        dim3(group_grid(Pin) * (H * SP / HW)), dim3(HW * WAVE), 0, s, *Pin, (const bf16_t *)q, (const bf16_t *)k, (const bf16_t *)v, (const bf16_t *)o,             \
                        (const bf16_t *)d_o, lse, (bf16_t *)dq, (uint32_t *)ws, (float2 *)ws, ws_rows, scale, scale * LOG2E, drop.thr,       \
-                       drop.seed, drop.inv, bias, ds_out, Narrow{})
+                       drop.seed, drop.inv, bias, ds_out)
 #define LAUNCH_DST_TILE(DR, BI, PD)                                                                                                      \
     do {                                                                                                                                 \
         if (parts == 4) LAUNCH_DST_TILE_PARTS(DR, BI, PD, 4);                                                                            \
@@ -5606,9 +5974,9 @@ int run_attn_fwd_narrow(const bpt_plan *P, const void *q, const void *k, const v
             hipLaunchKernelGGL((k_attn_fwd_tile<T, 16, 64, HW, DR, 0, true, SP>), grid, block, 0, s, *P, (const T *)q, (const T *)k,         \
                                (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed, drop.inv, (const float *)nullptr, np, keep); \
         else                                                                                                                             \
-            hipLaunchKernelGGL((k_attn_fwd_tile_bf16<16, 64, HW, TILE_BF16_WPE, DR, 0, true, SP>), grid, block, 0, s, *P,                    \
+            hipLaunchKernelGGL((k_attn_fwd_tile_bf16<16, 64, HW, TILE_BF16_WPE, DR, SP>), grid, block, 0, s, *P,                             \
                                (const T *)q, (const T *)k, (const T *)v, (T *)o, lse, ws_acc, ws_ml, scale * LOG2E, drop.thr, drop.seed,       \
-                               drop.inv, (const float *)nullptr, np, keep);                                                                \
+                               drop.inv, np, keep);                                                                                        \
     } while (0)
 #define LAUNCH_FWD(DR)                                                                                                                   \
     do {                                                                                                                                 \
@@ -5648,9 +6016,9 @@ int run_attn_bwd_narrow(const bpt_plan *Pin, const bpt_plan *Pout, const void *q
                                (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pds, ws_dq, scale, scale * LOG2E,       \
                                drop.thr, drop.seed, drop.inv, (const float *)nullptr, (float *)nullptr, np);                                \
         else                                                                                                                             \
-            hipLaunchKernelGGL((k_attn_bwd_dst_tile_bf16<16, 64, HW, TILE_BF16_WPE_DST, DR, 0, true, true, SP>), grid, block, 0, s, *Pin,    \
-                               (const T *)q, (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pds, (float2 *)nullptr, ws_dq, \
-                               scale, scale * LOG2E, drop.thr, drop.seed, drop.inv, (const float *)nullptr, (float *)nullptr, np);          \
+            hipLaunchKernelGGL((k_attn_bwd_dst_tile_bf16<16, 64, HW, TILE_BF16_WPE_DST, DR, SP>), grid, block, 0, s, *Pin,                   \
+                               (const T *)q, (const T *)k, (const T *)v, (const T *)o, (const T *)d_o, lse, (T *)dq, pds, ws_dq, \
+                               scale, scale * LOG2E, drop.thr, drop.seed, drop.inv, np);          \
     } while (0)
 #define LAUNCH_DST(DR)                                                                                                                   \
     do {                                                                                                                                 \
