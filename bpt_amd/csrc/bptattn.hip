@@ -2402,6 +2402,18 @@ __device__ __forceinline__ void tile_rows_to_operand(float *kt, const float4 (&r
     wave_lds_fence();                                             // (read before the next block's rows are written)
 }
 
+// The members' rows likewise: lane (c, g) asks for columns 4 c .. 4 c + 3 of the row of member 4 g + r, and tile_rows_to_operand gives lane c
+// the row of member c: 16 cycles of the texture addresser a load instead of 64.  Destination side, 32-graph batch 102.8 -> 99.7 us, 6 x 50 with
+// dropout 90.9 -> 87.4 and its forward 97.9 -> 96.4, L = 8192, k = 4 level.  (The forward that asks for its K rows a block ahead has no
+// registers for it: asked for with the entries and turned behind the first K rows, it spills: 32.8 -> 38.0 and 67 -> 75.)
+template <bool NARROW, typename T>
+__device__ __forceinline__ void tile_ask_members(const TileCtx &t, const T *base, uint32_t RB, float4 (&rows)[4]) {
+    const int row = max(t.member.x, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+        rows[r] = tile_row4<NARROW>(reinterpret_cast<const char *>(base) + ((uint32_t)lane_bcast(row, 4 * t.g + r) * RB + t.offv));
+}
+
 // Block after block, a block's loads ahead of its products.  Forms measured at L = 8192, k = 4 (1217 tiles of 4 blocks) and
 // dropped: the rows of the next block loaded while one is used (a two-stage register pipeline: 47 us against 44, a wavefront
 // per SIMD fewer; on few, tall tiles it was the better form until the parts of a tile came to be walked side by side, see
@@ -2490,7 +2502,11 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
     // (with the score term the sixteen registers are not there; with dropout they just are, and it does not pay: L = 8192 level, 6 x 50
     // with dropout 97.7 -> 100 us)
     constexpr bool AHEAD = !DROP && BIAS == 0;
-    if constexpr (!AHEAD) tile_load16<NARROW>(qrow, qb, g, nw);
+    if constexpr (!AHEAD) {
+        float4 qr[4];
+        tile_ask_members<NARROW>(t, q, RB, qr);
+        tile_rows_to_operand<NARROW>(kt, qr, c, g, qb, nw);
+    }
     floatx4v acc[4];
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) acc[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
@@ -2668,9 +2684,13 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(DROP 
         }
     } else {
         float ob[16], dob[16];
-        tile_load16<NARROW>(reinterpret_cast<const char *>(q) + mrow, qb, g, nw);
-        tile_load16<NARROW>(reinterpret_cast<const char *>(d_o) + mrow, dob, g, nw);
-        tile_load16<NARROW>(reinterpret_cast<const char *>(o) + mrow, ob, g, nw);
+        float4 qr[4], dr[4], orow[4];
+        tile_ask_members<NARROW>(t, d_o, RB, dr);
+        tile_ask_members<NARROW>(t, o, RB, orow);
+        tile_ask_members<NARROW>(t, q, RB, qr);
+        tile_rows_to_operand<NARROW>(kt, dr, c, g, dob, nw);
+        tile_rows_to_operand<NARROW>(kt, orow, c, g, ob, nw);
+        tile_rows_to_operand<NARROW>(kt, qr, c, g, qb, nw);
         float part = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) part = fmaf(dob[i], ob[i], part);
