@@ -3240,7 +3240,7 @@ constexpr int TILE_KT_FLOATS_BF16 = TILE_R * TILE_KT_BYTES_BF16 / 4;
 //
 // What bounds the bfloat16 kernels is the texture addresser, which takes a vector memory instruction four lanes at a time: 16 cycles
 // for one whose neighbouring lanes read on in a line, whatever a lane reads of it, 64 where each lane's line is another
-// (busy 77 % of all three kernels at 16 heads, L = 32768, k = 8).  Rows of eight bytes a lane took twice the instructions, members' rows
+// (by that count 614 k of the source side's 750 k cycles at 16 heads, L = 32768, k = 8; 250 k now).  Rows of eight bytes a lane took twice the instructions, members' rows
 // read row by lane four times the cycles, (lse, delta) of a block's entries read by all 64 lanes as many as its rows.  So: rows, members'
 // rows and results in 16 bytes a lane, along the rows; single words of a row by one lane group.  Nothing else helped the source side there:
 // its rows a block ahead through LDS but 8 bytes a lane 333 -> 343 us; 16 bytes a lane 315; the members and (lse, delta) too 303;
