@@ -575,10 +575,9 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_fwd_heads(bpt_plan P, const T
     }
     s = head_reduce<acc_t, 1, false>(s, H, h, (acc_t *)nullptr);
     if (seg_slot >= 0) {
-        // a segment of a split row: y gets exp(x - m) of the segment; its (m, s) go to the workspace, from which
-        // k_softmax_seg_rows forms the factor exp(m - M) / S that k_softmax_seg_scale applies
+        // a segment of a split row: only its (m, s); k_softmax_seg_rows forms the row's of them and k_softmax_fwd_seg_finish writes y
         if (slot == 0) { seg[((size_t)seg_slot * H + h) * 2] = m; seg[((size_t)seg_slot * H + h) * 2 + 1] = s; }
-        s = 1;
+        return;
     }
     if (cached) {
 #pragma unroll
@@ -658,9 +657,9 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_bwd_heads(bpt_plan P, const T
     }
 }
 
-// Split rows of the softmax, second step: one block per split row.  Forward (PAIR): the segments' (m_i, s_i) become the
-// factors exp(m_i - M) / S with M = max(-1e9, m_i), S = sum s_i exp(m_i - M) (stored over m_i); backward: the segments'
-// partial sums are replaced by their total.  A lane handles head l % H of every n-th slot.
+// Split rows of the softmax, second step: one block per split row.  Forward (PAIR): the segments' (m_i, s_i) are replaced by the
+// row's, M = max(-1e9, m_i) and S = sum s_i exp(m_i - M); backward: the segments' partial sums are replaced by their total.  A
+// lane handles head l % H of every n-th slot.
 template <typename A, bool PAIR>
 __global__ __launch_bounds__(BLOCK) void k_softmax_seg_rows(const int32_t *__restrict__ heavy, A *__restrict__ seg, int H) {
     __shared__ A smem[WAVES_PER_BLOCK * WAVE];
@@ -676,7 +675,8 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_seg_rows(const int32_t *__res
         s = head_reduce<A, WAVES_PER_BLOCK, false>(s, H, h, smem);
         for (int j = j0; j < ns; j += nj) {
             A *q = seg + ((size_t)(s0 + j) * H + h) * ST;
-            q[0] = exp_acc(q[0] - m) / s;
+            q[0] = m;
+            q[1] = s;
         }
     } else {
         A s = 0;
@@ -686,18 +686,20 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_seg_rows(const int32_t *__res
     }
 }
 
-// third step, one wavefront per item, segments only.  Forward: y *= factor of the segment.
+// Third step, one wavefront per item, segments only.  Forward: x is read again and y = exp(x - M) / S, rounded once, as for a whole row (a
+// segment's exp(x - m) kept in y and scaled here would be rounded twice: bfloat16 results off by 7.5e-3 instead of 3.8e-3).
 template <typename T>
-__global__ __launch_bounds__(BLOCK) void k_softmax_seg_scale(bpt_plan P, T *__restrict__ y, int H, const typename Elem<T>::acc_t *__restrict__ seg) {
+__global__ __launch_bounds__(BLOCK) void k_softmax_fwd_seg_finish(bpt_plan P, const T *__restrict__ x, T *__restrict__ y, int H,
+                                                                  const typename Elem<T>::acc_t *__restrict__ seg) {
     using acc_t = typename Elem<T>::acc_t;
     Item it;
     if (!fetch_item(P, it) || it.slot < 0) return;
     const int tid = threadIdx.x & 63, h = tid % H, nslots = WAVE / H;
     if (tid / H >= nslots) return;
-    const acc_t f = seg[((size_t)it.slot * H + h) * 2];
+    const acc_t m = seg[((size_t)it.slot * H + h) * 2], s = seg[((size_t)it.slot * H + h) * 2 + 1];
     for (int p = it.begin + tid / H; p < it.end; p += nslots) {
         const size_t o = (size_t)P.eid[p] * H + h;
-        Elem<T>::st(y + o, (acc_t)Elem<T>::ld(y + o) * f);
+        Elem<T>::st(y + o, exp_acc((acc_t)Elem<T>::ld(x + o) - m) / s);
     }
 }
 
@@ -5080,7 +5082,7 @@ int run_softmax_fwd(const bpt_plan *P, const void *x, void *y, void *ws, int h, 
         hipLaunchKernelGGL((k_softmax_seg_rows<acc_t, true>), dim3((int)P->n_heavy), dim3(BLOCK), 0, s, P->heavy, seg, h);
         st = launch_status();
         if (st != BPT_OK) return st;
-        hipLaunchKernelGGL((k_softmax_seg_scale<T>), dim3(grid_for(P)), dim3(BLOCK), 0, s, *P, (T *)y, h, (const acc_t *)seg);
+        hipLaunchKernelGGL((k_softmax_fwd_seg_finish<T>), dim3(grid_for(P)), dim3(BLOCK), 0, s, *P, (const T *)x, (T *)y, h, (const acc_t *)seg);
         return launch_status();
     }
     hipLaunchKernelGGL((k_softmax_fwd<T, 1>), dim3(grid_for(P)), dim3(BLOCK), 0, s, *P, (const T *)x, (T *)y, h);

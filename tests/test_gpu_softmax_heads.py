@@ -28,8 +28,6 @@ def test_softmax_of_any_number_of_heads(h, dtype, seg, monkeypatch):
     want_dx = yh * (dy.double() - dot[dst])
     # exp and division to some ulp, sums of 5000 terms; bfloat16: one rounding of the result
     tol = {torch.float32: 3e-6, torch.bfloat16: 2 ** -8, torch.float64: 1e-13}[dtype]
-    if dtype == torch.bfloat16:
-        tol *= 2                                                  # (segments of split rows are stored, and rounded, before they are scaled)
     assert ((yh - want).abs() <= tol * (want.abs() + 1e-7)).all()
     bound = tol * (want_dx.abs() + yh * (dy.double().abs() + dot[dst].abs() + 1))
     assert ((dx.cpu().double() - want_dx).abs() <= bound).all()
