@@ -5555,14 +5555,38 @@ bool product_tiles_ok(const bpt_plan *P, int h, int d, int dtype) {
 }
 inline Narrow product_narrow(int h, int d) { return Narrow{d, h, product_tile_heads(h), (h + NARROW_HW - 1) / NARROW_HW}; }
 
+// How many heads of a workgroup access an edge's record together where one wavefront walks a tile (1: each its own), for node tensors and an
+// edge tensor that start on 16 bytes or not (two heads: the edge tensor on 8).
+inline bool product_whole_heads(int h, int d, bool nodes16) { return d == 64 && nodes16 && (h == 4 || h == 8 || h == 16); }
+inline int shared_heads(int h, int d, bool nodes16, bool edges16, bool edges8 = true) {
+    if (product_whole_heads(h, d, nodes16)) return edges16 ? 4 : 1;
+    return h % NARROW_HW == 0 && edges8 ? NARROW_HW : 1;
+}
+
+// Over how many wavefronts a tile and head of the separate operators is spread (shared: as shared_heads says).  Parts have blocks of their
+// own, so in parts every head goes to the edge tensor by itself: what tile_parts measured on the attention kernels holds for heads that do
+// so anyway, and only for them.  SDDMM + SpMM, out- and in-side added up, one part -> two -> four:
+//   four heads together: 1032 wavefronts of 9 blocks (8 x 64, window of 128, L = 2048)  54 -> 51 -> 48 us;   1084 of 5 (4 x 64, L = 2048, k = 8)  37 -> 34 -> 32
+//     1088 of 3 (8 x 64, L = 1024, k = 4)  26 -> 26 -> 27;   1448 of 3  30 -> 31 -> 34;   2056 of 9 (8 x 64, window of 128, L = 4096)  68 -> 79 -> 82;
+//     2064 of 9 (16 x 64)  68 -> 93 -> 97;   4112 of 9 (8 x 64, L = 8192)  95 -> 134 -> 140;   8080 of 13 (8 x 64, window of 256)  218 -> 292 -> 287
+//   two together: 1032 of 9 (8 x 40)  62 -> 51 -> 49;   1104 of 3 (6 x 50, L = 1400)  33 -> 29 -> 30;   1626 of 5 (6 x 50, L = 2048, k = 8)  48 -> 42 -> 43;
+//     2056 of 9 (8 x 40)  72 -> 78 -> 82;   2168 of 5  52 -> 50 -> 52;   3078 of 9 (6 x 50)  89 -> 96 -> 96
+//   each by itself: 1285 of 9 (5 x 30)  64 -> 52 -> 49;   2570 of 9  92 -> 80 -> 82;   5050 of 13  173 -> 156 -> 156;   5840 of 4  75 -> 77 -> 86
+inline int product_parts(const bpt_plan *P, int heads, int shared) {
+    if (shared == 1) return tile_parts(P, heads, 4);
+    const int64_t wavefronts = P->n_groups * heads;
+    if (wavefronts <= 768 || (wavefronts <= 1152 && P->n_grp_entries / TILE_R >= 4 * P->n_groups)) return 4;
+    return shared == 2 && wavefronts <= 1792 ? 2 : 1;
+}
+
 template <int H>
 int run_spmm_tile(const bpt_plan *P, const float *W, const float *X, float *Y, float *ws, hipStream_t s) {
-    const int parts = tile_parts(P, H, 4);
+    const int shared = aligned16(W) ? 4 : 1, parts = product_parts(P, H, shared);
 #define LAUNCH(SH, SP) \
     hipLaunchKernelGGL((k_spmm_tile<H, 64, 4, SH, false, SP>), dim3(group_grid(P) * (H * SP / 4)), dim3(4 * WAVE), 0, s, *P, W, X, Y, ws, Narrow{})
     if (parts == 4) LAUNCH(false, 4);
     else if (parts == 2) LAUNCH(false, 2);
-    else if (aligned16(W)) LAUNCH(true, 1);
+    else if (shared == 4) LAUNCH(true, 1);
     else LAUNCH(false, 1);
 #undef LAUNCH
     const int st = launch_status();
@@ -5574,18 +5598,19 @@ int run_spmm_tile(const bpt_plan *P, const float *W, const float *X, float *Y, f
 int spmm_tile(const bpt_plan *P, const void *W_, const void *X_, void *Y_, void *ws_, int h, int d, hipStream_t s) {
     const float *W = (const float *)W_, *X = (const float *)X_;
     float *Y = (float *)Y_, *ws = (float *)ws_;
-    if (d == 64 && aligned16(X) && aligned16(Y)) {
+    const bool nodes16 = aligned16(X) && aligned16(Y);
+    if (product_whole_heads(h, d, nodes16)) {
         if (h == 4) return run_spmm_tile<4>(P, W, X, Y, ws, s);
         if (h == 8) return run_spmm_tile<8>(P, W, X, Y, ws, s);
         if (h == 16) return run_spmm_tile<16>(P, W, X, Y, ws, s);
     }
-    const int parts = tile_parts(P, h, 4);
+    const int shared = shared_heads(h, d, nodes16, aligned16(W), (reinterpret_cast<uintptr_t>(W) & 7u) == 0), parts = product_parts(P, h, shared);
     const Narrow nw = narrow_parts(product_narrow(h, d), parts);
 #define LAUNCH(HW, SH, SP) \
     hipLaunchKernelGGL((k_spmm_tile<16, 64, HW, SH, true, SP>), dim3(group_grid(P) * nw.slices), dim3(HW * WAVE), 0, s, *P, W, X, Y, ws, nw)
     if (parts == 4) LAUNCH(4, false, 4);
     else if (parts == 2) LAUNCH(2, false, 2);
-    else if (h % NARROW_HW == 0 && (reinterpret_cast<uintptr_t>(W) & 7u) == 0) LAUNCH(NARROW_HW, true, 1);
+    else if (shared == NARROW_HW) LAUNCH(NARROW_HW, true, 1);
     else LAUNCH(NARROW_HW, false, 1);
 #undef LAUNCH
     const int st = launch_status();
@@ -5597,12 +5622,12 @@ int spmm_tile(const bpt_plan *P, const void *W_, const void *X_, void *Y_, void 
 
 template <int H>
 int run_sddmm_tile(const bpt_plan *P, const float *A, const float *B, float *y, hipStream_t s) {
-    const int parts = tile_parts(P, H, 4);
+    const int shared = aligned16(y) ? 4 : 1, parts = product_parts(P, H, shared);
 #define LAUNCH(SH, SP) \
     hipLaunchKernelGGL((k_sddmm_tile<H, 64, 4, SH, false, SP>), dim3(group_grid(P) * (H * SP / 4)), dim3(4 * WAVE), 0, s, *P, A, B, y, Narrow{})
     if (parts == 4) LAUNCH(false, 4);
     else if (parts == 2) LAUNCH(false, 2);
-    else if (aligned16(y)) LAUNCH(true, 1);
+    else if (shared == 4) LAUNCH(true, 1);
     else LAUNCH(false, 1);
 #undef LAUNCH
     return launch_status();
@@ -5610,18 +5635,19 @@ int run_sddmm_tile(const bpt_plan *P, const float *A, const float *B, float *y, 
 int sddmm_tile(const bpt_plan *P, const void *A_, const void *B_, void *y_, int h, int d, hipStream_t s) {
     const float *A = (const float *)A_, *B = (const float *)B_;
     float *y = (float *)y_;
-    if (d == 64 && aligned16(A) && aligned16(B)) {
+    const bool nodes16 = aligned16(A) && aligned16(B);
+    if (product_whole_heads(h, d, nodes16)) {
         if (h == 4) return run_sddmm_tile<4>(P, A, B, y, s);
         if (h == 8) return run_sddmm_tile<8>(P, A, B, y, s);
         if (h == 16) return run_sddmm_tile<16>(P, A, B, y, s);
     }
-    const int parts = tile_parts(P, h, 4);
+    const int shared = shared_heads(h, d, nodes16, aligned16(y), (reinterpret_cast<uintptr_t>(y) & 7u) == 0), parts = product_parts(P, h, shared);
     const Narrow nw = narrow_parts(product_narrow(h, d), parts);
 #define LAUNCH(HW, SH, SP) \
     hipLaunchKernelGGL((k_sddmm_tile<16, 64, HW, SH, true, SP>), dim3(group_grid(P) * nw.slices), dim3(HW * WAVE), 0, s, *P, A, B, y, nw)
     if (parts == 4) LAUNCH(4, false, 4);
     else if (parts == 2) LAUNCH(2, false, 2);
-    else if (h % NARROW_HW == 0 && (reinterpret_cast<uintptr_t>(y) & 7u) == 0) LAUNCH(NARROW_HW, true, 1);
+    else if (shared == NARROW_HW) LAUNCH(NARROW_HW, true, 1);
     else LAUNCH(NARROW_HW, false, 1);
 #undef LAUNCH
     return launch_status();
@@ -6198,6 +6224,13 @@ int bpt_wavefronts_per_item(const bpt_plan *plan, int kernel, int h, int d, int 
     const size_t elem = dtype == BPT_F32 ? 4 : 2;
     if (has_tiles(plan, h, d, elem)) return tile_parts(plan, h, elem, kernel == BPT_KERNEL_ATTN_FWD);
     return row_parts(plan, h * d, kernel == BPT_KERNEL_ATTN_FWD && dtype == BPT_F32);
+}
+
+int bpt_wavefronts_per_product(const bpt_plan *plan, int h, int d) {
+    if (!plan) return BPT_ERR_NULL;
+    if (h < 1 || d < 1) return BPT_ERR_SHAPE;
+    if (!product_tiles_ok(plan, h, d, BPT_F32)) return 0;
+    return product_parts(plan, h, shared_heads(h, d, true, true));
 }
 
 int bpt_profile_kernel(int which, void *start_event, void *stop_event) {

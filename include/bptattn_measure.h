@@ -29,6 +29,10 @@ int bpt_profile_kernel(int which, void *start_event, void *stop_event);
  * sizes that the launch makes for a layer without dropout and score term.  For tests of that choice; negative: bpt_status. */
 int bpt_wavefronts_per_item(const bpt_plan *plan, int kernel, int h, int d, int dtype);
 
+/* The same for the separate operators in float32 on a plan that carries tiles (0: they do not take them), for tensors that start on
+ * 16 bytes. */
+int bpt_wavefronts_per_product(const bpt_plan *plan, int h, int d);
+
 /* Measurement aid (no counterpart in the reference): launches a kernel in which waves_per_cu wavefronts per compute unit
  * (a multiple of 4, at most 64) each read `iters` batches of in_flight (2, 4 or 8) pseudo-random 1 KB rows of `region`
  * (region_bytes of device memory, 16-byte aligned), the access pattern of the attention kernels' neighbour-row gathers.

@@ -248,3 +248,35 @@ def test_wavefronts_of_a_tile_and_head():
         # bfloat16
         assert [parts(n, 1, kernel, dtype=BF16) for n in (75, 76, 150, 151)] == [4, 2, 2, 1]
         assert [parts(n, 8, kernel, dtype=BF16) for n in (150, 151, 288, 289)] == [2, 2, 2, 1]
+
+
+def test_wavefronts_of_a_tile_and_head_of_the_separate_operators():
+    """Heads that access the edge tensor together lose that in parts: they take them only where a launch leaves SIMDs idle.  Heads that
+    go to it one by one follow the attention kernels' rule."""
+    lib = _lib.attn_lib()
+
+    def plan_of(n_groups, blocks):
+        p = _lib.PlanStruct()
+        p.n_rows = p.n_items = p.n_index_nodes = 16 * n_groups
+        p.n_edges = 16 * 16 * n_groups * blocks
+        p.grp_R, p.n_groups, p.grp_max_chunk, p.n_grp_entries = 16, n_groups, n_groups, 16 * n_groups * blocks
+        p.grp_members = p.grp_ptr = p.grp_entries = p.grp_chunks = p.grp_eids = 16          # (looked at for null only)
+        return p
+
+    def parts(n_groups, blocks, h, d):
+        return lib.bpt_wavefronts_per_product(ctypes.byref(plan_of(n_groups, blocks)), h, d)
+
+    for h in (4, 8, 16):
+        few, some = 768 // h, 1152 // h
+        assert [parts(n, 3, h, 64) for n in (1, few, few + 1, some)] == [4, 4, 1, 1]
+        assert [parts(n, 4, h, 64) for n in (few + 1, some, some + 1, 4 * some)] == [4, 4, 1, 1]
+    for h, d in ((6, 50), (8, 40), (2, 64), (16, 63)):
+        assert [parts(n, 3, h, d) for n in (768 // h, 768 // h + 1, 1792 // h, 1792 // h + 1)] == [4, 2, 2, 1]
+        assert [parts(n, 9, h, d) for n in (1152 // h, 1152 // h + 1, 1792 // h, 1792 // h + 1)] == [4, 2, 2, 1]
+    for h, d in ((5, 30), (1, 64), (7, 63)):
+        for n, blocks in ((1, 9), (200, 9), (800, 4), (1000, 9), (5000, 9)):
+            p = plan_of(n, blocks)
+            assert parts(n, blocks, h, d) == lib.bpt_wavefronts_per_item(ctypes.byref(p), DST, h, 64, F32)
+    assert parts(8, 4, 17, 64) == parts(8, 4, 8, 65) == parts(8, 4, 8, 3) == 0
+    assert lib.bpt_wavefronts_per_product(ctypes.byref(_lib.PlanStruct()), 8, 64) == 0
+    assert lib.bpt_wavefronts_per_product(ctypes.byref(_lib.PlanStruct()), 0, 64) < 0 and lib.bpt_wavefronts_per_product(None, 8, 64) < 0
