@@ -511,7 +511,8 @@ struct MaskedMM : torch::autograd::Function<MaskedMM> {
         auto r = masked_mm_backward_known(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], dy);
         if (!r)
             r = with_python([&] {
-                const auto two = python("maskedmm_csr_backward")(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], dy)
+                const auto two = python("maskedmm_csr_backward")(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], dy,
+                                                                       py::arg("_native_call") = true)
                                      .template cast<std::vector<Tensor>>();
                 return Two{two[0], two[1]};
             });
@@ -524,7 +525,7 @@ struct MaskedMM : torch::autograd::Function<MaskedMM> {
 struct EdgeSoftmax : torch::autograd::Function<EdgeSoftmax> {
     static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &row, const Tensor &indptr, const Tensor &eid, const Tensor &x) {
         auto y = softmax_known(row, indptr, eid, x, nullptr);
-        if (!y) y = python("sparse_softmax_forward")(row, indptr, eid, x).cast<Tensor>();
+        if (!y) y = python("sparse_softmax_forward")(row, indptr, eid, x, py::arg("_native_call") = true).cast<Tensor>();
         ctx->save_for_backward({row, indptr, eid, *y});
         return *y;
     }
@@ -532,7 +533,10 @@ struct EdgeSoftmax : torch::autograd::Function<EdgeSoftmax> {
         const auto t = ctx->get_saved_variables();
         const Tensor dy = grads[0].contiguous();
         auto dx = softmax_known(t[0], t[1], t[2], t[3], &dy);
-        if (!dx) dx = with_python([&] { return python("sparse_softmax_backward")(t[0], t[1], t[2], t[3], dy).template cast<Tensor>(); });
+        if (!dx)
+            dx = with_python([&] {
+                return python("sparse_softmax_backward")(t[0], t[1], t[2], t[3], dy, py::arg("_native_call") = true).template cast<Tensor>();
+            });
         return {Tensor(), Tensor(), Tensor(), *dx};
     }
 };
@@ -542,7 +546,7 @@ struct VecSpmm : torch::autograd::Function<VecSpmm> {
                           const Tensor &col, const Tensor &indptr_t, const Tensor &eid_t, const Tensor &indices_t, const Tensor &w, const Tensor &x) {
         ctx->save_for_backward({row, indptr, eid, indices, col, indptr_t, eid_t, indices_t, w, x});
         auto y = vec_spmm_known(row, indptr, eid, indices, w, x);
-        if (!y) y = python("vector_spmm_forward")(row, indptr, eid, indices, w, x).cast<Tensor>();
+        if (!y) y = python("vector_spmm_forward")(row, indptr, eid, indices, w, x, py::arg("_native_call") = true).cast<Tensor>();
         return *y;
     }
     static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
@@ -551,7 +555,8 @@ struct VecSpmm : torch::autograd::Function<VecSpmm> {
         auto r = vec_spmm_backward_known(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], dy, t[9]);
         if (!r)
             r = with_python([&] {
-                const auto two = python("vector_spmm_backward")(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], dy, t[9])
+                const auto two = python("vector_spmm_backward")(t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], dy, t[9],
+                                                                       py::arg("_native_call") = true)
                                      .template cast<std::vector<Tensor>>();
                 return Two{two[0], two[1]};
             });
@@ -575,7 +580,7 @@ Tensor masked_mm(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r,
 Tensor sparse_softmax(const Tensor &row, const Tensor &indptr, const Tensor &eid, const Tensor &x) {
     if (differentiated({&x})) return EdgeSoftmax::apply(row, indptr, eid, x);
     auto y = softmax_known(row, indptr, eid, x, nullptr);
-    if (!y) y = python("sparse_softmax_forward")(row, indptr, eid, x).cast<Tensor>();
+    if (!y) y = python("sparse_softmax_forward")(row, indptr, eid, x, py::arg("_native_call") = true).cast<Tensor>();
     return *y;
 }
 
@@ -583,7 +588,7 @@ Tensor vec_spmm(const Tensor &row, const Tensor &indptr, const Tensor &eid, cons
                 const Tensor &eid_t, const Tensor &indices_t, const Tensor &w, const Tensor &x) {
     if (differentiated({&w, &x})) return VecSpmm::apply(row, indptr, eid, indices, col, indptr_t, eid_t, indices_t, w, x);
     auto y = vec_spmm_known(row, indptr, eid, indices, w, x);
-    if (!y) y = python("vector_spmm_forward")(row, indptr, eid, indices, w, x).cast<Tensor>();
+    if (!y) y = python("vector_spmm_forward")(row, indptr, eid, indices, w, x, py::arg("_native_call") = true).cast<Tensor>();
     return *y;
 }
 

@@ -172,7 +172,8 @@ def _workspace(op, plan, plan_t, h, d, dt, device, plan_ref=None, plan_t_ref=Non
 # from the capture's own pool as before.  release_workspaces() gives the memory back.
 # Fused attention without a score term keeps none: from its second call on a graph it is served by the native host path, which
 # asks the allocator (the same block comes back call after call), and what the first call had left here would lie idle beside it
-# (422 MB at L = 32768, k = 8, 16 heads in float32).
+# (422 MB at L = 32768, k = 8, 16 heads in float32).  Nor do the separate operators on behalf of that path (_native_call), for calls that it
+# is going to serve.
 _SCRATCH = {}
 _SCRATCH_LOCK = threading.Lock()
 KEEP_WORKSPACES = True
@@ -230,9 +231,15 @@ def prepare_products(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indi
                                (row, indptr_r, eid_r, indices_r, n, n, seg, _plan.tile_order_src(n, eid_r.numel()))])
 
 
+def _native_next(plans):
+    """Whether the native host path takes over a call of one of the separate operators from the next one on: it takes plans that cover every
+    edge.  (Of rows of heads, (n, h, d) and (E, h), between as many rows.)"""
+    return all(p.covers_all_edges and p.n_edges > 0 for p in plans)
+
+
 def _remember_op(plans, generation, kind, index, numbers, struct, struct_t=None):
-    """Leaves the choice of one of the separate operators to the native host path, which takes plans that cover every edge."""
-    if all(p.covers_all_edges and p.n_edges > 0 for p in plans):
+    """Leaves the choice of one of the separate operators to the native host path."""
+    if _native_next(plans):
         plan_cache.remember(plans, generation, kind, index, numbers, ctypes.addressof(struct), 0 if struct_t is None else ctypes.addressof(struct_t))
 
 
@@ -278,7 +285,7 @@ def maskedmm_csr_forward(row, indptr, eid, indices, A, B):
     return y
 
 
-def maskedmm_csr_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, A, B, dy):
+def maskedmm_csr_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, A, B, dy, *, _native_call=False):
     """[dA, dB] (graphop.cpp:108-139, graphop_kernel.cu:355-409)."""
     generation, cfg = _native.generation(), _SETTINGS
     _check_all(row=row, indptr_r=indptr_r, eid_r=eid_r, indices_r=indices_r, col=col, indptr_c=indptr_c,
@@ -296,7 +303,8 @@ def maskedmm_csr_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c,
     dA, dB = torch.empty_like(A), torch.empty_like(B)
     dt = _dtype(A)
     ref_r, ref_c = ctypes.byref(struct_r), ctypes.byref(struct_c)
-    ws, nws = _workspace(OP_MASKEDMM_BWD, plan_r, plan_c, h, d, dt, A.device, plan_ref=ref_r, plan_t_ref=ref_c)
+    ws, nws = _workspace(OP_MASKEDMM_BWD, plan_r, plan_c, h, d, dt, A.device, plan_ref=ref_r, plan_t_ref=ref_c,
+                         keep=not (_native_call and A.dim() == 3 and _native_next((plan_r, plan_c))))
     with _on_device_of(A):
         check_attn(_LIB.bpt_maskedmm_csr_backward(ref_r, ref_c, _ptr(A), _ptr(B), _ptr(dy), _ptr(dA), _ptr(dB),
                                                   _ptr(ws), nws, h, d, dt, _stream()), "maskedmm_csr_backward")
@@ -342,7 +350,7 @@ def node_mul_edge_backward(row, indptr, eid, A, B, dy):
     return [dA, dB]
 
 
-def sparse_softmax_forward(row, indptr, eid, x):
+def sparse_softmax_forward(row, indptr, eid, x, *, _native_call=False):
     """softmax of x over the slots of each row (graphop.cpp:59-71, graphop_kernel.cu:411-463)."""
     generation = _native.generation()
     _check_all(row=row, indptr=indptr, eid=eid, x=x)
@@ -351,7 +359,8 @@ def sparse_softmax_forward(row, indptr, eid, x):
         raise ValueError(f"x must be ({eid.size(0)},) or ({eid.size(0)}, h), got {tuple(x.shape)}")
     plan = plan_cache.get(row, indptr, eid, None, None, None, prefer_device=True)
     y = (torch.empty_like if plan.covers_all_edges else torch.zeros_like)(x)
-    ws, nws = _workspace(OP_SOFTMAX_FWD, plan, None, _edge_h(x), 1, _dtype(x), x.device)
+    ws, nws = _workspace(OP_SOFTMAX_FWD, plan, None, _edge_h(x), 1, _dtype(x), x.device,
+                         keep=not (_native_call and x.dim() == 2 and _native_next((plan,))))
     with _on_device_of(x):
         check_attn(_LIB.bpt_sparse_softmax_forward(plan.ref, _ptr(x), _ptr(y), _ptr(ws), nws, _edge_h(x), _dtype(x), _stream()),
                    "sparse_softmax_forward")
@@ -360,7 +369,7 @@ def sparse_softmax_forward(row, indptr, eid, x):
     return y
 
 
-def sparse_softmax_backward(row, indptr, eid, y, dy):
+def sparse_softmax_backward(row, indptr, eid, y, dy, *, _native_call=False):
     """dx = y * (dy - sum_row dy*y) (graphop.cpp:163-177, graphop_kernel.cu:465-507)."""
     generation = _native.generation()
     _check_all(row=row, indptr=indptr, eid=eid, y=y, dy=dy)
@@ -371,7 +380,8 @@ def sparse_softmax_backward(row, indptr, eid, y, dy):
     _expect_shape(dy, y.shape, "dy")
     plan = plan_cache.get(row, indptr, eid, None, None, None, prefer_device=True)
     dx = (torch.empty_like if plan.covers_all_edges else torch.zeros_like)(dy)
-    ws, nws = _workspace(OP_SOFTMAX_BWD, plan, None, _edge_h(dy), 1, _dtype(y), y.device)
+    ws, nws = _workspace(OP_SOFTMAX_BWD, plan, None, _edge_h(dy), 1, _dtype(y), y.device,
+                         keep=not (_native_call and y.dim() == 2 and _native_next((plan,))))
     with _on_device_of(y):
         check_attn(_LIB.bpt_sparse_softmax_backward(plan.ref, _ptr(y), _ptr(dy), _ptr(dx), _ptr(ws), nws, _edge_h(dy), _dtype(y),
                                                     _stream()),
@@ -381,7 +391,7 @@ def sparse_softmax_backward(row, indptr, eid, y, dy):
     return dx
 
 
-def vector_spmm_forward(row, indptr, eid, indices, edata, x, *, n_rows=None, out=None):
+def vector_spmm_forward(row, indptr, eid, indices, edata, x, *, n_rows=None, out=None, _native_call=False):
     """y[row] = sum_p edata[eid[p]] * x[indices[p]] (graphop.cpp:79-95, graphop_kernel.cu:509-542).
 
     n_rows (keyword only, not in the reference): number of rows of y when it differs from x.size(0) — a
@@ -402,7 +412,9 @@ def vector_spmm_forward(row, indptr, eid, indices, edata, x, *, n_rows=None, out
         plan = plan_cache.get(row, indptr, eid, indices, n_out, x.size(0))
     y = torch.empty_like(x) if n_rows is None else torch.empty((n_out,) + tuple(x.shape[1:]), dtype=x.dtype, device=x.device)
     dt = _dtype(x)
-    ws, nws = _workspace(OP_SPMM_FWD, plan, None, h, d, dt, x.device, plan_ref=ctypes.byref(struct) if square else None)
+    known_next = square and x.dim() == 3 and edata.dim() == 2
+    ws, nws = _workspace(OP_SPMM_FWD, plan, None, h, d, dt, x.device, plan_ref=ctypes.byref(struct) if square else None,
+                         keep=not (_native_call and known_next and _native_next((plan,))))
     if out is not None and (out.shape != y.shape or out.dtype != y.dtype or out.device != y.device or not out.is_contiguous()):
         raise ValueError("out must be a contiguous tensor of the result's shape, dtype and device")
     with _on_device_of(x):
@@ -417,12 +429,12 @@ def vector_spmm_forward(row, indptr, eid, indices, edata, x, *, n_rows=None, out
                 check_attn(st, "vector_spmm_accumulate")
         check_attn(_LIB.bpt_vector_spmm_forward(ref, _ptr(edata), _ptr(x), _ptr(y), _ptr(ws), nws, h, d, dt, _stream()),
                    "vector_spmm_forward")
-    if square and x.dim() == 3 and edata.dim() == 2:
+    if known_next:
         _remember_op((plan,), generation, _native.SPMM_FWD, [row, indptr, eid, indices], [x.size(0), h, d, dt], struct)
     return y if out is None else out.add_(y)
 
 
-def vector_spmm_backward(row, indptr, eid, indices, col, indptr_t, eid_t, indices_t, edata, dy, x):
+def vector_spmm_backward(row, indptr, eid, indices, col, indptr_t, eid_t, indices_t, edata, dy, x, *, _native_call=False):
     """[dedata, dx] (graphop.cpp:190-214, graphop_kernel.cu:544-600; dx over all units of the transposed side)."""
     generation, cfg = _native.generation(), _SETTINGS
     _check_all(row=row, indptr=indptr, eid=eid, indices=indices, col=col, indptr_t=indptr_t, eid_t=eid_t,
@@ -443,7 +455,8 @@ def vector_spmm_backward(row, indptr, eid, indices, col, indptr_t, eid_t, indice
     dt = _dtype(x)
     ref, ref_t = ctypes.byref(struct), ctypes.byref(struct_t)
     square = x.dim() == 3 and dy.size(0) == x.size(0) and edata.dim() == 2
-    ws, nws = _workspace(OP_SPMM_BWD, plan, plan_t, h, d, dt, x.device, plan_ref=ref, plan_t_ref=ref_t)
+    ws, nws = _workspace(OP_SPMM_BWD, plan, plan_t, h, d, dt, x.device, plan_ref=ref, plan_t_ref=ref_t,
+                         keep=not (_native_call and square and _native_next((plan, plan_t))))
     with _on_device_of(x):
         check_attn(_LIB.bpt_vector_spmm_backward(ref, ref_t, _ptr(edata), _ptr(dy), _ptr(x), _ptr(dedata), _ptr(dx),
                                                  _ptr(ws), nws, h, d, dt, _stream()), "vector_spmm_backward")
