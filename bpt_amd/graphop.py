@@ -227,8 +227,10 @@ def prepare_products(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indi
     if A.dim() != 3 or not _product_tiles(eid_r.numel(), n, B.size(0), A, A.size(1), A.size(2), cfg):
         return
     seg = _tile_seg_of(eid_r.numel(), n, n)
-    plan_cache.put_tile_plans([(col, indptr_c, eid_c, indices_c, n, n, seg, None),
-                               (row, indptr_r, eid_r, indices_r, n, n, seg, _plan.tile_order_src(n, eid_r.numel()))])
+    sides = [(col, indptr_c, eid_c, indices_c, n, n, seg, None),
+             (row, indptr_r, eid_r, indices_r, n, n, seg, _plan.tile_order_src(n, eid_r.numel()))]
+    if plan_cache.may_hold(sides):       # (the operator that asks for the other plan is another call: only the cache can hand it on)
+        plan_cache.put_tile_plans(sides)
 
 
 def _native_next(plans):

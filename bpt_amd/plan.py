@@ -836,6 +836,13 @@ class PlanCache:
             self._evict()
         return plan
 
+    def may_hold(self, sides):
+        """False if the tile plans of these sides (as put_tile_plans takes them) cannot stand here together: by their number, or by
+        the bytes that they hold at the least (row pointers, neighbours and edge ids, the groups' edge ids twice, their entries)."""
+        at_least = sum(4 * side[4] + 17 * side[2].numel() for side in sides)
+        with self._lock:
+            return len(sides) <= self._cap and at_least <= self._max_bytes
+
     def put_tile_plans(self, sides):
         """What get() would build one after the other for a training step on tiles, built together (DevicePlan.tile_plans; sides as
         there: the in-side, then the out-side), unless one of them is already here or they have to be built one by one.  A side that is

@@ -105,3 +105,23 @@ def test_first_calls_leave_no_workspace_behind():
     graphop.release_workspaces()
     graphop.vector_spmm_forward(*s.inn, rand((s.E, 6), 5), x[0].detach())      # nor has a caller of the function itself
     assert graphop._SCRATCH
+
+
+@pytest.mark.parametrize("limits", [dict(capacity=1), dict(max_bytes=0), dict(max_bytes=1 << 18)])
+def test_a_cache_too_small_for_both_sides_builds_neither_for_nothing(limits):
+    from bpt_amd import op, plan
+    s = sides("bpt512")
+    x = [rand((s.n, 8, 64), i).requires_grad_(True) for i in (1, 2, 3)]
+    calls = (op.masked_mm, op.sparse_softmax, op.vec_spmm)
+    plan.plan_cache.clear()
+    want = chain(calls, s, *x)
+    old = plan.plan_cache.set_limits(**limits)
+    try:
+        plan.plan_cache.clear()
+        built = plan.plan_cache.misses
+        got = chain(calls, s, *x)
+        assert plan.plan_cache.misses == built + 3                # one for each operator
+    finally:
+        plan.plan_cache.set_limits(*old)
+        plan.plan_cache.clear()
+    assert torch.equal(got, want)
