@@ -256,8 +256,8 @@ def _product_plan(row, indptr, eid, indices, n_rows, n_index_nodes, x, h, d, cfg
     if indices is not None and _product_tiles(eid.numel(), n_rows, n_index_nodes, x, h, d, cfg):
         plan = plan_cache.get(row, indptr, eid, indices, n_rows, n_index_nodes, seg_len=_tile_seg_of(eid.numel(), n_rows, n_index_nodes),
                               prefer_device=True, groups=(TILE_ROWS, order))
-        if plan.covers_all_edges:
-            return plan, plan.ensure_groups(TILE_ROWS, order)["struct"]
+        # (tiles are formed where a plan covers every edge; one that does not is walked row by row, as it is)
+        return plan, plan.ensure_groups(TILE_ROWS, order)["struct"] if plan.covers_all_edges else plan.struct
     plan = plan_cache.get(row, indptr, eid, indices, n_rows, n_index_nodes)
     return plan, _spmm_struct(plan, x, h, d, cfg)
 

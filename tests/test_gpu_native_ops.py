@@ -125,3 +125,31 @@ def test_a_cache_too_small_for_both_sides_builds_neither_for_nothing(limits):
         plan.plan_cache.set_limits(*old)
         plan.plan_cache.clear()
     assert torch.equal(got, want)
+
+
+def test_a_plan_that_does_not_cover_every_edge_is_built_once():
+    """Two slots with one edge id: the operators on tiles do not take such a graph."""
+    from bpt_amd import op, plan
+    from test_gpu_product_tiles import product_ok, sum_ok
+    s = sides("bpt512")
+
+    def twice(side):
+        row, indptr, eid, indices = side
+        eid = eid.clone()
+        eid[eid == 1] = 0
+        return row, indptr, eid, indices
+
+    out, inn = twice(s.out), twice(s.inn)
+    k, q, w = rand((s.n, 8, 64), 1), rand((s.n, 8, 64), 2), rand((s.E, 8), 3)
+    one_weight = w.clone()
+    one_weight[1] = w[0]
+    distinct = torch.arange(s.E, device=DEV) > 1                  # (edge 0 is written by two slots, edge 1 by none)
+    for grad in (False, True):
+        plan.plan_cache.clear()
+        built = plan.plan_cache.misses
+        e = op.masked_mm(*out, *inn, k.requires_grad_(grad), q)
+        assert product_ok(e[distinct], k[s.src[distinct]], q[s.dst[distinct]]) and not e[1].any()
+        assert sum_ok(op.vec_spmm(*inn, *out, w, k), s.dst, one_weight, k.detach()[s.src], s.n)
+        assert plan.plan_cache.misses == built + 2
+    dk, = torch.autograd.grad(e, k, w)
+    assert sum_ok(dk, s.src, one_weight, q[s.dst], s.n)
