@@ -213,7 +213,26 @@ def _product_tiles(n_edges, n_rows, n_index_nodes, x, h, d, cfg):
     """Whether a SpMM- or SDDMM-shaped op takes the tile kernels if its plan covers every edge (_product_plan says why)."""
     return (cfg.use_groups and cfg.grouped_ops and cfg.use_tiles and cfg.group_rows is None and not _FORCE_GENERIC and x.dim() == 3
             and x.dtype == torch.float32 and 4 <= d <= 64 and h <= 16 and n_edges > 0 and n_rows == n_index_nodes
-            and n_rows * h * d * 4 < 2 ** 32 and n_edges * h < 2 ** 32)
+            and n_rows * h * d * 4 < 2 ** 32 and n_edges * h < 2 ** 32 and not (d == 32 and h == 8 and n_rows >= 24576))
+
+
+def _worth_tiles(struct, x):
+    """Whether the tiles at hand are worth it for a shape that has row-group kernels of its own: a tile's block costs the same whatever is in
+    it, so that sixteen rows have to share their neighbours.  Heads that no other specialised kernel has always are (2 to 29 times as fast as
+    the general kernels on BPT graphs, windows and random graphs).  Both products on both sides, row groups / tiles, by pairs an entry (1: no two of
+    a tile's rows share a neighbour; BPT graphs 3 to 11, windows up to 14), 24 random neighbours a row out of a window around it:
+      8 x 64, 8192 rows   1.24 pairs 0.67, 1.5 0.79, 2.0 0.96;  16 384 rows  1.05 0.98, 1.25 0.83, 1.5 1.16, 2.0 1.44;  40 000 rows  1.05 0.90, 1.25 0.92, 1.5 1.04
+      4 x 64              0.75, 0.86, 1.09;                     1.01, 1.09, 1.40, 1.75;                                 0.92, 1.34, 1.46
+      16 x 64             0.81, 0.92, 1.11;                     1.00, 1.13, 1.34, 1.70;                                 0.96, 1.08, 1.22
+      8 x 32              0.50, 0.57, 0.70;                     0.69, 0.67, 0.82, 1.02;                                 0.70, 0.66, 0.74
+    2048 rows are as 8192, and 2.7 pairs 2.0, 1.8, 1.4, 1.5.  8 x 32, of which a lane group's loads are half padding, wins on small graphs (BPT,
+    L = 512 2.0 to 2.5, L = 8192 1.02 to 1.10; window of 128 at L = 4096 1.6) and from 32 767 rows on loses whatever the graph (k = 1 ... 16
+    0.79 to 1.06): _product_tiles leaves those to the row groups without a look.  Few edges are level (512 rows with 4000 edges, 1.2 pairs
+    1.15, 1.10, 0.99, 1.02; 2048 with 10 000, 1.4 pairs 0.98, 1.13, 0.96, 0.88), and a new graph's row groups are built on the host."""
+    if struct.n_edges <= 10000 or not attention_supported(x):
+        return True
+    least = 2.5 if x.size(2) == 32 else 2.0 if struct.n_rows < 12288 else 1.4
+    return struct.n_edges >= least * struct.n_grp_entries
 
 
 def prepare_products(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, A, B):
@@ -247,7 +266,7 @@ def _remember_op(plans, generation, kind, index, numbers, struct, struct_t=None)
 
 def _product_plan(row, indptr, eid, indices, n_rows, n_index_nodes, x, h, d, cfg, order=None):
     """(plan, the struct to hand over) for a SpMM- or SDDMM-shaped op over one CSR side: tiles for float32 rows of 4 to 64
-    columns a head and up to 16 heads of a graph of one node set, built on the GPU, else _spmm_struct's choice.  Both products of
+    columns a head and up to 16 heads of a graph of one node set, built on the GPU, where _worth_tiles says so, else _spmm_struct's choice.  Both products of
     a tile's blocks go to the matrix cores, a row is loaded once per 16 rows instead of 8 or 4, and heads that no other
     specialised kernel has are read as they are: L = 8192, k = 4, 8 x 64, per launch 33 -> 22 to 27 us (comment at k_spmm_tile), and the plans of a
     new graph take 0.6 ms instead of the 22 of the host's row groups.  A SpMM into another number of rows stays with the row groups: the CSR
@@ -256,8 +275,11 @@ def _product_plan(row, indptr, eid, indices, n_rows, n_index_nodes, x, h, d, cfg
     if indices is not None and _product_tiles(eid.numel(), n_rows, n_index_nodes, x, h, d, cfg):
         plan = plan_cache.get(row, indptr, eid, indices, n_rows, n_index_nodes, seg_len=_tile_seg_of(eid.numel(), n_rows, n_index_nodes),
                               prefer_device=True, groups=(TILE_ROWS, order))
-        # (tiles are formed where a plan covers every edge; one that does not is walked row by row, as it is)
-        return plan, plan.ensure_groups(TILE_ROWS, order)["struct"] if plan.covers_all_edges else plan.struct
+        if not plan.covers_all_edges:                             # (no tiles then: it is walked row by row, as it is)
+            return plan, plan.struct
+        struct = plan.ensure_groups(TILE_ROWS, order)["struct"]
+        if _worth_tiles(struct, x):
+            return plan, struct
     plan = plan_cache.get(row, indptr, eid, indices, n_rows, n_index_nodes)
     return plan, _spmm_struct(plan, x, h, d, cfg)
 

@@ -110,3 +110,40 @@ def test_rows_that_are_not_finite_stay_with_their_neighbours(name, h, d):
         assert sum_ok(y[~bad], (torch.cumsum(~bad, 0) - 1)[to[keep]], W[keep], A[frm[keep]], int((~bad).sum()))
         e = G.maskedmm_csr_forward(*side, rand((s.n, h, d), 4), A)
         assert torch.equal(~torch.isfinite(e).all(1), (frm == 5) | (frm == 6))
+
+
+def in_a_window(n, E, width):                                     # sources from the `width` rows around a row
+    rng = np.random.default_rng(2)
+    dst = np.sort(rng.integers(0, n, E))
+    return ((dst + rng.integers(0, width, E)) % n).astype(np.int64), dst.astype(np.int64), n
+
+
+@pytest.mark.parametrize("graph,h,d,tiles", [((2048, 20000, 2048), 8, 64, False), ((2048, 20000, 2048), 8, 32, False), ((2048, 20000, 2048), 6, 50, True),
+                                             ((2048, 20000, 2048), 8, 30, True), ((2048, 40000, 60), 8, 64, True), ((2048, 40000, 60), 8, 32, True),
+                                             ((2048, 40000, 130), 8, 64, True), ((2048, 40000, 130), 8, 32, False), ((13000, 107000, 100), 4, 64, True),
+                                             ((11000, 90000, 100), 4, 64, False), ((2048, 10000, 2048), 8, 64, True), ((2048, 10001, 2048), 8, 64, False), ((25000, 25000 * 8, 8), 8, 32, False), ((25000, 25000 * 8, 8), 8, 64, True)])
+def test_tiles_where_rows_share_their_neighbours(graph, h, d, tiles):
+    """Shapes with row-group kernels of their own take those where the tiles' rows have few neighbours in common, and 8 x 32 on large
+    graphs; the others always take tiles."""
+    from bpt_amd import graphbuilder as gb, graphop as G, plan
+    src, dst, n = in_a_window(*graph)
+    out_csr, in_csr, ROW, IR, COL, IC = gb.get_csrs(src, dst, n)
+    out, inn = (tuple(t.to(DEV) for t in side) for side in ((ROW, IR, out_csr[2], out_csr[1]), (COL, IC, in_csr[2], in_csr[1])))
+    src, dst = torch.from_numpy(src).to(DEV), torch.from_numpy(dst).to(DEV)
+    A, B, W = rand((n, h, d), 1), rand((n, h, d), 2), rand((len(src), h), 3)
+    plan.plan_cache.clear()
+    for side, frm, to in ((out, dst, src), (inn, src, dst)):
+        assert sum_ok(G.vector_spmm_forward(*side, W, A), to, W, A[frm], n)
+        assert product_ok(G.maskedmm_csr_forward(*side, A, B), A[to], B[frm])
+    dA, dB = G.maskedmm_csr_backward(*out, *inn, A, B, W)
+    assert sum_ok(dA, src, W, B[dst], n) and sum_ok(dB, dst, W, A[src], n)
+    dW, dx = G.vector_spmm_backward(*inn, *out, W, B, A)
+    assert product_ok(dW, B[dst], A[src]) and sum_ok(dx, src, W, B[dst], n)
+    grouped = [R for p, _ in plan.plan_cache._d.values() for R, _ in p._groups]
+    assert (4 in grouped or 8 in grouped) != tiles
+    # bit for bit what the family computes that was chosen
+    old = G.set_tiles(tiles)
+    try:
+        assert torch.equal(dA, G.maskedmm_csr_backward(*out, *inn, A, B, W)[0])
+    finally:
+        G.set_tiles(old)
