@@ -34,7 +34,7 @@ def multigraph(n=97, E=3000):
     return src.astype(np.int64), dst.astype(np.int64), n
 
 
-GRAPHS = {"bpt512": lambda: bpt(512, 4, False), "bpt9000": lambda: bpt(9000, 1), "window": lambda: window(2000, 100), "multigraph": multigraph,
+GRAPHS = {"bpt512": lambda: bpt(512, 4, False), "bpt2000": lambda: bpt(2000, 1), "bpt9000": lambda: bpt(9000, 1), "window": lambda: window(2000, 100), "multigraph": multigraph,
           "one token": lambda: bpt(1, 1)}
 SHAPES = [(8, 64), (4, 64), (16, 64), (6, 50), (8, 40), (5, 30), (3, 4), (1, 64), (7, 63)]
 
@@ -110,6 +110,25 @@ def test_rows_that_are_not_finite_stay_with_their_neighbours(name, h, d):
         assert sum_ok(y[~bad], (torch.cumsum(~bad, 0) - 1)[to[keep]], W[keep], A[frm[keep]], int((~bad).sum()))
         e = G.maskedmm_csr_forward(*side, rand((s.n, h, d), 4), A)
         assert torch.equal(~torch.isfinite(e).all(1), (frm == 5) | (frm == 6))
+
+
+@pytest.mark.parametrize("h", [4, 8, 16])
+@pytest.mark.parametrize("name", ["bpt512", "bpt2000", "bpt9000", "multigraph"])
+def test_node_tensors_that_start_on_four_bytes(name, h):
+    """64 columns a head, which take the kernels of narrow heads then, on tiles in four, two and one parts, and split rows."""
+    from bpt_amd import graphop as G
+    s = sides(name)
+    off = lambda x: torch.cat([x.new_zeros(1), x.flatten()])[1:].view(x.shape)
+    A, B, W = off(rand((s.n, h, 64), 1)), off(rand((s.n, h, 64), 2)), rand((s.E, h), 3)
+    assert A.data_ptr() % 16 == B.data_ptr() % 16 == 4
+    for W in (W, off(W)):
+        for side, frm, to in ((s.out, s.dst, s.src), (s.inn, s.src, s.dst)):
+            assert sum_ok(G.vector_spmm_forward(*side, W, A), to, W, A[frm], s.n)
+            assert product_ok(G.maskedmm_csr_forward(*side, A, B), A[to], B[frm])
+        dA, dB = G.maskedmm_csr_backward(*s.out, *s.inn, A, B, W)
+        assert sum_ok(dA, s.src, W, B[s.dst], s.n) and sum_ok(dB, s.dst, W, A[s.src], s.n)
+        dW, dx = G.vector_spmm_backward(*s.inn, *s.out, W, B, A)
+        assert product_ok(dW, B[s.dst], A[s.src]) and sum_ok(dx, s.src, W, B[s.dst], s.n)
 
 
 def in_a_window(n, E, width):                                     # sources from the `width` rows around a row
