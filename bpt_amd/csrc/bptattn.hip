@@ -5565,18 +5565,24 @@ inline int shared_heads(int h, int d, bool nodes16, bool edges16, bool edges8 = 
 
 // Over how many wavefronts a tile and head of the separate operators is spread (shared: as shared_heads says).  Parts have blocks of their
 // own, so in parts every head goes to the edge tensor by itself: what tile_parts measured on the attention kernels holds for heads that do
-// so anyway, and only for them.  SDDMM + SpMM, out- and in-side added up, one part -> two -> four:
-//   four heads together: 1032 wavefronts of 9 blocks (8 x 64, window of 128, L = 2048)  54 -> 51 -> 48 us;   1084 of 5 (4 x 64, L = 2048, k = 8)  37 -> 34 -> 32
-//     1088 of 3 (8 x 64, L = 1024, k = 4)  26 -> 26 -> 27;   1448 of 3  30 -> 31 -> 34;   2056 of 9 (8 x 64, window of 128, L = 4096)  68 -> 79 -> 82;
-//     2064 of 9 (16 x 64)  68 -> 93 -> 97;   4112 of 9 (8 x 64, L = 8192)  95 -> 134 -> 140;   8080 of 13 (8 x 64, window of 256)  218 -> 292 -> 287
-//   two together: 1032 of 9 (8 x 40)  62 -> 51 -> 49;   1104 of 3 (6 x 50, L = 1400)  33 -> 29 -> 30;   1626 of 5 (6 x 50, L = 2048, k = 8)  48 -> 42 -> 43;
-//     2056 of 9 (8 x 40)  72 -> 78 -> 82;   2168 of 5  52 -> 50 -> 52;   3078 of 9 (6 x 50)  89 -> 96 -> 96
-//   each by itself: 1285 of 9 (5 x 30)  64 -> 52 -> 49;   2570 of 9  92 -> 80 -> 82;   5050 of 13  173 -> 156 -> 156;   5840 of 4  75 -> 77 -> 86
+// so anyway.  Heads that share take one part where a launch has wavefronts enough without parts.  SDDMM + SpMM of one side, one part ->
+// two -> four:
+//   four together, 8 x 64: 4112 wavefronts of 9 blocks (window of 128, L = 8192)  49 -> 70 -> 71 us;   3976 of 16 (window of 256, L = 4096)  66 -> 90 -> 86;
+//     8080 of 16  129 -> 172 -> 166;   4160 of 5 (L = 4096, k = 4, both ways)  32 -> 41 -> 44;   4448 of 8  46 -> 53 -> 56
+//     below, by how unequal a graph's tiles are: 2056 of 9 (window of 128)  31 -> 38 -> 40, 3288 of 18 (L = 3000, k = 16, both ways)  96 -> 86 -> 79,
+//     1576 of 15 (L = 1500)  81 -> 63 -> 43, 2352 of 21 (L = 2048, k = 32)  94 -> 81 -> 74
+//   16 x 64, whose edges' records are half a line: 2064 of 9 (window of 128, L = 2048)  37 -> 47 -> 49;   4112 of 9  47 -> 80 -> 85;   2176 of 3 (L = 1024,
+//     k = 4)  18 -> 20 -> 22;   3024 of 9 (L = 1500, k = 16, both ways)  49 -> 59 -> 60;   of more blocks 3152 of 15 there  92 -> 78 -> 76, 2368 of 17  71 -> 72 -> 77
+//   two together: 4112 of 9 (8 x 40, window of 128)  52 -> 69 -> 70;   3420 of 10 (6 x 50, L = 4096, k = 32)  52 -> 62 -> 58;   3336 of 8 (6 x 50, L = 4096, k = 4,
+//     both ways)  45 -> 43 -> 43;   3288 of 18  108 -> 87 -> 77;   2982 of 9 (window of 256)  49 -> 47 -> 45
+//   each by itself: 5050 of 13 (5 x 30, window of 256; both sides)  173 -> 156 -> 156
+// Of 304 pairs of launches (windows, BPT graphs one way and both, k up to 64) none is slower by it than by tile_parts and those from the line
+// on up to 1.9 times as fast.
 inline int product_parts(const bpt_plan *P, int heads, int shared) {
-    if (shared == 1) return tile_parts(P, heads, 4);
     const int64_t wavefronts = P->n_groups * heads;
-    if (wavefronts <= 768 || (wavefronts <= 1152 && P->n_grp_entries / TILE_R >= 4 * P->n_groups)) return 4;
-    return shared == 2 && wavefronts <= 1792 ? 2 : 1;
+    const bool half_lines = shared == 4 && heads == 16 && P->n_grp_entries < 12 * TILE_R * P->n_groups;
+    if (shared > 1 && wavefronts >= (half_lines ? 2050 : 3400)) return 1;
+    return tile_parts(P, heads, 4);
 }
 
 template <int H>

@@ -225,9 +225,9 @@ def _worth_tiles(struct, x):
       4 x 64              0.75, 0.86, 1.09;                     1.01, 1.09, 1.40, 1.75;                                 0.92, 1.34, 1.46
       16 x 64             0.81, 0.92, 1.11;                     1.00, 1.13, 1.34, 1.70;                                 0.96, 1.08, 1.22
       8 x 32              0.50, 0.57, 0.70;                     0.69, 0.67, 0.82, 1.02;                                 0.70, 0.66, 0.74
-    2048 rows are as 8192, and 2.7 pairs 2.0, 1.8, 1.4, 1.5.  8 x 32, of which a lane group's loads are half padding, wins on small graphs (BPT,
-    L = 512 2.0 to 2.5, L = 8192 1.02 to 1.10; window of 128 at L = 4096 1.6) and from 32 767 rows on loses whatever the graph (k = 1 ... 16
-    0.79 to 1.06): _product_tiles leaves those to the row groups without a look.  Few edges are level (512 rows with 4000 edges, 1.2 pairs
+    2048 rows are as 8192, and with 2.7 pairs 1.8, 2.0, 1.3, 1.5.  8 x 32, of which a lane group's loads are half padding, wins on small graphs (BPT,
+    L = 512 2.0 to 2.5, L = 8192 1.02 to 1.10; window of 128 at L = 4096 1.6) and from 32 767 rows on mostly loses (k = 1 ... 16 0.79
+    to 1.06, a window of 32 0.87): _product_tiles leaves those to the row groups without a look.  Few edges are level (512 rows with 4000 edges, 1.2 pairs
     1.15, 1.10, 0.99, 1.02; 2048 with 10 000, 1.4 pairs 0.98, 1.13, 0.96, 0.88), and a new graph's row groups are built on the host."""
     if struct.n_edges <= 10000 or not attention_supported(x):
         return True
@@ -237,7 +237,9 @@ def _worth_tiles(struct, x):
 
 def prepare_products(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, A, B):
     """Builds the two sides' tile plans together that masked_mm, vec_spmm and their backwards are going to ask for, where neither is in
-    the cache (a new graph).  A convenience, as prepare_training: what is not built here is built when it is asked for."""
+    the cache (a new graph).  A convenience, as prepare_training: what is not built here is built when it is asked for.  Without gradients
+    too, where masked_mm itself needs one side: the layer's vec_spmm asks for the other (first pass of the three operators forward, L = 512,
+    2048, 8192: 436, 449, 461 us against 576, 554, 623 built one by one; masked_mm by itself 238, 238, 286 against 219, 218, 260)."""
     cfg = _SETTINGS
     graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
     if any(t.dim() != 1 or t.dtype != torch.int64 or t.device != A.device or not t.is_contiguous() for t in graph) or not A.is_cuda:

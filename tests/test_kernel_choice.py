@@ -251,8 +251,8 @@ def test_wavefronts_of_a_tile_and_head():
 
 
 def test_wavefronts_of_a_tile_and_head_of_the_separate_operators():
-    """Heads that access the edge tensor together lose that in parts: they take them only where a launch leaves SIMDs idle.  Heads that
-    go to it one by one follow the attention kernels' rule."""
+    """Heads that access the edge tensor together lose that in parts: they take one where the launch has wavefronts enough without.  The
+    others, and smaller launches, follow the attention kernels' rule."""
     lib = _lib.attn_lib()
 
     def plan_of(n_groups, blocks):
@@ -266,17 +266,20 @@ def test_wavefronts_of_a_tile_and_head_of_the_separate_operators():
     def parts(n_groups, blocks, h, d):
         return lib.bpt_wavefronts_per_product(ctypes.byref(plan_of(n_groups, blocks)), h, d)
 
-    for h in (4, 8, 16):
-        few, some = 768 // h, 1152 // h
-        assert [parts(n, 3, h, 64) for n in (1, few, few + 1, some)] == [4, 4, 1, 1]
-        assert [parts(n, 4, h, 64) for n in (few + 1, some, some + 1, 4 * some)] == [4, 4, 1, 1]
-    for h, d in ((6, 50), (8, 40), (2, 64), (16, 63)):
-        assert [parts(n, 3, h, d) for n in (768 // h, 768 // h + 1, 1792 // h, 1792 // h + 1)] == [4, 2, 2, 1]
-        assert [parts(n, 9, h, d) for n in (1152 // h, 1152 // h + 1, 1792 // h, 1792 // h + 1)] == [4, 2, 2, 1]
+    def attention(n_groups, blocks, h):
+        return lib.bpt_wavefronts_per_item(ctypes.byref(plan_of(n_groups, blocks)), DST, h, 64, F32)
+
+    for h, d, first in ((4, 64, 850), (8, 64, 425), (6, 50, 567), (8, 40, 425), (2, 64, 1700), (16, 63, 213)):
+        for blocks in (3, 9, 20):
+            assert [parts(n, blocks, h, d) for n in (first, 2 * first, 9 * first)] == [1, 1, 1]
+            assert all(parts(n, blocks, h, d) == attention(n, blocks, h) for n in (1, 60, 100, first // 2, first - 1))
+    assert parts(424, 9, 8, 64) == parts(566, 9, 6, 50) == parts(849, 9, 4, 64) == 2
+    for blocks in (3, 9, 11):
+        assert parts(129, blocks, 16, 64) == 1 and parts(128, blocks, 16, 64) == attention(128, blocks, 16)
+    assert parts(128, 9, 16, 64) == 2 and parts(212, 12, 16, 64) == 2 and parts(213, 12, 16, 64) == 1
     for h, d in ((5, 30), (1, 64), (7, 63)):
         for n, blocks in ((1, 9), (200, 9), (800, 4), (1000, 9), (5000, 9)):
-            p = plan_of(n, blocks)
-            assert parts(n, blocks, h, d) == lib.bpt_wavefronts_per_item(ctypes.byref(p), DST, h, 64, F32)
+            assert parts(n, blocks, h, d) == attention(n, blocks, h)
     assert parts(8, 4, 17, 64) == parts(8, 4, 8, 65) == parts(8, 4, 8, 3) == 0
     assert lib.bpt_wavefronts_per_product(ctypes.byref(_lib.PlanStruct()), 8, 64) == 0
     assert lib.bpt_wavefronts_per_product(ctypes.byref(_lib.PlanStruct()), 0, 64) < 0 and lib.bpt_wavefronts_per_product(None, 8, 64) < 0
