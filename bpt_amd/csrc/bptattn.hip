@@ -501,7 +501,7 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_bwd(bpt_plan P, const T *__re
 // 64 / H whole (E, H) rows per step, for up to 64 heads; lanes past the last whole row have none.  One wavefront per item.  Rows of up
 // to SM_CACHE steps keep their values in registers and read memory once; longer rows re-read.  Loads are issued SM_CACHE at a time.
 // Heads that do not divide 64 ran the kernels above, a pass over the row for every head: 6 heads float32, L = 8192, k = 4, all launches,
-// forward 249 -> 34 us, backward 350 -> 39.
+// forward 249 -> 30 us, backward 350 -> 39.
 constexpr int SM_CACHE = 8;
 
 // reduction over the threads of a block that share a head, l % H: first inside each wavefront, then over LDS
@@ -2941,7 +2941,7 @@ __global__ __launch_bounds__(HW * WAVE) __attribute__((amdgpu_waves_per_eu(4))) 
 // itself: the texture addresser works through 64 places per instruction, four instructions a block and head.
 // 8 heads, per launch without merges, row groups of 8 -> each for itself -> shared: L = 8192, k = 4 SpMM 33.9 -> 31 -> 26.6 (out-CSR) and 33 ->
 // 27 -> 22.6 us (in-CSR), SDDMM 32.5 -> 27.7 -> 23.4 and 31.5 -> 28 -> 21.6; 32-graph batch SpMM 43 -> 40 -> 34, SDDMM 43 -> 41 -> 34;
-// window 128 SpMM 38 -> 17 to 23 -> 12 to 19, SDDMM 29 -> 19 to 23 -> 15 to 18.  What bounds them now: at L = 8192 the node rows read and
+// window 128 SpMM 38 -> 17 to 23 -> 12 to 19, SDDMM 29 -> 19 to 23 -> 15 to 18 (one wavefront a tile; product_parts says where).  What bounds them now: at L = 8192 the node rows read and
 // written by themselves are 13 us at the rate of a large copy, the products 7; the rest is the tiles' first loads and the edge tensor's places.
 template <int HW> struct HeadPack;
 template <> struct HeadPack<4> { typedef floatx4v vec; };
@@ -5513,17 +5513,18 @@ inline bool has_tiles(const bpt_plan *P, int h, int d, size_t elem) {
 //   8080 of 16 / 8072 of 9 (window of 256, L = 8192)    91.0 / 142 / 93.8  -> 93.2 / 140 / 85.0  -> 101 / 149 / 88.6
 //   8256 of 5 (window of 64, L = 16384)                 46.5 / 72.1 / 51.4 -> 49.6 / 72.2 / 50.1 -> 57.4 / 84.7 / 61.6
 // bfloat16, whose blocks are shorter against their headers:
-//   584 of 3 (L = 512)      5.8 / 6.6 / 8.1 -> 5.1 / 6.0 / 6.4 -> 5.0 / 6.4 / 5.5;    1048 of 3    6.6 / 7.5 / 8.5 -> 6.4 / 7.6 / 8.4 -> 6.9 / 9.2 / 9.1
-//   1032 of 9              11.4 / 12.9 / 12.0 -> 9.0 / 11.2 / 10.0 -> 8.3 / 10.1 / 10.4;  2056 of 9   13.1 / 14.8 / 14.8 -> 11.8 / 14.0 / 14.4 -> 12.8 / 18.7 / 15.8
-//   4112 of 9              18.3 / 21.0 / 22.1 -> 17.8 / 23.8 / 22.3 -> 20.1 / 30.3 / 27.1
+//   552 of 5 (L = 512)      5.4 / 6.5 / 9.6 -> 5.1 / 5.7 / 7.3 -> 5.1 / 5.9 / 6.6;    1048 of 3    5.3 / 6.3 / 6.8 -> 5.7 / 6.4 / 7.2 -> 6.4 / 7.4 / 8.6
+//   1032 of 9               9.6 / 11.8 / 9.0 -> 7.7 / 8.8 / 9.5 -> 7.6 / 8.4 / 10.2;  2056 of 9   10.6 / 14.1 / 11.5 -> 10.4 / 12.8 / 12.2 -> 12.0 / 14.2 / 14.4
+//   2072 of 4               8.2 / 10.0 / 10.4 -> 7.9 / 10.2 / 11.9 -> 9.3 / 12.7 / 14.2;  4112 of 9   15.0 / 18.4 / 19.0 -> 16.6 / 20.0 / 21.9 -> 19.3 / 23.5 / 27.0
+//   (two parts cost the last launches that take them up to 5 %: 1048 of 3)
 // The same line holds with dropout, the score term and narrow heads (one head a workgroup in parts, two otherwise); float32:
 //   L = 512, dropout                10.9 / 13.6 / 15.6 -> 7.9 / 10.2 / 10.4  -> 7.8 / 10.3 / 9.1;   term and dropout 11.8 / 16.5 / 16.2 -> 8.6 / 12.3 / 10.5 -> 8.0 / 11.9 / 8.2
 //   window 128, L = 4096, dropout   27.9 / 39.4 / 24.5 -> 22.3 / 35.6 / 20.9 -> 25.0 / 37.2 / 22.6; 6 x 50 with dropout 34.8 / 37.8 / 21.7 -> 26.6 / 28.0 / 20.8 -> 26.8 / 30.9 / 19.9
 //   L = 4096, k = 32, dropout       39.5 / 56.2 / 48.2 -> 34.8 / 54.5 / 43.6 -> 40.1 / 61.7 / 46.8; term and dropout 43.0 / 64.8 / 49.2 -> 37.5 / 63.9 / 45.1 -> 42.0 / 72.0 / 48.6
 //                                   6 x 50 with dropout 55.9 / 59.4 / 42.7 -> 33.5 / 44.1 / 34.5 -> 38.4 / 49.3 / 37.4
 //   L = 8192, k = 4 (one part)      35.8 / 55.6 / 38.3 -> 38.9 / 62.7 / 40.6;  6 x 50 with dropout 44.3 / 46.2 / 36.2 -> 47.0 / 50.1 / 38.4
-// bfloat16, dropout: L = 512 7.2 / 7.9 / 13.4 -> 5.9 / 6.6 / 9.7 -> 5.6 / 6.7 / 6.7; window 128, L = 4096 15.4 / 16.2 / 15.6 -> 12.5 / 14.7 / 15.0 -> 13.9 /
-// 19.3 / 16.4; 6 x 50 there 19.2 / 21.3 / 13.0 -> 14.4 / 17.3 / 12.8 -> 15.3 / 18.9 / 12.6.  Of 290 kernels of a hundred graphs drawn at random over all
+// bfloat16, dropout: L = 512 6.3 / 7.0 / 12.8 -> 5.5 / 5.9 / 10.7 -> 5.5 / 6.2 / 7.8; window 128, L = 4096 13.2 / 14.1 / 16.6 -> 11.7 / 12.6 / 16.7 -> 13.8 /
+// 15.4 / 18.8; 6 x 50 there 19.2 / 21.3 / 13.0 -> 14.4 / 17.3 / 12.8 -> 15.3 / 18.9 / 12.6.  Of 290 kernels of a hundred graphs drawn at random over all
 // of these the rule slowed one by more than 1 % against one part (a window of 52, forward 16.9 -> 17.8).
 // Two parts of launches that fill the chip about twice (6500 to 8192 wavefronts) pay on the source side (window 256, above) and with dropout
 // (forward there 108.2 -> 106.8), not for a float32 forward without: L = 7000, k = 32 51.7 -> 53.9, L = 6000, k = 64 63.5 -> 66.0, window 128, L =
