@@ -820,7 +820,8 @@ class PlanCache:
         if seg_len == SEG_BY_ROWS:
             seg_len, = seg_lens_by_rows([(row, indptr, eid.numel())])
         nr = n_rows if n_rows is not None or not on_device else (int(row[-1]) + 1 if row.numel() else 0)
-        if on_device and 0 <= nr < 2 ** 31 - 1:         # (a last row that is no row: the host builder says so)
+        # (a last row that is no row: the host builder says so; more units than rows and edges together: only that one takes them)
+        if on_device and 0 <= nr < 2 ** 31 - 1 and row.numel() <= eid.numel() + nr:
             ni = n_index_nodes if n_index_nodes is not None else nr
             plan = DevicePlan(row, indptr, eid, indices, nr, ni, eid.device, seg_len, groups=groups)
         else:

@@ -156,3 +156,28 @@ def test_a_plan_that_does_not_cover_every_edge_is_built_once():
         assert plan.plan_cache.misses == built + 2
     dk, = torch.autograd.grad(e, k, w)
     assert sum_ok(dk, s.src, one_weight, q[s.dst], s.n)
+
+
+def test_rows_cut_into_many_empty_units():
+    """More units than rows and edges together, which the builder on the GPU has no room for: the host's takes them."""
+    from bpt_amd import op, plan
+    s = sides("bpt512")
+    x = [rand((s.n, 8, 64), i).requires_grad_(True) for i in (1, 2, 3)]
+    do = rand((s.n, 8, 64), 4)
+    calls = (op.masked_mm, op.sparse_softmax, op.vec_spmm)
+
+    def cut(side):
+        row, indptr, eid, indices = side
+        more = s.E + s.n
+        return torch.cat([row[:1].expand(more), row]), torch.cat([indptr[:1].expand(more), indptr]), eid, indices
+
+    class Cut:
+        out, inn = cut(s.out), cut(s.inn)
+
+    plan.plan_cache.clear()
+    runs = []
+    for g in (s, Cut):
+        o = chain(calls, g, *x)
+        runs.append((o.detach(),) + torch.autograd.grad(o, x, do))
+    for a, b in zip(*runs):
+        assert ((a - b).norm() <= 1e-6 * a.norm()).all()          # (other groups of rows, other orders of the same float32 sums)
