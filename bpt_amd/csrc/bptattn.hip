@@ -91,15 +91,16 @@ __device__ __forceinline__ double exp_acc(double x) { return exp(x); }
 // ------------------------------------------------------------------------------------------
 struct Item { int row, begin, end, slot; };
 
-// Blocks go round-robin to the 8 XCDs; remap so XCD x gets a contiguous run of block indices.
-__device__ __forceinline__ int xcd_contiguous_block() {
-    const int nb = gridDim.x, b = blockIdx.x;
+// Blocks go round-robin to the 8 XCDs; remap so XCD x gets a contiguous run of block indices (of those behind the first `skip`,
+// a multiple of 8).
+__device__ __forceinline__ int xcd_contiguous_block(int skip = 0) {
+    const int nb = gridDim.x - skip, b = blockIdx.x - skip;
     const int q = nb >> 3, rem = nb & 7, x = b & 7, k = b >> 3;
     return x * q + (x < rem ? x : rem) + k;
 }
 
-__device__ __forceinline__ bool fetch_item(const bpt_plan &P, Item &it) {
-    const int w = xcd_contiguous_block() * WAVES_PER_BLOCK + (int)(threadIdx.x >> 6);
+__device__ __forceinline__ bool fetch_item(const bpt_plan &P, Item &it, int waves_per_block = WAVES_PER_BLOCK, int skip = 0) {
+    const int w = xcd_contiguous_block(skip) * waves_per_block + (int)(threadIdx.x >> 6);
     if (w >= (int)P.n_items) return false;
     const int4 v = reinterpret_cast<const int4 *>(P.items)[w];
     // the item is the same for all lanes of the wavefront: keep it in scalar registers
@@ -530,23 +531,35 @@ template <typename A, int NW, bool IS_MAX> __device__ __forceinline__ A head_red
     return r;
 }
 
-// seg_slot: NULL = whole rows only (segments of split rows are skipped); else it receives the item's slot (-1 = whole row)
-__device__ __forceinline__ bool softmax_range(const bpt_plan &P, int &begin, int &end, int *seg_slot = nullptr) {
-    Item it;
-    if (!fetch_item(P, it) || (it.slot >= 0 && !seg_slot)) return false;
-    begin = it.begin; end = it.end;
-    if (seg_slot) *seg_slot = it.slot;
+// WHOLE: split rows are taken whole by the first `whole` workgroups of the launch over the items, one each, and the items that are
+// segments do nothing: no second and third launch, each a chain of loads of its own, and nothing kept per segment (softmax_whole_rows
+// says where).
+constexpr int SM_BLOCK = 512, SM_WAVES = SM_BLOCK / WAVE;
+template <bool WHOLE> constexpr int sm_block() { return WHOLE ? SM_BLOCK : BLOCK; }
+__device__ __forceinline__ bool split_row(const bpt_plan &P, int i, int &begin, int &end) {
+    if (i >= (int)P.n_heavy) return false;                        // (their number is rounded up to a multiple of 8)
+    const int row = P.heavy[3 * i];
+    begin = P.rowptr[row];
+    end = P.rowptr[row + 1];
     return true;
 }
 
-template <typename T>
-__global__ __launch_bounds__(BLOCK) void k_softmax_fwd_heads(bpt_plan P, const T *__restrict__ x, T *__restrict__ y, int H,
-                                                                                   typename Elem<T>::acc_t *__restrict__ seg) {
+// seg_slot: the item's slot (-1 = whole row)
+template <bool WHOLE> __device__ __forceinline__ bool softmax_range(const bpt_plan &P, int &begin, int &end, int &seg_slot, int whole) {
+    Item it;
+    if (!fetch_item(P, it, sm_block<WHOLE>() / WAVE, WHOLE ? whole : 0) || (WHOLE && it.slot >= 0)) return false;
+    begin = it.begin; end = it.end;
+    seg_slot = it.slot;
+    return true;
+}
+
+// NW wavefronts share a row: SM_WAVES for a split row taken whole, else 1 an item
+template <typename T, int NW>
+__device__ __forceinline__ void softmax_fwd_heads(const bpt_plan &P, int begin, int end, int seg_slot, const T *__restrict__ x, T *__restrict__ y, int H,
+                                                  typename Elem<T>::acc_t *__restrict__ seg, typename Elem<T>::acc_t *smem) {
     using acc_t = typename Elem<T>::acc_t;
-    int begin, end, seg_slot = -1;
-    if (!softmax_range(P, begin, end, seg ? &seg_slot : nullptr)) return;
-    const int lane = threadIdx.x & 63, h = lane % H, slot = lane / H, nslots = WAVE / H;
-    const int first = slot < nslots ? begin + slot : end;         // (the lanes that are left over: no edges)
+    const int lane = threadIdx.x & 63, h = lane % H, slot = lane / H, per = WAVE / H, nslots = NW * per;
+    const int first = slot < per ? begin + (NW > 1 ? (int)(threadIdx.x >> 6) * per : 0) + slot : end;         // (the lanes that are left over: no edges)
     const bool cached = end - begin <= SM_CACHE * nslots;
     acc_t vc[SM_CACHE];
     size_t oc[SM_CACHE];
@@ -565,7 +578,7 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_fwd_heads(bpt_plan P, const T
             if (e[u] < 0) oc[u] = (size_t)-1;
         }
     }
-    m = head_reduce<acc_t, 1, true>(m, H, h, (acc_t *)nullptr);
+    m = head_reduce<acc_t, NW, true>(m, H, h, smem);
     acc_t s = 0;
     if (cached) {
 #pragma unroll
@@ -573,8 +586,8 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_fwd_heads(bpt_plan P, const T
     } else {
         for (int p = first; p < end; p += nslots) s += exp_acc((acc_t)Elem<T>::ld(x + (size_t)P.eid[p] * H + h) - m);
     }
-    s = head_reduce<acc_t, 1, false>(s, H, h, (acc_t *)nullptr);
-    if (seg_slot >= 0) {
+    s = head_reduce<acc_t, NW, false>(s, H, h, smem);
+    if (NW == 1 && seg_slot >= 0) {
         // a segment of a split row: only its (m, s); k_softmax_seg_rows forms the row's of them and k_softmax_fwd_seg_finish writes y
         if (slot == 0) { seg[((size_t)seg_slot * H + h) * 2] = m; seg[((size_t)seg_slot * H + h) * 2 + 1] = s; }
         return;
@@ -597,16 +610,26 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_fwd_heads(bpt_plan P, const T
         }
     }
 }
+template <typename T, bool WHOLE>
+__global__ __launch_bounds__(sm_block<WHOLE>()) void k_softmax_fwd_heads(bpt_plan P, const T *__restrict__ x, T *__restrict__ y, int H,
+                                                                typename Elem<T>::acc_t *__restrict__ seg, int whole) {
+    int begin, end, slot = -1;
+    if constexpr (WHOLE) {
+        __shared__ typename Elem<T>::acc_t smem[SM_WAVES * WAVE];
+        if ((int)blockIdx.x < whole) {
+            if (split_row(P, blockIdx.x, begin, end)) softmax_fwd_heads<T, SM_WAVES>(P, begin, end, -1, x, y, H, nullptr, smem);
+            return;
+        }
+    }
+    if (softmax_range<WHOLE>(P, begin, end, slot, whole)) softmax_fwd_heads<T, 1>(P, begin, end, slot, x, y, H, seg, nullptr);
+}
 
-template <typename T>
-__global__ __launch_bounds__(BLOCK) void k_softmax_bwd_heads(bpt_plan P, const T *__restrict__ y, const T *__restrict__ dy,
-                                                                                   T *__restrict__ dx, int H,
-                                                                                   typename Elem<T>::acc_t *__restrict__ seg) {
+template <typename T, int NW>
+__device__ __forceinline__ void softmax_bwd_heads(const bpt_plan &P, int begin, int end, int seg_slot, const T *__restrict__ y, const T *__restrict__ dy,
+                                                  T *__restrict__ dx, int H, typename Elem<T>::acc_t *__restrict__ seg, typename Elem<T>::acc_t *smem) {
     using acc_t = typename Elem<T>::acc_t;
-    int begin, end, seg_slot = -1;
-    if (!softmax_range(P, begin, end, seg ? &seg_slot : nullptr)) return;
-    const int lane = threadIdx.x & 63, h = lane % H, slot = lane / H, nslots = WAVE / H;
-    const int first = slot < nslots ? begin + slot : end;         // (the lanes that are left over: no edges)
+    const int lane = threadIdx.x & 63, h = lane % H, slot = lane / H, per = WAVE / H, nslots = NW * per;
+    const int first = slot < per ? begin + (NW > 1 ? (int)(threadIdx.x >> 6) * per : 0) + slot : end;         // (the lanes that are left over: no edges)
     const bool cached = end - begin <= SM_CACHE * nslots;
     acc_t yc[SM_CACHE], dc[SM_CACHE];
     size_t oc[SM_CACHE];
@@ -627,8 +650,8 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_bwd_heads(bpt_plan P, const T
 #pragma unroll
         for (int u = 0; u < SM_CACHE; ++u) s += dc[u] * yc[u];
     }
-    s = head_reduce<acc_t, 1, false>(s, H, h, (acc_t *)nullptr);
-    if (seg_slot >= 0) {
+    s = head_reduce<acc_t, NW, false>(s, H, h, smem);
+    if (NW == 1 && seg_slot >= 0) {
         // a segment of a split row: only its part of sum(dy * y); k_softmax_seg_rows adds the parts up and
         // k_softmax_bwd_seg_finish writes dx
         if (slot == 0) seg[(size_t)seg_slot * H + h] = s;
@@ -655,6 +678,19 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_bwd_heads(bpt_plan P, const T
                 if (e[u] >= 0) Elem<T>::st(dx + (size_t)e[u] * H + h, dv[u] * yv[u] - s * yv[u]);
         }
     }
+}
+template <typename T, bool WHOLE>
+__global__ __launch_bounds__(sm_block<WHOLE>()) void k_softmax_bwd_heads(bpt_plan P, const T *__restrict__ y, const T *__restrict__ dy, T *__restrict__ dx,
+                                                                int H, typename Elem<T>::acc_t *__restrict__ seg, int whole) {
+    int begin, end, slot = -1;
+    if constexpr (WHOLE) {
+        __shared__ typename Elem<T>::acc_t smem[SM_WAVES * WAVE];
+        if ((int)blockIdx.x < whole) {
+            if (split_row(P, blockIdx.x, begin, end)) softmax_bwd_heads<T, SM_WAVES>(P, begin, end, -1, y, dy, dx, H, nullptr, smem);
+            return;
+        }
+    }
+    if (softmax_range<WHOLE>(P, begin, end, slot, whole)) softmax_bwd_heads<T, 1>(P, begin, end, slot, y, dy, dx, H, seg, nullptr);
 }
 
 // Split rows of the softmax, second step: one block per split row.  Forward (PAIR): the segments' (m_i, s_i) are replaced by the
@@ -747,25 +783,42 @@ template <> struct Quad<bf16_t> {
     }
 };
 
-// over the slots of an item: the 8 Q lanes that share it, those of one quad of heads
-template <int Q, bool IS_MAX> __device__ __forceinline__ void quad_reduce(float (&v)[4]) {
+// over the slots of an item: the 8 Q lanes that share it, those of one quad of heads (or LANES)
+template <int Q, bool IS_MAX, int LANES = 8 * Q> __device__ __forceinline__ void quad_reduce(float (&v)[4]) {
 #pragma unroll
-    for (int off = Q; off < 8 * Q; off <<= 1)
+    for (int off = Q; off < LANES; off <<= 1)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const float o = __shfl_xor(v[i], off);
             v[i] = IS_MAX ? (v[i] > o ? v[i] : o) : v[i] + o;
         }
 }
+// over all threads of a workgroup of SM_WAVES wavefronts; part: SM_WAVES x 4 Q floats that nothing else uses
+template <int Q, bool IS_MAX> __device__ __forceinline__ void quad_reduce_block(float (&v)[4], float *part) {
+    quad_reduce<Q, IS_MAX, WAVE>(v);
+    const int lane = threadIdx.x & 63, q4 = 4 * (lane % Q);
+    if (lane < Q)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part[(threadIdx.x >> 6) * 4 * Q + q4 + i] = v[i];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = part[q4 + i];
+    for (int w = 1; w < SM_WAVES; ++w)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float o = part[w * 4 * Q + q4 + i];
+            v[i] = IS_MAX ? (v[i] > o ? v[i] : o) : v[i] + o;
+        }
+}
 
 // an item for every 8 Q lanes: eight slots a load, QUAD_U loads in flight (64 slots: an item of the usual length at once)
 constexpr int QUAD_SLOTS = 8, QUAD_U = 8;
-template <int Q> __device__ __forceinline__ bool fetch_quad_item(const bpt_plan &P, Item &it) {
-    const int64_t w = ((int64_t)xcd_contiguous_block() * BLOCK + threadIdx.x) / (QUAD_SLOTS * Q);
+template <int Q, bool WHOLE> __device__ __forceinline__ bool fetch_quad_item(const bpt_plan &P, Item &it, int whole) {
+    const int64_t w = ((int64_t)xcd_contiguous_block(WHOLE ? whole : 0) * sm_block<WHOLE>() + threadIdx.x) / (QUAD_SLOTS * Q);
     if (w >= P.n_items) return false;
     const int4 v = reinterpret_cast<const int4 *>(P.items)[w];
     it = Item{v.x, v.y, v.z, v.w};
-    return true;
+    return !WHOLE || it.slot < 0;
 }
 // ids of this lane's slots p, p + step, ...: -1 past the end of the range
 template <int U> __device__ __forceinline__ void quad_eids(const bpt_plan &P, int p, int step, int end, int (&e)[U]) {
@@ -773,11 +826,80 @@ template <int U> __device__ __forceinline__ void quad_eids(const bpt_plan &P, in
     for (int u = 0; u < U; ++u) e[u] = p + u * step < end ? P.eid[p + u * step] : -1;
 }
 
-template <typename T, int Q>
-__global__ __launch_bounds__(BLOCK) void k_softmax_fwd_quads(bpt_plan P, const T *__restrict__ x, T *__restrict__ y, float *__restrict__ seg) {
+// a split row, by a workgroup: what its threads' loads hold at once is read once, a longer row twice (max and sum of a thread together)
+template <typename T, int Q> __device__ __forceinline__ void softmax_fwd_whole_row(const bpt_plan &P, const T *__restrict__ x, T *__restrict__ y) {
+    constexpr int H = 4 * Q, SL = SM_BLOCK / Q, U = QUAD_U;
+    __shared__ float part[2][SM_WAVES * H];
+    int begin, end, e[U];
+    if (!split_row(P, blockIdx.x, begin, end)) return;
+    const int q4 = 4 * ((int)threadIdx.x % Q), p0 = begin + (int)threadIdx.x / Q;
+    const bool once = end - begin <= U * SL;
+    float v[U][4], m[4] = {-1e9f, -1e9f, -1e9f, -1e9f}, s[4] = {0.f, 0.f, 0.f, 0.f};
+    auto load = [&](int p) {
+        quad_eids<U>(P, p, SL, end, e);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            v[u][0] = v[u][1] = v[u][2] = v[u][3] = -INFINITY;
+            if (e[u] >= 0) Quad<T>::ld(x + (size_t)e[u] * H + q4, v[u]);
+        }
+    };
+    for (int p = p0; p < end || p == p0; p += U * SL) {
+        load(p);
+        float mn[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            mn[i] = m[i];
+#pragma unroll
+            for (int u = 0; u < U; ++u) mn[i] = v[u][i] > mn[i] ? v[u][i] : mn[i];
+            if (!once) {
+                s[i] *= expf(m[i] - mn[i]);
+#pragma unroll
+                for (int u = 0; u < U; ++u) s[i] += expf(v[u][i] - mn[i]);
+            }
+            m[i] = mn[i];
+        }
+    }
+    float M[4] = {m[0], m[1], m[2], m[3]};
+    quad_reduce_block<Q, true>(M, part[0]);
+    if (once) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { v[u][i] = expf(v[u][i] - M[i]); s[i] += v[u][i]; }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[i] *= expf(m[i] - M[i]);
+    }
+    quad_reduce_block<Q, false>(s, part[1]);
+    for (int p = p0; p < end; p += U * SL) {
+        if (!once) {
+            load(p);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[u][i] = expf(v[u][i] - M[i]);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (e[u] < 0) continue;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[u][i] = v[u][i] / s[i];
+            Quad<T>::st(y + (size_t)e[u] * H + q4, v[u]);
+        }
+    }
+}
+
+template <typename T, int Q, bool WHOLE>
+__global__ __launch_bounds__(sm_block<WHOLE>()) void k_softmax_fwd_quads(bpt_plan P, const T *__restrict__ x, T *__restrict__ y, float *__restrict__ seg, int whole) {
     constexpr int H = 4 * Q, SL = QUAD_SLOTS, U = QUAD_U;
+    if constexpr (WHOLE) {
+        if ((int)blockIdx.x < whole) {
+            softmax_fwd_whole_row<T, Q>(P, x, y);
+            return;
+        }
+    }
     Item it;
-    if (!fetch_quad_item<Q>(P, it)) return;
+    if (!fetch_quad_item<Q, WHOLE>(P, it, whole)) return;
     const int lane = threadIdx.x % (SL * Q), q4 = 4 * (lane % Q), p0 = it.begin + lane / Q;
     const bool once = it.end - it.begin <= U * SL;
     int e[U];
@@ -833,11 +955,58 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_fwd_quads(bpt_plan P, const T
 }
 
 template <typename T, int Q>
-__global__ __launch_bounds__(BLOCK) void k_softmax_bwd_quads(bpt_plan P, const T *__restrict__ y, const T *__restrict__ dy, T *__restrict__ dx,
-                                                             float *__restrict__ seg) {
+__device__ __forceinline__ void softmax_bwd_whole_row(const bpt_plan &P, const T *__restrict__ y, const T *__restrict__ dy, T *__restrict__ dx) {
+    constexpr int H = 4 * Q, SL = SM_BLOCK / Q, U = QUAD_U;
+    __shared__ float part[SM_WAVES * H];
+    int begin, end, e[U];
+    if (!split_row(P, blockIdx.x, begin, end)) return;
+    const int q4 = 4 * ((int)threadIdx.x % Q), p0 = begin + (int)threadIdx.x / Q;
+    const bool once = end - begin <= U * SL;
+    float yv[U][4], dv[U][4], s[4] = {0.f, 0.f, 0.f, 0.f};
+    auto load = [&](int p) {
+        quad_eids<U>(P, p, SL, end, e);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) yv[u][i] = dv[u][i] = 0.f;
+            if (e[u] >= 0) {
+                Quad<T>::ld(y + (size_t)e[u] * H + q4, yv[u]);
+                Quad<T>::ld(dy + (size_t)e[u] * H + q4, dv[u]);
+            }
+        }
+    };
+    for (int p = p0; p < end || p == p0; p += U * SL) {
+        load(p);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s[i] += dv[u][i] * yv[u][i];
+    }
+    quad_reduce_block<Q, false>(s, part);
+    for (int p = p0; p < end; p += U * SL) {
+        if (!once) load(p);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (e[u] < 0) continue;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) dv[u][i] = dv[u][i] * yv[u][i] - s[i] * yv[u][i];
+            Quad<T>::st(dx + (size_t)e[u] * H + q4, dv[u]);
+        }
+    }
+}
+
+template <typename T, int Q, bool WHOLE>
+__global__ __launch_bounds__(sm_block<WHOLE>()) void k_softmax_bwd_quads(bpt_plan P, const T *__restrict__ y, const T *__restrict__ dy, T *__restrict__ dx,
+                                                                float *__restrict__ seg, int whole) {
     constexpr int H = 4 * Q, SL = QUAD_SLOTS, U = QUAD_U;
+    if constexpr (WHOLE) {
+        if ((int)blockIdx.x < whole) {
+            softmax_bwd_whole_row<T, Q>(P, y, dy, dx);
+            return;
+        }
+    }
     Item it;
-    if (!fetch_quad_item<Q>(P, it)) return;
+    if (!fetch_quad_item<Q, WHOLE>(P, it, whole)) return;
     const int lane = threadIdx.x % (SL * Q), q4 = 4 * (lane % Q), p0 = it.begin + lane / Q;
     const bool once = it.end - it.begin <= U * SL;
     int e[U];
@@ -881,38 +1050,23 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_bwd_quads(bpt_plan P, const T
     }
 }
 
+// (Longer rows; L = 8192, k = 4: 7.7 -> 7.1 us with the first edges asked for ahead of the segments' sums, backward 8.0 -> 7.8.)
 // Split rows, second launch: block (i, j) is the j-th of gridDim.y blocks of split row i.  Every block reduces the row's segments
 // by itself (16 bytes a segment and head at most: they come from the L2), then writes its share of the row's edges.
 template <typename T, int Q, bool FWD>
 __global__ __launch_bounds__(BLOCK) void k_softmax_split_quads(bpt_plan P, const T *__restrict__ x, const T *__restrict__ dy, T *__restrict__ y,
                                                                const float *__restrict__ seg) {
-    constexpr int H = 4 * Q, SL = BLOCK / Q, U = 4;               // slots of a load of the block
+    constexpr int H = 4 * Q, SL = BLOCK / Q, U = 4, SU = 4;       // slots of a load of the block; its segments of a round a thread
     __shared__ float smem[WAVES_PER_BLOCK * WAVE];
     __shared__ float of_head[2][H];
     const int row = P.heavy[3 * blockIdx.x], s0 = P.heavy[3 * blockIdx.x + 1], ns = P.heavy[3 * blockIdx.x + 2];
     const int h = threadIdx.x % H, j0 = threadIdx.x / H, nj = BLOCK / H;
     const int begin = P.rowptr[row], deg = P.rowptr[row + 1] - begin;
     const int per = (deg + (int)gridDim.y - 1) / (int)gridDim.y, first = begin + (int)blockIdx.y * per, end = min(first + per, begin + deg);
-    if constexpr (FWD) {
-        float m = -1e9f, s = 0.f;
-        for (int j = j0; j < ns; j += nj) { const float v = seg[((size_t)(s0 + j) * H + h) * 2]; m = v > m ? v : m; }
-        m = head_reduce<float, WAVES_PER_BLOCK, true>(m, H, h, smem);
-        for (int j = j0; j < ns; j += nj) s += seg[((size_t)(s0 + j) * H + h) * 2 + 1] * expf(seg[((size_t)(s0 + j) * H + h) * 2] - m);
-        s = head_reduce<float, WAVES_PER_BLOCK, false>(s, H, h, smem);
-        if (threadIdx.x < H) { of_head[0][h] = m; of_head[1][h] = s; }
-    } else {
-        float s = 0.f;
-        for (int j = j0; j < ns; j += nj) s += seg[(size_t)(s0 + j) * H + h];
-        s = head_reduce<float, WAVES_PER_BLOCK, false>(s, H, h, smem);
-        if (threadIdx.x < H) of_head[0][h] = s;
-    }
-    __syncthreads();
-    const int q4 = 4 * ((int)threadIdx.x % Q);
+    const int q4 = 4 * ((int)threadIdx.x % Q), mine = first + (int)threadIdx.x / Q;
     float a[4], b[4], v[U][4], d[U][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { a[i] = of_head[0][q4 + i]; b[i] = FWD ? of_head[1][q4 + i] : 0.f; }
     int e[U];
-    for (int p = first + (int)threadIdx.x / Q; p < end; p += U * SL) {
+    auto load = [&](int p) {
         quad_eids<U>(P, p, SL, end, e);
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -920,6 +1074,44 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_split_quads(bpt_plan P, const
                 Quad<T>::ld(x + (size_t)e[u] * H + q4, v[u]);
                 if constexpr (!FWD) Quad<T>::ld(dy + (size_t)e[u] * H + q4, d[u]);
             }
+    };
+    // the first edges are on their way while the segments are added up
+    load(mine);
+    const float *const sg = seg + ((size_t)s0 * H + h) * (FWD ? 2 : 1);
+    if constexpr (FWD) {
+        float m = -1e9f, s = 0.f;
+        for (int j = j0; j < ns; j += SU * nj) {
+            float2 ms[SU];
+#pragma unroll
+            for (int u = 0; u < SU; ++u) ms[u] = j + u * nj < ns ? *reinterpret_cast<const float2 *>(sg + (size_t)(j + u * nj) * H * 2) : make_float2(-1e9f, 0.f);
+            float mn = m;
+#pragma unroll
+            for (int u = 0; u < SU; ++u) mn = ms[u].x > mn ? ms[u].x : mn;
+            s *= expf(m - mn);
+#pragma unroll
+            for (int u = 0; u < SU; ++u) s += ms[u].y * expf(ms[u].x - mn);
+            m = mn;
+        }
+        const float M = head_reduce<float, WAVES_PER_BLOCK, true>(m, H, h, smem);
+        s = head_reduce<float, WAVES_PER_BLOCK, false>(s * expf(m - M), H, h, smem);
+        if (threadIdx.x < H) { of_head[0][h] = M; of_head[1][h] = s; }
+    } else {
+        float s = 0.f;
+        for (int j = j0; j < ns; j += SU * nj) {
+            float t[SU];
+#pragma unroll
+            for (int u = 0; u < SU; ++u) t[u] = j + u * nj < ns ? sg[(size_t)(j + u * nj) * H] : 0.f;
+#pragma unroll
+            for (int u = 0; u < SU; ++u) s += t[u];
+        }
+        s = head_reduce<float, WAVES_PER_BLOCK, false>(s, H, h, smem);
+        if (threadIdx.x < H) of_head[0][h] = s;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { a[i] = of_head[0][q4 + i]; b[i] = FWD ? of_head[1][q4 + i] : 0.f; }
+    for (int p = mine; p < end; p += U * SL) {
+        if (p != mine) load(p);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (e[u] < 0) continue;
@@ -5041,22 +5233,43 @@ int run_spmm_generic(const bpt_plan *P, const void *W, const void *X, void *Y, v
 inline unsigned softmax_split_blocks(const bpt_plan *P) {
     return (unsigned)std::min<int64_t>(64, std::max<int64_t>(16, P->n_slots / P->n_heavy));
 }
-inline unsigned softmax_item_blocks(const bpt_plan *P, int q) { return (unsigned)((P->n_items * QUAD_SLOTS * q + BLOCK - 1) / BLOCK); }
+inline unsigned softmax_item_blocks(const bpt_plan *P, int q, int block) { return (unsigned)((P->n_items * QUAD_SLOTS * q + block - 1) / block); }
+// How many workgroups in front of the items' take a split row each: none where the plan does not say how long its longest row is, or where
+// one is longer than SM_WHOLE_EDGES.  A workgroup's CU keeps some 64 lines in flight and the records of a span's edges lie in a line
+// each: with the 8192 edges of the longest row of L = 8192 the forward took 39 us and the backward 51, in two launches 22 and 27.  Kernels,
+// two or three launches -> one, forward and backward: 8 heads, L = 500, both ways 9.7 + 8.6 -> 7.2 + 6.4 us; L = 1000 10.9 + 10.0 -> 8.4 + 7.6;
+// 16 graphs of up to 1024 17.9 + 15.4 -> 14.6 + 13.2; 6 heads, L = 1024, k = 8 14.4 + 12.2 -> 13.8 + 11.3.  Passes of the separate operators, which
+// the host bounds there: L = 100 146 -> 139 us, L = 500 151 -> 143, 6 x 50, L = 1024 152 -> 142, the 16 graphs 212 -> 206.
+constexpr int SM_WHOLE_EDGES = 1024;
+inline int softmax_whole_rows(const bpt_plan *P) {
+    if (P->n_heavy == 0 || P->max_degree <= 0 || P->max_degree > SM_WHOLE_EDGES) return 0;
+    return (int)((P->n_heavy + 7) & ~(int64_t)7);
+}
 
 template <typename T, int Q>
 int run_softmax_fwd_quads(const bpt_plan *P, const void *x, void *y, void *ws, hipStream_t s) {
-    hipLaunchKernelGGL((k_softmax_fwd_quads<T, Q>), dim3(softmax_item_blocks(P, Q)), dim3(BLOCK), 0, s, *P, (const T *)x, (T *)y, (float *)ws);
+    const int whole = softmax_whole_rows(P);
+    if (whole > 0)
+        hipLaunchKernelGGL((k_softmax_fwd_quads<T, Q, true>), dim3(whole + softmax_item_blocks(P, Q, SM_BLOCK)), dim3(SM_BLOCK), 0, s, *P, (const T *)x, (T *)y,
+                           (float *)nullptr, whole);
+    else
+        hipLaunchKernelGGL((k_softmax_fwd_quads<T, Q, false>), dim3(softmax_item_blocks(P, Q, BLOCK)), dim3(BLOCK), 0, s, *P, (const T *)x, (T *)y, (float *)ws, 0);
     const int st = launch_status();
-    if (st != BPT_OK || P->n_heavy == 0) return st;
+    if (st != BPT_OK || P->n_heavy == 0 || whole > 0) return st;
     hipLaunchKernelGGL((k_softmax_split_quads<T, Q, true>), dim3((int)P->n_heavy, softmax_split_blocks(P)), dim3(BLOCK), 0, s, *P, (const T *)x,
                        (const T *)nullptr, (T *)y, (const float *)ws);
     return launch_status();
 }
 template <typename T, int Q>
 int run_softmax_bwd_quads(const bpt_plan *P, const void *y, const void *dy, void *dx, void *ws, hipStream_t s) {
-    hipLaunchKernelGGL((k_softmax_bwd_quads<T, Q>), dim3(softmax_item_blocks(P, Q)), dim3(BLOCK), 0, s, *P, (const T *)y, (const T *)dy, (T *)dx, (float *)ws);
+    const int whole = softmax_whole_rows(P);
+    if (whole > 0)
+        hipLaunchKernelGGL((k_softmax_bwd_quads<T, Q, true>), dim3(whole + softmax_item_blocks(P, Q, SM_BLOCK)), dim3(SM_BLOCK), 0, s, *P, (const T *)y, (const T *)dy, (T *)dx,
+                           (float *)nullptr, whole);
+    else
+        hipLaunchKernelGGL((k_softmax_bwd_quads<T, Q, false>), dim3(softmax_item_blocks(P, Q, BLOCK)), dim3(BLOCK), 0, s, *P, (const T *)y, (const T *)dy, (T *)dx, (float *)ws, 0);
     const int st = launch_status();
-    if (st != BPT_OK || P->n_heavy == 0) return st;
+    if (st != BPT_OK || P->n_heavy == 0 || whole > 0) return st;
     hipLaunchKernelGGL((k_softmax_split_quads<T, Q, false>), dim3((int)P->n_heavy, softmax_split_blocks(P)), dim3(BLOCK), 0, s, *P, (const T *)y,
                        (const T *)dy, (T *)dx, (const float *)ws);
     return launch_status();
@@ -5076,9 +5289,14 @@ int run_softmax_fwd(const bpt_plan *P, const void *x, void *y, void *ws, int h, 
     }
     if (h <= WAVE) {           // heads side by side; split rows in three steps over their segments
         acc_t *seg = P->n_heavy > 0 ? (acc_t *)ws : nullptr;
-        hipLaunchKernelGGL((k_softmax_fwd_heads<T>), dim3(grid_for(P)), dim3(BLOCK), 0, s, *P, (const T *)x, (T *)y, h, seg);
+        const int whole = softmax_whole_rows(P);
+        if (whole > 0)
+            hipLaunchKernelGGL((k_softmax_fwd_heads<T, true>), dim3(whole + (unsigned)((P->n_items + SM_WAVES - 1) / SM_WAVES)), dim3(SM_BLOCK), 0, s,
+                               *P, (const T *)x, (T *)y, h, (acc_t *)nullptr, whole);
+        else
+            hipLaunchKernelGGL((k_softmax_fwd_heads<T, false>), dim3(grid_for(P)), dim3(BLOCK), 0, s, *P, (const T *)x, (T *)y, h, seg, 0);
         int st = launch_status();
-        if (st != BPT_OK || P->n_heavy == 0) return st;
+        if (st != BPT_OK || P->n_heavy == 0 || whole > 0) return st;
         hipLaunchKernelGGL((k_softmax_seg_rows<acc_t, true>), dim3((int)P->n_heavy), dim3(BLOCK), 0, s, P->heavy, seg, h);
         st = launch_status();
         if (st != BPT_OK) return st;
@@ -5102,9 +5320,14 @@ int run_softmax_bwd(const bpt_plan *P, const void *y, const void *dy, void *dx, 
     }
     if (h <= WAVE) {           // heads side by side; split rows in three steps over their segments
         acc_t *seg = P->n_heavy > 0 ? (acc_t *)ws : nullptr;
-        hipLaunchKernelGGL((k_softmax_bwd_heads<T>), dim3(grid_for(P)), dim3(BLOCK), 0, s, *P, (const T *)y, (const T *)dy, (T *)dx, h, seg);
+        const int whole = softmax_whole_rows(P);
+        if (whole > 0)
+            hipLaunchKernelGGL((k_softmax_bwd_heads<T, true>), dim3(whole + (unsigned)((P->n_items + SM_WAVES - 1) / SM_WAVES)), dim3(SM_BLOCK), 0, s,
+                               *P, (const T *)y, (const T *)dy, (T *)dx, h, (acc_t *)nullptr, whole);
+        else
+            hipLaunchKernelGGL((k_softmax_bwd_heads<T, false>), dim3(grid_for(P)), dim3(BLOCK), 0, s, *P, (const T *)y, (const T *)dy, (T *)dx, h, seg, 0);
         int st = launch_status();
-        if (st != BPT_OK || P->n_heavy == 0) return st;
+        if (st != BPT_OK || P->n_heavy == 0 || whole > 0) return st;
         hipLaunchKernelGGL((k_softmax_seg_rows<acc_t, false>), dim3((int)P->n_heavy), dim3(BLOCK), 0, s, P->heavy, seg, h);
         st = launch_status();
         if (st != BPT_OK) return st;

@@ -273,7 +273,7 @@ class Plan:
             d["eid"].data_ptr() if self.n_edges else None, d["items"].data_ptr() if self.n_items else None,
             d["heavy"].data_ptr() if self.n_heavy else None,
             self.n_rows, self.n_edges, self.n_items, self.n_heavy, self.n_slots)
-        self.struct.n_index_nodes = self.n_index_nodes
+        self.struct.n_index_nodes, self.struct.max_degree = self.n_index_nodes, int(self.max_degree)
 
     @property
     def ref(self):
@@ -525,7 +525,7 @@ class DevicePlan:
             d["rowptr"].data_ptr(), d["idx"].data_ptr() if E else None, d["eid"].data_ptr() if E else None,
             d["items"].data_ptr() if self.n_items else None, d["heavy"].data_ptr() if self.n_heavy else None,
             self.n_rows, E, self.n_items, self.n_heavy, self.n_slots)
-        self.struct.n_index_nodes = self.n_index_nodes
+        self.struct.n_index_nodes, self.struct.max_degree = self.n_index_nodes, int(self.max_degree)
 
     def _auto_seg_len(self, row, indptr):
         """auto_seg_len on the device: the 90 % quantile of the non-empty rows' degrees."""

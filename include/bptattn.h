@@ -94,6 +94,8 @@ typedef struct {
                                     row-group and tile kernels address rows of BOTH node tensors with 32-bit byte offsets and
                                     are taken only when max(n_rows, n_index_nodes) * h * d * sizeof(element) < 4 GiB; a
                                     caller whose neighbour tensor has more rows than n_rows must say so here */
+    int64_t max_degree;          /* edges of the longest row; 0 = not known (the edge softmax then merges split rows in
+                                    launches of their own).  Only a choice of kernels goes by it, never an address */
 } bpt_plan;
 
 /* sizeof(bpt_plan) as this library was compiled: a binding checks its own mirror of the struct against it before the first call
