@@ -4752,6 +4752,11 @@ template <> __device__ __forceinline__ void rel_load16<bf16_t>(const bf16_t *p, 
     }
 }
 
+// floats of LDS that a wavefront of k_rel_bias_bwd stages the ds values (H heads, rows 4 floats longer than 64 slots: other banks) and the types
+// of 64 slots in
+constexpr int REL_STAGE_PITCH = WAVE + 4;
+constexpr int REL_BWD_STAGE(int h) { return REL_STAGE_PITCH * h + WAVE; }
+
 // A work item (a row or a segment of a long row) and the types and edge ids of its first 64 slots (lane l: slot b + l).
 struct RelHead {
     int row, b, e, out_slot;
@@ -4761,9 +4766,9 @@ __device__ __forceinline__ void rel_head_load(const bpt_plan &P, const int4 item
     // the item is the same for all lanes of the wavefront: keep it in scalar registers
     r.row = __builtin_amdgcn_readfirstlane(item.x); r.b = __builtin_amdgcn_readfirstlane(item.y);
     r.e = __builtin_amdgcn_readfirstlane(item.z); r.out_slot = __builtin_amdgcn_readfirstlane(item.w);
-    const int slot = r.b + min(lane, max(min(WAVE, r.e - r.b), 1) - 1);        // lanes past the end repeat the last slot
-    r.type = r.b < r.e ? P.idx[slot] : 0;
-    r.edge = r.b < r.e ? P.eid[slot] : 0;
+    const int slot = min(r.b + min(lane, max(min(WAVE, r.e - r.b), 1) - 1), (int)P.n_edges - 1);   // lanes past the end repeat the last slot
+    r.type = P.idx[slot];
+    r.edge = P.eid[slot];
 }
 
 // The rows of the table that a graph uses, as floats in LDS: row u (`pitch` floats apart) = table[used_types[u]].  All
@@ -4771,9 +4776,18 @@ __device__ __forceinline__ void rel_head_load(const bpt_plan &P, const int4 item
 template <typename T>
 __device__ __forceinline__ void rel_table_to_lds(const T *__restrict__ table, const int32_t *__restrict__ used_types, int n_used, float *lds,
                                                  int pitch) {
-    for (int x = threadIdx.x; x < n_used * 16; x += blockDim.x) {
-        const int u = x >> 4, c4 = (x & 15) * 4;
-        *reinterpret_cast<float4 *>(lds + u * pitch + c4) = load4<T>(table + (size_t)used_types[u] * 64 + c4);
+    constexpr int AHEAD = 4;                                      // (round trips of two dependent loads each: four rows a thread side by side)
+    const int n = n_used * 16, step = (int)blockDim.x;
+    for (int x = threadIdx.x; x < n; x += AHEAD * step) {
+        int type[AHEAD];
+        float4 row[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) type[i] = used_types[min(x + i * step, n - 1) >> 4];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) row[i] = load4<T>(table + (size_t)type[i] * 64 + (min(x + i * step, n - 1) & 15) * 4);
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i)
+            if (x + i * step < n) *reinterpret_cast<float4 *>(lds + ((x + i * step) >> 4) * pitch + ((x + i * step) & 15) * 4) = row[i];
     }
 }
 
@@ -4928,154 +4942,217 @@ __global__ __launch_bounds__(HW * WAVE) void k_rel_bias_tiles(bpt_plan P, const 
 
 // Gradients of that term from ds[e, head] = dL/d(score of edge e before scaling): dq[row] += sum over the row's slots of
 // ds[eid] * table row of the slot's type (all heads), and the table's gradient, for type number u, the sum over the slots
-// with idx = u and the heads of ds[eid, head] * q[row, head].  Lane l owns column l.  Each wavefront walks every GW-th of
-// the plan's work items (rows and segments of long rows; a segment's part of dq goes to the workspace slot of the item,
-// which k_combine_sum_v4 adds to dq) and keeps its own sums per type number in LDS, beside the workgroup's copy of the
-// table rows in use; the wavefronts of a workgroup add theirs in a fixed order and the workgroup writes one partial
-// table, part[(u * gridDim.x + block) * 64 + column], which k_rel_table_sum adds up.  Every sum has one owner and a fixed
-// order.  The loads of an item run ahead of its use in three steps (descriptor; type numbers and edge ids of its first 64
-// slots; their ds values and the item's q and dq rows), each one item further ahead than the one that needs its result.
+// with idx = u and the heads of ds[eid, head] * q[row, head].  The wavefronts walk the plan's work items (rows and
+// segments of long rows; a segment's part of dq goes to the workspace slot of the item, which k_rel_finish adds to dq), sixteen
+// slots at a time, on v_mfma_f32_16x16x4f32 (lane (c, g) = (lane % 16, lane / 16)):
+//   dq rows (16 x 64 columns, heads in the order that spreads a row over all lanes, fewer heads than 16: zeros) += ds (heads x slots) * table rows (slots x columns): step s takes slots
+//     4 g + s; the table rows in use lie in LDS, columns 4 c .. 4 c + 3 of a row are one read a lane;
+//   U (slots x 64 columns) = ds^T (slots x heads) * q (heads x columns): register r of lane (c, g) is slot 4 g + r, columns 4 c ...
+// Both read ds from LDS, where an item's values of 64 slots are staged.  U's rows are added to the wavefront's own sums per type number
+// in LDS: all at once where the sixteen types differ (66 % of the sixteens at L = 8192, k = 4), as one row where they are the same
+// (34 %: a span's edges), one slot after the other else.  The wavefronts of a workgroup add their sums in a fixed order and the
+// workgroup writes one partial table, part[(u * gridDim.x + block) * 64 + column], which k_rel_finish adds up.  Every sum has one
+// owner and a fixed order.
+// The sums leave two wavefronts a SIMD, so what bounds the walk are the round trips of an item's loads: two items' bodies (ds, q, dq) are
+// in flight while one is used, and their types and edge ids two items ahead of that, so that no wait (they are in order) includes a
+// load that has just left.  A launch has a wavefront for every item up to 512 workgroups.  Against a walk that took one slot after the other
+// on the vector pipeline, with one item's loads ahead and a workgroup for 512 edges, kernel alone: 8 heads float32 L = 8192, k = 4 45.5 -> 39.5 us
+// (30.7 of them without any of the products: 132 MB take 26 at the rate of a copy), k = 8 both ways 297 -> 189, L = 100 25.7 -> 8.0; 16 heads
+// L = 4096, k = 16 186 -> 119; bfloat16 8 heads L = 32768, k = 2 177 -> 116, 16 heads L = 2048 57 -> 24, 666 nodes 136 -> 14; 4 heads L = 1024 20 -> 14,
+// L = 16384, k = 2 48 -> 49.5, the one shape that gained nothing.  Neighbouring items in neighbouring wavefronts, for the lines that
+// their ds values share: 39.5 -> 42.
 template <int H>
-struct RelBody {             // what the walk of those slots needs: per lane the ds values of its slot; the item's q row
-    float dsv[H];            // and, for a whole row, the dq row it adds to (lane l: column l)
-    float qh[H], old[H];
+struct RelBody {
+    float d[H];              // ds of the lane's slot
+    float4 q[H / 4], old[H / 4];      // columns 4 c .. 4 c + 3 of heads 4 s + g: q, and the dq row that a whole row adds to
 };
-// the H values of ds that belong to `edge`: a row of (n_edges, H), or with head_major one of each head's n_edges values
-template <int H>
-__device__ __forceinline__ void rel_ds_load(const float *__restrict__ ds, int edge, bool head_major, size_t n_edges, float (&out)[H]) {
-    if (head_major) {
-#pragma unroll
-        for (int h = 0; h < H; ++h) out[h] = ds[(size_t)h * n_edges + edge];
+// four columns of q or dq, which start on any element here (attention itself asks for 16 bytes)
+typedef uint32_t uintx2e __attribute__((ext_vector_type(2), aligned(2)));
+template <typename T> __device__ __forceinline__ float4 rel_load4(const T *p) {
+    if constexpr (sizeof(T) == 4) {
+        const floatx4u x = *reinterpret_cast<const floatx4u *>(p);
+        return make_float4(x[0], x[1], x[2], x[3]);
     } else {
-#pragma unroll
-        for (int h = 0; h < H; h += 4) {
-            const float4 x = *reinterpret_cast<const float4 *>(ds + (size_t)edge * H + h);
-            out[h] = x.x; out[h + 1] = x.y; out[h + 2] = x.z; out[h + 3] = x.w;
-        }
+        const uintx2e x = *reinterpret_cast<const uintx2e *>(p);
+        return make_float4(__uint_as_float(x[0] << 16), __uint_as_float(x[0] & 0xffff0000u), __uint_as_float(x[1] << 16), __uint_as_float(x[1] & 0xffff0000u));
     }
 }
+template <typename T> __device__ __forceinline__ void rel_store4(T *p, float4 v) {
+    if constexpr (sizeof(T) == 4) *reinterpret_cast<floatx4u *>(p) = floatx4u{v.x, v.y, v.z, v.w};
+    else *reinterpret_cast<uintx2e *>(p) = uintx2e{pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)};
+}
+// the H values of ds that belong to `edge`: of a row of (n_edges, H), or one of each head's n_edges values
+struct RelStride {
+    uint32_t edge, head;
+};
+template <int H> __device__ __forceinline__ void rel_ds_load(const float *__restrict__ ds, int edge, RelStride by, float (&out)[H]) {
+#pragma unroll
+    for (int h = 0; h < H; ++h) out[h] = ds[(size_t)h * by.head + (size_t)edge * by.edge];
+}
+// (No load stands behind a condition: where paths meet, the waits count for the one with the fewest loads.  An item without edges reads
+// places that are there, and a segment its row's dq.)
 template <typename T, int H>
-__device__ __forceinline__ void rel_body_load(const RelHead &r, const float *__restrict__ ds, bool head_major, size_t n_edges, const T *__restrict__ q,
+__device__ __forceinline__ void rel_body_load(const RelHead &r, const float *__restrict__ ds, RelStride by, const T *__restrict__ q,
                                               const T *__restrict__ dq, int lane, RelBody<H> &y) {
     constexpr int D = 64;
-    rel_ds_load<H>(ds, r.edge, head_major, n_edges, y.dsv);
+    const int c = lane & 15, g = lane >> 4;
+    rel_ds_load<H>(ds, r.edge, by, y.d);
 #pragma unroll
-    for (int h = 0; h < H; ++h) {
-        y.qh[h] = Elem<T>::ld(q + ((size_t)r.row * H + h) * D + lane);
-        y.old[h] = r.out_slot < 0 ? Elem<T>::ld(dq + ((size_t)r.row * H + h) * D + lane) : 0.f;
-    }
+    for (int s = 0; s < H / 4; ++s) y.q[s] = rel_load4<T>(q + ((size_t)r.row * H + 4 * s + g) * D + 4 * c);
+#pragma unroll
+    for (int s = 0; s < H / 4; ++s) y.old[s] = rel_load4<T>(dq + ((size_t)r.row * H + 4 * s + g) * D + 4 * c);
+}
+__device__ __forceinline__ void rel_add4(float *at, float x, float y, float z, float w) {
+    float4 v = *reinterpret_cast<const float4 *>(at);
+    v.x += x; v.y += y; v.z += z; v.w += w;
+    *reinterpret_cast<float4 *>(at) = v;
 }
 template <typename T, int H, int NW>
 __global__ __launch_bounds__(NW * WAVE) void k_rel_bias_bwd(bpt_plan P, const float *__restrict__ ds, const T *__restrict__ q,
                                                             const T *__restrict__ table, const int32_t *__restrict__ used_types, int n_used,
                                                             T *__restrict__ dq, float *__restrict__ ws_dq, float *__restrict__ part) {
-    constexpr int D = 64, C = H * D, AHEAD = H >= 16 ? 4 : 8;
-    extern __shared__ float rel_lds[];                    // NW tables of n_used x 64 sums, the table rows in use, NW x 64 x H staged ds values
-    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const bool head_major = P.bias_by_pair != 0;                // ds[head * n_edges + eid] instead of ds[eid * H + head]
+    constexpr int D = 64, C = H * D, PITCH = REL_STAGE_PITCH;
+    extern __shared__ float rel_lds[];                    // NW tables of n_used x 64 sums, the table rows in use, per wavefront 64 x H staged ds values and 64 types
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), c = lane & 15, g = lane >> 4;
+    const RelStride by = P.bias_by_pair != 0 ? RelStride{1u, (uint32_t)P.n_edges} : RelStride{(uint32_t)H, 1u};
     float *acc = rel_lds + (size_t)w * n_used * D;
     const float *rows = rel_lds + (size_t)NW * n_used * D;
-    float *stage = rel_lds + (size_t)(NW + 1) * n_used * D + (size_t)w * WAVE * H;
-    for (int u = 0; u < n_used; ++u) acc[u * D + lane] = 0.f;
-    rel_table_to_lds<T>(table, used_types, n_used, rel_lds + (size_t)NW * n_used * D, D);
+    float *stage = rel_lds + (size_t)(NW + 1) * n_used * D + (size_t)w * REL_BWD_STAGE(H);
+    int *types = reinterpret_cast<int *>(stage + PITCH * H);
     // wavefront gw of GW takes the items gw, gw + GW, ...: the segments of a long row, which are neighbours, go to different wavefronts
-    const int GW = (int)gridDim.x * NW, i_begin = (int)blockIdx.x * NW + w, i_end = (int)P.n_items;
+    const int GW = (int)gridDim.x * NW, i0 = (int)blockIdx.x * NW + w, n_items = (int)P.n_items, n_mine = i0 < n_items ? (n_items - i0 + GW - 1) / GW : 0;
     const int4 *items = reinterpret_cast<const int4 *>(P.items);
-    const int4 none = make_int4(0, 0, 0, -1);             // (an empty row: nothing to read, nothing to write)
-    RelHead hd, hd_next;
-    RelBody<H> bd, bd_next;
-    rel_head_load(P, i_begin < i_end ? items[i_begin] : none, lane, hd_next);
-    rel_body_load<T, H>(hd_next, ds, head_major, (size_t)P.n_edges, q, dq, lane, bd_next);
-    hd = hd_next;
-    rel_head_load(P, i_begin + GW < i_end ? items[i_begin + GW] : none, lane, hd_next);
-    int4 desc = i_begin + 2 * GW < i_end ? items[i_begin + 2 * GW] : none;
-    __syncthreads();
-    // one chunk of at most 64 slots whose ds values are staged: lane j of u (type numbers) belongs to slot j of the chunk
-    auto walk = [&](int cnt, int u, const float (&qh)[H], float (&dqa)[H]) {
-        wave_lds_fence();
-        for (int j0 = 0; j0 < cnt; j0 += AHEAD) {
-            // the ds values of AHEAD slots first (zeros are staged for the slots past the chunk's end, which so add nothing),
-            // then four slots at a time: the sums so far and the table rows, the products, the new sums.  The reads of
-            // the sums come before the products so that their latency is covered; where slots of a four have the same
-            // type, the later one's sum takes the earlier ones' terms in slot order, as if the four were added one
-            // after the other.
-            float4 dv[AHEAD][H / 4];
+    RelHead hd[4];
+    RelBody<H> bd[2];
+    auto body = [&](const RelHead &r, RelBody<H> &y) { rel_body_load<T, H>(r, ds, by, q, dq, lane, y); };
+    // ds and types of up to 64 slots (past the end: zeros; negative types, no two alike)
+    auto put = [&](int cnt, const float (&d)[H], int type) {
 #pragma unroll
-            for (int x = 0; x < AHEAD; ++x)
-#pragma unroll
-                for (int h = 0; h < H; h += 4) dv[x][h / 4] = *reinterpret_cast<const float4 *>(stage + min(j0 + x, WAVE - 1) * H + h);
-#pragma unroll
-            for (int x0 = 0; x0 < AHEAD; x0 += 4) {
-                if (j0 + x0 < cnt) {
-                    int un[4];
-                    float before[4], gsum[4], tv[4];
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) {
-                        un[x] = __builtin_amdgcn_readlane(u, min(j0 + x0 + x, cnt - 1));
-                        before[x] = acc[un[x] * D + lane];
-                        tv[x] = rows[un[x] * D + lane];
-                    }
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) {
-                        gsum[x] = 0.f;
-#pragma unroll
-                        for (int h = 0; h < H; h += 4) {
-                            const float4 d4 = dv[x0 + x][h / 4];
-                            gsum[x] = fmaf(d4.x, qh[h], gsum[x]); gsum[x] = fmaf(d4.y, qh[h + 1], gsum[x]);
-                            gsum[x] = fmaf(d4.z, qh[h + 2], gsum[x]); gsum[x] = fmaf(d4.w, qh[h + 3], gsum[x]);
-                            dqa[h] = fmaf(d4.x, tv[x], dqa[h]); dqa[h + 1] = fmaf(d4.y, tv[x], dqa[h + 1]);
-                            dqa[h + 2] = fmaf(d4.z, tv[x], dqa[h + 2]); dqa[h + 3] = fmaf(d4.w, tv[x], dqa[h + 3]);
-                        }
-                    }
-#pragma unroll
-                    for (int x = 0; x < 4; ++x) {
-                        float v = before[x];
-#pragma unroll
-                        for (int y = 0; y < x; ++y) v += un[y] == un[x] ? gsum[y] : 0.f;
-                        acc[un[x] * D + lane] = v + gsum[x];
-                    }
-                }
-            }
-        }
+        for (int h = 0; h < H; ++h) stage[h * PITCH + lane] = lane < cnt ? d[h] : 0.f;
+        types[lane] = lane < cnt ? type : -1 - lane;
         wave_lds_fence();
     };
-    for (int i = i_begin; i < i_end; i += GW) {
-        bd = bd_next;
-        rel_body_load<T, H>(hd_next, ds, head_major, (size_t)P.n_edges, q, dq, lane, bd_next);                // the item after this one
-        const RelHead cur = hd;
-        hd = hd_next;
-        rel_head_load(P, desc, lane, hd_next);                                   // the second after
-        desc = i + 3 * GW < i_end ? items[i + 3 * GW] : none;
-        float dqa[H];
+    // sixteen slots of those, cnt of them exist
+    auto sixteen = [&](int j, int cnt, const float4 (&qr)[H / 4], floatx4v (&dqa)[4]) {
+        const int4 t4 = *reinterpret_cast<const int4 *>(types + j + 4 * g);               // of slots 4 g .. 4 g + 3
+        const int ty[4] = {t4.x, t4.y, t4.z, t4.w}, mine = types[j + c];
+        // row c of the product is head 4 (c % 4) + c / 4, so that register s of lane group g is head 4 s + g
+        floatx4v a4 = *reinterpret_cast<const floatx4v *>(stage + (4 * min(c & 3, H / 4 - 1) + (c >> 2)) * PITCH + j + 4 * g);   // the same slots
+        if (H < 16 && (c & 3) >= H / 4) a4 = floatx4v{0.f, 0.f, 0.f, 0.f};
+        float d[H / 4];
 #pragma unroll
-        for (int h = 0; h < H; ++h) dqa[h] = 0.f;
-        if (cur.b < cur.e) {
+        for (int s = 0; s < H / 4; ++s) d[s] = stage[(4 * s + g) * PITCH + j + c];
+        float4 tv[4], before[4];                                  // table rows of those slots; the sums of their types so far
 #pragma unroll
-            for (int h = 0; h < H; h += 4)
-                *reinterpret_cast<float4 *>(stage + lane * H + h) =
-                    lane < cur.e - cur.b ? make_float4(bd.dsv[h], bd.dsv[h + 1], bd.dsv[h + 2], bd.dsv[h + 3]) : make_float4(0.f, 0.f, 0.f, 0.f);
-            walk(min(WAVE, cur.e - cur.b), cur.type, bd.qh, dqa);
+        for (int r = 0; r < 4; ++r) tv[r] = *reinterpret_cast<const float4 *>(rows + max(ty[r], 0) * D + 4 * c);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) before[r] = *reinterpret_cast<const float4 *>(acc + max(ty[r], 0) * D + 4 * c);
+        // slots of one type: lane (c, g) compares the type of slot c with those of slots 4 g + s
+        bool twice = false;
+        uint64_t same0 = 0;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const bool same = mine == ty[s];
+            twice = twice || (same && c != 4 * g + s);
+            if (s == 0) same0 = __builtin_amdgcn_ballot_w64(same);
         }
-        for (int p0 = cur.b + WAVE; p0 < cur.e; p0 += WAVE) {                  // (items longer than 64 slots: the rest, fetched on the spot)
-            const int cnt = min(WAVE, cur.e - p0);
-            const int slot = p0 + min(lane, cnt - 1);
-            const int u = P.idx[slot], edge = P.eid[slot];
-            float rest[H];
-            rel_ds_load<H>(ds, edge, head_major, (size_t)P.n_edges, rest);
+        issue_loads_first();                                      // (one round trip through LDS after the types', not one a product)
+        floatx4v u[4];
 #pragma unroll
-            for (int h = 0; h < H; h += 4)
-                *reinterpret_cast<float4 *>(stage + lane * H + h) =
-                    lane < cnt ? make_float4(rest[h], rest[h + 1], rest[h + 2], rest[h + 3]) : make_float4(0.f, 0.f, 0.f, 0.f);
-            walk(cnt, u, bd.qh, dqa);
+        for (int nb = 0; nb < 4; ++nb) u[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < H / 4; ++s) {
+            u[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[s], qr[s].x, u[0], 0, 0, 0);
+            u[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[s], qr[s].y, u[1], 0, 0, 0);
+            u[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[s], qr[s].z, u[2], 0, 0, 0);
+            u[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[s], qr[s].w, u[3], 0, 0, 0);
         }
-        if (cur.out_slot < 0) {
-            if (cur.b < cur.e) {
 #pragma unroll
-                for (int h = 0; h < H; ++h) Elem<T>::st(dq + ((size_t)cur.row * H + h) * D + lane, bd.old[h] + dqa[h]);
-            }
+        for (int s = 0; s < 4; ++s) {
+            dqa[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[s], tv[s].x, dqa[0], 0, 0, 0);
+            dqa[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[s], tv[s].y, dqa[1], 0, 0, 0);
+            dqa[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[s], tv[s].z, dqa[2], 0, 0, 0);
+            dqa[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[s], tv[s].w, dqa[3], 0, 0, 0);
+        }
+        if (__builtin_amdgcn_ballot_w64(twice) == 0) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (ty[r] >= 0)
+                    *reinterpret_cast<float4 *>(acc + ty[r] * D + 4 * c) =
+                        make_float4(before[r].x + u[0][r], before[r].y + u[1][r], before[r].z + u[2][r], before[r].w + u[3][r]);
+        } else if ((int)__popcll(same0 & 0xffffu) == cnt) {       // every slot that exists has the first one's type (those past the end add nothing)
+            float x[4];
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) x[nb] = groups_sum((u[nb][0] + u[nb][1]) + (u[nb][2] + u[nb][3]));
+            if (g == 0) rel_add4(acc + ty[0] * D + 4 * c, x[0], x[1], x[2], x[3]);
         } else {
 #pragma unroll
-            for (int h = 0; h < H; ++h) ws_dq[(size_t)cur.out_slot * C + h * D + lane] = dqa[h];
+            for (int r = 0; r < 4; ++r)
+                for (int gg = 0; gg < 4; ++gg) {
+                    if (g == gg && ty[r] >= 0) rel_add4(acc + ty[r] * D + 4 * c, u[0][r], u[1][r], u[2][r], u[3][r]);
+                    wave_lds_fence();
+                }
+        }
+        wave_lds_fence();                                         // (read before the next are staged, and written before they are added)
+    };
+    auto item = [&](const RelHead &cur, const RelBody<H> &b) {
+        floatx4v dqa[4];
+#pragma unroll
+        for (int nb = 0; nb < 4; ++nb) dqa[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
+        if (cur.b < cur.e) put(min(WAVE, cur.e - cur.b), b.d, cur.type);
+        for (int p0 = cur.b; p0 < cur.e; p0 += TILE_R) {
+            const int at = p0 - cur.b;
+            if (at > 0 && (at & (WAVE - 1)) == 0) {               // (items longer than 64 slots: the rest, fetched on the spot)
+                const int cnt = min(WAVE, cur.e - p0), slot = p0 + min(lane, cnt - 1);
+                float rest[H];
+                rel_ds_load<H>(ds, P.eid[slot], by, rest);
+                put(cnt, rest, P.idx[slot]);
+            }
+            sixteen(at & (WAVE - 1), min(TILE_R, cur.e - p0), b.q, dqa);
+        }
+        if (cur.out_slot >= 0 || cur.b < cur.e) {
+#pragma unroll
+            for (int s = 0; s < H / 4; ++s) {
+                const int at = (4 * s + g) * D + 4 * c;
+                const float4 x = make_float4(dqa[0][s], dqa[1][s], dqa[2][s], dqa[3][s]), o = b.old[s];
+                if (cur.out_slot < 0) rel_store4<T>(dq + (size_t)cur.row * C + at, make_float4(o.x + x.x, o.y + x.y, o.z + x.z, o.w + x.w));
+                else *reinterpret_cast<float4 *>(ws_dq + (size_t)cur.out_slot * C + at) = x;
+            }
+        }
+    };
+    int4 descs;                                                   // of 64 items, one a lane
+    int n_here = 0;
+    auto head = [&](int n, RelHead &r) {                          // (past the last one: nothing to read, nothing to write)
+        auto of = [&](int x, int none) {
+            const int v = __builtin_amdgcn_readlane(x, n & (WAVE - 1));
+            return n < n_here ? v : none;
+        };
+        rel_head_load(P, make_int4(of(descs.x, 0), of(descs.y, 0), of(descs.z, 0), of(descs.w, -1)), lane, r);
+    };
+    auto begin = [&](int first) {
+        n_here = min(WAVE, n_mine - first);
+        descs = items[min(i0 + (first + min(lane, max(n_here, 1) - 1)) * GW, n_items - 1)];
+#pragma unroll
+        for (int n = 0; n < 4; ++n) head(n, hd[n]);
+#pragma unroll
+        for (int n = 0; n < 2; ++n) body(hd[n], bd[n]);
+    };
+    begin(0);
+    issue_loads_first();                                          // (on their way while the table rows are fetched)
+    for (int u = 0; u < n_used; ++u) acc[u * D + lane] = 0.f;
+    rel_table_to_lds<T>(table, used_types, n_used, rel_lds + (size_t)NW * n_used * D, D);
+    __syncthreads();
+    for (int first = 0; first < n_mine; first += WAVE) {
+        if (first > 0) begin(first);
+        for (int n0 = 0; n0 < n_here; n0 += 4) {
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                issue_loads_first();
+                item(hd[n], bd[n & 1]);
+                issue_loads_first();
+                body(hd[(n + 2) & 3], bd[n & 1]);
+                head(n0 + n + 4, hd[n]);
+            }
         }
     }
     __syncthreads();
@@ -5438,8 +5515,8 @@ inline bool rel_rows_shape(int h, int d, int dtype) {
 constexpr int REL_MAX_PARTS = 512;        // partial tables of the gradient kernel: two workgroups per compute unit
 constexpr int REL_MAX_USED = 240;         // type numbers whose table rows fit the 64 KB of LDS of the score kernel
 
-// LDS of k_rel_bias_bwd with nw wavefronts: their sums, the table rows, their staged ds values
-inline size_t rel_bwd_lds(int nw, int64_t n_used, int h) { return ((size_t)(nw + 1) * n_used * 64 + (size_t)nw * WAVE * h) * 4; }
+// LDS of k_rel_bias_bwd with nw wavefronts: their sums, the table rows, their staged ds values and types
+inline size_t rel_bwd_lds(int nw, int64_t n_used, int h) { return ((size_t)(nw + 1) * n_used * 64 + (size_t)nw * REL_BWD_STAGE(h)) * 4; }
 // wavefronts per workgroup of k_rel_bias_bwd for n_used types: the 4, 2 or 1 that put most wavefronts on a compute unit
 // (workgroups that fit its 160 KB of LDS x wavefronts each; more per workgroup on a tie: fewer partial tables), a
 // workgroup taking at most 144 KB (large_lds false: at most the 64 KB every kernel may take).  0: no configuration fits.
@@ -5494,7 +5571,7 @@ int run_rel_bias_bwd(const bpt_plan *P, const float *ds, const void *q, const vo
     float *ws_dq = ws, *part = ws + (size_t)P->n_slots * H * 64;       // partial rows of dq of the split rows, then the partial tables
     int n_parts = 0;
     auto launch = [&](int nw) {
-        n_parts = (int)std::min<int64_t>(REL_MAX_PARTS, std::max<int64_t>(1, (P->n_edges + nw * 128 - 1) / (nw * 128)));
+        n_parts = (int)std::min<int64_t>(REL_MAX_PARTS, std::max<int64_t>(1, (P->n_items + nw - 1) / nw));      // (an item a wavefront at the least)
         return nw == 4   ? launch_rel_bias_bwd<T, H, 4>(P, ds, q, table, used_types, n_used, dq, ws_dq, part, n_parts, s)
                : nw == 2 ? launch_rel_bias_bwd<T, H, 2>(P, ds, q, table, used_types, n_used, dq, ws_dq, part, n_parts, s)
                          : launch_rel_bias_bwd<T, H, 1>(P, ds, q, table, used_types, n_used, dq, ws_dq, part, n_parts, s);
