@@ -35,9 +35,9 @@ using at::Tensor;
 
 namespace {
 
-enum Kind { ATTN_FWD = 0, ATTN_BWD = 1, ATTN_FWD_NARROW = 2, ATTN_BWD_NARROW = 3, MM_FWD = 4, MM_BWD = 5, SPMM_FWD = 6, SPMM_BWD = 7, SOFTMAX = 8 };
+enum Kind { ATTN_FWD = 0, ATTN_BWD = 1, ATTN_FWD_NARROW = 2, ATTN_BWD_NARROW = 3, MM_FWD = 4, MM_BWD = 5, SPMM_FWD = 6, SPMM_BWD = 7, SOFTMAX = 8, REL_FWD = 9, REL_TRAIN = 10 };
 
-constexpr size_t MAX_TENSORS = 8, MAX_EXTRA = 7, MAX_ENTRIES = 512;
+constexpr size_t MAX_TENSORS = 9, MAX_EXTRA = 7, MAX_ENTRIES = 512;
 
 struct Key {                          // compared and hashed as bytes: always zeroed first
     int64_t kind, device;
@@ -61,7 +61,8 @@ struct KeyHash {
 };
 
 struct Entry {
-    bpt_plan a{}, b{};
+    bpt_plan a{}, b{}, c{};
+    std::vector<Tensor> more;         // REL_*: the index tensors of the score term (RelTensor)
     std::vector<PyObject *> plans;    // owned: what the structs point into lives as long as the entry
     std::vector<Tensor> index;        // whose addresses the key holds: they are not given to other tensors meanwhile
     std::atomic<bool> used{false};
@@ -392,6 +393,125 @@ Tensor attention_narrow(const Tensor &row, const Tensor &indptr_r, const Tensor 
     if (differentiated({&q, &k, &v}))
         return NarrowAttention::apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, h, scale, p, (int64_t)seed);
     return std::get<0>(narrow_forward(col, indptr_c, eid_c, indices_c, rows(q), rows(k), rows(v), h, scale, p, (int64_t)seed, Copies{}));
+}
+
+// ---- fused attention with the relative-position term, in the order of the tile plan's pairs (op.BPTRelAttention) ---------------
+// A training pass through the Python function cost the host 157 or 267 us by the process (89 forward and 113 backward at its best), L = 100 as
+// L = 8192, whose kernels take 225.  Passes on a machine of the slower kind: L = 100 267 -> 109 us, L = 2048 16 heads bfloat16 277 -> 110, 6 x 50 on padded
+// copies, 16 graphs, 444 -> 249; with the gradient's kernel of now L = 8192, k = 8 both ways 905 -> 785, L = 32768 bfloat16 576 -> 515.
+// An entry holds what both passes need (REL_FWD: the forward only), and the autograd node keeps the entry: its backward looks nothing up.
+enum RelTensor { REL_USED_TYPES = 0, REL_PAIR_TYPES = 1, REL_USED = 2, REL_ROWS_SLOT = 3, REL_NUMBER_SLOT = 4 };
+
+EntryPtr rel_entry(Kind kind, const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r, const Tensor &indices_r, const Tensor &col,
+                   const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c, const Tensor &q, const Tensor &k, const Tensor &v, double p,
+                   const Tensor &table, const Tensor &etype) {
+    Shape s;
+    if (!attention_shape(q, k, v, p, s) || indices_c.sizes() != eid_c.sizes() || indices_r.sizes() != eid_r.sizes() || eid_r.sizes() != eid_c.sizes())
+        return nullptr;
+    if (!like(table, q) || table.dim() != 2 || table.size(1) != s.d) return nullptr;
+    Key key;
+    if (!make_key(key, kind, {&row, &indptr_r, &eid_r, &indices_r, &col, &indptr_c, &eid_c, &indices_c, &etype}, q.device(),
+                  {s.nq, s.nk, s.h, s.d, s.dt, p > 0.0, table.size(0)}))
+        return nullptr;
+    return find(key);
+}
+
+// (o, lse, the term)
+std::optional<Three> rel_forward_known(const EntryPtr &e, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &table, double scale, double p,
+                                       uint64_t seed) {
+    const int h = (int)q.size(1), d = (int)q.size(2), dt = dtype_code(q.scalar_type());
+    c10::DeviceGuard guard(q.device());
+    void *stream = stream_of(q.device());
+    Tensor bias = at::empty({h, e->a.n_edges}, q.options().dtype(at::kFloat));
+    const Tensor &types = e->more[REL_USED_TYPES];
+    if (bpt_rel_bias_forward_tiles(&e->a, q.data_ptr(), table.data_ptr(), types.const_data_ptr<int32_t>(), types.numel(),
+                                   e->more[REL_PAIR_TYPES].const_data_ptr<int32_t>(), bias.data_ptr<float>(), h, d, dt, stream) != BPT_OK)
+        return std::nullopt;
+    Tensor o = at::empty_like(q), lse = at::empty({q.size(0), h}, q.options().dtype(at::kFloat));
+    Workspace ws(BPT_OP_ATTN_FWD, &e->a, nullptr, h, d, dt, q);
+    if (bpt_attention_forward(&e->a, q.data_ptr(), k.data_ptr(), v.data_ptr(), bias.data_ptr<float>(), o.data_ptr(), lse.data_ptr<float>(), ws.ptr, ws.bytes,
+                              (float)scale, (float)p, seed, h, d, dt, stream) != BPT_OK)
+        return std::nullopt;
+    return Three{o, lse, bias};
+}
+
+std::optional<std::array<Tensor, 4>> rel_backward_known(const EntryPtr &e, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &o,
+                                                        const Tensor &lse, const Tensor &bias, const Tensor &table, const Tensor &d_o, double scale,
+                                                        double p, uint64_t seed) {
+    if (!like(d_o, q) || d_o.sizes() != q.sizes()) return std::nullopt;
+    const int h = (int)q.size(1), d = (int)q.size(2), dt = dtype_code(q.scalar_type());
+    c10::DeviceGuard guard(q.device());
+    void *stream = stream_of(q.device());
+    Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), ds = at::empty_like(bias), dtable = at::empty_like(table);
+    {
+        Workspace ws(BPT_OP_ATTN_BWD, &e->a, &e->b, h, d, dt, q);
+        if (bpt_attention_backward(&e->a, &e->b, q.data_ptr(), k.data_ptr(), v.data_ptr(), bias.data_ptr<float>(), o.data_ptr(), d_o.data_ptr(),
+                                   lse.data_ptr<float>(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ds.data_ptr<float>(), ws.ptr, ws.bytes,
+                                   (float)scale, (float)p, seed, h, d, dt, stream) != BPT_OK)
+            return std::nullopt;
+    }
+    const Tensor &types = e->more[REL_USED_TYPES];
+    const int64_t bytes = std::max<int64_t>(bpt_rel_bias_backward_workspace_bytes(&e->c, types.numel(), h), 16);
+    Tensor ws = at::empty({bytes}, q.options().dtype(at::kByte));
+    if (bpt_rel_bias_backward(&e->c, ds.data_ptr<float>(), q.data_ptr(), table.data_ptr(), e->more[REL_USED].const_data_ptr<int32_t>(),
+                              types.const_data_ptr<int32_t>(), table.size(0), types.numel(), dq.data_ptr(), dtable.data_ptr(), ws.data_ptr(), bytes, h, d, dt,
+                              stream) != BPT_OK)
+        return std::nullopt;
+    return std::array<Tensor, 4>{dq, dk, dv, dtable};
+}
+
+struct RelHold : torch::CustomClassHolder {
+    EntryPtr e;
+    explicit RelHold(EntryPtr x) : e(std::move(x)) {}
+};
+
+// (r: what the forward has computed already: a call that the library refuses never becomes a node)
+struct RelAttention : torch::autograd::Function<RelAttention> {
+    static Tensor forward(torch::autograd::AutogradContext *ctx, const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r,
+                          const Tensor &indices_r, const Tensor &col, const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c,
+                          const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &table, const EntryPtr &e, const Three &r, double scale,
+                          double p, int64_t seed) {
+        const auto &[o, lse, bias] = r;
+        ctx->save_for_backward({row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, o, lse, bias, table});
+        ctx->saved_data["entry"] = c10::IValue::make_capsule(c10::make_intrusive<RelHold>(e));
+        ctx->saved_data["scale"] = scale;
+        ctx->saved_data["p"] = p;
+        ctx->saved_data["seed"] = seed;
+        return o;
+    }
+    static torch::autograd::variable_list backward(torch::autograd::AutogradContext *ctx, torch::autograd::variable_list grads) {
+        const auto t = ctx->get_saved_variables();
+        const double scale = ctx->saved_data["scale"].toDouble(), p = ctx->saved_data["p"].toDouble();
+        const uint64_t seed = (uint64_t)ctx->saved_data["seed"].toInt();
+        const EntryPtr e = c10::static_intrusive_pointer_cast<RelHold>(ctx->saved_data["entry"].toCapsule())->e;
+        const Tensor d_o = grads[0].contiguous();
+        auto r = rel_backward_known(e, t[8], t[9], t[10], t[11], t[12], t[13], t[14], d_o, scale, p, seed);
+        if (!r)
+            r = with_python([&] {
+                const auto four = py::module_::import("bpt_amd.op").attr("_rel_backward")(
+                                       t[0], t[1], t[2], t[3], t[4], t[5], t[6], t[7], t[8], t[9], t[10], t[11], t[12], t[13], t[14], d_o, scale, p, seed,
+                                       e->more[REL_ROWS_SLOT], e->more[REL_NUMBER_SLOT], e->more[REL_USED], e->more[REL_USED_TYPES])
+                                      .template cast<std::vector<Tensor>>();
+                return std::array<Tensor, 4>{four[0], four[1], four[2], four[3]};
+            });
+        torch::autograd::variable_list out(17);
+        for (int i = 0; i < 4; ++i) out[8 + i] = (*r)[i];
+        return out;
+    }
+};
+
+// op.BPTRelAttention of a call whose plans are known, or None
+std::optional<Tensor> rel_attention(const Tensor &row, const Tensor &indptr_r, const Tensor &eid_r, const Tensor &indices_r, const Tensor &col,
+                                    const Tensor &indptr_c, const Tensor &eid_c, const Tensor &indices_c, const Tensor &q, const Tensor &k,
+                                    const Tensor &v, double scale, double p, uint64_t seed, const Tensor &table, const Tensor &etype) {
+    const bool train = differentiated({&q, &k, &v, &table});
+    EntryPtr e = rel_entry(REL_TRAIN, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, p, table, etype);
+    if (!e && !train) e = rel_entry(REL_FWD, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, p, table, etype);
+    if (!e) return std::nullopt;
+    const auto r = rel_forward_known(e, q, k, v, table, scale, p, seed);
+    if (!r) return std::nullopt;
+    if (!train) return std::get<0>(*r);
+    return RelAttention::apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, table, e, *r, scale, p, (int64_t)seed);
 }
 
 // ---- the separate operators (modules/op.py:10-58 of the reference) -----------------------------------------------------------
@@ -736,7 +856,8 @@ py::object build_tile_plans(const std::vector<std::tuple<Tensor, Tensor, Tensor,
 // `kind`'s choice for these index tensors and numbers: the bpt_plan structs at the addresses a and b (0: none), which point into
 // what `plans` holds.  generation: what generation() said before the choice was begun; a table that was cleared since does not take
 // it, since a switch may have changed under it.  True if it was taken.
-bool remember(int64_t generation, int kind, const std::vector<Tensor> &index, const std::vector<int64_t> &extra, int64_t a, int64_t b, py::tuple plans) {
+bool remember_more(int64_t generation, int kind, const std::vector<Tensor> &index, const std::vector<int64_t> &extra, int64_t a, int64_t b, int64_t c,
+                   const std::vector<Tensor> &more, py::tuple plans) {
     if (index.empty() || index.size() > MAX_TENSORS || extra.size() > MAX_EXTRA || !index[0].defined() || !index[0].is_cuda() || !a) return false;
     std::vector<const Tensor *> ptrs;
     for (const Tensor &t : index) ptrs.push_back(&t);
@@ -746,6 +867,8 @@ bool remember(int64_t generation, int kind, const std::vector<Tensor> &index, co
     auto e = std::make_shared<Entry>();
     std::memcpy(&e->a, reinterpret_cast<const void *>(a), sizeof(bpt_plan));
     if (b) std::memcpy(&e->b, reinterpret_cast<const void *>(b), sizeof(bpt_plan));
+    if (c) std::memcpy(&e->c, reinterpret_cast<const void *>(c), sizeof(bpt_plan));
+    e->more = more;
     for (auto p : plans) e->plans.push_back(p.inc_ref().ptr());
     e->index = index;
     e->used.store(true);
@@ -762,6 +885,22 @@ bool remember(int64_t generation, int kind, const std::vector<Tensor> &index, co
         slot = e;
     }
     return true;
+}
+
+bool remember(int64_t generation, int kind, const std::vector<Tensor> &index, const std::vector<int64_t> &extra, int64_t a, int64_t b, py::tuple plans) {
+    return remember_more(generation, kind, index, extra, a, b, 0, {}, std::move(plans));
+}
+
+// the same for the attention with relative positions: c, the plan of the term's gradient, and the term's index tensors in the order of RelTensor
+bool remember_rel(int64_t generation, int kind, const std::vector<Tensor> &index, const std::vector<int64_t> &extra, int64_t a, int64_t b, int64_t c,
+                  const std::vector<Tensor> &more, py::tuple plans) {
+    if (kind != REL_FWD && kind != REL_TRAIN) return false;
+    if (more.size() != (kind == REL_FWD ? 2 : 5) || (kind == REL_TRAIN && (!b || !c))) return false;
+    for (const Tensor &t : more)
+        if (!t.is_cuda() || t.dim() != 1 || !t.is_contiguous()) return false;
+    for (RelTensor i : {REL_USED_TYPES, REL_PAIR_TYPES, REL_USED})
+        if ((size_t)i < more.size() && more[i].scalar_type() != at::kInt) return false;
+    return remember_more(generation, kind, index, extra, a, b, c, more, std::move(plans));
 }
 
 // drops what was chosen with this plan object
@@ -819,6 +958,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.attr("SPMM_FWD") = (int)SPMM_FWD;
     m.attr("SPMM_BWD") = (int)SPMM_BWD;
     m.attr("SOFTMAX") = (int)SOFTMAX;
+    m.attr("REL_FWD") = (int)REL_FWD;
+    m.attr("REL_TRAIN") = (int)REL_TRAIN;
     m.def("masked_mm", &masked_mm);
     m.def("sparse_softmax", &sparse_softmax);
     m.def("vec_spmm", &vec_spmm);
@@ -830,7 +971,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("build_csrs", &build_csrs);
     m.def("build_tile_plans", &build_tile_plans);
     m.def("count_rows", &count_rows);
+    m.def("rel_attention", &rel_attention);
     m.def("remember", &remember);
+    m.def("remember_rel", &remember_rel);
     m.def("forget", &forget);
     m.def("clear", &clear);
     m.def("generation", &generation);

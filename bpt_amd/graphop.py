@@ -977,6 +977,51 @@ def rel_bias_forward_tiles(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c
     return bias
 
 
+def prepare_rel_training(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p):
+    """prepare_training for a layer with the relative-position term: the tile plans of both sides built together, where neither is in the
+    cache and the tile kernels are certain.  A convenience: what is not built here is built when it is asked for."""
+    cfg, graph = _SETTINGS, (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
+    if q.dim() != 3 or not q.is_cuda or any(t.dim() != 1 or t.dtype != torch.int64 or t.device != q.device or not t.is_contiguous() for t in graph):
+        return
+    h, d = _hd(q)
+    if k.dim() != 3 or not attention_supported(q) or not _tiles_backward(None, q.dtype, q):
+        return
+    seg = _tile_seg_without_plan(col, eid_c.size(0), q, k, h, d, dropout_p, q, cfg)
+    if seg is not None:
+        plan_cache.put_tile_plans([(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg, None),
+                                   (row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg, _plan.tile_order_src(k.size(0), eid_r.size(0)))])
+
+
+def remember_rel(generation, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p, table, etype, aux, train):
+    """Leaves with the native host path what a forward (train: and a backward) with the relative-position term takes for these arguments, of
+    which rel_bias_forward_tiles has just been found to run: the in-CSR's tile plan, the out-CSR's linked to it, the plan of the term's
+    gradient, and the term's index tensors (op._rel_aux)."""
+    graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
+    if any(t.dtype != torch.int64 for t in graph) or TILE_BACKWARD is not None:
+        return                       # (with the hook set the passes choose for themselves)
+    hit, held = _pair_order(*graph, q, k, dropout_p), aux["rows_slot"]
+    if hit is None or held[0] is not hit[1]["pair_of_eid"]:
+        return
+    pi, in_struct = hit[0], hit[1]["struct"]
+    index, numbers = list(graph) + [etype], [q.size(0), k.size(0), q.size(1), q.size(2), _dtype(q), int(dropout_p > 0.0), table.size(0)]
+    with torch.cuda.device(q.device):
+        torch.cuda.current_stream().synchronize()          # (the term's index tensors are there for whichever stream serves the next call)
+    if not train:
+        plan_cache.remember((pi,), generation, _native.REL_FWD, index, numbers, ctypes.addressof(in_struct), 0, 0, [aux["used_types"], held[2]],
+                            how="remember_rel")
+        return
+    order_src = _plan.tile_order_src(k.size(0), eid_r.size(0))
+    po = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg_len=_tile_seg_of(eid_c.size(0), q.size(0), k.size(0)),
+                        prefer_device=True, groups=(TILE_ROWS, order_src))
+    if po.n_edges != pi.n_edges or not po.covers_all_edges:
+        return
+    out_struct = po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True)
+    rel = plan_cache.get(col, indptr_c, held[1], aux["number_slot"], q.size(0), max(aux["n_used"], 1), prefer_device=True)     # (rel_bias_backward's)
+    rel_struct = _by_pair(rel.struct)
+    plan_cache.remember((pi, po, rel), generation, _native.REL_TRAIN, index, numbers, ctypes.addressof(in_struct), ctypes.addressof(out_struct),
+                        ctypes.addressof(rel_struct), [aux["used_types"], held[2], aux["used"], held[1], aux["number_slot"]], how="remember_rel")
+
+
 def attention_dropout_mask(col, indptr_c, eid_c, indices_c, q, k, dropout_p, seed):
     """The (E, h) float32 multipliers (0 or 1 / (1 - p)) that attention_forward(..., dropout_p, seed) applies to the
     attention probabilities, computed on the host (testing and debugging aid).  The decision is a hash of

@@ -124,8 +124,10 @@ class BPTRelAttention(Function):
                 types = torch.empty_like(aux["number_slot"]).index_copy_(0, rows_slot, aux["number_slot"]).to(torch.int32)
                 held = aux["rows_slot"] = (pair, rows_slot, (types | (_g.attention_pair_members(*graph, dropout_p) << 8)).contiguous())
             ctx.rows_slot = held[1]
+            aux["on_tiles"] = False
             try:
                 bias = _g.rel_bias_forward_tiles(*graph, table, aux["used_types"], held[2], dropout_p)
+                aux["on_tiles"] = True
             except _g.BptStatusError as err:
                 # (many types in use need more than 64 KB of LDS there, which a runtime may refuse: the kernel over the
                 # in-CSR writes the same layout from within 64 KB)
@@ -147,12 +149,14 @@ class BPTRelAttention(Function):
     def backward(ctx, do):
         row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, o, lse, bias, table = ctx.saved_tensors
         aux = ctx.aux
+        if ctx.rows_slot is not None:
+            dq, dk, dv, dtable = _rel_backward(*ctx.saved_tensors, do, ctx.scale, ctx.dropout_p, ctx.seed, ctx.rows_slot, aux["number_slot"],
+                                               aux["used"], aux["used_types"])
+            return None, None, None, None, None, None, None, None, dq, dk, dv, None, None, None, dtable, None
         dq, dk, dv, ds = _g.attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c,
-                                               q, k, v, o, lse, do, ctx.scale, ctx.dropout_p, ctx.seed, bias=bias,
-                                               bias_by_pair=ctx.rows_slot is not None)
+                                               q, k, v, o, lse, do, ctx.scale, ctx.dropout_p, ctx.seed, bias=bias)
         if ctx.on_chip:
-            dtable = _g.rel_bias_backward(col, indptr_c, eid_c if ctx.rows_slot is None else ctx.rows_slot, aux["number_slot"], aux["used"],
-                                          aux["used_types"], ds, q, table, dq, by_pair=ctx.rows_slot is not None)
+            dtable = _g.rel_bias_backward(col, indptr_c, eid_c, aux["number_slot"], aux["used"], aux["used_types"], ds, q, table, dq)
         else:
             t_row, t_indptr, t_order, t_dst = _rel_type_rows(aux, ctx.etype, col, indptr_c, eid_c, table.size(0))
             h = q.size(1)
@@ -162,6 +166,37 @@ class BPTRelAttention(Function):
             dtable = vector_spmm_forward(t_row, t_indptr, t_order, t_dst, ds, q, n_rows=table.size(0))
             dtable = dtable.float().sum(1).to(table.dtype)
         return None, None, None, None, None, None, None, None, dq, dk, dv, None, None, None, dtable, None
+
+
+def _rel_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, o, lse, bias, table, do, scale, dropout_p, seed, rows_slot,
+                  number_slot, used, used_types):
+    """(dq, dk, dv, dtable) where the term and its gradient are stored in the order of the tiles' pairs; also what the native host path's
+    node comes to with a call that its table does not serve."""
+    dq, dk, dv, ds = _g.attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, o, lse, do, scale, dropout_p,
+                                           seed, bias=bias, bias_by_pair=True)
+    return dq, dk, dv, _g.rel_bias_backward(col, indptr_c, rows_slot, number_slot, used, used_types, ds, q, table, dq, by_pair=True)
+
+
+_REL_FORM = _g.rel_bias_forward_tiles        # what the native host path stands for: where a caller has put another function in its place, it does not
+
+
+def _rel_attention(*args):
+    """BPTRelAttention, by the native host path where it knows the call (the second one of a graph, shape and type on)."""
+    graph, (q, k, v, scale, dropout_p, seed, table, etype) = args[:8], args[8:]
+    if not (_served_natively(graph) and _native_takes(etype) and _g.rel_bias_forward_tiles is _REL_FORM):
+        return BPTRelAttention.apply(*args)
+    o = _native.rel_attention(*graph, q, k, v, scale, dropout_p, seed & (2 ** 64 - 1), table, etype)
+    if o is not None:
+        return o
+    generation = _native.generation()
+    train = torch.is_grad_enabled() and any(x.requires_grad for x in (q, k, v, table))
+    if train:
+        _g.prepare_rel_training(*graph, q, k, dropout_p)
+    o = BPTRelAttention.apply(*args)
+    aux = _rel_aux(etype, graph[4], graph[5], graph[6], table.size(0))
+    if aux.get("on_tiles"):                          # (the call that has just run took the tile form)
+        _g.remember_rel(generation, *graph, q, k, dropout_p, table, etype, aux, train)
+    return o
 
 
 _rel_aux_cache = {}
@@ -342,15 +377,15 @@ def bpt_attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices
                 return _native.attention_narrow(*graph, q, k, v, hp, scale, float(dropout_p), int(seed or 0) & (2 ** 64 - 1))
             o = BPTAttention.apply(*graph, grow(q), grow(k), grow(v), scale, float(dropout_p), int(seed or 0))
             return o[:, :h, :d].contiguous()
-        o = BPTRelAttention.apply(*graph, grow(q), grow(k), grow(v), scale, float(dropout_p), int(seed or 0),
-                                  torch.nn.functional.pad(rel_table, (0, dp - d)), etype)
+        o = _rel_attention(*graph, grow(q), grow(k), grow(v), scale, float(dropout_p), int(seed or 0),
+                           torch.nn.functional.pad(rel_table, (0, dp - d)), etype)
         return o[:, :h, :d].contiguous()
     if fused:
         if dropout_p > 0 and seed is None:
             seed = int(torch.randint(0, 2 ** 62, (1,)).item())
         if rel_table is not None:
-            return BPTRelAttention.apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale,
-                                         float(dropout_p), int(seed or 0), rel_table, etype)
+            return _rel_attention(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale, float(dropout_p), int(seed or 0),
+                                  rel_table, etype)
         if not _served_natively((row, indptr_r, eid_r, indices_r)):
             return BPTAttention.apply(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale,
                                       float(dropout_p), int(seed or 0))

@@ -764,12 +764,12 @@ class PlanCache:
         self._d[key] = (plan, tensors)
         self._total += plan.device_bytes()
 
-    def remember(self, plans, *choice):
-        """native.remember(*choice, plans): what was chosen with these plans, as long as all of them are here.  Another thread may
-        have dropped one since the caller got it; nobody would tell the native host path when its index tensors go."""
+    def remember(self, plans, *choice, how="remember"):
+        """native.remember(*choice, plans) (or remember_rel): what was chosen with these plans, as long as all of them are here.  Another
+        thread may have dropped one since the caller got it; nobody would tell the native host path when its index tensors go."""
         with self._lock:
             if all(any(p is plan for p, _ in reversed(self._d.values())) for plan in plans):
-                self.native.remember(*choice, plans)
+                getattr(self.native, how)(*choice, plans)
 
     def _evict(self):
         # called with the lock held; the newest entry always stays
