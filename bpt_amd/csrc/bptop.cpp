@@ -783,6 +783,58 @@ std::vector<int64_t> count_rows(const std::vector<std::tuple<Tensor, Tensor>> &i
     return counts;
 }
 
+// The arrays of a side's base plan, for the largest numbers of items and split rows that its sizes allow
+std::vector<Tensor> base_arrays(const bpt_build_side &s, const at::TensorOptions &i32) {
+    const int64_t E = std::max<int64_t>(s.n_edges, 1), items = std::max<int64_t>(s.n_rows + s.n_edges / s.seg_len, 1);
+    return {at::empty({s.n_rows + 1}, i32), at::empty({E}, i32), at::empty({E}, i32), at::empty({items, 4}, i32), at::empty({items, 2}, i32),
+            at::empty({std::max<int64_t>(s.n_edges / (s.seg_len + 1), 1), 3}, i32), at::empty({16}, i32)};
+}
+void point_at(bpt_build_side &s, const std::vector<Tensor> &base, const Tensor &row, const Tensor &indptr, const Tensor &eid, const Tensor &indices) {
+    s.row = row.const_data_ptr<int64_t>(); s.indptr_units = indptr.const_data_ptr<int64_t>();
+    s.eid = eid.const_data_ptr<int64_t>(); s.indices = indices.const_data_ptr<int64_t>();
+    int32_t **to[7] = {&s.rowptr, &s.idx32, &s.eid32, &s.items, &s.item_bounds, &s.heavy, &s.info};
+    for (int j = 0; j < 7; ++j) *to[j] = base[j].data_ptr<int32_t>();
+}
+
+// The base plans of one or two sides, in one launch where they are small and with one wait: per side its info block and base arrays, or None where
+// an array is not what the kernels read.
+py::object build_plans(const std::vector<std::tuple<Tensor, Tensor, Tensor, Tensor, int64_t, int64_t, int>> &in) {
+    const int n = (int)in.size();
+    if (n < 1 || n > 2) throw std::invalid_argument("one or two sides");
+    const at::Device dev = std::get<2>(in[0]).device();
+    for (const auto &[row, indptr, eid, indices, n_rows, n_index, seg] : in)
+        for (const Tensor *t : {&row, &indptr, &eid, &indices})
+            if (!index_ok(*t, dev)) return py::none();
+    c10::DeviceGuard guard(dev);
+    const auto i32 = at::TensorOptions().dtype(at::kInt).device(dev);
+    bpt_build_side sides[2] = {};
+    std::vector<std::vector<Tensor>> base(n);
+    for (int i = 0; i < n; ++i) {
+        const auto &[row, indptr, eid, indices, n_rows, n_index, seg] = in[i];
+        bpt_build_side &s = sides[i];
+        s.n_units = row.numel(); s.n_edges = eid.numel(); s.n_rows = n_rows; s.n_index_nodes = n_index; s.seg_len = seg;
+        if (indptr.numel() != s.n_units + 1 || indices.numel() != s.n_edges || n_rows < 0 || n_index < 0 || seg < 1) return py::none();
+    }
+    int64_t bytes = 0;
+    if (bpt_build_plans_bounds(sides, n, &bytes) != BPT_OK) return py::none();
+    for (int i = 0; i < n; ++i) {
+        const auto &[row, indptr, eid, indices, n_rows, n_index, seg] = in[i];
+        base[i] = base_arrays(sides[i], i32);
+        point_at(sides[i], base[i], row, indptr, eid, indices);
+    }
+    Tensor ws = at::empty({bytes}, i32.dtype(at::kByte));
+    Tensor infos = at::empty({16 * n}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+    void *stream = stream_of(dev);
+    check_build(bpt_build_plans(sides, n, infos.data_ptr<int32_t>(), ws.data_ptr(), bytes, stream), "bpt_build_plans");
+    wait_for(stream);
+    py::list result;
+    for (int i = 0; i < n; ++i) {
+        const int32_t *c = infos.data_ptr<int32_t>() + 16 * i;
+        result.append(py::make_tuple(std::vector<int>(c, c + 16), base[i]));
+    }
+    return result;
+}
+
 // None where the short form does not build them; else (per side: its info block, base arrays, group arrays; the pair mapping of
 // the second side).  A side's info block holds an error where its arrays are malformed (then nothing else is valid).
 py::object build_tile_plans(const std::vector<std::tuple<Tensor, Tensor, Tensor, Tensor, int64_t, int64_t, int, int>> &in) {
@@ -807,14 +859,8 @@ py::object build_tile_plans(const std::vector<std::tuple<Tensor, Tensor, Tensor,
     if (bpt_build_tiles_bounds(sides, n, &bytes) != BPT_OK) return py::none();
     for (int i = 0; i < n; ++i) {
         const auto &[row, indptr, eid, indices, n_rows, n_index, seg, mask] = in[i];
-        bpt_build_side &s = sides[i];
-        const int64_t E = std::max<int64_t>(s.n_edges, 1), items = std::max<int64_t>(s.n_rows + s.n_edges / seg, 1);
-        base[i] = {at::empty({s.n_rows + 1}, i32), at::empty({E}, i32), at::empty({E}, i32), at::empty({items, 4}, i32), at::empty({items, 2}, i32),
-                   at::empty({std::max<int64_t>(s.n_edges / (seg + 1), 1), 3}, i32), at::empty({16}, i32)};
-        s.row = row.const_data_ptr<int64_t>(); s.indptr_units = indptr.const_data_ptr<int64_t>();
-        s.eid = eid.const_data_ptr<int64_t>(); s.indices = indices.const_data_ptr<int64_t>();
-        int32_t **to[7] = {&s.rowptr, &s.idx32, &s.eid32, &s.items, &s.item_bounds, &s.heavy, &s.info};
-        for (int j = 0; j < 7; ++j) *to[j] = base[i][j].data_ptr<int32_t>();
+        base[i] = base_arrays(sides[i], i32);
+        point_at(sides[i], base[i], row, indptr, eid, indices);
     }
     Tensor ws = at::empty({bytes}, i32.dtype(at::kByte));
     Tensor counts = at::empty({32 * n}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
@@ -969,6 +1015,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("attention_forward", &attention_forward_known);
     m.def("attention_backward", &attention_backward_known);
     m.def("build_csrs", &build_csrs);
+    m.def("build_plans", &build_plans);
     m.def("build_tile_plans", &build_tile_plans);
     m.def("count_rows", &count_rows);
     m.def("rel_attention", &rel_attention);

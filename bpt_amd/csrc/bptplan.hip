@@ -306,6 +306,57 @@ struct RsToArrays {
     }
 };
 
+// Stable radix sort of n words in LDS by a workgroup of 16 wavefronts: by bits [shift, shift + bits), a digit of at most 8 a pass, each
+// wavefront a run of up to KPT * 64 words, ranked as k_rs_scatter does.  hist: 16 x 256 ints.  (A bitonic sort in its place, 5 600 edges in
+// 8 192 places: k_csr_small 17 -> 36 us, k_plan_small 19 -> 27.)
+constexpr int SMALL_TPB = 1024, SMALL_NW = SMALL_TPB / 64, SMALL_BINS = 256;
+template <int KPT> __device__ __forceinline__ void lds_radix(uint32_t *word, int n, int shift, int bits, int32_t *hist, int32_t *sh) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, passes = (bits + 7) / 8, digit = (bits + passes - 1) / passes, bins = 1 << digit;
+    const int per = (n + SMALL_NW * 64 - 1) / (SMALL_NW * 64), i0 = wave * per * 64 + lane;          // (at most KPT)
+    const uint64_t below = (uint64_t(1) << lane) - 1;
+    for (int p = 0; p < passes; ++p, shift += digit) {
+        uint32_t key[KPT];
+        int32_t rank[KPT];
+        for (int b = tid; b < SMALL_NW * bins; b += SMALL_TPB) hist[b] = 0;
+#pragma unroll
+        for (int r = 0; r < KPT; ++r) key[r] = r < per && i0 + r * 64 < n ? word[i0 + r * 64] : 0u;
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < KPT; ++r) {
+            const bool on = r < per && i0 + r * 64 < n;
+            if (__ballot(on) == 0) continue;
+            const int d = (int)((key[r] >> shift) & (uint32_t)(bins - 1));
+            uint64_t peers = __ballot(on);
+            for (int b = 0; b < digit; ++b) {
+                const bool bit = (d >> b) & 1;
+                const uint64_t m = __ballot(bit);
+                peers &= bit ? m : ~m;
+            }
+            const int32_t before = hist[wave * bins + d];
+            rank[r] = before + __popcll(peers & below);
+            wave_lds_order();
+            if (on && (peers & below) == 0) hist[wave * bins + d] = before + __popcll(peers);
+            wave_lds_order();
+        }
+        __syncthreads();
+        int32_t sum = 0, all;
+        if (tid < bins)
+            for (int w = 0; w < SMALL_NW; ++w) sum += hist[w * bins + tid];
+        int32_t at = block_excl_sum<SMALL_NW>(sum, sh, all);
+        if (tid < bins)
+            for (int w = 0; w < SMALL_NW; ++w) {
+                const int32_t c = hist[w * bins + tid];
+                hist[w * bins + tid] = at;
+                at += c;
+            }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < KPT; ++r)
+            if (r < per && i0 + r * 64 < n) word[hist[wave * bins + (int)((key[r] >> shift) & (uint32_t)(bins - 1))] + rank[r]] = key[r];
+        __syncthreads();
+    }
+}
+
 // ---- base plan ---------------------------------------------------------------------------------------------------------
 // Five launches and the sort: clear; narrow the indices, check the units, find the rows; emit the items; their smallest and
 // largest neighbour; sort by the smallest.
@@ -583,6 +634,166 @@ struct ItemsSorted {
         if (S.bounds) S.bounds[at] = S.bounds_tmp[i];
     }
 };
+
+// The items in LDS: by their smallest neighbour (word: that and their place, BITS bits), the records moved, then, where groups follow, the
+// order by the largest.  A sort key is n_index_nodes at most (an item without edges).
+template <int BITS, int KPT> __device__ __forceinline__ void order_by_largest(const PlanSide &S, int n_items, uint32_t *word, int32_t *hist, int32_t *sh) {
+    const int tid = threadIdx.x, key_bits = 32 - __clz((int)S.n_index_nodes | 1);
+    for (int at = tid; at < n_items; at += SMALL_TPB) word[at] = ((uint32_t)S.bounds[at].y << BITS) | (uint32_t)at;
+    __syncthreads();
+    lds_radix<KPT>(word, n_items, BITS, key_bits, hist, sh);
+    for (int at = tid; at < n_items; at += SMALL_TPB) S.jorder[at] = (int32_t)(word[at] & ((1u << BITS) - 1u));
+}
+template <int BITS, int KPT> __device__ __forceinline__ void order_items(const PlanSide &S, int n_items, uint32_t *word, int32_t *hist, int32_t *sh) {
+    const int tid = threadIdx.x, key_bits = 32 - __clz((int)S.n_index_nodes | 1);
+    lds_radix<KPT>(word, n_items, BITS, key_bits, hist, sh);
+    for (int at = tid; at < n_items; at += SMALL_TPB) {
+        const int i = (int)(word[at] & ((1u << BITS) - 1u));
+        S.items[at] = S.items_tmp[i];
+        if (S.bounds) S.bounds[at] = S.bounds_tmp[i];
+    }
+    if (!S.jorder || !S.bounds) return;
+    __syncthreads();
+    order_by_largest<BITS, KPT>(S, n_items, word, hist, sh);
+}
+
+// Both orders of up to 11 264 items (60 KB of LDS) by a workgroup a side, in place of the eight launches of the two sorts (5 to 7 us each).
+// One CU is the bound, so the line lies where its LDS ends: 8 trees of 400 leaves, 10 900 items a side, 46 us of launches -> 27.5, a training
+// pass on a new graph 551 -> 532 us (three processes each way); 16 of 100 leaves 575 -> 545.
+constexpr int ORDER_ITEM_BITS = 14, ORDER_ITEMS = 11 * SMALL_TPB;
+inline bool order_in_lds(const PlanSide &S) { return S.max_items <= ORDER_ITEMS && S.n_index_nodes < 1 << (32 - ORDER_ITEM_BITS); }
+__global__ __launch_bounds__(SMALL_TPB) void k_item_order(PlanSides b) {
+    const PlanSide &S = b.side[blockIdx.x];
+    __shared__ uint32_t word[ORDER_ITEMS];
+    __shared__ int32_t hist[SMALL_NW * SMALL_BINS], sh[SMALL_NW + 1];
+    if (S.info[BPT_PI_ERR]) return;
+    const int n_items = min(S.info[BPT_PI_N_ITEMS], ORDER_ITEMS);
+    for (int i = threadIdx.x; i < n_items; i += SMALL_TPB) word[i] = ((uint32_t)S.bounds_tmp[i].x << ORDER_ITEM_BITS) | (uint32_t)i;
+    __syncthreads();
+    order_items<ORDER_ITEM_BITS, ORDER_ITEMS / SMALL_TPB>(S, n_items, word, hist, sh);
+}
+
+// The base plans of a small graph, and the order of their items by the largest neighbour where groups follow (jorder): a workgroup a
+// side does in one launch what the launches above and their two sorts, thirteen or seventeen of 4 us and more whatever they have to do, do for
+// larger ones, bit for bit.  Neighbours (16 bits) and sort words (key and place) stay in LDS, 57 KB, which set the limits; bound by the
+// latency of the six steps: 19 us at 5 600 edges in place of some 70 of launches.  With k_csr_small, a training pass on new graphs: 5 trees
+// of 51 leaves 725 -> 311 us, 59 of 16 in bfloat16 775 -> 357.
+constexpr int SMALL_ITEM_BITS = 12, SMALL_ITEMS = 1 << SMALL_ITEM_BITS, SMALL_EDGES = 12288;
+inline bool small_plan(const PlanSide &S) { return S.n_edges <= SMALL_EDGES && S.max_items <= SMALL_ITEMS && S.n_index_nodes <= 0xFFFF; }
+
+__global__ __launch_bounds__(SMALL_TPB) void k_plan_small(PlanSides b, int32_t *info_out) {
+    constexpr int NW = SMALL_TPB / 64;
+    const PlanSide &S = b.side[blockIdx.x];
+    const int64_t *row = S.row, *ipu = S.ipu, *eid = S.eid, *indices = S.indices;
+    const int n_units = (int)S.n_units, n_edges = (int)S.n_edges, n_rows = (int)S.n_rows, seg_len = S.seg_len, tid = threadIdx.x;
+    __shared__ uint32_t word[SMALL_ITEMS + 1];                    // the rows' starts, then the sort words
+    __shared__ uint16_t nbr[SMALL_EDGES];
+    __shared__ int32_t hist[SMALL_NW * SMALL_BINS], sh[NW + 1], err, perm;
+    int32_t *const start = reinterpret_cast<int32_t *>(word);
+    const int64_t first = n_units > 0 ? ipu[0] : 0, last = n_units > 0 ? ipu[n_units] : 0;
+    const bool covers = n_units > 0 ? first == 0 && last == n_edges : n_edges == 0;
+    if (tid == 0) {
+        err = first < 0 || last >= INT32_MAX ? 3 : last > n_edges ? 1 : 0;
+        perm = 1;
+    }
+    for (int r = tid; r <= n_rows; r += SMALL_TPB) start[r] = (int32_t)last;
+    __syncthreads();
+    // edge slots: indices to 32 bits, eid a permutation? (the check below); units: sorted? where the rows start
+#pragma unroll 4
+    for (int p = tid; p < n_edges; p += SMALL_TPB) {
+        const int64_t e = eid[p], c = indices ? indices[p] : 0;
+        const bool ok = e >= 0 && e < n_edges && c >= 0 && (!indices || c < S.n_index_nodes);
+        if (!ok) atomicMax(&err, 1);
+        S.eid32[p] = ok ? (int32_t)e : 0;
+        S.idx32[p] = ok ? (int32_t)c : 0;
+        nbr[p] = ok ? (uint16_t)c : (uint16_t)0;
+        if (ok) S.seen[e] = p;
+    }
+    for (int u = tid; u < n_units; u += SMALL_TPB) {
+        const int64_t r = row[u], before = u > 0 ? row[u - 1] : -1, at = ipu[u];
+        int bad = r < 0 || r >= n_rows ? 1 : 0;
+        if (r < before || ipu[u + 1] < at) bad = 2;
+        if (bad) atomicMax(&err, bad);
+        else if (before >= -1)
+            for (int64_t x = before + 1; x <= r; ++x) start[x] = (int32_t)at;
+    }
+    __syncthreads();
+    int32_t n_items = 0, n_heavy = 0, n_slots = 0, degree = 0;
+    if (err == 0) {
+        for (int r = tid; r <= n_rows; r += SMALL_TPB) S.rowptr[r] = start[r];
+        // items of every row in row order, the heavy rows: a run of rows a thread
+        int4 *const items = indices ? S.items_tmp : S.items;
+        const int per = (n_rows + SMALL_TPB - 1) / SMALL_TPB, r0 = min(tid * per, n_rows), r1 = min(r0 + per, n_rows);
+        auto segments = [&](int deg) { return deg > seg_len ? (deg - 1) / seg_len + 1 : 0; };
+        int32_t mine = 0, heavy = 0, slots = 0;
+        for (int r = r0; r < r1; ++r) {
+            const int deg = start[r + 1] - start[r], n = segments(deg);
+            mine += max(n, 1);
+            heavy += n > 0 ? 1 : 0;
+            slots += n;
+            degree = max(degree, deg);
+        }
+        int32_t item = block_excl_sum<NW>(mine, sh, n_items), hv = block_excl_sum<NW>(heavy, sh, n_heavy), slot = block_excl_sum<NW>(slots, sh, n_slots);
+        for (int d = 32; d > 0; d >>= 1) degree = max(degree, __shfl_xor(degree, d));
+        __syncthreads();
+        if ((tid & 63) == 0) sh[tid >> 6] = degree;
+        __syncthreads();
+        for (int w = 0; w < NW; ++w) degree = max(degree, sh[w]);
+        for (int r = r0; r < r1; ++r) {
+            const int begin = start[r], end = start[r + 1], n = segments(end - begin);
+            if (n == 0) items[item++] = make_int4(r, begin, end, -1);
+            else {
+                S.heavy[3 * hv] = r;
+                S.heavy[3 * hv + 1] = slot;
+                S.heavy[3 * hv + 2] = n;
+                ++hv;
+                for (int t = 0; t < n; ++t) items[item++] = make_int4(r, begin + t * seg_len, min(end, begin + (t + 1) * seg_len), slot++);
+            }
+        }
+        for (int p = tid; p < n_edges; p += SMALL_TPB)
+            if (S.seen[S.eid32[p]] != p) perm = 0;
+        __syncthreads();                                          // (the items are written, the rows' starts read)
+        // smallest and largest neighbour of every item, four lanes an item; an empty item: its own row id clipped to n_index_nodes
+        int2 *const bounds = indices ? S.bounds_tmp : S.bounds;
+        if (bounds)
+            for (int i = tid >> 2; i < n_items; i += SMALL_TPB / 4) {
+                int32_t lo = INT32_MAX, hi = 0;
+                const int4 it = items[i];
+                if (it.z > it.y) {
+                    for (int p = it.y + (tid & 3); p < it.z; p += 4) {
+                        lo = min(lo, (int32_t)nbr[p]);
+                        hi = max(hi, (int32_t)nbr[p]);
+                    }
+                    lo = min(lo, __shfl_xor(lo, 1, 4));
+                    hi = max(hi, __shfl_xor(hi, 1, 4));
+                    lo = min(lo, __shfl_xor(lo, 2, 4));
+                    hi = max(hi, __shfl_xor(hi, 2, 4));
+                } else {
+                    lo = hi = (int32_t)min((int64_t)it.x, S.n_index_nodes);
+                }
+                if ((tid & 3) == 0) {
+                    bounds[i] = make_int2(lo, hi);
+                    word[i] = ((uint32_t)lo << SMALL_ITEM_BITS) | (uint32_t)i;
+                }
+            }
+        if (indices) {
+            __syncthreads();
+            order_items<SMALL_ITEM_BITS, SMALL_ITEMS / SMALL_TPB>(S, n_items, word, hist, sh);
+        } else if (S.jorder && S.bounds) {                        // (no edges, and groups are asked for: the items as they are)
+            __syncthreads();
+            order_by_largest<SMALL_ITEM_BITS, SMALL_ITEMS / SMALL_TPB>(S, n_items, word, hist, sh);
+        }
+    }
+    if (tid < 16) {
+        const int32_t v = tid == BPT_PI_ERR ? err : tid == BPT_PI_N_ITEMS ? n_items : tid == BPT_PI_N_HEAVY ? n_heavy : tid == BPT_PI_N_SLOTS ? n_slots
+                          : tid == BPT_PI_MAX_DEGREE ? degree : tid == BPT_PI_FLAGS ? (covers && perm ? 1 : 0) : 0;
+        S.info[tid] = v;
+        if (info_out) info_out[16 * blockIdx.x + tid] = v;
+    }
+}
+
+// info blocks to memory that the host reads
+__global__ void k_info_out(PlanSides b, int32_t *info_out) { info_out[16 * blockIdx.x + threadIdx.x] = b.side[blockIdx.x].info[threadIdx.x]; }
 
 // Sort key of every item: smallest (LARGEST = false) or largest neighbour id; an empty item takes its own row id,
 // clipped to n_index_nodes.  Positions past n_items get the padding key, which sorts behind every real one.
@@ -1785,6 +1996,57 @@ __global__ __launch_bounds__(TPB) void k_csr_units(CsrSides g, int64_t n_edges, 
     }
 }
 
+// Both sides' CSRs of a small graph, a workgroup a side in one launch: the edges sorted in LDS by (row, edge id), what the eight
+// launches for larger graphs leave bit for bit: 15 to 17 us at 5 600 edges, in place of 40.  The limits are what LDS holds.
+constexpr int CSR_SMALL_BITS = 14, CSR_SMALL_EDGES = 10240, CSR_SMALL_NODES = 4096;
+inline bool csr_small(int64_t n_edges, int64_t n_nodes) { return n_edges <= CSR_SMALL_EDGES && n_nodes <= CSR_SMALL_NODES; }
+__global__ __launch_bounds__(SMALL_TPB) void k_csr_small(CsrSides g, int n_edges, int n_nodes, int chunk) {
+    constexpr int NW = SMALL_TPB / 64;
+    const CsrSide &c = g.side[blockIdx.x];
+    __shared__ uint32_t word[CSR_SMALL_EDGES];
+    __shared__ int32_t start[CSR_SMALL_NODES + 1], sh[NW + 1];       // (start: before it is one, the sort's counts)
+    static_assert(SMALL_NW * SMALL_BINS <= CSR_SMALL_NODES + 1, "the counts fit");
+    const int tid = threadIdx.x;
+    bool bad = false;
+#pragma unroll 4
+    for (int e = tid; e < n_edges; e += SMALL_TPB) {
+        const int64_t r = c.rows[e], k = c.cols[e];
+        const bool ok = r >= 0 && r < n_nodes && k >= 0 && k < n_nodes;
+        bad = bad || !ok;
+        word[e] = ((uint32_t)(ok ? r : n_nodes) << CSR_SMALL_BITS) | (uint32_t)e;
+    }
+    const int any_bad = __syncthreads_or(bad ? 1 : 0);
+    lds_radix<CSR_SMALL_EDGES / SMALL_TPB>(word, n_edges, CSR_SMALL_BITS, 32 - __clz(n_nodes | 1), start, sh);
+    // slots, and where the rows start: a slot whose row is not the one before's starts the rows in between too
+    for (int at = tid; at < n_edges; at += SMALL_TPB) {
+        const uint32_t w = word[at];
+        const int e = (int)(w & ((1 << CSR_SMALL_BITS) - 1)), r = (int)(w >> CSR_SMALL_BITS), before = at > 0 ? (int)(word[at - 1] >> CSR_SMALL_BITS) : -1;
+        c.eid[at] = e;
+        c.indices[at] = c.cols[e];
+        for (int x = before + 1; x <= r; ++x) start[x] = at;
+    }
+    const int from = n_edges > 0 ? (int)(word[n_edges - 1] >> CSR_SMALL_BITS) + 1 : 0;
+    for (int x = from + tid; x <= n_nodes; x += SMALL_TPB) start[x] = n_edges;
+    __syncthreads();
+    for (int r = tid; r <= n_nodes; r += SMALL_TPB) c.indptr[r] = start[r];
+    // the units of builder.pyx:305-321: a run of rows a thread
+    const int per = (n_nodes + SMALL_TPB - 1) / SMALL_TPB, r0 = min(tid * per, n_nodes), r1 = min(r0 + per, n_nodes);
+    auto units_of = [&](int r) { return (start[r + 1] - start[r] + chunk - 1) / chunk; };
+    int32_t units = 0, total;
+    for (int r = r0; r < r1; ++r) units += units_of(r);
+    int32_t at = block_excl_sum<NW>(units, sh, total);
+    for (int r = r0; r < r1; ++r)
+        for (int u = 0, n = units_of(r); u < n; ++u, ++at) {
+            c.unit_row[at] = r;
+            c.unit_ptr[at] = start[r] + (int64_t)u * chunk;
+        }
+    if (tid == 0) {
+        c.info[0] = any_bad ? 1 : 0;
+        c.info[1] = total;
+        c.unit_ptr[total] = n_edges;
+    }
+}
+
 struct CsrWs {
     uint32_t *key[2];
     int32_t *val[2];
@@ -1938,8 +2200,22 @@ template <typename F> int64_t most_of(const PlanSides &b, int n_sides, F &&f) {
     return x > y ? x : y;
 }
 
+inline bool small_plans(const PlanSides &b, int n_sides) { return small_plan(b.side[0]) && (n_sides < 2 || small_plan(b.side[1])); }
+
+// base_build leaves both orders of the items
+inline bool ordered_plans(const PlanSides &b, int n_sides) {
+    bool fit = true;
+    for (int i = 0; i < n_sides; ++i) fit = fit && b.side[i].indices && order_in_lds(b.side[i]);
+    return fit || small_plans(b, n_sides);
+}
+
 int base_build(const PlanSides &b, int n_sides, const SortWs &w, hipStream_t s) {
     const unsigned ns = (unsigned)n_sides;
+    if (small_plans(b, n_sides)) {
+        hipLaunchKernelGGL(k_plan_small, dim3(ns), dim3(SMALL_TPB), 0, s, b, (int32_t *)nullptr);
+        HIP_TRY(hipGetLastError());
+        return BPT_OK;
+    }
     hipLaunchKernelGGL(k_plan_clear, dim3(1, ns), dim3(64), 0, s, b);
     HIP_TRY(hipGetLastError());
     const unsigned edge_blocks = blocks_for(most_of(b, n_sides, [](const PlanSide &S) { return S.n_edges; }));
@@ -1955,18 +2231,24 @@ int base_build(const PlanSides &b, int n_sides, const SortWs &w, hipStream_t s) 
     hipLaunchKernelGGL(k_item_bounds, dim3(blocks_for(max_items * 16), ns), dim3(TPB), 0, s, b);
     HIP_TRY(hipGetLastError());
     if (!sorted) return BPT_OK;
+    if (ordered_plans(b, n_sides)) {
+        hipLaunchKernelGGL(k_item_order, dim3(ns), dim3(SMALL_TPB), 0, s, b);
+        HIP_TRY(hipGetLastError());
+        return BPT_OK;
+    }
     const int64_t pad = most_of(b, n_sides, [](const PlanSide &S) { return S.n_index_nodes; }) + 1;
     return rs_sort(ItemRecs{b, 0}, ItemsSorted{b}, RsSizes{{b.side[0].max_items, b.side[1].max_items}}, n_sides, (uint64_t)pad, w.key, w.val, w.counts,
                    w.totals, s);
 }
 
-int groups_count(const PlanSides &b, int n_sides, int32_t R, const SortWs &w, hipStream_t s) {
+// ordered: base_build has left the items' order by the largest neighbour (jorder)
+int groups_count(const PlanSides &b, int n_sides, int32_t R, const SortWs &w, hipStream_t s, bool ordered = false) {
     const unsigned ns = (unsigned)n_sides;
     const int64_t max_items = most_of(b, n_sides, [](const PlanSide &S) { return S.max_items; });
     if (max_items > 0) {
         // the items in the order of their largest neighbour; R consecutive ones are a group
         const int64_t n_index = most_of(b, n_sides, [](const PlanSide &S) { return S.n_index_nodes; });
-        const int st = rs_sort(ItemRecs{b, 1}, ItemOrder{b}, RsSizes{{b.side[0].max_items, b.side[1].max_items}}, n_sides, (uint64_t)n_index + 1, w.key,
+        const int st = ordered ? BPT_OK : rs_sort(ItemRecs{b, 1}, ItemOrder{b}, RsSizes{{b.side[0].max_items, b.side[1].max_items}}, n_sides, (uint64_t)n_index + 1, w.key,
                                w.val, w.counts, w.totals, s);
         if (st != BPT_OK) return st;
         const int64_t place_bits = most_of(b, n_sides, [](const PlanSide &S) { return S.place_bits; });
@@ -2025,6 +2307,11 @@ int csr_build(CsrSides g, int n_sides, int64_t n_edges, int64_t n_nodes, int32_t
     Bump bump{(char *)workspace, 0};
     CsrWs w = csr_layout(bump, n_edges, n_nodes, n_sides, g);
     if (workspace_bytes < (int64_t)bump.off) return BPT_ERR_WORKSPACE;
+    if (csr_small(n_edges, n_nodes)) {
+        hipLaunchKernelGGL(k_csr_small, dim3((unsigned)n_sides), dim3(SMALL_TPB), 0, s, g, (int)n_edges, (int)n_nodes, chunk);
+        HIP_TRY(hipGetLastError());
+        return BPT_OK;
+    }
     // (n_nodes: the key of an edge with a bad id)
     const int st = rs_sort(CsrEdges{g, n_nodes}, CsrSlots{g}, RsSizes{{n_edges, n_edges}}, n_sides, (uint64_t)n_nodes, w.key, w.val, w.counts,
                            w.totals, s);
@@ -2259,6 +2546,60 @@ int bpt_build_groups_write(const int32_t *items, const int32_t *plan_info, int64
     return groups_write(b, 1, R, group_counts, &out, pad_entries, (hipStream_t)stream);
 }
 
+// where the call below puts the sides' arrays in its workspace
+static int base_sides(const bpt_build_side *sides, int n_sides, PlanSides &b, SortWs &w, Bump &bump) {
+    int64_t most = 0;
+    for (int i = 0; i < n_sides; ++i) {
+        const bpt_build_side &side = sides[i];
+        PlanSide &S = b.side[i];
+        const int st = sizes_ok(side.n_units, side.n_edges, side.n_rows, side.n_index_nodes, side.seg_len);
+        if (st != BPT_OK) return st;
+        S.n_edges = side.n_edges;
+        S.n_rows = side.n_rows;
+        S.max_items = side.n_rows + side.n_edges / side.seg_len;
+        if (S.max_items >= INT32_MAX) return BPT_ERR_SIZE;
+        base_layout(bump, S);
+        most = S.max_items > most ? S.max_items : most;
+    }
+    w = sort_layout(bump, most, n_sides);
+    return BPT_OK;
+}
+
+int bpt_build_plans_bounds(const bpt_build_side *sides, int n_sides, int64_t bounds[1]) {
+    if (!sides || !bounds || n_sides < 1 || n_sides > 2) return BPT_ERR_NULL;
+    PlanSides b{};
+    SortWs w;
+    Bump dry{nullptr, 0};
+    const int st = base_sides(sides, n_sides, b, w, dry);
+    bounds[0] = (int64_t)dry.off + 256;
+    return st;
+}
+
+int bpt_build_plans(const bpt_build_side *sides, int n_sides, int32_t *out_info, void *workspace, int64_t workspace_bytes, void *stream) {
+    if (!sides || !out_info || !workspace || n_sides < 1 || n_sides > 2) return BPT_ERR_NULL;
+    PlanSides b{};
+    SortWs w;
+    Bump bump{(char *)workspace, 0};
+    int st = base_sides(sides, n_sides, b, w, bump);
+    if (st != BPT_OK) return st;
+    if (workspace_bytes < (int64_t)bump.off) return BPT_ERR_WORKSPACE;
+    for (int i = 0; i < n_sides; ++i) {
+        st = fill_side(sides[i], b.side[i]);
+        if (st != BPT_OK) return st;
+        if (!sides[i].indices && sides[i].n_edges > 0) return BPT_ERR_NULL;
+    }
+    hipStream_t s = (hipStream_t)stream;
+    if (small_plans(b, n_sides)) {
+        hipLaunchKernelGGL(k_plan_small, dim3((unsigned)n_sides), dim3(SMALL_TPB), 0, s, b, out_info);
+    } else {
+        st = base_build(b, n_sides, w, s);
+        if (st != BPT_OK) return st;
+        hipLaunchKernelGGL(k_info_out, dim3((unsigned)n_sides), dim3(16), 0, s, b, out_info);
+    }
+    HIP_TRY(hipGetLastError());
+    return BPT_OK;
+}
+
 // where the two calls below put a side's arrays in its part of the workspace
 static int tiles_sides(const bpt_build_side *sides, int n_sides, PlanSides &b, SortWs &w, Bump &bump) {
     int64_t most = 0;
@@ -2310,7 +2651,7 @@ int bpt_build_tiles_count(const bpt_build_side *sides, int n_sides, int32_t *out
     if (workspace_bytes < (int64_t)bump.off) return BPT_ERR_WORKSPACE;
     for (int i = 0; i < n_sides; ++i) b.side[i].out_info = out_info + 32 * i;
     st = base_build(b, n_sides, w, (hipStream_t)stream);
-    return st != BPT_OK ? st : groups_count(b, n_sides, 16, w, (hipStream_t)stream);
+    return st != BPT_OK ? st : groups_count(b, n_sides, 16, w, (hipStream_t)stream, ordered_plans(b, n_sides));
 }
 
 int bpt_build_tiles_write(const bpt_build_side *sides, int n_sides, const int32_t *infos, const bpt_build_tiles *out, int32_t pad_entries,

@@ -514,6 +514,26 @@ class DevicePlan:
         plans[0]._wait()                                  # (the last kernels ran beside all this)
         return plans
 
+    @classmethod
+    def base_plans(cls, sides):
+        """The plans, without groups, of one side of a graph or of both, built together (bpt_build_plans in bptop.so).  sides: (row, indptr,
+        eid, indices, n_rows, n_index_nodes, seg_len).  None where they have to be built one by one."""
+        from ._native import native
+        built = native.build_plans([tuple(side) for side in sides])
+        if built is None:
+            return None
+        plans = []
+        for (row, indptr, eid, indices, n_rows, n_index_nodes, seg_len), (info, base) in zip(sides, built):
+            self = cls.__new__(cls)
+            self.device, self.seg_len, self.has_indices = eid.device, int(seg_len), True
+            self.n_rows, self.n_edges, self.n_index_nodes = int(n_rows), int(eid.numel()), int(n_index_nodes)
+            self._groups, self._links, self._bias_rows, self._lock = {}, {}, {}, threading.Lock()
+            self._max_items, self._info = self.n_rows + self.n_edges // self.seg_len, base[6]
+            self._dev = dict(zip(("rowptr", "idx", "eid", "items", "bounds", "heavy"), base))
+            self._describe(info)
+            plans.append(self)
+        return plans
+
     def _describe(self, h):
         """The plan's numbers and its struct from the info block that came back."""
         if h[0] != 0:
@@ -860,8 +880,22 @@ class PlanCache:
             built_of = [(*side[:6], seg_len, side[7]) for side, seg_len in zip(sides, seg_lens)]
         else:
             built_of = sides
+        return self._put(keys, sides, DevicePlan.tile_plans, built_of)
+
+    def put_plans(self, sides):
+        """The same for the plans, without groups and with work items of the default length, of a graph too small for tiles.  sides: (row,
+        indptr, eid, indices, n_rows, n_index_nodes) of the in-side, then of the out-side."""
+        if self.native is None or DEVICE_BUILD is not None or not sides[0][2].is_cuda or any(side[4] >= 8 * 3072 for side in sides):
+            return None                             # (longer graphs: the length is chosen by a look at the rows)
+        keys = [self._key(side[:4], side[4], side[5], DEFAULT_SEG_LEN, True) for side in sides]
+        with self._lock:
+            if any(key in self._d for key in keys):
+                return None
+        return self._put(keys, sides, DevicePlan.base_plans, [(*side, 64 if FORCE_SEG_LEN is None else FORCE_SEG_LEN) for side in sides])
+
+    def _put(self, keys, sides, build, built_of):
         try:
-            plans = DevicePlan.tile_plans(built_of)
+            plans = build(built_of)
         except ValueError:
             plans = None
         if plans is None:

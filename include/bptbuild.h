@@ -69,6 +69,11 @@ int bpt_build_tiles_count(const bpt_build_side *sides, int n_sides, int32_t *out
 int bpt_build_tiles_write(const bpt_build_side *sides, int n_sides, const int32_t *infos, const bpt_build_tiles *out,
                           int32_t pad_entries, int32_t *pairs, void *workspace, int64_t workspace_bytes, void *stream);
 
+/* The base plans alone of one or two sides, with indices: out_info int32[16] per side (their info blocks), in memory the device can write;
+ * by_mask is not read, item_bounds may be NULL.  bpt_build_plans_bounds: workspace bytes, from the sizes alone. */
+int bpt_build_plans_bounds(const bpt_build_side *sides, int n_sides, int64_t bounds[1]);
+int bpt_build_plans(const bpt_build_side *sides, int n_sides, int32_t *out_info, void *workspace, int64_t workspace_bytes, void *stream);
+
 /* For every (entry, member) of one side's groups (grp_eids_mine, n_slots) the number of the same edge's pair on the other side
  * (pair_eid_theirs, n_edges), 0 where there is none.  number: n_edges int32 of scratch. */
 int bpt_build_pair_numbers(const int32_t *pair_eid_theirs, const int32_t *grp_eids_mine, int64_t n_slots, int64_t n_edges,
