@@ -4957,30 +4957,69 @@ __global__ __launch_bounds__(HW * WAVE) void k_rel_bias_tiles(bpt_plan P, const 
 // in flight while one is used, and their types and edge ids two items ahead of that, so that no wait (they are in order) includes a
 // load that has just left.  A launch has a wavefront for every item up to 512 workgroups.  Against a walk that took one slot after the other
 // on the vector pipeline, with one item's loads ahead and a workgroup for 512 edges, kernel alone: 8 heads float32 L = 8192, k = 4 45.5 -> 39.5 us
-// (30.7 of them without any of the products: 132 MB take 26 at the rate of a copy), k = 8 both ways 297 -> 189, L = 100 25.7 -> 8.0; 16 heads
-// L = 4096, k = 16 186 -> 119; bfloat16 8 heads L = 32768, k = 2 177 -> 116, 16 heads L = 2048 57 -> 24, 666 nodes 136 -> 14; 4 heads L = 1024 20 -> 14,
+// (30.7 of them without any of the products: 132 MB take 26 at the rate of a copy), k = 8 both ways 297 -> 180, L = 100 25.7 -> 8.0; 16 heads
+// L = 4096, k = 16 186 -> 107; bfloat16 8 heads L = 32768, k = 2 177 -> 116, 16 heads L = 2048 57 -> 24, 666 nodes 136 -> 14; 4 heads L = 1024 20 -> 14,
 // L = 16384, k = 2 48 -> 49.5, the one shape that gained nothing.  Neighbouring items in neighbouring wavefronts, for the lines that
 // their ds values share: 39.5 -> 42.
-template <int H>
-struct RelBody {
-    float d[H];              // ds of the lane's slot
-    float4 q[H / 4], old[H / 4];      // columns 4 c .. 4 c + 3 of heads 4 s + g: q, and the dq row that a whole row adds to
+// CS = 2: two wavefronts take an item together, each half of the columns of q, dq and the sums (rel_bwd_shape says when).
+// NB (4 or 2) neighbouring columns of a lane: of q or dq, which start on any element here (attention itself asks for 16 bytes), and of the rows in LDS
+template <int NB>
+struct RelCols {
+    float v[NB];
 };
-// four columns of q or dq, which start on any element here (attention itself asks for 16 bytes)
-typedef uint32_t uintx2e __attribute__((ext_vector_type(2), aligned(2)));
-template <typename T> __device__ __forceinline__ float4 rel_load4(const T *p) {
+template <int NB, typename T> __device__ __forceinline__ RelCols<NB> rel_load(const T *p) {
+    RelCols<NB> y;
     if constexpr (sizeof(T) == 4) {
-        const floatx4u x = *reinterpret_cast<const floatx4u *>(p);
-        return make_float4(x[0], x[1], x[2], x[3]);
+        typedef float floatxu __attribute__((ext_vector_type(NB), aligned(4)));
+        const floatxu x = *reinterpret_cast<const floatxu *>(p);
+#pragma unroll
+        for (int i = 0; i < NB; ++i) y.v[i] = x[i];
     } else {
-        const uintx2e x = *reinterpret_cast<const uintx2e *>(p);
-        return make_float4(__uint_as_float(x[0] << 16), __uint_as_float(x[0] & 0xffff0000u), __uint_as_float(x[1] << 16), __uint_as_float(x[1] & 0xffff0000u));
+        typedef uint32_t uintxe __attribute__((ext_vector_type(NB / 2), aligned(2)));
+        const uintxe x = *reinterpret_cast<const uintxe *>(p);
+#pragma unroll
+        for (int i = 0; i < NB / 2; ++i) {
+            y.v[2 * i] = __uint_as_float(x[i] << 16);
+            y.v[2 * i + 1] = __uint_as_float(x[i] & 0xffff0000u);
+        }
+    }
+    return y;
+}
+template <int NB, typename T> __device__ __forceinline__ void rel_store(T *p, const RelCols<NB> &y) {
+    if constexpr (sizeof(T) == 4) {
+        typedef float floatxu __attribute__((ext_vector_type(NB), aligned(4)));
+        floatxu x;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) x[i] = y.v[i];
+        *reinterpret_cast<floatxu *>(p) = x;
+    } else {
+        typedef uint32_t uintxe __attribute__((ext_vector_type(NB / 2), aligned(2)));
+        uintxe x;
+#pragma unroll
+        for (int i = 0; i < NB / 2; ++i) x[i] = pack_bf16(y.v[2 * i], y.v[2 * i + 1]);
+        *reinterpret_cast<uintxe *>(p) = x;
     }
 }
-template <typename T> __device__ __forceinline__ void rel_store4(T *p, float4 v) {
-    if constexpr (sizeof(T) == 4) *reinterpret_cast<floatx4u *>(p) = floatx4u{v.x, v.y, v.z, v.w};
-    else *reinterpret_cast<uintx2e *>(p) = uintx2e{pack_bf16(v.x, v.y), pack_bf16(v.z, v.w)};
+template <int NB> __device__ __forceinline__ RelCols<NB> rel_row_load(const float *p) {        // (p: a multiple of NB floats)
+    typedef float floatx __attribute__((ext_vector_type(NB)));
+    const floatx x = *reinterpret_cast<const floatx *>(p);
+    RelCols<NB> y;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) y.v[i] = x[i];
+    return y;
 }
+template <int NB> __device__ __forceinline__ void rel_row_store(float *p, const RelCols<NB> &y) {
+    typedef float floatx __attribute__((ext_vector_type(NB)));
+    floatx x;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) x[i] = y.v[i];
+    *reinterpret_cast<floatx *>(p) = x;
+}
+template <int H, int NB>
+struct RelBody {
+    float d[H];              // ds of the lane's slot
+    RelCols<NB> q[H / 4], old[H / 4]; // the lane's columns of heads 4 s + g: q, and the dq row that a whole row adds to
+};
 // the H values of ds that belong to `edge`: of a row of (n_edges, H), or one of each head's n_edges values
 struct RelStride {
     uint32_t edge, head;
@@ -4991,40 +5030,42 @@ template <int H> __device__ __forceinline__ void rel_ds_load(const float *__rest
 }
 // (No load stands behind a condition: where paths meet, the waits count for the one with the fewest loads.  An item without edges reads
 // places that are there, and a segment its row's dq.)
-template <typename T, int H>
+template <typename T, int H, int NB>
 __device__ __forceinline__ void rel_body_load(const RelHead &r, const float *__restrict__ ds, RelStride by, const T *__restrict__ q,
-                                              const T *__restrict__ dq, int lane, RelBody<H> &y) {
+                                              const T *__restrict__ dq, int g, int col, RelBody<H, NB> &y) {
     constexpr int D = 64;
-    const int c = lane & 15, g = lane >> 4;
     rel_ds_load<H>(ds, r.edge, by, y.d);
 #pragma unroll
-    for (int s = 0; s < H / 4; ++s) y.q[s] = rel_load4<T>(q + ((size_t)r.row * H + 4 * s + g) * D + 4 * c);
+    for (int s = 0; s < H / 4; ++s) y.q[s] = rel_load<NB, T>(q + ((size_t)r.row * H + 4 * s + g) * D + col);
 #pragma unroll
-    for (int s = 0; s < H / 4; ++s) y.old[s] = rel_load4<T>(dq + ((size_t)r.row * H + 4 * s + g) * D + 4 * c);
+    for (int s = 0; s < H / 4; ++s) y.old[s] = rel_load<NB, T>(dq + ((size_t)r.row * H + 4 * s + g) * D + col);
 }
-__device__ __forceinline__ void rel_add4(float *at, float x, float y, float z, float w) {
-    float4 v = *reinterpret_cast<const float4 *>(at);
-    v.x += x; v.y += y; v.z += z; v.w += w;
-    *reinterpret_cast<float4 *>(at) = v;
+template <int NB> __device__ __forceinline__ void rel_add(float *at, const RelCols<NB> &x) {
+    RelCols<NB> v = rel_row_load<NB>(at);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) v.v[i] += x.v[i];
+    rel_row_store<NB>(at, v);
 }
-template <typename T, int H, int NW>
-__global__ __launch_bounds__(NW * WAVE) void k_rel_bias_bwd(bpt_plan P, const float *__restrict__ ds, const T *__restrict__ q,
+template <typename T, int H, int NW, int CS>
+__global__ __launch_bounds__(NW * CS * WAVE) void k_rel_bias_bwd(bpt_plan P, const float *__restrict__ ds, const T *__restrict__ q,
                                                             const T *__restrict__ table, const int32_t *__restrict__ used_types, int n_used,
                                                             T *__restrict__ dq, float *__restrict__ ws_dq, float *__restrict__ part) {
-    constexpr int D = 64, C = H * D, PITCH = REL_STAGE_PITCH;
+    constexpr int D = 64, C = H * D, PITCH = REL_STAGE_PITCH, NB = 4 / CS;
     extern __shared__ float rel_lds[];                    // NW tables of n_used x 64 sums, the table rows in use, per wavefront 64 x H staged ds values and 64 types
-    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), c = lane & 15, g = lane >> 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), c = lane & 15, g = lane >> 4;
+    const int w = wave / CS, col = (wave % CS) * (D / CS) + NB * c;       // whose items; the lane's first column
     const RelStride by = P.bias_by_pair != 0 ? RelStride{1u, (uint32_t)P.n_edges} : RelStride{(uint32_t)H, 1u};
     float *acc = rel_lds + (size_t)w * n_used * D;
     const float *rows = rel_lds + (size_t)NW * n_used * D;
-    float *stage = rel_lds + (size_t)(NW + 1) * n_used * D + (size_t)w * REL_BWD_STAGE(H);
+    float *stage = rel_lds + (size_t)(NW + 1) * n_used * D + (size_t)wave * REL_BWD_STAGE(H);
     int *types = reinterpret_cast<int *>(stage + PITCH * H);
-    // wavefront gw of GW takes the items gw, gw + GW, ...: the segments of a long row, which are neighbours, go to different wavefronts
+    // wavefront (CS > 1: the CS wavefronts) gw of GW takes the items gw, gw + GW, ...: the segments of a long row, which are neighbours, go to
+    // different ones
     const int GW = (int)gridDim.x * NW, i0 = (int)blockIdx.x * NW + w, n_items = (int)P.n_items, n_mine = i0 < n_items ? (n_items - i0 + GW - 1) / GW : 0;
     const int4 *items = reinterpret_cast<const int4 *>(P.items);
     RelHead hd[4];
-    RelBody<H> bd[2];
-    auto body = [&](const RelHead &r, RelBody<H> &y) { rel_body_load<T, H>(r, ds, by, q, dq, lane, y); };
+    RelBody<H, NB> bd[2];
+    auto body = [&](const RelHead &r, RelBody<H, NB> &y) { rel_body_load<T, H, NB>(r, ds, by, q, dq, g, col, y); };
     // ds and types of up to 64 slots (past the end: zeros; negative types, no two alike)
     auto put = [&](int cnt, const float (&d)[H], int type) {
 #pragma unroll
@@ -5033,7 +5074,7 @@ __global__ __launch_bounds__(NW * WAVE) void k_rel_bias_bwd(bpt_plan P, const fl
         wave_lds_fence();
     };
     // sixteen slots of those, cnt of them exist
-    auto sixteen = [&](int j, int cnt, const float4 (&qr)[H / 4], floatx4v (&dqa)[4]) {
+    auto sixteen = [&](int j, int cnt, const RelCols<NB> (&qr)[H / 4], floatx4v (&dqa)[NB]) {
         const int4 t4 = *reinterpret_cast<const int4 *>(types + j + 4 * g);               // of slots 4 g .. 4 g + 3
         const int ty[4] = {t4.x, t4.y, t4.z, t4.w}, mine = types[j + c];
         // row c of the product is head 4 (c % 4) + c / 4, so that register s of lane group g is head 4 s + g
@@ -5042,11 +5083,11 @@ __global__ __launch_bounds__(NW * WAVE) void k_rel_bias_bwd(bpt_plan P, const fl
         float d[H / 4];
 #pragma unroll
         for (int s = 0; s < H / 4; ++s) d[s] = stage[(4 * s + g) * PITCH + j + c];
-        float4 tv[4], before[4];                                  // table rows of those slots; the sums of their types so far
+        RelCols<NB> tv[4], before[4];                             // table rows of those slots; the sums of their types so far
 #pragma unroll
-        for (int r = 0; r < 4; ++r) tv[r] = *reinterpret_cast<const float4 *>(rows + max(ty[r], 0) * D + 4 * c);
+        for (int r = 0; r < 4; ++r) tv[r] = rel_row_load<NB>(rows + max(ty[r], 0) * D + col);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) before[r] = *reinterpret_cast<const float4 *>(acc + max(ty[r], 0) * D + 4 * c);
+        for (int r = 0; r < 4; ++r) before[r] = rel_row_load<NB>(acc + max(ty[r], 0) * D + col);
         // slots of one type: lane (c, g) compares the type of slot c with those of slots 4 g + s
         bool twice = false;
         uint64_t same0 = 0;
@@ -5057,48 +5098,50 @@ __global__ __launch_bounds__(NW * WAVE) void k_rel_bias_bwd(bpt_plan P, const fl
             if (s == 0) same0 = __builtin_amdgcn_ballot_w64(same);
         }
         issue_loads_first();                                      // (one round trip through LDS after the types', not one a product)
-        floatx4v u[4];
+        floatx4v u[NB];
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) u[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
+        for (int nb = 0; nb < NB; ++nb) u[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int s = 0; s < H / 4; ++s) {
-            u[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[s], qr[s].x, u[0], 0, 0, 0);
-            u[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[s], qr[s].y, u[1], 0, 0, 0);
-            u[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[s], qr[s].z, u[2], 0, 0, 0);
-            u[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[s], qr[s].w, u[3], 0, 0, 0);
-        }
+        for (int s = 0; s < H / 4; ++s)
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            dqa[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[s], tv[s].x, dqa[0], 0, 0, 0);
-            dqa[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[s], tv[s].y, dqa[1], 0, 0, 0);
-            dqa[2] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[s], tv[s].z, dqa[2], 0, 0, 0);
-            dqa[3] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[s], tv[s].w, dqa[3], 0, 0, 0);
-        }
+            for (int nb = 0; nb < NB; ++nb) u[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(d[s], qr[s].v[nb], u[nb], 0, 0, 0);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) dqa[nb] = __builtin_amdgcn_mfma_f32_16x16x4f32(a4[s], tv[s].v[nb], dqa[nb], 0, 0, 0);
+        auto slot = [&](int r) {                                  // what slot 4 g + r adds to its type's sums
+            RelCols<NB> x;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) x.v[nb] = u[nb][r];
+            return x;
+        };
         if (__builtin_amdgcn_ballot_w64(twice) == 0) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (ty[r] >= 0)
-                    *reinterpret_cast<float4 *>(acc + ty[r] * D + 4 * c) =
-                        make_float4(before[r].x + u[0][r], before[r].y + u[1][r], before[r].z + u[2][r], before[r].w + u[3][r]);
-        } else if ((int)__popcll(same0 & 0xffffu) == cnt) {       // every slot that exists has the first one's type (those past the end add nothing)
-            float x[4];
+            for (int r = 0; r < 4; ++r) {
+                RelCols<NB> x = slot(r);
 #pragma unroll
-            for (int nb = 0; nb < 4; ++nb) x[nb] = groups_sum((u[nb][0] + u[nb][1]) + (u[nb][2] + u[nb][3]));
-            if (g == 0) rel_add4(acc + ty[0] * D + 4 * c, x[0], x[1], x[2], x[3]);
+                for (int nb = 0; nb < NB; ++nb) x.v[nb] = before[r].v[nb] + x.v[nb];
+                if (ty[r] >= 0) rel_row_store<NB>(acc + ty[r] * D + col, x);
+            }
+        } else if ((int)__popcll(same0 & 0xffffu) == cnt) {       // every slot that exists has the first one's type (those past the end add nothing)
+            RelCols<NB> x;
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) x.v[nb] = groups_sum((u[nb][0] + u[nb][1]) + (u[nb][2] + u[nb][3]));
+            if (g == 0) rel_add<NB>(acc + ty[0] * D + col, x);
         } else {
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 for (int gg = 0; gg < 4; ++gg) {
-                    if (g == gg && ty[r] >= 0) rel_add4(acc + ty[r] * D + 4 * c, u[0][r], u[1][r], u[2][r], u[3][r]);
+                    if (g == gg && ty[r] >= 0) rel_add<NB>(acc + ty[r] * D + col, slot(r));
                     wave_lds_fence();
                 }
         }
         wave_lds_fence();                                         // (read before the next are staged, and written before they are added)
     };
-    auto item = [&](const RelHead &cur, const RelBody<H> &b) {
-        floatx4v dqa[4];
+    auto item = [&](const RelHead &cur, const RelBody<H, NB> &b) {
+        floatx4v dqa[NB];
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) dqa[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
+        for (int nb = 0; nb < NB; ++nb) dqa[nb] = floatx4v{0.f, 0.f, 0.f, 0.f};
         if (cur.b < cur.e) put(min(WAVE, cur.e - cur.b), b.d, cur.type);
         for (int p0 = cur.b; p0 < cur.e; p0 += TILE_R) {
             const int at = p0 - cur.b;
@@ -5113,10 +5156,12 @@ __global__ __launch_bounds__(NW * WAVE) void k_rel_bias_bwd(bpt_plan P, const fl
         if (cur.out_slot >= 0 || cur.b < cur.e) {
 #pragma unroll
             for (int s = 0; s < H / 4; ++s) {
-                const int at = (4 * s + g) * D + 4 * c;
-                const float4 x = make_float4(dqa[0][s], dqa[1][s], dqa[2][s], dqa[3][s]), o = b.old[s];
-                if (cur.out_slot < 0) rel_store4<T>(dq + (size_t)cur.row * C + at, make_float4(o.x + x.x, o.y + x.y, o.z + x.z, o.w + x.w));
-                else *reinterpret_cast<float4 *>(ws_dq + (size_t)cur.out_slot * C + at) = x;
+                const int at = (4 * s + g) * D + col;
+                RelCols<NB> x;
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) x.v[nb] = cur.out_slot < 0 ? b.old[s].v[nb] + dqa[nb][s] : dqa[nb][s];
+                if (cur.out_slot < 0) rel_store<NB, T>(dq + (size_t)cur.row * C + at, x);
+                else rel_row_store<NB>(ws_dq + (size_t)cur.out_slot * C + at, x);
             }
         }
     };
@@ -5139,7 +5184,7 @@ __global__ __launch_bounds__(NW * WAVE) void k_rel_bias_bwd(bpt_plan P, const fl
     };
     begin(0);
     issue_loads_first();                                          // (on their way while the table rows are fetched)
-    for (int u = 0; u < n_used; ++u) acc[u * D + lane] = 0.f;
+    for (int u = wave % CS; u < n_used; u += CS) acc[u * D + lane] = 0.f;
     rel_table_to_lds<T>(table, used_types, n_used, rel_lds + (size_t)NW * n_used * D, D);
     __syncthreads();
     for (int first = 0; first < n_mine; first += WAVE) {
@@ -5156,7 +5201,7 @@ __global__ __launch_bounds__(NW * WAVE) void k_rel_bias_bwd(bpt_plan P, const fl
         }
     }
     __syncthreads();
-    for (int u = w; u < n_used; u += NW) {
+    for (int u = wave; u < n_used; u += NW * CS) {
         float sum = rel_lds[(size_t)u * D + lane];
 #pragma unroll
         for (int x = 1; x < NW; ++x) sum += rel_lds[((size_t)x * n_used + u) * D + lane];
@@ -5515,19 +5560,31 @@ inline bool rel_rows_shape(int h, int d, int dtype) {
 constexpr int REL_MAX_PARTS = 512;        // partial tables of the gradient kernel: two workgroups per compute unit
 constexpr int REL_MAX_USED = 240;         // type numbers whose table rows fit the 64 KB of LDS of the score kernel
 
-// LDS of k_rel_bias_bwd with nw wavefronts: their sums, the table rows, their staged ds values and types
-inline size_t rel_bwd_lds(int nw, int64_t n_used, int h) { return ((size_t)(nw + 1) * n_used * 64 + (size_t)nw * REL_BWD_STAGE(h)) * 4; }
-// wavefronts per workgroup of k_rel_bias_bwd for n_used types: the 4, 2 or 1 that put most wavefronts on a compute unit
-// (workgroups that fit its 160 KB of LDS x wavefronts each; more per workgroup on a tie: fewer partial tables), a
-// workgroup taking at most 144 KB (large_lds false: at most the 64 KB every kernel may take).  0: no configuration fits.
-inline int rel_bwd_waves(int64_t n_used, int h, bool large_lds = true) {
+// LDS of k_rel_bias_bwd with nw tables of sums of cs wavefronts each: the sums, the table rows, the wavefronts' staged ds values and types
+inline size_t rel_bwd_lds(int nw, int cs, int64_t n_used, int h) { return ((size_t)(nw + 1) * n_used * 64 + (size_t)nw * cs * REL_BWD_STAGE(h)) * 4; }
+// How k_rel_bias_bwd is launched for n_used types: a workgroup of nw (4, 2 or 1) tables of sums, cs wavefronts (1 or 2) sharing the columns of each.
+struct RelBwdShape {
+    int nw, cs;
+};
+// One wavefront a table where that puts eight on a compute unit (workgroups that fit its 160 KB of LDS x wavefronts each; more tables per
+// workgroup on a tie: fewer partial tables), which holds up to 62 types; else the shape with most of them.  Two wavefronts a table read and stage
+// an item's ds and types twice: at 48 types, where LDS holds eight either way, 39.5 against 39.6 us (8 heads, L = 8192, k = 4), at 55
+// 113 against 123 (bfloat16, L = 32768, k = 2).  Where it holds two or four: 173 types (8 heads, L = 8192, k = 8 both ways) 180 -> 142 us, 140 (4
+// heads, L = 6215, k = 6 both ways) 98 -> 76, 134 (16 heads bfloat16, a batch with k = 20) 124 -> 107; 16 heads, L = 4096, k = 16 level.  Four a
+// table: 77, 130 and 138 in the last three places.
+// A workgroup takes at most 144 KB (large_lds false: at most the 64 KB every kernel may take).  nw 0: no configuration fits.
+inline RelBwdShape rel_bwd_shape(int64_t n_used, int h, bool large_lds = true) {
     const size_t cap = (large_lds ? 144 : 64) * 1024;
-    int best = 0, best_waves = 0;
-    for (int nw = 4; nw >= 1; nw >>= 1) {
-        const size_t lds = rel_bwd_lds(nw, n_used, h);
-        if (lds > cap) continue;
-        const int waves = nw * (int)((160 * 1024) / lds);
-        if (waves > best_waves) { best = nw; best_waves = waves; }
+    RelBwdShape best{0, 0};
+    int best_waves = 0;
+    for (int cs = 1; cs <= 2; ++cs) {
+        if (best_waves >= 8) break;
+        for (int nw = 4; nw >= 1; nw >>= 1) {
+            const size_t lds = rel_bwd_lds(nw, cs, n_used, h);
+            if (lds > cap) continue;
+            const int waves = nw * cs * (int)((160 * 1024) / lds);
+            if (waves > best_waves) { best = RelBwdShape{nw, cs}; best_waves = waves; }
+        }
     }
     return best;
 }
@@ -5554,15 +5611,23 @@ inline int allow_large_lds_at(const void *kernel, size_t bytes) {
 template <typename K>
 int allow_large_lds(K kernel, size_t bytes) { return allow_large_lds_at(reinterpret_cast<const void *>(kernel), bytes); }
 
-template <typename T, int H, int NW>
+template <typename T, int H, int NW, int CS>
 int launch_rel_bias_bwd(const bpt_plan *P, const float *ds, const void *q, const void *table, const int32_t *used_types, int64_t n_used,
                         void *dq, float *ws_dq, float *part, int n_parts, hipStream_t s) {
-    const size_t lds = rel_bwd_lds(NW, n_used, H);
-    const int st = allow_large_lds(k_rel_bias_bwd<T, H, NW>, lds);
+    const size_t lds = rel_bwd_lds(NW, CS, n_used, H);
+    const int st = allow_large_lds(k_rel_bias_bwd<T, H, NW, CS>, lds);
     if (st != BPT_OK) return st;
-    hipLaunchKernelGGL((k_rel_bias_bwd<T, H, NW>), dim3(n_parts), dim3(NW * WAVE), lds, s, *P, ds, (const T *)q, (const T *)table, used_types,
+    hipLaunchKernelGGL((k_rel_bias_bwd<T, H, NW, CS>), dim3(n_parts), dim3(NW * CS * WAVE), lds, s, *P, ds, (const T *)q, (const T *)table, used_types,
                        (int)n_used, (T *)dq, ws_dq, part);
     return launch_status();
+}
+
+// f(NW, CS as compile-time numbers)
+template <typename F> int rel_bwd_pick(RelBwdShape x, F &&f) {
+    auto cs = [&](auto NW) -> int {
+        return x.cs == 1 ? f(NW, std::integral_constant<int, 1>{}) : f(NW, std::integral_constant<int, 2>{});
+    };
+    return x.nw == 4 ? cs(std::integral_constant<int, 4>{}) : x.nw == 2 ? cs(std::integral_constant<int, 2>{}) : cs(std::integral_constant<int, 1>{});
 }
 
 template <typename T, int H>
@@ -5570,18 +5635,19 @@ int run_rel_bias_bwd(const bpt_plan *P, const float *ds, const void *q, const vo
                      int64_t n_types, int64_t n_used, void *dq, void *dtable, float *ws, hipStream_t s) {
     float *ws_dq = ws, *part = ws + (size_t)P->n_slots * H * 64;       // partial rows of dq of the split rows, then the partial tables
     int n_parts = 0;
-    auto launch = [&](int nw) {
-        n_parts = (int)std::min<int64_t>(REL_MAX_PARTS, std::max<int64_t>(1, (P->n_items + nw - 1) / nw));      // (an item a wavefront at the least)
-        return nw == 4   ? launch_rel_bias_bwd<T, H, 4>(P, ds, q, table, used_types, n_used, dq, ws_dq, part, n_parts, s)
-               : nw == 2 ? launch_rel_bias_bwd<T, H, 2>(P, ds, q, table, used_types, n_used, dq, ws_dq, part, n_parts, s)
-                         : launch_rel_bias_bwd<T, H, 1>(P, ds, q, table, used_types, n_used, dq, ws_dq, part, n_parts, s);
+    auto launch = [&](RelBwdShape x) {
+        const int64_t fit = 256 * std::min<int64_t>(2, (160 * 1024) / (int64_t)rel_bwd_lds(x.nw, x.cs, n_used, H));
+        n_parts = (int)std::min<int64_t>(std::min<int64_t>(REL_MAX_PARTS, fit), std::max<int64_t>(1, (P->n_items + x.nw - 1) / x.nw));      // (an item a table of sums at the least)
+        return rel_bwd_pick(x, [&](auto NW, auto CS) {
+            return launch_rel_bias_bwd<T, H, decltype(NW)::value, decltype(CS)::value>(P, ds, q, table, used_types, n_used, dq, ws_dq, part, n_parts, s);
+        });
     };
     if (P->n_edges > 0) {
-        const int nw = rel_bwd_waves(n_used, H);
-        int st = launch(nw);
-        if (st == BPT_ERR_UNSUPPORTED && rel_bwd_lds(nw, n_used, H) > 64 * 1024) {      // more than 64 KB of LDS refused by the runtime
-            const int small = rel_bwd_waves(n_used, H, false);
-            if (small == 0) return BPT_ERR_UNSUPPORTED;
+        const RelBwdShape x = rel_bwd_shape(n_used, H);
+        int st = launch(x);
+        if (st == BPT_ERR_UNSUPPORTED && rel_bwd_lds(x.nw, x.cs, n_used, H) > 64 * 1024) {      // more than 64 KB of LDS refused by the runtime
+            const RelBwdShape small = rel_bwd_shape(n_used, H, false);
+            if (small.nw == 0) return BPT_ERR_UNSUPPORTED;
             st = launch(small);
         }
         if (st != BPT_OK) return st;
@@ -5597,14 +5663,12 @@ int run_rel_bias_bwd(const bpt_plan *P, const float *ds, const void *q, const vo
 // whether run_rel_bias_bwd has a configuration that this device accepts for n_used types (nothing is launched)
 template <typename T, int H>
 int rel_bias_bwd_config(int64_t n_used) {
-    const int nw = rel_bwd_waves(n_used, H);
-    if (nw == 0) return BPT_ERR_UNSUPPORTED;
-    const size_t lds = rel_bwd_lds(nw, n_used, H);
-    const int st = nw == 4   ? allow_large_lds(k_rel_bias_bwd<T, H, 4>, lds)
-                   : nw == 2 ? allow_large_lds(k_rel_bias_bwd<T, H, 2>, lds)
-                             : allow_large_lds(k_rel_bias_bwd<T, H, 1>, lds);
+    const RelBwdShape x = rel_bwd_shape(n_used, H);
+    if (x.nw == 0) return BPT_ERR_UNSUPPORTED;
+    const size_t lds = rel_bwd_lds(x.nw, x.cs, n_used, H);
+    const int st = rel_bwd_pick(x, [&](auto NW, auto CS) { return allow_large_lds(k_rel_bias_bwd<T, H, decltype(NW)::value, decltype(CS)::value>, lds); });
     if (st == BPT_OK) return BPT_OK;
-    return rel_bwd_waves(n_used, H, false) != 0 ? BPT_OK : BPT_ERR_UNSUPPORTED;      // inside the 64 KB every kernel may take
+    return rel_bwd_shape(n_used, H, false).nw != 0 ? BPT_OK : BPT_ERR_UNSUPPORTED;      // inside the 64 KB every kernel may take
 }
 
 // the score term with the table rows in LDS: plan indices are type numbers
@@ -6658,7 +6722,7 @@ int bpt_rel_bias_backward(const bpt_plan *plan, const float *ds, const void *q, 
     CHECK(check_plan(plan, true));
     CHECK(check_shape(h, d, dtype));
     if (n_types < 0 || n_used < 0 || n_used > n_types) return BPT_ERR_SIZE;
-    if (!rel_rows_shape(h, d, dtype) || n_used > REL_MAX_USED || rel_bwd_waves(n_used, h) == 0) return BPT_ERR_UNSUPPORTED;
+    if (!rel_rows_shape(h, d, dtype) || n_used > REL_MAX_USED || rel_bwd_shape(n_used, h).nw == 0) return BPT_ERR_UNSUPPORTED;
     if (n_types == 0) return BPT_OK;
     if (!used || !dtable || (n_used > 0 && !used_types) || (plan->n_edges > 0 && (!ds || !q || !table || !dq))) return BPT_ERR_NULL;
     if (!aligned16(ds) || !aligned16(table)) return BPT_ERR_UNSUPPORTED;

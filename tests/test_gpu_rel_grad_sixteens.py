@@ -91,3 +91,18 @@ def test_an_infinite_value_stays_in_its_row_and_type(kind):
     got_q, got_t, want_q, _, want_t, _ = run(LENGTHS, lambda rng, deg: KINDS[kind](rng, deg).astype(np.int64), 50, 8, torch.float32, 6, poison=(1000, 3))
     assert torch.equal(got_q.isfinite(), want_q.isfinite()) and torch.equal(got_t.isfinite(), want_t.isfinite())
     assert not want_q.isfinite().all() and not want_t.isfinite().all()
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("n_types", [66, 88, 150, 238])
+@pytest.mark.parametrize("h,dtype", [(4, torch.float32), (8, torch.float32), (16, torch.bfloat16)])
+def test_two_wavefronts_share_the_columns(h, dtype, n_types, offset):
+    """From 57 types on (65 at 4 heads, 50 at 16): four, two or one table of sums a workgroup; sixteens of different types, of one and of a mix."""
+    def types_of(rng, deg):
+        draw = (lambda k: (np.arange(k) + rng.integers(0, n_types)) % n_types, lambda k: np.full(k, rng.integers(0, n_types)), lambda k: rng.integers(0, n_types, k))
+        out = np.concatenate([draw[i % 3](k) for i, k in enumerate(deg)])
+        out[:n_types] = np.arange(n_types)                        # (all of them are in use)
+        return out.astype(np.int64)
+    got_q, got_t, want_q, size_q, want_t, size_t = run(LENGTHS, types_of, n_types, h, dtype, 6, offset=offset)
+    close(got_q, want_q, size_q, dtype, 700)
+    close(got_t, want_t, size_t, dtype, sum(LENGTHS) * h)
