@@ -4874,69 +4874,159 @@ __global__ __launch_bounds__(BLOCK) void k_rel_bias_rows(bpt_plan P, const T *__
 // type number | member << 8 says.  The per-pair arrays are read and written in runs; the table rows in use are staged in
 // LDS once per workgroup (fetched from memory step by step, each step waits for two dependent loads: 32 us against
 // the products' 7).
-template <typename T>
-__device__ __forceinline__ void rel_cols16(const T *row, int g, float (&out)[16]) {     // columns 16 t + 4 g + e of a 64-column row
+//
+// QT takes 64 bytes a type and wavefront, so with many types a compute unit holds a workgroup of eight wavefronts or less, and what counts is how
+// few round trips and products a tile costs: a workgroup then keeps the table rows for all of its tiles, and a wavefront has its next tile's
+// pairs, q rows and places in the plan on their way.  ONE: a workgroup for every tile, where all fit the chip at once or a compute unit holds 24
+// wavefronts; other wavefronts are what hides the round trips there (float32 L = 8192, k = 4 25.6 -> 21.8 us, bfloat16 level).
+// float32 leaves out the sixteens of types that no pair of the tile has, which its first loads tell for up to 256 (512) pairs (6 of 11 sixteens
+// are left at L = 8192, k = 8 both ways, 3 of 4 at k = 4; a look through longer tiles' pairs cost what it gave).  bfloat16 multiplies on
+// bfloat16 matrix instructions: the same products, summed in float32.
+// Against a workgroup for every tile and float32 products throughout: float32 8 heads L = 8192, k = 4 (55 types) 25.7 -> 21.8 us, 32-graph batch (43)
+// 36.7 -> 32.6, L = 8192, k = 8 both ways (173) 222 -> 65, 16 heads L = 4096, k = 16 (140) 56 -> 45, L = 100 5.1 -> 5.3; bfloat16 8 heads L = 32768,
+// k = 2 (33) 59 -> 30, 16 heads a batch with k = 20 (105) 68 -> 24, L = 2048 12.5 -> 6.9.
+template <typename T> struct RelTile;
+template <> struct RelTile<float> {
+    static constexpr int PITCH = REL_LDS_PITCH * 4;              // bytes between the table rows in LDS
+    struct Row { float v[16]; };                                  // columns 16 t + 4 g + e of a 64-column row
+    static __device__ __forceinline__ void cols(const float *row, int g, Row &out) {
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        const float4 x = load4<T>(row + 16 * t + 4 * g);
-        out[4 * t] = x.x; out[4 * t + 1] = x.y; out[4 * t + 2] = x.z; out[4 * t + 3] = x.w;
+        for (int t = 0; t < 4; ++t) {
+            const float4 x = *reinterpret_cast<const float4 *>(row + 16 * t + 4 * g);
+            out.v[4 * t] = x.x; out.v[4 * t + 1] = x.y; out.v[4 * t + 2] = x.z; out.v[4 * t + 3] = x.w;
+        }
     }
-}
-template <typename T, int H, int HW>
+    static __device__ __forceinline__ floatx4v dot(const Row &a, const Row &b) { return tile_dot(a.v, b.v); }
+};
+template <> struct RelTile<bf16_t> {
+    static constexpr int PITCH = TILE_KT_BYTES_BF16;
+    struct Row { Bf8 v[2]; };                                     // columns 16 g .. 16 g + 15
+    static __device__ __forceinline__ void cols(const bf16_t *row, int g, Row &out) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) out.v[t].q = *reinterpret_cast<const uint4 *>(row + 16 * g + 8 * t);
+    }
+    static __device__ __forceinline__ floatx4v dot(const Row &a, const Row &b) { return tile_dot_bf16(a.v, b.v); }
+};
+template <typename T, int H, int HW, bool ONE>
 __global__ __launch_bounds__(HW * WAVE) void k_rel_bias_tiles(bpt_plan P, const T *__restrict__ q, const T *__restrict__ table,
                                                               const int32_t *__restrict__ used_types, int n_used,
                                                               const int32_t *__restrict__ pair_tm, float *__restrict__ bias) {
-    constexpr int D = 64, C = H * D;
+    typedef RelTile<T> R;
+    constexpr int D = 64, C = H * D, HS = H / HW, PIECES = D * sizeof(T) / 16;
+    constexpr int AHEAD = ONE ? 4 : 8;                          // pairs per lane whose loads are in flight together
     extern __shared__ float rel_lds[];                        // the table rows in use, then QT of every wavefront
+    char *const rows = reinterpret_cast<char *>(rel_lds);
+    const int lane = threadIdx.x & (WAVE - 1), wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), c = lane & 15, g = lane >> 4;
     const int n16 = (n_used + 15) & ~15;
-    rel_table_to_lds<T>(table, used_types, n_used, rel_lds, REL_LDS_PITCH);
-    TileCtx t;
-    const bool mine = tile_begin<T, H, D, HW>(P, t, Narrow{}) && t.p_begin < t.p_end;
-    __syncthreads();
-    if (!mine) return;
-    float *qt = rel_lds + (size_t)n_used * REL_LDS_PITCH + (size_t)t.wv * n16 * TILE_R;
-    auto table_rows = [&](int tb, float (&out)[16]) {           // of type numbers tb + c: this lane's columns
-        const float *row = rel_lds + min(tb + t.c, n_used - 1) * REL_LDS_PITCH + 4 * t.g;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const float4 x = *reinterpret_cast<const float4 *>(row + 16 * i);
-            out[4 * i] = x.x; out[4 * i + 1] = x.y; out[4 * i + 2] = x.z; out[4 * i + 3] = x.w;
-        }
+    float *const qt = reinterpret_cast<float *>(rows + (size_t)n_used * R::PITCH) + (size_t)wv * n16 * TILE_R;
+    // the workgroup's places w in the XCD's range (tile w / HS, heads from (w % HS) HW): w0, w0 + step, ...
+    const int x = blockIdx.x & 7, step = (int)(gridDim.x >> 3), w0 = (int)(blockIdx.x >> 3);
+    const int grp0 = __builtin_amdgcn_readfirstlane(P.grp_chunks[x]), n_places = (__builtin_amdgcn_readfirstlane(P.grp_chunks[x + 1]) - grp0) * HS;
+    const int n_mine = w0 < n_places ? (ONE ? 1 : (n_places - w0 + step - 1) / step) : 0;
+    struct Place { int head, p_begin, p_end, row; };            // row: of member c
+    struct Pairs { int first, end; };                           // the tile's pair numbers
+    struct Asked { int tm[AHEAD]; typename R::Row q; };
+    auto ask_place = [&](int i, Place &y) {
+        const int w = w0 + min(i, n_mine - 1) * step, grp = grp0 + w / HS;
+        y.head = (w % HS) * HW + wv;
+        y.p_begin = P.grp_ptr[grp];
+        y.p_end = P.grp_ptr[grp + 1];
+        y.row = reinterpret_cast<const int2 *>(P.grp_members)[(size_t)grp * TILE_R + c].x;
     };
-    const int4 *entries = reinterpret_cast<const int4 *>(P.grp_entries);
-    const int4 last = entries[t.p_end - 1];
-    const int first = __builtin_amdgcn_readfirstlane(entries[t.p_begin].z), end = __builtin_amdgcn_readfirstlane(last.z + __popc((uint32_t)last.y));
-    if (end <= first) return;
-    constexpr int AHEAD = 4;                                    // pairs per lane whose loads are in flight together
-    int tm[AHEAD];
+    auto ask_pairs = [&](const Place &y, Pairs &e) {
+        const int4 *entries = reinterpret_cast<const int4 *>(P.grp_entries);
+        const int b = __builtin_amdgcn_readfirstlane(y.p_begin), l = __builtin_amdgcn_readfirstlane(y.p_end);
+        const int4 last = entries[max(l - 1, 0)];
+        e.first = b < l ? entries[b].z : 0;
+        e.end = b < l ? last.z + __popc((uint32_t)last.y) : 0;
+    };
+    auto ask = [&](const Place &y, const Pairs &e, Asked &a) {
 #pragma unroll
-    for (int k = 0; k < AHEAD; ++k) tm[k] = pair_tm[min(first + t.lane + k * WAVE, end - 1)];
-    float qb[16];
-    rel_cols16<T>(q + (size_t)max(t.member.x, 0) * C + t.head * D, t.g, qb);
-    for (int tb = 0; tb < n16; tb += TILE_R) {
-        float kr[16];
-        table_rows(tb, kr);
-        const floatx4v st = tile_dot(kr, qb);                   // register r: (type number tb + 4 g + r, member c)
+        for (int k = 0; k < AHEAD; ++k) a.tm[k] = pair_tm[max(min(e.first + lane + k * WAVE, e.end - 1), 0)];
+        R::cols(q + (size_t)max(y.row, 0) * C + y.head * D, g, a.q);
+    };
+    Place at[3];
+    Pairs pairs[2];
+    Asked cur;
+    if (n_mine > 0) ask_place(0, at[0]);
+    if (!ONE && n_mine > 1) ask_place(1, at[1]);
+    // four pieces of the table rows a thread side by side, by two dependent loads
+    for (int y = threadIdx.x, n = n_used * PIECES; y < n; y += 4 * HW * WAVE) {
+        int type[4];
+        uint4 piece[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) qt[(tb + 4 * t.g + r) * TILE_R + t.c] = st[r];
+        for (int i = 0; i < 4; ++i) type[i] = used_types[min(y + i * HW * WAVE, n - 1) / PIECES];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            piece[i] = *reinterpret_cast<const uint4 *>(reinterpret_cast<const char *>(table + (size_t)type[i] * D) + 16 * (min(y + i * HW * WAVE, n - 1) % PIECES));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (y + i * HW * WAVE < n)
+                *reinterpret_cast<uint4 *>(rows + (size_t)((y + i * HW * WAVE) / PIECES) * R::PITCH + 16 * ((y + i * HW * WAVE) % PIECES)) = piece[i];
     }
-    wave_lds_fence();
-    float *out = bias + (size_t)t.head * (size_t)P.n_edges;
-    for (int x = first + t.lane; x < end; x += AHEAD * WAVE) {
-        int nt[AHEAD];
-#pragma unroll
-        for (int k = 0; k < AHEAD; ++k) nt[k] = pair_tm[min(x + (AHEAD + k) * WAVE, end - 1)];
-        float val[AHEAD];
-#pragma unroll
-        for (int k = 0; k < AHEAD; ++k) val[k] = qt[(tm[k] & 0xff) * TILE_R + (tm[k] >> 8)];
-        // (the next round's loads are waited for before this round's stores: behind them the wait would include the stores)
-#pragma unroll
-        for (int k = 0; k < AHEAD; ++k) asm volatile("" ::"v"(nt[k]));
-#pragma unroll
-        for (int k = 0; k < AHEAD; ++k) {
-            if (x + k * WAVE < end) out[x + k * WAVE] = val[k];
-            tm[k] = nt[k];
+    if (n_mine > 0) {
+        ask_pairs(at[0], pairs[0]);
+        ask(at[0], pairs[0], cur);
+    }
+    if (!ONE && n_mine > 1) {
+        ask_pairs(at[1], pairs[1]);
+        ask_place(2, at[2]);
+    }
+    __syncthreads();
+    for (int i = 0; i < n_mine; ++i) {
+        Asked next;
+        Pairs after = pairs[1];
+        Place later = at[2];
+        if constexpr (!ONE) next = cur;
+        if (!ONE && i + 1 < n_mine) {
+            ask(at[1], pairs[1], next);
+            ask_pairs(at[2], after);
+            ask_place(i + 3, later);
         }
+        issue_loads_first();
+        const int first = pairs[0].first, end = pairs[0].end;
+        // bit x: one of the lane's pairs has a type number in 16 x .. 16 x + 15.  Only where all pairs are at hand and a product takes long
+        uint32_t sixteens = sizeof(T) == 4 && end - first <= AHEAD * WAVE ? 0u : ~0u;
+        if (sizeof(T) == 4) {
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) sixteens |= 1u << ((cur.tm[k] >> 4) & 15);
+        }
+        for (int tb = 0; tb < n16; tb += TILE_R) {
+            if (__builtin_amdgcn_ballot_w64((sixteens >> (tb / TILE_R)) & 1) == 0) continue;
+            typename R::Row kr;
+            R::cols(reinterpret_cast<const T *>(rows + (size_t)min(tb + c, n_used - 1) * R::PITCH), g, kr);
+            const floatx4v st = R::dot(kr, cur.q);                // register r: (type number tb + 4 g + r, member c)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) qt[(tb + 4 * g + r) * TILE_R + c] = st[r];
+        }
+        wave_lds_fence();
+        // (the next tile's loads, and each round's, are waited for before this round's stores: behind them the wait would include the stores)
+#pragma unroll
+        for (int k = 0; k < (ONE ? 0 : AHEAD); ++k) asm volatile("" ::"v"(next.tm[k]));
+        float *out = bias + (size_t)at[0].head * (size_t)P.n_edges;
+        for (int y = first + lane; y < end; y += AHEAD * WAVE) {
+            int nt[AHEAD];
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) nt[k] = pair_tm[min(y + (AHEAD + k) * WAVE, end - 1)];
+            float val[AHEAD];
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) val[k] = qt[(cur.tm[k] & 0xff) * TILE_R + (cur.tm[k] >> 8)];
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) asm volatile("" ::"v"(nt[k]));
+#pragma unroll
+            for (int k = 0; k < AHEAD; ++k) {
+                if (y + k * WAVE < end) out[y + k * WAVE] = val[k];
+                cur.tm[k] = nt[k];
+            }
+        }
+        if constexpr (ONE) return;
+        wave_lds_fence();                                         // (read before the next tile's products are written)
+        cur = next;
+        pairs[0] = pairs[1];
+        pairs[1] = after;
+        at[0] = at[1];
+        at[1] = at[2];
+        at[2] = later;
     }
 }
 
@@ -5558,6 +5648,7 @@ inline bool rel_rows_shape(int h, int d, int dtype) {
 }
 
 constexpr int REL_MAX_PARTS = 512;        // partial tables of the gradient kernel: two workgroups per compute unit
+constexpr int REL_TILES_WAVES = 24;       // wavefronts a compute unit needs to hide the score kernel's round trips, and where several tiles share a workgroup the most of them
 constexpr int REL_MAX_USED = 240;         // type numbers whose table rows fit the 64 KB of LDS of the score kernel
 
 // LDS of k_rel_bias_bwd with nw tables of sums of cs wavefronts each: the sums, the table rows, the wavefronts' staged ds values and types
@@ -5682,24 +5773,34 @@ int run_rel_bias_rows(const bpt_plan *P, const void *q, const void *table, const
 }
 
 // the score term over the attention kernels' tile plan, in that plan's pair order
+template <typename T> size_t rel_tiles_lds(int hw, int64_t n_used) {      // the table rows, and QT of every wavefront
+    return (size_t)n_used * RelTile<T>::PITCH + (size_t)hw * (size_t)((n_used + 15) & ~(int64_t)15) * TILE_R * 4;
+}
 template <typename T, int H, int HW>
 int launch_rel_bias_tiles(const bpt_plan *P, const void *q, const void *table, const int32_t *used_types, int64_t n_used, const int32_t *pair_tm,
-                          float *bias, size_t lds, hipStream_t s) {
-    const int st = allow_large_lds(k_rel_bias_tiles<T, H, HW>, lds);
-    if (st != BPT_OK) return st;
-    hipLaunchKernelGGL((k_rel_bias_tiles<T, H, HW>), dim3(group_grid(P) * (H / HW)), dim3(HW * WAVE), lds, s, *P, (const T *)q, (const T *)table,
-                       used_types, (int)n_used, pair_tm, bias);
-    return launch_status();
+                          float *bias, hipStream_t s) {
+    const size_t lds = rel_tiles_lds<T>(HW, n_used);
+    const int resident = 256 * std::min(REL_TILES_WAVES / HW, (int)((160 * 1024) / lds)), tiles = group_grid(P) * (H / HW);   // (resident: what the chip holds)
+    auto launch = [&](auto kernel, int grid) -> int {
+        const int st = allow_large_lds(kernel, lds);
+        if (st != BPT_OK) return st;
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(HW * WAVE), lds, s, *P, (const T *)q, (const T *)table, used_types, (int)n_used, pair_tm, bias);
+        return launch_status();
+    };
+    return tiles <= resident || (int)((160 * 1024) / lds) * HW >= REL_TILES_WAVES ? launch(k_rel_bias_tiles<T, H, HW, true>, tiles) : launch(k_rel_bias_tiles<T, H, HW, false>, resident);
 }
 template <typename T, int H>
 int run_rel_bias_tiles(const bpt_plan *P, const void *q, const void *table, const int32_t *used_types, int64_t n_used, const int32_t *pair_tm,
                        float *bias, hipStream_t s) {
-    // the table rows once per workgroup, QT once per wavefront (= head); eight heads share the rows where that fits 64 KB
-    auto lds = [&](int hw) { return ((size_t)n_used * REL_LDS_PITCH + (size_t)hw * (size_t)((n_used + 15) & ~(int64_t)15) * TILE_R) * 4; };
+    // eight heads share the table rows where that puts no fewer wavefronts on a compute unit
     if constexpr (H >= 8) {
-        if (lds(8) <= 64 * 1024) return launch_rel_bias_tiles<T, H, 8>(P, q, table, used_types, n_used, pair_tm, bias, lds(8), s);
+        const size_t l8 = rel_tiles_lds<T>(8, n_used), l4 = rel_tiles_lds<T>(4, n_used);
+        if (l8 <= 160 * 1024 && 2 * ((160 * 1024) / l8) >= (160 * 1024) / l4) {
+            const int st = launch_rel_bias_tiles<T, H, 8>(P, q, table, used_types, n_used, pair_tm, bias, s);
+            if (st != BPT_ERR_UNSUPPORTED) return st;             // (more than 64 KB of LDS refused by the runtime)
+        }
     }
-    return launch_rel_bias_tiles<T, H, 4>(P, q, table, used_types, n_used, pair_tm, bias, lds(4), s);
+    return launch_rel_bias_tiles<T, H, 4>(P, q, table, used_types, n_used, pair_tm, bias, s);
 }
 
 template <typename T, int H, int D>
