@@ -4757,7 +4757,8 @@ template <> __device__ __forceinline__ void rel_load16<bf16_t>(const bf16_t *p, 
 constexpr int REL_STAGE_PITCH = WAVE + 4;
 constexpr int REL_BWD_STAGE(int h) { return REL_STAGE_PITCH * h + WAVE; }
 
-// A work item (a row or a segment of a long row) and the types and edge ids of its first 64 slots (lane l: slot b + l).
+// A work item (a row or a segment of a long row) and the types and edge ids of its first 64 slots (lane l: slot b + l).  The plan has an edge:
+// an item without any reads the types and ids of a slot that is there.
 struct RelHead {
     int row, b, e, out_slot;
     int type, edge;
@@ -4808,6 +4809,9 @@ __global__ __launch_bounds__(BLOCK) void k_rel_bias_rows(bpt_plan P, const T *__
     static_assert(H == 4 || H == 8 || H == 16, "four consecutive heads per lane");
     extern __shared__ float rel_lds[];
     const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    const bool head_major = P.bias_by_pair != 0;                // results at bias[head * n_edges + eid] instead of bias[eid * H + head]
+    if (blockIdx.x == 0 && threadIdx.x < H && !head_major) bias[(size_t)P.n_edges * H + threadIdx.x] = 0.f;     // the spare row the fused kernels read for absent pairs
+    if (P.n_edges == 0) return;                                 // (rows, but no slot to read)
     // wavefront gw of GW takes the items gw, gw + GW, ...: the segments of a long row, which are neighbours and all full, go to
     // different wavefronts
     const int GW = (int)gridDim.x * WAVES_PER_BLOCK, i0 = (int)blockIdx.x * WAVES_PER_BLOCK + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -4817,8 +4821,6 @@ __global__ __launch_bounds__(BLOCK) void k_rel_bias_rows(bpt_plan P, const T *__
 #pragma unroll
     for (int k = 0; k < K; ++k) desc[k] = items[min(i0 + k * GW, n_items - 1)];
     rel_table_to_lds<T>(table, used_types, n_used, rel_lds, REL_LDS_PITCH);
-    const bool head_major = P.bias_by_pair != 0;                // results at bias[head * n_edges + eid] instead of bias[eid * H + head]
-    if (blockIdx.x == 0 && threadIdx.x < H && !head_major) bias[(size_t)P.n_edges * H + threadIdx.x] = 0.f;     // the spare row the fused kernels read for absent pairs
     RelHead hd[K];
     float aq[K][16];
 #pragma unroll
@@ -6800,6 +6802,7 @@ int bpt_rel_bias_forward(const bpt_plan *plan, const void *q, const void *table,
     if (used_types) {                       // plan indices are type numbers: the kernel with the table rows in LDS
         if (n_used < 0) return BPT_ERR_SIZE;
         if (!rel_rows_shape(h, d, dtype) || n_used > REL_MAX_USED || !aligned16(q) || !aligned16(table) || !aligned16(bias)) return BPT_ERR_UNSUPPORTED;
+        if (plan->n_edges == 0 && (!bias || plan->bias_by_pair)) return BPT_OK;      // (no spare row to clear)
 #define X(HH) if (h == HH) return run_rel_bias_rows<T, HH>(plan, q, table, used_types, n_used, bias, s);
         if (dtype == BPT_F32) { using T = float; X(4) X(8) X(16) }
         if (dtype == BPT_BF16) { using T = bf16_t; X(4) X(8) X(16) }
