@@ -4757,6 +4757,8 @@ template <> __device__ __forceinline__ void rel_load16<bf16_t>(const bf16_t *p, 
 constexpr int REL_STAGE_PITCH = WAVE + 4;
 constexpr int REL_BWD_STAGE(int h) { return REL_STAGE_PITCH * h + WAVE; }
 
+constexpr int REL_MAX_USED = 240;         // type numbers whose table rows fit the 64 KB of LDS of the score kernel
+
 // A work item (a row or a segment of a long row) and the types and edge ids of its first 64 slots (lane l: slot b + l).  The plan has an edge:
 // an item without any reads the types and ids of a slot that is there.
 struct RelHead {
@@ -5158,13 +5160,17 @@ __global__ __launch_bounds__(NW * CS * WAVE) void k_rel_bias_bwd(bpt_plan P, con
     RelHead hd[4];
     RelBody<H, NB> bd[2];
     auto body = [&](const RelHead &r, RelBody<H, NB> &y) { rel_body_load<T, H, NB>(r, ds, by, q, dq, g, col, y); };
-    // ds and types of up to 64 slots (past the end: zeros; negative types, no two alike)
+    // ds and types of up to 64 slots (past the end: zeros; the last slot's type as a negative number, no two alike)
     auto put = [&](int cnt, const float (&d)[H], int type) {
 #pragma unroll
         for (int h = 0; h < H; ++h) stage[h * PITCH + lane] = lane < cnt ? d[h] : 0.f;
-        types[lane] = lane < cnt ? type : -1 - lane;
+        types[lane] = lane < cnt ? type : ~(type | lane << 8);    // (lanes past the end hold the last slot's type, which is less than 256)
         wave_lds_fence();
     };
+    // the table row of a slot: past the end one of the item's own, whatever is multiplied by zero there (an infinite row of a type that the item
+    // does not have stays out of it)
+    static_assert(REL_MAX_USED <= 256, "a type fits eight bits");
+    auto row_of = [](int type) { return (type ^ (type >> 31)) & 255; };
     // sixteen slots of those, cnt of them exist
     auto sixteen = [&](int j, int cnt, const RelCols<NB> (&qr)[H / 4], floatx4v (&dqa)[NB]) {
         const int4 t4 = *reinterpret_cast<const int4 *>(types + j + 4 * g);               // of slots 4 g .. 4 g + 3
@@ -5177,9 +5183,9 @@ __global__ __launch_bounds__(NW * CS * WAVE) void k_rel_bias_bwd(bpt_plan P, con
         for (int s = 0; s < H / 4; ++s) d[s] = stage[(4 * s + g) * PITCH + j + c];
         RelCols<NB> tv[4], before[4];                             // table rows of those slots; the sums of their types so far
 #pragma unroll
-        for (int r = 0; r < 4; ++r) tv[r] = rel_row_load<NB>(rows + max(ty[r], 0) * D + col);
+        for (int r = 0; r < 4; ++r) tv[r] = rel_row_load<NB>(rows + row_of(ty[r]) * D + col);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) before[r] = rel_row_load<NB>(acc + max(ty[r], 0) * D + col);
+        for (int r = 0; r < 4; ++r) before[r] = rel_row_load<NB>(acc + row_of(ty[r]) * D + col);
         // slots of one type: lane (c, g) compares the type of slot c with those of slots 4 g + s
         bool twice = false;
         uint64_t same0 = 0;
@@ -5651,7 +5657,6 @@ inline bool rel_rows_shape(int h, int d, int dtype) {
 
 constexpr int REL_MAX_PARTS = 512;        // partial tables of the gradient kernel: two workgroups per compute unit
 constexpr int REL_TILES_WAVES = 24;       // wavefronts a compute unit needs to hide the score kernel's round trips, and where several tiles share a workgroup the most of them
-constexpr int REL_MAX_USED = 240;         // type numbers whose table rows fit the 64 KB of LDS of the score kernel
 
 // LDS of k_rel_bias_bwd with nw tables of sums of cs wavefronts each: the sums, the table rows, the wavefronts' staged ds values and types
 inline size_t rel_bwd_lds(int nw, int cs, int64_t n_used, int h) { return ((size_t)(nw + 1) * n_used * 64 + (size_t)nw * cs * REL_BWD_STAGE(h)) * 4; }

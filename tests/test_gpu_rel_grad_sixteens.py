@@ -1,6 +1,7 @@
 """Gradients of the rel_pos score term (graphop.rel_bias_backward) where the kernel's sixteens of slots can go wrong, against float64: rows
 of 1 to 17, 63 to 65, 127 to 130 and several hundred slots (segments), whose sixteens hold sixteen types, one type or a mix; more work items than a
-wavefront keeps descriptors of; q and dq that start on any element; an infinite value of ds, which reaches its own row and type only."""
+wavefront keeps descriptors of; q and dq that start on any element; an infinite value of ds, which reaches its own row and type only; a table row
+that is not finite, which reaches the rows that have an edge of its type."""
 import numpy as np
 import pytest
 import torch
@@ -10,7 +11,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-def run(deg, types_of, n_types, h, dtype, seed, offset=0, poison=None):
+def run(deg, types_of, n_types, h, dtype, seed, offset=0, poison=None, poison_number=None):
     from bpt_amd import graphbuilder as gb, graphop, plan
     plan.plan_cache.clear()
     n, E, d, rng = len(deg), int(sum(deg)), 64, np.random.default_rng(seed)
@@ -31,6 +32,8 @@ def run(deg, types_of, n_types, h, dtype, seed, offset=0, poison=None):
     table, ds = torch.randn(n_types, d, generator=gen).to(dtype), torch.randn(E, h, generator=gen) * 0.1
     if poison is not None:
         ds[poison] = float("inf")
+    if poison_number is not None:
+        table[used_types[poison_number], 9], table[used_types[poison_number], 50] = float("nan"), float("-inf")
     dq = at_offset(dq0)
     to = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
     dtable = graphop.rel_bias_backward(col.to(DEV), ic.to(DEV), in_csr[2].to(DEV), to(used[et[in_csr[2].numpy()]].astype(np.int64)), to(used),
@@ -91,6 +94,28 @@ def test_an_infinite_value_stays_in_its_row_and_type(kind):
     got_q, got_t, want_q, _, want_t, _ = run(LENGTHS, lambda rng, deg: KINDS[kind](rng, deg).astype(np.int64), 50, 8, torch.float32, 6, poison=(1000, 3))
     assert torch.equal(got_q.isfinite(), want_q.isfinite()) and torch.equal(got_t.isfinite(), want_t.isfinite())
     assert not want_q.isfinite().all() and not want_t.isfinite().all()
+
+
+@pytest.mark.parametrize("kind", ["different", "the same", "mixed"])
+@pytest.mark.parametrize("number", [0, 17, -1])
+@pytest.mark.parametrize("h,dtype,n_types", [(4, torch.float32, 40), (8, torch.float32, 40), (16, torch.bfloat16, 40), (8, torch.float32, 88),
+                                             (16, torch.bfloat16, 150)])
+def test_a_table_row_that_is_not_finite_stays_in_its_types_rows(h, dtype, n_types, number, kind):
+    """The first, one and the last of the types in use, rows with and without edges of it, of lengths that leave sixteens and chunks of 64
+    slots part empty."""
+    draw = {"different": lambda rng, k: (np.arange(k) + rng.integers(0, n_types)) % n_types, "the same": lambda rng, k: np.full(k, rng.integers(0, n_types)),
+            "mixed": lambda rng, k: rng.integers(0, n_types, k)}[kind]
+    lengths = LENGTHS[:-1] + list(range(1, n_types))
+
+    def types_of(rng, deg):
+        out = np.concatenate([draw(rng, k) for k in deg])
+        out[-n_types:] = np.arange(n_types)                       # (all of them are in use)
+        return out.astype(np.int64)
+    got_q, got_t, want_q, size_q, want_t, size_t = run(lengths, types_of, n_types, h, dtype, 8, poison_number=number)
+    assert torch.equal(got_q.isfinite(), want_q.isfinite()) and not want_q.isfinite().all() and (want_q.isfinite().all(2).all(1)[1:]).any()
+    whole = want_q.isfinite()
+    close(got_q[whole], want_q[whole], size_q[whole], dtype, max(lengths))
+    close(got_t, want_t, size_t, dtype, sum(lengths) * h)
 
 
 @pytest.mark.parametrize("offset", [0, 1])
