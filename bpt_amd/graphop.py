@@ -151,6 +151,12 @@ def _on_device_of(t):
     return _NO_GUARD if t.device.index == _current_device() else torch.cuda.device_of(t)
 
 
+def capturing(t):
+    """Whether the current stream of t's device is being captured into a graph."""
+    with _on_device_of(t):
+        return torch.cuda.is_current_stream_capturing()
+
+
 def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None and t.numel() else None
 
@@ -1015,31 +1021,48 @@ def prepare_rel_training(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, 
                                    (row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg, _plan.tile_order_src(k.size(0), eid_r.size(0)))])
 
 
-def remember_rel(generation, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p, table, etype, aux, train):
-    """Leaves with the native host path what a forward (train: and a backward) with the relative-position term takes for these arguments, of
-    which rel_bias_forward_tiles has just been found to run: the in-CSR's tile plan, the out-CSR's linked to it, the plan of the term's
-    gradient, and the term's index tensors (op._rel_aux)."""
+def prepare_rel_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p, rows_slot, number_slot, n_used):
+    """Where the term is in the order of the tiles: the linked out-side and the plan of the term's gradient, which the backward is going to ask
+    for, ahead of the forward's kernels.  Both are waited for when they are new, and the backward's wait would be for all that is queued by
+    then.  Nothing under stream capture."""
     graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
-    if any(t.dtype != torch.int64 for t in graph) or TILE_BACKWARD is not None:
-        return                       # (with the hook set the passes choose for themselves)
-    hit, held = _pair_order(*graph, q, k, dropout_p), aux["rows_slot"]
-    if hit is None or held[0] is not hit[1]["pair_of_eid"]:
-        return
-    pi, in_struct = hit[0], hit[1]["struct"]
-    index, numbers = list(graph) + [etype], [q.size(0), k.size(0), q.size(1), q.size(2), _dtype(q), int(dropout_p > 0.0), table.size(0)]
-    with torch.cuda.device(q.device):
-        torch.cuda.current_stream().synchronize()          # (the term's index tensors are there for whichever stream serves the next call)
-    if not train:
-        plan_cache.remember((pi,), generation, _native.REL_FWD, index, numbers, ctypes.addressof(in_struct), 0, 0, [aux["used_types"], held[2]],
-                            how="remember_rel")
-        return
+    hit = None if capturing(q) else _pair_order(*graph, q, k, dropout_p)
+    if hit is not None:
+        _rel_backward_plans(hit[0], *graph, q, k, rows_slot, number_slot, n_used)
+
+
+def _rel_backward_plans(pi, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, rows_slot, number_slot, n_used):
+    """(the out-side's plan, its struct linked to the in-side's plan pi, the plan of the term's gradient), as attention_backward and
+    rel_bias_backward ask for them; None where the sides do not belong together."""
     order_src = _plan.tile_order_src(k.size(0), eid_r.size(0))
     po = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg_len=_tile_seg_of(eid_c.size(0), q.size(0), k.size(0)),
                         prefer_device=True, groups=(TILE_ROWS, order_src))
     if po.n_edges != pi.n_edges or not po.covers_all_edges:
+        return None
+    return (po, po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True),
+            plan_cache.get(col, indptr_c, rows_slot, number_slot, q.size(0), max(n_used, 1), prefer_device=True))
+
+
+def remember_rel(generation, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p, table, etype, aux, held, train):
+    """Leaves with the native host path what a forward (train: and a backward) with the relative-position term takes for these arguments, of
+    which rel_bias_forward_tiles has just been found to run: the in-CSR's tile plan, the out-CSR's linked to it, the plan of the term's
+    gradient, and the term's index tensors (op._rel_aux; held: those in the order of the tiles)."""
+    graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
+    if any(t.dtype != torch.int64 for t in graph) or TILE_BACKWARD is not None:
+        return                       # (with the hook set the passes choose for themselves)
+    hit = _pair_order(*graph, q, k, dropout_p)
+    if hit is None or held[0] is not hit[1]["pair_of_eid"]:
         return
-    out_struct = po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True)
-    rel = plan_cache.get(col, indptr_c, held[1], aux["number_slot"], q.size(0), max(aux["n_used"], 1), prefer_device=True)     # (rel_bias_backward's)
+    pi, in_struct = hit[0], hit[1]["struct"]
+    index, numbers = list(graph) + [etype], [q.size(0), k.size(0), q.size(1), q.size(2), _dtype(q), int(dropout_p > 0.0), table.size(0)]
+    if not train:
+        plan_cache.remember((pi,), generation, _native.REL_FWD, index, numbers, ctypes.addressof(in_struct), 0, 0, [aux["used_types"], held[2]],
+                            how="remember_rel")
+        return
+    plans = _rel_backward_plans(pi, *graph, q, k, held[1], aux["number_slot"], aux["n_used"])
+    if plans is None:
+        return
+    po, out_struct, rel = plans
     rel_struct = _by_pair(rel.struct)
     plan_cache.remember((pi, po, rel), generation, _native.REL_TRAIN, index, numbers, ctypes.addressof(in_struct), ctypes.addressof(out_struct),
                         ctypes.addressof(rel_struct), [aux["used_types"], held[2], aux["used"], held[1], aux["number_slot"]], how="remember_rel")

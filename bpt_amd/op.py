@@ -105,7 +105,9 @@ class BPTRelAttention(Function):
 
     @staticmethod
     def forward(ctx, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale, dropout_p, seed,
-                table, etype):
+                table, etype, on_tiles=None):
+        """on_tiles: None or a list, which receives the term's index tensors (_rel_aux, and those in the order of the tiles) where the term is
+        formed over the tiles."""
         aux = _rel_aux(etype, col, indptr_c, eid_c, table.size(0))
         table = table.contiguous()
         # (the gradient kernel's configuration is asked for here: the SpMM form is then chosen for both passes up front)
@@ -122,12 +124,17 @@ class BPTRelAttention(Function):
                 rows_slot = pair.index_select(0, eid_c).contiguous()
                 # per pair number: the number of its edge's type and which row of its tile its destination is
                 types = torch.empty_like(aux["number_slot"]).index_copy_(0, rows_slot, aux["number_slot"]).to(torch.int32)
-                held = aux["rows_slot"] = (pair, rows_slot, (types | (_g.attention_pair_members(*graph, dropout_p) << 8)).contiguous())
+                held = (pair, rows_slot, (types | (_g.attention_pair_members(*graph, dropout_p) << 8)).contiguous())
+                if not _g.capturing(q):                           # (what a captured graph fills is there after its replays only)
+                    _written(q.device)
+                    aux["rows_slot"] = held
             ctx.rows_slot = held[1]
-            aux["on_tiles"] = False
+            if on_tiles is not None and any(ctx.needs_input_grad):
+                _g.prepare_rel_backward(*graph, dropout_p, held[1], aux["number_slot"], aux["n_used"])
             try:
                 bias = _g.rel_bias_forward_tiles(*graph, table, aux["used_types"], held[2], dropout_p)
-                aux["on_tiles"] = True
+                if on_tiles is not None:
+                    on_tiles.extend((aux, held))
             except _g.BptStatusError as err:
                 # (many types in use need more than 64 KB of LDS there, which a runtime may refuse: the kernel over the
                 # in-CSR writes the same layout from within 64 KB)
@@ -152,7 +159,7 @@ class BPTRelAttention(Function):
         if ctx.rows_slot is not None:
             dq, dk, dv, dtable = _rel_backward(*ctx.saved_tensors, do, ctx.scale, ctx.dropout_p, ctx.seed, ctx.rows_slot, aux["number_slot"],
                                                aux["used"], aux["used_types"])
-            return None, None, None, None, None, None, None, None, dq, dk, dv, None, None, None, dtable, None
+            return None, None, None, None, None, None, None, None, dq, dk, dv, None, None, None, dtable, None, None
         dq, dk, dv, ds = _g.attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c,
                                                q, k, v, o, lse, do, ctx.scale, ctx.dropout_p, ctx.seed, bias=bias)
         if ctx.on_chip:
@@ -165,7 +172,7 @@ class BPTRelAttention(Function):
             dq = vector_spmm_forward(col, indptr_c, eid_c, aux["etype_slot"], ds, table_h, n_rows=q.size(0), out=dq)
             dtable = vector_spmm_forward(t_row, t_indptr, t_order, t_dst, ds, q, n_rows=table.size(0))
             dtable = dtable.float().sum(1).to(table.dtype)
-        return None, None, None, None, None, None, None, None, dq, dk, dv, None, None, None, dtable, None
+        return None, None, None, None, None, None, None, None, dq, dk, dv, None, None, None, dtable, None, None
 
 
 def _rel_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, o, lse, bias, table, do, scale, dropout_p, seed, rows_slot,
@@ -181,25 +188,38 @@ _REL_FORM = _g.rel_bias_forward_tiles        # what the native host path stands 
 
 
 def _rel_attention(*args):
-    """BPTRelAttention, by the native host path where it knows the call (the second one of a graph, shape and type on)."""
+    """BPTRelAttention, by the native host path where it knows the call (the second one of a graph, shape and type on).  What the first one leaves
+    with that path is made before its kernels are queued and waits for none of them, so that the backward can be queued behind the forward; a
+    call under stream capture leaves nothing."""
     graph, (q, k, v, scale, dropout_p, seed, table, etype) = args[:8], args[8:]
     if not (_served_natively(graph) and _native_takes(etype) and _g.rel_bias_forward_tiles is _REL_FORM):
         return BPTRelAttention.apply(*args)
     o = _native.rel_attention(*graph, q, k, v, scale, dropout_p, seed & (2 ** 64 - 1), table, etype)
     if o is not None:
         return o
-    generation = _native.generation()
+    if not q.is_cuda or _g.capturing(q):
+        return BPTRelAttention.apply(*args)
+    generation, on_tiles = _native.generation(), []
     train = torch.is_grad_enabled() and any(x.requires_grad for x in (q, k, v, table))
-    if train:
+    if train and _rel_aux_key(etype, *graph[4:7], table.size(0)) not in _rel_aux_cache:      # (a new graph)
         _g.prepare_rel_training(*graph, q, k, dropout_p)
-    o = BPTRelAttention.apply(*args)
-    aux = _rel_aux(etype, graph[4], graph[5], graph[6], table.size(0))
-    if aux.get("on_tiles"):                          # (the call that has just run took the tile form)
-        _g.remember_rel(generation, *graph, q, k, dropout_p, table, etype, aux, train)
+    o = BPTRelAttention.apply(*args, on_tiles)
+    if on_tiles:
+        _g.remember_rel(generation, *graph, q, k, dropout_p, table, etype, *on_tiles, train)
     return o
 
 
 _rel_aux_cache = {}
+
+
+def _rel_aux_key(etype, col, indptr_c, eid_c, n_types):
+    return tuple((t.data_ptr(), t.numel(), t._version) for t in (etype, col, indptr_c, eid_c)) + (str(etype.device), n_types)
+
+
+def _written(device):
+    """Waits until the current stream has written the index tensors just made: whichever stream serves the next call reads them."""
+    if device.type == "cuda":
+        torch.cuda.current_stream(device).synchronize()
 
 
 def _rel_aux(etype, col, indptr_c, eid_c, n_types):
@@ -207,7 +227,7 @@ def _rel_aux(etype, col, indptr_c, eid_c, n_types):
     used_types (n_used,) int32, the types that occur in a slot, ascending; used (n_types,) int32, the number of every
     type in that list (-1 for the others); number_slot, the number of every slot's type.  Built where etype lives;
     two scalars are read back (the range check and n_used)."""
-    key = tuple((t.data_ptr(), t.numel(), t._version) for t in (etype, col, indptr_c, eid_c)) + (str(etype.device), n_types)
+    key = _rel_aux_key(etype, col, indptr_c, eid_c, n_types)
     hit = _rel_aux_cache.get(key)
     if hit is None:
         et = etype.detach()
@@ -222,6 +242,7 @@ def _rel_aux(etype, col, indptr_c, eid_c, n_types):
         used_types = torch.nonzero(present).flatten().to(torch.int32)           # (the read-back of n_used)
         hit = {"etype_slot": etype_slot, "used": used, "used_types": used_types, "n_used": used_types.numel(),
                "number_slot": used.index_select(0, etype_slot).to(torch.int64), "keep": (etype, col, indptr_c, eid_c)}
+        _written(et.device)
         if len(_rel_aux_cache) > 16:
             _rel_aux_cache.clear()
         _rel_aux_cache[key] = hit           # "keep" holds the tensors so that their data_ptrs are not reused while cached
