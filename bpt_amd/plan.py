@@ -9,6 +9,7 @@ layers, forward and backward) hit the cache.  The cache keeps the key tensors al
 """
 import collections
 import ctypes
+import itertools
 import sys
 import threading
 import types
@@ -791,17 +792,17 @@ class PlanCache:
             if all(any(p is plan for p, _ in reversed(self._d.values())) for plan in plans):
                 getattr(self.native, how)(*choice, plans)
 
-    def _evict(self):
-        # called with the lock held; the newest entry always stays
+    def _evict(self, new=1):
+        # called with the lock held; new: how many have just been put here together.  The newest entry always stays, and those before it go last
         if self._counted != PlanCache.grown:
             self._counted, self._total = PlanCache.grown, sum(p.device_bytes() for p, _ in self._d.values())
         total = self._total
         if len(self._d) <= self._cap and total <= self._max_bytes:
             return
-        if self.native is not None and len(self._d) > 1:
-            newest = next(reversed(self._d))
+        if self.native is not None and len(self._d) > new:
+            newest = list(itertools.islice(reversed(self._d), new))[::-1]
             used = {id(p) for p in self.native.take_used()}
-            for key in [k for k, (p, _) in self._d.items() if id(p) in used] + [newest]:
+            for key in [k for k, (p, _) in self._d.items() if id(p) in used] + newest:
                 self._d.move_to_end(key)
         while len(self._d) > max(self._cap, 1) or (len(self._d) > 1 and total > self._max_bytes):
             _, (p, _) = self._d.popitem(last=False)
@@ -906,7 +907,7 @@ class PlanCache:
                 return None                         # (as in get: another thread's stay)
             for key, plan, side in zip(keys, plans, sides):
                 self._insert(key, plan, side[:4])
-            self._evict()
+            self._evict(len(keys))
         return plans
 
     def clear(self):
