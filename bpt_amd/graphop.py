@@ -923,7 +923,8 @@ def _prepare_rows(generation, cfg, graph, q, k, dropout_p):
     h, d = q.size(1), q.size(2)
     if not (cfg.use_groups and _tiles(q, h, d, None, dropout_p, None, cfg)) or TILE_BACKWARD is not None:
         return
-    plans = plan_cache.put_plans([(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0)), (row, indptr_r, eid_r, indices_r, k.size(0), q.size(0))])
+    sides = [(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0)), (row, indptr_r, eid_r, indices_r, k.size(0), q.size(0))]
+    plans = plan_cache.put_plans(sides) if plan_cache.may_hold((), sides) else None
     if plans is None:
         return
     pi = plan_cache.get(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), prefer_device=True, built=plans[0])
@@ -1017,8 +1018,17 @@ def prepare_rel_training(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, 
         return
     seg = _tile_seg_without_plan(col, eid_c.size(0), q, k, h, d, dropout_p, q, cfg)
     if seg is not None:
-        plan_cache.put_tile_plans([(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg, None),
-                                   (row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg, _plan.tile_order_src(k.size(0), eid_r.size(0)))])
+        sides = [(col, indptr_c, eid_c, indices_c, q.size(0), k.size(0), seg, None),
+                 (row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg, _plan.tile_order_src(k.size(0), eid_r.size(0)))]
+        if plan_cache.may_hold(sides):       # (they are asked for again through the cache)
+            plan_cache.put_tile_plans(sides)
+
+
+def _rel_plans_fit(col, eid_c, row, eid_r, q, k, train):
+    """Whether the cache may hold the plans of a layer with relative positions together: both sides' and, for a backward, that of the term's
+    gradient.  Where it does not, asking for them ahead of the backward or again for the native host path drops one for the next."""
+    side = lambda units, eid, n: (units, None, eid, None, n)
+    return plan_cache.may_hold([side(col, eid_c, q.size(0)), side(row, eid_r, k.size(0))], [side(col, eid_c, q.size(0))] if train else ())
 
 
 def prepare_rel_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p, rows_slot, number_slot, n_used):
@@ -1026,20 +1036,23 @@ def prepare_rel_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, 
     for, ahead of the forward's kernels.  Both are waited for when they are new, and the backward's wait would be for all that is queued by
     then.  Nothing under stream capture."""
     graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
-    hit = None if capturing(q) else _pair_order(*graph, q, k, dropout_p)
+    hit = None if capturing(q) or not _rel_plans_fit(col, eid_c, row, eid_r, q, k, True) else _pair_order(*graph, q, k, dropout_p)
     if hit is not None:
         _rel_backward_plans(hit[0], *graph, q, k, rows_slot, number_slot, n_used)
 
 
 def _rel_backward_plans(pi, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, rows_slot, number_slot, n_used):
     """(the out-side's plan, its struct linked to the in-side's plan pi, the plan of the term's gradient), as attention_backward and
-    rel_bias_backward ask for them; None where the sides do not belong together."""
+    rel_bias_backward ask for them; None where the sides do not belong together or the cache cannot hold the third plan beside them."""
     order_src = _plan.tile_order_src(k.size(0), eid_r.size(0))
     po = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg_len=_tile_seg_of(eid_c.size(0), q.size(0), k.size(0)),
                         prefer_device=True, groups=(TILE_ROWS, order_src))
     if po.n_edges != pi.n_edges or not po.covers_all_edges:
         return None
-    return (po, po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True),
+    out_struct = po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True)
+    if not plan_cache.may_hold((), [(col, indptr_c, rows_slot, number_slot, q.size(0))], (pi, po)):
+        return None
+    return (po, out_struct,
             plan_cache.get(col, indptr_c, rows_slot, number_slot, q.size(0), max(n_used, 1), prefer_device=True))
 
 
@@ -1048,7 +1061,7 @@ def remember_rel(generation, row, indptr_r, eid_r, indices_r, col, indptr_c, eid
     which rel_bias_forward_tiles has just been found to run: the in-CSR's tile plan, the out-CSR's linked to it, the plan of the term's
     gradient, and the term's index tensors (op._rel_aux; held: those in the order of the tiles)."""
     graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
-    if any(t.dtype != torch.int64 for t in graph) or TILE_BACKWARD is not None:
+    if any(t.dtype != torch.int64 for t in graph) or TILE_BACKWARD is not None or not _rel_plans_fit(col, eid_c, row, eid_r, q, k, train):
         return                       # (with the hook set the passes choose for themselves)
     hit = _pair_order(*graph, q, k, dropout_p)
     if hit is None or held[0] is not hit[1]["pair_of_eid"]:

@@ -858,12 +858,14 @@ class PlanCache:
             self._evict()
         return plan
 
-    def may_hold(self, sides):
-        """False if the tile plans of these sides (as put_tile_plans takes them) cannot stand here together: by their number, or by
-        the bytes that they hold at the least (row pointers, neighbours and edge ids, the groups' edge ids twice, their entries)."""
-        at_least = sum(4 * side[4] + 17 * side[2].numel() for side in sides)
+    def may_hold(self, sides, plain=(), plans=()):
+        """False if the tile plans of these sides (as put_tile_plans takes them), the plans without groups of the sides in `plain` and these
+        plans cannot stand here together: by their number, or by the bytes that they hold, where they are not built at the least (row
+        pointers, neighbours and edge ids; the groups' edge ids twice, their entries)."""
+        at_least = sum(4 * side[4] + 17 * side[2].numel() for side in sides) + sum(4 * side[4] + 8 * side[2].numel() for side in plain)
+        at_least += sum(p.device_bytes() for p in plans)
         with self._lock:
-            return len(sides) <= self._cap and at_least <= self._max_bytes
+            return len(sides) + len(plain) + len(plans) <= self._cap and at_least <= self._max_bytes
 
     def put_tile_plans(self, sides):
         """What get() would build one after the other for a training step on tiles, built together (DevicePlan.tile_plans; sides as

@@ -41,9 +41,35 @@ def built(cache, passes, call):
     return (cache.misses - before) / passes
 
 
-@pytest.mark.parametrize("capacity", [2])
+def test_relative_positions_with_two_plans(cache_of):
+    """Three plans (both sides, the term's gradient), each built once a pass; with room for three, none once they are there."""
+    args, etype, n = graph(700)
+    x = [torch.randn(n, 8, 64, device=DEV, requires_grad=True) for _ in range(3)]
+    table = torch.randn(1000, 64, device=DEV, requires_grad=True)
+    for capacity, most in ((2, 3), (3, 0)):
+        cache = cache_of(capacity=capacity)
+        training_pass(args, etype, x, table)
+        assert built(cache, 4, lambda: training_pass(args, etype, x, table)) == most
+
+
+def test_relative_positions_with_room_for_two_plans_bytes(cache_of):
+    """The same where what stands in the way are bytes: what both sides' plans hold, and some more than that of the third."""
+    args, etype, n = graph(700)
+    x = [torch.randn(n, 8, 64, device=DEV, requires_grad=True) for _ in range(3)]
+    table = torch.randn(1000, 64, device=DEV, requires_grad=True)
+    cache = cache_of(capacity=64)
+    training_pass(args, etype, x, table)
+    held = [p.device_bytes() for p, _ in cache._d.values()]
+    assert len(held) == 3
+    for room, most in ((sum(held) - 1, 3), (sum(held), 0)):
+        cache = cache_of(max_bytes=room)
+        training_pass(args, etype, x, table)
+        assert built(cache, 4, lambda: training_pass(args, etype, x, table)) <= most
+
+
+@pytest.mark.parametrize("capacity", [1, 2])
 def test_new_small_graphs(cache_of, capacity):
-    """A new graph that is left to the kernels that walk rows: one plan for each side."""
+    """A new graph that is left to the kernels that walk rows: one plan for each side, with room for one as with room for both."""
     cache = cache_of(capacity=capacity)
     x = None
 
