@@ -99,6 +99,10 @@ bool like(const Tensor &t, const Tensor &q) {
     return t.scalar_type() == q.scalar_type() && t.device() == q.device() && t.is_contiguous();
 }
 
+bool float_matrix(const Tensor &t, const at::Device &dev, int64_t rows, int64_t columns) {
+    return t.scalar_type() == at::kFloat && t.device() == dev && t.is_contiguous() && t.dim() == 2 && t.size(0) == rows && t.size(1) == columns;
+}
+
 // false: an index tensor is not what the kernels take
 bool make_key(Key &k, Kind kind, const std::vector<const Tensor *> &index, const at::Device &dev, std::initializer_list<int64_t> extra) {
     std::memset(static_cast<void *>(&k), 0, sizeof(Key));
@@ -438,8 +442,13 @@ std::optional<Three> rel_forward_known(const EntryPtr &e, const Tensor &q, const
 std::optional<std::array<Tensor, 4>> rel_backward_known(const EntryPtr &e, const Tensor &q, const Tensor &k, const Tensor &v, const Tensor &o,
                                                         const Tensor &lse, const Tensor &bias, const Tensor &table, const Tensor &d_o, double scale,
                                                         double p, uint64_t seed) {
-    if (!like(d_o, q) || d_o.sizes() != q.sizes()) return std::nullopt;
-    const int h = (int)q.size(1), d = (int)q.size(2), dt = dtype_code(q.scalar_type());
+    // (the entry was found for the forward's tensors; a hook on saved tensors may give back others)
+    Shape s;
+    if (!attention_shape(q, k, v, p, s) || !like(o, q) || !like(d_o, q) || o.sizes() != q.sizes() || d_o.sizes() != q.sizes()) return std::nullopt;
+    if (s.nq != e->a.n_rows || s.nk != e->b.n_rows || !float_matrix(lse, q.device(), s.nq, s.h) || !float_matrix(bias, q.device(), s.h, e->a.n_edges) ||
+        !like(table, q) || table.dim() != 2 || table.size(0) != e->more[REL_USED].numel() || table.size(1) != s.d)
+        return std::nullopt;
+    const int h = s.h, d = s.d, dt = s.dt;
     c10::DeviceGuard guard(q.device());
     void *stream = stream_of(q.device());
     Tensor dq = at::empty_like(q), dk = at::empty_like(k), dv = at::empty_like(v), ds = at::empty_like(bias), dtable = at::empty_like(table);
