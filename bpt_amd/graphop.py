@@ -1031,19 +1031,16 @@ def _rel_plans_fit(col, eid_c, row, eid_r, q, k, train):
     return plan_cache.may_hold([side(col, eid_c, q.size(0)), side(row, eid_r, k.size(0))], [side(col, eid_c, q.size(0))] if train else ())
 
 
-def prepare_rel_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p, rows_slot, number_slot, n_used):
-    """Where the term is in the order of the tiles: the linked out-side and the plan of the term's gradient, which the backward is going to ask
-    for, ahead of the forward's kernels.  Both are waited for when they are new, and the backward's wait would be for all that is queued by
-    then.  Nothing under stream capture."""
+def prepare_rel_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p, held, number_slot, n_used):
+    """Where the term is in the order of the tiles (held): (the in-side's plan, its struct, the out-side's plan, its struct linked to the in-side's,
+    the plan of the term's gradient) as both passes are going to ask for them, ahead of the forward's kernels: they are waited for when they
+    are new, and the backward's wait would be for all that is queued by then.  None where the sides do not belong together or the cache
+    cannot hold the plans together."""
     graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
-    hit = None if capturing(q) or not _rel_plans_fit(col, eid_c, row, eid_r, q, k, True) else _pair_order(*graph, q, k, dropout_p)
-    if hit is not None:
-        _rel_backward_plans(hit[0], *graph, q, k, rows_slot, number_slot, n_used)
-
-
-def _rel_backward_plans(pi, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, rows_slot, number_slot, n_used):
-    """(the out-side's plan, its struct linked to the in-side's plan pi, the plan of the term's gradient), as attention_backward and
-    rel_bias_backward ask for them; None where the sides do not belong together or the cache cannot hold the third plan beside them."""
+    hit = _pair_order(*graph, q, k, dropout_p) if _rel_plans_fit(col, eid_c, row, eid_r, q, k, True) else None
+    if hit is None or held[0] is not hit[1]["pair_of_eid"]:
+        return None
+    pi, rows_slot = hit[0], held[1]
     order_src = _plan.tile_order_src(k.size(0), eid_r.size(0))
     po = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg_len=_tile_seg_of(eid_c.size(0), q.size(0), k.size(0)),
                         prefer_device=True, groups=(TILE_ROWS, order_src))
@@ -1052,30 +1049,24 @@ def _rel_backward_plans(pi, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_
     out_struct = po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True)
     if not plan_cache.may_hold((), [(col, indptr_c, rows_slot, number_slot, q.size(0))], (pi, po)):
         return None
-    return (po, out_struct,
-            plan_cache.get(col, indptr_c, rows_slot, number_slot, q.size(0), max(n_used, 1), prefer_device=True))
+    return pi, hit[1]["struct"], po, out_struct, plan_cache.get(col, indptr_c, rows_slot, number_slot, q.size(0), max(n_used, 1), prefer_device=True)
 
 
-def remember_rel(generation, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p, table, etype, aux, held, train):
+def remember_rel(generation, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p, table, etype, aux, held, plans, train):
     """Leaves with the native host path what a forward (train: and a backward) with the relative-position term takes for these arguments, of
-    which rel_bias_forward_tiles has just been found to run: the in-CSR's tile plan, the out-CSR's linked to it, the plan of the term's
-    gradient, and the term's index tensors (op._rel_aux; held: those in the order of the tiles)."""
+    which rel_bias_forward_tiles has just been found to run: the plans (train: prepare_rel_backward's, or None) and the term's index
+    tensors (op._rel_aux; held: those in the order of the tiles)."""
     graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
-    if any(t.dtype != torch.int64 for t in graph) or TILE_BACKWARD is not None or not _rel_plans_fit(col, eid_c, row, eid_r, q, k, train):
+    if any(t.dtype != torch.int64 for t in graph) or TILE_BACKWARD is not None or (plans is None if train else not _rel_plans_fit(col, eid_c, row, eid_r, q, k, False)):
         return                       # (with the hook set the passes choose for themselves)
-    hit = _pair_order(*graph, q, k, dropout_p)
-    if hit is None or held[0] is not hit[1]["pair_of_eid"]:
-        return
-    pi, in_struct = hit[0], hit[1]["struct"]
     index, numbers = list(graph) + [etype], [q.size(0), k.size(0), q.size(1), q.size(2), _dtype(q), int(dropout_p > 0.0), table.size(0)]
     if not train:
-        plan_cache.remember((pi,), generation, _native.REL_FWD, index, numbers, ctypes.addressof(in_struct), 0, 0, [aux["used_types"], held[2]],
-                            how="remember_rel")
+        hit = _pair_order(*graph, q, k, dropout_p)
+        if hit is not None and held[0] is hit[1]["pair_of_eid"]:
+            plan_cache.remember((hit[0],), generation, _native.REL_FWD, index, numbers, ctypes.addressof(hit[1]["struct"]), 0, 0,
+                                [aux["used_types"], held[2]], how="remember_rel")
         return
-    plans = _rel_backward_plans(pi, *graph, q, k, held[1], aux["number_slot"], aux["n_used"])
-    if plans is None:
-        return
-    po, out_struct, rel = plans
+    pi, in_struct, po, out_struct, rel = plans
     rel_struct = _by_pair(rel.struct)
     plan_cache.remember((pi, po, rel), generation, _native.REL_TRAIN, index, numbers, ctypes.addressof(in_struct), ctypes.addressof(out_struct),
                         ctypes.addressof(rel_struct), [aux["used_types"], held[2], aux["used"], held[1], aux["number_slot"]], how="remember_rel")

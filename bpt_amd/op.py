@@ -105,9 +105,9 @@ class BPTRelAttention(Function):
 
     @staticmethod
     def forward(ctx, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, scale, dropout_p, seed,
-                table, etype, on_tiles=None):
-        """on_tiles: None or a list, which receives the term's index tensors (_rel_aux, and those in the order of the tiles) where the term is
-        formed over the tiles."""
+                table, etype, on_tiles=None, train=False):
+        """on_tiles: None or, outside of stream capture, a list, which receives the term's index tensors (_rel_aux, and those in the order of the
+        tiles) and, for a call that is going to have a backward (train), both passes' plans, where the term is formed over the tiles."""
         aux = _rel_aux(etype, col, indptr_c, eid_c, table.size(0))
         table = table.contiguous()
         # (the gradient kernel's configuration is asked for here: the SpMM form is then chosen for both passes up front)
@@ -119,22 +119,23 @@ class BPTRelAttention(Function):
         pair = _g.attention_pair_rows(*graph, dropout_p) if ctx.on_chip else None
         ctx.rows_slot = None
         if pair is not None:
-            held = aux.get("rows_slot")
-            if held is None or held[0] is not pair:
+            held, plans = aux.get("rows_slot"), None
+            new = held is None or held[0] is not pair
+            if new:
                 rows_slot = pair.index_select(0, eid_c).contiguous()
                 # per pair number: the number of its edge's type and which row of its tile its destination is
                 types = torch.empty_like(aux["number_slot"]).index_copy_(0, rows_slot, aux["number_slot"]).to(torch.int32)
                 held = (pair, rows_slot, (types | (_g.attention_pair_members(*graph, dropout_p) << 8)).contiguous())
-                if not _g.capturing(q):                           # (what a captured graph fills is there after its replays only)
-                    _written(q.device)
-                    aux["rows_slot"] = held
             ctx.rows_slot = held[1]
-            if on_tiles is not None and any(ctx.needs_input_grad):
-                _g.prepare_rel_backward(*graph, dropout_p, held[1], aux["number_slot"], aux["n_used"])
+            if on_tiles is not None and train:
+                plans = _g.prepare_rel_backward(*graph, dropout_p, held, aux["number_slot"], aux["n_used"])
+            if new and not _g.capturing(q):                       # (what a captured graph fills is there after its replays only)
+                _written(q.device)                                # (a new plan, where one was just built, has been waited for with these)
+                aux["rows_slot"] = held
             try:
                 bias = _g.rel_bias_forward_tiles(*graph, table, aux["used_types"], held[2], dropout_p)
                 if on_tiles is not None:
-                    on_tiles.extend((aux, held))
+                    on_tiles.extend((aux, held, plans))
             except _g.BptStatusError as err:
                 # (many types in use need more than 64 KB of LDS there, which a runtime may refuse: the kernel over the
                 # in-CSR writes the same layout from within 64 KB)
@@ -159,7 +160,7 @@ class BPTRelAttention(Function):
         if ctx.rows_slot is not None:
             dq, dk, dv, dtable = _rel_backward(*ctx.saved_tensors, do, ctx.scale, ctx.dropout_p, ctx.seed, ctx.rows_slot, aux["number_slot"],
                                                aux["used"], aux["used_types"])
-            return None, None, None, None, None, None, None, None, dq, dk, dv, None, None, None, dtable, None, None
+            return None, None, None, None, None, None, None, None, dq, dk, dv, None, None, None, dtable, None, None, None
         dq, dk, dv, ds = _g.attention_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c,
                                                q, k, v, o, lse, do, ctx.scale, ctx.dropout_p, ctx.seed, bias=bias)
         if ctx.on_chip:
@@ -172,7 +173,7 @@ class BPTRelAttention(Function):
             dq = vector_spmm_forward(col, indptr_c, eid_c, aux["etype_slot"], ds, table_h, n_rows=q.size(0), out=dq)
             dtable = vector_spmm_forward(t_row, t_indptr, t_order, t_dst, ds, q, n_rows=table.size(0))
             dtable = dtable.float().sum(1).to(table.dtype)
-        return None, None, None, None, None, None, None, None, dq, dk, dv, None, None, None, dtable, None, None
+        return None, None, None, None, None, None, None, None, dq, dk, dv, None, None, None, dtable, None, None, None
 
 
 def _rel_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, v, o, lse, bias, table, do, scale, dropout_p, seed, rows_slot,
@@ -203,7 +204,7 @@ def _rel_attention(*args):
     train = torch.is_grad_enabled() and any(x.requires_grad for x in (q, k, v, table))
     if train and _rel_aux_key(etype, *graph[4:7], table.size(0)) not in _rel_aux_cache:      # (a new graph)
         _g.prepare_rel_training(*graph, q, k, dropout_p)
-    o = BPTRelAttention.apply(*args, on_tiles)
+    o = BPTRelAttention.apply(*args, on_tiles, train)
     if on_tiles:
         _g.remember_rel(generation, *graph, q, k, dropout_p, table, etype, *on_tiles, train)
     return o
@@ -237,12 +238,16 @@ def _rel_aux(etype, col, indptr_c, eid_c, n_types):
             raise ValueError("edge type out of range")
         etype_slot = et.index_select(0, eid_c).contiguous()
         present = torch.zeros(n_types, dtype=torch.bool, device=et.device).index_fill_(0, etype_slot, True)
-        number = torch.cumsum(present, 0, dtype=torch.int32) - 1
-        used = torch.where(present, number, torch.full_like(number, -1)).contiguous()
-        used_types = torch.nonzero(present).flatten().to(torch.int32)           # (the read-back of n_used)
-        hit = {"etype_slot": etype_slot, "used": used, "used_types": used_types, "n_used": used_types.numel(),
-               "number_slot": used.index_select(0, etype_slot).to(torch.int64), "keep": (etype, col, indptr_c, eid_c)}
-        _written(et.device)
+        number = torch.cumsum(present, 0) - 1
+        used = torch.where(present, number, -1).to(torch.int32)
+        # every type in use at its number, the others behind all of them
+        types = torch.empty(n_types + 1, dtype=torch.int32, device=et.device).scatter_(
+            0, torch.where(present, number, n_types), torch.arange(n_types, dtype=torch.int32, device=et.device))
+        number_slot = number.index_select(0, etype_slot)
+        # the read-back of n_used comes last: all of them are there for whichever stream serves the next call
+        n_used = int(number[-1]) + 1 if n_types else 0
+        hit = {"etype_slot": etype_slot, "used": used, "used_types": types[:n_used], "n_used": n_used, "number_slot": number_slot,
+               "keep": (etype, col, indptr_c, eid_c)}
         if len(_rel_aux_cache) > 16:
             _rel_aux_cache.clear()
         _rel_aux_cache[key] = hit           # "keep" holds the tensors so that their data_ptrs are not reused while cached

@@ -99,6 +99,22 @@ def test_a_new_graphs_forward_waits_for_none_of_its_kernels(train, monkeypatch):
     assert torch.equal(o, again)
 
 
+def test_a_forward_alone_builds_no_plan_of_the_backward():
+    """Inference with parameters that would have gradients: both sides' tile plans, without the gradient's."""
+    from bpt_amd import op, plan
+    args, etype, n = graph(700)
+    (q, k, v), table, _ = inputs(n, 8, 64, torch.float32)
+    held = {}
+    for train in (False, True):
+        forget_all()
+        with torch.set_grad_enabled(train):
+            op.bpt_attention(*args, q, k, v, rel_table=table, etype=etype)
+        held[train] = len(plan.plan_cache.held())
+        with torch.no_grad():
+            assert known(args, q, k, v, 0.0, table, etype)
+    assert held == {False: 2, True: 3}
+
+
 def test_calls_off_the_tiles_leave_nothing(monkeypatch):
     from bpt_amd import graphop, op
     forget_all()
