@@ -357,6 +357,44 @@ template <int KPT> __device__ __forceinline__ void lds_radix(uint32_t *word, int
     }
 }
 
+// start[0 .. n] of a workgroup of 16 wavefronts: where nothing was put (INT32_MAX), what was put next behind it; start[n] was put.  (The thread
+// of an edge or unit that filled in the rows before its own went over all of them when only some late rows have edges: 4000 nodes whose edges all
+// point to the last, both sides' CSRs 60 us by the launches for larger graphs, 153 filled in by one thread, 47 by the workgroup.)
+__device__ __forceinline__ void fill_starts(int32_t *start, int n, int32_t *sh) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, per = (n + SMALL_TPB) / SMALL_TPB;
+    const int r0 = min(tid * per, n + 1), r1 = min(r0 + per, n + 1);
+    int32_t least = INT32_MAX;
+    for (int r = r0; r < r1; ++r) least = min(least, start[r]);
+    for (int d = 1; d < 64; d <<= 1) {
+        const int32_t y = __shfl_down(least, d);
+        if (lane + d < 64) least = min(least, y);
+    }
+    __syncthreads();                              // (sh may still be in use by the caller's previous step)
+    if (lane == 0) sh[wave] = least;
+    const int32_t next = __shfl_down(least, 1);
+    int32_t after = lane < 63 ? next : INT32_MAX;
+    __syncthreads();
+    for (int w = wave + 1; w < SMALL_NW; ++w) after = min(after, sh[w]);
+    for (int r = r1 - 1; r >= r0; --r) start[r] = after = min(start[r], after);
+    __syncthreads();
+}
+
+// f(own, t) for t = 0 .. n - 1 of every lane: by itself where it has few, by the wavefront together where it has many (a row with most of a graph's
+// edges).  All lanes of the wavefront are here.
+template <int K, typename F> __device__ __forceinline__ void for_each_of_lane(int n, const int32_t (&own)[K], F &&f) {
+    constexpr int FEW = 8;
+    const int lane = threadIdx.x & 63;
+    if (n <= FEW)
+        for (int t = 0; t < n; ++t) f(own, t);
+    for (uint64_t many = __ballot(n > FEW); many != 0; many &= many - 1) {
+        const int owner = __ffsll((unsigned long long)many) - 1, k = __shfl(n, owner);
+        int32_t of[K];
+#pragma unroll
+        for (int i = 0; i < K; ++i) of[i] = __shfl(own[i], owner);
+        for (int t = lane; t < k; t += 64) f(of, t);
+    }
+}
+
 // ---- base plan ---------------------------------------------------------------------------------------------------------
 // Five launches and the sort: clear; narrow the indices, check the units, find the rows; emit the items; their smallest and
 // largest neighbour; sort by the smallest.
@@ -696,7 +734,7 @@ __global__ __launch_bounds__(SMALL_TPB) void k_plan_small(PlanSides b, int32_t *
         err = first < 0 || last >= INT32_MAX ? 3 : last > n_edges ? 1 : 0;
         perm = 1;
     }
-    for (int r = tid; r <= n_rows; r += SMALL_TPB) start[r] = (int32_t)last;
+    for (int r = tid; r <= n_rows; r += SMALL_TPB) start[r] = r < n_rows ? INT32_MAX : (int32_t)last;
     __syncthreads();
     // edge slots: indices to 32 bits, eid a permutation? (the check below); units: sorted? where the rows start
 #pragma unroll 4
@@ -714,12 +752,12 @@ __global__ __launch_bounds__(SMALL_TPB) void k_plan_small(PlanSides b, int32_t *
         int bad = r < 0 || r >= n_rows ? 1 : 0;
         if (r < before || ipu[u + 1] < at) bad = 2;
         if (bad) atomicMax(&err, bad);
-        else if (before >= -1)
-            for (int64_t x = before + 1; x <= r; ++x) start[x] = (int32_t)at;
+        else if (r > before) start[r] = (int32_t)at;
     }
     __syncthreads();
     int32_t n_items = 0, n_heavy = 0, n_slots = 0, degree = 0;
     if (err == 0) {
+        fill_starts(start, n_rows, sh);
         for (int r = tid; r <= n_rows; r += SMALL_TPB) S.rowptr[r] = start[r];
         // items of every row in row order, the heavy rows: a run of rows a thread
         int4 *const items = indices ? S.items_tmp : S.items;
@@ -739,16 +777,22 @@ __global__ __launch_bounds__(SMALL_TPB) void k_plan_small(PlanSides b, int32_t *
         if ((tid & 63) == 0) sh[tid >> 6] = degree;
         __syncthreads();
         for (int w = 0; w < NW; ++w) degree = max(degree, sh[w]);
-        for (int r = r0; r < r1; ++r) {
-            const int begin = start[r], end = start[r + 1], n = segments(end - begin);
-            if (n == 0) items[item++] = make_int4(r, begin, end, -1);
-            else {
+        for (int i = 0; i < per; ++i) {
+            const int r = r0 + i, begin = r < r1 ? start[r] : 0, end = r < r1 ? start[r + 1] : 0, n = segments(end - begin);
+            if (n == 0) {
+                if (r < r1) items[item++] = make_int4(r, begin, end, -1);
+            } else {
                 S.heavy[3 * hv] = r;
                 S.heavy[3 * hv + 1] = slot;
                 S.heavy[3 * hv + 2] = n;
                 ++hv;
-                for (int t = 0; t < n; ++t) items[item++] = make_int4(r, begin + t * seg_len, min(end, begin + (t + 1) * seg_len), slot++);
             }
+            const int32_t own[5] = {r, begin, end, item, slot};
+            for_each_of_lane(n, own, [&](const int32_t (&o)[5], int t) {
+                items[o[3] + t] = make_int4(o[0], o[1] + t * seg_len, min(o[2], o[1] + (t + 1) * seg_len), o[4] + t);
+            });
+            item += n;
+            slot += n;
         }
         for (int p = tid; p < n_edges; p += SMALL_TPB)
             if (S.seen[S.eid32[p]] != p) perm = 0;
@@ -2017,17 +2061,18 @@ __global__ __launch_bounds__(SMALL_TPB) void k_csr_small(CsrSides g, int n_edges
     }
     const int any_bad = __syncthreads_or(bad ? 1 : 0);
     lds_radix<CSR_SMALL_EDGES / SMALL_TPB>(word, n_edges, CSR_SMALL_BITS, 32 - __clz(n_nodes | 1), start, sh);
-    // slots, and where the rows start: a slot whose row is not the one before's starts the rows in between too
+    for (int x = tid; x <= n_nodes; x += SMALL_TPB) start[x] = x < n_nodes ? INT32_MAX : n_edges;
+    __syncthreads();
+    // slots, and where the rows start
     for (int at = tid; at < n_edges; at += SMALL_TPB) {
         const uint32_t w = word[at];
         const int e = (int)(w & ((1 << CSR_SMALL_BITS) - 1)), r = (int)(w >> CSR_SMALL_BITS), before = at > 0 ? (int)(word[at - 1] >> CSR_SMALL_BITS) : -1;
         c.eid[at] = e;
         c.indices[at] = c.cols[e];
-        for (int x = before + 1; x <= r; ++x) start[x] = at;
+        if (r != before) start[r] = at;                           // (row n_nodes: the first bad edge)
     }
-    const int from = n_edges > 0 ? (int)(word[n_edges - 1] >> CSR_SMALL_BITS) + 1 : 0;
-    for (int x = from + tid; x <= n_nodes; x += SMALL_TPB) start[x] = n_edges;
     __syncthreads();
+    fill_starts(start, n_nodes, sh);
     for (int r = tid; r <= n_nodes; r += SMALL_TPB) c.indptr[r] = start[r];
     // the units of builder.pyx:305-321: a run of rows a thread
     const int per = (n_nodes + SMALL_TPB - 1) / SMALL_TPB, r0 = min(tid * per, n_nodes), r1 = min(r0 + per, n_nodes);
@@ -2035,11 +2080,15 @@ __global__ __launch_bounds__(SMALL_TPB) void k_csr_small(CsrSides g, int n_edges
     int32_t units = 0, total;
     for (int r = r0; r < r1; ++r) units += units_of(r);
     int32_t at = block_excl_sum<NW>(units, sh, total);
-    for (int r = r0; r < r1; ++r)
-        for (int u = 0, n = units_of(r); u < n; ++u, ++at) {
-            c.unit_row[at] = r;
-            c.unit_ptr[at] = start[r] + (int64_t)u * chunk;
-        }
+    for (int i = 0; i < per; ++i) {
+        const int r = r0 + i, n = r < r1 ? units_of(r) : 0;
+        const int32_t own[3] = {r, at, r < r1 ? start[r] : 0};
+        for_each_of_lane(n, own, [&](const int32_t (&o)[3], int u) {
+            c.unit_row[o[1] + u] = o[0];
+            c.unit_ptr[o[1] + u] = o[2] + (int64_t)u * chunk;
+        });
+        at += n;
+    }
     if (tid == 0) {
         c.info[0] = any_bad ? 1 : 0;
         c.info[1] = total;
