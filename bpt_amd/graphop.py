@@ -937,7 +937,7 @@ def _prepare_rows(generation, cfg, graph, q, k, dropout_p):
         plan_cache.remember((pi, po), generation, _native.ATTN_BWD, list(graph), numbers, ctypes.addressof(pi.struct), ctypes.addressof(po.struct))
 
 
-def _pair_order(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p):
+def attention_pair_order(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p):
     """The in-CSR's tile plan and its pair-order tables (DevicePlan.bias_rows) where attention_forward and
     attention_backward will both run on the tile kernels with a per-edge score term for these arguments, else None."""
     cfg = _SETTINGS
@@ -969,14 +969,14 @@ def attention_pair_rows(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, i
     numbers of the in-CSR's tile plan).  A score term stored in that order, head-major ((h, E): the value of edge e and a
     head at [head, number[e]]), and passed with bias_by_pair=True is read, and its gradient written, in runs of
     neighbouring values per tile, with no index read on the way, instead of rows scattered by edge id."""
-    hit = _pair_order(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p)
+    hit = attention_pair_order(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p)
     return None if hit is None else hit[1]["pair_of_eid"]
 
 
 def attention_pair_members(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p=0.0):
     """Where attention_pair_rows gives numbers: the (E,) int32 tensor with, for every pair number, which of its tile's
     16 rows the pair's destination is (what rel_bias_forward_tiles needs beside the pair's edge type); else None."""
-    hit = _pair_order(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p)
+    hit = attention_pair_order(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p)
     return None if hit is None else hit[1]["member_of_pair"]
 
 
@@ -997,7 +997,7 @@ def rel_bias_forward_tiles(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c
         raise ValueError("used_types must be a 1-D int32 tensor of at most table.size(0) elements")
     if pair_types.dtype != torch.int32 or tuple(pair_types.shape) != (E,):
         raise ValueError(f"pair_types must be int32 ({E},)")
-    hit = _pair_order(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p)
+    hit = attention_pair_order(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p)
     if hit is None:
         raise RuntimeError("rel_bias_forward_tiles: these arguments do not run on the tile kernels (ask attention_pair_rows() first)")
     bias = torch.empty((h, E), dtype=torch.float32, device=q.device)
@@ -1031,16 +1031,14 @@ def _rel_plans_fit(col, eid_c, row, eid_r, q, k, train):
     return plan_cache.may_hold([side(col, eid_c, q.size(0)), side(row, eid_r, k.size(0))], [side(col, eid_c, q.size(0))] if train else ())
 
 
-def prepare_rel_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p, held, number_slot, n_used):
-    """Where the term is in the order of the tiles (held): (the in-side's plan, its struct, the out-side's plan, its struct linked to the in-side's,
-    the plan of the term's gradient) as both passes are going to ask for them, ahead of the forward's kernels: they are waited for when they
+def prepare_rel_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, order, rows_slot, number_slot, n_used):
+    """Where the term is in the order of the tiles (order: attention_pair_order's): (the out-side's plan, its struct linked to the in-side's, the
+    plan of the term's gradient) as the backward is going to ask for them, ahead of the forward's kernels: they are waited for when they
     are new, and the backward's wait would be for all that is queued by then.  None where the sides do not belong together or the cache
     cannot hold the plans together."""
-    graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
-    hit = _pair_order(*graph, q, k, dropout_p) if _rel_plans_fit(col, eid_c, row, eid_r, q, k, True) else None
-    if hit is None or held[0] is not hit[1]["pair_of_eid"]:
+    if not _rel_plans_fit(col, eid_c, row, eid_r, q, k, True):
         return None
-    pi, rows_slot = hit[0], held[1]
+    pi = order[0]
     order_src = _plan.tile_order_src(k.size(0), eid_r.size(0))
     po = plan_cache.get(row, indptr_r, eid_r, indices_r, k.size(0), q.size(0), seg_len=_tile_seg_of(eid_c.size(0), q.size(0), k.size(0)),
                         prefer_device=True, groups=(TILE_ROWS, order_src))
@@ -1049,24 +1047,23 @@ def prepare_rel_backward(row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, 
     out_struct = po.linked_to(pi, TILE_ROWS, order=order_src, partner_order=None, pair_numbers=True)
     if not plan_cache.may_hold((), [(col, indptr_c, rows_slot, number_slot, q.size(0))], (pi, po)):
         return None
-    return pi, hit[1]["struct"], po, out_struct, plan_cache.get(col, indptr_c, rows_slot, number_slot, q.size(0), max(n_used, 1), prefer_device=True)
+    return po, out_struct, plan_cache.get(col, indptr_c, rows_slot, number_slot, q.size(0), max(n_used, 1), prefer_device=True)
 
 
-def remember_rel(generation, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p, table, etype, aux, held, plans, train):
+def remember_rel(generation, row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k, dropout_p, table, etype, aux, held, order, plans, train):
     """Leaves with the native host path what a forward (train: and a backward) with the relative-position term takes for these arguments, of
-    which rel_bias_forward_tiles has just been found to run: the plans (train: prepare_rel_backward's, or None) and the term's index
-    tensors (op._rel_aux; held: those in the order of the tiles)."""
+    which rel_bias_forward_tiles has just been found to run: the plans (order: attention_pair_order's; train: prepare_rel_backward's, or
+    None) and the term's index tensors (op._rel_aux; held: those in the order of the tiles)."""
     graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c)
     if any(t.dtype != torch.int64 for t in graph) or TILE_BACKWARD is not None or (plans is None if train else not _rel_plans_fit(col, eid_c, row, eid_r, q, k, False)):
         return                       # (with the hook set the passes choose for themselves)
     index, numbers = list(graph) + [etype], [q.size(0), k.size(0), q.size(1), q.size(2), _dtype(q), int(dropout_p > 0.0), table.size(0)]
+    pi, in_struct = order[0], order[1]["struct"]
     if not train:
-        hit = _pair_order(*graph, q, k, dropout_p)
-        if hit is not None and held[0] is hit[1]["pair_of_eid"]:
-            plan_cache.remember((hit[0],), generation, _native.REL_FWD, index, numbers, ctypes.addressof(hit[1]["struct"]), 0, 0,
-                                [aux["used_types"], held[2]], how="remember_rel")
+        plan_cache.remember((pi,), generation, _native.REL_FWD, index, numbers, ctypes.addressof(in_struct), 0, 0, [aux["used_types"], held[2]],
+                            how="remember_rel")
         return
-    pi, in_struct, po, out_struct, rel = plans
+    po, out_struct, rel = plans
     rel_struct = _by_pair(rel.struct)
     plan_cache.remember((pi, po, rel), generation, _native.REL_TRAIN, index, numbers, ctypes.addressof(in_struct), ctypes.addressof(out_struct),
                         ctypes.addressof(rel_struct), [aux["used_types"], held[2], aux["used"], held[1], aux["number_slot"]], how="remember_rel")

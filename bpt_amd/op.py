@@ -116,26 +116,27 @@ class BPTRelAttention(Function):
         # where forward and backward both run on the tile kernels, the term and its gradient are stored head-major in the
         # order in which the tiles meet the edges (rows_slot: the place of every in-CSR slot) instead of by edge id
         graph = (row, indptr_r, eid_r, indices_r, col, indptr_c, eid_c, indices_c, q, k)
-        pair = _g.attention_pair_rows(*graph, dropout_p) if ctx.on_chip else None
+        order = _g.attention_pair_order(*graph, dropout_p) if ctx.on_chip else None
         ctx.rows_slot = None
-        if pair is not None:
+        if order is not None:
+            pair = order[1]["pair_of_eid"]
             held, plans = aux.get("rows_slot"), None
             new = held is None or held[0] is not pair
             if new:
                 rows_slot = pair.index_select(0, eid_c).contiguous()
                 # per pair number: the number of its edge's type and which row of its tile its destination is
                 types = torch.empty_like(aux["number_slot"]).index_copy_(0, rows_slot, aux["number_slot"]).to(torch.int32)
-                held = (pair, rows_slot, (types | (_g.attention_pair_members(*graph, dropout_p) << 8)).contiguous())
+                held = (pair, rows_slot, (types | (order[1]["member_of_pair"] << 8)).contiguous())
             ctx.rows_slot = held[1]
             if on_tiles is not None and train:
-                plans = _g.prepare_rel_backward(*graph, dropout_p, held, aux["number_slot"], aux["n_used"])
+                plans = _g.prepare_rel_backward(*graph, order, held[1], aux["number_slot"], aux["n_used"])
             if new and not _g.capturing(q):                       # (what a captured graph fills is there after its replays only)
                 _written(q.device)                                # (a new plan, where one was just built, has been waited for with these)
                 aux["rows_slot"] = held
             try:
                 bias = _g.rel_bias_forward_tiles(*graph, table, aux["used_types"], held[2], dropout_p)
                 if on_tiles is not None:
-                    on_tiles.extend((aux, held, plans))
+                    on_tiles.extend((aux, held, order, plans))
             except _g.BptStatusError as err:
                 # (many types in use need more than 64 KB of LDS there, which a runtime may refuse: the kernel over the
                 # in-CSR writes the same layout from within 64 KB)
