@@ -1050,23 +1050,38 @@ __global__ __launch_bounds__(sm_block<WHOLE>()) void k_softmax_bwd_quads(bpt_pla
     }
 }
 
-// (Longer rows; L = 8192, k = 4: 7.7 -> 7.1 us with the first edges asked for ahead of the segments' sums, backward 8.0 -> 7.8.)
 // Split rows, second launch: block (i, j) is the j-th of gridDim.y blocks of split row i.  Every block reduces the row's segments
 // by itself (16 bytes a segment and head at most: they come from the L2), then writes its share of the row's edges.
 template <typename T, int Q, bool FWD>
 __global__ __launch_bounds__(BLOCK) void k_softmax_split_quads(bpt_plan P, const T *__restrict__ x, const T *__restrict__ dy, T *__restrict__ y,
                                                                const float *__restrict__ seg) {
-    constexpr int H = 4 * Q, SL = BLOCK / Q, U = 4, SU = 4;       // slots of a load of the block; its segments of a round a thread
+    constexpr int H = 4 * Q, SL = BLOCK / Q, U = 4;               // slots of a load of the block
     __shared__ float smem[WAVES_PER_BLOCK * WAVE];
     __shared__ float of_head[2][H];
     const int row = P.heavy[3 * blockIdx.x], s0 = P.heavy[3 * blockIdx.x + 1], ns = P.heavy[3 * blockIdx.x + 2];
     const int h = threadIdx.x % H, j0 = threadIdx.x / H, nj = BLOCK / H;
     const int begin = P.rowptr[row], deg = P.rowptr[row + 1] - begin;
     const int per = (deg + (int)gridDim.y - 1) / (int)gridDim.y, first = begin + (int)blockIdx.y * per, end = min(first + per, begin + deg);
-    const int q4 = 4 * ((int)threadIdx.x % Q), mine = first + (int)threadIdx.x / Q;
+    if constexpr (FWD) {
+        float m = -1e9f, s = 0.f;
+        for (int j = j0; j < ns; j += nj) { const float v = seg[((size_t)(s0 + j) * H + h) * 2]; m = v > m ? v : m; }
+        m = head_reduce<float, WAVES_PER_BLOCK, true>(m, H, h, smem);
+        for (int j = j0; j < ns; j += nj) s += seg[((size_t)(s0 + j) * H + h) * 2 + 1] * expf(seg[((size_t)(s0 + j) * H + h) * 2] - m);
+        s = head_reduce<float, WAVES_PER_BLOCK, false>(s, H, h, smem);
+        if (threadIdx.x < H) { of_head[0][h] = m; of_head[1][h] = s; }
+    } else {
+        float s = 0.f;
+        for (int j = j0; j < ns; j += nj) s += seg[(size_t)(s0 + j) * H + h];
+        s = head_reduce<float, WAVES_PER_BLOCK, false>(s, H, h, smem);
+        if (threadIdx.x < H) of_head[0][h] = s;
+    }
+    __syncthreads();
+    const int q4 = 4 * ((int)threadIdx.x % Q);
     float a[4], b[4], v[U][4], d[U][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { a[i] = of_head[0][q4 + i]; b[i] = FWD ? of_head[1][q4 + i] : 0.f; }
     int e[U];
-    auto load = [&](int p) {
+    for (int p = first + (int)threadIdx.x / Q; p < end; p += U * SL) {
         quad_eids<U>(P, p, SL, end, e);
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -1074,44 +1089,6 @@ __global__ __launch_bounds__(BLOCK) void k_softmax_split_quads(bpt_plan P, const
                 Quad<T>::ld(x + (size_t)e[u] * H + q4, v[u]);
                 if constexpr (!FWD) Quad<T>::ld(dy + (size_t)e[u] * H + q4, d[u]);
             }
-    };
-    // the first edges are on their way while the segments are added up
-    load(mine);
-    const float *const sg = seg + ((size_t)s0 * H + h) * (FWD ? 2 : 1);
-    if constexpr (FWD) {
-        float m = -1e9f, s = 0.f;
-        for (int j = j0; j < ns; j += SU * nj) {
-            float2 ms[SU];
-#pragma unroll
-            for (int u = 0; u < SU; ++u) ms[u] = j + u * nj < ns ? *reinterpret_cast<const float2 *>(sg + (size_t)(j + u * nj) * H * 2) : make_float2(-1e9f, 0.f);
-            float mn = m;
-#pragma unroll
-            for (int u = 0; u < SU; ++u) mn = ms[u].x > mn ? ms[u].x : mn;
-            s *= expf(m - mn);
-#pragma unroll
-            for (int u = 0; u < SU; ++u) s += ms[u].y * expf(ms[u].x - mn);
-            m = mn;
-        }
-        const float M = head_reduce<float, WAVES_PER_BLOCK, true>(m, H, h, smem);
-        s = head_reduce<float, WAVES_PER_BLOCK, false>(s * expf(m - M), H, h, smem);
-        if (threadIdx.x < H) { of_head[0][h] = M; of_head[1][h] = s; }
-    } else {
-        float s = 0.f;
-        for (int j = j0; j < ns; j += SU * nj) {
-            float t[SU];
-#pragma unroll
-            for (int u = 0; u < SU; ++u) t[u] = j + u * nj < ns ? sg[(size_t)(j + u * nj) * H] : 0.f;
-#pragma unroll
-            for (int u = 0; u < SU; ++u) s += t[u];
-        }
-        s = head_reduce<float, WAVES_PER_BLOCK, false>(s, H, h, smem);
-        if (threadIdx.x < H) of_head[0][h] = s;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { a[i] = of_head[0][q4 + i]; b[i] = FWD ? of_head[1][q4 + i] : 0.f; }
-    for (int p = mine; p < end; p += U * SL) {
-        if (p != mine) load(p);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (e[u] < 0) continue;
