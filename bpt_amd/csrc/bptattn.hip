@@ -544,12 +544,12 @@ __device__ __forceinline__ bool split_row(const bpt_plan &P, int i, int &begin, 
     return true;
 }
 
-// seg_slot: the item's slot (-1 = whole row)
-template <bool WHOLE> __device__ __forceinline__ bool softmax_range(const bpt_plan &P, int &begin, int &end, int &seg_slot, int whole) {
+// seg_slot: NULL = whole rows only (segments of split rows are skipped); else it receives the item's slot (-1 = whole row)
+__device__ __forceinline__ bool softmax_range(const bpt_plan &P, int &begin, int &end, int *seg_slot, int waves_per_block = WAVES_PER_BLOCK, int skip = 0) {
     Item it;
-    if (!fetch_item(P, it, sm_block<WHOLE>() / WAVE, WHOLE ? whole : 0) || (WHOLE && it.slot >= 0)) return false;
+    if (!fetch_item(P, it, waves_per_block, skip) || (it.slot >= 0 && !seg_slot)) return false;
     begin = it.begin; end = it.end;
-    seg_slot = it.slot;
+    if (seg_slot) *seg_slot = it.slot;
     return true;
 }
 
@@ -584,7 +584,16 @@ __device__ __forceinline__ void softmax_fwd_heads(const bpt_plan &P, int begin, 
 #pragma unroll
         for (int u = 0; u < SM_CACHE; ++u) { vc[u] = exp_acc(vc[u] - m); s += vc[u]; }      // exp(-inf) = 0 for the empty slots
     } else {
-        for (int p = first; p < end; p += nslots) s += exp_acc((acc_t)Elem<T>::ld(x + (size_t)P.eid[p] * H + h) - m);
+        for (int p0 = first; p0 < end; p0 += SM_CACHE * nslots) {
+            int e[SM_CACHE];
+#pragma unroll
+            for (int u = 0; u < SM_CACHE; ++u) { const int p = p0 + u * nslots; e[u] = p < end ? P.eid[p] : -1; }
+            acc_t v[SM_CACHE];
+#pragma unroll
+            for (int u = 0; u < SM_CACHE; ++u) v[u] = e[u] < 0 ? (acc_t)-INFINITY : (acc_t)Elem<T>::ld(x + (size_t)e[u] * H + h);
+#pragma unroll
+            for (int u = 0; u < SM_CACHE; ++u) s += exp_acc(v[u] - m);
+        }
     }
     s = head_reduce<acc_t, NW, false>(s, H, h, smem);
     if (NW == 1 && seg_slot >= 0) {
@@ -618,10 +627,12 @@ __global__ __launch_bounds__(sm_block<WHOLE>()) void k_softmax_fwd_heads(bpt_pla
         __shared__ typename Elem<T>::acc_t smem[SM_WAVES * WAVE];
         if ((int)blockIdx.x < whole) {
             if (split_row(P, blockIdx.x, begin, end)) softmax_fwd_heads<T, SM_WAVES>(P, begin, end, -1, x, y, H, nullptr, smem);
-            return;
+        } else if (softmax_range(P, begin, end, nullptr, SM_WAVES, whole)) {
+            softmax_fwd_heads<T, 1>(P, begin, end, -1, x, y, H, nullptr, nullptr);
         }
+    } else if (softmax_range(P, begin, end, seg ? &slot : nullptr)) {
+        softmax_fwd_heads<T, 1>(P, begin, end, slot, x, y, H, seg, nullptr);
     }
-    if (softmax_range<WHOLE>(P, begin, end, slot, whole)) softmax_fwd_heads<T, 1>(P, begin, end, slot, x, y, H, seg, nullptr);
 }
 
 template <typename T, int NW>
@@ -687,10 +698,12 @@ __global__ __launch_bounds__(sm_block<WHOLE>()) void k_softmax_bwd_heads(bpt_pla
         __shared__ typename Elem<T>::acc_t smem[SM_WAVES * WAVE];
         if ((int)blockIdx.x < whole) {
             if (split_row(P, blockIdx.x, begin, end)) softmax_bwd_heads<T, SM_WAVES>(P, begin, end, -1, y, dy, dx, H, nullptr, smem);
-            return;
+        } else if (softmax_range(P, begin, end, nullptr, SM_WAVES, whole)) {
+            softmax_bwd_heads<T, 1>(P, begin, end, -1, y, dy, dx, H, nullptr, nullptr);
         }
+    } else if (softmax_range(P, begin, end, seg ? &slot : nullptr)) {
+        softmax_bwd_heads<T, 1>(P, begin, end, slot, y, dy, dx, H, seg, nullptr);
     }
-    if (softmax_range<WHOLE>(P, begin, end, slot, whole)) softmax_bwd_heads<T, 1>(P, begin, end, slot, y, dy, dx, H, seg, nullptr);
 }
 
 // Split rows of the softmax, second step: one block per split row.  Forward (PAIR): the segments' (m_i, s_i) are replaced by the
@@ -5432,15 +5445,29 @@ inline unsigned softmax_split_blocks(const bpt_plan *P) {
 }
 inline unsigned softmax_item_blocks(const bpt_plan *P, int q, int block) { return (unsigned)((P->n_items * QUAD_SLOTS * q + block - 1) / block); }
 // How many workgroups in front of the items' take a split row each: none where the plan does not say how long its longest row is, or where
-// one is longer than SM_WHOLE_EDGES.  A workgroup's CU keeps some 64 lines in flight and the records of a span's edges lie in a line
+// one is longer than `longest`.  A workgroup's CU keeps some 64 lines in flight and the records of a span's edges lie in a line
 // each: with the 8192 edges of the longest row of L = 8192 the forward took 39 us and the backward 51, in two launches 22 and 27.  Kernels,
 // two or three launches -> one, forward and backward: 8 heads, L = 500, both ways 9.7 + 8.6 -> 7.2 + 6.4 us; L = 1000 10.9 + 10.0 -> 8.4 + 7.6;
-// 16 graphs of up to 1024 17.9 + 15.4 -> 14.6 + 13.2; 6 heads, L = 1024, k = 8 14.4 + 12.2 -> 13.8 + 11.3.  Passes of the separate operators, which
-// the host bounds there: L = 100 146 -> 139 us, L = 500 151 -> 143, 6 x 50, L = 1024 152 -> 142, the 16 graphs 212 -> 206.
+// 16 graphs of up to 1024 17.9 + 15.4 -> 14.6 + 13.2.  Passes of the separate operators, which
+// the host bounds there: L = 100 146 -> 139 us, L = 500 151 -> 143, the 16 graphs 212 -> 206.
+// Rows of `deg` edges each, forward and backward, times as fast as the launches over segments: 4, 8 or 16 heads 1.2-1.8 and 1.3-2.5 for 100 to 16 000
+// rows of 70 to 1000 edges.
 constexpr int SM_WHOLE_EDGES = 1024;
-inline int softmax_whole_rows(const bpt_plan *P) {
-    if (P->n_heavy == 0 || P->max_degree <= 0 || P->max_degree > SM_WHOLE_EDGES) return 0;
+inline int softmax_whole_rows(const bpt_plan *P, int longest = SM_WHOLE_EDGES) {
+    if (P->n_heavy == 0 || P->max_degree <= 0 || P->max_degree > longest) return 0;
     return (int)((P->n_heavy + 7) & ~(int64_t)7);
+}
+// The same for the kernels with the heads side by side, whose workgroups have fewer slots the more heads there are.  Times as fast as the launches over
+// segments, forward and backward: where the longest row is held at once (SM_CACHE edges a slot) 1.7-2.0 and 1.7-2.1 (1000 or 700 tokens of 1, 3
+// and 5 heads), just past it 1.0 and 1.0 (6 heads, 700 or 1000), 0.85 and 0.9 with one row of 1024 beside 1000 of 64 (5 and 6 heads), 0.6-0.75 and 0.8 at
+// 1024 with 12 heads and more; rows of up to 512 1.6 and 1.3-1.6 with 10 and 12 heads, 1.2-1.3 and 1.1-1.4 with 32 and 64.  A short row leaves
+// most of its workgroup idle, which shows once the chip is full of them: one head, 70 edges 2 and 2.2 at 100 rows, 1.07 and 1.3 at 3000, 0.76
+// and 0.83 at 16 000; 200 edges (four segments) 1.2 and 1.45 at 4000; in float64 1.0 and 1.5 at 1500 rows of 70, 0.8 and 1.1 at 3000, 1.1 and 1.3 at
+// 3000 of 300 (five segments).
+template <typename T> inline int softmax_whole_rows_heads(const bpt_plan *P, int h) {
+    constexpr bool F64 = sizeof(T) == 8;
+    if (P->n_heavy > (F64 ? 1536 : 3072) && P->n_slots < (F64 ? 5 : 4) * P->n_heavy) return 0;
+    return softmax_whole_rows(P, std::min(SM_WHOLE_EDGES, std::max(SM_WHOLE_EDGES / 2, SM_CACHE * SM_WAVES * (WAVE / h))));
 }
 
 template <typename T, int Q>
@@ -5486,7 +5513,7 @@ int run_softmax_fwd(const bpt_plan *P, const void *x, void *y, void *ws, int h, 
     }
     if (h <= WAVE) {           // heads side by side; split rows in three steps over their segments
         acc_t *seg = P->n_heavy > 0 ? (acc_t *)ws : nullptr;
-        const int whole = softmax_whole_rows(P);
+        const int whole = softmax_whole_rows_heads<T>(P, h);
         if (whole > 0)
             hipLaunchKernelGGL((k_softmax_fwd_heads<T, true>), dim3(whole + (unsigned)((P->n_items + SM_WAVES - 1) / SM_WAVES)), dim3(SM_BLOCK), 0, s,
                                *P, (const T *)x, (T *)y, h, (acc_t *)nullptr, whole);
@@ -5517,7 +5544,7 @@ int run_softmax_bwd(const bpt_plan *P, const void *y, const void *dy, void *dx, 
     }
     if (h <= WAVE) {           // heads side by side; split rows in three steps over their segments
         acc_t *seg = P->n_heavy > 0 ? (acc_t *)ws : nullptr;
-        const int whole = softmax_whole_rows(P);
+        const int whole = softmax_whole_rows_heads<T>(P, h);
         if (whole > 0)
             hipLaunchKernelGGL((k_softmax_bwd_heads<T, true>), dim3(whole + (unsigned)((P->n_items + SM_WAVES - 1) / SM_WAVES)), dim3(SM_BLOCK), 0, s,
                                *P, (const T *)y, (const T *)dy, (T *)dx, h, (acc_t *)nullptr, whole);
