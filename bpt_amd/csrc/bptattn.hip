@@ -1064,7 +1064,9 @@ __global__ __launch_bounds__(sm_block<WHOLE>()) void k_softmax_bwd_quads(bpt_pla
 }
 
 // Split rows, second launch: block (i, j) is the j-th of gridDim.y blocks of split row i.  Every block reduces the row's segments
-// by itself (16 bytes a segment and head at most: they come from the L2), then writes its share of the row's edges.
+// by itself (16 bytes a segment and head at most: they come from the L2), then writes its share of the row's edges.  (Its first edges asked for
+// ahead of the sums: 7.7 -> 7.0 us forward and 7.8 -> 7.4 backward at L = 8192, k = 4, which has 127 split rows, but 66 -> 76 and 45 -> 52 at a
+// window of 200, L = 4096, which has 4033.)
 template <typename T, int Q, bool FWD>
 __global__ __launch_bounds__(BLOCK) void k_softmax_split_quads(bpt_plan P, const T *__restrict__ x, const T *__restrict__ dy, T *__restrict__ y,
                                                                const float *__restrict__ seg) {
@@ -5669,11 +5671,11 @@ struct RelBwdShape {
     int nw, cs;
 };
 // One wavefront a table where that puts eight on a compute unit (workgroups that fit its 160 KB of LDS x wavefronts each; more tables per
-// workgroup on a tie: fewer partial tables), which holds up to 62 types; else the shape with most of them.  Two wavefronts a table read and stage
-// an item's ds and types twice: at 48 types, where LDS holds eight either way, 39.5 against 39.6 us (8 heads, L = 8192, k = 4), at 55
-// 113 against 123 (bfloat16, L = 32768, k = 2).  Where it holds two or four: 173 types (8 heads, L = 8192, k = 8 both ways) 180 -> 142 us, 140 (4
-// heads, L = 6215, k = 6 both ways) 98 -> 76, 134 (16 heads bfloat16, a batch with k = 20) 124 -> 107; 16 heads, L = 4096, k = 16 level.  Four a
-// table: 77, 130 and 138 in the last three places.
+// workgroup on a tie: fewer partial tables), which it does up to 59 types with 4 heads, 56 with 8 and 49 with 16; else the shape with most of
+// them.  Two wavefronts a table read and stage an item's ds and types twice.  Kernel alone, one against two: where LDS holds eight, 55 types (8
+// heads, L = 8192, k = 4) 41.4 us against 52.0, 33 (8 heads bfloat16, L = 32768, k = 2) 116 against 126; where it holds two, 173 (8 heads, L = 8192,
+// k = 8 both ways) 182 against 148, 134 (4 heads, L = 6215, k = 6 both ways) 101 against 79, 140 (16 heads, L = 4096, k = 16) 110 against 106.  Four a
+// table: 77 in the fourth place and 138 in the last.
 // A workgroup takes at most 144 KB (large_lds false: at most the 64 KB every kernel may take).  nw 0: no configuration fits.
 inline RelBwdShape rel_bwd_shape(int64_t n_used, int h, bool large_lds = true) {
     const size_t cap = (large_lds ? 144 : 64) * 1024;
